@@ -1407,8 +1407,9 @@ struct Layout {
   void* binned;
   size_t binned_bytes;
   uint32_t* tables;
-  void* cell_lo;
-  void* cell_invw;
+  void* map_x;
+  float* map_t;
+  int32_t* straight;
   // quantiser
   double* part_a[2];
   double* part_b[2];
@@ -1479,9 +1480,10 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
   // bin cache: one or two bytes per (row, feature); used when the tree has at least two levels
   L.binned_bytes = max_depth >= 2 ? static_cast<size_t>(N) * bin_row_bytes_max(F, S) : 0;
   L.binned       = max_depth >= 2 ? static_cast<void*>(ar.take<char>(L.binned_bytes + 16)) : nullptr;
-  L.tables       = ar.take<uint32_t>(static_cast<size_t>(F) * kMaxCells / 16);
-  L.cell_lo      = ar.take<double>(F);
-  L.cell_invw    = ar.take<double>(F);
+  L.tables       = ar.take<uint32_t>(2 * static_cast<size_t>(F) * kMaxCells / 16);
+  L.map_x        = ar.take<double>(4 * static_cast<size_t>(F));
+  L.map_t        = ar.take<float>(2 * static_cast<size_t>(F));
+  L.straight     = ar.take<int32_t>(F);
   int64_t n_chunks = (N * K + 4095) / 4096;
   for (int i = 0; i < 2; i++) {
     L.part_a[i] = ar.take<double>(n_chunks);
@@ -1711,8 +1713,9 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
   hs.groups     = L.groups;
   hs.sgroups    = L.sgroups;
   hs.tables     = L.tables;
-  hs.cell_lo    = L.cell_lo;
-  hs.cell_invw  = L.cell_invw;
+  hs.map_x      = L.map_x;
+  hs.map_t      = L.map_t;
+  hs.straight   = L.straight;
   hs.tile_start = L.tile_start;
   hs.tiles      = L.tiles;
   hs.binned     = L.binned;
@@ -2359,8 +2362,9 @@ struct HistStageLayout {
   void* binned;
   size_t binned_bytes;
   uint32_t* tables;
-  void* cell_lo;
-  void* cell_invw;
+  void* map_x;
+  float* map_t;
+  int32_t* straight;
   int32_t* bin_feature;
   unsigned long long* qstats;
   int32_t* flag;
@@ -2392,9 +2396,10 @@ void make_hist_stage_layout(Arena& ar, HistStageLayout& L, int64_t N, int F, int
   L.upload_bytes = ar.used - upload_at;
   L.binned_bytes = static_cast<size_t>(N) * bin_row_bytes_max(F, S);
   L.binned       = ar.take<char>(L.binned_bytes + 16);
-  L.tables       = ar.take<uint32_t>(static_cast<size_t>(F) * kMaxCells / 16);
-  L.cell_lo      = ar.take<double>(F);
-  L.cell_invw    = ar.take<double>(F);
+  L.tables       = ar.take<uint32_t>(2 * static_cast<size_t>(F) * kMaxCells / 16);
+  L.map_x        = ar.take<double>(4 * static_cast<size_t>(F));
+  L.map_t        = ar.take<float>(2 * static_cast<size_t>(F));
+  L.straight     = ar.take<int32_t>(F);
   L.bin_feature  = ar.take<int32_t>(static_cast<size_t>(F) * S);
   L.qstats       = ar.take<unsigned long long>(2);
   L.flag         = ar.take<int32_t>(4);
@@ -2552,7 +2557,7 @@ int lbt_histogram_level(void* stream, const void* X, int32_t x_dtype, int64_t n_
   LBT_REQUIRE(bad == 0, "positions must be (node, row) pairs sorted by node whose nodes are -1 or of level %d", level);
 
   HistSetup hs;
-  hs.groups = L.groups; hs.sgroups = L.sgroups; hs.tables = L.tables; hs.cell_lo = L.cell_lo; hs.cell_invw = L.cell_invw;
+  hs.groups = L.groups; hs.sgroups = L.sgroups; hs.tables = L.tables; hs.map_x = L.map_x; hs.map_t = L.map_t; hs.straight = L.straight;
   hs.tile_start = L.tile_start; hs.tiles = L.tiles; hs.binned = L.binned; hs.binned_capacity = L.binned_bytes;
   hs.bin_base = L.bin_base; hs.bin_stride = L.bin_stride; hs.bin_tail = L.bin_tail; hs.rec = L.rec;
   hs.upload_block = L.upload_block; hs.upload_bytes = L.upload_bytes;

@@ -10,10 +10,10 @@
 //     bin cache). The histograms of all levels, the root included, are then
 //     accumulated from the cache (binned_histogram_kernel); a level reads a
 //     quarter of the bytes X would cost and does no search.
-//   * Bin search: cell = clamp((x - lo) * invw) indexes a per-feature table that
-//     gives the number of proposals in cells before it; a short forward probe over
-//     the proposals finishes the search. Any monotone cell function is exact
-//     here; the table is built on the device with the same function. Proposals
+//   * Bin search: a monotone function of the value, fitted to the feature's proposals, gives a
+//     cell of a per-feature table that holds the number of proposals in cells before it; a
+//     short forward probe over the proposals finishes the search. Any monotone cell function
+//     is exact here; the table is built on the device with the same function. Proposals
 //     and tables of a search group of features sit in LDS (all 100 features of a
 //     10M x 100 matrix with 256 proposals each are one group).
 //   * The packed sub-histogram of a histogram group of features (8 bytes per bin)
@@ -38,6 +38,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 namespace lbt {
 namespace {
@@ -252,22 +253,51 @@ __global__ void __launch_bounds__(kPlanThreads)
   }
 }
 
-// The cell of a value, t = x * invw + nlo clamped to [0, cmax]: monotone non-decreasing in x
-// for any nlo and invw >= 0 (a fused multiply-add rounds once, and rounding and clamping keep
-// order); NaN goes to cell 0. Table construction and lookup share this function, which is
-// all that exactness needs.
-__device__ inline int cell_of(float x, float nlo, float invw, float cmax)
+// The cell of a value. Equal cells over the range of the proposals serve evenly spread columns only:
+// with a long tail (lognormal columns) most proposals crowd into a few of them, the table's start then
+// lies far before the bin and nearly every wave has a lane that walks on (4M x 100 lognormal values: 1.74 ms
+// where uniform ones took 0.54). So the axis is bent first:
+//   d = (x - centre) * scale,  g = sign(d) * log2(1 + |d|) in its piecewise linear form
+// (the bits of the float 1 + |d| read as an integer), which is exactly linear for |d| <= 1 and
+// logarithmic beyond; build_cells_kernel picks centre and scale per feature, a scale that keeps the
+// whole range inside |d| <= 1 being one of its choices. The cell is then g * invw + nlo clamped to
+// [0, cmax]. Every step is monotone non-decreasing in x (a fused multiply-add with a non-negative factor
+// rounds once, and rounding, the bit pattern of positive floats and clamping keep order), and table
+// construction and lookup share this function, which is all that exactness needs. NaN goes to cell 0.
+template <typename T>
+struct CellMap {
+  T scale, shift;      // d = x * scale + shift
+  float invw, nlo;     // t = g * invw + nlo
+};
+__device__ __forceinline__ float bend(float d)
 {
-  // the median of (t, 0, cmax) is the clamp; with a NaN operand the instruction returns the
-  // minimum of the others, 0
-  return static_cast<int>(__builtin_amdgcn_fmed3f(fmaf(x, invw, nlo), 0.0f, cmax));
+  const int k = __float_as_int(fabsf(d) + 1.0f) - 0x3f800000;
+  return copysignf(static_cast<float>(k), d);
 }
-__device__ inline int cell_of(double x, double nlo, double invw, double cmax)
+template <typename T>
+__device__ __forceinline__ float bend_axis(T x, T scale, T shift)
 {
-  double t = fma(x, invw, nlo);
-  t        = t > 0.0 ? t : 0.0;  // false for NaN
-  t        = t < cmax ? t : cmax;
-  return static_cast<int>(t);
+  // the median of (x, -max, max) clamps infinities; with a NaN operand it is the minimum of the others
+  if constexpr (sizeof(T) == 4) {
+    constexpr float kMax = std::numeric_limits<float>::max();
+    return bend(fmaf(__builtin_amdgcn_fmed3f(x, -kMax, kMax), scale, shift));
+  } else {
+    constexpr double kMax = std::numeric_limits<double>::max();
+    const double v        = x > -kMax ? x : -kMax;  // false for NaN
+    return bend(static_cast<float>(fma(v, scale, shift)));
+  }
+}
+template <typename T>
+__device__ __forceinline__ int cell_of(T x, T scale, T shift, float invw, float nlo, float cmax)
+{
+  return static_cast<int>(__builtin_amdgcn_fmed3f(fmaf(bend_axis(x, scale, shift), invw, nlo), 0.0f, cmax));
+}
+// Without the bend, for features whose proposals spread evenly: six vector instructions less per value,
+// which the binning pass feels (4M x 100 uniform values: 0.60 ms bent, 0.54 straight).
+template <typename T>
+__device__ __forceinline__ int straight_cell_of(T x, T a, T b, float cmax)
+{
+  return static_cast<int>(__builtin_amdgcn_fmed3f(static_cast<float>(fma(x, a, b)), 0.0f, cmax));
 }
 
 // Lookup table of a feature: the value range is cut into C fine cells (many more than there
@@ -288,41 +318,48 @@ __device__ inline int table_start(uint32_t word, int cell)
   return static_cast<int>(word >> 16) + __popc(word & ((1u << (cell & (kCellsPerWord - 1))) - 1u));
 }
 
+// The bent map of a feature is the one of a few candidates (linear; logarithmic on both sides of a
+// centre at the low end, the median or the high end of the proposals, at three scales) that leaves the
+// fewest proposals in a cell with their predecessor: the proposals are a sample of the column, so they
+// say where its values fall. Each wave tries every fourth candidate.
+constexpr int kCellMaps = 10;
 template <typename T>
-__global__ void __launch_bounds__(256)
-  build_cells_kernel(const T* proposals, const int32_t* row_pointers, int C, uint32_t* tables, T* lo_out,
-                     T* invw_out)
+__device__ inline CellMap<T> cell_map_candidate(int c, const T* p, int n, float cells)
 {
-  __shared__ T s_lo, s_invw;
-  const int f = blockIdx.x;
-  const T* p  = proposals + row_pointers[f];
-  const int n = row_pointers[f + 1] - row_pointers[f];
-  if (threadIdx.x == 0) {
-    T lo = T(0), invw = T(0);
-    if (n >= 3) {  // at least two finite proposals (the last one is +inf)
-      lo   = p[0];
-      T hi = p[n - 2];
-      T w  = hi - lo;
-      if (w > T(0) && w < std::numeric_limits<T>::infinity()) {
-        invw = static_cast<T>(C) / w;
-        if (!(invw < std::numeric_limits<T>::infinity())) invw = T(0);
-      }
-      if (!(lo == lo) || lo == -std::numeric_limits<T>::infinity()) {
-        lo   = T(0);
-        invw = T(0);
-      }
-    }
-    // the kernels evaluate x * invw + nlo
-    T nlo = -lo * invw;
-    if (!(nlo == nlo)) nlo = T(0);
-    s_lo        = nlo;
-    s_invw      = invw;
-    lo_out[f]   = nlo;
-    invw_out[f] = invw;
+  CellMap<T> m{T(0), T(0), 0.0f, 0.0f};
+  if (n < 3) return m;  // at least two finite proposals (the last one is +inf)
+  const T lo = p[0], hi = p[n - 2], mid = p[(n - 1) / 2];
+  const T width = hi - lo;
+  // (a -inf proposal, or a range that overflows: everything in cell 0)
+  if (!(width > T(0) && width < std::numeric_limits<T>::infinity())) return m;
+  T centre = lo, scale = T(1) / width;
+  if (c > 0) {
+    const int where = (c - 1) % 3, fine = (c - 1) / 3;
+    centre          = where == 0 ? mid : (where == 1 ? lo : hi);
+    // half of the proposals lie inside one unit of d (fine = 0), a quarter, an eighth
+    const int q  = max(1, (n - 1) >> (2 + fine));
+    const int at = (n - 1) / 2;
+    T reach      = where == 0 ? (p[min(n - 2, at + q)] - p[max(0, at - q)]) / T(2)
+                              : (where == 1 ? p[min(n - 2, 2 * q)] - lo : hi - p[max(0, n - 2 - 2 * q)]);
+    if (!(reach > width * T(1e-6))) reach = width * T(1e-6);
+    scale = T(1) / reach;
   }
-  __syncthreads();
-  const T nlo = s_lo, invw = s_invw, cmax = static_cast<T>(C - 1);
-  const int words = C / kCellsPerWord;
+  const T shift = -centre * scale;
+  if (!(scale < std::numeric_limits<T>::infinity()) || !(shift - shift == T(0))) return m;
+  const float g_lo = bend_axis(lo, scale, shift), g_hi = bend_axis(hi, scale, shift);
+  const float invw = cells / (g_hi - g_lo);
+  if (!(g_hi > g_lo) || !(invw < std::numeric_limits<float>::infinity())) return m;
+  m.scale = scale;
+  m.shift = shift;
+  m.invw  = invw;
+  m.nlo   = -g_lo * invw;
+  return m;
+}
+
+// Table words of a feature under the cell function `cell`.
+template <typename T, typename CellFn>
+__device__ inline void write_cell_words(const T* p, int n, int words, uint32_t* table, CellFn cell)
+{
   for (int w = threadIdx.x; w < words; w += blockDim.x) {
     // first proposal whose cell is >= the first cell of the word (the cells of the ascending
     // proposals ascend too)
@@ -330,7 +367,7 @@ __global__ void __launch_bounds__(256)
     int a = 0, len = n;
     while (len > 0) {
       int half = len >> 1;
-      if (cell_of(p[a + half], nlo, invw, cmax) < c0) {
+      if (cell(p[a + half]) < c0) {
         a += half + 1;
         len -= half + 1;
       } else {
@@ -339,11 +376,70 @@ __global__ void __launch_bounds__(256)
     }
     uint32_t bits = 0;
     for (int i = a; i < n; i++) {
-      const int c = cell_of(p[i], nlo, invw, cmax);
+      const int c = cell(p[i]);
       if (c >= c0 + kCellsPerWord) break;
       bits |= 1u << (c - c0);
     }
-    tables[static_cast<int64_t>(f) * words + w] = (static_cast<uint32_t>(a) << 16) | bits;
+    table[w] = (static_cast<uint32_t>(a) << 16) | bits;
+  }
+}
+
+// tables: [2][F][words], the bent maps' tables first. A feature is straight when the plain linear map
+// leaves few of its proposals in a cell with their predecessor (normal columns: one in seven); only
+// then its second table is written, and a search group all of whose features are straight uses those.
+// Maps: map_x [2][F][2] (bent: scale, shift; straight: a, b), map_t [F][2], straight [F].
+template <typename T>
+__global__ void __launch_bounds__(256)
+  build_cells_kernel(const T* proposals, const int32_t* row_pointers, int F, int C, uint32_t* tables, T* map_x,
+                     float* map_t, int32_t* straight)
+{
+  __shared__ T s_p[LBT_MAX_SPLIT_SAMPLES];
+  __shared__ int s_crowded[kCellMaps];
+  const int f = blockIdx.x;
+  const int b0 = row_pointers[f];
+  const int n  = row_pointers[f + 1] - b0;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) s_p[i] = proposals[b0 + i];
+  __syncthreads();
+  const T* p       = s_p;
+  const float cmax = static_cast<float>(C - 1);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int c = wave; c < kCellMaps; c += 4) {
+    const CellMap<T> m = cell_map_candidate(c, p, n, static_cast<float>(C));
+    int crowded        = 0;
+    for (int i = 1 + lane; i < n - 1; i += 64)
+      crowded += cell_of(p[i], m.scale, m.shift, m.invw, m.nlo, cmax) ==
+                 cell_of(p[i - 1], m.scale, m.shift, m.invw, m.nlo, cmax) ? 1 : 0;
+    for (int off = 32; off >= 1; off >>= 1) crowded += __shfl_xor(crowded, off, 64);
+    if (lane == 0) s_crowded[c] = crowded;
+  }
+  __syncthreads();
+  int best = 0;
+  for (int c = 1; c < kCellMaps; c++)
+    if (s_crowded[c] < s_crowded[best]) best = c;
+  const CellMap<T> m = cell_map_candidate(best, p, n, static_cast<float>(C));
+  const int words    = C / kCellsPerWord;
+  write_cell_words(p, n, words, tables + static_cast<int64_t>(f) * words,
+                   [&](T x) { return cell_of(x, m.scale, m.shift, m.invw, m.nlo, cmax); });
+  // candidate 0 stands for the straight map, whose cells differ from it by roundings only
+  T a = T(0), b = T(0);
+  bool even = 4 * s_crowded[0] <= n;
+  if (n >= 3 && even) {
+    const T lo = p[0], width = p[n - 2] - lo;
+    if (width > T(0) && width < std::numeric_limits<T>::infinity()) a = static_cast<T>(C) / width;
+    b = -lo * a;
+    if (!(a < std::numeric_limits<T>::infinity()) || !(b - b == T(0))) a = b = T(0);
+  }
+  if (even)
+    write_cell_words(p, n, words, tables + static_cast<int64_t>(F + f) * words,
+                     [&](T x) { return straight_cell_of(x, a, b, cmax); });
+  if (threadIdx.x == 0) {
+    map_x[2 * f]           = m.scale;
+    map_x[2 * f + 1]       = m.shift;
+    map_x[2 * (F + f)]     = a;
+    map_x[2 * (F + f) + 1] = b;
+    map_t[2 * f]           = m.invw;
+    map_t[2 * f + 1]       = m.nlo;
+    straight[f]            = even ? 1 : 0;
   }
 }
 
@@ -414,8 +510,8 @@ struct HistArgs {
   const int32_t* row_pointers;
   const int32_t* groups;  // feature groups: [n_groups+1]
   const uint32_t* tables;
-  const T* cell_lo;
-  const T* cell_invw;
+  const T* map_x;      // scale, shift (see build_cells_kernel)
+  const float* map_t;  // invw, nlo
   int cells;
   int search_steps;
   HistView hist;
@@ -722,18 +818,21 @@ __global__ void __launch_bounds__(kHistThreads)
   const bool active       = rsub < w.rpp;
   const int fl            = lr * VEC;  // first group-local feature of this lane
 
-  T c_lo[VEC], c_invw[VEC];
+  T c_scale[VEC], c_shift[VEC];
+  float c_invw[VEC], c_nlo[VEC];
   int c_cell[VEC], c_prop[VEC], c_end[VEC];
 #pragma unroll
   for (int v = 0; v < VEC; v++) {
     int f     = min(f0 + fl + v, f1 - 1);
-    c_lo[v]   = a.cell_lo[f];
-    c_invw[v] = a.cell_invw[f];
+    c_scale[v] = a.map_x[2 * f];
+    c_shift[v] = a.map_x[2 * f + 1];
+    c_invw[v]  = a.map_t[2 * f];
+    c_nlo[v]   = a.map_t[2 * f + 1];
     c_cell[v] = (f - f0) * (C / kCellsPerWord);
     c_prop[v] = a.row_pointers[f] - bin0;
     c_end[v]  = a.row_pointers[f + 1] - bin0;
   }
-  const T cmax = static_cast<T>(C - 1);
+  const float cmax = static_cast<float>(C - 1);
   const unsigned long long max_abs = qstats[0];
 
   const int n_tiles = meta->n_tiles;
@@ -838,7 +937,7 @@ __global__ void __launch_bounds__(kHistThreads)
 #pragma unroll
         for (int v = 0; v < VEC; v++) {
           const T x = xs[v];
-          const int cell = cell_of(x, c_lo[v], c_invw[v], cmax);
+          const int cell = cell_of(x, c_scale[v], c_shift[v], c_invw[v], c_nlo[v], cmax);
           int bn         = c_prop[v] + table_start(s_cell[c_cell[v] + (static_cast<unsigned>(cell) >> kCellShift)], cell);
           bool lt    = s_prop[bn] < x;
           int probes = 0;
@@ -898,8 +997,9 @@ struct BinRowsArgs {
   const int32_t* bin_feature;  // [bins] feature of every proposal
   const int32_t* sgroups;      // search groups: [n_sgroups+1]
   const uint32_t* tables;
-  const T* cell_lo;
-  const T* cell_invw;
+  const T* map_x;      // maps and tables as build_cells_kernel writes them
+  const float* map_t;
+  const int32_t* straight;  // [F] the feature has a table for the straight cell function too
   int cells;
   int search_steps;
   int n_sgroups;
@@ -942,8 +1042,12 @@ __global__ void __launch_bounds__(kHistThreads)
     const int f = min(i / kProbePad, gs - 1);  // the slack follows the last feature
     s_prop[a.row_pointers[f0 + f + 1] - bin0 + kProbePad * f + (i - kProbePad * f)] = std::numeric_limits<T>::infinity();
   }
+  // the straight cell function and its tables when every feature of the group has them
+  bool bent_feature = false;
+  for (int i = threadIdx.x; i < gs; i += kHistThreads) bent_feature |= a.straight[f0 + i] == 0;
+  const bool bent = __syncthreads_or(bent_feature);
   {
-    const uint32_t* src = a.tables + static_cast<int64_t>(f0) * (C / kCellsPerWord);
+    const uint32_t* src = a.tables + static_cast<int64_t>(bent ? f0 : a.F + f0) * (C / kCellsPerWord);
     const int words     = gs * (C / kCellsPerWord);
     for (int i = threadIdx.x; i < words; i += kHistThreads) s_cell[i] = src[i];
   }
@@ -956,18 +1060,22 @@ __global__ void __launch_bounds__(kHistThreads)
   const int fb            = f0 + lr * VEC;  // first feature of this lane
   const int mine          = kRagged ? min(VEC, f1 - fb) : VEC;
   const int shift         = VEC - mine;     // its values are the last `mine` of the VEC it loads
-  T c_lo[VEC], c_invw[VEC];
+  T c_scale[VEC], c_shift[VEC];
+  float c_invw[VEC], c_nlo[VEC];
   int c_cell[VEC], c_prop[VEC], c_end[VEC];
 #pragma unroll
   for (int v = 0; v < VEC; v++) {
     const int f = kRagged ? min(fb + v, f1 - 1) : fb + v;
-    c_lo[v]   = a.cell_lo[f];
-    c_invw[v] = a.cell_invw[f];
+    const int at = 2 * (bent ? f : a.F + f);
+    c_scale[v] = a.map_x[at];
+    c_shift[v] = a.map_x[at + 1];
+    c_invw[v]  = a.map_t[2 * f];
+    c_nlo[v]   = a.map_t[2 * f + 1];
     c_cell[v] = (f - f0) * (C / kCellsPerWord);
     c_prop[v] = a.row_pointers[f] - bin0 + kProbePad * (f - f0);
     c_end[v]  = a.row_pointers[f + 1] - bin0 + kProbePad * (f - f0);
   }
-  const T cmax         = static_cast<T>(C - 1);
+  const float cmax     = static_cast<float>(C - 1);
   const int pitch      = a.bin_stride[fb];
   BinT* const bin_base = binned + a.bin_base[fb];
   // what this lane writes behind its own bins (byte offsets from its first bin). A record ends
@@ -1036,7 +1144,7 @@ __global__ void __launch_bounds__(kHistThreads)
       }
     }
   };
-  auto search_pass = [&](int first, const Vec (&x_c)[kUnroll]) {
+  auto search_pass = [&](auto bent_cells, int first, const Vec (&x_c)[kUnroll]) {
     // the few lanes that copy gradient pairs fetch them now; the search below hides the latency
     int2 q_c[kUnroll];
     if (tq >= 0) {
@@ -1083,7 +1191,8 @@ __global__ void __launch_bounds__(kHistThreads)
 #pragma unroll
         for (int v = 0; v < VEC; v++) {
           const T x      = xs[v];
-          const int cell = cell_of(x, c_lo[v], c_invw[v], cmax);
+          const int cell = decltype(bent_cells)::value ? cell_of(x, c_scale[v], c_shift[v], c_invw[v], c_nlo[v], cmax)
+                                                       : straight_cell_of(x, c_scale[v], c_shift[v], cmax);
           bn[v]          = c_prop[v] + table_start(s_cell[c_cell[v] + (static_cast<unsigned>(cell) >> kCellShift)], cell);
           const T* pp    = s_prop + bn[v];
           cnt[v]         = (pp[0] < x ? 1 : 0) + (pp[1] < x ? 1 : 0) + (pp[2] < x ? 1 : 0);
@@ -1136,14 +1245,20 @@ __global__ void __launch_bounds__(kHistThreads)
       }
     }
   };
-  Vec x_c[kUnroll], x_n[kUnroll];
-  if (n_local > 0) load_pass(0, x_c);
-  for (int first = 0; first < n_local; first += pass_rows) {
-    if (first + pass_rows < n_local) load_pass(first + pass_rows, x_n);
-    search_pass(first, x_c);
+  auto walk = [&](auto bent_cells) {
+    Vec x_c[kUnroll], x_n[kUnroll];
+    if (n_local > 0) load_pass(0, x_c);
+    for (int first = 0; first < n_local; first += pass_rows) {
+      if (first + pass_rows < n_local) load_pass(first + pass_rows, x_n);
+      search_pass(bent_cells, first, x_c);
 #pragma unroll
-    for (int u = 0; u < kUnroll; u++) x_c[u] = x_n[u];
-  }
+      for (int u = 0; u < kUnroll; u++) x_c[u] = x_n[u];
+    }
+  };
+  if (bent)
+    walk(std::true_type{});
+  else
+    walk(std::false_type{});
 }
 
 // Histogram of one level from the cached bins: a lane loads BV cached bins of its
@@ -1723,8 +1838,9 @@ int hist_launch_t(hipStream_t stream, const HistSetup& hs, const HistBatch& b, i
     a.bin_feature  = b.bin_feature;
     a.sgroups      = hs.sgroups;
     a.tables       = hs.tables;
-    a.cell_lo      = static_cast<const T*>(hs.cell_lo);
-    a.cell_invw    = static_cast<const T*>(hs.cell_invw);
+    a.map_x        = static_cast<const T*>(hs.map_x);
+    a.map_t        = hs.map_t;
+    a.straight     = hs.straight;
     a.cells        = hs.cells;
     a.search_steps = hs.search_steps;
     a.n_sgroups    = hs.n_sgroups;
@@ -1826,8 +1942,8 @@ int hist_launch_t(hipStream_t stream, const HistSetup& hs, const HistBatch& b, i
   a.row_pointers = b.row_pointers;
   a.groups       = hs.groups;
   a.tables       = hs.tables;
-  a.cell_lo      = static_cast<const T*>(hs.cell_lo);
-  a.cell_invw    = static_cast<const T*>(hs.cell_invw);
+  a.map_x        = static_cast<const T*>(hs.map_x);
+  a.map_t        = hs.map_t;
   a.cells        = hs.cells;
   a.search_steps = hs.search_steps;
   a.hist         = b.hist;
@@ -2184,13 +2300,11 @@ int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, i
   LBT_TRY(up.send(stream, hs.upload_block, hs.upload_bytes));
   ProfScope ps(LBT_PROF_PROPOSALS, stream);
   if (is_f64)
-    build_cells_kernel<double><<<F, 256, 0, stream>>>(static_cast<const double*>(proposals), row_pointers, cells,
-                                                     hs.tables, static_cast<double*>(hs.cell_lo),
-                                                     static_cast<double*>(hs.cell_invw));
+    build_cells_kernel<double><<<F, 256, 0, stream>>>(static_cast<const double*>(proposals), row_pointers, F, cells,
+                                                     hs.tables, static_cast<double*>(hs.map_x), hs.map_t, hs.straight);
   else
-    build_cells_kernel<float><<<F, 256, 0, stream>>>(static_cast<const float*>(proposals), row_pointers, cells,
-                                                    hs.tables, static_cast<float*>(hs.cell_lo),
-                                                    static_cast<float*>(hs.cell_invw));
+    build_cells_kernel<float><<<F, 256, 0, stream>>>(static_cast<const float*>(proposals), row_pointers, F, cells,
+                                                    hs.tables, static_cast<float*>(hs.map_x), hs.map_t, hs.straight);
   return LBT_OK;
 }
 

@@ -344,9 +344,11 @@ struct HistSetup {
   // device buffers (carved from the caller's workspace)
   int32_t* groups    = nullptr;  // [n_groups + 1]
   int32_t* sgroups   = nullptr;  // [n_sgroups + 1]; the same array as groups when the cache is off
-  uint32_t* tables   = nullptr;  // [n_features][cells / 16]: one word per 16 cells
-  void* cell_lo      = nullptr;  // X dtype [n_features]
-  void* cell_invw    = nullptr;  // X dtype [n_features]
+  // lookup tables and cell functions of the search (see build_cells_kernel)
+  uint32_t* tables   = nullptr;  // [2][n_features][cells / 16]: one word per 16 cells
+  void* map_x        = nullptr;  // X dtype [2][n_features][2]
+  float* map_t       = nullptr;  // [n_features][2]
+  int32_t* straight  = nullptr;  // [n_features]
   int32_t* tile_start = nullptr;
   int4* tiles         = nullptr;  // one descriptor per tile of the batch in flight
   LevelMeta* meta    = nullptr;
