@@ -6,6 +6,7 @@
 // Semantics follow rapidsai/legate-boost src/models/tree/build_tree.cu and
 // build_tree.h (cited per kernel); the decomposition into kernels is this
 // library's own and is written for gfx950 (64-wide waves, 160 KB LDS per CU).
+#include "lbt_device.h"
 #include "lbt_internal.h"
 
 #include <algorithm>
@@ -17,48 +18,6 @@ namespace lbt {
 namespace {
 
 constexpr int kThreads = 256;
-
-// ---------------------------------------------------------------------------
-// small helpers
-// ---------------------------------------------------------------------------
-
-template <typename T>
-struct KeyOf;
-template <>
-struct KeyOf<float> {
-  using type = uint32_t;
-};
-template <>
-struct KeyOf<double> {
-  using type = uint64_t;
-};
-
-// Order-preserving map from IEEE bits to unsigned integers (-0.0 < +0.0).
-__device__ inline uint32_t to_key(float v)
-{
-  uint32_t u = __float_as_uint(v);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ inline uint64_t to_key(double v)
-{
-  uint64_t u = static_cast<uint64_t>(__double_as_longlong(v));
-  return (u & 0x8000000000000000ULL) ? ~u : (u | 0x8000000000000000ULL);
-}
-__device__ inline float from_key(uint32_t k)
-{
-  uint32_t u = (k & 0x80000000u) ? (k & 0x7fffffffu) : ~k;
-  return __uint_as_float(u);
-}
-__device__ inline double from_key(uint64_t k)
-{
-  uint64_t u = (k & 0x8000000000000000ULL) ? (k & 0x7fffffffffffffffULL) : ~k;
-  return __longlong_as_double(static_cast<long long>(u));
-}
-
-__device__ inline void atomic_add_i64(int64_t* p, int64_t v)
-{
-  atomicAdd(reinterpret_cast<unsigned long long*>(p), static_cast<unsigned long long>(v));
-}
 
 // ---------------------------------------------------------------------------
 // tree initialisation / output (build_tree.cu:785-861)
@@ -429,36 +388,6 @@ __global__ void root_leaf_kernel(double* leaf, const I64Pair* node_sums, int K,
 // (feature, node), 64 bins per step
 // ---------------------------------------------------------------------------
 
-// Running sums over the 64 lanes of a wave through the lanes' own data paths (DPP operands)
-// instead of LDS permutes, of which a 64-bit scan by shuffles needs two dozen: inside every row
-// of 16 lanes by shifts of 1, 2, 4 and 8 lanes (a lane without a source reads zero), then the
-// last lane of row 0 into row 1 and of row 2 into row 3, then lane 31 into rows 2 and 3.
-// All 64 lanes must be active.
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ int64_t dpp_take(int64_t v)
-{
-  const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(static_cast<uint32_t>(v)), kCtrl, kRowMask, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(v >> 32), kCtrl, kRowMask, 0xf, true);
-  return static_cast<int64_t>((static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo));
-}
-__device__ __forceinline__ int64_t wave_inclusive_sum(int64_t v)
-{
-  v += dpp_take<0x111, 0xf>(v);  // row_shr:1
-  v += dpp_take<0x112, 0xf>(v);  // row_shr:2
-  v += dpp_take<0x114, 0xf>(v);  // row_shr:4
-  v += dpp_take<0x118, 0xf>(v);  // row_shr:8
-  v += dpp_take<0x142, 0xa>(v);  // row_bcast:15, rows 1 and 3
-  v += dpp_take<0x143, 0xc>(v);  // row_bcast:31, rows 2 and 3
-  return v;
-}
-// value of lane `src` (the same for the whole wave) in every lane
-__device__ __forceinline__ int64_t wave_read_lane(int64_t v, int src)
-{
-  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(v)), src));
-  const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), src));
-  return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
-}
-
 __global__ void __launch_bounds__(kThreads)
   scan_kernel(HistView hist, const I64Pair* node_sums, int F, const int32_t* row_pointers,
               int node_begin, int n_nodes)
@@ -507,25 +436,6 @@ __global__ void __launch_bounds__(kThreads)
 // ---------------------------------------------------------------------------
 // split evaluation (build_tree.cu:682-782)
 // ---------------------------------------------------------------------------
-
-struct Cand {
-  double gain;
-  int bin;
-};
-
-// Total order equivalent to the reference's 512 strided threads followed by a
-// rank-ordered reduction with op(a,b) = a.gain > b.gain ? a : b: larger gain
-// wins; among equal gains the larger (bin mod 512); inside one residue class
-// the smaller bin. Only bins with gain > 0 are candidates.
-__device__ inline bool cand_better(const Cand& a, const Cand& b)
-{
-  if (a.bin < 0) return false;
-  if (b.bin < 0) return true;
-  if (a.gain != b.gain) return a.gain > b.gain;
-  int ra = a.bin & 511, rb = b.bin & 511;
-  if (ra != rb) return ra > rb;
-  return a.bin < b.bin;
-}
 
 constexpr int kSplitChunk = 2048;  // bins per workgroup
 
@@ -601,23 +511,6 @@ __global__ void __launch_bounds__(kThreads)
 // :613) the bins of that output stay as they are in memory, for the node and for its sibling,
 // and the gains are formed from those values, as the reference's split kernel would read them.
 constexpr int kFusedMaxK   = 64;  // lane k of the wave keeps the running sums of output k
-
-__device__ inline void add_gain(double& gain, bool& dead, const I64Pair& ls, const I64Pair& ns, double inv_g,
-                                double inv_h, double l1, double reg, double min_split_gain)
-{
-  const int64_t rg = ns.grad - ls.grad, rh = ns.hess - ls.hess;
-  if (dead) return;
-  if (ls.hess <= 0 || rh <= 0) {
-    // build_tree.cu:727-730: one output without a valid split on this bin voids the bin
-    dead = true;
-    gain = 0;
-    return;
-  }
-  gain += calculate_gain(static_cast<double>(ls.grad) * inv_g, static_cast<double>(ls.hess) * inv_h,
-                         static_cast<double>(rg) * inv_g, static_cast<double>(rh) * inv_h,
-                         static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, l1, reg,
-                         min_split_gain);
-}
 
 __device__ inline Cand wave_best(Cand c)
 {
@@ -1440,6 +1333,7 @@ struct Layout {
   Cand* partial;
   I64Pair* hist;
   size_t hist_bytes;
+  SmallTreeState small;  // null pointers when the shape is not one for the few-rows builder
 };
 
 size_t hist_bytes_bound(int F, int K, int S, int max_depth, int64_t cache_bytes)
@@ -1526,6 +1420,28 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
   L.partial       = ar.take<Cand>(level_nodes * max_chunks);
   L.hist_bytes    = hist_bytes_bound(F, K, S, max_depth, cache_bytes);
   L.hist          = reinterpret_cast<I64Pair*>(ar.take<char>(L.hist_bytes));
+  L.small = SmallTreeState{};
+  if (small_tree_fits(N, F, K, max_depth, S)) {
+    SmallTreeState& st    = L.small;
+    st.pitch              = (N + 7) / 8 * 8;
+    const size_t per_row  = static_cast<size_t>(F) * st.pitch;
+    st.order[0]    = ar.take<uint16_t>(per_row);
+    st.order[1]    = ar.take<uint16_t>(per_row);
+    st.bins        = ar.take<uint16_t>(per_row);
+    st.proposals   = ar.take<double>(static_cast<size_t>(F) * S);
+    st.counts      = ar.take<int32_t>(F);
+    st.rp          = ar.take<int32_t>(F);
+    st.node_of_pos = ar.take<uint16_t>(st.pitch);
+    st.code        = ar.take<uint8_t>(N);
+    st.seg_start   = ar.take<int32_t>(max_nodes);
+    st.seg_count   = ar.take<int32_t>(max_nodes);
+    st.live        = ar.take<int32_t>(max_depth + 1);
+    st.base        = ar.take<I64Pair>(max_nodes * K);
+    st.node_sums   = L.node_sums;
+    st.qgh         = L.qgh;
+    st.scales      = L.scales;
+    st.cand        = ar.take<Cand>(level_nodes * F);
+  }
 }
 
 int validate(int64_t N, int F, int K, const lbt_build_params* p, int x_dtype)
@@ -1639,6 +1555,27 @@ int run_quantiser(hipStream_t stream, const double* g, const double* h, int64_t 
   }
   LBT_HIP(hipGetLastError());
   return LBT_OK;
+}
+
+// The nodes whose histograms the level loop below ends up with (GetHistogram, build_tree.cu:1191-1205).
+void final_histogram_range(int K, int B, const lbt_build_params& prm, int32_t* begin, int32_t* end)
+{
+  const uint64_t max_bytes = prm.hist_cache_bytes > 0 ? static_cast<uint64_t>(prm.hist_cache_bytes) : 1000000000ULL;
+  const int64_t nodes      = static_cast<int64_t>(std::max<uint64_t>(1, max_bytes / (static_cast<uint64_t>(K) * B * 16ULL)));
+  int cdepth = 0;
+  while (level_end(cdepth + 1) <= nodes && cdepth <= prm.max_depth) cdepth++;
+  const int64_t used_end = prm.max_depth > 0 ? level_end(prm.max_depth - 1) : 0;
+  const int64_t batch    = static_cast<int64_t>(static_cast<int>(nodes));
+  int64_t lo = 0, hi = level_end(cdepth);
+  for (int d = 0; d < prm.max_depth; d++) {
+    const int64_t in_level = int64_t(1) << d;
+    for (int64_t j0 = 0; j0 < in_level; j0 += batch) {
+      const int64_t b0 = level_begin(d) + j0, b1 = level_begin(d) + std::min(j0 + batch, in_level);
+      if (!(b0 >= lo && b1 <= hi)) lo = b0, hi = b1;
+    }
+  }
+  *begin = static_cast<int32_t>(lo);
+  *end   = static_cast<int32_t>(std::max<int64_t>(lo, std::min<int64_t>(hi, used_end)));
 }
 
 template <typename T>
@@ -2082,8 +2019,38 @@ static int build_tree_entry(void* stream, const void* X, int32_t x_dtype, int64_
     return LBT_ERR_WORKSPACE;
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int rc;
-  if (x_dtype == LBT_F32)
+  int rc        = LBT_OK;
+  bool done     = false;
+  // few rows: the builder that keeps no histograms, unless the caller wants to see what it does not have
+  const lbt_build_taps* t = taps;
+  const bool plain        = t == nullptr ||
+                     !(t->proposals || t->row_pointers || t->quantised || t->node_sums || t->positions ||
+                       t->positions_per_level || t->histogram || t->level_instances || t->level_built_instances ||
+                       t->level_built_nodes);
+  if (plain && L.small.order[0] != nullptr) {
+    int32_t* const row_leaf = taps ? taps->row_leaf : nullptr;
+    if (x_dtype == LBT_F32)
+      rc = lbt::small_tree_build<float>(s, L.small, static_cast<const float*>(X), row_offset, n_rows, n_features,
+                                        n_outputs, g, h, feature_set, *params, leaf, feature, split, gain, hessian,
+                                        row_leaf, taps ? &taps->n_bins : nullptr, &done);
+    else
+      rc = lbt::small_tree_build<double>(s, L.small, static_cast<const double*>(X), row_offset, n_rows, n_features,
+                                         n_outputs, g, h, feature_set, *params, leaf, feature, split, gain, hessian,
+                                         row_leaf, taps ? &taps->n_bins : nullptr, &done);
+    if (rc == LBT_OK && done) {
+      if (taps) {
+        lbt::final_histogram_range(n_outputs, taps->n_bins, *params, &taps->hist_node_begin, &taps->hist_node_end);
+        if (sync_at_end) LBT_HIP(hipMemcpyAsync(taps->scales, L.scales, sizeof(double) * 4, hipMemcpyDeviceToHost, s));
+      }
+      if (!sync_at_end) return LBT_OK;
+      LBT_HIP(hipStreamSynchronize(s));
+      LBT_HIP(hipGetLastError());
+      if (lbt::profiler().mode != 0) lbt::profiler().collect();
+      return LBT_OK;
+    }
+  }
+  if (rc != LBT_OK) {
+  } else if (x_dtype == LBT_F32)
     rc = lbt::build_tree_impl<float>(s, static_cast<const float*>(X), row_offset, n_rows, n_features, g, h, n_outputs,
                                      feature_set, *params, leaf, feature, split, gain, hessian, L, taps, sync_at_end);
   else

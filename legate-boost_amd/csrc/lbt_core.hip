@@ -143,6 +143,7 @@ int release_thread_resources()
   if (old.counts_here != nullptr) note(hipEventSynchronize(old.counts_here), "hipEventSynchronize");
   if (old.stats_here != nullptr) note(hipEventSynchronize(old.stats_here), "hipEventSynchronize");
   if (old.stage != nullptr) note(hipHostFree(old.stage), "hipHostFree");
+  if (old.answer != nullptr) note(hipHostFree(old.answer), "hipHostFree");
   if (old.mirror != nullptr) note(hipHostFree(old.mirror), "hipHostFree");
   if (old.stage_free != nullptr) note(hipEventDestroy(old.stage_free), "hipEventDestroy");
   if (old.counts_here != nullptr) note(hipEventDestroy(old.counts_here), "hipEventDestroy");
@@ -162,7 +163,7 @@ int thread_resources_here(ThreadResources** out)
   LBT_HIP(hipGetDevice(&device));
   ThreadResources& tr = thread_resources();
   const bool holds = tr.mirror != nullptr || tr.stage != nullptr || tr.counts_here != nullptr ||
-                     tr.stats_here != nullptr || tr.stage_free != nullptr;
+                     tr.stats_here != nullptr || tr.stage_free != nullptr || tr.answer != nullptr;
   if (holds && tr.device != device) {
     const int now = device;
     LBT_HIP(hipSetDevice(tr.device));

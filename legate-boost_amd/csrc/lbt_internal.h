@@ -142,6 +142,10 @@ struct ThreadResources {
   char* stage           = nullptr;
   size_t stage_bytes    = 0;
   hipEvent_t stage_free = nullptr;
+  // one pinned word in which a kernel of the few-rows builder reports to the host, and the tag of the
+  // last call that waited for it
+  uint32_t* answer    = nullptr;
+  uint32_t answer_tag = 0;
 };
 ThreadResources& thread_resources();
 // the same after making sure that what it holds belongs to the current device
@@ -447,5 +451,43 @@ int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, i
                  const void* X);
 // Plans tiles for the batch and launches the histogram kernel.
 int hist_launch(hipStream_t stream, const HistSetup& hs, const HistBatch& b, int depth);
+
+// ---------------------------------------------------------------- builder for few rows
+// (lbt_small_tree.hip)
+
+constexpr int kSmallMaxRows    = 8192;
+constexpr int kSmallMaxOutputs = 16;
+constexpr int kSmallMaxDepth   = 13;
+
+struct Cand;
+
+// Device buffers of a build, carved from the caller's workspace.
+struct SmallTreeState {
+  int64_t pitch;          // elements between the rows of a feature and those of the next (multiple of 8)
+  uint16_t* order[2];     // [F][pitch] rows by (node, bin); the order of level d is order[d & 1]
+  uint16_t* bins;         // [F][pitch] bin of every row
+  double* proposals;      // [F][S]
+  int32_t* counts;        // [F] proposals
+  int32_t* rp;            // [F] first bin of the feature among all bins
+  uint16_t* node_of_pos;  // [pitch] node of the level that holds a place of the order, 0xffff: a leaf's
+  uint8_t* code;          // [N] side a row of a split node takes: 1 left, 2 right
+  int32_t* seg_start;     // [max_nodes] places of a node's rows
+  int32_t* seg_count;     // [max_nodes]
+  int32_t* live;          // [max_depth + 1] the level has nodes
+  I64Pair* base;          // [max_nodes][K] sums of the rows in front of the node's places
+  I64Pair* node_sums;     // [max_nodes][K]
+  int2* qgh;              // [N][K]
+  double* scales;         // [4]
+  Cand* cand;             // [nodes of a level][F]
+};
+bool small_tree_fits(int64_t N, int F, int K, int max_depth, int S);
+// n_bins: receives the number of bins of all features (null: not wanted).
+// *taken: the tree has been queued; false (with LBT_OK): the data need the other builder, which has to
+// write every output again.
+template <typename T>
+int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, int64_t row_offset, int64_t N, int F,
+                     int K, const double* g, const double* h, const uint8_t* feature_set, const lbt_build_params& prm,
+                     double* leaf, int32_t* feature, double* split, double* gain, double* hessian, int32_t* row_leaf,
+                     int32_t* n_bins, bool* taken);
 
 }  // namespace lbt

@@ -1,0 +1,882 @@
+// BuildTreeTask for inputs of few rows: 1 + 2 * max_depth launches instead of about ten per level.
+//
+// The builder of lbt_build_tree.hip is made for rows by the million. With a few thousand of them its
+// launches do almost nothing (5 us each, about 90 for a tree of depth 8) and its histograms are
+// mostly empty: 128 nodes x 500 features x 256 bins for 5,000 rows. Here no histogram exists. Every
+// feature keeps the rows sorted by (node, bin of that feature); the running sums along that order
+// are the scanned histogram at its occupied bins (build_tree.cu:597-668), and a bin without rows
+// has the sums, and with them the gain, of the last occupied bin before it.
+//
+//   small_prologue_kernel   one workgroup per feature: split proposals (build_tree.cu:867-964), the bin of
+//                           every row, the rows sorted by bin; one workgroup: quantiser and root
+//                           (build_tree.cu:51-204, 1154-1187); the rest clear the outputs
+//   small_scan_kernel       one workgroup per feature and level: carries its order over to the level
+//                           (a stable partition inside every node), running sums, gains, and the best
+//                           split of the feature per node (build_tree.cu:682-740)
+//   small_apply_kernel      one workgroup per node and level: best feature, the node's outputs and its
+//                           children (build_tree.cu:740-782), the side of each of its rows
+//
+// The sums are integers, so they do not depend on the order of rows; gains and leaf values are formed
+// by the same functions from the same sums as in the other builder: the trees are identical. One rule of
+// the reference needs the histogram itself: a running sum that is positive in neither half leaves the bin
+// unscanned (build_tree.cu:645). That matters only if some row has a non-positive rounded hessian and a
+// pair other than (0, 0); the prologue reports such rows and the caller takes the other builder.
+#include <algorithm>
+#include <limits>
+
+#include "lbt_device.h"
+#include "lbt_internal.h"
+
+namespace lbt {
+namespace {
+
+constexpr int kPrologueThreads = 1024;
+constexpr int kNone            = 0xffff;  // node_of_pos of a row whose node did not split
+constexpr int kRankSortMax     = 512;     // split samples sorted by counting smaller ones; more: bitonic
+constexpr int kQuantChunks     = 8;       // chunks of 4096 entries the quantiser's workgroup takes
+
+// Inclusive sums over a wave, 32 bits (see wave_inclusive_sum)
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ int dpp_take32(int v)
+{
+  return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xf, true);
+}
+__device__ __forceinline__ int wave_inclusive_sum32(int v)
+{
+  v += dpp_take32<0x111, 0xf>(v);
+  v += dpp_take32<0x112, 0xf>(v);
+  v += dpp_take32<0x114, 0xf>(v);
+  v += dpp_take32<0x118, 0xf>(v);
+  v += dpp_take32<0x142, 0xa>(v);
+  v += dpp_take32<0x143, 0xc>(v);
+  return v;
+}
+
+// Sum of the threads before this one; all threads of the workgroup call it. s_wave: one int per wave.
+template <int kT>
+__device__ inline int block_exclusive_sum32(int v, int* s_wave)
+{
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int incl = wave_inclusive_sum32(v);
+  if (lane == 63) s_wave[wave] = incl;
+  __syncthreads();
+  int before = 0;
+  for (int w = 0; w < kT / 64; w++) before += w < wave ? s_wave[w] : 0;
+  return before + incl - v;
+}
+
+struct PrologueArgs {
+  int64_t row_offset;
+  int N, F, K, S;
+  int32_t seed;
+  int64_t dataset_rows;
+  const double* g;
+  const double* h;
+  const double* first_level;  // the quantiser's chunk sums if the caller has them, else null
+  double l1, l2;
+  int64_t max_nodes;
+  int max_depth;
+  double* leaf;
+  int32_t* feature;
+  double* split;
+  double* gain;
+  double* hessian;
+  uint32_t* answer;  // pinned host memory: what the host has to know, tagged with `tag`
+  uint32_t tag;
+};
+
+// Quantiser, root sums and root outputs: the arithmetic and the order of sums of abs_sum_level_kernel,
+// scales_kernel and quantise_kernel (lbt_build_tree.hip), for at most kQuantChunks chunks.
+__device__ inline void small_quantise(const PrologueArgs& a, const SmallTreeState& st, unsigned char* smem)
+{
+  double* s_a = reinterpret_cast<double*>(smem);           // [4][256]
+  double* s_b = s_a + 1024;                                 // [4][256]
+  double* s_chunk_a = s_b + 1024;                           // [kQuantChunks]
+  double* s_chunk_b = s_chunk_a + kQuantChunks;
+  double* s_scale   = s_chunk_b + kQuantChunks;             // [4]
+  unsigned long long* s_sum = reinterpret_cast<unsigned long long*>(s_scale + 4);  // [2 * K]
+  __shared__ unsigned s_flags;
+  const int n = a.N * a.K;
+  const int m = (n + 4095) / 4096;
+  const int quarter = threadIdx.x >> 8, t = threadIdx.x & 255;
+  if (threadIdx.x == 0) s_flags = 0;
+  for (int i = threadIdx.x; i < 2 * a.K; i += kPrologueThreads) s_sum[i] = 0;
+  if (threadIdx.x < kQuantChunks) s_chunk_a[threadIdx.x] = s_chunk_b[threadIdx.x] = 0.0;
+  __syncthreads();
+  if (a.first_level != nullptr) {
+    if (static_cast<int>(threadIdx.x) < m) {
+      s_chunk_a[threadIdx.x] = a.first_level[threadIdx.x];
+      s_chunk_b[threadIdx.x] = a.first_level[m + threadIdx.x];
+    }
+    __syncthreads();
+  } else {
+    // four chunks at a time, 256 threads each
+    for (int c0 = 0; c0 < m; c0 += 4) {
+      const int c = c0 + quarter;
+      double xa = 0.0, xb = 0.0;
+      for (int j = 0; j < 16; j++) {
+        const int e = c * 4096 + t + 256 * j;
+        if (e < n) {
+          xa += fabs(a.g[e]);
+          xb += fabs(a.h[e]);
+        }
+      }
+      s_a[quarter * 256 + t] = xa;
+      s_b[quarter * 256 + t] = xb;
+      __syncthreads();
+      for (int stride = 128; stride >= 1; stride >>= 1) {
+        if (t < stride) {
+          s_a[quarter * 256 + t] += s_a[quarter * 256 + t + stride];
+          s_b[quarter * 256 + t] += s_b[quarter * 256 + t + stride];
+        }
+        __syncthreads();
+      }
+      if (t == 0 && c < m) {
+        s_chunk_a[c] = s_a[quarter * 256];
+        s_chunk_b[c] = s_b[quarter * 256];
+      }
+      __syncthreads();
+    }
+  }
+  if (threadIdx.x == 0) {
+    // the second level's tree over at most kQuantChunks sums; the lanes past them add zeros
+    for (int stride = kQuantChunks / 2; stride >= 1 && m > 1; stride >>= 1)
+      for (int i = 0; i < stride; i++) {
+        s_chunk_a[i] += s_chunk_a[i + stride];
+        s_chunk_b[i] += s_chunk_b[i + stride];
+      }
+    const double max_int = 2147483647.0;
+    const double sg = s_chunk_a[0] == 0 ? 1 : max_int / s_chunk_a[0];
+    const double sh = s_chunk_b[0] == 0 ? 1 : max_int / s_chunk_b[0];
+    s_scale[0] = sg;
+    s_scale[1] = sh;
+    s_scale[2] = 1.0 / sg;
+    s_scale[3] = 1.0 / sh;
+  }
+  __syncthreads();
+  const double sg = s_scale[0], sh = s_scale[1];
+  int64_t sum_g = 0, sum_h = 0;  // single output
+  unsigned flags = 0;
+  for (int e = threadIdx.x; e < n; e += kPrologueThreads) {
+    const int row = a.K == 1 ? e : e / a.K, k = a.K == 1 ? 0 : e - row * a.K;
+    const double grad = a.g[e], hess = a.h[e];
+    uint32_t x = minstd_seed(static_cast<uint32_t>(
+      static_cast<uint64_t>(gpair_seed(static_cast<int64_t>(a.seed), row + a.row_offset, static_cast<int64_t>(k)))));
+    const double scaled_grad    = grad * sg;
+    const double scaled_hess    = hess * sh;
+    const double grad_remainder = scaled_grad - floor(scaled_grad);
+    const double hess_remainder = scaled_hess - floor(scaled_hess);
+    x = minstd_next(x);
+    const int64_t qg = static_cast<int64_t>(floor(scaled_grad) + static_cast<double>(uniform01(x) < grad_remainder));
+    x = minstd_next(x);
+    const int64_t qh = static_cast<int64_t>(floor(scaled_hess) + static_cast<double>(uniform01(x) < hess_remainder));
+    if (qg > 2147483647LL || qg < -2147483647LL || qh > 2147483647LL || qh < -2147483647LL) flags |= 2u;
+    if (qh <= 0 && (qg != 0 || qh != 0)) flags |= 1u;
+    st.qgh[e] = make_int2(static_cast<int>(qg), static_cast<int>(qh));
+    if (a.K == 1) {
+      sum_g += qg;
+      sum_h += qh;
+    } else {
+      atomicAdd(&s_sum[k], static_cast<unsigned long long>(qg));
+      atomicAdd(&s_sum[a.K + k], static_cast<unsigned long long>(qh));
+    }
+  }
+  if (a.K == 1) {
+    sum_g = wave_inclusive_sum(sum_g);
+    sum_h = wave_inclusive_sum(sum_h);
+    if ((threadIdx.x & 63) == 63) {
+      atomicAdd(&s_sum[0], static_cast<unsigned long long>(sum_g));
+      atomicAdd(&s_sum[1], static_cast<unsigned long long>(sum_h));
+    }
+  }
+  if (flags != 0) atomicOr(&s_flags, flags);
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(a.answer, (a.tag << 2) | s_flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (threadIdx.x < 4) st.scales[threadIdx.x] = s_scale[threadIdx.x];
+  for (int k = threadIdx.x; k < a.K; k += kPrologueThreads) {
+    const I64Pair ns{static_cast<int64_t>(s_sum[k]), static_cast<int64_t>(s_sum[a.K + k])};
+    st.node_sums[k] = ns;
+    st.base[k]      = I64Pair{0, 0};
+    a.leaf[k]       = calculate_leaf_value(static_cast<double>(ns.grad) * s_scale[2],
+                                           static_cast<double>(ns.hess) * s_scale[3], a.l1, a.l2);
+    a.hessian[k]    = static_cast<double>(ns.hess) * s_scale[3];
+  }
+  if (threadIdx.x == 0) {
+    a.feature[0]    = -1;
+    a.split[0]      = 0.0;
+    a.gain[0]       = 0.0;
+    st.seg_start[0] = 0;
+    st.seg_count[0] = a.N;
+    st.live[0]      = 1;
+  }
+}
+
+// Proposals, bins and the order of one feature.
+template <typename T>
+__device__ inline void small_feature(const T* __restrict__ X, const PrologueArgs& a, const SmallTreeState& st, int f,
+                                     unsigned char* smem)
+{
+  using Key = typename KeyOf<T>::type;
+  int P = 1;
+  while (P < a.S) P <<= 1;
+  // [P] unsorted keys, [P] sorted keys, [P] ranks, then bin counts / places
+  Key* s_in      = reinterpret_cast<Key*>(smem);
+  Key* s_key     = s_in + P;
+  int* s_rank    = reinterpret_cast<int*>(s_key + P);
+  int* s_count   = s_rank + P;                                       // [P + 1]
+  uint16_t* s_order = reinterpret_cast<uint16_t*>(s_count + P + 4);  // [N]
+  __shared__ int s_wave[kPrologueThreads / 64];
+  __shared__ int s_n;
+  const int tid = threadIdx.x;
+  // the sampled rows (build_tree.cu:882-898)
+  for (int i = tid; i < P; i += kPrologueThreads) {
+    Key key = ~Key(0);
+    if (i < a.S) {
+      uint32_t x = minstd_seed(static_cast<uint32_t>(a.seed));
+      x          = minstd_next(minstd_discard(x, static_cast<uint64_t>(i)));
+      const double u    = uniform01(x);
+      const double b    = static_cast<double>(a.dataset_rows - 1) + 1.0;
+      const int64_t row = static_cast<int64_t>((u * (b - 0.0)) + 0.0) - a.row_offset;
+      key               = to_key(row >= 0 && row < a.N ? X[row * a.F + f] : T(0));
+    }
+    s_in[i]   = key;
+    s_rank[i] = 0;
+  }
+  __syncthreads();
+  if (P <= kRankSortMax) {
+    // a sample's place is the number of samples before it; several threads share the counting
+    const int parts = kPrologueThreads / P, i = tid & (P - 1), part = tid / P;
+    const int per = (a.S + parts - 1) / parts, j0 = part * per, j1 = min(a.S, j0 + per);
+    if (i < a.S) {
+      const Key mine = s_in[i];
+      int before     = 0;
+      for (int j = j0; j < j1; j++) {
+        const Key o = s_in[j];
+        before += (o < mine || (o == mine && j < i)) ? 1 : 0;
+      }
+      atomicAdd(&s_rank[i], before);
+    }
+    __syncthreads();
+    for (int j = tid; j < a.S; j += kPrologueThreads) s_key[s_rank[j]] = s_in[j];
+    __syncthreads();
+  } else {
+    for (int i = tid; i < P; i += kPrologueThreads) s_key[i] = s_in[i];
+    __syncthreads();
+    for (int size = 2; size <= P; size <<= 1)
+      for (int stride = size >> 1; stride > 0; stride >>= 1) {
+        for (int i = tid; i < P / 2; i += kPrologueThreads) {
+          const int lo = 2 * i - (i & (stride - 1)), hi = lo + stride;
+          const bool up = (lo & size) == 0;
+          const Key x = s_key[lo], y = s_key[hi];
+          if ((x > y) == up) {
+            s_key[lo] = y;
+            s_key[hi] = x;
+          }
+        }
+        __syncthreads();
+      }
+  }
+  // drop values equal to their predecessor; two consecutive samples per thread (S <= 2048)
+  T* s_prop = reinterpret_cast<T*>(s_in);
+  T v[2]    = {T(0), T(0)};
+  bool keep[2];
+  int mine = 0;
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int i = 2 * tid + u;
+    keep[u]     = false;
+    if (i < a.S) {
+      v[u]    = from_key(s_key[i]);
+      keep[u] = i == 0 || !(v[u] == from_key(s_key[i - 1]));
+    }
+    mine += keep[u] ? 1 : 0;
+  }
+  int at = block_exclusive_sum32<kPrologueThreads>(mine, s_wave);
+  if (tid == kPrologueThreads - 1) s_n = at + mine;
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+    if (keep[u]) s_prop[at++] = v[u];
+  for (int i = tid; i <= P; i += kPrologueThreads) s_count[i] = 0;
+  __syncthreads();
+  const int n = s_n;
+  // the last proposal becomes +inf (build_tree.cu:953-956)
+  for (int i = tid; i < n; i += kPrologueThreads)
+    st.proposals[static_cast<int64_t>(f) * a.S + i] =
+      i == n - 1 ? std::numeric_limits<double>::infinity() : static_cast<double>(s_prop[i]);
+  if (tid == 0) st.counts[f] = n;
+  // bins: the number of proposals below the value, the last one never being below
+  uint16_t* bins = st.bins + static_cast<int64_t>(f) * st.pitch;
+  int my_bin[kSmallMaxRows / kPrologueThreads];
+#pragma unroll
+  for (int u = 0; u < kSmallMaxRows / kPrologueThreads; u++) {
+    const int r = tid + u * kPrologueThreads;
+    my_bin[u]   = -1;
+    if (r < a.N) {
+      const T x = X[static_cast<int64_t>(r) * a.F + f];
+      int lo = 0, len = n - 1;
+      while (len > 0) {
+        const int half = len >> 1;
+        const bool go  = s_prop[lo + half] < x;
+        lo             = go ? lo + half + 1 : lo;
+        len            = go ? len - half - 1 : half;
+      }
+      my_bin[u] = lo;
+      bins[r]   = static_cast<uint16_t>(lo);
+      atomicAdd(&s_count[lo], 1);
+    }
+  }
+  __syncthreads();
+  // counting sort of the rows by bin; which of a bin's rows comes first does not matter
+  const int c0 = 2 * tid < n ? s_count[2 * tid] : 0, c1 = 2 * tid + 1 < n ? s_count[2 * tid + 1] : 0;
+  const int place = block_exclusive_sum32<kPrologueThreads>(c0 + c1, s_wave);
+  if (2 * tid < n) s_count[2 * tid] = place;
+  if (2 * tid + 1 < n) s_count[2 * tid + 1] = place + c0;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kSmallMaxRows / kPrologueThreads; u++)
+    if (my_bin[u] >= 0) s_order[atomicAdd(&s_count[my_bin[u]], 1)] = static_cast<uint16_t>(tid + u * kPrologueThreads);
+  __syncthreads();
+  uint16_t* order = st.order[0] + static_cast<int64_t>(f) * st.pitch;
+  for (int i = tid; i < a.N; i += kPrologueThreads) order[i] = s_order[i];
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kPrologueThreads)
+  small_prologue_kernel(const T* __restrict__ X, PrologueArgs a, SmallTreeState st)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int block = blockIdx.x;
+  if (block == 0) {
+    small_quantise(a, st, smem_raw);
+    return;
+  }
+  if (block <= a.F) {
+    small_feature<T>(X, a, st, block - 1, smem_raw);
+    return;
+  }
+  // the outputs of every node but the root, and what the levels count on being zero
+  const int64_t stride = static_cast<int64_t>(gridDim.x - 1 - a.F) * kPrologueThreads;
+  const int64_t first  = static_cast<int64_t>(block - 1 - a.F) * kPrologueThreads + threadIdx.x;
+  for (int64_t i = first; i < a.max_nodes * a.K; i += stride)
+    if (i >= a.K) {
+      a.leaf[i]    = 0.0;
+      a.hessian[i] = 0.0;
+    }
+  for (int64_t i = first; i < a.max_nodes; i += stride)
+    if (i >= 1) {
+      a.feature[i]    = -1;
+      a.split[i]      = 0.0;
+      a.gain[i]       = 0.0;
+      st.seg_count[i] = 0;
+    }
+  for (int64_t i = first; i < a.N; i += stride) st.node_of_pos[i] = 0;
+  if (first >= 1 && first <= a.max_depth) st.live[first] = 0;
+}
+
+struct LevelArgs {
+  int N, F, K, S;
+  int depth;
+  int level_first;  // first node of the level; its node j is level_first + j
+  int n_nodes;
+  bool last;        // no further level follows
+  unsigned long long* n_bins;  // pinned host memory: the number of all bins, tagged like PrologueArgs::answer
+  uint32_t tag;
+  const uint8_t* feature_set;
+  double l1, l2, min_split_gain;
+};
+
+// Consecutive 16-bit values of one thread, kE of them from an address aligned to their size.
+template <int kE>
+__device__ __forceinline__ void load_u16(const uint16_t* p, int (&out)[kE])
+{
+  static_assert(kE == 4 || kE == 8, "8 or 16 bytes per thread");
+  uint32_t w[kE / 2];
+  if constexpr (kE == 4) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    w[0] = v.x, w[1] = v.y;
+  } else {
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
+    w[0] = v.x, w[1] = v.y, w[2] = v.z, w[3] = v.w;
+  }
+#pragma unroll
+  for (int i = 0; i < kE / 2; i++) {
+    out[2 * i]     = w[i] & 0xffff;
+    out[2 * i + 1] = w[i] >> 16;
+  }
+}
+
+// kT threads take kE consecutive places of the order each (kT * kE >= N).
+template <int kT, int kE>
+__global__ void __launch_bounds__(kT)
+  small_scan_kernel(SmallTreeState st, LevelArgs a)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  unsigned long long* s_gain = reinterpret_cast<unsigned long long*>(smem_raw);  // [n_nodes] bits of the best gain
+  unsigned* s_key            = reinterpret_cast<unsigned*>(s_gain + a.n_nodes);  // [n_nodes] its place in the order of ties
+  int* s_left_before         = reinterpret_cast<int*>(s_key + a.n_nodes);        // [n_nodes / 2 + 1]
+  uint16_t* s_order          = reinterpret_cast<uint16_t*>(s_left_before + a.n_nodes / 2 + 1);  // [kT * kE + 1]
+  __shared__ I64Pair s_pair[2][kT / 64];
+  __shared__ int s_wave[kT / 64];
+  __shared__ int s_rp;
+  if (st.live[a.depth] == 0) return;
+  const int f = blockIdx.x, tid = threadIdx.x;
+  const int wave = tid >> 6, lane = tid & 63;
+  // first bin of the feature among all bins
+  int rp = 0;
+  if (a.depth == 0) {
+    int mine = 0;
+    for (int i = tid; i < f; i += kT) mine += st.counts[i];
+    const int excl = block_exclusive_sum32<kT>(mine, s_wave);
+    if (tid == kT - 1) {
+      s_rp = st.rp[f] = excl + mine;
+      if (f == a.F - 1)
+        __hip_atomic_store(a.n_bins, (static_cast<unsigned long long>(a.tag) << 32) | static_cast<unsigned>(s_rp + st.counts[f]),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __syncthreads();
+    rp = s_rp;
+  } else {
+    rp = st.rp[f];
+  }
+  const bool usable = a.feature_set == nullptr || a.feature_set[f] != 0;
+  Cand* const out   = st.cand + f;  // node j: out[j * F]
+  if (!usable) {
+    for (int j = tid; j < a.n_nodes; j += kT) out[static_cast<int64_t>(j) * a.F] = Cand{0.0, -1};
+    if (f != 0) return;  // small_apply_kernel walks the rows in feature 0's order
+  }
+  for (int j = tid; j < a.n_nodes; j += kT) {
+    s_gain[j] = 0;
+    s_key[j]  = 0;
+  }
+  const int i0 = tid * kE;
+  int row[kE], node[kE];
+  const uint16_t* order_in = st.order[a.depth == 0 ? 0 : (a.depth - 1) & 1] + static_cast<int64_t>(f) * st.pitch;
+  if (i0 < a.N) {
+    load_u16<kE>(order_in + i0, row);
+    load_u16<kE>(st.node_of_pos + i0, node);
+  }
+#pragma unroll
+  for (int e = 0; e < kE; e++)
+    if (i0 + e >= a.N) {
+      row[e]  = 0;
+      node[e] = kNone;
+    }
+  if (a.depth > 0) {
+    // node[] already is the node of this level at the place: both children of a parent lie where the
+    // parent's rows lay, the left one first
+    unsigned left = 0;
+    int start[kE];
+#pragma unroll
+    for (int e = 0; e < kE; e++) {
+      start[e] = -1;
+      if (node[e] != kNone) {
+        left |= st.code[row[e]] == 1 ? 1u << e : 0u;
+        start[e] = st.seg_start[a.level_first + (node[e] & ~1)];
+      }
+    }
+    const int before = block_exclusive_sum32<kT>(__popc(left), s_wave);
+#pragma unroll
+    for (int e = 0; e < kE; e++)
+      if (start[e] == i0 + e) s_left_before[node[e] >> 1] = before + __popc(left & ((1u << e) - 1u));
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kE; e++) {
+      const int i = i0 + e;
+      if (i < a.N) {
+        int to = i;
+        if (node[e] != kNone) {
+          const int l = before + __popc(left & ((1u << e) - 1u)) - s_left_before[node[e] >> 1];
+          to = (left >> e) & 1u ? start[e] + l
+                                : start[e] + st.seg_count[a.level_first + (node[e] & ~1)] + (i - start[e] - l);
+        }
+        s_order[to] = static_cast<uint16_t>(row[e]);
+      }
+    }
+    __syncthreads();
+    uint16_t* order_out = st.order[a.depth & 1] + static_cast<int64_t>(f) * st.pitch;
+#pragma unroll
+    for (int e = 0; e < kE; e++)
+      if (i0 + e < a.N) {
+        row[e]           = s_order[i0 + e];
+        order_out[i0 + e] = static_cast<uint16_t>(row[e]);
+      }
+  } else {
+    // the neighbour's first row is looked up below
+#pragma unroll
+    for (int e = 0; e < kE; e++)
+      if (i0 + e < a.N) s_order[i0 + e] = static_cast<uint16_t>(row[e]);
+    __syncthreads();
+  }
+  if (!usable) return;
+
+  // occupied bins: the places that are the last of their (node, bin)
+  const uint16_t* bins = st.bins + static_cast<int64_t>(f) * st.pitch;
+  int bin[kE + 1], node_next = kNone;
+#pragma unroll
+  for (int e = 0; e < kE; e++) bin[e] = i0 + e < a.N ? bins[row[e]] : 0;
+  bin[kE] = 0;
+  if (i0 + kE < a.N) {
+    bin[kE]   = bins[s_order[i0 + kE]];
+    node_next = st.node_of_pos[i0 + kE];
+  }
+  unsigned ends = 0;
+#pragma unroll
+  for (int e = 0; e < kE; e++) {
+    const int nn = e + 1 < kE ? node[e + 1] : node_next;
+    // (the last rows of a node leave nothing on the right: never a split)
+    if (node[e] != kNone && nn == node[e] && bin[e + 1] != bin[e]) ends |= 1u << e;
+  }
+  const double inv_g = st.scales[2], inv_h = st.scales[3];
+  const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
+  double gain[kE];
+  unsigned dead = 0;
+#pragma unroll
+  for (int e = 0; e < kE; e++) gain[e] = 0.0;
+  for (int k = 0; k < a.K; k++) {
+    I64Pair q[kE];
+    I64Pair sum{0, 0};
+#pragma unroll
+    for (int e = 0; e < kE; e++) {
+      if (i0 + e < a.N) {
+        const int2 v = st.qgh[row[e] * a.K + k];
+        sum.grad += v.x;
+        sum.hess += v.y;
+      }
+      q[e] = sum;
+    }
+    const int64_t ig = wave_inclusive_sum(sum.grad), ih = wave_inclusive_sum(sum.hess);
+    I64Pair* const s_tot = s_pair[k & 1];
+    if (lane == 63) s_tot[wave] = I64Pair{ig, ih};
+    __syncthreads();
+    I64Pair before{ig - sum.grad, ih - sum.hess};
+    for (int w = 0; w < kT / 64; w++) {
+      before.grad += w < wave ? s_tot[w].grad : 0;
+      before.hess += w < wave ? s_tot[w].hess : 0;
+    }
+#pragma unroll
+    for (int e = 0; e < kE; e++)
+      if ((ends >> e) & 1u) {
+        const int64_t at = static_cast<int64_t>(a.level_first + node[e]) * a.K + k;
+        const I64Pair ns = st.node_sums[at], base = st.base[at];
+        const I64Pair ls{before.grad + q[e].grad - base.grad, before.hess + q[e].hess - base.hess};
+        bool d = (dead >> e) & 1u;
+        add_gain(gain[e], d, ls, ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
+        dead |= d ? 1u << e : 0u;
+      }
+  }
+  // best gain per node: a thread's runs of one node first, then, where a whole wave lies in one
+  // node, the wave
+  {
+    int run_node = kNone, runs = 0;
+    double run_gain = 0.0;
+#pragma unroll
+    for (int e = 0; e < kE; e++) {
+      const bool has = ((ends >> e) & 1u) != 0 && gain[e] > 0;
+      if (has) {
+        if (node[e] != run_node) {
+          if (runs > 0) atomicMax(&s_gain[run_node], static_cast<unsigned long long>(__double_as_longlong(run_gain)));
+          run_node = node[e];
+          run_gain = gain[e];
+          runs++;
+        } else {
+          run_gain = gain[e] > run_gain ? gain[e] : run_gain;
+        }
+      }
+    }
+    const unsigned long long have = __ballot(runs > 0);
+    if (have != 0) {
+      const int first_lane = __ffsll(have) - 1;
+      const int wave_node  = __shfl(run_node, first_lane, 64);
+      if (__all(runs == 0 || run_node == wave_node)) {
+        for (int off = 32; off >= 1; off >>= 1) {
+          const double o = __shfl_xor(run_gain, off, 64);
+          run_gain       = o > run_gain ? o : run_gain;
+        }
+        if (lane == 0) atomicMax(&s_gain[wave_node], static_cast<unsigned long long>(__double_as_longlong(run_gain)));
+      } else if (runs > 0) {
+        atomicMax(&s_gain[run_node], static_cast<unsigned long long>(__double_as_longlong(run_gain)));
+      }
+    }
+  }
+  __syncthreads();
+  // among the places with that gain, and the empty bins behind each of them, the reference's choice
+  // (cand_better): the largest bin mod 512 among all bins, then the smallest bin
+#pragma unroll
+  for (int e = 0; e < kE; e++) {
+    if (((ends >> e) & 1u) != 0 && gain[e] > 0 &&
+        static_cast<unsigned long long>(__double_as_longlong(gain[e])) == s_gain[node[e]]) {
+      // bins [first, last] share the gain; one of them is 511 mod 512, or the residues ascend
+      const int first = rp + bin[e], last = rp + bin[e + 1] - 1;
+      const int pick  = min(first | 511, last);
+      atomicMax(&s_key[node[e]], (static_cast<unsigned>(pick & 511) << 11 | static_cast<unsigned>(2047 - (pick - rp))) + 1u);
+    }
+  }
+  __syncthreads();
+  for (int j = tid; j < a.n_nodes; j += kT) {
+    if (st.seg_count[a.level_first + j] == 0) continue;
+    const unsigned key = s_key[j];
+    Cand c{0.0, -1};
+    if (key != 0) {
+      c.gain = __longlong_as_double(static_cast<long long>(s_gain[j]));
+      c.bin  = rp + 2047 - static_cast<int>((key - 1u) & 2047u);
+    }
+    out[static_cast<int64_t>(j) * a.F] = c;
+  }
+}
+
+// Split of one node, its outputs, its children and the side of each of its rows.
+template <int kT>
+__global__ void __launch_bounds__(kT)
+  small_apply_kernel(SmallTreeState st, LevelArgs a, double* leaf, int32_t* feature, double* split, double* gain,
+                     double* hessian, int32_t* row_leaf)
+{
+  __shared__ Cand s_cand[kT / 64];
+  __shared__ int s_feature[kT / 64];
+  __shared__ int s_cnt[kT / 64];
+  __shared__ I64Pair s_sum[2][kT / 64];
+  if (st.live[a.depth] == 0) return;
+  const int j    = blockIdx.x;
+  const int node = a.level_first + j;
+  const int n    = st.seg_count[node];
+  if (n == 0) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int s0 = st.seg_start[node];
+  const uint16_t* order = st.order[a.depth & 1];  // feature 0's
+  Cand best{0.0, -1};
+  int ft = -1;
+  if (st.node_sums[static_cast<int64_t>(node) * a.K].hess > 0) {
+    const Cand* c = st.cand + static_cast<int64_t>(j) * a.F;
+    for (int i = tid; i < a.F; i += kT)
+      if (cand_better(c[i], best)) {
+        best = c[i];
+        ft   = i;
+      }
+  }
+  for (int off = 32; off >= 1; off >>= 1) {
+    Cand o;
+    o.gain      = __shfl_xor(best.gain, off, 64);
+    o.bin       = __shfl_xor(best.bin, off, 64);
+    const int g = __shfl_xor(ft, off, 64);
+    if (cand_better(o, best)) {
+      best = o;
+      ft   = g;
+    }
+  }
+  if (lane == 0) {
+    s_cand[wave]    = best;
+    s_feature[wave] = ft;
+  }
+  __syncthreads();
+  for (int w = 0; w < kT / 64; w++)
+    if (cand_better(s_cand[w], best)) {
+      best = s_cand[w];
+      ft   = s_feature[w];
+    }
+  if (!(best.bin >= 0 && best.gain > 1e-5)) {
+    for (int i = s0 + tid; i < s0 + n; i += kT) {
+      st.node_of_pos[i] = kNone;
+      if (row_leaf != nullptr) row_leaf[order[i]] = node;
+    }
+    return;
+  }
+  const int lc = left_child(node), rc = right_child(node);
+  const int rel        = best.bin - st.rp[ft];
+  const uint16_t* bins = st.bins + static_cast<int64_t>(ft) * st.pitch;
+  int nl = 0;
+  I64Pair sum{0, 0};
+  for (int i = s0 + tid; i < s0 + n; i += kT) {
+    const int r     = order[i];
+    const bool left = bins[r] <= rel;
+    if (!a.last) st.code[r] = left ? 1 : 2;
+    if (a.last && row_leaf != nullptr) row_leaf[r] = left ? lc : rc;
+    if (left) {
+      const int2 q = st.qgh[r * a.K];
+      nl++;
+      sum.grad += q.x;
+      sum.hess += q.y;
+    }
+  }
+  const double inv_g = st.scales[2], inv_h = st.scales[3];
+  for (int k = 0;;) {
+    const int64_t ig = wave_inclusive_sum(sum.grad), ih = wave_inclusive_sum(sum.hess);
+    if (lane == 63) s_sum[k & 1][wave] = I64Pair{ig, ih};
+    if (k == 0) {
+      const int c = wave_inclusive_sum32(nl);
+      if (lane == 63) s_cnt[wave] = c;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      I64Pair ls{0, 0};
+      for (int w = 0; w < kT / 64; w++) {
+        ls.grad += s_sum[k & 1][w].grad;
+        ls.hess += s_sum[k & 1][w].hess;
+      }
+      const int64_t at = static_cast<int64_t>(node) * a.K + k, l = static_cast<int64_t>(lc) * a.K + k,
+                    r = static_cast<int64_t>(rc) * a.K + k;
+      const I64Pair ns = st.node_sums[at], base = st.base[at];
+      const I64Pair rs{ns.grad - ls.grad, ns.hess - ls.hess};
+      st.node_sums[l] = ls;
+      st.node_sums[r] = rs;
+      st.base[l]      = base;
+      st.base[r]      = I64Pair{base.grad + ls.grad, base.hess + ls.hess};
+      const double lg = static_cast<double>(ls.grad) * inv_g, lh = static_cast<double>(ls.hess) * inv_h;
+      const double rg = static_cast<double>(rs.grad) * inv_g, rh = static_cast<double>(rs.hess) * inv_h;
+      leaf[l]    = calculate_leaf_value(lg, lh, a.l1, a.l2);
+      leaf[r]    = calculate_leaf_value(rg, rh, a.l1, a.l2);
+      hessian[l] = lh;
+      hessian[r] = rh;
+    }
+    if (++k == a.K) break;
+    sum = I64Pair{0, 0};
+    for (int i = s0 + tid; i < s0 + n; i += kT) {
+      const int r = order[i];
+      if (bins[r] <= rel) {
+        const int2 q = st.qgh[r * a.K + k];
+        sum.grad += q.x;
+        sum.hess += q.y;
+      }
+    }
+  }
+  int lefts = 0;
+  for (int w = 0; w < kT / 64; w++) lefts += s_cnt[w];
+  if (tid == 0) {
+    feature[node] = ft;
+    split[node]   = st.proposals[static_cast<int64_t>(ft) * a.S + rel];
+    gain[node]    = best.gain;
+    st.seg_start[lc] = s0;
+    st.seg_count[lc] = lefts;
+    st.seg_start[rc] = s0 + lefts;
+    st.seg_count[rc] = n - lefts;
+    st.live[a.depth + 1] = 1;
+  }
+  if (!a.last)
+    for (int i = tid; i < n; i += kT) st.node_of_pos[s0 + i] = static_cast<uint16_t>(2 * j + (i < lefts ? 0 : 1));
+}
+
+template <int kT, int kE>
+int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a)
+{
+  static std::atomic<bool> attr_set[kMaxDevices] = {};
+  const size_t lds = static_cast<size_t>(a.n_nodes) * 12 + (a.n_nodes / 2 + 1) * 4 + (kT * kE + 8) * 2;
+  LBT_TRY(allow_dynamic_lds(small_scan_kernel<kT, kE>, 120 * 1024, attr_set));
+  small_scan_kernel<kT, kE><<<a.F, kT, lds, stream>>>(st, a);
+  return LBT_OK;
+}
+
+}  // namespace
+
+// By size: a row number has to fit 16 bits and a feature's order the registers of one workgroup; the
+// quantiser's workgroup takes kQuantChunks chunks; a level's nodes get a slot each in the LDS. At
+// 8192 rows a level takes about as long here as in the other builder's launches for it.
+bool small_tree_fits(int64_t N, int F, int K, int max_depth, int S)
+{
+  return N <= kSmallMaxRows && K <= kSmallMaxOutputs && N * K <= kQuantChunks * 4096 && max_depth >= 1 &&
+         max_depth <= kSmallMaxDepth && S <= LBT_MAX_SPLIT_SAMPLES && F <= 32768 &&
+         (static_cast<int64_t>(F) << (max_depth - 1)) <= (int64_t(1) << 22);
+}
+
+template <typename T>
+int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, int64_t row_offset, int64_t N, int F,
+                     int K, const double* g, const double* h, const uint8_t* feature_set, const lbt_build_params& prm,
+                     double* leaf, int32_t* feature, double* split, double* gain, double* hessian, int32_t* row_leaf,
+                     int32_t* n_bins, bool* taken)
+{
+  *taken = false;
+  ThreadResources* here = nullptr;
+  LBT_TRY(thread_resources_here(&here));
+  if (here->answer == nullptr) {
+    LBT_HIP(hipHostMalloc(reinterpret_cast<void**>(&here->answer), 64, hipHostMallocDefault));
+    here->answer[0] = here->answer[2] = here->answer[3] = 0;
+  }
+  const uint32_t tag = here->answer_tag = (here->answer_tag + 1) & 0x3fffffffu;
+  PrologueArgs pa;
+  pa.row_offset = row_offset;
+  pa.N = static_cast<int>(N); pa.F = F; pa.K = K; pa.S = prm.split_samples;
+  pa.seed         = prm.seed;
+  pa.dataset_rows = prm.dataset_rows;
+  pa.g = g; pa.h = h; pa.first_level = prm.abs_sum_chunks;
+  pa.l1 = prm.l1_regularization; pa.l2 = prm.l2_regularization;
+  pa.max_nodes = prm.max_nodes;
+  pa.max_depth = prm.max_depth;
+  pa.leaf = leaf; pa.feature = feature; pa.split = split; pa.gain = gain; pa.hessian = hessian;
+  pa.answer = here->answer;
+  pa.tag    = tag;
+  {
+    ProfScope ps(LBT_PROF_PROPOSALS, stream);
+    static std::atomic<bool> attr_set[kMaxDevices] = {};
+    LBT_TRY(allow_dynamic_lds(small_prologue_kernel<T>, 120 * 1024, attr_set));
+    int P = 1;
+    while (P < prm.split_samples) P <<= 1;
+    const size_t feature_lds = static_cast<size_t>(P) * (2 * sizeof(T) + 8) + 16 + N * 2 + 16;
+    const size_t quant_lds   = (2048 + 2 * kQuantChunks + 4 + 2 * static_cast<size_t>(K)) * 8;
+    const int64_t clear      = std::max<int64_t>(static_cast<int64_t>(prm.max_nodes) * K, N);
+    const int clearers       = static_cast<int>(std::min<int64_t>((clear + kPrologueThreads - 1) / kPrologueThreads, 64));
+    small_prologue_kernel<T><<<1 + F + clearers, kPrologueThreads, std::max(feature_lds, quant_lds), stream>>>(X, pa, st);
+  }
+  LevelArgs a;
+  a.N = static_cast<int>(N); a.F = F; a.K = K; a.S = prm.split_samples;
+  a.feature_set = feature_set;
+  a.n_bins = reinterpret_cast<unsigned long long*>(here->answer + 2);
+  a.tag    = tag;
+  a.l1 = prm.l1_regularization; a.l2 = prm.l2_regularization; a.min_split_gain = prm.min_split_gain;
+  for (int d = 0; d < prm.max_depth; d++) {
+    a.depth       = d;
+    a.level_first = static_cast<int>(level_begin(d));
+    a.n_nodes     = 1 << d;
+    a.last        = d + 1 == prm.max_depth;
+    {
+      ProfScope ps(LBT_PROF_HISTOGRAM, stream, 0.0, d);
+      if (N <= 1024)
+        LBT_TRY((launch_small_scan<256, 4>(stream, st, a)));
+      else if (N <= 2048)
+        LBT_TRY((launch_small_scan<512, 4>(stream, st, a)));
+      else if (N <= 4096)
+        LBT_TRY((launch_small_scan<1024, 4>(stream, st, a)));
+      else
+        LBT_TRY((launch_small_scan<1024, 8>(stream, st, a)));
+    }
+    ProfScope ps(LBT_PROF_SPLIT, stream);
+    // few nodes of many rows near the root, many small ones below
+    if ((N >> d) > 1024)
+      small_apply_kernel<1024><<<a.n_nodes, 1024, 0, stream>>>(st, a, leaf, feature, split, gain, hessian, row_leaf);
+    else if (d <= 8)
+      small_apply_kernel<256><<<a.n_nodes, 256, 0, stream>>>(st, a, leaf, feature, split, gain, hessian, row_leaf);
+    else
+      small_apply_kernel<64><<<a.n_nodes, 64, 0, stream>>>(st, a, leaf, feature, split, gain, hessian, row_leaf);
+  }
+  LBT_HIP(hipGetLastError());
+  // What the prologue found, and the number of bins if it is asked for, written to pinned memory long
+  // before the levels above are done. Should they not arrive (the stream has failed), the stream's
+  // own state ends the wait.
+  volatile uint32_t* const answer         = here->answer;
+  volatile unsigned long long* const bins = reinterpret_cast<unsigned long long*>(here->answer + 2);
+  auto arrived = [&]() { return (*answer >> 2) == tag && (n_bins == nullptr || (*bins >> 32) == tag); };
+  for (int64_t spin = 1; !arrived(); spin++) {
+    if (spin % 16384 != 0) continue;
+    const hipError_t e = hipStreamQuery(stream);
+    if (e == hipErrorNotReady) continue;
+    LBT_HIP(e);
+    if (arrived()) break;
+    set_error("the tree builder's kernels did not report");
+    return LBT_ERR_HIP;
+  }
+  const uint32_t got = *answer;
+  if (n_bins != nullptr) *n_bins = static_cast<int32_t>(*bins & 0xffffffffULL);
+  if ((got & 2u) != 0) {
+    set_error("a quantised gradient or hessian reaches 2^31 and does not fit the packed 32-bit form: one entry "
+              "holds the whole absolute sum and was rounded up");
+    return LBT_ERR_UNSUPPORTED;
+  }
+  *taken = (got & 1u) == 0;
+  return LBT_OK;
+}
+
+template int small_tree_build<float>(hipStream_t, const SmallTreeState&, const float*, int64_t, int64_t, int, int,
+                                     const double*, const double*, const uint8_t*, const lbt_build_params&, double*,
+                                     int32_t*, double*, double*, double*, int32_t*, int32_t*, bool*);
+template int small_tree_build<double>(hipStream_t, const SmallTreeState&, const double*, int64_t, int64_t, int, int,
+                                      const double*, const double*, const uint8_t*, const lbt_build_params&, double*,
+                                      int32_t*, double*, double*, double*, int32_t*, int32_t*, bool*);
+
+}  // namespace lbt

@@ -52,3 +52,102 @@ def test_cell_functions_of_the_bin_search(kinds, dtype, samples):
     g, h = rs.randn(n, 1), rs.rand(n, 1) + 0.5
     gr, cr = gu.both(X, g, h, levels=True, max_depth=4, split_samples=samples, seed=77, feature_set=usable)
     gu.assert_tree_parity(gr, cr, levels=True)
+
+
+def _assert_tree(got, cr):
+    import gpu_util as gu
+
+    assert np.array_equal(gu.cpu(got.feature), cr.feature)
+    for name in ("split_value", "gain", "leaf_value", "hessian"):
+        gu.assert_same_floats(gu.cpu(getattr(got, name)), getattr(cr, name), name)
+
+
+@pytest.mark.parametrize("n,f,k,depth,s,dtype", [
+    (1, 1, 1, 1, 1, np.float32),
+    (2, 1, 1, 13, 256, np.float64),
+    (63, 3, 1, 4, 7, np.float32),
+    (64, 2, 2, 5, 64, np.float64),
+    (1000, 10, 1, 8, 256, np.float64),
+    (1024, 5, 1, 6, 512, np.float32),      # one workgroup width of rows, and one more
+    (1025, 5, 3, 6, 513, np.float32),      # samples sorted by counting, and by the bitonic network
+    (2048, 70, 1, 9, 2048, np.float64),
+    (2049, 4, 16, 5, 256, np.float32),
+    (4095, 33, 1, 10, 100, np.float32),
+    (4097, 300, 1, 7, 256, np.float32),
+    (8191, 6, 4, 12, 1024, np.float64),
+    (8192, 9, 4, 8, 256, np.float32),      # the most rows and entries the few-rows builder takes
+    (8193, 9, 1, 8, 256, np.float32),
+    (8192, 3, 5, 4, 64, np.float32),       # more entries than it takes
+    (500, 4, 1, 14, 64, np.float32),       # deeper than it takes
+])
+def test_few_rows(n, f, k, depth, s, dtype):
+    """The builder for few rows at the edges of what it takes (and just past them), with constant and
+    two-valued columns, ties between features, a feature set, an offset and regularisation in turn."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + 7 * f + depth)
+    X = rs.randn(n, f).astype(dtype)
+    if f > 2:
+        X[:, 1] = rs.randint(0, 3, n)
+        X[:, 2] = X[:, 0]  # the same splits twice: the tie rule decides between features
+    if f > 4:
+        X[:, 3] = 1.25
+    g = rs.randn(n, k)
+    h = rs.rand(n, k) + 0.1
+    if n > 100:
+        h[n // 2:] = 0.0  # rows left out, as row subsampling leaves them
+        g[n // 2:] = 0.0
+    fs = None
+    if f > 5:
+        fs = rs.rand(f) < 0.7
+        fs[0] = False
+    opt = dict(l1_regularization=0.05, l2_regularization=0.5, min_split_gain=1e-3) if depth % 2 else {}
+    cr = orc.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=n, feature_set=fs, l1=opt.get("l1_regularization", 0.0),
+                        l2=opt.get("l2_regularization", 1.0), min_split_gain=opt.get("min_split_gain", 0.0))
+    for wait in (True, False):
+        got = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=n, feature_set=fs, row_leaf=True,
+                             wait=wait, **opt)
+        torch.cuda.synchronize()
+        _assert_tree(got, cr)
+        gu.check_row_leaf(got, X)
+
+
+@pytest.mark.parametrize("case", ["negative_hessian", "zero_hessian", "all_zero", "constant_target"])
+def test_few_rows_special_gradients(case):
+    """Rows whose rounded hessian is not positive need the reference's unscanned bins: such data take the other
+    builder, whatever the size."""
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(5)
+    n, f, k = 3000, 7, 2
+    X = rs.randn(n, f).astype(np.float32)
+    X[:, 0] = np.round(X[:, 0])
+    g, h = rs.randn(n, k), rs.rand(n, k) + 0.1
+    if case == "negative_hessian":
+        h[::5] *= -1.0
+    elif case == "zero_hessian":
+        h[::3] = 0.0
+    elif case == "all_zero":
+        g[:], h[:] = 0.0, 0.0
+    else:
+        g[:] = 1.0
+        h[:] = 1.0
+    cr = orc.build_tree(X, g, h, max_depth=6, split_samples=64, seed=3)
+    _assert_tree(ops.build_tree(X, g, h, max_depth=6, split_samples=64, seed=3), cr)
+
+
+def test_few_rows_takes_the_chunk_sums_of_the_gradient_pass():
+    from lbtree import ops
+
+    rs = np.random.RandomState(8)
+    n, k = 6000, 3
+    X = torch.from_numpy(rs.randn(n, 12).astype(np.float32)).cuda()
+    pred, y = torch.from_numpy(rs.randn(n, k)).cuda(), torch.from_numpy(rs.randn(n, k)).cuda()
+    g, h, sums = ops.weighted_gradient("squared_error", y, pred, None, 0.1, sums=True)
+    a = ops.build_tree(X, g, h, max_depth=5, split_samples=64, seed=4)
+    b = ops.build_tree(X, g, h, max_depth=5, split_samples=64, seed=4, abs_sum_chunks=sums)
+    for name in ("leaf_value", "feature", "split_value", "gain", "hessian"):
+        assert torch.equal(getattr(a, name), getattr(b, name)), name
