@@ -1425,22 +1425,21 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     SmallTreeState& st    = L.small;
     st.pitch              = (N + 7) / 8 * 8;
     const size_t per_row  = static_cast<size_t>(F) * st.pitch;
-    st.order[0]    = ar.take<uint16_t>(per_row);
-    st.order[1]    = ar.take<uint16_t>(per_row);
+    st.order[0]    = ar.take<uint32_t>(per_row);
+    st.order[1]    = ar.take<uint32_t>(per_row);
     st.bins        = ar.take<uint16_t>(per_row);
     st.proposals   = ar.take<double>(static_cast<size_t>(F) * S);
     st.counts      = ar.take<int32_t>(F);
     st.rp          = ar.take<int32_t>(F);
     st.node_of_pos = ar.take<uint16_t>(st.pitch);
-    st.code        = ar.take<uint8_t>(N);
-    st.seg_start   = ar.take<int32_t>(max_nodes);
-    st.seg_count   = ar.take<int32_t>(max_nodes);
+    st.code        = ar.take<uint8_t>(st.pitch);
+    st.seg         = ar.take<int2>(max_nodes);
     st.live        = ar.take<int32_t>(max_depth + 1);
     st.base        = ar.take<I64Pair>(max_nodes * K);
     st.node_sums   = L.node_sums;
     st.qgh         = L.qgh;
     st.scales      = L.scales;
-    st.cand        = ar.take<Cand>(level_nodes * F);
+    st.cand        = ar.take<SmallCand>(level_nodes * F);
   }
 }
 

@@ -459,26 +459,29 @@ constexpr int kSmallMaxRows    = 8192;
 constexpr int kSmallMaxOutputs = 16;
 constexpr int kSmallMaxDepth   = 13;
 
-struct Cand;
+struct SmallCand {
+  double gain;
+  uint32_t key;  // order among equal gains, larger wins; 0: no candidate
+  int32_t rel;   // bin of the feature
+};
 
 // Device buffers of a build, carved from the caller's workspace.
 struct SmallTreeState {
   int64_t pitch;          // elements between the rows of a feature and those of the next (multiple of 8)
-  uint16_t* order[2];     // [F][pitch] rows by (node, bin); the order of level d is order[d & 1]
+  uint32_t* order[2];     // [F][pitch] row | bin << 16 by (node, bin); the order of level d is order[d & 1]
   uint16_t* bins;         // [F][pitch] bin of every row
   double* proposals;      // [F][S]
   int32_t* counts;        // [F] proposals
   int32_t* rp;            // [F] first bin of the feature among all bins
   uint16_t* node_of_pos;  // [pitch] node of the level that holds a place of the order, 0xffff: a leaf's
   uint8_t* code;          // [N] side a row of a split node takes: 1 left, 2 right
-  int32_t* seg_start;     // [max_nodes] places of a node's rows
-  int32_t* seg_count;     // [max_nodes]
+  int2* seg;              // [max_nodes] places of a node's rows: the first one, and how many
   int32_t* live;          // [max_depth + 1] the level has nodes
   I64Pair* base;          // [max_nodes][K] sums of the rows in front of the node's places
   I64Pair* node_sums;     // [max_nodes][K]
   int2* qgh;              // [N][K]
   double* scales;         // [4]
-  Cand* cand;             // [nodes of a level][F]
+  SmallCand* cand;        // [nodes of a level][F]
 };
 bool small_tree_fits(int64_t N, int F, int K, int max_depth, int S);
 // n_bins: receives the number of bins of all features (null: not wanted).

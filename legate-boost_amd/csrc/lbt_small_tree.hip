@@ -206,8 +206,7 @@ __device__ inline void small_quantise(const PrologueArgs& a, const SmallTreeStat
     a.feature[0]    = -1;
     a.split[0]      = 0.0;
     a.gain[0]       = 0.0;
-    st.seg_start[0] = 0;
-    st.seg_count[0] = a.N;
+    st.seg[0]       = make_int2(0, a.N);
     st.live[0]      = 1;
   }
 }
@@ -225,7 +224,7 @@ __device__ inline void small_feature(const T* __restrict__ X, const PrologueArgs
   Key* s_key     = s_in + P;
   int* s_rank    = reinterpret_cast<int*>(s_key + P);
   int* s_count   = s_rank + P;                                       // [P + 1]
-  uint16_t* s_order = reinterpret_cast<uint16_t*>(s_count + P + 4);  // [N]
+  uint32_t* s_order = reinterpret_cast<uint32_t*>(s_count + P + 4);  // [N]
   __shared__ int s_wave[kPrologueThreads / 64];
   __shared__ int s_n;
   const int tid = threadIdx.x;
@@ -327,7 +326,7 @@ __device__ inline void small_feature(const T* __restrict__ X, const PrologueArgs
     }
   }
   __syncthreads();
-  // counting sort of the rows by bin; which of a bin's rows comes first does not matter
+  // counting sort of the rows by bin (an entry of the order is row | bin << 16); which of a bin's rows comes first does not matter
   const int c0 = 2 * tid < n ? s_count[2 * tid] : 0, c1 = 2 * tid + 1 < n ? s_count[2 * tid + 1] : 0;
   const int place = block_exclusive_sum32<kPrologueThreads>(c0 + c1, s_wave);
   if (2 * tid < n) s_count[2 * tid] = place;
@@ -335,9 +334,11 @@ __device__ inline void small_feature(const T* __restrict__ X, const PrologueArgs
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < kSmallMaxRows / kPrologueThreads; u++)
-    if (my_bin[u] >= 0) s_order[atomicAdd(&s_count[my_bin[u]], 1)] = static_cast<uint16_t>(tid + u * kPrologueThreads);
+    if (my_bin[u] >= 0)
+      s_order[atomicAdd(&s_count[my_bin[u]], 1)] = static_cast<uint32_t>(tid + u * kPrologueThreads) |
+                                                   (static_cast<uint32_t>(my_bin[u]) << 16);
   __syncthreads();
-  uint16_t* order = st.order[0] + static_cast<int64_t>(f) * st.pitch;
+  uint32_t* order = st.order[0] + static_cast<int64_t>(f) * st.pitch;
   for (int i = tid; i < a.N; i += kPrologueThreads) order[i] = s_order[i];
 }
 
@@ -368,7 +369,7 @@ __global__ void __launch_bounds__(kPrologueThreads)
       a.feature[i]    = -1;
       a.split[i]      = 0.0;
       a.gain[i]       = 0.0;
-      st.seg_count[i] = 0;
+      st.seg[i] = make_int2(0, 0);
     }
   for (int64_t i = first; i < a.N; i += stride) st.node_of_pos[i] = 0;
   if (first >= 1 && first <= a.max_depth) st.live[first] = 0;
@@ -386,7 +387,8 @@ struct LevelArgs {
   double l1, l2, min_split_gain;
 };
 
-// Consecutive 16-bit values of one thread, kE of them from an address aligned to their size.
+// Consecutive values of one thread, kE of them from an address aligned to 16 bytes (16-bit values: to
+// their size).
 template <int kE>
 __device__ __forceinline__ void load_u16(const uint16_t* p, int (&out)[kE])
 {
@@ -405,25 +407,77 @@ __device__ __forceinline__ void load_u16(const uint16_t* p, int (&out)[kE])
     out[2 * i + 1] = w[i] >> 16;
   }
 }
+template <int kE>
+__device__ __forceinline__ void load_u32(const uint32_t* p, uint32_t (&out)[kE])
+{
+#pragma unroll
+  for (int i = 0; i < kE / 4; i++) {
+    const uint4 v = reinterpret_cast<const uint4*>(p)[i];
+    out[4 * i] = v.x, out[4 * i + 1] = v.y, out[4 * i + 2] = v.z, out[4 * i + 3] = v.w;
+  }
+}
 
-// kT threads take kE consecutive places of the order each (kT * kE >= N).
-template <int kT, int kE>
+// Where a split falls among equal gains of a node (cand_better): the largest bin mod 512, counted over all
+// bins, then the smallest bin. Bins [bin, next) of the feature, of which only the first has rows, share a
+// gain; one of them is 511 mod 512, or their residues ascend. Larger keys win, none is 0.
+__device__ __forceinline__ unsigned tie_key(int rp, int bin, int next)
+{
+  const int pick = min((rp + bin) | 511, rp + next - 1);
+  return (static_cast<unsigned>(pick & 511) << 11 | static_cast<unsigned>(2047 - (pick - rp))) + 1u;
+}
+
+// The same rule between bins of different features (fewer than 2^26 bins: small_tree_fits).
+__device__ __forceinline__ unsigned tie_key_of_bin(int bin)
+{
+  return (static_cast<unsigned>(bin & 511) << 17 | static_cast<unsigned>(0x1ffff - (bin >> 9))) + 1u;
+}
+
+// kT threads take kE consecutive places of the order each (kT * kE >= N). What a place needs of its row
+// (its pair of the first output, its side) is staged in the LDS in row order: gathered from the L2 these
+// are three scattered accesses per place, and a workgroup's 8192 places then take a level 90 us
+// (5,000 rows x 500 features). Everything that does not depend on another load is asked for first: the
+// levels of a small tree are a chain of memory latencies.
+template <int kT, int kE, bool kSingle>
 __global__ void __launch_bounds__(kT)
   small_scan_kernel(SmallTreeState st, LevelArgs a)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  unsigned long long* s_gain = reinterpret_cast<unsigned long long*>(smem_raw);  // [n_nodes] bits of the best gain
+  int2* s_q                  = reinterpret_cast<int2*>(smem_raw);               // [N]
+  uint32_t* s_order          = reinterpret_cast<uint32_t*>(s_q + (a.N + 1) / 2 * 2);  // [kT * kE + 4]
+  unsigned long long* s_gain = reinterpret_cast<unsigned long long*>(s_order + kT * kE + 4);  // [n_nodes] bits of the best gain
   unsigned* s_key            = reinterpret_cast<unsigned*>(s_gain + a.n_nodes);  // [n_nodes] its place in the order of ties
   int* s_left_before         = reinterpret_cast<int*>(s_key + a.n_nodes);        // [n_nodes / 2 + 1]
-  uint16_t* s_order          = reinterpret_cast<uint16_t*>(s_left_before + a.n_nodes / 2 + 1);  // [kT * kE + 1]
+  uint8_t* s_code            = reinterpret_cast<uint8_t*>(s_left_before + a.n_nodes / 2 + 1);  // [N]
   __shared__ I64Pair s_pair[2][kT / 64];
   __shared__ int s_wave[kT / 64];
   __shared__ int s_rp;
-  if (st.live[a.depth] == 0) return;
   const int f = blockIdx.x, tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
-  // first bin of the feature among all bins
-  int rp = 0;
+  const int i0   = tid * kE;
+  const bool usable = a.feature_set == nullptr || a.feature_set[f] != 0;
+  SmallCand* const out = st.cand + f;  // node j: out[j * F]
+  const uint32_t* order_in = st.order[a.depth == 0 ? 0 : (a.depth - 1) & 1] + static_cast<int64_t>(f) * st.pitch;
+  uint32_t entry[kE];
+  int node[kE];
+#pragma unroll
+  for (int e = 0; e < kE; e++) {
+    entry[e] = 0;
+    node[e]  = kNone;
+  }
+  int node_next = kNone;
+  if (i0 < a.N) {
+    load_u32<kE>(order_in + i0, entry);
+    load_u16<kE>(st.node_of_pos + i0, node);
+    if (i0 + kE < a.N) node_next = st.node_of_pos[i0 + kE];
+  }
+  const int live = st.live[a.depth];
+  int rp         = a.depth == 0 ? 0 : st.rp[f];  // first bin of the feature among all bins
+  if (kSingle && usable)
+    for (int i = tid; i < a.N; i += kT) s_q[i] = st.qgh[i];
+  if (a.depth > 0)
+    for (int i = tid * 4; i < a.N; i += kT * 4)
+      *reinterpret_cast<uint32_t*>(s_code + i) = *reinterpret_cast<const uint32_t*>(st.code + i);
+  if (live == 0) return;
   if (a.depth == 0) {
     int mine = 0;
     for (int i = tid; i < f; i += kT) mine += st.counts[i];
@@ -436,49 +490,33 @@ __global__ void __launch_bounds__(kT)
     }
     __syncthreads();
     rp = s_rp;
-  } else {
-    rp = st.rp[f];
   }
-  const bool usable = a.feature_set == nullptr || a.feature_set[f] != 0;
-  Cand* const out   = st.cand + f;  // node j: out[j * F]
   if (!usable) {
-    for (int j = tid; j < a.n_nodes; j += kT) out[static_cast<int64_t>(j) * a.F] = Cand{0.0, -1};
+    for (int j = tid; j < a.n_nodes; j += kT) out[static_cast<int64_t>(j) * a.F] = SmallCand{0.0, 0u, 0};
     if (f != 0) return;  // small_apply_kernel walks the rows in feature 0's order
   }
   for (int j = tid; j < a.n_nodes; j += kT) {
     s_gain[j] = 0;
     s_key[j]  = 0;
   }
-  const int i0 = tid * kE;
-  int row[kE], node[kE];
-  const uint16_t* order_in = st.order[a.depth == 0 ? 0 : (a.depth - 1) & 1] + static_cast<int64_t>(f) * st.pitch;
-  if (i0 < a.N) {
-    load_u16<kE>(order_in + i0, row);
-    load_u16<kE>(st.node_of_pos + i0, node);
-  }
 #pragma unroll
   for (int e = 0; e < kE; e++)
-    if (i0 + e >= a.N) {
-      row[e]  = 0;
-      node[e] = kNone;
-    }
+    if (i0 + e >= a.N) node[e] = kNone;
   if (a.depth > 0) {
     // node[] already is the node of this level at the place: both children of a parent lie where the
     // parent's rows lay, the left one first
-    unsigned left = 0;
-    int start[kE];
+    int2 seg[kE];  // the left child's
 #pragma unroll
-    for (int e = 0; e < kE; e++) {
-      start[e] = -1;
-      if (node[e] != kNone) {
-        left |= st.code[row[e]] == 1 ? 1u << e : 0u;
-        start[e] = st.seg_start[a.level_first + (node[e] & ~1)];
-      }
-    }
+    for (int e = 0; e < kE; e++) seg[e] = node[e] != kNone ? st.seg[a.level_first + (node[e] & ~1)] : make_int2(-1, 0);
+    __syncthreads();
+    unsigned left = 0;
+#pragma unroll
+    for (int e = 0; e < kE; e++)
+      if (node[e] != kNone) left |= s_code[entry[e] & 0xffff] == 1 ? 1u << e : 0u;
     const int before = block_exclusive_sum32<kT>(__popc(left), s_wave);
 #pragma unroll
     for (int e = 0; e < kE; e++)
-      if (start[e] == i0 + e) s_left_before[node[e] >> 1] = before + __popc(left & ((1u << e) - 1u));
+      if (seg[e].x == i0 + e) s_left_before[node[e] >> 1] = before + __popc(left & ((1u << e) - 1u));
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < kE; e++) {
@@ -487,139 +525,233 @@ __global__ void __launch_bounds__(kT)
         int to = i;
         if (node[e] != kNone) {
           const int l = before + __popc(left & ((1u << e) - 1u)) - s_left_before[node[e] >> 1];
-          to = (left >> e) & 1u ? start[e] + l
-                                : start[e] + st.seg_count[a.level_first + (node[e] & ~1)] + (i - start[e] - l);
+          to = (left >> e) & 1u ? seg[e].x + l : i + seg[e].y - l;
         }
-        s_order[to] = static_cast<uint16_t>(row[e]);
+        s_order[to] = entry[e];
       }
     }
     __syncthreads();
-    uint16_t* order_out = st.order[a.depth & 1] + static_cast<int64_t>(f) * st.pitch;
+    uint32_t* order_out = st.order[a.depth & 1] + static_cast<int64_t>(f) * st.pitch;
+    if (i0 < a.N) {
 #pragma unroll
-    for (int e = 0; e < kE; e++)
-      if (i0 + e < a.N) {
-        row[e]           = s_order[i0 + e];
-        order_out[i0 + e] = static_cast<uint16_t>(row[e]);
+      for (int u = 0; u < kE / 4; u++) {
+        const uint4 v = reinterpret_cast<const uint4*>(s_order + i0)[u];
+        reinterpret_cast<uint4*>(order_out + i0)[u] = v;  // (entries past N are never looked at)
+        entry[4 * u] = v.x, entry[4 * u + 1] = v.y, entry[4 * u + 2] = v.z, entry[4 * u + 3] = v.w;
       }
+    }
   } else {
-    // the neighbour's first row is looked up below
-#pragma unroll
-    for (int e = 0; e < kE; e++)
-      if (i0 + e < a.N) s_order[i0 + e] = static_cast<uint16_t>(row[e]);
+    // the neighbour's first bin is looked up below
+    if (i0 < a.N) s_order[i0] = entry[0];
     __syncthreads();
   }
   if (!usable) return;
 
-  // occupied bins: the places that are the last of their (node, bin)
-  const uint16_t* bins = st.bins + static_cast<int64_t>(f) * st.pitch;
-  int bin[kE + 1], node_next = kNone;
+  // occupied bins: the places that are the last of their (node, bin); the last rows of a node leave
+  // nothing on the right: never a split
+  int bin[kE + 1];
 #pragma unroll
-  for (int e = 0; e < kE; e++) bin[e] = i0 + e < a.N ? bins[row[e]] : 0;
-  bin[kE] = 0;
-  if (i0 + kE < a.N) {
-    bin[kE]   = bins[s_order[i0 + kE]];
-    node_next = st.node_of_pos[i0 + kE];
-  }
+  for (int e = 0; e < kE; e++) bin[e] = static_cast<int>(entry[e] >> 16);
+  bin[kE] = i0 + kE < a.N ? static_cast<int>(s_order[i0 + kE] >> 16) : 0;
   unsigned ends = 0;
 #pragma unroll
   for (int e = 0; e < kE; e++) {
     const int nn = e + 1 < kE ? node[e + 1] : node_next;
-    // (the last rows of a node leave nothing on the right: never a split)
     if (node[e] != kNone && nn == node[e] && bin[e + 1] != bin[e]) ends |= 1u << e;
   }
   const double inv_g = st.scales[2], inv_h = st.scales[3];
   const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
-  double gain[kE];
-  unsigned dead = 0;
-#pragma unroll
-  for (int e = 0; e < kE; e++) gain[e] = 0.0;
-  for (int k = 0; k < a.K; k++) {
-    I64Pair q[kE];
+  if constexpr (kSingle) {
+    // A thread's places are consecutive, so its nodes come one after the other: the best split of a node
+    // that begins and ends inside the thread is final, those of its first and last node meet the
+    // other threads' in the LDS. Sums, parent's term and best split of the node at hand stay in registers.
     I64Pair sum{0, 0};
 #pragma unroll
-    for (int e = 0; e < kE; e++) {
+    for (int e = 0; e < kE; e++)
       if (i0 + e < a.N) {
-        const int2 v = st.qgh[row[e] * a.K + k];
+        const int2 v = s_q[entry[e] & 0xffff];
         sum.grad += v.x;
         sum.hess += v.y;
       }
-      q[e] = sum;
-    }
     const int64_t ig = wave_inclusive_sum(sum.grad), ih = wave_inclusive_sum(sum.hess);
-    I64Pair* const s_tot = s_pair[k & 1];
-    if (lane == 63) s_tot[wave] = I64Pair{ig, ih};
+    if (lane == 63) s_pair[0][wave] = I64Pair{ig, ih};
     __syncthreads();
-    I64Pair before{ig - sum.grad, ih - sum.hess};
+    I64Pair run{ig - sum.grad, ih - sum.hess};
     for (int w = 0; w < kT / 64; w++) {
-      before.grad += w < wave ? s_tot[w].grad : 0;
-      before.hess += w < wave ? s_tot[w].hess : 0;
+      run.grad += w < wave ? s_pair[0][w].grad : 0;
+      run.hess += w < wave ? s_pair[0][w].hess : 0;
     }
-#pragma unroll
-    for (int e = 0; e < kE; e++)
-      if ((ends >> e) & 1u) {
-        const int64_t at = static_cast<int64_t>(a.level_first + node[e]) * a.K + k;
-        const I64Pair ns = st.node_sums[at], base = st.base[at];
-        const I64Pair ls{before.grad + q[e].grad - base.grad, before.hess + q[e].hess - base.hess};
-        bool d = (dead >> e) & 1u;
-        add_gain(gain[e], d, ls, ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
-        dead |= d ? 1u << e : 0u;
-      }
-  }
-  // best gain per node: a thread's runs of one node first, then, where a whole wave lies in one
-  // node, the wave
-  {
-    int run_node = kNone, runs = 0;
-    double run_gain = 0.0;
+    int first_node = kNone, cur = kNone;
+    double first_gain = 0.0, cur_gain = 0.0, parent = 0.0;
+    unsigned first_key = 0, cur_key = 0;
+    I64Pair ns{0, 0}, base{0, 0};
 #pragma unroll
     for (int e = 0; e < kE; e++) {
-      const bool has = ((ends >> e) & 1u) != 0 && gain[e] > 0;
-      if (has) {
-        if (node[e] != run_node) {
-          if (runs > 0) atomicMax(&s_gain[run_node], static_cast<unsigned long long>(__double_as_longlong(run_gain)));
-          run_node = node[e];
-          run_gain = gain[e];
-          runs++;
-        } else {
-          run_gain = gain[e] > run_gain ? gain[e] : run_gain;
+      if (i0 + e < a.N) {
+        const int2 v = s_q[entry[e] & 0xffff];
+        run.grad += v.x;
+        run.hess += v.y;
+      }
+      if ((ends >> e) & 1u) {
+        if (node[e] != cur) {
+          if (first_node == kNone) {
+            first_node = cur;  // (kNone again while there was none before)
+            first_gain = cur_gain;
+            first_key  = cur_key;
+          } else if (cur_key != 0) {
+            s_gain[cur] = static_cast<unsigned long long>(__double_as_longlong(cur_gain));
+            s_key[cur]  = cur_key;
+          }
+          cur      = node[e];
+          cur_gain = 0.0;
+          cur_key  = 0;
+          ns       = st.node_sums[a.level_first + cur];
+          base     = st.base[a.level_first + cur];
+          parent   = leaf_gain(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, a.l1, reg);
+        }
+        const I64Pair ls{run.grad - base.grad, run.hess - base.hess}, rs{ns.grad - ls.grad, ns.hess - ls.hess};
+        if (ls.hess > 0 && rs.hess > 0) {
+          // calculate_gain with the parent's term formed once per node
+          const double gain =
+            0.0 + ((0.5 * (leaf_gain(static_cast<double>(ls.grad) * inv_g, static_cast<double>(ls.hess) * inv_h, a.l1, reg) +
+                           leaf_gain(static_cast<double>(rs.grad) * inv_g, static_cast<double>(rs.hess) * inv_h, a.l1, reg) -
+                           parent)) -
+                   a.min_split_gain);
+          if (gain > 0 && gain >= cur_gain) {
+            const unsigned key = tie_key(rp, bin[e], bin[e + 1]);
+            cur_key            = gain > cur_gain ? key : max(cur_key, key);
+            cur_gain           = gain;
+          }
         }
       }
     }
-    const unsigned long long have = __ballot(runs > 0);
+    // one slot for the node the thread begins with, one for the node it ends with (the same one, or none)
+    if (first_node == kNone) {
+      first_node = cur;
+      first_gain = cur_gain;
+      first_key  = cur_key;
+      cur_key    = 0;
+    }
+    const unsigned long long first_bits = static_cast<unsigned long long>(__double_as_longlong(first_gain));
+    const unsigned long long cur_bits   = static_cast<unsigned long long>(__double_as_longlong(cur_gain));
+    // where a whole wave lies in one node its lanes meet first
+    const unsigned long long have = __ballot(first_key != 0 || cur_key != 0);
+    bool alone = true;
     if (have != 0) {
-      const int first_lane = __ffsll(have) - 1;
-      const int wave_node  = __shfl(run_node, first_lane, 64);
-      if (__all(runs == 0 || run_node == wave_node)) {
+      const int wave_node = __shfl(first_node, __ffsll(have) - 1, 64);
+      alone               = !__all(cur_key == 0 && (first_key == 0 || first_node == wave_node));
+      if (!alone) {
+        double top = first_key != 0 ? first_gain : 0.0;
         for (int off = 32; off >= 1; off >>= 1) {
-          const double o = __shfl_xor(run_gain, off, 64);
-          run_gain       = o > run_gain ? o : run_gain;
+          const double o = __shfl_xor(top, off, 64);
+          top            = o > top ? o : top;
         }
-        if (lane == 0) atomicMax(&s_gain[wave_node], static_cast<unsigned long long>(__double_as_longlong(run_gain)));
-      } else if (runs > 0) {
-        atomicMax(&s_gain[run_node], static_cast<unsigned long long>(__double_as_longlong(run_gain)));
+        unsigned key = first_key != 0 && first_gain == top ? first_key : 0u;
+        for (int off = 32; off >= 1; off >>= 1) key = max(key, static_cast<unsigned>(__shfl_xor(static_cast<int>(key), off, 64)));
+        first_node = wave_node;
+        first_gain = top;
+        first_key  = lane == 0 ? key : 0u;
       }
     }
-  }
-  __syncthreads();
-  // among the places with that gain, and the empty bins behind each of them, the reference's choice
-  // (cand_better): the largest bin mod 512 among all bins, then the smallest bin
+    const unsigned long long mine_bits = alone ? first_bits : static_cast<unsigned long long>(__double_as_longlong(first_gain));
+    if (first_key != 0) atomicMax(&s_gain[first_node], mine_bits);
+    if (cur_key != 0) atomicMax(&s_gain[cur], cur_bits);
+    __syncthreads();
+    if (first_key != 0 && mine_bits == s_gain[first_node]) atomicMax(&s_key[first_node], first_key);
+    if (cur_key != 0 && cur_bits == s_gain[cur]) atomicMax(&s_key[cur], cur_key);
+    __syncthreads();
+  } else {
+    double gain[kE];
+    unsigned dead = 0;
 #pragma unroll
-  for (int e = 0; e < kE; e++) {
-    if (((ends >> e) & 1u) != 0 && gain[e] > 0 &&
-        static_cast<unsigned long long>(__double_as_longlong(gain[e])) == s_gain[node[e]]) {
-      // bins [first, last] share the gain; one of them is 511 mod 512, or the residues ascend
-      const int first = rp + bin[e], last = rp + bin[e + 1] - 1;
-      const int pick  = min(first | 511, last);
-      atomicMax(&s_key[node[e]], (static_cast<unsigned>(pick & 511) << 11 | static_cast<unsigned>(2047 - (pick - rp))) + 1u);
+    for (int e = 0; e < kE; e++) gain[e] = 0.0;
+    for (int k = 0; k < a.K; k++) {
+      int2 q[kE];
+      I64Pair sum{0, 0};
+#pragma unroll
+      for (int e = 0; e < kE; e++) {
+        q[e] = make_int2(0, 0);
+        if (i0 + e < a.N) {
+          const int r = static_cast<int>(entry[e] & 0xffff);
+          q[e]        = st.qgh[r * a.K + k];
+        }
+        sum.grad += q[e].x;
+        sum.hess += q[e].y;
+      }
+      const int64_t ig = wave_inclusive_sum(sum.grad), ih = wave_inclusive_sum(sum.hess);
+      I64Pair* const s_tot = s_pair[k & 1];
+      if (lane == 63) s_tot[wave] = I64Pair{ig, ih};
+      __syncthreads();
+      I64Pair before{ig - sum.grad, ih - sum.hess};
+      for (int w = 0; w < kT / 64; w++) {
+        before.grad += w < wave ? s_tot[w].grad : 0;
+        before.hess += w < wave ? s_tot[w].hess : 0;
+      }
+#pragma unroll
+      for (int e = 0; e < kE; e++) {
+        before.grad += q[e].x;
+        before.hess += q[e].y;
+        if ((ends >> e) & 1u) {
+          const int64_t at = static_cast<int64_t>(a.level_first + node[e]) * a.K + k;
+          const I64Pair ns = st.node_sums[at], base = st.base[at];
+          const I64Pair ls{before.grad - base.grad, before.hess - base.hess};
+          bool d = (dead >> e) & 1u;
+          add_gain(gain[e], d, ls, ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
+          dead |= d ? 1u << e : 0u;
+        }
+      }
     }
+    // best gain per node: a thread's runs of one node first, then, where a whole wave lies in one
+    // node, the wave
+    {
+      int run_node = kNone, runs = 0;
+      double run_gain = 0.0;
+#pragma unroll
+      for (int e = 0; e < kE; e++) {
+        const bool has = ((ends >> e) & 1u) != 0 && gain[e] > 0;
+        if (has) {
+          if (node[e] != run_node) {
+            if (runs > 0) atomicMax(&s_gain[run_node], static_cast<unsigned long long>(__double_as_longlong(run_gain)));
+            run_node = node[e];
+            run_gain = gain[e];
+            runs++;
+          } else {
+            run_gain = gain[e] > run_gain ? gain[e] : run_gain;
+          }
+        }
+      }
+      const unsigned long long have = __ballot(runs > 0);
+      if (have != 0) {
+        const int first_lane = __ffsll(have) - 1;
+        const int wave_node  = __shfl(run_node, first_lane, 64);
+        if (__all(runs == 0 || run_node == wave_node)) {
+          for (int off = 32; off >= 1; off >>= 1) {
+            const double o = __shfl_xor(run_gain, off, 64);
+            run_gain       = o > run_gain ? o : run_gain;
+          }
+          if (lane == 0) atomicMax(&s_gain[wave_node], static_cast<unsigned long long>(__double_as_longlong(run_gain)));
+        } else if (runs > 0) {
+          atomicMax(&s_gain[run_node], static_cast<unsigned long long>(__double_as_longlong(run_gain)));
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kE; e++) {
+      if (((ends >> e) & 1u) != 0 && gain[e] > 0 &&
+          static_cast<unsigned long long>(__double_as_longlong(gain[e])) == s_gain[node[e]]) {
+        atomicMax(&s_key[node[e]], tie_key(rp, bin[e], bin[e + 1]));
+      }
+    }
+    __syncthreads();
   }
-  __syncthreads();
   for (int j = tid; j < a.n_nodes; j += kT) {
-    if (st.seg_count[a.level_first + j] == 0) continue;
-    const unsigned key = s_key[j];
-    Cand c{0.0, -1};
+    const unsigned key = s_key[j];  // (nodes without rows have none)
+    SmallCand c{0.0, 0u, 0};
     if (key != 0) {
       c.gain = __longlong_as_double(static_cast<long long>(s_gain[j]));
-      c.bin  = rp + 2047 - static_cast<int>((key - 1u) & 2047u);
+      c.rel  = 2047 - static_cast<int>((key - 1u) & 2047u);
+      c.key  = tie_key_of_bin(rp + c.rel);
     }
     out[static_cast<int64_t>(j) * a.F] = c;
   }
@@ -631,67 +763,73 @@ __global__ void __launch_bounds__(kT)
   small_apply_kernel(SmallTreeState st, LevelArgs a, double* leaf, int32_t* feature, double* split, double* gain,
                      double* hessian, int32_t* row_leaf)
 {
-  __shared__ Cand s_cand[kT / 64];
-  __shared__ int s_feature[kT / 64];
+  __shared__ double s_best[kT / 64];
+  __shared__ int4 s_pick[kT / 64];
   __shared__ int s_cnt[kT / 64];
   __shared__ I64Pair s_sum[2][kT / 64];
-  if (st.live[a.depth] == 0) return;
   const int j    = blockIdx.x;
   const int node = a.level_first + j;
-  const int n    = st.seg_count[node];
-  if (n == 0) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int s0 = st.seg_start[node];
-  const uint16_t* order = st.order[a.depth & 1];  // feature 0's
-  Cand best{0.0, -1};
-  int ft = -1;
-  if (st.node_sums[static_cast<int64_t>(node) * a.K].hess > 0) {
-    const Cand* c = st.cand + static_cast<int64_t>(j) * a.F;
-    for (int i = tid; i < a.F; i += kT)
-      if (cand_better(c[i], best)) {
-        best = c[i];
-        ft   = i;
-      }
+  const int live      = st.live[a.depth];
+  const int2 seg      = st.seg[node];
+  const int64_t hess0 = st.node_sums[static_cast<int64_t>(node) * a.K].hess;
+  const int s0 = seg.x, n = seg.y;
+  if (live == 0 || n == 0) return;
+  const uint32_t* order = st.order[a.depth & 1] + s0;  // feature 0's
+  // a thread's first row is asked for together with the candidates
+  const uint32_t first_row = tid < n ? order[tid] & 0xffffu : 0u;
+  auto row_at = [&](int i) { return i == tid ? first_row : order[i] & 0xffffu; };
+  // the best candidate by (gain, key of the tie rule), without branches
+  double best = 0.0;
+  unsigned best_key = 0;
+  int ft = 0, rel = 0;
+  auto take = [&](double gain_o, unsigned key_o, int ft_o, int rel_o) {
+    const bool better = gain_o > best || (gain_o == best && key_o > best_key);
+    best     = better ? gain_o : best;
+    best_key = better ? key_o : best_key;
+    ft       = better ? ft_o : ft;
+    rel      = better ? rel_o : rel;
+  };
+  const SmallCand* c = st.cand + static_cast<int64_t>(j) * a.F;
+  for (int i = tid; i < a.F; i += kT) {
+    const SmallCand o = c[i];
+    take(o.gain, o.key, i, o.rel);
   }
   for (int off = 32; off >= 1; off >>= 1) {
-    Cand o;
-    o.gain      = __shfl_xor(best.gain, off, 64);
-    o.bin       = __shfl_xor(best.bin, off, 64);
-    const int g = __shfl_xor(ft, off, 64);
-    if (cand_better(o, best)) {
-      best = o;
-      ft   = g;
+    const double g   = __shfl_xor(best, off, 64);
+    const unsigned k = static_cast<unsigned>(__shfl_xor(static_cast<int>(best_key), off, 64));
+    const int f_o = __shfl_xor(ft, off, 64), r_o = __shfl_xor(rel, off, 64);
+    take(g, k, f_o, r_o);
+  }
+  if (kT > 64) {
+    if (lane == 0) {
+      s_best[wave] = best;
+      s_pick[wave] = make_int4(static_cast<int>(best_key), ft, rel, 0);
+    }
+    __syncthreads();
+    for (int w = 0; w < kT / 64; w++) {
+      const int4 p = s_pick[w];
+      take(s_best[w], static_cast<unsigned>(p.x), p.y, p.z);
     }
   }
-  if (lane == 0) {
-    s_cand[wave]    = best;
-    s_feature[wave] = ft;
-  }
-  __syncthreads();
-  for (int w = 0; w < kT / 64; w++)
-    if (cand_better(s_cand[w], best)) {
-      best = s_cand[w];
-      ft   = s_feature[w];
-    }
-  if (!(best.bin >= 0 && best.gain > 1e-5)) {
-    for (int i = s0 + tid; i < s0 + n; i += kT) {
-      st.node_of_pos[i] = kNone;
-      if (row_leaf != nullptr) row_leaf[order[i]] = node;
+  if (!(hess0 > 0 && best_key != 0 && best > 1e-5)) {
+    for (int i = tid; i < n; i += kT) {
+      st.node_of_pos[s0 + i] = kNone;
+      if (row_leaf != nullptr) row_leaf[row_at(i)] = node;
     }
     return;
   }
   const int lc = left_child(node), rc = right_child(node);
-  const int rel        = best.bin - st.rp[ft];
   const uint16_t* bins = st.bins + static_cast<int64_t>(ft) * st.pitch;
   int nl = 0;
   I64Pair sum{0, 0};
-  for (int i = s0 + tid; i < s0 + n; i += kT) {
-    const int r     = order[i];
+  for (int i = tid; i < n; i += kT) {
+    const int r     = static_cast<int>(row_at(i));
+    const int2 q    = st.qgh[r * a.K];  // (asked for beside the bin)
     const bool left = bins[r] <= rel;
     if (!a.last) st.code[r] = left ? 1 : 2;
     if (a.last && row_leaf != nullptr) row_leaf[r] = left ? lc : rc;
     if (left) {
-      const int2 q = st.qgh[r * a.K];
       nl++;
       sum.grad += q.x;
       sum.hess += q.y;
@@ -729,8 +867,8 @@ __global__ void __launch_bounds__(kT)
     }
     if (++k == a.K) break;
     sum = I64Pair{0, 0};
-    for (int i = s0 + tid; i < s0 + n; i += kT) {
-      const int r = order[i];
+    for (int i = tid; i < n; i += kT) {
+      const int r = static_cast<int>(row_at(i));
       if (bins[r] <= rel) {
         const int2 q = st.qgh[r * a.K + k];
         sum.grad += q.x;
@@ -743,25 +881,29 @@ __global__ void __launch_bounds__(kT)
   if (tid == 0) {
     feature[node] = ft;
     split[node]   = st.proposals[static_cast<int64_t>(ft) * a.S + rel];
-    gain[node]    = best.gain;
-    st.seg_start[lc] = s0;
-    st.seg_count[lc] = lefts;
-    st.seg_start[rc] = s0 + lefts;
-    st.seg_count[rc] = n - lefts;
+    gain[node]    = best;
+    st.seg[lc]    = make_int2(s0, lefts);
+    st.seg[rc]    = make_int2(s0 + lefts, n - lefts);
     st.live[a.depth + 1] = 1;
   }
   if (!a.last)
     for (int i = tid; i < n; i += kT) st.node_of_pos[s0 + i] = static_cast<uint16_t>(2 * j + (i < lefts ? 0 : 1));
 }
 
+template <int kT, int kE, bool kSingle>
+int launch_small_scan_as(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a)
+{
+  static std::atomic<bool> attr_set[kMaxDevices] = {};
+  const size_t lds = static_cast<size_t>((a.N + 1) / 2 * 2) * 8 + (kT * kE + 4) * 4 + static_cast<size_t>(a.n_nodes) * 12 +
+                     (a.n_nodes / 2 + 1) * 4 + (a.N + 3) / 4 * 4 + 16;
+  LBT_TRY(allow_dynamic_lds(small_scan_kernel<kT, kE, kSingle>, 156 * 1024, attr_set));
+  small_scan_kernel<kT, kE, kSingle><<<a.F, kT, lds, stream>>>(st, a);
+  return LBT_OK;
+}
 template <int kT, int kE>
 int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a)
 {
-  static std::atomic<bool> attr_set[kMaxDevices] = {};
-  const size_t lds = static_cast<size_t>(a.n_nodes) * 12 + (a.n_nodes / 2 + 1) * 4 + (kT * kE + 8) * 2;
-  LBT_TRY(allow_dynamic_lds(small_scan_kernel<kT, kE>, 120 * 1024, attr_set));
-  small_scan_kernel<kT, kE><<<a.F, kT, lds, stream>>>(st, a);
-  return LBT_OK;
+  return a.K == 1 ? launch_small_scan_as<kT, kE, true>(stream, st, a) : launch_small_scan_as<kT, kE, false>(stream, st, a);
 }
 
 }  // namespace
@@ -772,7 +914,7 @@ int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelA
 bool small_tree_fits(int64_t N, int F, int K, int max_depth, int S)
 {
   return N <= kSmallMaxRows && K <= kSmallMaxOutputs && N * K <= kQuantChunks * 4096 && max_depth >= 1 &&
-         max_depth <= kSmallMaxDepth && S <= LBT_MAX_SPLIT_SAMPLES && F <= 32768 &&
+         max_depth <= kSmallMaxDepth && S <= LBT_MAX_SPLIT_SAMPLES && static_cast<int64_t>(F) * S < (int64_t(1) << 26) &&
          (static_cast<int64_t>(F) << (max_depth - 1)) <= (int64_t(1) << 22);
 }
 
@@ -808,7 +950,7 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
     LBT_TRY(allow_dynamic_lds(small_prologue_kernel<T>, 120 * 1024, attr_set));
     int P = 1;
     while (P < prm.split_samples) P <<= 1;
-    const size_t feature_lds = static_cast<size_t>(P) * (2 * sizeof(T) + 8) + 16 + N * 2 + 16;
+    const size_t feature_lds = static_cast<size_t>(P) * (2 * sizeof(T) + 8) + 16 + N * 4 + 16;
     const size_t quant_lds   = (2048 + 2 * kQuantChunks + 4 + 2 * static_cast<size_t>(K)) * 8;
     const int64_t clear      = std::max<int64_t>(static_cast<int64_t>(prm.max_nodes) * K, N);
     const int clearers       = static_cast<int>(std::min<int64_t>((clear + kPrologueThreads - 1) / kPrologueThreads, 64));
