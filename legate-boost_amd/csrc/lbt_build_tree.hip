@@ -1333,7 +1333,9 @@ struct Layout {
   Cand* partial;
   I64Pair* hist;
   size_t hist_bytes;
-  SmallTreeState small;  // null pointers when the shape is not one for the few-rows builder
+  // null pointers when the shape is not one for these builders
+  SmallTreeState small;
+  MidTreeState mid;
 };
 
 size_t hist_bytes_bound(int F, int K, int S, int max_depth, int64_t cache_bytes)
@@ -1440,6 +1442,31 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     st.qgh         = L.qgh;
     st.scales      = L.scales;
     st.cand        = ar.take<SmallCand>(level_nodes * F);
+  }
+  L.mid = MidTreeState{};
+  if (L.small.pitch == 0 && mid_tree_fits(N, F, K, max_depth, S)) {
+    MidTreeState& st   = L.mid;
+    st.pitch           = (N + 255) / 256 * 256;
+    st.bin_bytes       = S <= 256 ? 1 : 2;
+    const size_t fs    = static_cast<size_t>(F) * S;
+    const size_t level_hist = static_cast<size_t>(level_nodes) * K * fs;
+    st.bins       = ar.take<char>(static_cast<size_t>(F) * st.pitch * st.bin_bytes);
+    st.props      = ar.take<char>(fs * elem);
+    st.proposals  = ar.take<double>(fs);
+    st.counts     = ar.take<int32_t>(F);
+    st.rp         = ar.take<int32_t>(F + 1);
+    st.chunk_sums = ar.take<double>(2 * ((N * K + 4095) / 4096));
+    st.q          = ar.take<int2>(static_cast<size_t>(K) * st.pitch);
+    st.row_node   = ar.take<uint16_t>(st.pitch);
+    st.q_stats    = ar.take<unsigned long long>(4);
+    st.images     = ar.take<unsigned long long>(mid_image_words(N, F, K, max_depth, S));
+    st.hist[0]    = ar.take<I64Pair>(level_hist);
+    st.hist[1]    = ar.take<I64Pair>(level_hist);
+    st.node_sums  = L.node_sums;
+    st.scales     = L.scales;
+    st.cand       = ar.take<SmallCand>(level_nodes * F);
+    st.splits     = ar.take<int2>(level_nodes);
+    st.live       = ar.take<int32_t>(max_depth + 1);
   }
 }
 
@@ -1553,6 +1580,18 @@ int run_quantiser(hipStream_t stream, const double* g, const double* h, int64_t 
                                                    root_sums, qstats);
   }
   LBT_HIP(hipGetLastError());
+  return LBT_OK;
+}
+
+// Hands the level counts of a build to the profiler: copied to the host in stream order.
+int profile_levels(hipStream_t stream, const LevelMeta* totals, int max_depth, double per_row, double per_node,
+                   double root_extra)
+{
+  static_assert(sizeof(LevelMeta) == sizeof(LevelCounts), "the host mirror of LevelMeta");
+  ProfLevels* const levels = profiler().begin_levels(std::min(max_depth, 64), per_row, per_node, root_extra);
+  if (levels == nullptr) return LBT_OK;
+  LBT_HIP(hipMemcpyAsync(levels->host, totals, sizeof(LevelMeta) * levels->levels, hipMemcpyDeviceToHost, stream));
+  LBT_HIP(hipEventRecord(levels->arrived, stream));
   return LBT_OK;
 }
 
@@ -1847,23 +1886,16 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
   }
 
   // ---- observation points
-  static_assert(sizeof(LevelMeta) == sizeof(LevelCounts), "the host mirror of LevelMeta");
   const bool tap_levels =
     taps && (taps->level_instances || taps->level_built_instances || taps->level_built_nodes) && max_depth > 0;
-  ProfLevels* prof_levels = nullptr;
   if (profiler().mode != 0 && max_depth > 0) {
     // bytes of one feature value as the level reads it (X itself, or its cached bin)
     const bool cached      = hs.binned != nullptr;
     const double per_value = cached ? hs.bin_bytes : static_cast<double>(sizeof(T));
-    prof_levels            = profiler().begin_levels(
-      std::min(max_depth, 64), static_cast<double>(F) * per_value + K * 8.0 + 8.0, static_cast<double>(K) * B * 16.0,
-      // the root launch also writes the feature-major copy of the bins
-      hs.bins_t != nullptr ? static_cast<double>(N) * F * hs.bin_bytes : 0.0);
-    if (prof_levels != nullptr) {
-      LBT_HIP(hipMemcpyAsync(prof_levels->host, L.level_totals, sizeof(LevelMeta) * prof_levels->levels,
-                             hipMemcpyDeviceToHost, stream));
-      LBT_HIP(hipEventRecord(prof_levels->arrived, stream));
-    }
+    LBT_TRY(profile_levels(stream, L.level_totals, max_depth, static_cast<double>(F) * per_value + K * 8.0 + 8.0,
+                           static_cast<double>(K) * B * 16.0,
+                           // the root launch also writes the feature-major copy of the bins
+                           hs.bins_t != nullptr ? static_cast<double>(N) * F * hs.bin_bytes : 0.0));
   }
   std::vector<LevelMeta> h_levels(max_depth > 0 ? max_depth : 1);
   if (tap_levels && sync_at_end)
@@ -2026,20 +2058,37 @@ static int build_tree_entry(void* stream, const void* X, int32_t x_dtype, int64_
                      !(t->proposals || t->row_pointers || t->quantised || t->node_sums || t->positions ||
                        t->positions_per_level || t->histogram || t->level_instances || t->level_built_instances ||
                        t->level_built_nodes);
-  if (plain && L.small.order[0] != nullptr) {
+  if (plain && (L.small.order[0] != nullptr || L.mid.bins != nullptr)) {
     int32_t* const row_leaf = taps ? taps->row_leaf : nullptr;
-    if (x_dtype == LBT_F32)
-      rc = lbt::small_tree_build<float>(s, L.small, static_cast<const float*>(X), row_offset, n_rows, n_features,
-                                        n_outputs, g, h, feature_set, *params, leaf, feature, split, gain, hessian,
-                                        row_leaf, taps ? &taps->n_bins : nullptr, &done);
+    int32_t* const n_bins   = taps ? &taps->n_bins : nullptr;
+    const float* const Xf   = static_cast<const float*>(X);
+    const double* const Xd  = static_cast<const double*>(X);
+    lbt::LevelMeta* totals  = nullptr;
+    if (lbt::profiler().mode != 0) {
+      totals = L.level_totals;
+      lbt::zero_kernel<<<1, lbt::kThreads, 0, s>>>(reinterpret_cast<uint4*>(totals), 2 * params->max_depth);
+    }
+    if (L.small.order[0] != nullptr)
+      rc = x_dtype == LBT_F32
+             ? lbt::small_tree_build<float>(s, L.small, Xf, row_offset, n_rows, n_features, n_outputs, g, h, feature_set,
+                                            *params, leaf, feature, split, gain, hessian, row_leaf, n_bins, totals, &done)
+             : lbt::small_tree_build<double>(s, L.small, Xd, row_offset, n_rows, n_features, n_outputs, g, h, feature_set,
+                                             *params, leaf, feature, split, gain, hessian, row_leaf, n_bins, totals, &done);
     else
-      rc = lbt::small_tree_build<double>(s, L.small, static_cast<const double*>(X), row_offset, n_rows, n_features,
-                                         n_outputs, g, h, feature_set, *params, leaf, feature, split, gain, hessian,
-                                         row_leaf, taps ? &taps->n_bins : nullptr, &done);
+      rc = x_dtype == LBT_F32
+             ? lbt::mid_tree_build<float>(s, L.mid, Xf, row_offset, n_rows, n_features, n_outputs, g, h, feature_set,
+                                          *params, leaf, feature, split, gain, hessian, row_leaf, n_bins, totals, &done)
+             : lbt::mid_tree_build<double>(s, L.mid, Xd, row_offset, n_rows, n_features, n_outputs, g, h, feature_set,
+                                           *params, leaf, feature, split, gain, hessian, row_leaf, n_bins, totals, &done);
     if (rc == LBT_OK && done) {
       if (taps) {
         lbt::final_histogram_range(n_outputs, taps->n_bins, *params, &taps->hist_node_begin, &taps->hist_node_end);
         if (sync_at_end) LBT_HIP(hipMemcpyAsync(taps->scales, L.scales, sizeof(double) * 4, hipMemcpyDeviceToHost, s));
+      }
+      if (totals != nullptr) {
+        const double row_bytes = static_cast<double>(n_features) * (params->split_samples <= 256 ? 1 : 2) + n_outputs * 8.0 + 8.0;
+        LBT_TRY(lbt::profile_levels(s, L.level_totals, params->max_depth, row_bytes,
+                                    static_cast<double>(n_outputs) * n_features * params->split_samples * 16.0, 0.0));
       }
       if (!sync_at_end) return LBT_OK;
       LBT_HIP(hipStreamSynchronize(s));

@@ -176,6 +176,45 @@ int thread_resources_here(ThreadResources** out)
   return LBT_OK;
 }
 
+int DeviceAnswer::open()
+{
+  ThreadResources* here = nullptr;
+  LBT_TRY(thread_resources_here(&here));
+  if (here->answer == nullptr) {
+    LBT_HIP(hipHostMalloc(reinterpret_cast<void**>(&here->answer), 64, hipHostMallocDefault));
+    here->answer[0] = here->answer[1] = 0;
+  }
+  words = here->answer;
+  tag   = ++here->answer_tag;
+  if (tag == 0) tag = here->answer_tag = 1;
+  return LBT_OK;
+}
+
+int DeviceAnswer::wait(hipStream_t stream, unsigned* flags, int32_t* n_bins)
+{
+  volatile unsigned long long* const w = words;
+  auto arrived = [&]() { return (w[0] >> 32) == tag && (n_bins == nullptr || (w[1] >> 32) == tag); };
+  // should the words not come (the stream has failed), the stream's own state ends the wait
+  for (int64_t spin = 1; !arrived(); spin++) {
+    if (spin % 16384 != 0) continue;
+    const hipError_t e = hipStreamQuery(stream);
+    if (e == hipErrorNotReady) continue;
+    LBT_HIP(e);
+    if (arrived()) break;
+    set_error("the tree builder's kernels did not report");
+    return LBT_ERR_HIP;
+  }
+  const unsigned got = static_cast<unsigned>(w[0] & 0xffffffffULL);
+  if (n_bins != nullptr) *n_bins = static_cast<int32_t>(w[1] & 0xffffffffULL);
+  if ((got & 2u) != 0) {
+    set_error("a quantised gradient or hessian reaches 2^31 and does not fit the packed 32-bit form: one entry "
+              "holds the whole absolute sum and was rounded up");
+    return LBT_ERR_UNSUPPORTED;
+  }
+  *flags = got & 1u;
+  return LBT_OK;
+}
+
 }  // namespace lbt
 
 extern "C" {

@@ -1,6 +1,8 @@
 // Device functions shared by the two tree builders (lbt_build_tree.hip, lbt_small_tree.hip).
 #pragma once
 
+#include <limits>
+
 #include "lbt_internal.h"
 
 namespace lbt {
@@ -102,6 +104,159 @@ __device__ inline void add_gain(double& gain, bool& dead, const I64Pair& ls, con
                          static_cast<double>(rg) * inv_g, static_cast<double>(rh) * inv_h,
                          static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, l1, reg,
                          min_split_gain);
+}
+
+// Inclusive sums over a wave, 32 bits (see wave_inclusive_sum)
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ int dpp_take32(int v)
+{
+  return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xf, true);
+}
+__device__ __forceinline__ int wave_inclusive_sum32(int v)
+{
+  v += dpp_take32<0x111, 0xf>(v);
+  v += dpp_take32<0x112, 0xf>(v);
+  v += dpp_take32<0x114, 0xf>(v);
+  v += dpp_take32<0x118, 0xf>(v);
+  v += dpp_take32<0x142, 0xa>(v);
+  v += dpp_take32<0x143, 0xc>(v);
+  return v;
+}
+
+// Sum of the threads before this one; all threads of the workgroup call it. s_wave: one int per wave.
+template <int kT>
+__device__ __forceinline__ int block_exclusive_sum32(int v, int* s_wave)
+{
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int incl = wave_inclusive_sum32(v);
+  if (lane == 63) s_wave[wave] = incl;
+  __syncthreads();
+  int before = 0;
+  for (int w = 0; w < kT / 64; w++) before += w < wave ? s_wave[w] : 0;
+  return before + incl - v;
+}
+
+// The order of cand_better among equal gains as one number, for fewer than 2^26 bins: larger wins, none is 0.
+__device__ __forceinline__ unsigned tie_key_of_bin(int bin)
+{
+  return (static_cast<unsigned>(bin & 511) << 17 | static_cast<unsigned>(0x1ffff - (bin >> 9))) + 1u;
+}
+
+__device__ __forceinline__ int bin_of_tie_key(unsigned key)
+{
+  return static_cast<int>(((key - 1u) >> 17) | ((0x1ffffu - ((key - 1u) & 0x1ffffu)) << 9));
+}
+
+// Split proposals of one feature by one workgroup (build_tree.cu:867-964): the sampled rows' values,
+// sorted on order-preserving keys, without repetitions.
+struct SampleSpec {
+  int S;
+  int32_t seed;
+  int64_t dataset_rows, row_offset, n_rows;
+  int F;
+};
+constexpr int kRankSortMax = 512;  // samples sorted by counting the smaller ones; more: a bitonic network
+template <typename T>
+constexpr int kProposalScratch = 2 * sizeof(T) + 4;  // bytes of LDS per sample (of P, the power of two)
+
+// Returns their number; *proposals points to them in the LDS (the last one stands for +inf,
+// build_tree.cu:953-956). P: power of two that holds S, at most 2 * kT. s_wave: kT / 64 ints.
+template <typename T, int kT>
+__device__ __forceinline__ int feature_proposals(const T* __restrict__ X, const SampleSpec& a, int f, int P,
+                                                 unsigned char* smem, int* s_wave, const T** proposals)
+{
+  using Key   = typename KeyOf<T>::type;
+  Key* s_in   = reinterpret_cast<Key*>(smem);           // [P] as drawn; later the distinct values
+  Key* s_key  = s_in + P;                               // [P] sorted
+  int* s_rank = reinterpret_cast<int*>(s_key + P);      // [P]
+  __shared__ int s_n;
+  const int tid = threadIdx.x;
+  // the sampled rows (build_tree.cu:882-898)
+  for (int i = tid; i < P; i += kT) {
+    Key key = ~Key(0);
+    if (i < a.S) {
+      uint32_t x = minstd_seed(static_cast<uint32_t>(a.seed));
+      x          = minstd_next(minstd_discard(x, static_cast<uint64_t>(i)));
+      const double u    = uniform01(x);
+      const double b    = static_cast<double>(a.dataset_rows - 1) + 1.0;
+      const int64_t row = static_cast<int64_t>((u * (b - 0.0)) + 0.0) - a.row_offset;
+      key               = to_key(row >= 0 && row < a.n_rows ? X[row * a.F + f] : T(0));
+    }
+    s_in[i]   = key;
+    s_rank[i] = 0;
+  }
+  __syncthreads();
+  if (P <= kRankSortMax && P <= kT) {
+    // a sample's place is the number of samples before it; several threads share the counting
+    const int parts = kT / P, i = tid & (P - 1), part = tid / P;
+    const int per = (a.S + parts - 1) / parts, j0 = part * per, j1 = min(a.S, j0 + per);
+    if (i < a.S) {
+      const Key mine = s_in[i];
+      int before     = 0;
+      for (int j = j0; j < j1; j++) {
+        const Key o = s_in[j];
+        before += (o < mine || (o == mine && j < i)) ? 1 : 0;
+      }
+      atomicAdd(&s_rank[i], before);
+    }
+    __syncthreads();
+    for (int j = tid; j < a.S; j += kT) s_key[s_rank[j]] = s_in[j];
+    __syncthreads();
+  } else {
+    for (int i = tid; i < P; i += kT) s_key[i] = s_in[i];
+    __syncthreads();
+    for (int size = 2; size <= P; size <<= 1)
+      for (int stride = size >> 1; stride > 0; stride >>= 1) {
+        for (int i = tid; i < P / 2; i += kT) {
+          const int lo = 2 * i - (i & (stride - 1)), hi = lo + stride;
+          const bool up = (lo & size) == 0;
+          const Key x = s_key[lo], y = s_key[hi];
+          if ((x > y) == up) {
+            s_key[lo] = y;
+            s_key[hi] = x;
+          }
+        }
+        __syncthreads();
+      }
+  }
+  // drop values equal to their predecessor; two consecutive samples per thread
+  T* s_prop = reinterpret_cast<T*>(s_in);
+  T v[2]    = {T(0), T(0)};
+  bool keep[2];
+  int mine = 0;
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int i = 2 * tid + u;
+    keep[u]     = false;
+    if (i < a.S) {
+      v[u]    = from_key(s_key[i]);
+      keep[u] = i == 0 || !(v[u] == from_key(s_key[i - 1]));
+    }
+    mine += keep[u] ? 1 : 0;
+  }
+  int at = block_exclusive_sum32<kT>(mine, s_wave);
+  if (tid == kT - 1) s_n = at + mine;
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+    if (keep[u]) s_prop[at++] = v[u];
+  __syncthreads();
+  *proposals = s_prop;
+  return s_n;
+}
+
+// One stochastic rounding of a (grad, hess) pair (build_tree.cu:112-129).
+__device__ __forceinline__ void quantise_pair(double grad, double hess, double sg, double sh, int64_t seed, int64_t row,
+                                              int64_t k, int64_t* qg, int64_t* qh)
+{
+  uint32_t x = minstd_seed(static_cast<uint32_t>(static_cast<uint64_t>(gpair_seed(seed, row, k))));
+  const double scaled_grad    = grad * sg;
+  const double scaled_hess    = hess * sh;
+  const double grad_remainder = scaled_grad - floor(scaled_grad);
+  const double hess_remainder = scaled_hess - floor(scaled_hess);
+  x   = minstd_next(x);
+  *qg = static_cast<int64_t>(floor(scaled_grad) + static_cast<double>(uniform01(x) < grad_remainder));
+  x   = minstd_next(x);
+  *qh = static_cast<int64_t>(floor(scaled_hess) + static_cast<double>(uniform01(x) < hess_remainder));
 }
 
 }  // namespace lbt

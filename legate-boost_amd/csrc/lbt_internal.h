@@ -142,15 +142,26 @@ struct ThreadResources {
   char* stage           = nullptr;
   size_t stage_bytes    = 0;
   hipEvent_t stage_free = nullptr;
-  // one pinned word in which a kernel of the few-rows builder reports to the host, and the tag of the
-  // last call that waited for it
-  uint32_t* answer    = nullptr;
-  uint32_t answer_tag = 0;
+  // two pinned words in which kernels report to the host (see DeviceAnswer), and the last call's tag
+  unsigned long long* answer = nullptr;
+  uint32_t answer_tag        = 0;
 };
 ThreadResources& thread_resources();
 // the same after making sure that what it holds belongs to the current device
 int thread_resources_here(ThreadResources** out);
 int release_thread_resources();
+
+// What the builders without a wait in their middle have to learn from the device: two words of the thread's
+// pinned memory that a kernel early in the queue writes, each (tag << 32) | value: words[0] flags (1: the
+// data need the other builder, 2: a rounded value does not fit 32 bits), words[1] the number of bins.
+// The host looks at them once everything is queued; the tag tells one call's answer from another's.
+struct DeviceAnswer {
+  unsigned long long* words = nullptr;
+  uint32_t tag              = 0;
+  int open();
+  // flags: receives bit 0; bit 1 is returned as LBT_ERR_UNSUPPORTED. n_bins: null when not wanted.
+  int wait(hipStream_t stream, unsigned* flags, int32_t* n_bins);
+};
 
 // ---------------------------------------------------------------- device math
 
@@ -484,13 +495,51 @@ struct SmallTreeState {
   SmallCand* cand;        // [nodes of a level][F]
 };
 bool small_tree_fits(int64_t N, int F, int K, int max_depth, int S);
-// n_bins: receives the number of bins of all features (null: not wanted).
+// n_bins: receives the number of bins of all features (null: not wanted). level_totals: [max_depth], added
+// to (null: not wanted).
 // *taken: the tree has been queued; false (with LBT_OK): the data need the other builder, which has to
 // write every output again.
 template <typename T>
 int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, int64_t row_offset, int64_t N, int F,
                      int K, const double* g, const double* h, const uint8_t* feature_set, const lbt_build_params& prm,
                      double* leaf, int32_t* feature, double* split, double* gain, double* hessian, int32_t* row_leaf,
-                     int32_t* n_bins, bool* taken);
+                     int32_t* n_bins, LevelMeta* level_totals, bool* taken);
+
+// ---------------------------------------------------------------- builder for medium sizes
+// (lbt_mid_tree.hip)
+
+constexpr int kMidMaxDepth      = 10;
+constexpr int kMidMaxLevelNodes = 1 << (kMidMaxDepth - 1);
+constexpr int kMidMaxOutputs    = 16;
+constexpr int64_t kMidMaxValues = int64_t(80) * 1000 * 1000;
+
+struct MidTreeState {
+  int64_t pitch;          // elements between features, outputs (multiple of 256, at least the rows)
+  int bin_bytes;          // 1 or 2
+  void* bins;             // [F][pitch]
+  void* props;            // X dtype [F][S]
+  double* proposals;      // [F][S] the same
+  int32_t* counts;        // [F]
+  int32_t* rp;            // [F + 1]
+  double* chunk_sums;     // [2][chunks of 4096 entries]
+  int2* q;                // [K][pitch]
+  uint16_t* row_node;     // [pitch] node of the level, 0xffff: none
+  unsigned long long* q_stats;  // [4] sum of the positive rounded grads, of the negative ones, flags
+  unsigned long long* images;   // packed histograms of the row ranges
+  I64Pair* hist[2];       // scanned histograms, [node][K][F][S]; level d in hist[d & 1]
+  I64Pair* node_sums;     // [max_nodes][K]
+  double* scales;         // [4]
+  SmallCand* cand;        // [nodes of a level][F]
+  int2* splits;           // [nodes of a level]
+  int32_t* live;          // [max_depth + 1]
+};
+bool mid_tree_fits(int64_t N, int F, int K, int max_depth, int S);
+int64_t mid_image_words(int64_t N, int F, int K, int max_depth, int S);
+// As small_tree_build.
+template <typename T>
+int mid_tree_build(hipStream_t stream, const MidTreeState& st, const T* X, int64_t row_offset, int64_t N, int F, int K,
+                   const double* g, const double* h, const uint8_t* feature_set, const lbt_build_params& prm,
+                   double* leaf, int32_t* feature, double* split, double* gain, double* hessian, int32_t* row_leaf,
+                   int32_t* n_bins, LevelMeta* level_totals, bool* taken);
 
 }  // namespace lbt

@@ -1,0 +1,852 @@
+// BuildTreeTask for inputs of medium size: 2 + 3 * max_depth launches, rows in their own order.
+//
+// With some ten thousand to a million values per level the builder of lbt_build_tree.hip is a chain of
+// ten short launches per level (100,000 x 32: 65 us a level, of which the histogram's atomics are one).
+// Here rows stay where they are: a row carries the number of its node, and a level is three launches.
+//
+//   mid_prologue_kernel   split proposals, one workgroup per feature (build_tree.cu:867-964); chunk sums of
+//                         |g| and |h|; the rest clears outputs and state
+//   mid_bin_kernel        quantiser and root sums (build_tree.cu:51-204); bins of all values, stored
+//                         feature by feature
+//   mid_histogram_kernel  a workgroup = (range of rows) x (some features) x (some built nodes) x (output)
+//                         with a packed histogram of all those nodes in the LDS, written out whole
+//   mid_scan_kernel       a workgroup = (pair of siblings, feature): adds the row ranges' images, running
+//                         sums, the sibling as parent minus node, gains (build_tree.cu:597-740)
+//   mid_apply_kernel      best features, the nodes' outputs and children (build_tree.cu:740-782), new node
+//                         of every row
+//
+// What the reference's rule on unscanned bins (build_tree.cu:645) could change needs a row whose rounded
+// hessian is not positive: such data take the other builder (see small_tree_build, which has the same
+// condition). Otherwise a scanned histogram is the running sums everywhere, and it does not matter
+// which histograms the reference would have kept.
+#include <algorithm>
+#include <limits>
+
+#include "lbt_device.h"
+#include "lbt_internal.h"
+
+namespace lbt {
+namespace {
+
+constexpr int kWide     = 1024;  // threads of all kernels but the scan
+constexpr int kScan     = 256;
+constexpr int kNone     = 0xffff;
+constexpr int kRowsBin  = 256;   // rows of a binning tile
+constexpr int kQuantPer = 8192;  // entries a workgroup rounds
+constexpr int kRowsApply = 4 * kWide;
+constexpr size_t kHistLds = 128 * 1024;
+
+struct MidArgs {
+  int N, F, K, S;
+  int64_t row_offset;
+  int32_t seed;
+  int64_t dataset_rows;
+  const double* g;
+  const double* h;
+  const double* chunk_a;  // chunk sums of |g| and |h|, m each
+  const double* chunk_b;
+  int m;
+  const uint8_t* feature_set;
+  double l1, l2, min_split_gain;
+  int64_t max_nodes;
+  int max_depth;
+  double* leaf;
+  int32_t* feature;
+  double* split;
+  double* gain;
+  double* hessian;
+  int32_t* row_leaf;
+  unsigned long long* answer;  // pinned host memory: flags, and the number of bins, each with `tag` above
+  uint32_t tag;
+};
+
+// Fixed-order sum of one chunk of up to 4096 entries by 256 threads (see abs_sum_level_kernel): every thread
+// of the workgroup calls it, thread t of each quarter with its own chunk. s_a, s_b: [kWide].
+template <bool kAbs>
+__device__ __forceinline__ void quarter_sums(const double* __restrict__ a, const double* __restrict__ b, int64_t first,
+                                             int64_t n, double* s_a, double* s_b, double* sum_a, double* sum_b)
+{
+  const int quarter = threadIdx.x >> 8, t = threadIdx.x & 255;
+  double xa = 0.0, xb = 0.0;
+#pragma unroll 4
+  for (int j = 0; j < 16; j++) {
+    const int64_t e = first + t + 256 * j;
+    if (e < n) {
+      xa += kAbs ? fabs(a[e]) : a[e];
+      xb += kAbs ? fabs(b[e]) : b[e];
+    }
+  }
+  s_a[quarter * 256 + t] = xa;
+  s_b[quarter * 256 + t] = xb;
+  __syncthreads();
+  for (int stride = 128; stride >= 1; stride >>= 1) {
+    if (t < stride) {
+      s_a[quarter * 256 + t] += s_a[quarter * 256 + t + stride];
+      s_b[quarter * 256 + t] += s_b[quarter * 256 + t + stride];
+    }
+    __syncthreads();
+  }
+  *sum_a = s_a[quarter * 256];
+  *sum_b = s_b[quarter * 256];
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kWide)
+  mid_prologue_kernel(const T* __restrict__ X, MidArgs a, MidTreeState st, int P, int sum_groups)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ int s_wave[kWide / 64];
+  const int block = blockIdx.x, tid = threadIdx.x;
+  if (block < a.F) {
+    const SampleSpec sp{a.S, a.seed, a.dataset_rows, a.row_offset, a.N, a.F};
+    const T* s_prop = nullptr;
+    const int n     = feature_proposals<T, kWide>(X, sp, block, P, smem_raw, s_wave, &s_prop);
+    const int64_t at = static_cast<int64_t>(block) * a.S;
+    for (int i = tid; i < n; i += kWide) {
+      // the last proposal becomes +inf (build_tree.cu:953-956)
+      const T v = i == n - 1 ? std::numeric_limits<T>::infinity() : s_prop[i];
+      static_cast<T*>(st.props)[at + i] = v;
+      st.proposals[at + i]              = static_cast<double>(v);
+    }
+    if (tid == 0) st.counts[block] = n;
+    return;
+  }
+  if (block < a.F + sum_groups) {
+    double* s_a = reinterpret_cast<double*>(smem_raw);
+    const int c = (block - a.F) * 4 + (tid >> 8);
+    double xa, xb;
+    quarter_sums<true>(a.g, a.h, static_cast<int64_t>(c) * 4096, static_cast<int64_t>(a.N) * a.K, s_a, s_a + kWide, &xa, &xb);
+    if ((tid & 255) == 0 && c < a.m) {
+      st.chunk_sums[c]       = xa;
+      st.chunk_sums[a.m + c] = xb;
+    }
+    return;
+  }
+  const int at         = block - a.F - sum_groups;
+  const int64_t stride = static_cast<int64_t>(gridDim.x - a.F - sum_groups) * kWide;
+  const int64_t first  = static_cast<int64_t>(at) * kWide + tid;
+  for (int64_t i = first; i < a.max_nodes * a.K; i += stride) {
+    a.leaf[i]       = 0.0;
+    a.hessian[i]    = 0.0;
+    st.node_sums[i] = I64Pair{0, 0};
+  }
+  for (int64_t i = first; i < a.max_nodes; i += stride) {
+    a.feature[i] = -1;
+    a.split[i]   = 0.0;
+    a.gain[i]    = 0.0;
+  }
+  // all rows start in the root; the places behind the last row belong to no node
+  for (int64_t i = first; i < st.pitch; i += stride) st.row_node[i] = i < a.N ? 0 : kNone;
+  if (first <= a.max_depth) st.live[first] = first == 0 ? 1 : 0;
+  if (first < 4) st.q_stats[first] = 0;
+}
+
+struct BinPlan {
+  int quant_groups;  // workgroups of the quantiser
+  int fb;            // features of a binning workgroup
+  int fb_log;        // lanes per row, log2
+  int n_fb;          // feature blocks
+  int row_groups;    // workgroups that share the row tiles of a feature block
+};
+
+template <typename T, typename BinT>
+__global__ void __launch_bounds__(kWide)
+  mid_bin_kernel(const T* __restrict__ X, MidArgs a, MidTreeState st, BinPlan p)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int tid = threadIdx.x;
+  if (static_cast<int>(blockIdx.x) < p.quant_groups) {
+    // the scales, formed by every workgroup in the same fixed order, then this workgroup's entries
+    double* s_a = reinterpret_cast<double*>(smem_raw);
+    __shared__ unsigned long long s_sum[2 * kMidMaxOutputs + 2];
+    __shared__ unsigned s_flags;
+    if (tid < 2 * a.K + 2) s_sum[tid] = 0;
+    if (tid == 0) s_flags = 0;
+    double sum_a, sum_b;
+    if (a.m > 1) {
+      quarter_sums<false>(a.chunk_a, a.chunk_b, 0, a.m, s_a, s_a + kWide, &sum_a, &sum_b);
+    } else {
+      __syncthreads();
+      sum_a = a.chunk_a[0];
+      sum_b = a.chunk_b[0];
+    }
+    const double max_int = 2147483647.0;
+    const double sg = sum_a == 0 ? 1 : max_int / sum_a, sh = sum_b == 0 ? 1 : max_int / sum_b;
+    if (blockIdx.x == 0 && tid == 0) {
+      st.scales[0] = sg;
+      st.scales[1] = sh;
+      st.scales[2] = 1.0 / sg;
+      st.scales[3] = 1.0 / sh;
+    }
+    if (blockIdx.x == 0) {
+      // first bin of every feature among all bins
+      __shared__ int s_wave[kWide / 64];
+      const int per = (a.F + kWide - 1) / kWide, f0 = min(a.F, tid * per), f1 = min(a.F, f0 + per);
+      int mine = 0;
+      for (int f = f0; f < f1; f++) mine += st.counts[f];
+      int run = block_exclusive_sum32<kWide>(mine, s_wave);
+      for (int f = f0; f < f1; f++) {
+        st.rp[f] = run;
+        run += st.counts[f];
+      }
+      if (tid == kWide - 1) st.rp[a.F] = run;
+    }
+    const int64_t n  = static_cast<int64_t>(a.N) * a.K;
+    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * kQuantPer, e1 = e0 + kQuantPer < n ? e0 + kQuantPer : n;
+    int64_t sum_g = 0, sum_h = 0;
+    unsigned long long up = 0, down = 0;
+    unsigned flags = 0;
+    for (int64_t e = e0 + tid; e < e1; e += kWide) {
+      const int64_t row = a.K == 1 ? e : e / a.K;
+      const int k       = a.K == 1 ? 0 : static_cast<int>(e - row * a.K);
+      int64_t qg, qh;
+      quantise_pair(a.g[e], a.h[e], sg, sh, static_cast<int64_t>(a.seed), row + a.row_offset, k, &qg, &qh);
+      if (qg > 2147483647LL || qg < -2147483647LL || qh > 2147483647LL || qh < -2147483647LL) flags |= 2u;
+      if (qh <= 0 && (qg != 0 || qh != 0)) flags |= 1u;
+      st.q[static_cast<int64_t>(k) * st.pitch + row] = make_int2(static_cast<int>(qg), static_cast<int>(qh));
+      up += qg > 0 ? static_cast<unsigned long long>(qg) : 0ULL;
+      down += qg < 0 ? static_cast<unsigned long long>(-qg) : 0ULL;
+      if (a.K == 1) {
+        sum_g += qg;
+        sum_h += qh;
+      } else {
+        atomicAdd(&s_sum[2 * k], static_cast<unsigned long long>(qg));
+        atomicAdd(&s_sum[2 * k + 1], static_cast<unsigned long long>(qh));
+      }
+    }
+    const int64_t wu = wave_inclusive_sum(static_cast<int64_t>(up)), wd = wave_inclusive_sum(static_cast<int64_t>(down));
+    sum_g = wave_inclusive_sum(sum_g);
+    sum_h = wave_inclusive_sum(sum_h);
+    if ((tid & 63) == 63) {
+      if (a.K == 1) {
+        atomicAdd(&s_sum[0], static_cast<unsigned long long>(sum_g));
+        atomicAdd(&s_sum[1], static_cast<unsigned long long>(sum_h));
+      }
+      atomicAdd(&s_sum[2 * a.K], static_cast<unsigned long long>(wu));
+      atomicAdd(&s_sum[2 * a.K + 1], static_cast<unsigned long long>(wd));
+    }
+    if (flags != 0) atomicOr(&s_flags, flags);
+    __syncthreads();
+    if (tid < a.K) {
+      atomic_add_i64(&st.node_sums[tid].grad, static_cast<int64_t>(s_sum[2 * tid]));
+      atomic_add_i64(&st.node_sums[tid].hess, static_cast<int64_t>(s_sum[2 * tid + 1]));
+    }
+    if (tid == 0) {
+      atomicAdd(&st.q_stats[0], s_sum[2 * a.K]);
+      atomicAdd(&st.q_stats[1], s_sum[2 * a.K + 1]);
+      if (s_flags != 0) atomicOr(&st.q_stats[2], static_cast<unsigned long long>(s_flags));
+    }
+    return;
+  }
+  // binning: proposals of the block's features in the LDS (odd pitch: the lanes of a row start in different
+  // banks), a tile of rows at a time, turned in the LDS and stored feature by feature
+  const int block = static_cast<int>(blockIdx.x) - p.quant_groups;
+  const int fblk = block % p.n_fb, rg = block / p.n_fb;
+  const int f0 = fblk * p.fb, nf = min(p.fb, a.F - f0);
+  const int pitch = a.S | 1;
+  T* s_prop       = reinterpret_cast<T*>(smem_raw);
+  int* s_n        = reinterpret_cast<int*>(s_prop + static_cast<size_t>(p.fb) * pitch);
+  constexpr int kTilePitch = kRowsBin + 4 / sizeof(BinT);
+  BinT* s_bin     = reinterpret_cast<BinT*>(s_n + p.fb);  // [fb][kTilePitch]
+  for (int i = tid; i < nf; i += kWide) s_n[i] = st.counts[f0 + i];
+  __syncthreads();
+  for (int i = tid; i < nf * a.S; i += kWide) {
+    const int fi = i / a.S, j = i - fi * a.S;
+    if (j < s_n[fi]) s_prop[fi * pitch + j] = static_cast<const T*>(st.props)[static_cast<int64_t>(f0 + fi) * a.S + j];
+  }
+  const int fi = tid & ((1 << p.fb_log) - 1), r_first = tid >> p.fb_log, r_step = kWide >> p.fb_log;
+  const int tiles = (a.N + kRowsBin - 1) / kRowsBin;
+  BinT* const out = static_cast<BinT*>(st.bins);
+  for (int tile = rg; tile < tiles; tile += p.row_groups) {
+    __syncthreads();
+    if (fi < nf) {
+      const T* prop = s_prop + fi * pitch;
+      const int n   = s_n[fi] - 1;  // the last one, +inf, is never below a value
+      // four rows at a time, their searches side by side
+      for (int r = r_first; r < kRowsBin; r += 4 * r_step) {
+        T x[4];
+        int lo[4], len[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int64_t row = static_cast<int64_t>(tile) * kRowsBin + r + u * r_step;
+          x[u]   = r + u * r_step < kRowsBin && row < a.N ? X[row * a.F + f0 + fi] : T(0);
+          lo[u]  = 0;
+          len[u] = n;
+        }
+        for (int left = n; left > 0; left >>= 1) {
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            const int half = len[u] >> 1;
+            const bool go  = len[u] > 0 && prop[lo[u] + half] < x[u];
+            lo[u]          = go ? lo[u] + half + 1 : lo[u];
+            len[u]         = go ? len[u] - half - 1 : half;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (r + u * r_step < kRowsBin) s_bin[fi * kTilePitch + r + u * r_step] = static_cast<BinT>(lo[u]);
+      }
+    }
+    __syncthreads();
+    constexpr int kPer = 4 / sizeof(BinT);  // bins per word
+    for (int i = tid; i < nf * (kRowsBin / kPer); i += kWide) {
+      const int c = i / (kRowsBin / kPer), w = i - c * (kRowsBin / kPer);
+      *reinterpret_cast<uint32_t*>(out + static_cast<int64_t>(f0 + c) * st.pitch + static_cast<int64_t>(tile) * kRowsBin + w * kPer) =
+        *reinterpret_cast<const uint32_t*>(s_bin + c * kTilePitch + w * kPer);
+    }
+  }
+}
+
+// How a level's histograms are dealt to workgroups.
+struct LevelPlan {
+  int depth, level_first, n_nodes;
+  int built;        // nodes whose histogram is accumulated: one of every pair
+  int fw, n_fb;     // features per workgroup, blocks of them
+  int bw, n_bb;     // built nodes per workgroup, blocks of them
+  int chunks;       // row ranges
+  int chunk_rows;   // multiple of 4
+  bool last;
+};
+
+constexpr int kMaxFw = 8;
+
+// Which of a pair of siblings is accumulated (build_tree.h:92-104).
+__device__ __forceinline__ int built_of_pair(const I64Pair* __restrict__ node_sums, int level_first, int pair, int K)
+{
+  const int64_t hl = node_sums[static_cast<int64_t>(level_first + 2 * pair) * K].hess;
+  const int64_t hr = node_sums[static_cast<int64_t>(level_first + 2 * pair + 1) * K].hess;
+  return hl < hr ? 2 * pair : 2 * pair + 1;
+}
+
+// A packed word holds the sum of grads in its upper and the sum of hessians in its lower half. Rounded
+// hessians are not negative here and sum up to less than 2^32. The grads of all rows sum up to -down and +up
+// with up + down < 2^32, so a sum that left the 32 bits is recognised by lying outside these limits
+// (decode_grad).
+template <typename BinT>
+__global__ void __launch_bounds__(kWide)
+  mid_histogram_kernel(MidArgs a, MidTreeState st, LevelPlan p)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  unsigned long long* s_hist = reinterpret_cast<unsigned long long*>(smem_raw);  // [fw][bw][S]
+  __shared__ uint16_t s_slot[kMidMaxLevelNodes];                                 // node -> its histogram here, kNone: none
+  const int tid = threadIdx.x;
+  // ranges of rows vary fastest over the XCDs, so that one range's workgroups share an L2
+  const int lanes8 = p.chunks >= 8 ? 8 : 1;
+  const int low = blockIdx.x % lanes8;
+  int rest      = blockIdx.x / lanes8;
+  const int inner = p.n_fb * p.n_bb * a.K;
+  const int chunk = rest / inner * lanes8 + low;
+  rest            = rest % inner;
+  if (chunk >= p.chunks) return;
+  const int k = rest % a.K, fb = rest / a.K % p.n_fb, bb = rest / a.K / p.n_fb;
+  const int live = st.live[p.depth];
+  if (p.depth == 0 && blockIdx.x == 0 && tid == 0) {
+    __hip_atomic_store(a.answer + 1, (static_cast<unsigned long long>(a.tag) << 32) | static_cast<unsigned>(st.rp[a.F]),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(a.answer, (static_cast<unsigned long long>(a.tag) << 32) | st.q_stats[2], __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (live == 0) return;
+  const int f0 = fb * p.fw, nf = min(p.fw, a.F - f0);
+  const int b0 = bb * p.bw, nb = min(p.bw, p.built - b0);
+  for (int j = tid; j < p.n_nodes; j += kWide) {
+    int slot = kNone;
+    if (p.depth == 0)
+      slot = 0;
+    else if (j / 2 >= b0 && j / 2 < b0 + nb && built_of_pair(st.node_sums, p.level_first, j / 2, a.K) == j)
+      slot = j / 2 - b0;
+    s_slot[j] = static_cast<uint16_t>(slot);
+  }
+  for (int i = tid; i < p.fw * p.bw * a.S; i += kWide) s_hist[i] = 0;
+  __syncthreads();
+  const int r_begin = chunk * p.chunk_rows, r_end = min(a.N, r_begin + p.chunk_rows);
+  const BinT* const bins = static_cast<const BinT*>(st.bins) + static_cast<int64_t>(f0) * st.pitch;
+  const int2* const q    = st.q + static_cast<int64_t>(k) * st.pitch;
+  for (int r = r_begin + 4 * tid; r < r_end; r += 4 * kWide) {
+    const uint2 nd = *reinterpret_cast<const uint2*>(st.row_node + r);
+    const uint4 qa = *reinterpret_cast<const uint4*>(q + r), qb = *reinterpret_cast<const uint4*>(q + r + 2);
+    uint32_t w[kMaxFw][sizeof(BinT)];
+#pragma unroll
+    for (int i = 0; i < kMaxFw; i++)
+      if (i < nf) {
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(bins + static_cast<int64_t>(i) * st.pitch + r);
+#pragma unroll
+        for (int u = 0; u < static_cast<int>(sizeof(BinT)); u++) w[i][u] = src[u];
+      }
+    const unsigned node[4] = {nd.x & 0xffffu, nd.x >> 16, nd.y & 0xffffu, nd.y >> 16};
+    const uint32_t qg[4] = {qa.x, qa.z, qb.x, qb.z}, qh[4] = {qa.y, qa.w, qb.y, qb.w};
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      // (rows past the last one belong to no node; a row past the chunk's end is the next chunk's)
+      const int slot = node[u] != kNone && r + u < r_end ? s_slot[node[u]] : kNone;
+      if (slot != kNone) {
+        const unsigned long long word = (static_cast<unsigned long long>(qg[u]) << 32) | qh[u];
+        unsigned long long* h         = s_hist + slot * a.S;
+#pragma unroll
+        for (int i = 0; i < kMaxFw; i++)
+          if (i < nf) {
+            const unsigned bin = sizeof(BinT) == 1 ? (w[i][0] >> (8 * u)) & 0xffu
+                                                   : (w[i][(u >> 1) & (sizeof(BinT) - 1)] >> (16 * (u & 1))) & 0xffffu;
+            atomicAdd(h + static_cast<int64_t>(i) * p.bw * a.S + bin, word);
+          }
+      }
+    }
+  }
+  __syncthreads();
+  // the image of this range of rows: [built node][output][feature][bin]
+  unsigned long long* image =
+    st.images + ((static_cast<int64_t>(chunk) * p.built + b0) * a.K + k) * static_cast<int64_t>(a.F) * a.S + static_cast<int64_t>(f0) * a.S;
+  for (int b = 0; b < nb; b++)
+    for (int i = tid; i < nf * a.S; i += kWide) {
+      const int fi = i / a.S, bin = i - fi * a.S;
+      image[static_cast<int64_t>(b) * a.K * a.F * a.S + i] = s_hist[(fi * p.bw + b) * a.S + bin];
+    }
+}
+
+__device__ __forceinline__ int64_t decode_grad(uint32_t v, int64_t up, int64_t down)
+{
+  int64_t s = static_cast<int32_t>(v);
+  s += s < -down ? int64_t(1) << 32 : 0;
+  s -= s > up ? int64_t(1) << 32 : 0;
+  return s;
+}
+
+__global__ void __launch_bounds__(kScan)
+  mid_scan_kernel(MidArgs a, MidTreeState st, LevelPlan p)
+{
+  __shared__ I64Pair s_tot[2][kScan / 64];
+  __shared__ I64Pair s_carry[kMidMaxOutputs];
+  __shared__ double s_best[2][kScan / 64];
+  __shared__ unsigned s_bkey[2][kScan / 64];
+  const int f = blockIdx.x % a.F, pair = blockIdx.x / a.F;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  if (st.live[p.depth] == 0) return;
+  const bool usable = a.feature_set == nullptr || a.feature_set[f] != 0;
+  const int left    = 2 * pair;
+  const bool root   = p.depth == 0;
+  // the children of a node that did not split have no rows
+  if (!root && st.node_sums[static_cast<int64_t>(p.level_first + left) * a.K].hess <= 0) return;
+  const int node = root ? 0 : built_of_pair(st.node_sums, p.level_first, pair, a.K);
+  const int sib  = root ? 0 : node ^ 1;
+  if (!usable) {
+    if (tid == 0) {
+      st.cand[static_cast<int64_t>(node) * a.F + f] = SmallCand{0.0, 0u, 0};
+      if (!root) st.cand[static_cast<int64_t>(sib) * a.F + f] = SmallCand{0.0, 0u, 0};
+    }
+    return;
+  }
+  const int n_bins = st.counts[f], rp = st.rp[f];
+  const int64_t fs = static_cast<int64_t>(a.F) * a.S;
+  const int64_t up = static_cast<int64_t>(st.q_stats[0]), down = static_cast<int64_t>(st.q_stats[1]);
+  const double inv_g = st.scales[2], inv_h = st.scales[3];
+  const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
+  I64Pair* const hist         = st.hist[p.depth & 1];
+  const I64Pair* const parent = st.hist[(p.depth & 1) ^ 1] + static_cast<int64_t>(pair) * a.K * fs + static_cast<int64_t>(f) * a.S;
+  double best_n = 0.0, best_s = 0.0;
+  unsigned key_n = 0, key_s = 0;
+  for (int base = 0; base < n_bins; base += kScan) {
+    const int bin = base + tid;
+    const bool in = bin < n_bins;
+    double gain_n = 0.0, gain_s = 0.0;
+    bool dead_n = !in, dead_s = !in || root;
+    for (int k = 0; k < a.K; k++) {
+      I64Pair v{0, 0}, pv{0, 0};
+      if (in) {
+        const unsigned long long* img = st.images + (static_cast<int64_t>(pair) * a.K + k) * fs + static_cast<int64_t>(f) * a.S + bin;
+        const int64_t step = static_cast<int64_t>(p.built) * a.K * fs;
+        if (!root) pv = parent[k * fs + bin];
+        int c = 0;
+        for (; c + 8 <= p.chunks; c += 8) {
+          unsigned long long w[8];
+#pragma unroll
+          for (int u = 0; u < 8; u++) w[u] = img[(c + u) * step];
+#pragma unroll
+          for (int u = 0; u < 8; u++) {
+            v.grad += decode_grad(static_cast<uint32_t>(w[u] >> 32), up, down);
+            v.hess += static_cast<uint32_t>(w[u]);
+          }
+        }
+        for (; c < p.chunks; c++) {
+          const unsigned long long w = img[c * step];
+          v.grad += decode_grad(static_cast<uint32_t>(w >> 32), up, down);
+          v.hess += static_cast<uint32_t>(w);
+        }
+      }
+      int64_t g = wave_inclusive_sum(v.grad), h = wave_inclusive_sum(v.hess);
+      if (lane == 63) s_tot[k & 1][wave] = I64Pair{g, h};
+      __syncthreads();
+      if (base > 0) {
+        g += s_carry[k].grad;
+        h += s_carry[k].hess;
+      }
+      for (int w = 0; w < kScan / 64; w++) {
+        g += w < wave ? s_tot[k & 1][w].grad : 0;
+        h += w < wave ? s_tot[k & 1][w].hess : 0;
+      }
+      const I64Pair ns = st.node_sums[static_cast<int64_t>(p.level_first + node) * a.K + k];
+      if (in) {
+        const int64_t at = static_cast<int64_t>(k) * fs + static_cast<int64_t>(f) * a.S + bin;
+        hist[static_cast<int64_t>(node) * a.K * fs + at] = I64Pair{g, h};
+        add_gain(gain_n, dead_n, I64Pair{g, h}, ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
+        if (!root) {
+          const I64Pair ss = st.node_sums[static_cast<int64_t>(p.level_first + sib) * a.K + k];
+          const I64Pair sv{pv.grad - g, pv.hess - h};
+          hist[static_cast<int64_t>(sib) * a.K * fs + at] = sv;
+          add_gain(gain_s, dead_s, sv, ss, inv_g, inv_h, a.l1, reg, a.min_split_gain);
+        }
+      }
+      // the carry of a tile is read by the next one; a barrier of the next output lies between
+      if (base + kScan < n_bins) {
+        __syncthreads();
+        if (tid == kScan - 1) s_carry[k] = I64Pair{g, h};
+      }
+    }
+    const unsigned key = tie_key_of_bin(rp + bin);
+    const bool take_n = in && gain_n > 0 && (gain_n > best_n || (gain_n == best_n && key > key_n));
+    const bool take_s = in && gain_s > 0 && (gain_s > best_s || (gain_s == best_s && key > key_s));
+    best_n = take_n ? gain_n : best_n;
+    key_n  = take_n ? key : key_n;
+    best_s = take_s ? gain_s : best_s;
+    key_s  = take_s ? key : key_s;
+    if (base + kScan < n_bins) __syncthreads();
+  }
+  auto reduce = [&](double& best, unsigned& key) {
+    for (int off = 32; off >= 1; off >>= 1) {
+      const double g   = __shfl_xor(best, off, 64);
+      const unsigned o = static_cast<unsigned>(__shfl_xor(static_cast<int>(key), off, 64));
+      const bool take  = g > best || (g == best && o > key);
+      best = take ? g : best;
+      key  = take ? o : key;
+    }
+  };
+  reduce(best_n, key_n);
+  reduce(best_s, key_s);
+  if (lane == 0) {
+    s_best[0][wave] = best_n;
+    s_bkey[0][wave] = key_n;
+    s_best[1][wave] = best_s;
+    s_bkey[1][wave] = key_s;
+  }
+  __syncthreads();
+  if (tid < (root ? 1 : 2)) {
+    double best  = 0.0;
+    unsigned key = 0;
+    for (int w = 0; w < kScan / 64; w++) {
+      const bool take = s_best[tid][w] > best || (s_best[tid][w] == best && s_bkey[tid][w] > key);
+      best = take ? s_best[tid][w] : best;
+      key  = take ? s_bkey[tid][w] : key;
+    }
+    st.cand[static_cast<int64_t>(tid == 0 ? node : sib) * a.F + f] = SmallCand{best, key, key != 0 ? bin_of_tie_key(key) - rp : 0};
+  }
+}
+
+// The split of node j of the level by 1 << lanes_log lanes of a wave (`sub` numbers them), and, if `write`,
+// what follows from it: the node's outputs, its children's sums and leaf values. x: feature, -1 for a leaf;
+// y: its last bin that goes left. Lanes whose j is no node call it too (j < 0).
+__device__ __forceinline__ int2 decide_node(const MidArgs& a, const MidTreeState& st, const LevelPlan& p, int j, int sub,
+                                            int lanes, bool write)
+{
+  const int node = p.level_first + j;
+  double best    = 0.0;
+  unsigned key   = 0;
+  int ft = 0, rel = 0;
+  auto take = [&](double gain_o, unsigned key_o, int ft_o, int rel_o) {
+    const bool better = gain_o > best || (gain_o == best && key_o > key);
+    best = better ? gain_o : best;
+    key  = better ? key_o : key;
+    ft   = better ? ft_o : ft;
+    rel  = better ? rel_o : rel;
+  };
+  const bool here = j >= 0 && st.node_sums[static_cast<int64_t>(node) * a.K].hess > 0;
+  if (here) {
+    const SmallCand* c = st.cand + static_cast<int64_t>(j) * a.F;
+    for (int i = sub; i < a.F; i += lanes) {
+      const SmallCand o = c[i];
+      take(o.gain, o.key, i, o.rel);
+    }
+  }
+  for (int off = lanes >> 1; off >= 1; off >>= 1) {
+    const double g   = __shfl_xor(best, off, 64);
+    const unsigned o = static_cast<unsigned>(__shfl_xor(static_cast<int>(key), off, 64));
+    const int f_o = __shfl_xor(ft, off, 64), r_o = __shfl_xor(rel, off, 64);
+    take(g, o, f_o, r_o);
+  }
+  const bool splits = here && key != 0 && best > 1e-5;
+  if (write && j >= 0) {
+    const double inv_g = st.scales[2], inv_h = st.scales[3];
+    if (p.depth == 0)
+      for (int k = sub; k < a.K; k += lanes) {
+        const I64Pair ns = st.node_sums[k];
+        const double G = static_cast<double>(ns.grad) * inv_g, H = static_cast<double>(ns.hess) * inv_h;
+        a.leaf[k]      = calculate_leaf_value(G, H, a.l1, a.l2);
+        a.hessian[k]   = H;
+      }
+    if (splits) {
+      const int64_t fs = static_cast<int64_t>(a.F) * a.S;
+      const int lc = left_child(node), rc = right_child(node);
+      const I64Pair* h = st.hist[p.depth & 1] + static_cast<int64_t>(j) * a.K * fs + static_cast<int64_t>(ft) * a.S + rel;
+      for (int k = sub; k < a.K; k += lanes) {
+        const int64_t at = static_cast<int64_t>(node) * a.K + k, l = static_cast<int64_t>(lc) * a.K + k,
+                      r = static_cast<int64_t>(rc) * a.K + k;
+        const I64Pair ns = st.node_sums[at], ls = h[k * fs];
+        const I64Pair rs{ns.grad - ls.grad, ns.hess - ls.hess};
+        const double lg = static_cast<double>(ls.grad) * inv_g, lh = static_cast<double>(ls.hess) * inv_h;
+        const double rg = static_cast<double>(rs.grad) * inv_g, rh = static_cast<double>(rs.hess) * inv_h;
+        st.node_sums[l] = ls;
+        st.node_sums[r] = rs;
+        a.leaf[l]       = calculate_leaf_value(lg, lh, a.l1, a.l2);
+        a.leaf[r]       = calculate_leaf_value(rg, rh, a.l1, a.l2);
+        a.hessian[l]    = lh;
+        a.hessian[r]    = rh;
+      }
+      if (sub == 0) {
+        a.feature[node] = ft;
+        a.split[node]   = st.proposals[static_cast<int64_t>(ft) * a.S + rel];
+        a.gain[node]    = best;
+        st.live[p.depth + 1] = 1;
+      }
+    }
+  }
+  return make_int2(splits ? ft : -1, rel);
+}
+
+// Splits of a level of many nodes, one group of lanes per node.
+__global__ void __launch_bounds__(kScan)
+  mid_decide_kernel(MidArgs a, MidTreeState st, LevelPlan p, int lanes_log)
+{
+  if (st.live[p.depth] == 0) return;
+  const int lanes = 1 << lanes_log, sub = threadIdx.x & (lanes - 1);
+  const int j     = (blockIdx.x * kScan + static_cast<int>(threadIdx.x)) >> lanes_log;
+  const int2 sp   = decide_node(a, st, p, j < p.n_nodes ? j : -1, sub, lanes, true);
+  if (sub == 0 && j < p.n_nodes) st.splits[j] = sp;
+}
+
+// kDecided: mid_decide_kernel has run; otherwise every workgroup finds the splits for itself (few nodes: it
+// saves a launch) and the nodes' outputs are dealt to the workgroups.
+template <typename BinT, bool kDecided>
+__global__ void __launch_bounds__(kWide)
+  mid_apply_kernel(MidArgs a, MidTreeState st, LevelPlan p, int lanes_log)
+{
+  __shared__ int2 s_split[kMidMaxLevelNodes];
+  const int tid = threadIdx.x;
+  const int r   = blockIdx.x * kRowsApply + 4 * tid;
+  uint2 nd      = make_uint2(0xffffffffu, 0xffffffffu);
+  if (r < a.N) nd = *reinterpret_cast<const uint2*>(st.row_node + r);
+  if (st.live[p.depth] == 0) return;
+  if constexpr (kDecided) {
+    for (int j = tid; j < p.n_nodes; j += kWide) s_split[j] = st.splits[j];
+  } else {
+    const int lanes = 1 << lanes_log, sub = tid & (lanes - 1);
+    for (int j0 = 0; j0 < p.n_nodes; j0 += kWide >> lanes_log) {
+      const int j   = j0 + (tid >> lanes_log);
+      const int2 sp = decide_node(a, st, p, j < p.n_nodes ? j : -1, sub, lanes,
+                                  j % static_cast<int>(gridDim.x) == static_cast<int>(blockIdx.x));
+      if (sub == 0 && j < p.n_nodes) s_split[j] = sp;
+    }
+  }
+  __syncthreads();
+  if (r >= a.N) return;
+  const BinT* const bins = static_cast<const BinT*>(st.bins);
+  const unsigned node[4] = {nd.x & 0xffffu, nd.x >> 16, nd.y & 0xffffu, nd.y >> 16};
+  int2 sp[4];
+  int bin[4];
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    sp[u]  = node[u] != kNone ? s_split[node[u]] : make_int2(-1, 0);
+    bin[u] = sp[u].x >= 0 ? static_cast<int>(bins[static_cast<int64_t>(sp[u].x) * st.pitch + r + u]) : 0;
+  }
+  unsigned next[4];
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    next[u] = kNone;
+    if (node[u] != kNone) {
+      const unsigned child = 2 * node[u] + (bin[u] <= sp[u].y ? 0u : 1u);
+      if (sp[u].x >= 0) next[u] = child;
+      if (a.row_leaf != nullptr && (sp[u].x < 0 || p.last))
+        a.row_leaf[r + u] = sp[u].x < 0 ? p.level_first + static_cast<int>(node[u])
+                                        : 2 * p.level_first + 1 + static_cast<int>(child);
+    }
+  }
+  if (!p.last) *reinterpret_cast<uint2*>(st.row_node + r) = make_uint2(next[0] | next[1] << 16, next[2] | next[3] << 16);
+}
+
+// For the profiler: the rows of the level's nodes and of those that are accumulated.
+__global__ void __launch_bounds__(kScan) mid_count_kernel(MidArgs a, MidTreeState st, LevelPlan p, LevelMeta* total)
+{
+  const int r    = blockIdx.x * kScan + threadIdx.x;
+  const int node = r < a.N ? st.row_node[r] : kNone;
+  const bool has = node != kNone && st.live[p.depth] != 0;
+  const bool built = has && (p.depth == 0 || built_of_pair(st.node_sums, p.level_first, node >> 1, a.K) == node);
+  const unsigned long long all = __ballot(has), some = __ballot(built);
+  if ((threadIdx.x & 63) == 0) {
+    atomicAdd(reinterpret_cast<unsigned long long*>(&total->instances), static_cast<unsigned long long>(__popcll(all)));
+    atomicAdd(reinterpret_cast<unsigned long long*>(&total->built_instances), static_cast<unsigned long long>(__popcll(some)));
+  }
+  if (r < p.built && (p.depth == 0 || st.node_sums[static_cast<int64_t>(p.level_first + 2 * r) * a.K].hess > 0))
+    atomicAdd(reinterpret_cast<unsigned long long*>(&total->built_nodes), 1ULL);
+}
+
+// One level's plan. A workgroup of the histogram pass keeps fw features of bw nodes in the LDS; near the root
+// several features share the loads of a row, deeper a feature's nodes fill the LDS and then come in
+// blocks. Ranges of rows are cut until there is a workgroup for every CU or so, not below 1024 rows,
+// and only so many that their images (written here, read by the scan) stay within 64 MB.
+LevelPlan plan_level(int64_t N, int F, int K, int S, int depth, int max_depth)
+{
+  LevelPlan p;
+  p.depth       = depth;
+  p.level_first = static_cast<int>(level_begin(depth));
+  p.n_nodes     = 1 << depth;
+  p.built       = depth == 0 ? 1 : p.n_nodes / 2;
+  p.last        = depth + 1 == max_depth;
+  const int rows_of_lds = std::max<int>(1, static_cast<int>(kHistLds / (static_cast<size_t>(S) * 8)));
+  p.fw   = std::max(1, std::min({rows_of_lds / p.built, kMaxFw / 2, F}));
+  p.bw   = std::max(1, std::min(p.built, rows_of_lds / p.fw));
+  p.n_fb = (F + p.fw - 1) / p.fw;
+  p.n_bb = (p.built + p.bw - 1) / p.bw;
+  const int64_t inner = static_cast<int64_t>(p.n_fb) * p.n_bb * K;
+  const int64_t image = static_cast<int64_t>(p.built) * K * F * S * 8;
+  int64_t chunks      = std::max<int64_t>(1, 320 / inner);
+  chunks              = std::min(chunks, std::max<int64_t>(1, N / 1024));
+  chunks              = std::min(chunks, std::max<int64_t>(1, (int64_t(64) << 20) / image));
+  if (chunks > 8) chunks = chunks / 8 * 8;
+  p.chunks     = static_cast<int>(chunks);
+  p.chunk_rows = static_cast<int>(((N + chunks - 1) / chunks + 3) / 4 * 4);
+  return p;
+}
+
+}  // namespace
+
+int64_t mid_image_words(int64_t N, int F, int K, int max_depth, int S)
+{
+  int64_t most = 0;
+  for (int d = 0; d < max_depth; d++) {
+    const LevelPlan p = plan_level(N, F, K, S, d, max_depth);
+    most              = std::max(most, static_cast<int64_t>(p.chunks) * p.built * K * F * S);
+  }
+  return most;
+}
+
+// By size: measured against the other builder (one output unless stated; depth 8 and 256 samples): 20,000 x 100
+// 521 -> 189 us at depth 6, 250,000 x 43 755 -> 373, 500,000 x 50 861 -> 502, 1,000,000 x 30 996 -> 491,
+// 200,000 x 50 with 8 outputs 971 -> 577, 800,000 x 80 1067 -> 882, 2,000,000 x 40 1156 -> 1127. Every pass
+// reads all rows; where a level's nodes come in several blocks it does so once per block (700,000 x 40
+// with 512 samples at depth 10, eight blocks: 1418 -> 1501), hence the second line.
+bool mid_tree_fits(int64_t N, int F, int K, int max_depth, int S)
+{
+  if (max_depth < 1 || max_depth > kMidMaxDepth || K > kMidMaxOutputs || S > LBT_MAX_SPLIT_SAMPLES) return false;
+  // the chunk sums are added up by one workgroup, bins numbered with 26 bits (tie_key_of_bin), rows with 31
+  if (N * K > int64_t(4096) * 4096 || static_cast<int64_t>(F) * S >= (int64_t(1) << 26)) return false;
+  const int64_t level_hist = (int64_t(1) << (max_depth - 1)) * K * F * S * 16;
+  if (level_hist > (int64_t(768) << 20)) return false;
+  const int64_t values = N * F * K;
+  return values <= kMidMaxValues && values * plan_level(N, F, K, S, max_depth - 1, max_depth).n_bb <= 2 * kMidMaxValues;
+}
+
+template <typename T, typename BinT>
+static int queue_levels(hipStream_t stream, const MidTreeState& st, const MidArgs& a, LevelMeta* level_totals)
+{
+  int lanes_log = 0;
+  while (lanes_log < 6 && (1 << lanes_log) < a.F) lanes_log++;
+  for (int d = 0; d < a.max_depth; d++) {
+    const LevelPlan p = plan_level(a.N, a.F, a.K, a.S, d, a.max_depth);
+    {
+      ProfScope ps(LBT_PROF_HISTOGRAM, stream, 0.0, d);
+      static std::atomic<bool> attr_set[kMaxDevices] = {};
+      LBT_TRY(allow_dynamic_lds(mid_histogram_kernel<BinT>, kHistLds + 4096, attr_set));
+      const int lanes8    = p.chunks >= 8 ? 8 : 1;
+      const unsigned grid = static_cast<unsigned>((p.chunks + lanes8 - 1) / lanes8 * lanes8 * p.n_fb * p.n_bb * a.K);
+      mid_histogram_kernel<BinT><<<grid, kWide, static_cast<size_t>(p.fw) * p.bw * a.S * 8, stream>>>(a, st, p);
+    }
+    if (level_totals != nullptr)
+      mid_count_kernel<<<static_cast<unsigned>((a.N + kScan - 1) / kScan), kScan, 0, stream>>>(a, st, p, level_totals + d);
+    {
+      ProfScope ps(LBT_PROF_SCAN, stream);
+      mid_scan_kernel<<<static_cast<unsigned>(p.built) * a.F, kScan, 0, stream>>>(a, st, p);
+    }
+    ProfScope ps(LBT_PROF_POSITIONS, stream);
+    const unsigned grid = static_cast<unsigned>((a.N + kRowsApply - 1) / kRowsApply);
+    if (p.n_nodes <= 2 * (kWide >> lanes_log)) {
+      mid_apply_kernel<BinT, false><<<grid, kWide, 0, stream>>>(a, st, p, lanes_log);
+    } else {
+      mid_decide_kernel<<<((p.n_nodes << lanes_log) + kScan - 1) / kScan, kScan, 0, stream>>>(a, st, p, lanes_log);
+      mid_apply_kernel<BinT, true><<<grid, kWide, 0, stream>>>(a, st, p, lanes_log);
+    }
+  }
+  LBT_HIP(hipGetLastError());
+  return LBT_OK;
+}
+
+template <typename T>
+int mid_tree_build(hipStream_t stream, const MidTreeState& st, const T* X, int64_t row_offset, int64_t N, int F, int K,
+                   const double* g, const double* h, const uint8_t* feature_set, const lbt_build_params& prm,
+                   double* leaf, int32_t* feature, double* split, double* gain, double* hessian, int32_t* row_leaf,
+                   int32_t* n_bins, LevelMeta* level_totals, bool* taken)
+{
+  *taken = false;
+  DeviceAnswer answer;
+  LBT_TRY(answer.open());
+  MidArgs a;
+  a.N = static_cast<int>(N); a.F = F; a.K = K; a.S = prm.split_samples;
+  a.row_offset = row_offset; a.seed = prm.seed; a.dataset_rows = prm.dataset_rows;
+  a.g = g; a.h = h;
+  a.m       = static_cast<int>((N * K + 4095) / 4096);
+  a.chunk_a = prm.abs_sum_chunks != nullptr ? prm.abs_sum_chunks : st.chunk_sums;
+  a.chunk_b = a.chunk_a + a.m;
+  a.feature_set = feature_set;
+  a.l1 = prm.l1_regularization; a.l2 = prm.l2_regularization; a.min_split_gain = prm.min_split_gain;
+  a.max_nodes = prm.max_nodes; a.max_depth = prm.max_depth;
+  a.leaf = leaf; a.feature = feature; a.split = split; a.gain = gain; a.hessian = hessian; a.row_leaf = row_leaf;
+  a.answer = answer.words; a.tag = answer.tag;
+  int P = 1;
+  while (P < a.S) P <<= 1;
+  {
+    ProfScope ps(LBT_PROF_PROPOSALS, stream);
+    static std::atomic<bool> attr_set[kMaxDevices] = {};
+    LBT_TRY(allow_dynamic_lds(mid_prologue_kernel<T>, 64 * 1024, attr_set));
+    const int sum_groups  = prm.abs_sum_chunks != nullptr ? 0 : (a.m + 3) / 4;
+    const int64_t clear   = std::max<int64_t>(static_cast<int64_t>(prm.max_nodes) * K, st.pitch / 4);
+    const int clearers    = static_cast<int>(std::min<int64_t>((clear + kWide - 1) / kWide, 128));
+    const size_t lds      = std::max<size_t>(static_cast<size_t>(P) * kProposalScratch<T>, 2 * kWide * sizeof(double));
+    mid_prologue_kernel<T><<<F + sum_groups + clearers, kWide, lds, stream>>>(X, a, st, P, sum_groups);
+  }
+  {
+    ProfScope ps(LBT_PROF_BINNING, stream);
+    BinPlan p;
+    p.quant_groups = static_cast<int>((N * K + kQuantPer - 1) / kQuantPer);
+    // features of a workgroup: their proposals take at most half of the 64 KB
+    p.fb     = std::max(1, std::min<int>(F, std::min<int>(32, static_cast<int>(40 * 1024 / ((a.S | 1) * sizeof(T))))));
+    p.fb_log = 0;
+    while ((1 << p.fb_log) < p.fb) p.fb_log++;
+    p.n_fb       = (F + p.fb - 1) / p.fb;
+    const int tiles = static_cast<int>((N + kRowsBin - 1) / kRowsBin);
+    p.row_groups = std::max(1, std::min(tiles, 1024 / p.n_fb));
+    const size_t lds = std::max<size_t>(
+      static_cast<size_t>(p.fb) * ((a.S | 1) * sizeof(T) + 4 + (kRowsBin + 4) * st.bin_bytes) + 16, 2 * kWide * sizeof(double));
+    static std::atomic<bool> attr_set[2][kMaxDevices] = {};
+    const unsigned grid = static_cast<unsigned>(p.quant_groups + p.n_fb * p.row_groups);
+    if (st.bin_bytes == 1) {
+      LBT_TRY((allow_dynamic_lds(mid_bin_kernel<T, uint8_t>, 80 * 1024, attr_set[0])));
+      mid_bin_kernel<T, uint8_t><<<grid, kWide, lds, stream>>>(X, a, st, p);
+    } else {
+      LBT_TRY((allow_dynamic_lds(mid_bin_kernel<T, uint16_t>, 80 * 1024, attr_set[1])));
+      mid_bin_kernel<T, uint16_t><<<grid, kWide, lds, stream>>>(X, a, st, p);
+    }
+  }
+  if (st.bin_bytes == 1)
+    LBT_TRY((queue_levels<T, uint8_t>(stream, st, a, level_totals)));
+  else
+    LBT_TRY((queue_levels<T, uint16_t>(stream, st, a, level_totals)));
+  unsigned flags = 0;
+  LBT_TRY(answer.wait(stream, &flags, n_bins));
+  *taken = flags == 0;
+  return LBT_OK;
+}
+
+template int mid_tree_build<float>(hipStream_t, const MidTreeState&, const float*, int64_t, int64_t, int, int,
+                                   const double*, const double*, const uint8_t*, const lbt_build_params&, double*,
+                                   int32_t*, double*, double*, double*, int32_t*, int32_t*, LevelMeta*, bool*);
+template int mid_tree_build<double>(hipStream_t, const MidTreeState&, const double*, int64_t, int64_t, int, int,
+                                    const double*, const double*, const uint8_t*, const lbt_build_params&, double*,
+                                    int32_t*, double*, double*, double*, int32_t*, int32_t*, LevelMeta*, bool*);
+
+}  // namespace lbt

@@ -32,38 +32,7 @@ namespace {
 
 constexpr int kPrologueThreads = 1024;
 constexpr int kNone            = 0xffff;  // node_of_pos of a row whose node did not split
-constexpr int kRankSortMax     = 512;     // split samples sorted by counting smaller ones; more: bitonic
 constexpr int kQuantChunks     = 8;       // chunks of 4096 entries the quantiser's workgroup takes
-
-// Inclusive sums over a wave, 32 bits (see wave_inclusive_sum)
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ int dpp_take32(int v)
-{
-  return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xf, true);
-}
-__device__ __forceinline__ int wave_inclusive_sum32(int v)
-{
-  v += dpp_take32<0x111, 0xf>(v);
-  v += dpp_take32<0x112, 0xf>(v);
-  v += dpp_take32<0x114, 0xf>(v);
-  v += dpp_take32<0x118, 0xf>(v);
-  v += dpp_take32<0x142, 0xa>(v);
-  v += dpp_take32<0x143, 0xc>(v);
-  return v;
-}
-
-// Sum of the threads before this one; all threads of the workgroup call it. s_wave: one int per wave.
-template <int kT>
-__device__ inline int block_exclusive_sum32(int v, int* s_wave)
-{
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int incl = wave_inclusive_sum32(v);
-  if (lane == 63) s_wave[wave] = incl;
-  __syncthreads();
-  int before = 0;
-  for (int w = 0; w < kT / 64; w++) before += w < wave ? s_wave[w] : 0;
-  return before + incl - v;
-}
 
 struct PrologueArgs {
   int64_t row_offset;
@@ -81,7 +50,7 @@ struct PrologueArgs {
   double* split;
   double* gain;
   double* hessian;
-  uint32_t* answer;  // pinned host memory: what the host has to know, tagged with `tag`
+  unsigned long long* answer;  // pinned host memory (see DeviceAnswer)
   uint32_t tag;
 };
 
@@ -160,16 +129,8 @@ __device__ inline void small_quantise(const PrologueArgs& a, const SmallTreeStat
   for (int e = threadIdx.x; e < n; e += kPrologueThreads) {
     const int row = a.K == 1 ? e : e / a.K, k = a.K == 1 ? 0 : e - row * a.K;
     const double grad = a.g[e], hess = a.h[e];
-    uint32_t x = minstd_seed(static_cast<uint32_t>(
-      static_cast<uint64_t>(gpair_seed(static_cast<int64_t>(a.seed), row + a.row_offset, static_cast<int64_t>(k)))));
-    const double scaled_grad    = grad * sg;
-    const double scaled_hess    = hess * sh;
-    const double grad_remainder = scaled_grad - floor(scaled_grad);
-    const double hess_remainder = scaled_hess - floor(scaled_hess);
-    x = minstd_next(x);
-    const int64_t qg = static_cast<int64_t>(floor(scaled_grad) + static_cast<double>(uniform01(x) < grad_remainder));
-    x = minstd_next(x);
-    const int64_t qh = static_cast<int64_t>(floor(scaled_hess) + static_cast<double>(uniform01(x) < hess_remainder));
+    int64_t qg, qh;
+    quantise_pair(grad, hess, sg, sh, static_cast<int64_t>(a.seed), row + a.row_offset, k, &qg, &qh);
     if (qg > 2147483647LL || qg < -2147483647LL || qh > 2147483647LL || qh < -2147483647LL) flags |= 2u;
     if (qh <= 0 && (qg != 0 || qh != 0)) flags |= 1u;
     st.qgh[e] = make_int2(static_cast<int>(qg), static_cast<int>(qh));
@@ -192,7 +153,8 @@ __device__ inline void small_quantise(const PrologueArgs& a, const SmallTreeStat
   if (flags != 0) atomicOr(&s_flags, flags);
   __syncthreads();
   if (threadIdx.x == 0)
-    __hip_atomic_store(a.answer, (a.tag << 2) | s_flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(a.answer, (static_cast<unsigned long long>(a.tag) << 32) | s_flags, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
   if (threadIdx.x < 4) st.scales[threadIdx.x] = s_scale[threadIdx.x];
   for (int k = threadIdx.x; k < a.K; k += kPrologueThreads) {
     const I64Pair ns{static_cast<int64_t>(s_sum[k]), static_cast<int64_t>(s_sum[a.K + k])};
@@ -216,90 +178,17 @@ template <typename T>
 __device__ inline void small_feature(const T* __restrict__ X, const PrologueArgs& a, const SmallTreeState& st, int f,
                                      unsigned char* smem)
 {
-  using Key = typename KeyOf<T>::type;
   int P = 1;
   while (P < a.S) P <<= 1;
-  // [P] unsorted keys, [P] sorted keys, [P] ranks, then bin counts / places
-  Key* s_in      = reinterpret_cast<Key*>(smem);
-  Key* s_key     = s_in + P;
-  int* s_rank    = reinterpret_cast<int*>(s_key + P);
-  int* s_count   = s_rank + P;                                       // [P + 1]
-  uint32_t* s_order = reinterpret_cast<uint32_t*>(s_count + P + 4);  // [N]
+  // the proposals' scratch, then counts (places) of the bins and the rows in order
+  int* s_count      = reinterpret_cast<int*>(smem + static_cast<size_t>(P) * kProposalScratch<T>);  // [P + 1]
+  uint32_t* s_order = reinterpret_cast<uint32_t*>(s_count + P + 4);                                  // [N]
   __shared__ int s_wave[kPrologueThreads / 64];
-  __shared__ int s_n;
   const int tid = threadIdx.x;
-  // the sampled rows (build_tree.cu:882-898)
-  for (int i = tid; i < P; i += kPrologueThreads) {
-    Key key = ~Key(0);
-    if (i < a.S) {
-      uint32_t x = minstd_seed(static_cast<uint32_t>(a.seed));
-      x          = minstd_next(minstd_discard(x, static_cast<uint64_t>(i)));
-      const double u    = uniform01(x);
-      const double b    = static_cast<double>(a.dataset_rows - 1) + 1.0;
-      const int64_t row = static_cast<int64_t>((u * (b - 0.0)) + 0.0) - a.row_offset;
-      key               = to_key(row >= 0 && row < a.N ? X[row * a.F + f] : T(0));
-    }
-    s_in[i]   = key;
-    s_rank[i] = 0;
-  }
-  __syncthreads();
-  if (P <= kRankSortMax) {
-    // a sample's place is the number of samples before it; several threads share the counting
-    const int parts = kPrologueThreads / P, i = tid & (P - 1), part = tid / P;
-    const int per = (a.S + parts - 1) / parts, j0 = part * per, j1 = min(a.S, j0 + per);
-    if (i < a.S) {
-      const Key mine = s_in[i];
-      int before     = 0;
-      for (int j = j0; j < j1; j++) {
-        const Key o = s_in[j];
-        before += (o < mine || (o == mine && j < i)) ? 1 : 0;
-      }
-      atomicAdd(&s_rank[i], before);
-    }
-    __syncthreads();
-    for (int j = tid; j < a.S; j += kPrologueThreads) s_key[s_rank[j]] = s_in[j];
-    __syncthreads();
-  } else {
-    for (int i = tid; i < P; i += kPrologueThreads) s_key[i] = s_in[i];
-    __syncthreads();
-    for (int size = 2; size <= P; size <<= 1)
-      for (int stride = size >> 1; stride > 0; stride >>= 1) {
-        for (int i = tid; i < P / 2; i += kPrologueThreads) {
-          const int lo = 2 * i - (i & (stride - 1)), hi = lo + stride;
-          const bool up = (lo & size) == 0;
-          const Key x = s_key[lo], y = s_key[hi];
-          if ((x > y) == up) {
-            s_key[lo] = y;
-            s_key[hi] = x;
-          }
-        }
-        __syncthreads();
-      }
-  }
-  // drop values equal to their predecessor; two consecutive samples per thread (S <= 2048)
-  T* s_prop = reinterpret_cast<T*>(s_in);
-  T v[2]    = {T(0), T(0)};
-  bool keep[2];
-  int mine = 0;
-#pragma unroll
-  for (int u = 0; u < 2; u++) {
-    const int i = 2 * tid + u;
-    keep[u]     = false;
-    if (i < a.S) {
-      v[u]    = from_key(s_key[i]);
-      keep[u] = i == 0 || !(v[u] == from_key(s_key[i - 1]));
-    }
-    mine += keep[u] ? 1 : 0;
-  }
-  int at = block_exclusive_sum32<kPrologueThreads>(mine, s_wave);
-  if (tid == kPrologueThreads - 1) s_n = at + mine;
-#pragma unroll
-  for (int u = 0; u < 2; u++)
-    if (keep[u]) s_prop[at++] = v[u];
   for (int i = tid; i <= P; i += kPrologueThreads) s_count[i] = 0;
-  __syncthreads();
-  const int n = s_n;
-  // the last proposal becomes +inf (build_tree.cu:953-956)
+  const SampleSpec sp{a.S, a.seed, a.dataset_rows, a.row_offset, a.N, a.F};
+  const T* s_prop = nullptr;
+  const int n     = feature_proposals<T, kPrologueThreads>(X, sp, f, P, smem, s_wave, &s_prop);
   for (int i = tid; i < n; i += kPrologueThreads)
     st.proposals[static_cast<int64_t>(f) * a.S + i] =
       i == n - 1 ? std::numeric_limits<double>::infinity() : static_cast<double>(s_prop[i]);
@@ -381,7 +270,7 @@ struct LevelArgs {
   int level_first;  // first node of the level; its node j is level_first + j
   int n_nodes;
   bool last;        // no further level follows
-  unsigned long long* n_bins;  // pinned host memory: the number of all bins, tagged like PrologueArgs::answer
+  unsigned long long* n_bins;  // pinned host memory: the number of all bins (see DeviceAnswer)
   uint32_t tag;
   const uint8_t* feature_set;
   double l1, l2, min_split_gain;
@@ -424,12 +313,6 @@ __device__ __forceinline__ unsigned tie_key(int rp, int bin, int next)
 {
   const int pick = min((rp + bin) | 511, rp + next - 1);
   return (static_cast<unsigned>(pick & 511) << 11 | static_cast<unsigned>(2047 - (pick - rp))) + 1u;
-}
-
-// The same rule between bins of different features (fewer than 2^26 bins: small_tree_fits).
-__device__ __forceinline__ unsigned tie_key_of_bin(int bin)
-{
-  return (static_cast<unsigned>(bin & 511) << 17 | static_cast<unsigned>(0x1ffff - (bin >> 9))) + 1u;
 }
 
 // kT threads take kE consecutive places of the order each (kT * kE >= N). What a place needs of its row
@@ -890,6 +773,21 @@ __global__ void __launch_bounds__(kT)
     for (int i = tid; i < n; i += kT) st.node_of_pos[s0 + i] = static_cast<uint16_t>(2 * j + (i < lefts ? 0 : 1));
 }
 
+// For the profiler: what the histograms of the level would be built from.
+__global__ void __launch_bounds__(256) small_count_kernel(SmallTreeState st, LevelArgs a, LevelMeta* total)
+{
+  for (int j = threadIdx.x; j < a.n_nodes; j += 256) {
+    const int node = a.level_first + j, n = st.seg[node].y;
+    if (n == 0 || st.live[a.depth] == 0) continue;
+    const bool built = compute_histogram_bin(node, st.node_sums, a.K, node != 0);
+    atomicAdd(reinterpret_cast<unsigned long long*>(&total->instances), static_cast<unsigned long long>(n));
+    if (built) {
+      atomicAdd(reinterpret_cast<unsigned long long*>(&total->built_instances), static_cast<unsigned long long>(n));
+      atomicAdd(reinterpret_cast<unsigned long long*>(&total->built_nodes), 1ULL);
+    }
+  }
+}
+
 template <int kT, int kE, bool kSingle>
 int launch_small_scan_as(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a)
 {
@@ -922,16 +820,11 @@ template <typename T>
 int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, int64_t row_offset, int64_t N, int F,
                      int K, const double* g, const double* h, const uint8_t* feature_set, const lbt_build_params& prm,
                      double* leaf, int32_t* feature, double* split, double* gain, double* hessian, int32_t* row_leaf,
-                     int32_t* n_bins, bool* taken)
+                     int32_t* n_bins, LevelMeta* level_totals, bool* taken)
 {
   *taken = false;
-  ThreadResources* here = nullptr;
-  LBT_TRY(thread_resources_here(&here));
-  if (here->answer == nullptr) {
-    LBT_HIP(hipHostMalloc(reinterpret_cast<void**>(&here->answer), 64, hipHostMallocDefault));
-    here->answer[0] = here->answer[2] = here->answer[3] = 0;
-  }
-  const uint32_t tag = here->answer_tag = (here->answer_tag + 1) & 0x3fffffffu;
+  DeviceAnswer answer;
+  LBT_TRY(answer.open());
   PrologueArgs pa;
   pa.row_offset = row_offset;
   pa.N = static_cast<int>(N); pa.F = F; pa.K = K; pa.S = prm.split_samples;
@@ -942,15 +835,15 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
   pa.max_nodes = prm.max_nodes;
   pa.max_depth = prm.max_depth;
   pa.leaf = leaf; pa.feature = feature; pa.split = split; pa.gain = gain; pa.hessian = hessian;
-  pa.answer = here->answer;
-  pa.tag    = tag;
+  pa.answer = answer.words;
+  pa.tag    = answer.tag;
   {
     ProfScope ps(LBT_PROF_PROPOSALS, stream);
     static std::atomic<bool> attr_set[kMaxDevices] = {};
     LBT_TRY(allow_dynamic_lds(small_prologue_kernel<T>, 120 * 1024, attr_set));
     int P = 1;
     while (P < prm.split_samples) P <<= 1;
-    const size_t feature_lds = static_cast<size_t>(P) * (2 * sizeof(T) + 8) + 16 + N * 4 + 16;
+    const size_t feature_lds = static_cast<size_t>(P) * (kProposalScratch<T> + 4) + 16 + N * 4 + 16;
     const size_t quant_lds   = (2048 + 2 * kQuantChunks + 4 + 2 * static_cast<size_t>(K)) * 8;
     const int64_t clear      = std::max<int64_t>(static_cast<int64_t>(prm.max_nodes) * K, N);
     const int clearers       = static_cast<int>(std::min<int64_t>((clear + kPrologueThreads - 1) / kPrologueThreads, 64));
@@ -959,8 +852,8 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
   LevelArgs a;
   a.N = static_cast<int>(N); a.F = F; a.K = K; a.S = prm.split_samples;
   a.feature_set = feature_set;
-  a.n_bins = reinterpret_cast<unsigned long long*>(here->answer + 2);
-  a.tag    = tag;
+  a.n_bins = answer.words + 1;
+  a.tag    = answer.tag;
   a.l1 = prm.l1_regularization; a.l2 = prm.l2_regularization; a.min_split_gain = prm.min_split_gain;
   for (int d = 0; d < prm.max_depth; d++) {
     a.depth       = d;
@@ -978,6 +871,7 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
       else
         LBT_TRY((launch_small_scan<1024, 8>(stream, st, a)));
     }
+    if (level_totals != nullptr) small_count_kernel<<<1, 256, 0, stream>>>(st, a, level_totals + d);
     ProfScope ps(LBT_PROF_SPLIT, stream);
     // few nodes of many rows near the root, many small ones below
     if ((N >> d) > 1024)
@@ -988,37 +882,17 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
       small_apply_kernel<64><<<a.n_nodes, 64, 0, stream>>>(st, a, leaf, feature, split, gain, hessian, row_leaf);
   }
   LBT_HIP(hipGetLastError());
-  // What the prologue found, and the number of bins if it is asked for, written to pinned memory long
-  // before the levels above are done. Should they not arrive (the stream has failed), the stream's
-  // own state ends the wait.
-  volatile uint32_t* const answer         = here->answer;
-  volatile unsigned long long* const bins = reinterpret_cast<unsigned long long*>(here->answer + 2);
-  auto arrived = [&]() { return (*answer >> 2) == tag && (n_bins == nullptr || (*bins >> 32) == tag); };
-  for (int64_t spin = 1; !arrived(); spin++) {
-    if (spin % 16384 != 0) continue;
-    const hipError_t e = hipStreamQuery(stream);
-    if (e == hipErrorNotReady) continue;
-    LBT_HIP(e);
-    if (arrived()) break;
-    set_error("the tree builder's kernels did not report");
-    return LBT_ERR_HIP;
-  }
-  const uint32_t got = *answer;
-  if (n_bins != nullptr) *n_bins = static_cast<int32_t>(*bins & 0xffffffffULL);
-  if ((got & 2u) != 0) {
-    set_error("a quantised gradient or hessian reaches 2^31 and does not fit the packed 32-bit form: one entry "
-              "holds the whole absolute sum and was rounded up");
-    return LBT_ERR_UNSUPPORTED;
-  }
-  *taken = (got & 1u) == 0;
+  unsigned flags = 0;
+  LBT_TRY(answer.wait(stream, &flags, n_bins));
+  *taken = flags == 0;
   return LBT_OK;
 }
 
 template int small_tree_build<float>(hipStream_t, const SmallTreeState&, const float*, int64_t, int64_t, int, int,
                                      const double*, const double*, const uint8_t*, const lbt_build_params&, double*,
-                                     int32_t*, double*, double*, double*, int32_t*, int32_t*, bool*);
+                                     int32_t*, double*, double*, double*, int32_t*, int32_t*, LevelMeta*, bool*);
 template int small_tree_build<double>(hipStream_t, const SmallTreeState&, const double*, int64_t, int64_t, int, int,
                                       const double*, const double*, const uint8_t*, const lbt_build_params&, double*,
-                                      int32_t*, double*, double*, double*, int32_t*, int32_t*, bool*);
+                                      int32_t*, double*, double*, double*, int32_t*, int32_t*, LevelMeta*, bool*);
 
 }  // namespace lbt

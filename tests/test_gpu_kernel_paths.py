@@ -76,7 +76,7 @@ def _assert_tree(got, cr):
     (4097, 300, 1, 7, 256, np.float32),
     (8191, 6, 4, 12, 1024, np.float64),
     (8192, 9, 4, 8, 256, np.float32),      # the most rows and entries the few-rows builder takes
-    (8193, 9, 1, 8, 256, np.float32),
+    (8193, 9, 1, 8, 256, np.float32),      # one row more
     (8192, 3, 5, 4, 64, np.float32),       # more entries than it takes
     (500, 4, 1, 14, 64, np.float32),       # deeper than it takes
 ])
@@ -151,3 +151,71 @@ def test_few_rows_takes_the_chunk_sums_of_the_gradient_pass():
     b = ops.build_tree(X, g, h, max_depth=5, split_samples=64, seed=4, abs_sum_chunks=sums)
     for name in ("leaf_value", "feature", "split_value", "gain", "hessian"):
         assert torch.equal(getattr(a, name), getattr(b, name)), name
+
+
+@pytest.mark.parametrize("n,f,k,depth,s,dtype,options", [
+    (8200, 4, 1, 1, 256, np.float32, {}),
+    (9000, 33, 1, 6, 256, np.float32, {"features": 0.7}),
+    (8448, 7, 1, 8, 64, np.float64, {}),                    # rows a multiple of the binning tile
+    (20001, 32, 1, 7, 256, np.float32, {"zeros": True}),
+    (16385, 5, 1, 9, 512, np.float32, {"l1": True}),        # two-byte bins, two tiles of bins in the scan
+    (12000, 3, 1, 10, 2048, np.float64, {}),                # most bins, deepest tree, blocks of nodes
+    (9001, 70, 3, 5, 100, np.float32, {"features": 0.5}),   # several outputs
+    (8300, 11, 16, 4, 300, np.float64, {"l1": True}),
+    (40000, 130, 1, 5, 256, np.float32, {}),
+    (8193, 6, 2, 10, 256, np.float32, {"zeros": True}),
+    (9000, 6, 1, 11, 64, np.float32, {}),                   # deeper than the builder for medium sizes takes
+])
+def test_medium_sizes(n, f, k, depth, s, dtype, options):
+    """The builder that leaves rows in their own order, at the edges of its tiles and plans."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + 7 * f + depth)
+    X = rs.randn(n, f).astype(dtype)
+    if f > 3:
+        X[:, 1] = rs.randint(0, 3, n)
+        X[:, 2] = X[:, 0]
+        X[:, 3] = np.exp(2.0 * rs.randn(n))
+    g = rs.randn(n, k) + X[:, :1]
+    h = rs.rand(n, k) + 0.1
+    if options.get("zeros"):
+        h[::3] = 0.0
+        g[::3] = 0.0
+    fs = rs.rand(f) < options["features"] if "features" in options else None
+    kw = dict(l1=0.05, l2=0.5, min_split_gain=1e-3) if options.get("l1") else {}
+    kw2 = dict(l1_regularization=0.05, l2_regularization=0.5, min_split_gain=1e-3) if kw else {}
+    cr = orc.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=n, feature_set=fs, **kw)
+    for wait in (True, False):
+        got = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=n, feature_set=fs, row_leaf=True,
+                             wait=wait, **kw2)
+        torch.cuda.synchronize()
+        _assert_tree(got, cr)
+        gu.check_row_leaf(got, X)
+
+
+@pytest.mark.parametrize("case", ["one_sign", "one_row", "negative_hessian", "all_zero"])
+def test_medium_sizes_special_gradients(case):
+    """Sums at the edge of the packed 32 bits (all gradients of one sign in one bin; nearly the whole mass in one
+    row) and data that the other builder has to take."""
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(6)
+    n, f = 30000, 5
+    X = rs.randn(n, f).astype(np.float32)
+    X[:, 0] = (rs.rand(n) < 1e-3).astype(np.float32)  # nearly all rows in one bin
+    g, h = rs.rand(n, 1) + 0.1, rs.rand(n, 1) + 0.1
+    if case == "one_row":
+        g = rs.randn(n, 1) * 1e-6
+        g[4321] = -5.0
+        h = np.full((n, 1), 1e-3)
+        h[17] = 900.0
+    elif case == "negative_hessian":
+        h[::7] *= -1.0
+    elif case == "all_zero":
+        g[:], h[:] = 0.0, 0.0
+    for sign in (1.0, -1.0):
+        cr = orc.build_tree(X, sign * g, h, max_depth=4, split_samples=64, seed=5)
+        _assert_tree(ops.build_tree(X, sign * g, h, max_depth=4, split_samples=64, seed=5), cr)
