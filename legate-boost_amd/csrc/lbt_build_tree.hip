@@ -1453,6 +1453,11 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     st.bins       = ar.take<char>(static_cast<size_t>(F) * st.pitch * st.bin_bytes);
     st.props      = ar.take<char>(fs * elem);
     st.proposals  = ar.take<double>(fs);
+    st.cells      = 128;  // eight cells per proposal
+    while (st.cells < 8 * S && st.cells < kMaxCells) st.cells *= 2;
+    st.tables     = ar.take<uint32_t>(static_cast<size_t>(F) * st.cells / 16);
+    st.map_x      = ar.take<char>(2 * static_cast<size_t>(F) * elem);
+    st.map_t      = ar.take<float>(2 * static_cast<size_t>(F));
     st.counts     = ar.take<int32_t>(F);
     st.rp         = ar.take<int32_t>(F + 1);
     st.chunk_sums = ar.take<double>(2 * ((N * K + 4095) / 4096));

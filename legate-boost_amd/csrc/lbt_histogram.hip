@@ -34,6 +34,7 @@
 //     of the record and walks rows; a tile is one pass of the workgroup (a few
 //     rows per lane); the loads of the next tile and the row indices of the one
 //     after are issued before the current tile is processed.
+#include "lbt_device.h"
 #include "lbt_internal.h"
 
 #include <algorithm>
@@ -253,53 +254,6 @@ __global__ void __launch_bounds__(kPlanThreads)
   }
 }
 
-// The cell of a value. Equal cells over the range of the proposals serve evenly spread columns only:
-// with a long tail (lognormal columns) most proposals crowd into a few of them, the table's start then
-// lies far before the bin and nearly every wave has a lane that walks on (4M x 100 lognormal values: 1.74 ms
-// where uniform ones took 0.54). So the axis is bent first:
-//   d = (x - centre) * scale,  g = sign(d) * log2(1 + |d|) in its piecewise linear form
-// (the bits of the float 1 + |d| read as an integer), which is exactly linear for |d| <= 1 and
-// logarithmic beyond; build_cells_kernel picks centre and scale per feature, a scale that keeps the
-// whole range inside |d| <= 1 being one of its choices. The cell is then g * invw + nlo clamped to
-// [0, cmax]. Every step is monotone non-decreasing in x (a fused multiply-add with a non-negative factor
-// rounds once, and rounding, the bit pattern of positive floats and clamping keep order), and table
-// construction and lookup share this function, which is all that exactness needs. NaN goes to cell 0.
-template <typename T>
-struct CellMap {
-  T scale, shift;      // d = x * scale + shift
-  float invw, nlo;     // t = g * invw + nlo
-};
-__device__ __forceinline__ float bend(float d)
-{
-  const int k = __float_as_int(fabsf(d) + 1.0f) - 0x3f800000;
-  return copysignf(static_cast<float>(k), d);
-}
-template <typename T>
-__device__ __forceinline__ float bend_axis(T x, T scale, T shift)
-{
-  // the median of (x, -max, max) clamps infinities; with a NaN operand it is the minimum of the others
-  if constexpr (sizeof(T) == 4) {
-    constexpr float kMax = std::numeric_limits<float>::max();
-    return bend(fmaf(__builtin_amdgcn_fmed3f(x, -kMax, kMax), scale, shift));
-  } else {
-    constexpr double kMax = std::numeric_limits<double>::max();
-    const double v        = x > -kMax ? x : -kMax;  // false for NaN
-    return bend(static_cast<float>(fma(v, scale, shift)));
-  }
-}
-template <typename T>
-__device__ __forceinline__ int cell_of(T x, T scale, T shift, float invw, float nlo, float cmax)
-{
-  return static_cast<int>(__builtin_amdgcn_fmed3f(fmaf(bend_axis(x, scale, shift), invw, nlo), 0.0f, cmax));
-}
-// Without the bend, for features whose proposals spread evenly: six vector instructions less per value,
-// which the binning pass feels (4M x 100 uniform values: 0.60 ms bent, 0.54 straight).
-template <typename T>
-__device__ __forceinline__ int straight_cell_of(T x, T a, T b, float cmax)
-{
-  return static_cast<int>(__builtin_amdgcn_fmed3f(static_cast<float>(fma(x, a, b)), 0.0f, cmax));
-}
-
 // Lookup table of a feature: the value range is cut into C fine cells (many more than there
 // are proposals) and the table holds one 32-bit word per 16 cells: the number of proposals in
 // all earlier words (high half) and a bit per cell of the word that holds at least one
@@ -310,80 +264,6 @@ __device__ __forceinline__ int straight_cell_of(T x, T a, T b, float cmax)
 // once), so the lower bound lies at or after start and is found by comparing the next few
 // proposals; with 8 cells per proposal three comparisons almost always suffice.
 // One workgroup per feature, one thread per table word.
-constexpr int kCellsPerWord = 16;
-constexpr int kCellShift    = 4;  // log2(kCellsPerWord); cells are never negative
-
-__device__ inline int table_start(uint32_t word, int cell)
-{
-  return static_cast<int>(word >> 16) + __popc(word & ((1u << (cell & (kCellsPerWord - 1))) - 1u));
-}
-
-// The bent map of a feature is the one of a few candidates (linear; logarithmic on both sides of a
-// centre at the low end, the median or the high end of the proposals, at three scales) that leaves the
-// fewest proposals in a cell with their predecessor: the proposals are a sample of the column, so they
-// say where its values fall. Each wave tries every fourth candidate.
-constexpr int kCellMaps = 10;
-template <typename T>
-__device__ inline CellMap<T> cell_map_candidate(int c, const T* p, int n, float cells)
-{
-  CellMap<T> m{T(0), T(0), 0.0f, 0.0f};
-  if (n < 3) return m;  // at least two finite proposals (the last one is +inf)
-  const T lo = p[0], hi = p[n - 2], mid = p[(n - 1) / 2];
-  const T width = hi - lo;
-  // (a -inf proposal, or a range that overflows: everything in cell 0)
-  if (!(width > T(0) && width < std::numeric_limits<T>::infinity())) return m;
-  T centre = lo, scale = T(1) / width;
-  if (c > 0) {
-    const int where = (c - 1) % 3, fine = (c - 1) / 3;
-    centre          = where == 0 ? mid : (where == 1 ? lo : hi);
-    // half of the proposals lie inside one unit of d (fine = 0), a quarter, an eighth
-    const int q  = max(1, (n - 1) >> (2 + fine));
-    const int at = (n - 1) / 2;
-    T reach      = where == 0 ? (p[min(n - 2, at + q)] - p[max(0, at - q)]) / T(2)
-                              : (where == 1 ? p[min(n - 2, 2 * q)] - lo : hi - p[max(0, n - 2 - 2 * q)]);
-    if (!(reach > width * T(1e-6))) reach = width * T(1e-6);
-    scale = T(1) / reach;
-  }
-  const T shift = -centre * scale;
-  if (!(scale < std::numeric_limits<T>::infinity()) || !(shift - shift == T(0))) return m;
-  const float g_lo = bend_axis(lo, scale, shift), g_hi = bend_axis(hi, scale, shift);
-  const float invw = cells / (g_hi - g_lo);
-  if (!(g_hi > g_lo) || !(invw < std::numeric_limits<float>::infinity())) return m;
-  m.scale = scale;
-  m.shift = shift;
-  m.invw  = invw;
-  m.nlo   = -g_lo * invw;
-  return m;
-}
-
-// Table words of a feature under the cell function `cell`.
-template <typename T, typename CellFn>
-__device__ inline void write_cell_words(const T* p, int n, int words, uint32_t* table, CellFn cell)
-{
-  for (int w = threadIdx.x; w < words; w += blockDim.x) {
-    // first proposal whose cell is >= the first cell of the word (the cells of the ascending
-    // proposals ascend too)
-    const int c0 = w * kCellsPerWord;
-    int a = 0, len = n;
-    while (len > 0) {
-      int half = len >> 1;
-      if (cell(p[a + half]) < c0) {
-        a += half + 1;
-        len -= half + 1;
-      } else {
-        len = half;
-      }
-    }
-    uint32_t bits = 0;
-    for (int i = a; i < n; i++) {
-      const int c = cell(p[i]);
-      if (c >= c0 + kCellsPerWord) break;
-      bits |= 1u << (c - c0);
-    }
-    table[w] = (static_cast<uint32_t>(a) << 16) | bits;
-  }
-}
-
 // tables: [2][F][words], the bent maps' tables first. A feature is straight when the plain linear map
 // leaves few of its proposals in a cell with their predecessor (normal columns: one in seven); only
 // then its second table is written, and a search group all of whose features are straight uses those.
@@ -404,12 +284,7 @@ __global__ void __launch_bounds__(256)
   const float cmax = static_cast<float>(C - 1);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int c = wave; c < kCellMaps; c += 4) {
-    const CellMap<T> m = cell_map_candidate(c, p, n, static_cast<float>(C));
-    int crowded        = 0;
-    for (int i = 1 + lane; i < n - 1; i += 64)
-      crowded += cell_of(p[i], m.scale, m.shift, m.invw, m.nlo, cmax) ==
-                 cell_of(p[i - 1], m.scale, m.shift, m.invw, m.nlo, cmax) ? 1 : 0;
-    for (int off = 32; off >= 1; off >>= 1) crowded += __shfl_xor(crowded, off, 64);
+    const int crowded = crowded_proposals(c, p, n, C, lane);
     if (lane == 0) s_crowded[c] = crowded;
   }
   __syncthreads();
@@ -546,21 +421,6 @@ template <typename T, int VEC>
 struct __attribute__((packed, aligned(sizeof(T)))) LooseVec {
   T v[VEC];
 };
-
-// Number of proposals in [p, p+n) that are < x (branch-free, fixed trip count).
-template <typename T>
-__device__ inline int count_less(const T* p, int n, T x, int steps)
-{
-  int lo = 0;
-  for (int s = 0; s < steps; s++) {
-    int half = n >> 1;
-    bool go  = n > 0 && p[lo + half] < x;
-    lo       = go ? lo + half + 1 : lo;
-    n        = go ? n - half - 1 : half;
-  }
-  return lo;
-}
-
 
 // A (grad, hess) pair as one 64-bit addend: grad * 2^32 + hess, both signed. Sums of such
 // words are sums of both halves as long as each total stays inside (-2^31, 2^31): the low

@@ -511,7 +511,7 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
 constexpr int kMidMaxDepth      = 10;
 constexpr int kMidMaxLevelNodes = 1 << (kMidMaxDepth - 1);
 constexpr int kMidMaxOutputs    = 16;
-constexpr int64_t kMidMaxValues = int64_t(80) * 1000 * 1000;
+constexpr int64_t kMidMaxValues = int64_t(200) * 1000 * 1000;
 
 struct MidTreeState {
   int64_t pitch;          // elements between features, outputs (multiple of 256, at least the rows)
@@ -519,6 +519,10 @@ struct MidTreeState {
   void* bins;             // [F][pitch]
   void* props;            // X dtype [F][S]
   double* proposals;      // [F][S] the same
+  int cells;              // cell functions and tables of the bin search, [F] each (see build_cells_kernel)
+  uint32_t* tables;       // [F][cells / 16]
+  void* map_x;            // X dtype [F][2]
+  float* map_t;           // [F][2]
   int32_t* counts;        // [F]
   int32_t* rp;            // [F + 1]
   double* chunk_sums;     // [2][chunks of 4096 entries]

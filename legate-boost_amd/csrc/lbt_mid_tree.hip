@@ -21,6 +21,7 @@
 // which histograms the reference would have kept.
 #include <algorithm>
 #include <limits>
+#include <type_traits>
 
 #include "lbt_device.h"
 #include "lbt_internal.h"
@@ -109,6 +110,31 @@ __global__ void __launch_bounds__(kWide)
       st.proposals[at + i]              = static_cast<double>(v);
     }
     if (tid == 0) st.counts[block] = n;
+    // the cell function and table of the bin search (see build_cells_kernel), a candidate per wave
+    __shared__ int s_crowded[kCellMaps];
+    static_assert(kCellMaps <= kWide / 64, "one wave per candidate");
+    T* const p = const_cast<T*>(s_prop);
+    if (tid == 0) p[n - 1] = std::numeric_limits<T>::infinity();
+    __syncthreads();
+    if ((tid >> 6) < kCellMaps) {
+      const int crowded = crowded_proposals(tid >> 6, p, n, st.cells, tid & 63);
+      if ((tid & 63) == 0) s_crowded[tid >> 6] = crowded;
+    }
+    __syncthreads();
+    int best = 0;
+    for (int c = 1; c < kCellMaps; c++)
+      if (s_crowded[c] < s_crowded[best]) best = c;
+    const CellMap<T> m = cell_map_candidate(best, p, n, static_cast<float>(st.cells));
+    const float cmax   = static_cast<float>(st.cells - 1);
+    const int words    = st.cells / kCellsPerWord;
+    write_cell_words(p, n, words, st.tables + static_cast<int64_t>(block) * words,
+                     [&](T x) { return cell_of(x, m.scale, m.shift, m.invw, m.nlo, cmax); });
+    if (tid == 0) {
+      static_cast<T*>(st.map_x)[2 * block]     = m.scale;
+      static_cast<T*>(st.map_x)[2 * block + 1] = m.shift;
+      st.map_t[2 * block]                      = m.invw;
+      st.map_t[2 * block + 1]                  = m.nlo;
+    }
     return;
   }
   if (block < a.F + sum_groups) {
@@ -147,7 +173,11 @@ struct BinPlan {
   int fb_log;        // lanes per row, log2
   int n_fb;          // feature blocks
   int row_groups;    // workgroups that share the row tiles of a feature block
+  int search_steps;  // of a binary search over a feature's proposals
 };
+
+// LDS elements per feature: the proposals, the +inf entries a window of probes may touch, and an odd pitch
+__host__ __device__ constexpr int prop_pitch(int S) { return (S + 8) | 1; }
 
 template <typename T, typename BinT>
 __global__ void __launch_bounds__(kWide)
@@ -238,53 +268,69 @@ __global__ void __launch_bounds__(kWide)
     }
     return;
   }
-  // binning: proposals of the block's features in the LDS (odd pitch: the lanes of a row start in different
-  // banks), a tile of rows at a time, turned in the LDS and stored feature by feature
+  // binning: proposals and tables of the block's features in the LDS (odd pitches: the lanes of a row start in
+  // different banks), a tile of rows at a time, turned in the LDS and stored feature by feature
   const int block = static_cast<int>(blockIdx.x) - p.quant_groups;
   const int fblk = block % p.n_fb, rg = block / p.n_fb;
   const int f0 = fblk * p.fb, nf = min(p.fb, a.F - f0);
-  const int pitch = a.S | 1;
-  T* s_prop       = reinterpret_cast<T*>(smem_raw);
-  int* s_n        = reinterpret_cast<int*>(s_prop + static_cast<size_t>(p.fb) * pitch);
+  const int pitch = prop_pitch(a.S), words = st.cells / kCellsPerWord, tpitch = words | 1;
+  T* s_prop         = reinterpret_cast<T*>(smem_raw);                              // [fb][pitch]
+  uint32_t* s_table = reinterpret_cast<uint32_t*>(s_prop + static_cast<size_t>(p.fb) * pitch);  // [fb][tpitch]
+  int* s_n          = reinterpret_cast<int*>(s_table + p.fb * tpitch);
   constexpr int kTilePitch = kRowsBin + 4 / sizeof(BinT);
-  BinT* s_bin     = reinterpret_cast<BinT*>(s_n + p.fb);  // [fb][kTilePitch]
+  BinT* s_bin       = reinterpret_cast<BinT*>(s_n + p.fb);  // [fb][kTilePitch]
   for (int i = tid; i < nf; i += kWide) s_n[i] = st.counts[f0 + i];
+  for (int i = tid; i < nf * words; i += kWide) {
+    const int fi = i / words, j = i - fi * words;
+    s_table[fi * tpitch + j] = st.tables[static_cast<int64_t>(f0 + fi) * words + j];
+  }
   __syncthreads();
-  for (int i = tid; i < nf * a.S; i += kWide) {
-    const int fi = i / a.S, j = i - fi * a.S;
-    if (j < s_n[fi]) s_prop[fi * pitch + j] = static_cast<const T*>(st.props)[static_cast<int64_t>(f0 + fi) * a.S + j];
+  for (int i = tid; i < nf * pitch; i += kWide) {
+    const int fi = i / pitch, j = i - fi * pitch;
+    // +inf behind the last proposal, for the probes that run past it
+    s_prop[i] = j < s_n[fi] ? static_cast<const T*>(st.props)[static_cast<int64_t>(f0 + fi) * a.S + j] : std::numeric_limits<T>::infinity();
   }
   const int fi = tid & ((1 << p.fb_log) - 1), r_first = tid >> p.fb_log, r_step = kWide >> p.fb_log;
+  const int fm = min(f0 + fi, a.F - 1);
+  const T scale = static_cast<const T*>(st.map_x)[2 * fm], shift = static_cast<const T*>(st.map_x)[2 * fm + 1];
+  const float invw = st.map_t[2 * fm], nlo = st.map_t[2 * fm + 1], cmax = static_cast<float>(st.cells - 1);
   const int tiles = (a.N + kRowsBin - 1) / kRowsBin;
   BinT* const out = static_cast<BinT*>(st.bins);
   for (int tile = rg; tile < tiles; tile += p.row_groups) {
     __syncthreads();
     if (fi < nf) {
-      const T* prop = s_prop + fi * pitch;
-      const int n   = s_n[fi] - 1;  // the last one, +inf, is never below a value
-      // four rows at a time, their searches side by side
+      const T* prop         = s_prop + fi * pitch;
+      const uint32_t* table = s_table + fi * tpitch;
+      // four rows at a time, their searches side by side: the table's start, three probes at once, and for the
+      // few lanes that need more four further ones and a binary search (as in bin_rows_kernel)
       for (int r = r_first; r < kRowsBin; r += 4 * r_step) {
         T x[4];
-        int lo[4], len[4];
+        int bn[4], cnt[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
           const int64_t row = static_cast<int64_t>(tile) * kRowsBin + r + u * r_step;
-          x[u]   = r + u * r_step < kRowsBin && row < a.N ? X[row * a.F + f0 + fi] : T(0);
-          lo[u]  = 0;
-          len[u] = n;
+          x[u]              = r + u * r_step < kRowsBin && row < a.N ? X[row * a.F + f0 + fi] : T(0);
         }
-        for (int left = n; left > 0; left >>= 1) {
 #pragma unroll
-          for (int u = 0; u < 4; u++) {
-            const int half = len[u] >> 1;
-            const bool go  = len[u] > 0 && prop[lo[u] + half] < x[u];
-            lo[u]          = go ? lo[u] + half + 1 : lo[u];
-            len[u]         = go ? len[u] - half - 1 : half;
+        for (int u = 0; u < 4; u++) {
+          const int cell = cell_of(x[u], scale, shift, invw, nlo, cmax);
+          bn[u]          = table_start(table[static_cast<unsigned>(cell) >> kCellShift], cell);
+          const T* pp    = prop + bn[u];
+          cnt[u]         = (pp[0] < x[u] ? 1 : 0) + (pp[1] < x[u] ? 1 : 0) + (pp[2] < x[u] ? 1 : 0);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          if (__any(cnt[u] == 3)) {
+            const T* pp  = prop + bn[u] + 3;
+            const int c2 = (pp[0] < x[u] ? 1 : 0) + (pp[1] < x[u] ? 1 : 0) + (pp[2] < x[u] ? 1 : 0) + (pp[3] < x[u] ? 1 : 0);
+            cnt[u] += cnt[u] == 3 ? c2 : 0;
+            if (__any(cnt[u] == 7)) {
+              const int left = cnt[u] == 7 ? s_n[fi] - (bn[u] + 7) : 0;
+              cnt[u] += count_less(pp + 4, left, x[u], p.search_steps);
+            }
           }
+          if (r + u * r_step < kRowsBin) s_bin[fi * kTilePitch + r + u * r_step] = static_cast<BinT>(bn[u] + cnt[u]);
         }
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-          if (r + u * r_step < kRowsBin) s_bin[fi * kTilePitch + r + u * r_step] = static_cast<BinT>(lo[u]);
       }
     }
     __syncthreads();
@@ -438,6 +484,7 @@ __global__ void __launch_bounds__(kScan)
   const int n_bins = st.counts[f], rp = st.rp[f];
   const int64_t fs = static_cast<int64_t>(a.F) * a.S;
   const int64_t up = static_cast<int64_t>(st.q_stats[0]), down = static_cast<int64_t>(st.q_stats[1]);
+  const bool fits    = up <= 2147483647LL && down <= 2147483647LL;  // no sum of grads leaves 32 bits
   const double inv_g = st.scales[2], inv_h = st.scales[3];
   const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
   I64Pair* const hist         = st.hist[p.depth & 1];
@@ -456,20 +503,25 @@ __global__ void __launch_bounds__(kScan)
         const int64_t step = static_cast<int64_t>(p.built) * a.K * fs;
         if (!root) pv = parent[k * fs + bin];
         int c = 0;
-        for (; c + 8 <= p.chunks; c += 8) {
-          unsigned long long w[8];
+        auto add = [&](auto width, auto plain) {
+          constexpr int kW = decltype(width)::value;
+          for (; c + kW <= p.chunks; c += kW) {
+            unsigned long long w[kW];
 #pragma unroll
-          for (int u = 0; u < 8; u++) w[u] = img[(c + u) * step];
+            for (int u = 0; u < kW; u++) w[u] = img[(c + u) * step];
 #pragma unroll
-          for (int u = 0; u < 8; u++) {
-            v.grad += decode_grad(static_cast<uint32_t>(w[u] >> 32), up, down);
-            v.hess += static_cast<uint32_t>(w[u]);
+            for (int u = 0; u < kW; u++) {
+              const uint32_t hi = static_cast<uint32_t>(w[u] >> 32);
+              v.grad += decltype(plain)::value ? static_cast<int64_t>(static_cast<int32_t>(hi)) : decode_grad(hi, up, down);
+              v.hess += static_cast<uint32_t>(w[u]);
+            }
           }
-        }
-        for (; c < p.chunks; c++) {
-          const unsigned long long w = img[c * step];
-          v.grad += decode_grad(static_cast<uint32_t>(w >> 32), up, down);
-          v.hess += static_cast<uint32_t>(w);
+        };
+        if (fits) {
+          add(std::integral_constant<int, 8>{}, std::true_type{});
+          add(std::integral_constant<int, 1>{}, std::true_type{});
+        } else {
+          add(std::integral_constant<int, 1>{}, std::false_type{});
         }
       }
       int64_t g = wave_inclusive_sum(v.grad), h = wave_inclusive_sum(v.hess);
@@ -699,14 +751,17 @@ LevelPlan plan_level(int64_t N, int F, int K, int S, int depth, int max_depth)
   p.built       = depth == 0 ? 1 : p.n_nodes / 2;
   p.last        = depth + 1 == max_depth;
   const int rows_of_lds = std::max<int>(1, static_cast<int>(kHistLds / (static_cast<size_t>(S) * 8)));
-  p.fw   = std::max(1, std::min({rows_of_lds / p.built, kMaxFw / 2, F}));
+  p.fw   = std::max(1, std::min({rows_of_lds / p.built, N >= 150000 ? kMaxFw : kMaxFw / 2, F}));
   p.bw   = std::max(1, std::min(p.built, rows_of_lds / p.fw));
   p.n_fb = (F + p.fw - 1) / p.fw;
   p.n_bb = (p.built + p.bw - 1) / p.bw;
   const int64_t inner = static_cast<int64_t>(p.n_fb) * p.n_bb * K;
   const int64_t image = static_cast<int64_t>(p.built) * K * F * S * 8;
-  int64_t chunks      = std::max<int64_t>(1, 320 / inner);
+  // two workgroups share a CU where their histograms do
+  const bool pairs    = static_cast<size_t>(p.fw) * p.bw * S * 8 <= 72 * 1024;
+  int64_t chunks      = std::max<int64_t>(1, (pairs ? 512 : 256) / inner);
   chunks              = std::min(chunks, std::max<int64_t>(1, N / 1024));
+  chunks              = std::min<int64_t>(chunks, 64);
   chunks              = std::min(chunks, std::max<int64_t>(1, (int64_t(64) << 20) / image));
   if (chunks > 8) chunks = chunks / 8 * 8;
   p.chunks     = static_cast<int>(chunks);
@@ -726,11 +781,12 @@ int64_t mid_image_words(int64_t N, int F, int K, int max_depth, int S)
   return most;
 }
 
-// By size: measured against the other builder (one output unless stated; depth 8 and 256 samples): 20,000 x 100
-// 521 -> 189 us at depth 6, 250,000 x 43 755 -> 373, 500,000 x 50 861 -> 502, 1,000,000 x 30 996 -> 491,
-// 200,000 x 50 with 8 outputs 971 -> 577, 800,000 x 80 1067 -> 882, 2,000,000 x 40 1156 -> 1127. Every pass
-// reads all rows; where a level's nodes come in several blocks it does so once per block (700,000 x 40
-// with 512 samples at depth 10, eight blocks: 1418 -> 1501), hence the second line.
+// By size: measured against the other builder (one output, depth 8 and 256 samples unless stated): 20,000 x 100
+// 521 -> 189 us at depth 6, 250,000 x 43 755 -> 350, 500,000 x 50 863 -> 417, 1,000,000 x 30 996 -> 418,
+// 2,000,000 x 40 1155 -> 834, 600,000 x 50 with 8 outputs 1745 -> 1535, 2,000,000 x 80 1444 -> 1174. Every pass
+// reads all rows, and where a level's nodes come in several blocks once per block (800,000 x 40 with 512
+// samples at depth 10, eight blocks: 1444 -> 1404), so what counts is values times blocks of the last
+// level: at 240 million the two are even (6,000,000 x 40 2100 -> 2108, 800,000 x 300 2034 -> 2113).
 bool mid_tree_fits(int64_t N, int F, int K, int max_depth, int S)
 {
   if (max_depth < 1 || max_depth > kMidMaxDepth || K > kMidMaxOutputs || S > LBT_MAX_SPLIT_SAMPLES) return false;
@@ -739,7 +795,7 @@ bool mid_tree_fits(int64_t N, int F, int K, int max_depth, int S)
   const int64_t level_hist = (int64_t(1) << (max_depth - 1)) * K * F * S * 16;
   if (level_hist > (int64_t(768) << 20)) return false;
   const int64_t values = N * F * K;
-  return values <= kMidMaxValues && values * plan_level(N, F, K, S, max_depth - 1, max_depth).n_bb <= 2 * kMidMaxValues;
+  return values * plan_level(N, F, K, S, max_depth - 1, max_depth).n_bb <= kMidMaxValues;
 }
 
 template <typename T, typename BinT>
@@ -813,15 +869,17 @@ int mid_tree_build(hipStream_t stream, const MidTreeState& st, const T* X, int64
     ProfScope ps(LBT_PROF_BINNING, stream);
     BinPlan p;
     p.quant_groups = static_cast<int>((N * K + kQuantPer - 1) / kQuantPer);
-    // features of a workgroup: their proposals take at most half of the 64 KB
-    p.fb     = std::max(1, std::min<int>(F, std::min<int>(32, static_cast<int>(40 * 1024 / ((a.S | 1) * sizeof(T))))));
+    p.search_steps = 0;
+    while ((1 << p.search_steps) < a.S + 1) p.search_steps++;
+    // features of a workgroup: what the search needs of them fits 64 KB, two workgroups a CU
+    const size_t per_feature = prop_pitch(a.S) * sizeof(T) + (st.cells / 16 + 1) * 4 + 4 + (kRowsBin + 4) * st.bin_bytes;
+    p.fb     = std::max(1, std::min<int>(F, std::min<int>(32, static_cast<int>(64 * 1024 / per_feature))));
     p.fb_log = 0;
     while ((1 << p.fb_log) < p.fb) p.fb_log++;
     p.n_fb       = (F + p.fb - 1) / p.fb;
     const int tiles = static_cast<int>((N + kRowsBin - 1) / kRowsBin);
     p.row_groups = std::max(1, std::min(tiles, 1024 / p.n_fb));
-    const size_t lds = std::max<size_t>(
-      static_cast<size_t>(p.fb) * ((a.S | 1) * sizeof(T) + 4 + (kRowsBin + 4) * st.bin_bytes) + 16, 2 * kWide * sizeof(double));
+    const size_t lds = std::max<size_t>(static_cast<size_t>(p.fb) * per_feature + 16, 2 * kWide * sizeof(double));
     static std::atomic<bool> attr_set[2][kMaxDevices] = {};
     const unsigned grid = static_cast<unsigned>(p.quant_groups + p.n_fb * p.row_groups);
     if (st.bin_bytes == 1) {
