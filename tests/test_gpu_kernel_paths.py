@@ -219,3 +219,27 @@ def test_medium_sizes_special_gradients(case):
     for sign in (1.0, -1.0):
         cr = orc.build_tree(X, sign * g, h, max_depth=4, split_samples=64, seed=5)
         _assert_tree(ops.build_tree(X, sign * g, h, max_depth=4, split_samples=64, seed=5), cr)
+
+
+@pytest.mark.parametrize("f,k", [(13, 2), (13, 4), (13, 5), (13, 8), (13, 9), (100, 8), (100, 9), (100, 17), (200, 2),
+                                 (200, 16), (200, 17), (200, 33)])
+def test_predict_shares_the_outputs_out_among_the_lanes_of_a_row(f, k):
+    """Output counts around one and two per lane and around a whole walk, for 4, 8 and 16 lanes per row; few trees,
+    a batch that is not full, and several batches. Sums are formed in tree order: equal to the oracle's."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(f + k)
+    X = rs.rand(777, f).astype(np.float32)
+    trees_c, trees_g = [], []
+    for t in range(45):
+        depth = [6, 2, 8, 4][t % 4]
+        m, inner = 2 ** (depth + 1) - 1, 2 ** depth - 1
+        feat = -np.ones(m, np.int32)
+        feat[:inner] = rs.randint(0, f, inner)
+        trees_c.append((rs.randn(m, k), feat, rs.rand(m)))
+        trees_g.append(tuple(ops.as_device(a) for a in trees_c[-1]))
+    for n_trees in (1, 3, 18, 45):
+        want = orc.predict(X, trees_c[:n_trees], k)
+        assert np.array_equal(gu.cpu(ops.predict(X, trees_g[:n_trees], k)), want), n_trees
