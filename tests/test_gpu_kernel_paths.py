@@ -243,3 +243,24 @@ def test_predict_shares_the_outputs_out_among_the_lanes_of_a_row(f, k):
     for n_trees in (1, 3, 18, 45):
         want = orc.predict(X, trees_c[:n_trees], k)
         assert np.array_equal(gu.cpu(ops.predict(X, trees_g[:n_trees], k)), want), n_trees
+
+
+@pytest.mark.parametrize("n,f,k,s,depth", [(9001, 60, 8, 512, 9), (9001, 50, 1, 512, 12)])
+@pytest.mark.parametrize("zero_hessians", [False, True])
+def test_levels_that_outgrow_the_histogram_budget_give_the_same_tree(n, f, k, s, depth, zero_hessians):
+    """The library's own budget (parents kept, only built siblings cleared) against explicit budgets (every level
+    that outgrows them starts an empty buffer). With rows that have no hessian the tree depends on the budget (the
+    reference leaves bins unscanned), and the library's own is the reference's."""
+    from lbtree import ops
+
+    rs = np.random.RandomState(f)
+    X = torch.from_numpy(rs.randn(n, f).astype(np.float32)).cuda()
+    g = torch.from_numpy(rs.randn(n, k)).cuda()
+    h = torch.from_numpy(0.1 + rs.random_sample((n, k))).cuda()
+    if zero_hessians:
+        h[::97] = 0.0
+    got = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=3, row_leaf=True)
+    for budget in (10 ** 9,) if zero_hessians else (10 ** 9, 4 * 10 ** 7):
+        want = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=3, row_leaf=True, hist_cache_bytes=budget)
+        for name in ("leaf_value", "feature", "split_value", "gain", "hessian", "row_leaf"):
+            assert torch.equal(getattr(got, name), getattr(want, name)), (budget, name)
