@@ -368,6 +368,14 @@ int lbt_update_tree(void* stream, const void* X, int32_t x_dtype, int64_t n_rows
                     double l1_regularization, double l2_regularization, double* leaf_out,
                     double* hessian_out, void* workspace, size_t workspace_bytes);
 
+/* lbt_update_tree that also stores the node every row stops in (row_leaf: int32 [n_rows], may be null), from which
+ * lbt_add_leaf_values forms the caller's `pred += tree.predict(X)` without a second traversal. */
+int lbt_update_tree_rows(void* stream, const void* X, int32_t x_dtype, int64_t n_rows,
+                         int32_t n_features, const double* g, const double* h, int32_t n_outputs,
+                         const int32_t* feature, const double* split, int32_t n_nodes,
+                         double l1_regularization, double l2_regularization, double* leaf_out,
+                         double* hessian_out, int32_t* row_leaf, void* workspace, size_t workspace_bytes);
+
 /* ---- the steps of a boosting round either side of BuildTreeTask ------------ */
 
 /* Objectives of lbt_weighted_gradient. */

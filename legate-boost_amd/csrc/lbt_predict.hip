@@ -687,61 +687,144 @@ __global__ void zero_doubles_kernel(double* a, int64_t n)
 
 // Every node on a row's path receives the row's (g, h) (update_tree.cc:76-90). The sums of an
 // inner node are the sums of its children, so a row adds to the node it stops in only and
-// propagate_sums_kernel fills in the rest. A workgroup collects its rows in an LDS copy of the
-// node sums (when that fits) and adds the copy to the global sums once.
-constexpr int kUpdateThreads = 256;
-constexpr int kUpdateLdsDoubles = 8192;  // 64 KB
+// finish_update_kernel fills in the rest. A workgroup collects its rows in an LDS copy of the
+// node sums (when that fits) and adds the copy to the global sums once; the tree lies in the LDS too.
+// What bounds it is how X is read. Walking it in place asks for a cache line per step and row, and the lines of the
+// rows in flight do not stay in the L2 (1,000,000 x 50, depth 8: 111 us, the rate of about eight million
+// scattered lines), so rows of up to kStagedBytesPerStep bytes per step of the walk are read whole, side by side,
+// into the LDS first (67 us). row_leaf, if given, receives the node every row stops in.
+constexpr int kUpdateThreads      = 1024;
+constexpr int kUpdateLdsDoubles   = 8192;  // node sums up to 64 KB
+constexpr int kStagedThreads      = 256;
+constexpr int kStagedBytesPerStep = 80;    // a scattered line costs as much as about 100 bytes in sequence
+constexpr size_t kStagedTile      = 60 * 1024;
+enum class UpdateMode { kGlobal, kLds, kStaged };  // where sums and tree lie; kStaged: rows in the LDS too
 
-template <typename T, bool kUseLds>
-__global__ void __launch_bounds__(kUpdateThreads)
-  update_accumulate_kernel(const T* __restrict__ X, int64_t n_rows, int F, const double* __restrict__ g,
-                           const double* __restrict__ h, int K, const int32_t* __restrict__ feature,
-                           const double* __restrict__ split, int n_nodes, double* G, double* H)
+struct UpdateArgs {
+  int64_t n_rows;
+  int F, K, n_nodes;
+  const double* g;
+  const double* h;
+  const int32_t* feature;
+  const double* split;
+  double* G;  // [n_nodes][K]
+  double* H;
+  int32_t* row_leaf;
+  int tile_rows;  // kStaged: a multiple of 64, at most kStagedThreads
+  int pitch;      // odd: the rows of a wave start in different banks
+};
+
+__host__ __device__ inline size_t update_lds_bytes(int n_nodes, int K)
 {
-  __shared__ double s_sum[kUseLds ? kUpdateLdsDoubles : 1];
-  const int n_sums = n_nodes * K;
+  return (static_cast<size_t>(n_nodes) * (2 * K * sizeof(double) + sizeof(double) + sizeof(int32_t)) + 15) & ~size_t(15);
+}
+
+template <typename T, UpdateMode kMode>
+__global__ void __launch_bounds__(kUpdateThreads) update_accumulate_kernel(const T* __restrict__ X, UpdateArgs a)
+{
+  constexpr bool kUseLds = kMode != UpdateMode::kGlobal;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  double* s_sum   = reinterpret_cast<double*>(smem_raw);  // [2][K][n_nodes]: nodes side by side in the banks
+  double* s_split = s_sum + 2 * static_cast<size_t>(a.n_nodes) * a.K;
+  int32_t* s_feat = reinterpret_cast<int32_t*>(s_split + a.n_nodes);
+  const int n_sums = a.n_nodes * a.K, tid = threadIdx.x, threads = blockDim.x;
   if constexpr (kUseLds) {
-    for (int i = threadIdx.x; i < 2 * n_sums; i += kUpdateThreads) s_sum[i] = 0.0;
+    for (int i = tid; i < 2 * n_sums; i += threads) s_sum[i] = 0.0;
+    for (int i = tid; i < a.n_nodes; i += threads) {
+      s_split[i] = a.split[i];
+      s_feat[i]  = a.feature[i];
+    }
     __syncthreads();
   }
-  for (int64_t row = blockIdx.x * static_cast<int64_t>(kUpdateThreads) + threadIdx.x; row < n_rows;
-       row += static_cast<int64_t>(gridDim.x) * kUpdateThreads) {
-    const T* xrow = X + row * F;
-    int pos       = 0;
+  auto take = [&](const T* xrow, int64_t row) {
+    int pos = 0;
     for (int depth = 0; depth < 100; depth++) {
-      const int ft = feature[pos];
+      const int ft = kUseLds ? s_feat[pos] : a.feature[pos];
       if (ft == -1) break;
       const double xv = static_cast<double>(xrow[ft]);
-      const int next  = xv <= split[pos] ? 2 * pos + 1 : 2 * pos + 2;
-      if (next >= n_nodes) break;
+      const int next  = xv <= (kUseLds ? s_split[pos] : a.split[pos]) ? 2 * pos + 1 : 2 * pos + 2;
+      if (next >= a.n_nodes) break;
       pos = next;
     }
-    for (int k = 0; k < K; k++) {
-      const double gv = g[row * K + k], hv = h[row * K + k];
+    if (a.row_leaf != nullptr) a.row_leaf[row] = pos;
+    for (int k = 0; k < a.K; k++) {
+      const double gv = a.g[row * a.K + k], hv = a.h[row * a.K + k];
       if constexpr (kUseLds) {
-        unsafeAtomicAdd(&s_sum[pos * K + k], gv);
-        unsafeAtomicAdd(&s_sum[n_sums + pos * K + k], hv);
+        unsafeAtomicAdd(&s_sum[k * a.n_nodes + pos], gv);
+        unsafeAtomicAdd(&s_sum[n_sums + k * a.n_nodes + pos], hv);
       } else {
-        unsafeAtomicAdd(&G[static_cast<int64_t>(pos) * K + k], gv);
-        unsafeAtomicAdd(&H[static_cast<int64_t>(pos) * K + k], hv);
+        unsafeAtomicAdd(&a.G[static_cast<int64_t>(pos) * a.K + k], gv);
+        unsafeAtomicAdd(&a.H[static_cast<int64_t>(pos) * a.K + k], hv);
       }
     }
+  };
+  if constexpr (kMode == UpdateMode::kStaged) {
+    T* s_x = reinterpret_cast<T*>(smem_raw + update_lds_bytes(a.n_nodes, a.K));  // [tile_rows][pitch]
+    const int64_t tiles = (a.n_rows + a.tile_rows - 1) / a.tile_rows;
+    const bool wide     = sizeof(T) == 4 && (a.F & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+    for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+      const int64_t row0 = tile * a.tile_rows;
+      const int here     = static_cast<int>(min<int64_t>(a.tile_rows, a.n_rows - row0));
+      const T* src       = X + row0 * a.F;
+      const int total    = here * a.F;
+      __syncthreads();  // the tile before is no longer read
+      if (wide) {
+        const float4* src4 = reinterpret_cast<const float4*>(src);
+#pragma unroll 4
+        for (int i = tid; i < total / 4; i += kStagedThreads) {
+          const float4 v = src4[i];
+          const int r    = i / (a.F / 4);
+          T* d           = s_x + r * a.pitch + (i - r * (a.F / 4)) * 4;
+          d[0] = v.x;
+          d[1] = v.y;
+          d[2] = v.z;
+          d[3] = v.w;
+        }
+      } else {
+#pragma unroll 4
+        for (int i = tid; i < total; i += kStagedThreads) {
+          const int r = i / a.F;
+          s_x[r * a.pitch + (i - r * a.F)] = src[i];
+        }
+      }
+      __syncthreads();
+      if (tid < here) take(s_x + tid * a.pitch, row0 + tid);
+    }
+  } else {
+    for (int64_t row = blockIdx.x * static_cast<int64_t>(threads) + tid; row < a.n_rows;
+         row += static_cast<int64_t>(gridDim.x) * threads)
+      take(X + row * a.F, row);
   }
   if constexpr (kUseLds) {
     __syncthreads();
-    for (int i = threadIdx.x; i < n_sums; i += kUpdateThreads) {
+    for (int i = tid; i < n_sums; i += threads) {
+      const int k = i / a.n_nodes, node = i - k * a.n_nodes;
       const double gv = s_sum[i], hv = s_sum[n_sums + i];
-      if (gv != 0.0) unsafeAtomicAdd(&G[i], gv);
-      if (hv != 0.0) unsafeAtomicAdd(&H[i], hv);
+      if (gv != 0.0) unsafeAtomicAdd(&a.G[node * a.K + k], gv);
+      if (hv != 0.0) unsafeAtomicAdd(&a.H[node * a.K + k], hv);
     }
   }
 }
 
-// sums of inner nodes, deepest level first: a node that leads on (the walk above leaves it)
-// adds what its two children hold
+// Sums of inner nodes, deepest level first: a node that leads on (the walk above leaves it)
+// adds what its two children hold. One workgroup. kUseLds: in the LDS, where a level costs no trip to the L2, and
+// with the leaf values (update_tree.cc:104-117) at the end.
+template <bool kUseLds>
 __global__ void __launch_bounds__(1024)
-  propagate_sums_kernel(const int32_t* __restrict__ feature, int n_nodes, int K, double* G, double* H)
+  finish_update_kernel(const int32_t* __restrict__ feature, int n_nodes, int K, double* G, double* H, double l1, double l2,
+                       double* leaf_out, double* hessian_out)
 {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int64_t n = static_cast<int64_t>(n_nodes) * K;
+  double* const g = kUseLds ? reinterpret_cast<double*>(smem_raw) : G;
+  double* const h = kUseLds ? g + n : H;
+  if constexpr (kUseLds) {
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+      g[i] = G[i];
+      h[i] = H[i];
+    }
+    __syncthreads();
+  }
   int depth = 0;
   while (((int64_t(1) << (depth + 1)) - 1) < n_nodes) depth++;
   for (int d = depth - 1; d >= 0; d--) {
@@ -752,22 +835,29 @@ __global__ void __launch_bounds__(1024)
       if (node < n_nodes && feature[node] != -1) {
         double gs = 0.0, hs = 0.0;
         if (2 * node + 1 < n_nodes) {
-          gs += G[(2 * node + 1) * K + k];
-          hs += H[(2 * node + 1) * K + k];
+          gs += g[(2 * node + 1) * K + k];
+          hs += h[(2 * node + 1) * K + k];
         }
         if (2 * node + 2 < n_nodes) {
-          gs += G[(2 * node + 2) * K + k];
-          hs += H[(2 * node + 2) * K + k];
+          gs += g[(2 * node + 2) * K + k];
+          hs += h[(2 * node + 2) * K + k];
         }
-        G[node * K + k] += gs;
-        H[node * K + k] += hs;
+        g[node * K + k] += gs;
+        h[node * K + k] += hs;
       }
     }
     __syncthreads();
   }
+  if constexpr (kUseLds) {
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+      const double hv = h[i];
+      leaf_out[i]     = hv > 0.0 ? calculate_leaf_value(g[i], hv, l1, l2) : 0.0;
+      hessian_out[i]  = hv;
+    }
+  }
 }
 
-// update_tree.cc:104-117
+// update_tree.cc:104-117, for trees whose sums do not fit the LDS
 __global__ void update_leaves_kernel(const double* G, const double* H, int64_t n, double l1, double l2,
                                      double* leaf_out, double* hessian_out)
 {
@@ -777,6 +867,52 @@ __global__ void update_leaves_kernel(const double* G, const double* H, int64_t n
     leaf_out[i]    = hv > 0.0 ? calculate_leaf_value(G[i], hv, l1, l2) : 0.0;
     hessian_out[i] = hv;
   }
+}
+
+template <typename T>
+int update_impl(hipStream_t stream, const T* X, UpdateArgs a, double l1, double l2, double* leaf_out,
+                double* hessian_out)
+{
+  const int64_t n = static_cast<int64_t>(a.n_nodes) * a.K;
+  zero_doubles_kernel<<<static_cast<unsigned>((2 * n + 255) / 256), 256, 0, stream>>>(a.G, 2 * n);
+  const bool lds = 2 * n <= kUpdateLdsDoubles;
+  int depth = 0;
+  while (((int64_t(1) << (depth + 1)) - 1) < a.n_nodes) depth++;
+  const size_t row_bytes = static_cast<size_t>(a.F | 1) * sizeof(T);
+  a.pitch                = a.F | 1;
+  a.tile_rows            = static_cast<int>(std::min<size_t>(kStagedThreads, kStagedTile / row_bytes / 64 * 64));
+  const size_t tree_lds  = update_lds_bytes(a.n_nodes, a.K);
+  const size_t lds_bytes = tree_lds + a.tile_rows * row_bytes;
+  if (a.n_rows > 0) {
+    static std::atomic<bool> attr[2][kMaxDevices] = {};
+    const int64_t per_launch = (a.n_rows + kUpdateThreads - 1) / kUpdateThreads;
+    const unsigned grid      = static_cast<unsigned>(std::min<int64_t>(per_launch, 512));
+    if (lds && a.tile_rows > 0 && static_cast<size_t>(a.F) * sizeof(T) <= static_cast<size_t>(kStagedBytesPerStep) * depth &&
+        lds_bytes <= kTileLds) {
+      const int per_cu         = std::max(1, static_cast<int>(kTileLds / lds_bytes));
+      const int64_t tiles      = (a.n_rows + a.tile_rows - 1) / a.tile_rows;
+      const unsigned tile_grid = static_cast<unsigned>(std::min<int64_t>(tiles, 256 * std::min(per_cu, 4)));
+      LBT_TRY((allow_dynamic_lds(update_accumulate_kernel<T, UpdateMode::kStaged>, kTileLds, attr[0])));
+      update_accumulate_kernel<T, UpdateMode::kStaged><<<tile_grid, kStagedThreads, lds_bytes, stream>>>(X, a);
+    } else if (lds) {
+      LBT_TRY((allow_dynamic_lds(update_accumulate_kernel<T, UpdateMode::kLds>, 128 * 1024, attr[1])));
+      update_accumulate_kernel<T, UpdateMode::kLds><<<grid, kUpdateThreads, tree_lds, stream>>>(X, a);
+    } else {
+      update_accumulate_kernel<T, UpdateMode::kGlobal><<<grid, kUpdateThreads, 0, stream>>>(X, a);
+    }
+  }
+  if (lds) {
+    static std::atomic<bool> attr[kMaxDevices] = {};
+    LBT_TRY(allow_dynamic_lds(finish_update_kernel<true>, kUpdateLdsDoubles * sizeof(double), attr));
+    finish_update_kernel<true><<<1, 1024, 2 * n * sizeof(double), stream>>>(a.feature, a.n_nodes, a.K, a.G, a.H, l1, l2,
+                                                                           leaf_out, hessian_out);
+  } else {
+    finish_update_kernel<false><<<1, 1024, 0, stream>>>(a.feature, a.n_nodes, a.K, a.G, a.H, l1, l2, leaf_out, hessian_out);
+    update_leaves_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, stream>>>(a.G, a.H, n, l1, l2, leaf_out,
+                                                                                     hessian_out);
+  }
+  LBT_HIP(hipGetLastError());
+  return LBT_OK;
 }
 
 }  // namespace
@@ -886,11 +1022,11 @@ size_t lbt_update_tree_workspace_bytes(int64_t n_rows, int32_t n_outputs, int32_
   return static_cast<size_t>(n_nodes) * n_outputs * 2 * sizeof(double) + 512;
 }
 
-int lbt_update_tree(void* stream, const void* X, int32_t x_dtype, int64_t n_rows,
-                    int32_t n_features, const double* g, const double* h, int32_t n_outputs,
-                    const int32_t* feature, const double* split, int32_t n_nodes,
-                    double l1_regularization, double l2_regularization, double* leaf_out,
-                    double* hessian_out, void* workspace, size_t workspace_bytes)
+int lbt_update_tree_rows(void* stream, const void* X, int32_t x_dtype, int64_t n_rows, int32_t n_features,
+                         const double* g, const double* h, int32_t n_outputs, const int32_t* feature,
+                         const double* split, int32_t n_nodes, double l1_regularization, double l2_regularization,
+                         double* leaf_out, double* hessian_out, int32_t* row_leaf, void* workspace,
+                         size_t workspace_bytes)
 {
   LBT_REQUIRE(x_dtype == LBT_F32 || x_dtype == LBT_F64, "unsupported X dtype %d", x_dtype);
   LBT_REQUIRE(n_rows >= 0 && n_features >= 1 && n_outputs >= 1 && n_nodes >= 1, "bad shape");
@@ -900,39 +1036,27 @@ int lbt_update_tree(void* stream, const void* X, int32_t x_dtype, int64_t n_rows
     lbt::set_error("workspace missing or too small for lbt_update_tree");
     return LBT_ERR_WORKSPACE;
   }
-  hipStream_t s   = static_cast<hipStream_t>(stream);
-  uintptr_t raw   = (reinterpret_cast<uintptr_t>(workspace) + 255) & ~uintptr_t(255);
-  double* G       = reinterpret_cast<double*>(raw);
-  const int64_t n = static_cast<int64_t>(n_nodes) * n_outputs;
-  double* H       = G + n;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  uintptr_t raw = (reinterpret_cast<uintptr_t>(workspace) + 255) & ~uintptr_t(255);
+  double* G     = reinterpret_cast<double*>(raw);
+  lbt::UpdateArgs a;
+  a.n_rows = n_rows; a.F = n_features; a.K = n_outputs; a.n_nodes = n_nodes;
+  a.g = g; a.h = h; a.feature = feature; a.split = split;
+  a.G = G; a.H = G + static_cast<int64_t>(n_nodes) * n_outputs; a.row_leaf = row_leaf;
   lbt::ProfScope ps(LBT_PROF_OTHER, s);
-  lbt::zero_doubles_kernel<<<static_cast<unsigned>((2 * n + 255) / 256), 256, 0, s>>>(G, 2 * n);
-  if (n_rows > 0) {
-    const unsigned grid = static_cast<unsigned>(std::min<int64_t>((n_rows + 255) / 256, 4096));
-    const bool lds      = 2 * n <= lbt::kUpdateLdsDoubles;
-    if (x_dtype == LBT_F32) {
-      const float* Xf = static_cast<const float*>(X);
-      if (lds)
-        lbt::update_accumulate_kernel<float, true><<<grid, 256, 0, s>>>(Xf, n_rows, n_features, g, h, n_outputs,
-                                                                        feature, split, n_nodes, G, H);
-      else
-        lbt::update_accumulate_kernel<float, false><<<grid, 256, 0, s>>>(Xf, n_rows, n_features, g, h, n_outputs,
-                                                                         feature, split, n_nodes, G, H);
-    } else {
-      const double* Xd = static_cast<const double*>(X);
-      if (lds)
-        lbt::update_accumulate_kernel<double, true><<<grid, 256, 0, s>>>(Xd, n_rows, n_features, g, h, n_outputs,
-                                                                         feature, split, n_nodes, G, H);
-      else
-        lbt::update_accumulate_kernel<double, false><<<grid, 256, 0, s>>>(Xd, n_rows, n_features, g, h, n_outputs,
-                                                                          feature, split, n_nodes, G, H);
-    }
-    lbt::propagate_sums_kernel<<<1, 1024, 0, s>>>(feature, n_nodes, n_outputs, G, H);
-  }
-  lbt::update_leaves_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(
-    G, H, n, l1_regularization, l2_regularization, leaf_out, hessian_out);
-  LBT_HIP(hipGetLastError());
-  return LBT_OK;
+  return x_dtype == LBT_F32
+           ? lbt::update_impl(s, static_cast<const float*>(X), a, l1_regularization, l2_regularization, leaf_out, hessian_out)
+           : lbt::update_impl(s, static_cast<const double*>(X), a, l1_regularization, l2_regularization, leaf_out, hessian_out);
+}
+
+int lbt_update_tree(void* stream, const void* X, int32_t x_dtype, int64_t n_rows, int32_t n_features, const double* g,
+                    const double* h, int32_t n_outputs, const int32_t* feature, const double* split, int32_t n_nodes,
+                    double l1_regularization, double l2_regularization, double* leaf_out, double* hessian_out,
+                    void* workspace, size_t workspace_bytes)
+{
+  return lbt_update_tree_rows(stream, X, x_dtype, n_rows, n_features, g, h, n_outputs, feature, split, n_nodes,
+                              l1_regularization, l2_regularization, leaf_out, hessian_out, nullptr, workspace,
+                              workspace_bytes);
 }
 
 }  // extern "C"

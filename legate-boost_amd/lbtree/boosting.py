@@ -164,8 +164,11 @@ class LBBase:
         pred = self.model_init_.reshape(1, -1).repeat(X.shape[0], 1).contiguous()
         for m in self.models_:
             g, h = self._get_weighted_gradient(y, pred, w, self.learning_rate)
-            m.update(X, g, h)
-            pred += m.predict(X)
+            if hasattr(m, "update_and_predict"):
+                m.update_and_predict(X, g, h, pred)
+            else:
+                m.update(X, g, h)
+                pred += m.predict(X)
         return self
 
 

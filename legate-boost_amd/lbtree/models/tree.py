@@ -111,6 +111,14 @@ class Tree(BaseModel):
         )
         return self
 
+    def update_and_predict(self, X, g, h, pred) -> "Tree":
+        """update(X, g, h), then pred += predict(X), without a second traversal of the rows."""
+        self.leaf_value, self.hessian, rows = ops.update_tree(
+            X, g, h, self.feature, self.split_value, self.l1_regularization, self.l2_regularization, row_leaf=True
+        )
+        ops.add_leaf_values(pred, self.leaf_value, rows)
+        return self
+
     def predict(self, X):
         return Tree.batch_predict([self], X)
 

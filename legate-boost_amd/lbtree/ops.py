@@ -233,8 +233,9 @@ def predict(X, trees, n_outputs, tiled=True):
     return out
 
 
-def update_tree(X, g, h, feature, split_value, l1_regularization, l2_regularization):
-    """UPDATE_TREE (legateboost/models/tree.py:197-240). Returns (leaf_value, hessian)."""
+def update_tree(X, g, h, feature, split_value, l1_regularization, l2_regularization, row_leaf=False):
+    """UPDATE_TREE (legateboost/models/tree.py:197-240). Returns (leaf_value, hessian), with row_leaf=True also the
+    node every row stops in (int32 [n_rows], see add_leaf_values)."""
     X = _check_x(X)
     g = as_device(g, torch.float64)
     h = as_device(h, torch.float64)
@@ -247,11 +248,13 @@ def update_tree(X, g, h, feature, split_value, l1_regularization, l2_regularizat
     hess = torch.empty((m, k), dtype=torch.float64, device=X.device)
     nbytes = _lib.lib.lbt_update_tree_workspace_bytes(n, k, m)
     ws = torch.empty(int(nbytes), dtype=torch.uint8, device=X.device)
-    rc = _lib.lib.lbt_update_tree(_stream(), X.data_ptr(), _DT[X.dtype], n, f, g.data_ptr(), h.data_ptr(), k,
-                                  feature.data_ptr(), split_value.data_ptr(), m, l1_regularization,
-                                  l2_regularization, leaf.data_ptr(), hess.data_ptr(), ws.data_ptr(), ws.numel())
+    rows = torch.empty(n, dtype=torch.int32, device=X.device) if row_leaf else None
+    rc = _lib.lib.lbt_update_tree_rows(_stream(), X.data_ptr(), _DT[X.dtype], n, f, g.data_ptr(), h.data_ptr(), k,
+                                       feature.data_ptr(), split_value.data_ptr(), m, l1_regularization,
+                                       l2_regularization, leaf.data_ptr(), hess.data_ptr(),
+                                       rows.data_ptr() if row_leaf else None, ws.data_ptr(), ws.numel())
     _lib.check(rc)
-    return leaf, hess
+    return (leaf, hess, rows) if row_leaf else (leaf, hess)
 
 
 _OBJECTIVES = {"squared_error": _lib.LBT_OBJ_SQUARED_ERROR, "log_loss": _lib.LBT_OBJ_LOG_LOSS}

@@ -264,3 +264,35 @@ def test_levels_that_outgrow_the_histogram_budget_give_the_same_tree(n, f, k, s,
         want = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=3, row_leaf=True, hist_cache_bytes=budget)
         for name in ("leaf_value", "feature", "split_value", "gain", "hessian", "row_leaf"):
             assert torch.equal(getattr(got, name), getattr(want, name)), (budget, name)
+
+
+@pytest.mark.parametrize("n,f,k,depth,dtype", [(1, 3, 1, 1, np.float32), (1023, 7, 1, 5, np.float64),
+                                               (1025, 50, 8, 8, np.float32), (70001, 13, 3, 8, np.float32),
+                                               (5003, 9, 9, 8, np.float64), (5003, 9, 1, 11, np.float32), (3001, 200, 1, 5, np.float32),
+                                               (3001, 9, 2, 11, np.float64)])
+def test_update_tree_and_the_rows_leaves(n, f, k, depth, dtype):
+    """Node sums that fit the LDS and that do not (more than 8192 doubles), rows around a workgroup: leaves within
+    rounding of the oracle's sequential sums (n additions of one sign: n * 2^-53 relative), rows as predict walks."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + k)
+    X = rs.rand(n, f).astype(dtype)
+    m, inner = 2 ** (depth + 1) - 1, 2 ** depth - 1
+    feat = -np.ones(m, np.int32)
+    feat[:inner] = rs.randint(0, f, inner)
+    feat[rs.randint(0, inner, 2) if inner > 4 else []] = -1
+    split = rs.rand(m)
+    g, h = 0.5 + rs.rand(n, k), 0.5 + rs.rand(n, k)
+    leaf_c, hess_c = orc.update_tree(X, g, h, feat, split, 0.0, 1.0)
+    Xd, gd, hd, fd, sd = (ops.as_device(a) for a in (X, g, h, feat, split))
+    leaf, hess, rows = ops.update_tree(Xd, gd, hd, fd, sd, 0.0, 1.0, row_leaf=True)
+    tol = 4 * n * 2.0 ** -53
+    assert np.allclose(gu.cpu(hess), hess_c, rtol=tol, atol=0)
+    assert np.allclose(gu.cpu(leaf), leaf_c, rtol=2 * tol, atol=0)
+    pred = torch.zeros((n, k), dtype=torch.float64, device="cuda")
+    ops.add_leaf_values(pred, leaf, rows)
+    assert torch.equal(pred, ops.predict(Xd, [(leaf, fd, sd)], k))
+    plain = ops.update_tree(Xd, gd, hd, fd, sd, 0.0, 1.0)
+    assert len(plain) == 2 and torch.allclose(plain[1], hess, rtol=tol, atol=0)
