@@ -2118,6 +2118,9 @@ int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, i
       pitch += ri.size;
     }
     hs.max_rec_stride = pitch;
+    hs.max_bins       = max_feature_bins;
+    hs.pieces         = 0;
+    for (int g = 0; g < hs.n_groups; g++) hs.pieces += (rec[g].bins_end + 15) / 16;
     // the same lanes per row for all groups (see binned_histogram_kernel): when the striped layout is
     // used, the records carry the gradient pair (one output: the groups' workgroups are bound by the
     // memory traffic they can share) and every record is long enough for the widest group's lanes

@@ -392,6 +392,8 @@ struct HistSetup {
   bool quad            = false;    // single-output trees, four lanes per 64-byte record in every group: the histogram kernel's kQuad mode
   RecInfo* rec         = nullptr;  // [n_groups]
   int64_t max_rec_stride = 0;      // widest record, bytes
+  int pieces           = 0;        // 16-byte pieces of bins of a row's records
+  int max_bins         = 0;        // bins of the widest feature
   int64_t* bin_base    = nullptr;  // [n_features] element offset of the feature's bin of row 0
   int32_t* bin_stride  = nullptr;  // [n_features] elements between consecutive rows
   int32_t* bin_tail    = nullptr;  // [n_features] g + 1 for the last feature of histogram group g, else 0
@@ -462,6 +464,33 @@ int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, i
                  const void* X);
 // Plans tiles for the batch and launches the histogram kernel.
 int hist_launch(hipStream_t stream, const HistSetup& hs, const HistBatch& b, int depth);
+
+// A level whose histograms stay in the LDS (see lbt_direct_level.hip).
+struct Cand;
+constexpr int kDirectMaxBins = 512;  // of a feature: 32 KB of LDS per workgroup
+struct DirectLevel {
+  int level_first, n_nodes, n_features, n_groups;
+  int64_t n_rows;
+  const void* binned;
+  const RecInfo* rec;
+  const int32_t* groups;
+  const int32_t* rows;
+  const int32_t* seg;
+  const int32_t* row_pointers;
+  const uint8_t* feature_set;
+  const double* scales;
+  double l1, l2, min_split_gain;
+  const double* proposals;
+  I64Pair* node_sums;
+  Cand* partial;   // [n_nodes][n_features] best split of a feature
+  I64Pair* left;   // and its left sums
+  double* leaf;
+  int32_t* feature;
+  double* split;
+  double* gain;
+  int32_t* split_bin;
+};
+int direct_level_launch(hipStream_t stream, const DirectLevel& a, const HistSetup& hs);
 
 // ---------------------------------------------------------------- builder for few rows
 // (lbt_small_tree.hip)

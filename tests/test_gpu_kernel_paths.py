@@ -296,3 +296,33 @@ def test_update_tree_and_the_rows_leaves(n, f, k, depth, dtype):
     assert torch.equal(pred, ops.predict(Xd, [(leaf, fd, sd)], k))
     plain = ops.update_tree(Xd, gd, hd, fd, sd, 0.0, 1.0)
     assert len(plain) == 2 and torch.allclose(plain[1], hess, rtol=tol, atol=0)
+
+
+@pytest.mark.parametrize("n,f,s,depth,kind", [(9001, 50, 512, 12, "plain"), (20011, 33, 200, 12, "feature_set"),
+                                              (9001, 7, 257, 13, "weighted"), (30011, 130, 256, 11, "whole")])
+def test_levels_without_histograms_in_memory_give_the_oracles_tree(n, f, s, depth, kind):
+    """Deep levels whose histograms stay in the LDS against explicit budgets, which keep them in memory, and the
+    oracle's decisions: bins of one and two bytes, features that end inside a 16-byte piece, several record groups,
+    unusable features, gradients that reach far into 32 bits, columns of few values (long empty runs)."""
+    import oracle_lib as orc
+    import gpu_util as gu
+    from lbtree import ops
+
+    rs = np.random.RandomState(depth)
+    X = rs.randn(n, f).astype(np.float32)
+    if kind == "whole":
+        X[:, ::2] = rs.randint(0, 5, X[:, ::2].shape)
+    g = rs.randn(n, 1)
+    h = 0.5 + rs.random_sample((n, 1))
+    if kind == "weighted":
+        g[:3] *= 3000.0
+    fs = rs.random_sample(f) < 0.6 if kind == "feature_set" else None
+    Xd, gd, hd = (torch.from_numpy(a).cuda() for a in (X, g, h))
+    kw = dict(max_depth=depth, split_samples=s, seed=5, feature_set=fs)
+    got = ops.build_tree(Xd, gd, hd, row_leaf=True, **kw)
+    want = ops.build_tree(Xd, gd, hd, row_leaf=True, taps=True, **kw)  # observed: histograms in memory
+    for name in ("leaf_value", "feature", "split_value", "gain", "hessian", "row_leaf"):
+        assert torch.equal(getattr(got, name), getattr(want, name)), name
+    if n < 10000 and f < 10:
+        cr = orc.build_tree(X, g, h, **kw)
+        assert np.array_equal(gu.cpu(got.feature), cr.feature)
