@@ -153,6 +153,7 @@ struct TileShape {
 };
 constexpr size_t kTileLds   = 160 * 1024 - 2048;  // dynamic LDS of the tile kernel
 constexpr int kCopyWords    = 6;  // 16-byte words a thread moves per batch: 6 * 1024 * 16 B >= any batch
+constexpr int kSmallRunGroups = 256;  // workgroups up to which more lanes share a row: one per CU
 constexpr size_t kSmallEnsembleLds = 78 * 1024;  // row tile + nodes of a small ensemble: two workgroups per CU
 constexpr int kMaxPackedNodes = 65535;  // the right child of a float node has 16 bits
 
@@ -344,8 +345,11 @@ __global__ void __launch_bounds__(kTileThreads)
   predict_tile_kernel(const T* __restrict__ X, int64_t n_rows, int F, int pitch, int n_batches,
                       const BatchInfo* __restrict__ batches, const PackedTree* __restrict__ desc,
                       const PackedNode<T>* __restrict__ nodes, const double* __restrict__ leaves, int K, int k0,
-                      double* __restrict__ out)
+                      int value_off, double* __restrict__ out)
 {
+  // value_off: where the LDS has room for a batch's leaf values (one output, 16 lanes per row), or 0. Handing a row's sum
+  // on through 16 lanes is a chain of 16 cross-lane moves per batch; with few rows, when nothing hides it, the
+  // values go through the LDS to the first wave instead, a row per lane.
   // k0: first of the (at most L * kOwn) outputs this launch sums; more outputs take a launch per chunk
   constexpr bool kSingle = kOwn == 0;
   using S = TileShape<L, kFew>;
@@ -401,6 +405,21 @@ __global__ void __launch_bounds__(kTileThreads)
 #pragma unroll
   for (int j = 0; j < kLaneTrees; j++) val[j] = 0.0;
 
+  constexpr bool kValues = kSingle && L == 16 && !kFew;
+  double* const s_value  = reinterpret_cast<double*>(smem_raw + value_off);  // [kBatchTrees][kTileRows]
+  const bool summing     = kValues && threadIdx.x < 64;
+  int handed             = 0;  // trees whose values lie in the LDS
+  auto hand_over = [&](int count) {
+#pragma unroll
+    for (int j = 0; j < kLaneTrees; j++)
+      if (q * kLaneTrees + j < count) s_value[(q * kLaneTrees + j) * kTileRows + r] = val[j];
+    handed = count;
+  };
+  auto add_handed = [&]() {
+#pragma unroll 8
+    for (int jj = 0; jj < handed; jj++) acc[0] += s_value[jj * kTileRows + threadIdx.x];
+  };
+
   for (int b = 0; b < n_batches; b++) {
     const BatchInfo info = info_n;
     __syncthreads();  // the previous batch is no longer read; on the first pass: X tile complete
@@ -412,6 +431,7 @@ __global__ void __launch_bounds__(kTileThreads)
         if (i < n16) s_words[i] = pf.words[c];
       }
     }
+    if (summing && value_off != 0) add_handed();
     int base[kLaneTrees], pos[kLaneTrees];
 #pragma unroll
     for (int j = 0; j < kLaneTrees; j++) {
@@ -439,7 +459,10 @@ __global__ void __launch_bounds__(kTileThreads)
     }
     if constexpr (kSingle) {
       // leaf values of the previous batch arrived while this one was walked
-      add_in_order<S>(acc[0], val, cnt_prev, q);
+      if (kValues && value_off != 0)
+        hand_over(cnt_prev);
+      else
+        add_in_order<S>(acc[0], val, cnt_prev, q);
 #pragma unroll
       for (int j = 0; j < kLaneTrees; j++) val[j] = leaves[info.node_off + base[j] + pos[j]];
       cnt_prev = info.count;
@@ -449,6 +472,16 @@ __global__ void __launch_bounds__(kTileThreads)
       for (int j = 0; j < kLaneTrees; j++) at[j] = base[j] + pos[j];
       add_leaves_in_order<S, kAcc>(acc, at, info.count, leaves + info.node_off * K + k_first, K, K - k_first);
     }
+  }
+  if (kValues && value_off != 0) {
+    __syncthreads();
+    if (summing) add_handed();
+    __syncthreads();
+    hand_over(cnt_prev);
+    __syncthreads();
+    if (summing) add_handed();
+    if (summing && static_cast<int>(threadIdx.x) < rows_here) out[row0 + threadIdx.x] = acc[0];
+    return;
   }
   if constexpr (kSingle) add_in_order<S>(acc[0], val, cnt_prev, q);
   // single output: the row's last lane holds the sum; several outputs: every lane holds its own
@@ -622,7 +655,14 @@ int pack_tiled(hipStream_t stream, int F, int n_trees, const double* const* leaf
 template <typename T>
 int run_tiled(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble& ens, double* out)
 {
-  const int F = ens.n_features, K = ens.n_outputs, lanes = ens.lanes, n_batches = ens.n_batches;
+  const int F = ens.n_features, K = ens.n_outputs, n_batches = ens.n_batches;
+  // The lanes the ensemble was laid out for suit many rows. Batches of so many trees fit the kernels for more lanes
+  // per row too (their last lanes then have no tree), and where the rows would leave most CUs without a
+  // workgroup these split them further and walk fewer trees per lane: 256 x 32, 100 trees of depth 6: 19.0 us
+  // with 4 lanes (one workgroup), 12.3 with 16 and the values through the LDS (18.7 with the sum handed on).
+  int lanes = ens.lanes;
+  for (const int more : {8, 16})
+    if (more > lanes && N <= static_cast<int64_t>(kTileThreads / more) * kSmallRunGroups) lanes = more;
   PackedLayout<T> lay(ens.data, ens.n_trees, ens.total_nodes);
   const int pitch     = F | 1;
   const int tile_rows = kTileThreads / lanes;
@@ -632,11 +672,16 @@ int run_tiled(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemb
   // chunk (each chunk's sums are formed in tree order, as in one walk).
   const int own   = K == 1 ? 0 : (K <= lanes ? 1 : 2);
   const int chunk = K == 1 ? 1 : lanes * own;
+  const size_t values  = static_cast<size_t>(TileShape<16>::kBatchTrees) * TileShape<16>::kRows * sizeof(double);
+  const size_t shared  = (static_cast<size_t>(ens.lds_bytes) + 15) & ~size_t(15);
+  const bool by_values = K == 1 && lanes == 16 && tiles <= kSmallRunGroups && shared + values <= kTileLds;
+  const int value_off  = by_values ? static_cast<int>(shared) : 0;
+  const size_t lds     = by_values ? shared + values : static_cast<size_t>(ens.lds_bytes);
   auto launch = [&](auto kernel, std::atomic<bool> (&flags)[kMaxDevices]) -> int {
     LBT_TRY(allow_dynamic_lds(kernel, kTileLds, flags));
     for (int k0 = 0; k0 < K; k0 += chunk)
-      kernel<<<tiles, kTileThreads, static_cast<size_t>(ens.lds_bytes), stream>>>(
-        X, N, F, pitch, n_batches, lay.batches, lay.desc, lay.nodes, lay.leaves, K, k0, out);
+      kernel<<<tiles, kTileThreads, lds, stream>>>(X, N, F, pitch, n_batches, lay.batches, lay.desc, lay.nodes, lay.leaves,
+                                                   K, k0, value_off, out);
     return LBT_OK;
   };
   static std::atomic<bool> attr[2][3][3][kMaxDevices] = {};

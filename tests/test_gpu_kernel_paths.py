@@ -326,3 +326,29 @@ def test_levels_without_histograms_in_memory_give_the_oracles_tree(n, f, s, dept
     if n < 10000 and f < 10:
         cr = orc.build_tree(X, g, h, **kw)
         assert np.array_equal(gu.cpu(got.feature), cr.feature)
+
+
+@pytest.mark.parametrize("f,k,n_trees", [(13, 1, 45), (13, 3, 45), (13, 1, 3), (100, 1, 45), (100, 9, 7), (200, 1, 45)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_predict_takes_more_lanes_per_row_for_few_rows(f, k, n_trees, dtype):
+    """Row counts either side of the two limits, ensembles laid out for 4, 8 and 16 lanes, few trees and several
+    outputs: equal to the per-node kernel."""
+    from lbtree import ops
+
+    rs = np.random.RandomState(f + k)
+    gen = torch.Generator(device="cuda").manual_seed(f)
+    X = torch.rand((33001, f), generator=gen, device="cuda", dtype=torch.float64).to(
+        torch.float32 if dtype == np.float32 else torch.float64)
+    trees = []
+    for t in range(n_trees):
+        depth = [6, 2, 8, 4][t % 4]
+        m, inner = 2 ** (depth + 1) - 1, 2 ** depth - 1
+        feat = -np.ones(m, np.int32)
+        feat[:inner] = rs.randint(0, f, inner)
+        trees.append(tuple(ops.as_device(a) for a in (rs.randn(m, k), feat, rs.rand(m))))
+    want = ops.predict(X, trees, k, tiled=False)
+    packed = ops.PackedEnsemble(trees, k, f, X.dtype) if f <= 100 else None
+    for rows in (1, 63, 65, 16384, 16385, 32768, 32769, 33001):
+        assert torch.equal(ops.predict(X[:rows], trees, k), want[:rows]), rows
+        if packed is not None:
+            assert torch.equal(packed.predict(X[:rows]), want[:rows]), rows
