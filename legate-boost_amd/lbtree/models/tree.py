@@ -112,7 +112,13 @@ class Tree(BaseModel):
         return self
 
     def update_and_predict(self, X, g, h, pred) -> "Tree":
-        """update(X, g, h), then pred += predict(X), without a second traversal of the rows."""
+        """update(X, g, h), then pred += predict(X), without a second traversal of the rows (unless a subclass
+        brings its own of either)."""
+        cls = type(self)
+        if cls.update is not Tree.update or cls.predict is not Tree.predict or cls.batch_predict is not Tree.batch_predict:
+            self.update(X, g, h)
+            pred += self.predict(X)
+            return self
         self.leaf_value, self.hessian, rows = ops.update_tree(
             X, g, h, self.feature, self.split_value, self.l1_regularization, self.l2_regularization, row_leaf=True
         )
