@@ -788,14 +788,23 @@ __global__ void __launch_bounds__(256) small_count_kernel(SmallTreeState st, Lev
   }
 }
 
+// Places of the order a scan workgroup holds, by rows, and the LDS it then asks for at a level of n_nodes nodes
+// (see small_scan_kernel). 156 KB of the 160 leave room for its static arrays (0.6 KB).
+constexpr size_t kScanLds = 156 * 1024;
+constexpr int small_scan_places(int64_t N) { return N <= 1024 ? 1024 : N <= 2048 ? 2048 : N <= 4096 ? 4096 : kSmallMaxRows; }
+constexpr size_t small_scan_lds(int64_t N, int64_t n_nodes)
+{
+  return static_cast<size_t>((N + 1) / 2 * 2 * 8 + (small_scan_places(N) + 4) * 4 + n_nodes * 12 + (n_nodes / 2 + 1) * 4 +
+                             (N + 3) / 4 * 4 + 16);
+}
+
 template <int kT, int kE, bool kSingle>
 int launch_small_scan_as(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a)
 {
   static std::atomic<bool> attr_set[kMaxDevices] = {};
-  const size_t lds = static_cast<size_t>((a.N + 1) / 2 * 2) * 8 + (kT * kE + 4) * 4 + static_cast<size_t>(a.n_nodes) * 12 +
-                     (a.n_nodes / 2 + 1) * 4 + (a.N + 3) / 4 * 4 + 16;
-  LBT_TRY(allow_dynamic_lds(small_scan_kernel<kT, kE, kSingle>, 156 * 1024, attr_set));
-  small_scan_kernel<kT, kE, kSingle><<<a.F, kT, lds, stream>>>(st, a);
+  LBT_REQUIRE(small_scan_places(a.N) == kT * kE, "%d rows do not take a workgroup of %d places", a.N, kT * kE);
+  LBT_TRY(allow_dynamic_lds(small_scan_kernel<kT, kE, kSingle>, kScanLds, attr_set));
+  small_scan_kernel<kT, kE, kSingle><<<a.F, kT, small_scan_lds(a.N, a.n_nodes), stream>>>(st, a);
   return LBT_OK;
 }
 template <int kT, int kE>
@@ -807,12 +816,14 @@ int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelA
 }  // namespace
 
 // By size: a row number has to fit 16 bits and a feature's order the registers of one workgroup; the
-// quantiser's workgroup takes kQuantChunks chunks; a level's nodes get a slot each in the LDS. At
-// 8192 rows a level takes about as long here as in the other builder's launches for it.
+// quantiser's workgroup takes kQuantChunks chunks; the rows and a slot for each node of a level share the LDS
+// (of 13 levels up to 7732 rows). At 8192 rows a level takes about as long here as in the other builder's launches
+// for it.
 bool small_tree_fits(int64_t N, int F, int K, int max_depth, int S)
 {
   return N <= kSmallMaxRows && K <= kSmallMaxOutputs && N * K <= kQuantChunks * 4096 && max_depth >= 1 &&
-         max_depth <= kSmallMaxDepth && S <= LBT_MAX_SPLIT_SAMPLES && static_cast<int64_t>(F) * S < (int64_t(1) << 26) &&
+         max_depth <= kSmallMaxDepth && small_scan_lds(N, int64_t(1) << (max_depth - 1)) <= kScanLds &&
+         S <= LBT_MAX_SPLIT_SAMPLES && static_cast<int64_t>(F) * S < (int64_t(1) << 26) &&
          (static_cast<int64_t>(F) << (max_depth - 1)) <= (int64_t(1) << 22);
 }
 
@@ -862,14 +873,12 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
     a.last        = d + 1 == prm.max_depth;
     {
       ProfScope ps(LBT_PROF_HISTOGRAM, stream, 0.0, d);
-      if (N <= 1024)
-        LBT_TRY((launch_small_scan<256, 4>(stream, st, a)));
-      else if (N <= 2048)
-        LBT_TRY((launch_small_scan<512, 4>(stream, st, a)));
-      else if (N <= 4096)
-        LBT_TRY((launch_small_scan<1024, 4>(stream, st, a)));
-      else
-        LBT_TRY((launch_small_scan<1024, 8>(stream, st, a)));
+      switch (small_scan_places(N)) {
+        case 1024: LBT_TRY((launch_small_scan<256, 4>(stream, st, a))); break;
+        case 2048: LBT_TRY((launch_small_scan<512, 4>(stream, st, a))); break;
+        case 4096: LBT_TRY((launch_small_scan<1024, 4>(stream, st, a))); break;
+        default: LBT_TRY((launch_small_scan<1024, 8>(stream, st, a)));
+      }
     }
     if (level_totals != nullptr) small_count_kernel<<<1, 256, 0, stream>>>(st, a, level_totals + d);
     ProfScope ps(LBT_PROF_SPLIT, stream);

@@ -51,6 +51,20 @@ def test_workspace_query():
     assert _lib.lib.lbt_predict_workspace_bytes(10, 100, 0, _lib.LBT_F32) == 0
 
 
+def test_the_builder_for_few_rows_is_not_offered_what_its_scan_cannot_hold():
+    """8192 rows and the 4096 nodes of a thirteenth level need more LDS than a workgroup has. Its buffers (ten bytes
+    a value) are carved where the builder is taken: one row more, which is not its size, must not need less scratch."""
+    from lbtree import _lib
+
+    def q(rows, depth):
+        return _lib.lib.lbt_build_tree_workspace_bytes(rows, 1024, 1, depth, 64, _lib.LBT_F32, 0)
+
+    per_value = 10 * 1024
+    assert q(8192, 12) - q(8193, 12) > 8000 * per_value  # taken at twelve levels
+    assert q(8192, 13) <= q(8193, 13)
+    assert q(7733, 13) < q(7732, 13) - 7000 * per_value  # the last size whose thirteen levels fit
+
+
 def test_bad_arguments_are_rejected_without_a_gpu():
     from lbtree import _lib
 

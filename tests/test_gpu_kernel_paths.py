@@ -79,6 +79,10 @@ def _assert_tree(got, cr):
     (8193, 9, 1, 8, 256, np.float32),      # one row more
     (8192, 3, 5, 4, 64, np.float32),       # more entries than it takes
     (500, 4, 1, 14, 64, np.float32),       # deeper than it takes
+    (7732, 3, 1, 13, 64, np.float32),      # the most rows whose thirteen levels fit the scan's LDS, one more, and
+    (7733, 3, 1, 13, 64, np.float32),      # the most rows at all
+    (8192, 3, 1, 13, 64, np.float64),
+    (8192, 4, 4, 13, 32, np.float32),
 ])
 def test_few_rows(n, f, k, depth, s, dtype):
     """The builder for few rows at the edges of what it takes (and just past them), with constant and
