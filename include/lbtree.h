@@ -42,8 +42,9 @@ int lbt_version(void);
 
 /*
  * State the library keeps between calls, all of it per host thread: the error string, and, once
- * the thread has called lbt_build_tree, two small pinned host buffers and three events (the
- * values a build reads back while it runs, and the staging buffer of the tables it sends).
+ * the thread has called lbt_build_tree, up to three small pinned host buffers and three events
+ * (the values a build reads back while it runs or that its kernels report, and the staging buffer
+ * of the tables it sends). Builds of one thread may run on several streams, each with a workspace of its own.
  * They are created on first use and reused; this call waits for the copies that still use them
  * and frees them (the next build on the thread creates them again). A thread that ends without
  * calling it leaves them allocated until the process ends. Beyond these and the optional

@@ -176,7 +176,7 @@ int thread_resources_here(ThreadResources** out)
   return LBT_OK;
 }
 
-int DeviceAnswer::open()
+int DeviceAnswer::open(hipStream_t on)
 {
   ThreadResources* here = nullptr;
   LBT_TRY(thread_resources_here(&here));
@@ -187,13 +187,15 @@ int DeviceAnswer::open()
   words = here->answer;
   tag   = ++here->answer_tag;
   if (tag == 0) tag = here->answer_tag = 1;
+  stream = on;
+  due    = true;
   return LBT_OK;
 }
 
-int DeviceAnswer::wait(hipStream_t stream, unsigned* flags, int32_t* n_bins)
+int DeviceAnswer::wait(unsigned* flags, int32_t* n_bins)
 {
   volatile unsigned long long* const w = words;
-  auto arrived = [&]() { return (w[0] >> 32) == tag && (n_bins == nullptr || (w[1] >> 32) == tag); };
+  auto arrived = [&]() { return (w[0] >> 32) == tag && (w[1] >> 32) == tag; };
   // should the words not come (the stream has failed), the stream's own state ends the wait
   for (int64_t spin = 1; !arrived(); spin++) {
     if (spin % 16384 != 0) continue;
@@ -204,6 +206,7 @@ int DeviceAnswer::wait(hipStream_t stream, unsigned* flags, int32_t* n_bins)
     set_error("the tree builder's kernels did not report");
     return LBT_ERR_HIP;
   }
+  due = false;
   const unsigned got = static_cast<unsigned>(w[0] & 0xffffffffULL);
   if (n_bins != nullptr) *n_bins = static_cast<int32_t>(w[1] & 0xffffffffULL);
   if ((got & 2u) != 0) {
@@ -213,6 +216,12 @@ int DeviceAnswer::wait(hipStream_t stream, unsigned* flags, int32_t* n_bins)
   }
   *flags = got & 1u;
   return LBT_OK;
+}
+
+DeviceAnswer::~DeviceAnswer()
+{
+  // a call that fails before its wait: kernels that store the words may be queued
+  if (due) (void)hipStreamSynchronize(stream);
 }
 
 }  // namespace lbt

@@ -850,7 +850,7 @@ int mid_tree_build(hipStream_t stream, const MidTreeState& st, const T* X, int64
 {
   *taken = false;
   DeviceAnswer answer;
-  LBT_TRY(answer.open());
+  LBT_TRY(answer.open(stream));
   MidArgs a;
   a.N = static_cast<int>(N); a.F = F; a.K = K; a.S = prm.split_samples;
   a.row_offset = row_offset; a.seed = prm.seed; a.dataset_rows = prm.dataset_rows;
@@ -905,7 +905,7 @@ int mid_tree_build(hipStream_t stream, const MidTreeState& st, const T* X, int64
   else
     LBT_TRY((queue_levels<T, uint16_t>(stream, st, a, level_totals)));
   unsigned flags = 0;
-  LBT_TRY(answer.wait(stream, &flags, n_bins));
+  LBT_TRY(answer.wait(&flags, n_bins));
   *taken = flags == 0;
   return LBT_OK;
 }

@@ -835,7 +835,7 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
 {
   *taken = false;
   DeviceAnswer answer;
-  LBT_TRY(answer.open());
+  LBT_TRY(answer.open(stream));
   PrologueArgs pa;
   pa.row_offset = row_offset;
   pa.N = static_cast<int>(N); pa.F = F; pa.K = K; pa.S = prm.split_samples;
@@ -892,7 +892,7 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
   }
   LBT_HIP(hipGetLastError());
   unsigned flags = 0;
-  LBT_TRY(answer.wait(stream, &flags, n_bins));
+  LBT_TRY(answer.wait(&flags, n_bins));
   *taken = flags == 0;
   return LBT_OK;
 }

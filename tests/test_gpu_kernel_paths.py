@@ -225,6 +225,44 @@ def test_medium_sizes_special_gradients(case):
         _assert_tree(ops.build_tree(X, sign * g, h, max_depth=4, split_samples=64, seed=5), cr)
 
 
+@pytest.mark.parametrize("rows", [(700, 900), (700, 9000), (9000, 9500)])
+def test_builds_of_one_thread_on_two_streams(rows, monkeypatch):
+    """All builds of a thread hear from their kernels through the same pinned words. Calls without observation points
+    beside calls that want the number of bins, in turn on two streams and with the words given back in between: every
+    call has to get its own answer, and no store of an earlier one may come after it has returned."""
+    from lbtree import _lib, ops
+
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    own = {}
+
+    def workspace(nbytes, device):
+        key = torch.cuda.current_stream().cuda_stream
+        if key not in own or own[key].numel() < nbytes:
+            own[key] = torch.empty(int(nbytes), dtype=torch.uint8, device=device)
+        return own[key]
+
+    monkeypatch.setattr(ops, "_get_workspace", workspace)
+    calls, want = [], []
+    for i, n in enumerate(rows):
+        rs = np.random.RandomState(n)
+        X, g, h = (torch.from_numpy(a).cuda() for a in (rs.randn(n, 20).astype(np.float32), rs.randn(n, 1), 0.1 + rs.rand(n, 1)))
+        calls.append((X, g, h, dict(max_depth=5, split_samples=64, seed=i, row_leaf=i == 1, wait=False)))
+        want.append(ops.build_tree(X, g, h, **dict(calls[i][3], wait=True)))
+    torch.cuda.synchronize()
+    for turn in range(100):
+        got = [None, None]
+        for i in ((0, 1) if turn % 2 else (1, 0)):
+            X, g, h, kw = calls[i]
+            with torch.cuda.stream(streams[i]):
+                got[i] = ops.build_tree(X, g, h, **kw)
+        if turn % 10 == 0:
+            assert _lib.lib.lbt_release_thread_resources() == 0
+        torch.cuda.synchronize()
+        for i in range(2):
+            for name in ("leaf_value", "feature", "split_value", "gain", "hessian"):
+                assert torch.equal(getattr(got[i], name), getattr(want[i], name)), (turn, i, name)
+
+
 @pytest.mark.parametrize("f,k", [(13, 2), (13, 4), (13, 5), (13, 8), (13, 9), (100, 8), (100, 9), (100, 17), (200, 2),
                                  (200, 16), (200, 17), (200, 33)])
 def test_predict_shares_the_outputs_out_among_the_lanes_of_a_row(f, k):
