@@ -154,7 +154,7 @@ int release_thread_resources();
 // What the builders without a wait in their middle have to learn from the device: two words of the thread's
 // pinned memory that kernels early in the queue write, each (tag << 32) | value: words[0] flags (1: the
 // data need the other builder, 2: a rounded value does not fit 32 bits), words[1] the number of bins.
-// The host looks at them once everything is queued; the tag tells one call's answer from another's. All builds
+// The host waits for them once everything is queued; the tag tells one call's answer from another's. All builds
 // of a thread share the words, on whatever streams, and lbt_release_thread_resources frees them: no call
 // returns while a store of its own is still to come. wait() sees both words, and a call that ends without
 // it drains its stream.
@@ -164,6 +164,12 @@ struct DeviceAnswer {
   hipStream_t stream        = nullptr;
   bool due                  = false;  // a kernel may still store them
   int open(hipStream_t on);
+  // the flags have come and say that this builder's levels are not wanted (false as long as they are out)
+  bool declined() const
+  {
+    const unsigned long long w = *static_cast<volatile const unsigned long long*>(words);
+    return (w >> 32) == tag && (w & 0xffffffffULL) != 0;
+  }
   // flags: receives bit 0; bit 1 is returned as LBT_ERR_UNSUPPORTED. n_bins: null when not wanted.
   int wait(unsigned* flags, int32_t* n_bins);
   DeviceAnswer() = default;

@@ -343,6 +343,12 @@ __global__ void __launch_bounds__(kWide)
   }
 }
 
+// Nothing to do at a level: no node was split into it, or (known at the root) the data are for the other builder.
+__device__ __forceinline__ bool level_is_empty(const MidTreeState& st, int depth)
+{
+  return st.live[depth] == 0 || (depth == 0 && st.q_stats[2] != 0);
+}
+
 // How a level's histograms are dealt to workgroups.
 struct LevelPlan {
   int depth, level_first, n_nodes;
@@ -385,14 +391,14 @@ __global__ void __launch_bounds__(kWide)
   rest            = rest % inner;
   if (chunk >= p.chunks) return;
   const int k = rest % a.K, fb = rest / a.K % p.n_fb, bb = rest / a.K / p.n_fb;
-  const int live = st.live[p.depth];
+  const bool empty = level_is_empty(st, p.depth);
   if (p.depth == 0 && blockIdx.x == 0 && tid == 0) {
     __hip_atomic_store(a.answer + 1, (static_cast<unsigned long long>(a.tag) << 32) | static_cast<unsigned>(st.rp[a.F]),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(a.answer, (static_cast<unsigned long long>(a.tag) << 32) | st.q_stats[2], __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
   }
-  if (live == 0) return;
+  if (empty) return;
   const int f0 = fb * p.fw, nf = min(p.fw, a.F - f0);
   const int b0 = bb * p.bw, nb = min(p.bw, p.built - b0);
   for (int j = tid; j < p.n_nodes; j += kWide) {
@@ -466,7 +472,7 @@ __global__ void __launch_bounds__(kScan)
   __shared__ unsigned s_bkey[2][kScan / 64];
   const int f = blockIdx.x % a.F, pair = blockIdx.x / a.F;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  if (st.live[p.depth] == 0) return;
+  if (level_is_empty(st, p.depth)) return;
   const bool usable = a.feature_set == nullptr || a.feature_set[f] != 0;
   const int left    = 2 * pair;
   const bool root   = p.depth == 0;
@@ -666,7 +672,7 @@ __device__ __forceinline__ int2 decide_node(const MidArgs& a, const MidTreeState
 __global__ void __launch_bounds__(kScan)
   mid_decide_kernel(MidArgs a, MidTreeState st, LevelPlan p, int lanes_log)
 {
-  if (st.live[p.depth] == 0) return;
+  if (level_is_empty(st, p.depth)) return;
   const int lanes = 1 << lanes_log, sub = threadIdx.x & (lanes - 1);
   const int j     = (blockIdx.x * kScan + static_cast<int>(threadIdx.x)) >> lanes_log;
   const int2 sp   = decide_node(a, st, p, j < p.n_nodes ? j : -1, sub, lanes, true);
@@ -684,7 +690,7 @@ __global__ void __launch_bounds__(kWide)
   const int r   = blockIdx.x * kRowsApply + 4 * tid;
   uint2 nd      = make_uint2(0xffffffffu, 0xffffffffu);
   if (r < a.N) nd = *reinterpret_cast<const uint2*>(st.row_node + r);
-  if (st.live[p.depth] == 0) return;
+  if (level_is_empty(st, p.depth)) return;
   if constexpr (kDecided) {
     for (int j = tid; j < p.n_nodes; j += kWide) s_split[j] = st.splits[j];
   } else {
@@ -727,7 +733,7 @@ __global__ void __launch_bounds__(kScan) mid_count_kernel(MidArgs a, MidTreeStat
 {
   const int r    = blockIdx.x * kScan + threadIdx.x;
   const int node = r < a.N ? st.row_node[r] : kNone;
-  const bool has = node != kNone && st.live[p.depth] != 0;
+  const bool has = node != kNone && !level_is_empty(st, p.depth);
   const bool built = has && (p.depth == 0 || built_of_pair(st.node_sums, p.level_first, node >> 1, a.K) == node);
   const unsigned long long all = __ballot(has), some = __ballot(built);
   if ((threadIdx.x & 63) == 0) {
@@ -809,11 +815,12 @@ bool mid_tree_fits(int64_t N, int F, int K, int max_depth, int S)
 }
 
 template <typename T, typename BinT>
-static int queue_levels(hipStream_t stream, const MidTreeState& st, const MidArgs& a, LevelMeta* level_totals)
+static int queue_levels(hipStream_t stream, const MidTreeState& st, const MidArgs& a, const DeviceAnswer& answer,
+                        LevelMeta* level_totals)
 {
   int lanes_log = 0;
   while (lanes_log < 6 && (1 << lanes_log) < a.F) lanes_log++;
-  for (int d = 0; d < a.max_depth; d++) {
+  for (int d = 0; d < a.max_depth && (d == 0 || !answer.declined()); d++) {
     const LevelPlan p = plan_level(a.N, a.F, a.K, a.S, d, a.max_depth);
     {
       ProfScope ps(LBT_PROF_HISTOGRAM, stream, 0.0, d);
@@ -901,9 +908,9 @@ int mid_tree_build(hipStream_t stream, const MidTreeState& st, const T* X, int64
     }
   }
   if (st.bin_bytes == 1)
-    LBT_TRY((queue_levels<T, uint8_t>(stream, st, a, level_totals)));
+    LBT_TRY((queue_levels<T, uint8_t>(stream, st, a, answer, level_totals)));
   else
-    LBT_TRY((queue_levels<T, uint16_t>(stream, st, a, level_totals)));
+    LBT_TRY((queue_levels<T, uint16_t>(stream, st, a, answer, level_totals)));
   unsigned flags = 0;
   LBT_TRY(answer.wait(&flags, n_bins));
   *taken = flags == 0;

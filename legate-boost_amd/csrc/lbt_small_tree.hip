@@ -20,7 +20,8 @@
 // by the same functions from the same sums as in the other builder: the trees are identical. One rule of
 // the reference needs the histogram itself: a running sum that is positive in neither half leaves the bin
 // unscanned (build_tree.cu:645). That matters only if some row has a non-positive rounded hessian and a
-// pair other than (0, 0); the prologue reports such rows and the caller takes the other builder.
+// pair other than (0, 0); the prologue reports such rows, the levels behind it then do nothing, and the caller
+// takes the other builder.
 #include <algorithm>
 #include <limits>
 
@@ -169,7 +170,7 @@ __device__ inline void small_quantise(const PrologueArgs& a, const SmallTreeStat
     a.split[0]      = 0.0;
     a.gain[0]       = 0.0;
     st.seg[0]       = make_int2(0, a.N);
-    st.live[0]      = 1;
+    st.live[0]      = s_flags == 0 ? 1 : 0;  // data for the other builder: the levels that are queued have nothing to do
   }
 }
 
@@ -360,7 +361,7 @@ __global__ void __launch_bounds__(kT)
   if (a.depth > 0)
     for (int i = tid * 4; i < a.N; i += kT * 4)
       *reinterpret_cast<uint32_t*>(s_code + i) = *reinterpret_cast<const uint32_t*>(st.code + i);
-  if (live == 0) return;
+  if (live == 0 && a.depth > 0) return;
   if (a.depth == 0) {
     int mine = 0;
     for (int i = tid; i < f; i += kT) mine += st.counts[i];
@@ -372,6 +373,7 @@ __global__ void __launch_bounds__(kT)
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     __syncthreads();
+    if (live == 0) return;  // (the number of bins is reported all the same)
     rp = s_rp;
   }
   if (!usable) {
@@ -866,7 +868,7 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
   a.n_bins = answer.words + 1;
   a.tag    = answer.tag;
   a.l1 = prm.l1_regularization; a.l2 = prm.l2_regularization; a.min_split_gain = prm.min_split_gain;
-  for (int d = 0; d < prm.max_depth; d++) {
+  for (int d = 0; d < prm.max_depth && (d == 0 || !answer.declined()); d++) {
     a.depth       = d;
     a.level_first = static_cast<int>(level_begin(d));
     a.n_nodes     = 1 << d;

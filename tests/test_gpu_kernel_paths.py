@@ -263,6 +263,33 @@ def test_builds_of_one_thread_on_two_streams(rows, monkeypatch):
                 assert torch.equal(getattr(got[i], name), getattr(want[i], name)), (turn, i, name)
 
 
+@pytest.mark.parametrize("n,f,k,depth", [(1, 2, 1, 1), (900, 12, 3, 7), (5000, 9, 1, 13), (9000, 9, 1, 1), (40000, 21, 2, 10)])
+def test_data_for_the_other_builder_leave_the_queue(n, f, k, depth):
+    """Negative hessians are met when the levels of the builders for few rows and medium sizes are being queued: what
+    is queued does nothing, and the general builder's tree is the result, call after call without a wait between."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + f)
+    X = rs.randn(n, f).astype(np.float32)
+    g, h = rs.randn(n, k), rs.rand(n, k) + 0.1
+    bad = h.copy()
+    bad[n // 2] = -0.3
+    Xd, gd, hd, bd = (torch.from_numpy(a).cuda() for a in (X, g, h, bad))
+    kw = dict(max_depth=depth, split_samples=32, seed=9)
+    got = []
+    for turn in range(3):
+        got.append(ops.build_tree(Xd, gd, bd, wait=False, row_leaf=True, **kw))
+        got.append(ops.build_tree(Xd, gd, hd, wait=False, row_leaf=turn == 1, **kw))
+    torch.cuda.synchronize()
+    want = [orc.build_tree(X, g, a, **kw) for a in (bad, h)]
+    for i, r in enumerate(got):
+        _assert_tree(r, want[i % 2])
+        if i % 2 == 0:
+            gu.check_row_leaf(r, X)
+
+
 @pytest.mark.parametrize("f,k", [(13, 2), (13, 4), (13, 5), (13, 8), (13, 9), (100, 8), (100, 9), (100, 17), (200, 2),
                                  (200, 16), (200, 17), (200, 33)])
 def test_predict_shares_the_outputs_out_among_the_lanes_of_a_row(f, k):
