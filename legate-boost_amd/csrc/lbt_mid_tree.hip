@@ -15,10 +15,13 @@
 //   mid_apply_kernel      best features, the nodes' outputs and children (build_tree.cu:740-782), new node
 //                         of every row
 //
-// What the reference's rule on unscanned bins (build_tree.cu:645) could change needs a row whose rounded
-// hessian is not positive: such data take the other builder (see small_tree_build, which has the same
-// condition). Otherwise a scanned histogram is the running sums everywhere, and it does not matter
-// which histograms the reference would have kept.
+// The reference leaves a bin as it was accumulated where neither half of its running sum is positive
+// (build_tree.cu:645). With hessians that are rounded to 0 or more, that is a bin in front of which no row of
+// the node has one, and a sum of grads that is not positive: no split of the node itself, but its sibling
+// is the parent minus that bin. The scan keeps to the rule; the histograms are then the reference's as long as it
+// keeps the same ones, which it does where those of all levels fit its buffer (zeros_kept). Data with a
+// negative rounded hessian, or with one of 0 where they do not fit, take the other builder (see small_tree_build).
+// Otherwise a scanned histogram is the running sums everywhere, and it does not matter which ones are kept.
 #include <algorithm>
 #include <limits>
 #include <type_traits>
@@ -51,6 +54,7 @@ struct MidArgs {
   double l1, l2, min_split_gain;
   int64_t max_nodes;
   int max_depth;
+  bool zeros_kept;  // a rounded hessian of 0 (beside a grad) is no reason to take the other builder
   double* leaf;
   int32_t* feature;
   double* split;
@@ -232,7 +236,7 @@ __global__ void __launch_bounds__(kWide)
       int64_t qg, qh;
       quantise_pair(a.g[e], a.h[e], sg, sh, static_cast<int64_t>(a.seed), row + a.row_offset, k, &qg, &qh);
       if (qg > 2147483647LL || qg < -2147483647LL || qh > 2147483647LL || qh < -2147483647LL) flags |= 2u;
-      if (qh <= 0 && (qg != 0 || qh != 0)) flags |= 1u;
+      if (qh < 0 || (qh == 0 && qg != 0 && !a.zeros_kept)) flags |= 1u;
       st.q[static_cast<int64_t>(k) * st.pitch + row] = make_int2(static_cast<int>(qg), static_cast<int>(qh));
       up += qg > 0 ? static_cast<unsigned long long>(qg) : 0ULL;
       down += qg < 0 ? static_cast<unsigned long long>(-qg) : 0ULL;
@@ -544,11 +548,13 @@ __global__ void __launch_bounds__(kScan)
       const I64Pair ns = st.node_sums[static_cast<int64_t>(p.level_first + node) * a.K + k];
       if (in) {
         const int64_t at = static_cast<int64_t>(k) * fs + static_cast<int64_t>(f) * a.S + bin;
-        hist[static_cast<int64_t>(node) * a.K * fs + at] = I64Pair{g, h};
-        add_gain(gain_n, dead_n, I64Pair{g, h}, ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
+        // the bin as it was accumulated where neither running sum is positive (build_tree.cu:645)
+        const I64Pair nv = g > 0 || h > 0 ? I64Pair{g, h} : v;
+        hist[static_cast<int64_t>(node) * a.K * fs + at] = nv;
+        add_gain(gain_n, dead_n, nv, ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
         if (!root) {
           const I64Pair ss = st.node_sums[static_cast<int64_t>(p.level_first + sib) * a.K + k];
-          const I64Pair sv{pv.grad - g, pv.hess - h};
+          const I64Pair sv{pv.grad - nv.grad, pv.hess - nv.hess};
           hist[static_cast<int64_t>(sib) * a.K * fs + at] = sv;
           add_gain(gain_s, dead_s, sv, ss, inv_g, inv_h, a.l1, reg, a.min_split_gain);
         }
@@ -868,6 +874,9 @@ int mid_tree_build(hipStream_t stream, const MidTreeState& st, const T* X, int64
   a.feature_set = feature_set;
   a.l1 = prm.l1_regularization; a.l2 = prm.l2_regularization; a.min_split_gain = prm.min_split_gain;
   a.max_nodes = prm.max_nodes; a.max_depth = prm.max_depth;
+  // every level's histograms within the reference's buffer, whatever the number of bins (see final_histogram_range)
+  const double buffer = prm.hist_cache_bytes > 0 ? static_cast<double>(prm.hist_cache_bytes) : 1e9;
+  a.zeros_kept        = static_cast<double>(level_end(prm.max_depth - 1)) * K * F * a.S * 16.0 <= buffer;
   a.leaf = leaf; a.feature = feature; a.split = split; a.gain = gain; a.hessian = hessian; a.row_leaf = row_leaf;
   a.answer = answer.words; a.tag = answer.tag;
   int P = 1;

@@ -290,6 +290,43 @@ def test_data_for_the_other_builder_leave_the_queue(n, f, k, depth):
             gu.check_row_leaf(r, X)
 
 
+@pytest.mark.parametrize("n,f,k,depth,s,kind,dtype", [
+    (9000, 6, 1, 5, 64, "low", np.float32),
+    (12000, 33, 1, 8, 256, "span", np.float32),
+    (20001, 7, 2, 6, 300, "most", np.float32),
+    (8200, 5, 3, 10, 512, "output", np.float64),
+    (30000, 12, 1, 9, 100, "most", np.float32),
+])
+def test_medium_sizes_with_hessians_that_round_to_zero(n, f, k, depth, s, kind, dtype):
+    """Rows with a gradient whose hessian rounds to 0 make the reference leave bins unscanned, and their siblings'
+    histograms differ by them (in every one of these cases the tree is another one without that rule). The medium
+    builder keeps to it where the reference would hold all histograms; an explicit budget under which it would not
+    gives the tree of that budget."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + f)
+    X = rs.randn(n, f).astype(dtype)
+    X[:, 0] = np.round(2 * X[:, 0]) / 2
+    g, h = rs.randn(n, k), rs.rand(n, k) + 0.1
+    if kind == "low":  # no hessian where a feature is small: its first bins have a sum of gradients only
+        h[X[:, 1] < -0.5] = 1e-12
+    elif kind == "most":
+        h[rs.rand(n) < 0.95] = 1e-12
+    elif kind == "span":
+        h = 10.0 ** (-10 * rs.rand(n, k))
+    else:  # of one output, of another one
+        h[::3, 0] = 0.0
+        h[X[:, 2] < 0, k - 1] = 1e-12
+    for budget in (0, f * s * k * 16 * 5):
+        cr = orc.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=n, hist_cache_bytes=budget)
+        assert ((cr.quantised[..., 1] == 0) & (cr.quantised[..., 0] != 0)).any()
+        got = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=n, row_leaf=True, hist_cache_bytes=budget)
+        _assert_tree(got, cr)
+        gu.check_row_leaf(got, X)
+
+
 @pytest.mark.parametrize("f,k", [(13, 2), (13, 4), (13, 5), (13, 8), (13, 9), (100, 8), (100, 9), (100, 17), (200, 2),
                                  (200, 16), (200, 17), (200, 33)])
 def test_predict_shares_the_outputs_out_among_the_lanes_of_a_row(f, k):
