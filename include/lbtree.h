@@ -56,10 +56,12 @@ int lbt_release_thread_resources(void);
 /* The eight task scalars of BUILD_TREE in their reference order
  * (legateboost/models/tree.py:121-129, build_tree.cu:1292-1299), plus the
  * histogram-cache budget that the reference hard-codes to 1e9 bytes
- * (build_tree.cu:1004). hist_cache_bytes == 0 selects that constant; a call that asks for no observation point
- * but row_leaf may then keep the histograms of more levels where the workspace has room for them (the tree is
- * the same; lbt_build_tree_workspace_bytes(..., 0) counts up to 4.5e9 bytes of them, a workspace without
- * that room is accepted too). */
+ * (build_tree.cu:1004): the bytes of histograms the call keeps (those of one node, where they are more). Where
+ * nothing but row_leaf is observed the library chooses how it builds within them; the tree is that of the
+ * reference with this budget. hist_cache_bytes == 0 selects the reference's constant; a call that observes nothing
+ * but row_leaf may then keep the histograms of more levels where the workspace has room for them (the tree is the
+ * same; lbt_build_tree_workspace_bytes(..., 0) counts up to 4.5e9 bytes of them, a workspace of
+ * lbt_build_tree_workspace_bytes(..., 1000000000) is accepted too). */
 typedef struct lbt_build_params {
   /* sizeof(lbt_build_params) of the header the caller was built against. The library refuses a
    * value that is not its own, so a struct of another version of this header, or one that was

@@ -1358,13 +1358,17 @@ struct Layout {
 // Room for the histograms of all levels, where the caller leaves the budget to the library: a 64th of the memory.
 constexpr double kWholeTreeBytes = 4.5e9;
 
-// roomy: see build_tree_impl, where a level that outgrows the reference's budget keeps its parents
+// The bytes of histograms a build may keep (where one node needs more: that node's). roomy: see build_tree_impl,
+// where a level that outgrows the reference's budget keeps its parents
+double hist_budget(int64_t cache_bytes, bool roomy)
+{
+  return cache_bytes > 0 ? static_cast<double>(cache_bytes) : (roomy ? kWholeTreeBytes : 1e9);
+}
 size_t hist_bytes_bound(int F, int K, int S, int max_depth, int64_t cache_bytes, bool roomy)
 {
   if (max_depth < 1) return 0;
   const double bpn = static_cast<double>(K) * F * S * 16.0;  // bytes per node with every bin distinct
-  const double max_bytes = cache_bytes > 0 ? static_cast<double>(cache_bytes) : (roomy ? kWholeTreeBytes : 1e9);
-  double a = std::max(max_bytes, bpn);
+  double a = std::max(hist_budget(cache_bytes, roomy), bpn);
   double b = static_cast<double>(level_end(max_depth - 1)) * bpn;
   return static_cast<size_t>(std::min(a, b)) + 256;
 }
@@ -1442,10 +1446,15 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
   const int64_t max_chunks = std::max<int64_t>((static_cast<int64_t>(F) * S + kSplitChunk - 1) / kSplitChunk, F);
   L.partial       = ar.take<Cand>(level_nodes * max_chunks);
   L.left          = K == 1 && max_depth >= 2 && S <= kDirectMaxBins ? ar.take<I64Pair>(level_nodes * F) : nullptr;
-  L.hist_bytes    = hist_bytes_bound(F, K, S, max_depth, cache_bytes, roomy);
-  L.hist          = reinterpret_cast<I64Pair*>(ar.take<char>(L.hist_bytes));
+  // one of the builders at a time uses the room for histograms
+  const bool small    = small_tree_fits(N, F, K, max_depth, S);
+  const size_t mid_bytes = !small && mid_tree_fits(N, F, K, max_depth, S) ? mid_hist_bytes(N, F, K, max_depth, S) : 0;
+  const bool mid      = mid_bytes > 0 && static_cast<double>(mid_bytes) <= hist_budget(cache_bytes, roomy);
+  L.hist_bytes        = hist_bytes_bound(F, K, S, max_depth, cache_bytes, roomy);
+  char* const hist    = ar.take<char>(std::max(L.hist_bytes, mid ? mid_bytes : 0));
+  L.hist              = reinterpret_cast<I64Pair*>(hist);
   L.small = SmallTreeState{};
-  if (small_tree_fits(N, F, K, max_depth, S)) {
+  if (small) {
     SmallTreeState& st    = L.small;
     st.pitch              = (N + 7) / 8 * 8;
     const size_t per_row  = static_cast<size_t>(F) * st.pitch;
@@ -1466,7 +1475,7 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     st.cand        = ar.take<SmallCand>(level_nodes * F);
   }
   L.mid = MidTreeState{};
-  if (L.small.pitch == 0 && mid_tree_fits(N, F, K, max_depth, S)) {
+  if (mid) {
     MidTreeState& st   = L.mid;
     st.pitch           = (N + 255) / 256 * 256;
     st.bin_bytes       = S <= 256 ? 1 : 2;
@@ -1486,9 +1495,11 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     st.q          = ar.take<int2>(static_cast<size_t>(K) * st.pitch);
     st.row_node   = ar.take<uint16_t>(st.pitch);
     st.q_stats    = ar.take<unsigned long long>(4);
-    st.images     = ar.take<unsigned long long>(mid_image_words(N, F, K, max_depth, S));
-    st.hist[0]    = ar.take<I64Pair>(level_hist);
-    st.hist[1]    = ar.take<I64Pair>(level_hist);
+    if (hist != nullptr) {
+      st.hist[0]  = L.hist;
+      st.hist[1]  = L.hist + level_hist;
+      st.images   = reinterpret_cast<unsigned long long*>(L.hist + 2 * level_hist);
+    }
     st.node_sums  = L.node_sums;
     st.scales     = L.scales;
     st.cand       = ar.take<SmallCand>(level_nodes * F);

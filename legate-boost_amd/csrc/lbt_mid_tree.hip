@@ -793,14 +793,16 @@ LevelPlan plan_level(int64_t N, int F, int K, int S, int depth, int max_depth)
 
 }  // namespace
 
-int64_t mid_image_words(int64_t N, int F, int K, int max_depth, int S)
+// Scanned histograms of two levels and the images of the level that has most of them.
+size_t mid_hist_bytes(int64_t N, int F, int K, int max_depth, int S)
 {
-  int64_t most = 0;
+  const int64_t fs = static_cast<int64_t>(K) * F * S;
+  int64_t images   = 0;
   for (int d = 0; d < max_depth; d++) {
     const LevelPlan p = plan_level(N, F, K, S, d, max_depth);
-    most              = std::max(most, static_cast<int64_t>(p.chunks) * p.built * K * F * S);
+    images            = std::max(images, static_cast<int64_t>(p.chunks) * p.built * fs);
   }
-  return most;
+  return static_cast<size_t>(2 * (int64_t(1) << (max_depth - 1)) * fs) * sizeof(I64Pair) + static_cast<size_t>(images) * 8;
 }
 
 // By size: measured against the other builder (one output, depth 8 and 256 samples unless stated): 20,000 x 100

@@ -65,6 +65,21 @@ def test_the_builder_for_few_rows_is_not_offered_what_its_scan_cannot_hold():
     assert q(7733, 13) < q(7732, 13) - 7000 * per_value  # the last size whose thirteen levels fit
 
 
+def test_an_explicit_histogram_budget_bounds_the_histograms():
+    """Sizes of the builder for medium sizes, whose two levels of histograms take more than the budget: one level
+    deeper, which is not its size, must not need less scratch; and a larger budget adds no more than itself."""
+    from lbtree import _lib
+
+    def q(depth, budget):
+        return _lib.lib.lbt_build_tree_workspace_bytes(12000, 180, 1, depth, 512, _lib.LBT_F32, budget)
+
+    node = 180 * 512 * 16
+    for budget in (1, 4 * 10 ** 7, 10 ** 9):
+        assert q(10, budget) <= q(11, budget) and q(10, budget) <= q(10, 1) + budget
+    # the library's own budget: two levels of 512 nodes, 8 bytes a bin for half of one, and no second copy of it
+    assert q(10, 0) <= q(10, 1) + (2 ** 10 + 2 ** 7) * node + (16 << 20)
+
+
 def test_bad_arguments_are_rejected_without_a_gpu():
     from lbtree import _lib
 

@@ -199,6 +199,22 @@ def test_medium_sizes(n, f, k, depth, s, dtype, options):
         gu.check_row_leaf(got, X)
 
 
+def test_medium_sizes_under_an_explicit_budget():
+    """Budgets either side of what the builder's histograms and images take, in a workspace of the size the query
+    names for the budget: the same tree, by that builder or by the general one."""
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(12)
+    n, f, k, depth, s = 12000, 14, 2, 6, 200
+    X, g, h = rs.randn(n, f).astype(np.float32), rs.randn(n, k), rs.rand(n, k) + 0.1
+    cr = orc.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=2)
+    two_levels = 2 * 2 ** (depth - 1) * k * f * s * 16
+    for budget in (1, two_levels - 1, two_levels + (64 << 20), 10 ** 9):
+        ops._workspace.clear()
+        _assert_tree(ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=2, hist_cache_bytes=budget), cr)
+
+
 @pytest.mark.parametrize("case", ["one_sign", "one_row", "negative_hessian", "all_zero"])
 def test_medium_sizes_special_gradients(case):
     """Sums at the edge of the packed 32 bits (all gradients of one sign in one bin; nearly the whole mass in one
