@@ -388,6 +388,36 @@ def test_levels_that_outgrow_the_histogram_budget_give_the_same_tree(n, f, k, s,
             assert torch.equal(getattr(got, name), getattr(want, name)), (budget, name)
 
 
+def test_a_build_does_without_the_room_that_it_cannot_have(monkeypatch):
+    """Where the room for the library's own budget of histograms cannot be had the build takes place in the
+    reference's, and gives the same tree; an explicit budget is not cut."""
+    from lbtree import _lib, ops
+
+    rs = np.random.RandomState(1)
+    n, f, k, depth, s = 9001, 60, 8, 9, 512
+    X, g, h = (torch.from_numpy(a).cuda() for a in (rs.randn(n, f).astype(np.float32), rs.randn(n, k), 0.1 + rs.rand(n, k)))
+    kw = dict(max_depth=depth, split_samples=s, seed=3)
+    want = ops.build_tree(X, g, h, **kw)
+    full, least = (_lib.lib.lbt_build_tree_workspace_bytes(n, f, k, depth, s, _lib.LBT_F32, b) for b in (0, 10 ** 9))
+    assert full > least + 10 ** 9
+    plain, asked = ops._get_workspace, []
+
+    def scarce(nbytes, device):
+        asked.append(nbytes)
+        if nbytes > least:
+            raise torch.OutOfMemoryError("not that much")
+        return plain(nbytes, device)
+
+    ops._workspace.clear()
+    monkeypatch.setattr(ops, "_get_workspace", scarce)
+    got = ops.build_tree(X, g, h, **kw)
+    assert asked == [full, least]
+    for name in ("leaf_value", "feature", "split_value", "gain", "hessian"):
+        assert torch.equal(getattr(got, name), getattr(want, name)), name
+    with pytest.raises(torch.OutOfMemoryError):
+        ops.build_tree(X, g, h, hist_cache_bytes=4 * 10 ** 9, **kw)
+
+
 @pytest.mark.parametrize("n,f,k,depth,dtype", [(1, 3, 1, 1, np.float32), (1023, 7, 1, 5, np.float64),
                                                (1025, 50, 8, 8, np.float32), (70001, 13, 3, 8, np.float32),
                                                (5003, 9, 9, 8, np.float64), (5003, 9, 1, 11, np.float32), (3001, 200, 1, 5, np.float32),
