@@ -1,6 +1,7 @@
 """Thin, allocation-owning wrappers over the C ABI. torch only provides device
 memory and the current stream; all computation happens in liblbtree.so."""
 import ctypes as C
+import threading
 
 import numpy as np
 import torch
@@ -37,17 +38,34 @@ def _check_x(X):
     return X
 
 
-_workspace = {}
+class _Scratch(threading.local):
+    """Scratch buffers of this host thread by (device, stream): builds that may overlap, on two streams or queued
+    by two threads, must not share one. What a thread holds is freed when it ends."""
+
+    def __init__(self):
+        self.held = {}
+
+    def clear(self):
+        self.held.clear()
+
+
+_workspace = _Scratch()
 
 
 def _get_workspace(nbytes, device):
-    """One grow-only scratch buffer per device, reused by successive calls."""
-    ws = _workspace.get(device)
+    """One grow-only scratch buffer per thread, device and stream, reused by successive calls."""
+    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    ws = _workspace.held.get(key)
     if ws is None or ws.numel() < nbytes:
-        _workspace[device] = None
+        _workspace.held[key] = None
         ws = torch.empty(int(nbytes), dtype=torch.uint8, device=device)
-        _workspace[device] = ws
+        _workspace.held[key] = ws
     return ws
+
+
+def release_workspace():
+    """Gives the scratch buffers that builds of this thread keep between calls back to torch's allocator."""
+    _workspace.clear()
 
 
 class BuildResult:

@@ -242,22 +242,13 @@ def test_medium_sizes_special_gradients(case):
 
 
 @pytest.mark.parametrize("rows", [(700, 900), (700, 9000), (9000, 9500)])
-def test_builds_of_one_thread_on_two_streams(rows, monkeypatch):
+def test_builds_of_one_thread_on_two_streams(rows):
     """All builds of a thread hear from their kernels through the same pinned words. Calls without observation points
     beside calls that want the number of bins, in turn on two streams and with the words given back in between: every
     call has to get its own answer, and no store of an earlier one may come after it has returned."""
     from lbtree import _lib, ops
 
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]
-    own = {}
-
-    def workspace(nbytes, device):
-        key = torch.cuda.current_stream().cuda_stream
-        if key not in own or own[key].numel() < nbytes:
-            own[key] = torch.empty(int(nbytes), dtype=torch.uint8, device=device)
-        return own[key]
-
-    monkeypatch.setattr(ops, "_get_workspace", workspace)
     calls, want = [], []
     for i, n in enumerate(rows):
         rs = np.random.RandomState(n)
@@ -416,6 +407,32 @@ def test_a_build_does_without_the_room_that_it_cannot_have(monkeypatch):
         assert torch.equal(getattr(got, name), getattr(want, name)), name
     with pytest.raises(torch.OutOfMemoryError):
         ops.build_tree(X, g, h, hist_cache_bytes=4 * 10 ** 9, **kw)
+
+
+def test_every_thread_and_stream_has_a_workspace_of_its_own():
+    """Builds that may overlap do not share scratch; a thread's is reused call after call, and given back."""
+    import threading
+
+    from lbtree import ops
+
+    device = torch.device("cuda", torch.cuda.current_device())
+
+    def scratch():
+        return ops._get_workspace(1000, device)
+
+    ops.release_workspace()
+    first, side = scratch(), torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        second = scratch()
+        assert scratch() is second
+    others = []
+    t = threading.Thread(target=lambda: others.append(scratch()))
+    t.start()
+    t.join()
+    assert len({first.data_ptr(), second.data_ptr(), others[0].data_ptr()}) == 3
+    assert scratch() is first and ops._get_workspace(900, device) is first and ops._get_workspace(2000, device) is not first
+    ops.release_workspace()
+    assert not ops._workspace.held
 
 
 @pytest.mark.parametrize("n,f,k,depth,dtype", [(1, 3, 1, 1, np.float32), (1023, 7, 1, 5, np.float64),
