@@ -1447,9 +1447,10 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
   L.partial       = ar.take<Cand>(level_nodes * max_chunks);
   L.left          = K == 1 && max_depth >= 2 && S <= kDirectMaxBins ? ar.take<I64Pair>(level_nodes * F) : nullptr;
   // one of the builders at a time uses the room for histograms
-  const bool small    = small_tree_fits(N, F, K, max_depth, S);
-  const size_t mid_bytes = !small && mid_tree_fits(N, F, K, max_depth, S) ? mid_hist_bytes(N, F, K, max_depth, S) : 0;
-  const bool mid      = mid_bytes > 0 && static_cast<double>(mid_bytes) <= hist_budget(cache_bytes, roomy);
+  const size_t mid_bytes = mid_tree_fits(N, F, K, max_depth, S) ? mid_hist_bytes(N, F, K, max_depth, S) : 0;
+  bool mid               = mid_bytes > 0 && static_cast<double>(mid_bytes) <= hist_budget(cache_bytes, roomy);
+  const bool small       = small_tree_fits(N, F, K, max_depth, S) && !(mid && mid_beats_small(N, F, K, max_depth, S));
+  mid                    = mid && !small;
   L.hist_bytes        = hist_bytes_bound(F, K, S, max_depth, cache_bytes, roomy);
   char* const hist    = ar.take<char>(std::max(L.hist_bytes, mid ? mid_bytes : 0));
   L.hist              = reinterpret_cast<I64Pair*>(hist);
@@ -2170,7 +2171,7 @@ static int build_tree_entry(void* stream, const void* X, int32_t x_dtype, int64_
   hipStream_t s = static_cast<hipStream_t>(stream);
   int rc        = LBT_OK;
   bool done     = false;
-  // few rows: the builder that keeps no histograms, unless the caller wants to see what it does not have
+  // the builders for few rows and medium sizes, unless the caller wants to see what they do not have
   if (lbt::observes_nothing(taps) && (L.small.order[0] != nullptr || L.mid.bins != nullptr)) {
     int32_t* const row_leaf = taps ? taps->row_leaf : nullptr;
     int32_t* const n_bins   = taps ? &taps->n_bins : nullptr;

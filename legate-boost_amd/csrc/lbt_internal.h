@@ -582,6 +582,7 @@ struct MidTreeState {
   int32_t* live;          // [max_depth + 1]
 };
 bool mid_tree_fits(int64_t N, int F, int K, int max_depth, int S);
+bool mid_beats_small(int64_t N, int F, int K, int max_depth, int S);
 // Bytes from hist[0] on: hist[0], hist[1] and images, one behind the other.
 size_t mid_hist_bytes(int64_t N, int F, int K, int max_depth, int S);
 // As small_tree_build.

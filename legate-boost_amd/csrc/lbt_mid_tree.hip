@@ -822,6 +822,25 @@ bool mid_tree_fits(int64_t N, int F, int K, int max_depth, int S)
   return values * plan_level(N, F, K, S, max_depth - 1, max_depth).n_bb <= kMidMaxValues;
 }
 
+// Of two builders that both could, the one for few rows or this one. A level costs the first less to begin with and
+// more per entry (one workgroup per feature walks them in order, output by output); here it is the histograms that
+// count, and a scan workgroup per node and feature. The two sums are times of a tree in us, fitted to 190 shapes (300
+// to 8192 rows, 3 to 500 features, 1 to 16 outputs, depth 2 to 10, 64 to 1024 samples, float and double) to within a
+// tenth or so, hence the 15 % in favour of the first: so none of the shapes where this builder is taken is more than 3 %
+// slower for it. Both, few rows against medium: 10 features, depth 8 at 1000, 4096 and 8192 rows 128, 180, 254 and 179,
+// 198, 205; 8192 x 32, depth 6 205 and 155; 8192 x 100, depth 8 262 and 290; 20 features, 4 outputs, depth 6 at
+// 1000, 2048 and 8192 rows 160, 201, 601 and 166, 180, 197.
+bool mid_beats_small(int64_t N, int F, int K, int max_depth, int S)
+{
+  const double d = max_depth, n = static_cast<double>(N), f = F, k = K;
+  const double small_us = 25.0 + d * (8.7 + 2.0 * k + 1.8e-3 * n * k * (N > 4096 && K > 1 ? 1.5 : 1.0) + 7.1e-6 * n * f);
+  const double nodes = static_cast<double>(int64_t(1) << max_depth), tiles = (S + kScan - 1) / kScan;
+  // histograms of all nodes in MB, or of those that rows reach: four bins per value and level
+  const double hist_mb = std::min(nodes * f * S * k * 16.0, n * f * k * d * 64.0) / 1048576.0;
+  const double mid_us  = 16.0 + d * (19.5 + 1.14 * k * tiles) + 0.29 * hist_mb + 1.0e-3 * nodes * f * k * tiles + 1.74e-6 * n * f * k * d;
+  return 1.15 * mid_us < small_us;
+}
+
 template <typename T, typename BinT>
 static int queue_levels(hipStream_t stream, const MidTreeState& st, const MidArgs& a, const DeviceAnswer& answer,
                         LevelMeta* level_totals)

@@ -83,6 +83,13 @@ def _assert_tree(got, cr):
     (7733, 3, 1, 13, 64, np.float32),      # the most rows at all
     (8192, 3, 1, 13, 64, np.float64),
     (8192, 4, 4, 13, 32, np.float32),
+    (8192, 5, 4, 11, 64, np.float32),      # deeper than the medium builder takes: several outputs at the most rows,
+    (2049, 4, 16, 11, 256, np.float32),    # and the most outputs
+    (6900, 10, 1, 8, 256, np.float32),     # either side of where the medium builder is the faster one
+    (7300, 10, 1, 8, 256, np.float32),
+    (1500, 20, 4, 6, 256, np.float32),
+    (2000, 20, 4, 6, 256, np.float64),
+    (600, 3, 16, 2, 64, np.float32),
 ])
 def test_few_rows(n, f, k, depth, s, dtype):
     """The builder for few rows at the edges of what it takes (and just past them), with constant and
@@ -270,10 +277,13 @@ def test_builds_of_one_thread_on_two_streams(rows):
                 assert torch.equal(getattr(got[i], name), getattr(want[i], name)), (turn, i, name)
 
 
-@pytest.mark.parametrize("n,f,k,depth", [(1, 2, 1, 1), (900, 12, 3, 7), (5000, 9, 1, 13), (9000, 9, 1, 1), (40000, 21, 2, 10)])
-def test_data_for_the_other_builder_leave_the_queue(n, f, k, depth):
-    """Negative hessians are met when the levels of the builders for few rows and medium sizes are being queued: what
-    is queued does nothing, and the general builder's tree is the result, call after call without a wait between."""
+@pytest.mark.parametrize("n,f,k,depth,hessian", [(1, 2, 1, 1, -0.3), (900, 12, 3, 7, -0.3), (5000, 9, 1, 13, -0.3),
+                                                 (900, 12, 3, 7, 1e-13), (5000, 9, 1, 13, 1e-13),
+                                                 (9000, 9, 1, 1, -0.3), (40000, 21, 2, 10, -0.3)])
+def test_data_for_the_other_builder_leave_the_queue(n, f, k, depth, hessian):
+    """Negative hessians (for the builder for few rows also those that round to 0) are met when the levels of the
+    builders for few rows and medium sizes are being queued: what is queued does nothing, and the general builder's
+    tree is the result, call after call without a wait between."""
     import gpu_util as gu
     import oracle_lib as orc
     from lbtree import ops
@@ -282,7 +292,7 @@ def test_data_for_the_other_builder_leave_the_queue(n, f, k, depth):
     X = rs.randn(n, f).astype(np.float32)
     g, h = rs.randn(n, k), rs.rand(n, k) + 0.1
     bad = h.copy()
-    bad[n // 2] = -0.3
+    bad[n // 2:] = hessian
     Xd, gd, hd, bd = (torch.from_numpy(a).cuda() for a in (X, g, h, bad))
     kw = dict(max_depth=depth, split_samples=32, seed=9)
     got = []
