@@ -7,6 +7,15 @@
 // bins) adds its rows, scans its features' bins and keeps the best split of each. What bounds it is the
 // gather of the records and the evaluation of the bins; 64 bins without a row cost one comparison.
 //
+// A tree need not be balanced: with gradients that are mostly noise one node of a level can hold nearly all rows, and
+// its few workgroups then were the whole level (1,000,000 x 50 with 512 samples, depth 12, noise: 3.55 ms a tree, where
+// histograms in memory took 2.55; 2,000,000 x 80, depth 11 3.93 and 2.14). So the rows of a node of more than 16384 are
+// dealt to workgroups by ranges of 8192 positions; each adds its sums to the node's histogram in memory, and the
+// last one to finish scans it: 2.07 and 2.24 ms, and 1.95 as before where the tree is balanced. It needs 8 bytes
+// per bin and 16384 rows, in the room of the histograms that are not kept. Shorter ranges add more often (4096: 2.56 and
+// 2.53 ms), longer ones leave nodes that fit none to one workgroup (16384: 2.01 and 2.13, but 250,000 x 43 1.36
+// where 8192 takes 1.20).
+//
 // Only where every rounded hessian is positive: a scanned histogram is then the running sums everywhere
 // (build_tree.cu:645 leaves nothing unscanned) and it does not matter that nothing is derived by subtraction.
 #include "lbt_device.h"
@@ -29,32 +38,17 @@ __device__ __forceinline__ I64Pair unpack_sums(unsigned long long w, int64_t up,
   return I64Pair{g, static_cast<int64_t>(static_cast<uint32_t>(w))};
 }
 
+constexpr int kDirectRange = 8192;              // positions of a range
+constexpr int kDirectLarge = 2 * kDirectRange;  // rows of a node that one workgroup takes: a range meets at most two larger ones
+
+// The rows at positions [begin, end) into the LDS histograms of the nf features of a piece, [kPer][width].
 template <typename BinT>
-__global__ void __launch_bounds__(kDirectThreads) direct_split_kernel(DirectLevel a, int pieces, int width)
+__device__ __forceinline__ void add_rows(const DirectLevel& a, const RecInfo& ri, int piece, int nf, int begin, int end,
+                                         int width, unsigned long long* s_hist)
 {
-  constexpr int kPer = 16 / sizeof(BinT);  // features of a workgroup
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  unsigned long long* s_hist = reinterpret_cast<unsigned long long*>(smem_raw);  // [kPer][width]
-  // the pieces of a node on one XCD, one after the other: they read the same cache lines
-  const int j     = static_cast<int>(blockIdx.x >> 3) / pieces * 8 + static_cast<int>(blockIdx.x & 7);
-  int piece       = static_cast<int>(blockIdx.x >> 3) % pieces;
-  if (j >= a.n_nodes) return;
-  const int node   = a.level_first + j;
-  const I64Pair ns = a.node_sums[node];
-  if (ns.hess <= 0) return;
-  int group = 0;
-  for (; group < a.n_groups - 1; group++) {
-    const int here = (a.rec[group].bins_end + 15) / 16;
-    if (piece < here) break;
-    piece -= here;
-  }
-  const RecInfo ri = a.rec[group];
-  const int f0 = a.groups[group] + piece * kPer, nf = min(kPer, a.groups[group + 1] - f0);
-  const int tid = threadIdx.x, lane = tid & 63;
-  for (int i = tid; i < nf * width; i += kDirectThreads) s_hist[i] = 0;
-  __syncthreads();
+  constexpr int kPer = 16 / sizeof(BinT);
+  const int tid      = threadIdx.x;
   const unsigned char* const cache = static_cast<const unsigned char*>(a.binned) + ri.base;
-  const int begin = a.seg[j], end = a.seg[j + 1];
   for (int i = begin + tid; i < end; i += kDirectThreads) {
     const unsigned char* r = cache + static_cast<int64_t>(a.rows[i]) * ri.stride;
     const uint4 w          = *reinterpret_cast<const uint4*>(r + piece * 16);
@@ -69,7 +63,13 @@ __global__ void __launch_bounds__(kDirectThreads) direct_split_kernel(DirectLeve
         atomicAdd(s_hist + v * width + bin, word);
       }
   }
-  __syncthreads();
+}
+
+// The best split of each of the features [f0, f0 + nf) of node j from its histograms in the LDS.
+__device__ __forceinline__ void scan_features(const DirectLevel& a, int j, const I64Pair& ns, int f0, int nf, int width,
+                                              const unsigned long long* s_hist)
+{
+  const int tid = threadIdx.x, lane = tid & 63;
   const int64_t root = a.node_sums[0].grad, all = (int64_t(1) << 31) + a.n_rows + 1024;
   const int64_t up = (all + root) / 2 + 1, down = (all - root) / 2 + 1;
   const double inv_g = a.scales[2], inv_h = a.scales[3];
@@ -121,6 +121,102 @@ __global__ void __launch_bounds__(kDirectThreads) direct_split_kernel(DirectLeve
   }
 }
 
+// Piece `part` of all records' pieces: its record group, its number there, its first feature and how many.
+struct Piece {
+  RecInfo rec;
+  int number, f0, nf;
+};
+template <typename BinT>
+__device__ __forceinline__ Piece piece_of(const DirectLevel& a, int part)
+{
+  constexpr int kPer = 16 / sizeof(BinT);
+  int group          = 0;
+  for (; group < a.n_groups - 1; group++) {
+    const int here = (a.rec[group].bins_end + 15) / 16;
+    if (part < here) break;
+    part -= here;
+  }
+  const int f0 = a.groups[group] + part * kPer;
+  return Piece{a.rec[group], part, f0, min(kPer, a.groups[group + 1] - f0)};
+}
+
+// The large nodes that lie in a range of positions: one may hold its first position, one may begin inside and go on
+// behind it. What the range adds of a node goes to the node's histogram in memory; the last of its ranges to arrive
+// finds the splits.
+template <typename BinT>
+__device__ __forceinline__ void add_range(const DirectLevel& a, int range, int part, int pieces, int width,
+                                          unsigned long long* s_hist)
+{
+  constexpr int kPer = 16 / sizeof(BinT);
+  const int tid   = threadIdx.x;
+  const int first = range * kDirectRange;
+  const int last  = static_cast<int>(min(a.n_rows, static_cast<int64_t>(first) + kDirectRange));
+  for (int side = 0; side < 2; side++) {
+    const int j = side == 0 ? a.block_seg[first / a.slab] : (last < a.n_rows ? a.block_seg[last / a.slab] : -1);
+    if (j < 0) continue;
+    const int begin = a.seg[j], end = a.seg[j + 1];
+    if (end - begin <= kDirectLarge || (side == 1 && (begin <= first || begin >= last))) continue;
+    const Piece p = piece_of<BinT>(a, part);
+    for (int i = tid; i < p.nf * width; i += kDirectThreads) s_hist[i] = 0;
+    __syncthreads();
+    add_rows<BinT>(a, p.rec, p.number, p.nf, max(first, begin), min(last, end), width, s_hist);
+    __syncthreads();
+    // large nodes begin more than kDirectLarge positions apart: a slot each. Slots and counters are zero between nodes.
+    const int64_t slot      = static_cast<int64_t>(begin / kDirectLarge) * pieces + part;
+    unsigned long long* sum = a.large + slot * kPer * width;
+    for (int i = tid; i < p.nf * width; i += kDirectThreads)
+      if (s_hist[i] != 0) atomicAdd(sum + i, s_hist[i]);
+    __threadfence();
+    __syncthreads();
+    // (the answer goes through the histograms' LDS: a word more and only four workgroups of 512 bins share a CU)
+    if (tid == 0) {
+      const int ranges = (end - 1) / kDirectRange - begin / kDirectRange + 1;
+      s_hist[0]        = atomicAdd(a.arrivals + slot, 1) + 1 == ranges ? 1 : 0;
+    }
+    __syncthreads();
+    const bool last_of_node = s_hist[0] != 0;
+    __syncthreads();
+    if (!last_of_node) continue;
+    __threadfence();
+    for (int i = tid; i < p.nf * width; i += kDirectThreads) {
+      s_hist[i] = __hip_atomic_load(sum + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sum[i]    = 0;
+    }
+    if (tid == 0) a.arrivals[slot] = 0;
+    __syncthreads();
+    scan_features(a, j, a.node_sums[a.level_first + j], p.f0, p.nf, width, s_hist);
+    __syncthreads();
+  }
+}
+
+// Workgroups [0, large_blocks): (range of positions, piece), the parts of large nodes that lie in it. The others:
+// (node, piece), the smaller nodes. The pieces of a range (a node) on one XCD, one after the other: they read the same
+// cache lines.
+template <typename BinT>
+__global__ void __launch_bounds__(kDirectThreads)
+  direct_split_kernel(DirectLevel a, int pieces, int width, int ranges, int large_blocks)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  unsigned long long* s_hist = reinterpret_cast<unsigned long long*>(smem_raw);  // [16 / sizeof(BinT)][width]
+  if (static_cast<int>(blockIdx.x) < large_blocks) {
+    const int id = static_cast<int>(blockIdx.x), range = (id >> 3) / pieces * 8 + (id & 7);
+    if (range < ranges) add_range<BinT>(a, range, (id >> 3) % pieces, pieces, width, s_hist);
+    return;
+  }
+  const int id = static_cast<int>(blockIdx.x) - large_blocks;
+  const int j  = (id >> 3) / pieces * 8 + (id & 7);
+  if (j >= a.n_nodes) return;
+  const I64Pair ns = a.node_sums[a.level_first + j];
+  const int begin = a.seg[j], end = a.seg[j + 1];
+  if (ns.hess <= 0 || end - begin > kDirectLarge) return;
+  const Piece p = piece_of<BinT>(a, (id >> 3) % pieces);
+  for (int i = threadIdx.x; i < p.nf * width; i += kDirectThreads) s_hist[i] = 0;
+  __syncthreads();
+  add_rows<BinT>(a, p.rec, p.number, p.nf, begin, end, width, s_hist);
+  __syncthreads();
+  scan_features(a, j, ns, p.f0, p.nf, width, s_hist);
+}
+
 // The best feature of every node and what follows from it (build_tree.cu:740-782), one wave per node.
 __global__ void __launch_bounds__(kDirectThreads) direct_apply_kernel(DirectLevel a)
 {
@@ -163,16 +259,31 @@ __global__ void __launch_bounds__(kDirectThreads) direct_apply_kernel(DirectLeve
 
 }  // namespace
 
-int direct_level_launch(hipStream_t stream, const DirectLevel& a, const HistSetup& hs)
+size_t direct_large_words(const HistSetup& hs, int64_t n_rows)
 {
-  const unsigned grid = static_cast<unsigned>((a.n_nodes + 7) / 8 * 8) * static_cast<unsigned>(hs.pieces);
+  return n_rows <= kDirectLarge ? 0 : static_cast<size_t>(n_rows / kDirectLarge + 1) * hs.pieces * (16 / hs.bin_bytes) * hs.max_bins;
+}
+
+size_t direct_large_bytes(const HistSetup& hs, int64_t n_rows)
+{
+  const size_t counters = static_cast<size_t>(n_rows / kDirectLarge + 1) * hs.pieces * sizeof(int32_t);
+  return n_rows <= kDirectLarge ? 0 : direct_large_words(hs, n_rows) * sizeof(unsigned long long) + (counters + 15) / 16 * 16;
+}
+
+int direct_level_launch(hipStream_t stream, DirectLevel a, const HistSetup& hs)
+{
+  LBT_REQUIRE(kDirectRange % a.slab == 0, "ranges of positions are whole slabs");
+  a.arrivals          = reinterpret_cast<int32_t*>(a.large + direct_large_words(hs, a.n_rows));
+  const int ranges    = a.n_rows <= kDirectLarge ? 0 : ceil_div(a.n_rows, kDirectRange);
+  const int large     = (ranges + 7) / 8 * 8 * hs.pieces;
+  const unsigned grid = static_cast<unsigned>(large) + static_cast<unsigned>((a.n_nodes + 7) / 8 * 8) * static_cast<unsigned>(hs.pieces);
   const size_t lds    = static_cast<size_t>(16 / hs.bin_bytes) * hs.max_bins * sizeof(unsigned long long);
   {
     ProfScope ps(LBT_PROF_HISTOGRAM, stream);
     if (hs.bin_bytes == 1)
-      direct_split_kernel<uint8_t><<<grid, kDirectThreads, lds, stream>>>(a, hs.pieces, hs.max_bins);
+      direct_split_kernel<uint8_t><<<grid, kDirectThreads, lds, stream>>>(a, hs.pieces, hs.max_bins, ranges, large);
     else
-      direct_split_kernel<uint16_t><<<grid, kDirectThreads, lds, stream>>>(a, hs.pieces, hs.max_bins);
+      direct_split_kernel<uint16_t><<<grid, kDirectThreads, lds, stream>>>(a, hs.pieces, hs.max_bins, ranges, large);
   }
   ProfScope ps(LBT_PROF_SPLIT, stream);
   direct_apply_kernel<<<static_cast<unsigned>((a.n_nodes + 3) / 4), kDirectThreads, 0, stream>>>(a);

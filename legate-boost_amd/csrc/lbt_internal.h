@@ -491,6 +491,10 @@ struct DirectLevel {
   const int32_t* groups;
   const int32_t* rows;
   const int32_t* seg;
+  const int32_t* block_seg;  // node that holds position b * slab (-1: a row that has stopped)
+  int slab;
+  unsigned long long* large;  // histograms of large nodes, direct_large_bytes, all zero between nodes and levels
+  int32_t* arrivals;          // ... of which counters (set by direct_level_launch)
   const int32_t* row_pointers;
   const uint8_t* feature_set;
   const double* scales;
@@ -505,7 +509,8 @@ struct DirectLevel {
   double* gain;
   int32_t* split_bin;
 };
-int direct_level_launch(hipStream_t stream, const DirectLevel& a, const HistSetup& hs);
+size_t direct_large_bytes(const HistSetup& hs, int64_t n_rows);  // multiple of 16
+int direct_level_launch(hipStream_t stream, DirectLevel a, const HistSetup& hs);
 
 // ---------------------------------------------------------------- builder for few rows
 // (lbt_small_tree.hip)

@@ -507,6 +507,34 @@ def test_levels_without_histograms_in_memory_give_the_oracles_tree(n, f, s, dept
         assert np.array_equal(gu.cpu(got.feature), cr.feature)
 
 
+@pytest.mark.parametrize("n,f,s,depth,kind", [(16385, 3, 64, 11, "outliers"), (30001, 7, 256, 11, "outliers"), (60000, 5, 300, 12, "noise"),
+                                              (70001, 20, 512, 11, "one_split"), (65536, 70, 64, 11, "stopped")])
+def test_deep_levels_with_one_large_node(n, f, s, depth, kind):
+    """Trees that are not balanced: nodes of more rows than one workgroup takes, which begin and end inside a range of
+    positions, beside small ones and behind rows that have stopped. Call after call: the sums of a large node have to
+    be zero again when the next one begins."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(n)
+    X = rs.randn(n, f).astype(np.float32)
+    g, h = rs.randn(n, 1), 0.5 + rs.rand(n, 1)
+    if kind == "outliers":
+        g = g ** 9
+    elif kind == "one_split":
+        g = 0.1 * g + 5.0 * (X[:, :1] > 3.0)
+    elif kind == "stopped":  # a third of the rows ends in leaves early, the others stay together for long
+        g = np.where(X[:, :1] > 0.5, 1e6, g ** 9)
+    kw = dict(max_depth=depth, split_samples=s, seed=4)
+    cr = orc.build_tree(X, g, h, **kw)
+    Xd, gd, hd = (torch.from_numpy(a).cuda() for a in (X, g, h))
+    for _ in range(3):
+        got = ops.build_tree(Xd, gd, hd, row_leaf=True, **kw)
+        _assert_tree(got, cr)
+    gu.check_row_leaf(got, Xd)
+
+
 @pytest.mark.parametrize("f,k,n_trees", [(13, 1, 45), (13, 3, 45), (13, 1, 3), (100, 1, 45), (100, 9, 7), (200, 1, 45)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_predict_takes_more_lanes_per_row_for_few_rows(f, k, n_trees, dtype):
