@@ -740,7 +740,7 @@ __global__ void zero_doubles_kernel(double* a, int64_t n)
 // into the LDS first (67 us). row_leaf, if given, receives the node every row stops in.
 constexpr int kUpdateThreads      = 1024;
 constexpr int kUpdateLdsDoubles   = 8192;  // node sums up to 64 KB
-constexpr int kStagedThreads      = 256;
+constexpr int kStagedThreads      = 512;  // tiles of wide rows have fewer of them, but all threads stage (256: 75 us a tree where 512 take 67)
 constexpr int kStagedBytesPerStep = 80;    // a scattered line costs as much as about 100 bytes in sequence
 constexpr size_t kStagedTile      = 60 * 1024;
 enum class UpdateMode { kGlobal, kLds, kStaged };  // where sums and tree lie; kStaged: rows in the LDS too
@@ -843,10 +843,10 @@ __global__ void __launch_bounds__(kUpdateThreads) update_accumulate_kernel(const
   if constexpr (kUseLds) {
     __syncthreads();
     for (int i = tid; i < n_sums; i += threads) {
-      const int k = i / a.n_nodes, node = i - k * a.n_nodes;
-      const double gv = s_sum[i], hv = s_sum[n_sums + i];
-      if (gv != 0.0) unsafeAtomicAdd(&a.G[node * a.K + k], gv);
-      if (hv != 0.0) unsafeAtomicAdd(&a.H[node * a.K + k], hv);
+      const int node = i / a.K, at = (i - node * a.K) * a.n_nodes + node;
+      const double gv = s_sum[at], hv = s_sum[n_sums + at];
+      if (gv != 0.0) unsafeAtomicAdd(&a.G[i], gv);
+      if (hv != 0.0) unsafeAtomicAdd(&a.H[i], hv);
     }
   }
 }
