@@ -1,4 +1,4 @@
-// Device functions shared by the two tree builders (lbt_build_tree.hip, lbt_small_tree.hip).
+// Device functions shared by the tree builders (lbt_build_tree.hip, lbt_small_tree.hip, lbt_mid_tree.hip, lbt_direct_level.hip).
 #pragma once
 
 #include <limits>

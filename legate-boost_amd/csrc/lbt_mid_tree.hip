@@ -756,7 +756,7 @@ __global__ void __launch_bounds__(kScan) mid_count_kernel(MidArgs a, MidTreeStat
 // One level's plan. A workgroup of the histogram pass keeps fw features of bw nodes in the LDS; near the root
 // several features share the loads of a row, deeper a feature's nodes fill the LDS and then come in
 // blocks. Ranges of rows are cut until there is a workgroup for every CU or so, not below 3072 rows (1024 up to
-// 16 ranges), and only so many that their images (written here, read by the scan) stay within 64 MB.
+// 16 ranges), and only so many that their images (written here, read by the scan) stay within 64 MB (one always).
 LevelPlan plan_level(int64_t N, int F, int K, int S, int depth, int max_depth)
 {
   LevelPlan p;
@@ -776,7 +776,7 @@ LevelPlan plan_level(int64_t N, int F, int K, int S, int depth, int max_depth)
   const bool pairs    = static_cast<size_t>(p.fw) * p.bw * S * 8 <= 72 * 1024;
   int64_t chunks      = std::max<int64_t>(1, (pairs ? 512 : 256) / inner);
   // (three quarters of a workgroup's threads have rows: with 1024 rows a range, most of them had none and the scan
-  // added up twice the images: 100,000 x 32, 10 rounds, 2.07 -> 1.94 ms; 60,000 x 20 with 4 outputs -5 %)
+  // added up twice the images: 100,000 x 32, 10 rounds, 2.06 -> 1.87 ms; 60,000 x 20 with 4 outputs -9 %)
   chunks              = std::min(chunks, std::max<int64_t>({1, N / 3072, std::min<int64_t>(16, N / 1024)}));
   chunks              = std::min<int64_t>(chunks, 64);
   chunks              = std::min(chunks, std::max<int64_t>(1, (int64_t(64) << 20) / image));
@@ -808,12 +808,12 @@ size_t mid_hist_bytes(int64_t N, int F, int K, int max_depth, int S)
   return static_cast<size_t>(2 * (int64_t(1) << (max_depth - 1)) * fs) * sizeof(I64Pair) + static_cast<size_t>(images) * 8;
 }
 
-// By size: measured against the other builder (one output, depth 8 and 256 samples unless stated): 20,000 x 100
-// 521 -> 189 us at depth 6, 250,000 x 43 755 -> 350, 500,000 x 50 863 -> 417, 1,000,000 x 30 996 -> 418,
-// 2,000,000 x 40 1155 -> 834, 600,000 x 50 with 8 outputs 1745 -> 1535, 2,000,000 x 80 1444 -> 1174. Every pass
-// reads all rows, and where a level's nodes come in several blocks once per block (800,000 x 40 with 512
-// samples at depth 10, eight blocks: 1444 -> 1404), so what counts is values times blocks of the last
-// level: at 240 million the two are even (6,000,000 x 40 2100 -> 2108, 800,000 x 300 2034 -> 2113).
+// By size: measured against the general builder (one output, depth 8 and 256 samples unless stated), us: 20,000 x 100
+// 470 -> 191 at depth 6, 250,000 x 43 764 -> 323, 500,000 x 50 849 -> 396, 1,000,000 x 30 955 -> 399, 2,000,000 x 40
+// 1139 -> 763, 600,000 x 50 with 8 outputs 1652 -> 1511, 2,000,000 x 80 1398 -> 1133. Every pass reads all rows, and
+// where a level's nodes come in several blocks once per block (800,000 x 40 with 512 samples at depth 10, eight
+// blocks: 1323 -> 1231), so what counts is values times blocks of the last level: at 240 million the two are about
+// even (6,000,000 x 40 2034 -> 1955, 800,000 x 300 1952 -> 1913, 3,000,000 x 80 1752 -> 1672).
 bool mid_tree_fits(int64_t N, int F, int K, int max_depth, int S)
 {
   if (max_depth < 1 || max_depth > kMidMaxDepth || K > kMidMaxOutputs || S > LBT_MAX_SPLIT_SAMPLES) return false;

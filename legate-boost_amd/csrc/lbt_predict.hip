@@ -308,7 +308,7 @@ __device__ __forceinline__ void add_in_order(double& run, const double (&val)[S:
 // leaf values of all trees of the batch for its own (in tree order). A tree's leaf of a row is then read once,
 // side by side by the row's lanes, eight trees' loads in flight. (With all outputs in every lane each of the
 // L lanes fetched the whole leaf again: 500,003 x 200, 50 trees of depth 8 with 8 outputs took 3.89 ms, of
-// which the walk is a tenth; now 0.57.) batch_leaves: at this lane's first output; own: how many it has.
+// which the walk is a tenth; now 0.60.) batch_leaves: at this lane's first output; own: how many it has.
 template <typename S, int kOwn>
 __device__ __forceinline__ void add_leaves_in_order(double (&acc)[kOwn], const int (&at)[S::kLaneTrees], int cnt,
                                                     const double* __restrict__ batch_leaves, int K, int own)

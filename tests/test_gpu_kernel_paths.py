@@ -372,8 +372,10 @@ def test_predict_shares_the_outputs_out_among_the_lanes_of_a_row(f, k):
 @pytest.mark.parametrize("zero_hessians", [False, True])
 def test_levels_that_outgrow_the_histogram_budget_give_the_same_tree(n, f, k, s, depth, zero_hessians):
     """The library's own budget (parents kept, only built siblings cleared) against explicit budgets (every level
-    that outgrows them starts an empty buffer). With rows that have no hessian the tree depends on the budget (the
-    reference leaves bins unscanned), and the library's own is the reference's."""
+    that outgrows them starts an empty buffer), and against observed builds, whose levels are all in memory and built as
+    the reference builds them (the deep case's otherwise stay in the LDS under any budget). With rows that have no
+    hessian the tree depends on the budget (the reference leaves bins unscanned), and the library's own is the
+    reference's."""
     from lbtree import ops
 
     rs = np.random.RandomState(f)
@@ -384,9 +386,11 @@ def test_levels_that_outgrow_the_histogram_budget_give_the_same_tree(n, f, k, s,
         h[::97] = 0.0
     got = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=3, row_leaf=True)
     for budget in (10 ** 9,) if zero_hessians else (10 ** 9, 4 * 10 ** 7):
-        want = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=3, row_leaf=True, hist_cache_bytes=budget)
-        for name in ("leaf_value", "feature", "split_value", "gain", "hessian", "row_leaf"):
-            assert torch.equal(getattr(got, name), getattr(want, name)), (budget, name)
+        for observed in (False, True):
+            want = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=3, row_leaf=True, hist_cache_bytes=budget,
+                                  taps=observed)
+            for name in ("leaf_value", "feature", "split_value", "gain", "hessian", "row_leaf"):
+                assert torch.equal(getattr(got, name), getattr(want, name)), (budget, observed, name)
 
 
 def test_a_build_does_without_the_room_that_it_cannot_have(monkeypatch):
@@ -480,11 +484,10 @@ def test_update_tree_and_the_rows_leaves(n, f, k, depth, dtype):
 @pytest.mark.parametrize("n,f,s,depth,kind", [(9001, 50, 512, 12, "plain"), (20011, 33, 200, 12, "feature_set"),
                                               (9001, 7, 257, 13, "weighted"), (30011, 130, 256, 11, "whole")])
 def test_levels_without_histograms_in_memory_give_the_oracles_tree(n, f, s, depth, kind):
-    """Deep levels whose histograms stay in the LDS against explicit budgets, which keep them in memory, and the
-    oracle's decisions: bins of one and two bytes, features that end inside a 16-byte piece, several record groups,
+    """Deep levels whose histograms stay in the LDS against an observed build, which keeps them in memory, and the
+    oracle's tree: bins of one and two bytes, features that end inside a 16-byte piece, several record groups,
     unusable features, gradients that reach far into 32 bits, columns of few values (long empty runs)."""
     import oracle_lib as orc
-    import gpu_util as gu
     from lbtree import ops
 
     rs = np.random.RandomState(depth)
@@ -502,9 +505,7 @@ def test_levels_without_histograms_in_memory_give_the_oracles_tree(n, f, s, dept
     want = ops.build_tree(Xd, gd, hd, row_leaf=True, taps=True, **kw)  # observed: histograms in memory
     for name in ("leaf_value", "feature", "split_value", "gain", "hessian", "row_leaf"):
         assert torch.equal(getattr(got, name), getattr(want, name)), name
-    if n < 10000 and f < 10:
-        cr = orc.build_tree(X, g, h, **kw)
-        assert np.array_equal(gu.cpu(got.feature), cr.feature)
+    _assert_tree(got, orc.build_tree(X, g, h, **kw))
 
 
 @pytest.mark.parametrize("n,f,s,depth,kind", [(16385, 3, 64, 11, "outliers"), (30001, 7, 256, 11, "outliers"), (60000, 5, 300, 12, "noise"),
