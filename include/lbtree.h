@@ -306,7 +306,8 @@ size_t lbt_predict_workspace_bytes(int32_t n_trees, int64_t total_nodes, int32_t
  *                       NULL. With it, rows are staged in LDS in tiles of 64 to 256 and walked
  *                       through the packed ensemble batch by batch; without it (or when a
  *                       row tile or a tree does not fit the LDS) every node step reads the
- *                       trees' own arrays. More than 8 outputs are walked 8 at a time. The
+ *                       trees' own arrays. A walk sums up to 8, 16 or 32 outputs (two per
+ *                       lane of a row), more take several walks. The
  *                       sums are the same: a row's leaf values are added in tree order either way.
  * Work is enqueued on `stream`; the call does not synchronise.
  */

@@ -737,7 +737,7 @@ __global__ void zero_doubles_kernel(double* a, int64_t n)
 // What bounds it is how X is read. Walking it in place asks for a cache line per step and row, and the lines of the
 // rows in flight do not stay in the L2 (1,000,000 x 50, depth 8: 111 us, the rate of about eight million
 // scattered lines), so rows of up to kStagedBytesPerStep bytes per step of the walk are read whole, side by side,
-// into the LDS first (67 us). row_leaf, if given, receives the node every row stops in.
+// into the LDS first (59 us). row_leaf, if given, receives the node every row stops in.
 constexpr int kUpdateThreads      = 1024;
 constexpr int kUpdateLdsDoubles   = 8192;  // node sums up to 64 KB
 constexpr int kStagedThreads      = 512;  // tiles of wide rows have fewer of them, but all threads stage (256: 75 us a tree where 512 take 67)
