@@ -296,6 +296,13 @@ int lbt_update_positions(void* stream, const void* X, int32_t x_dtype, int64_t n
  * leaf array (total_nodes = sum of the trees' node counts). Returns 0 for invalid arguments. */
 size_t lbt_predict_workspace_bytes(int32_t n_trees, int64_t total_nodes, int32_t n_outputs, int32_t x_dtype);
 
+/* The same for n_rows rows of n_features values, with the room that lets lbt_predict take large inputs by
+ * ranks (the values' places among the ensemble's thresholds, 2 bytes each, a bounded share of the rows at a
+ * time): at least lbt_predict_workspace_bytes(n_trees, the sum of tree_nodes, ...), and that where ranks would not
+ * be used. tree_nodes: host, nodes of every tree. */
+size_t lbt_predict_rows_workspace_bytes(int64_t n_rows, int32_t n_features, int32_t n_trees, const int32_t* tree_nodes,
+                                        int32_t n_outputs, int32_t x_dtype);
+
 /*
  * PredictTask::gpu_variant (src/models/tree/predict.cu:26-91).
  *   leaf/feature/split  HOST arrays of n_trees device pointers, in the order

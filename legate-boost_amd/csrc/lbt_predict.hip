@@ -4,6 +4,7 @@
 // and the per-tree, in-order accumulation into a zeroed f64 output) and
 // src/models/tree/update_tree.cc:36-122.
 #include "lbt_internal.h"
+#include "lbt_ranked.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -46,8 +47,10 @@ __device__ inline int walk(const T* xrow, const TreeRef& tr)
 
 template <typename T, bool kFirst>
 __global__ void __launch_bounds__(kThreads)
-  predict_kernel(const T* X, int64_t n_rows, int F, TreeBatch batch, int n_trees, int K, double* out)
+  predict_kernel(const T* X, int64_t n_rows, int F, TreeBatch batch, int n_trees, int K, const int32_t* wanted,
+                 double* out)
 {
+  if (wanted != nullptr && *wanted == 0) return;
   const int64_t row = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x;
   if (row >= n_rows) return;
   const T* xrow = X + row * F;
@@ -69,7 +72,7 @@ __global__ void __launch_bounds__(kThreads)
 template <typename T>
 int predict_impl(hipStream_t stream, const T* X, int64_t N, int F, int n_trees,
                  const double* const* leaf, const int32_t* const* feature,
-                 const double* const* split, const int32_t* tree_nodes, int K, double* out)
+                 const double* const* split, const int32_t* tree_nodes, int K, const int32_t* wanted, double* out)
 {
   const unsigned grid = static_cast<unsigned>((N + kThreads - 1) / kThreads);
   ProfScope ps(LBT_PROF_PREDICT, stream,
@@ -85,9 +88,9 @@ int predict_impl(hipStream_t stream, const T* X, int64_t N, int F, int n_trees,
       b.t[i].n_nodes = tree_nodes[done + i];
     }
     if (done == 0)
-      predict_kernel<T, true><<<grid, kThreads, 0, stream>>>(X, N, F, b, n, K, out);
+      predict_kernel<T, true><<<grid, kThreads, 0, stream>>>(X, N, F, b, n, K, wanted, out);
     else
-      predict_kernel<T, false><<<grid, kThreads, 0, stream>>>(X, N, F, b, n, K, out);
+      predict_kernel<T, false><<<grid, kThreads, 0, stream>>>(X, N, F, b, n, K, wanted, out);
     done += n;
   } while (done < n_trees);
   LBT_HIP(hipGetLastError());
@@ -165,23 +168,6 @@ struct PackBatch {
 struct BatchTable {
   BatchInfo b[kPackBatches];
 };
-
-// x <= t for a float x holds exactly when x <= (the largest float that is <= t)
-__device__ inline float round_down_to_float(double d)
-{
-  float f = static_cast<float>(d);
-  if (static_cast<double>(f) > d) {  // false for NaN
-    uint32_t b = __float_as_uint(f);
-    if (f > 0.0f)
-      b -= 1;
-    else if (f == 0.0f)
-      b = 0x80000001u;
-    else
-      b += 1;
-    f = __uint_as_float(b);
-  }
-  return f;
-}
 
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -345,8 +331,10 @@ __global__ void __launch_bounds__(kTileThreads)
   predict_tile_kernel(const T* __restrict__ X, int64_t n_rows, int F, int pitch, int n_batches,
                       const BatchInfo* __restrict__ batches, const PackedTree* __restrict__ desc,
                       const PackedNode<T>* __restrict__ nodes, const double* __restrict__ leaves, int K, int k0,
-                      int value_off, double* __restrict__ out)
+                      int value_off, const int32_t* __restrict__ wanted, double* __restrict__ out)
 {
+  // wanted: null, or a device word that is 0 when the rows have been predicted by ranks
+  if (wanted != nullptr && *wanted == 0) return;
   // value_off: where the LDS has room for a batch's leaf values (one output, 16 lanes per row), or 0. Handing a row's sum
   // on through 16 lanes is a chain of 16 cross-lane moves per batch; with few rows, when nothing hides it, the
   // values go through the LDS to the first wave instead, a row per lane.
@@ -653,7 +641,8 @@ int pack_tiled(hipStream_t stream, int F, int n_trees, const double* const* leaf
 
 // The tile kernel over a packed ensemble.
 template <typename T>
-int run_tiled(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble& ens, double* out)
+int run_tiled(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble& ens, double* out,
+              const int32_t* wanted = nullptr)
 {
   const int F = ens.n_features, K = ens.n_outputs, n_batches = ens.n_batches;
   // The lanes the ensemble was laid out for suit many rows. Batches of so many trees fit the kernels for more lanes
@@ -681,7 +670,7 @@ int run_tiled(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemb
     LBT_TRY(allow_dynamic_lds(kernel, kTileLds, flags));
     for (int k0 = 0; k0 < K; k0 += chunk)
       kernel<<<tiles, kTileThreads, lds, stream>>>(X, N, F, pitch, n_batches, lay.batches, lay.desc, lay.nodes, lay.leaves,
-                                                   K, k0, value_off, out);
+                                                   K, k0, value_off, wanted, out);
     return LBT_OK;
   };
   static std::atomic<bool> attr[2][3][3][kMaxDevices] = {};
@@ -711,15 +700,38 @@ int run_tiled(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemb
 template <typename T>
 int predict_tiled(hipStream_t stream, const T* X, int64_t N, int F, int n_trees, const double* const* leaf,
                   const int32_t* const* feature, const double* const* split, const int32_t* tree_nodes, int K,
-                  double* out, void* workspace, size_t workspace_bytes, bool* done)
+                  const int32_t* wanted, double* out, void* workspace, size_t workspace_bytes, bool* done)
 {
   *done = false;
   lbt_packed_ensemble ens;
   LBT_TRY(pack_tiled<T>(stream, F, n_trees, leaf, feature, split, tree_nodes, K, workspace, workspace_bytes, &ens));
   if (ens.data == nullptr) return LBT_OK;
-  LBT_TRY(run_tiled<T>(stream, X, N, ens, out));
+  LBT_TRY(run_tiled<T>(stream, X, N, ens, out, wanted));
   *done = true;
   return LBT_OK;
+}
+
+// By ranks where that is the faster way and the workspace has the room, else tiled, else per node.
+template <typename T>
+int predict_any(hipStream_t stream, const T* X, int64_t N, int F, int n_trees, const double* const* leaf,
+                const int32_t* const* feature, const double* const* split, const int32_t* tree_nodes, int K, double* out,
+                void* workspace, size_t workspace_bytes)
+{
+  int64_t total = 0;
+  for (int i = 0; i < n_trees; i++) total += tree_nodes[i];
+  const size_t packed = (packed_bytes(n_trees, total, K, sizeof(PackedNode<T>)) + 255) & ~size_t(255);
+  const int32_t* wanted = nullptr;
+  bool done = false;
+  if (workspace != nullptr && workspace_bytes > packed) {
+    LBT_TRY(predict_ranked<T>(stream, X, N, F, n_trees, leaf, feature, split, tree_nodes, K, out,
+                              static_cast<char*>(workspace) + packed, workspace_bytes - packed, &done, &wanted));
+    // wanted: only the device knows whether the ranks sufficed; what follows then runs or ends at once
+    if (done && wanted == nullptr) return LBT_OK;
+  }
+  LBT_TRY(predict_tiled<T>(stream, X, N, F, n_trees, leaf, feature, split, tree_nodes, K, wanted, out, workspace,
+                           workspace_bytes, &done));
+  if (done) return LBT_OK;
+  return predict_impl<T>(stream, X, N, F, n_trees, leaf, feature, split, tree_nodes, K, wanted, out);
 }
 
 // ---- update
@@ -984,19 +996,10 @@ int lbt_predict(void* stream, const void* X, int32_t x_dtype, int64_t n_rows, in
       out, n_rows * n_outputs);
     return LBT_OK;
   }
-  bool done = false;
-  if (x_dtype == LBT_F32) {
-    LBT_TRY(lbt::predict_tiled<float>(s, static_cast<const float*>(X), n_rows, n_features, n_trees, leaf, feature,
-                                      split, tree_nodes, n_outputs, out, workspace, workspace_bytes, &done));
-    if (done) return LBT_OK;
-    return lbt::predict_impl<float>(s, static_cast<const float*>(X), n_rows, n_features, n_trees, leaf,
-                                    feature, split, tree_nodes, n_outputs, out);
-  }
-  LBT_TRY(lbt::predict_tiled<double>(s, static_cast<const double*>(X), n_rows, n_features, n_trees, leaf, feature,
-                                     split, tree_nodes, n_outputs, out, workspace, workspace_bytes, &done));
-  if (done) return LBT_OK;
-  return lbt::predict_impl<double>(s, static_cast<const double*>(X), n_rows, n_features, n_trees, leaf,
-                                   feature, split, tree_nodes, n_outputs, out);
+  return x_dtype == LBT_F32 ? lbt::predict_any<float>(s, static_cast<const float*>(X), n_rows, n_features, n_trees, leaf,
+                                                      feature, split, tree_nodes, n_outputs, out, workspace, workspace_bytes)
+                            : lbt::predict_any<double>(s, static_cast<const double*>(X), n_rows, n_features, n_trees, leaf,
+                                                       feature, split, tree_nodes, n_outputs, out, workspace, workspace_bytes);
 }
 
 int lbt_pack_ensemble(void* stream, int32_t x_dtype, int32_t n_features, int32_t n_trees,
@@ -1058,6 +1061,21 @@ size_t lbt_predict_workspace_bytes(int32_t n_trees, int64_t total_nodes, int32_t
   if (n_trees < 0 || total_nodes < 0 || n_outputs < 1 || (x_dtype != LBT_F32 && x_dtype != LBT_F64)) return 0;
   return lbt::packed_bytes(n_trees, total_nodes, n_outputs,
                            x_dtype == LBT_F32 ? sizeof(lbt::PackedNode<float>) : sizeof(lbt::PackedNode<double>));
+}
+
+size_t lbt_predict_rows_workspace_bytes(int64_t n_rows, int32_t n_features, int32_t n_trees, const int32_t* tree_nodes,
+                                        int32_t n_outputs, int32_t x_dtype)
+{
+  if (n_rows < 0 || n_features < 1 || n_trees < 0 || (n_trees > 0 && tree_nodes == nullptr)) return 0;
+  int64_t total = 0;
+  for (int i = 0; i < n_trees; i++) {
+    if (tree_nodes[i] < 1) return 0;
+    total += tree_nodes[i];
+  }
+  const size_t packed = lbt_predict_workspace_bytes(n_trees, total, n_outputs, x_dtype);
+  if (packed == 0) return 0;
+  const size_t ranked = lbt::ranked_workspace_bytes(n_rows, n_features, n_trees, tree_nodes, n_outputs, x_dtype);
+  return ranked == 0 ? packed : ((packed + 255) & ~size_t(255)) + ranked;
 }
 
 size_t lbt_update_tree_workspace_bytes(int64_t n_rows, int32_t n_outputs, int32_t n_nodes)

@@ -246,11 +246,17 @@ def predict(X, trees, n_outputs, tiled=True):
             raise _lib.LbtError("tree %d has inconsistent shapes" % i)
         keep.append((lv, ft, sp))
         leaf_p[i], feat_p[i], split_p[i], nodes[i] = lv.data_ptr(), ft.data_ptr(), sp.data_ptr(), ft.shape[0]
-    total_nodes = sum(int(nodes[i]) for i in range(nt))
     ws = None
     if tiled:
-        ws = torch.empty(int(_lib.lib.lbt_predict_workspace_bytes(nt, total_nodes, n_outputs, _DT[X.dtype])), dtype=torch.uint8,
-                         device=X.device)
+        nbytes = int(_lib.lib.lbt_predict_rows_workspace_bytes(n, f, nt, nodes, n_outputs, _DT[X.dtype]))
+        try:
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=X.device)
+        except torch.OutOfMemoryError:
+            # the room for the rows' ranks is not needed, only faster
+            least = int(_lib.lib.lbt_predict_workspace_bytes(nt, sum(nodes[:nt]), n_outputs, _DT[X.dtype]))
+            if least >= nbytes:
+                raise
+            ws = torch.empty(least, dtype=torch.uint8, device=X.device)
     rc = _lib.lib.lbt_predict(_stream(), X.data_ptr(), _DT[X.dtype], n, f, nt, leaf_p, feat_p, split_p, nodes,
                               n_outputs, out.data_ptr(), ws.data_ptr() if ws is not None else None,
                               ws.numel() if ws is not None else 0)
