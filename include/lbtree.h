@@ -413,6 +413,26 @@ int lbt_weighted_gradient(void* stream, int32_t objective, const double* pred, c
                           int32_t n_outputs, double* g, double* h);
 
 /*
+ * LBBase.update (legateboost/legateboost.py:306-386) over n_trees trees in one call: for every tree in order
+ *   (g, h) = lbt_weighted_gradient(objective, pred, y, sample_weight, learning_rate)
+ *   leaf_out[t], hessian_out[t] = lbt_update_tree(X, g, h, feature[t], split[t], l1[t], l2[t])
+ *   pred += the leaf value of the node every row stops in
+ * with the sums of lbt_update_tree (double, in no fixed order). X is read once for many trees and no gradient is stored.
+ *   feature, split, tree_nodes, l1, l2, leaf_out, hessian_out  host arrays of n_trees entries (pointers to device)
+ *   pred       device double [n_rows][n_outputs]: the predictions to start from; updated
+ *   y, sample_weight, objective  as for lbt_weighted_gradient
+ *   workspace  at least lbt_update_trees_workspace_bytes(...), which is 0 for what this call does not take: trees that are
+ *              not of whole levels (2^d - 1 nodes), more than 4096 (node, output) sums of a tree, more than 16383 features
+ */
+size_t lbt_update_trees_workspace_bytes(int64_t n_rows, int32_t n_features, int32_t x_dtype, int32_t n_outputs, int32_t n_trees,
+                                        const int32_t* tree_nodes);
+int lbt_update_trees(void* stream, const void* X, int32_t x_dtype, int64_t n_rows, int32_t n_features, int32_t objective,
+                     const double* y, const double* sample_weight, double learning_rate, int32_t n_outputs, int32_t n_trees,
+                     const int32_t* const* feature, const double* const* split, const int32_t* tree_nodes, const double* l1,
+                     const double* l2, double* pred, double* const* leaf_out, double* const* hessian_out, void* workspace,
+                     size_t workspace_bytes);
+
+/*
  * lbt_weighted_gradient that also leaves the first level of the quantiser's two absolute sums
  * (legateboost.py:260-275 followed by build_tree.cu:77-83): the pass that produces g and h adds
  * up |g| and |h| per chunk of 4096 consecutive entries of the flat [n_rows * n_outputs] arrays,

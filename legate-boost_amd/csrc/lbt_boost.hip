@@ -10,14 +10,6 @@
 namespace lbt {
 
 constexpr int kBoostThreads = 256;
-constexpr double kMinHessian = 1e-8;  // legateboost.py:211
-
-__device__ inline void weigh(double g0, double h0, double w, double lr, double* g, double* h)
-{
-  *g = (g0 * w) * lr;
-  *h = fmax(h0 * w, kMinHessian);
-}
-
 // One element per thread: squared error (any number of outputs) and log loss with one output.
 template <bool kLogistic>
 __global__ void __launch_bounds__(kBoostThreads)

@@ -272,6 +272,14 @@ __host__ __device__ inline double calculate_leaf_value(double G, double H, doubl
   return -z / (H + l2);
 }
 
+// legateboost.py:209-211: weight, learning rate, least hessian
+constexpr double kMinHessian = 1e-8;
+__device__ inline void weigh(double g0, double h0, double w, double lr, double* g, double* h)
+{
+  *g = (g0 * w) * lr;
+  *h = fmax(h0 * w, kMinHessian);
+}
+
 // build_tree.h:64-74
 __host__ __device__ inline int parent_of(int i) { return (i - 1) / 2; }
 __host__ __device__ inline int left_child(int i) { return 2 * i + 1; }

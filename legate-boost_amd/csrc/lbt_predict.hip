@@ -4,7 +4,7 @@
 // and the per-tree, in-order accumulation into a zeroed f64 output) and
 // src/models/tree/update_tree.cc:36-122.
 #include "lbt_internal.h"
-#include "lbt_ranked.h"
+#include "lbt_trees.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -112,20 +112,6 @@ int predict_impl(hipStream_t stream, const T* X, int64_t N, int F, int n_trees,
 // fetched (from a packed copy) while the next one is walked. They are added in tree order, so a row's sum is formed
 // exactly as the per-tree launches of the reference form it.
 
-template <typename T>
-struct PackedNode;
-template <>
-struct alignas(8) PackedNode<float> {
-  float thr;
-  uint32_t feat_right;  // byte offset of the feature in a row (4 * feature) in the low half, right child in the high half
-};
-template <>
-struct alignas(16) PackedNode<double> {
-  double thr;
-  int32_t feat;
-  int32_t right;
-};
-
 struct alignas(16) PackedTree {
   const double* leaf;
   int32_t rel_off;  // first node, counted from the first node of the tree's batch
@@ -158,7 +144,6 @@ constexpr size_t kTileLds   = 160 * 1024 - 2048;  // dynamic LDS of the tile ker
 constexpr int kCopyWords    = 6;  // 16-byte words a thread moves per batch: 6 * 1024 * 16 B >= any batch
 constexpr int kSmallRunGroups = 256;  // workgroups up to which more lanes share a row: one per CU
 constexpr size_t kSmallEnsembleLds = 78 * 1024;  // row tile + nodes of a small ensemble: two workgroups per CU
-constexpr int kMaxPackedNodes = 65535;  // the right child of a float node has 16 bits
 
 struct PackBatch {
   TreeRef t[kPackTrees];
@@ -187,21 +172,7 @@ __global__ void __launch_bounds__(256)
   // leaf values move along, indexed like the nodes
   for (int k = 0; k < K; k++)
     leaves[(b.node_off[blockIdx.y] + i) * K + k] = tr.leaf[static_cast<int64_t>(i) * K + k];
-  int ft = tr.feature[i];
-  // a node whose children would lie past the arrays, or whose feature does not exist, ends the walk
-  const bool is_leaf = ft < 0 || ft >= F || 2 * static_cast<int64_t>(i) + 2 >= tr.n_nodes;
-  PackedNode<T> nd;
-  // a step goes to right - (x <= thr): the comparison is false against NaN, so a leaf stays
-  const int right = is_leaf ? i : 2 * i + 2;
-  if constexpr (sizeof(T) == 4) {
-    nd.thr        = is_leaf ? __uint_as_float(0x7fc00000u) : round_down_to_float(tr.split[i]);
-    nd.feat_right = (is_leaf ? 0u : static_cast<uint32_t>(ft) * 4u) | (static_cast<uint32_t>(right) << 16);
-  } else {
-    nd.thr   = is_leaf ? __longlong_as_double(0x7ff8000000000000LL) : tr.split[i];
-    nd.feat  = is_leaf ? 0 : ft;
-    nd.right = right;
-  }
-  nodes[b.node_off[blockIdx.y] + i] = nd;
+  nodes[b.node_off[blockIdx.y] + i] = pack_node<T>(i, tr.feature[i], tr.split[i], F, tr.n_nodes);
 }
 
 __global__ void write_batches_kernel(BatchTable t, int first, int n, BatchInfo* out)
@@ -535,7 +506,7 @@ int pack_tiled(hipStream_t stream, int F, int n_trees, const double* const* leaf
                lbt_packed_ensemble* ens)
 {
   *ens = lbt_packed_ensemble{};
-  if (buffer == nullptr || F > 16383) return LBT_OK;  // a float node holds 4 * feature in 16 bits
+  if (buffer == nullptr || F > kMaxPackedFeatures) return LBT_OK;
   int64_t total_nodes = 0;
   int max_nodes       = 0;
   for (int i = 0; i < n_trees; i++) {
@@ -882,33 +853,11 @@ __global__ void __launch_bounds__(1024)
     }
     __syncthreads();
   }
-  int depth = 0;
-  while (((int64_t(1) << (depth + 1)) - 1) < n_nodes) depth++;
-  for (int d = depth - 1; d >= 0; d--) {
-    const int64_t first = (int64_t(1) << d) - 1, count = int64_t(1) << d;
-    for (int64_t i = threadIdx.x; i < count * K; i += blockDim.x) {
-      const int64_t node = first + i / K;
-      const int k        = static_cast<int>(i % K);
-      if (node < n_nodes && feature[node] != -1) {
-        double gs = 0.0, hs = 0.0;
-        if (2 * node + 1 < n_nodes) {
-          gs += g[(2 * node + 1) * K + k];
-          hs += h[(2 * node + 1) * K + k];
-        }
-        if (2 * node + 2 < n_nodes) {
-          gs += g[(2 * node + 2) * K + k];
-          hs += h[(2 * node + 2) * K + k];
-        }
-        g[node * K + k] += gs;
-        h[node * K + k] += hs;
-      }
-    }
-    __syncthreads();
-  }
+  sum_inner_nodes(feature, n_nodes, K, g, h);
   if constexpr (kUseLds) {
     for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
       const double hv = h[i];
-      leaf_out[i]     = hv > 0.0 ? calculate_leaf_value(g[i], hv, l1, l2) : 0.0;
+      leaf_out[i]     = updated_leaf(g[i], hv, l1, l2);
       hessian_out[i]  = hv;
     }
   }
@@ -921,7 +870,7 @@ __global__ void update_leaves_kernel(const double* G, const double* H, int64_t n
   int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
   if (i < n) {
     double hv      = H[i];
-    leaf_out[i]    = hv > 0.0 ? calculate_leaf_value(G[i], hv, l1, l2) : 0.0;
+    leaf_out[i]    = updated_leaf(G[i], hv, l1, l2);
     hessian_out[i] = hv;
   }
 }

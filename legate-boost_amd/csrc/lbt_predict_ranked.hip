@@ -18,7 +18,7 @@
 #include <cmath>
 #include <type_traits>
 
-#include "lbt_ranked.h"
+#include "lbt_trees.h"
 
 namespace lbt {
 namespace {

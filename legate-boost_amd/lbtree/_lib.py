@@ -137,6 +137,12 @@ def _load():
     lib.lbt_update_tree_rows.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p,
                                     C.c_int32, C.c_void_p, C.c_void_p, C.c_int32, C.c_double, C.c_double, C.c_void_p,
                                     C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
+    lib.lbt_update_trees_workspace_bytes.restype = C.c_size_t
+    lib.lbt_update_trees_workspace_bytes.argtypes = [C.c_int64, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_void_p]
+    lib.lbt_update_trees.restype = C.c_int
+    lib.lbt_update_trees.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_int64, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p,
+                                     C.c_double, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
+                                     C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
     lib.lbt_pack_ensemble.restype = C.c_int
     lib.lbt_pack_ensemble.argtypes = [C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p,
                                       C.c_void_p, C.c_int32, C.c_void_p, C.c_size_t, C.POINTER(PackedEnsemble)]
@@ -205,7 +211,8 @@ lib = _load()
 EXPORTS = [
     "lbt_last_error", "lbt_version", "lbt_release_thread_resources", "lbt_build_tree_workspace_bytes", "lbt_build_tree", "lbt_build_tree_async", "lbt_predict",
     "lbt_predict_workspace_bytes", "lbt_predict_rows_workspace_bytes", "lbt_pack_ensemble", "lbt_predict_packed",
-    "lbt_update_tree_workspace_bytes", "lbt_update_tree", "lbt_update_tree_rows",
+    "lbt_update_tree_workspace_bytes", "lbt_update_tree", "lbt_update_tree_rows", "lbt_update_trees_workspace_bytes",
+    "lbt_update_trees",
     "lbt_weighted_gradient", "lbt_weighted_gradient_sums",
     "lbt_abs_sum_chunks", "lbt_add_leaf_values",
     "lbt_gather_rows", "lbt_select_split_samples_workspace_bytes", "lbt_select_split_samples",

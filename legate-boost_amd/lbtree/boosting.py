@@ -158,10 +158,18 @@ class LBBase:
         X, y = self._prepare(X, y)
         w = torch.ones(y.shape[0], dtype=torch.float64, device=y.device) if sample_weight is None \
             else ops.as_device(sample_weight, torch.float64)
-        for m in self.models_:
-            m.clear()
+        if self.models_ and all(type(m).clear is Tree.clear for m in self.models_):
+            torch._foreach_zero_([a for m in self.models_ for a in (m.leaf_value, m.hessian)])
+        else:
+            for m in self.models_:
+                m.clear()
         self.model_init_ = self._objective_instance.initialise_prediction(y, w, self.init == "average")
         pred = self.model_init_.reshape(1, -1).repeat(X.shape[0], 1).contiguous()
+        fused = getattr(self._objective_instance, "fused", None)
+        if (fused is not None and self.subsample == 1.0 and X.shape[0] > 0
+                and type(self)._get_weighted_gradient is LBBase._get_weighted_gradient
+                and Tree.update_rounds(self.models_, X, y, w, fused, self.learning_rate, pred)):
+            return self
         for m in self.models_:
             g, h = self._get_weighted_gradient(y, pred, w, self.learning_rate)
             if hasattr(m, "update_and_predict"):

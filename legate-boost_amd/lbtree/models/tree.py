@@ -125,6 +125,24 @@ class Tree(BaseModel):
         ops.add_leaf_values(pred, self.leaf_value, rows)
         return self
 
+    @staticmethod
+    def update_rounds(models: Sequence[BaseModel], X, y, sample_weight, objective, learning_rate, pred) -> bool:
+        """The update of `models` in order, each at the predictions of those before it (legateboost/legateboost.py:306-386),
+        for a plain objective ("squared_error" or "log_loss"); pred is updated. False, with nothing done, where a model
+        brings its own update or predict or the trees are not of the form that is updated together."""
+        own = ("update", "update_and_predict", "predict", "batch_predict", "update_rounds")
+        if not models or any(not isinstance(m, Tree) or any(getattr(type(m), a) is not getattr(Tree, a) or a in vars(m) for a in own)
+                             for m in models):
+            return False
+        out = ops.update_trees(
+            X, y, sample_weight, objective, learning_rate, pred,
+            [(m.feature, m.split_value, m.l1_regularization, m.l2_regularization) for m in models])
+        if out is None:
+            return False
+        for m, (leaf_value, hessian) in zip(models, out):
+            m.leaf_value, m.hessian = leaf_value, hessian
+        return True
+
     def predict(self, X):
         return Tree.batch_predict([self], X)
 

@@ -330,6 +330,50 @@ def weighted_gradient(objective, y, pred, sample_weight=None, learning_rate=1.0,
     return g, h
 
 
+def update_trees(X, y, sample_weight, objective, learning_rate, pred, trees):
+    """The loop of LBBase.update (legateboost/legateboost.py:306-386) over `trees`, a list of (feature, split_value,
+    l1_regularization, l2_regularization): per tree weighted_gradient at pred, update_tree and the prediction update.
+    pred (CUDA float64 [n_rows, n_outputs]) is updated. Returns a list of (leaf_value, hessian), or None, with nothing
+    done, for trees the call does not take."""
+    X = _check_x(X)
+    y = as_device(y, torch.float64)
+    if not (pred.is_cuda and pred.dtype == torch.float64 and pred.is_contiguous() and pred.dim() == 2):
+        raise _lib.LbtError("pred must be a contiguous CUDA float64 [n_rows, n_outputs] tensor")
+    n, f = X.shape
+    k, nt = pred.shape[1], len(trees)
+    if pred.shape[0] != n:
+        raise _lib.LbtError("pred must have a row per row of X")
+    if y.numel() != (n if objective == "log_loss" and k > 1 else n * k):
+        raise _lib.LbtError("y has %d elements, expected %d" % (y.numel(), n if objective == "log_loss" and k > 1 else n * k))
+    w = None
+    if sample_weight is not None:
+        w = as_device(sample_weight, torch.float64)
+        if w.numel() != n:
+            raise _lib.LbtError("sample_weight must have one entry per row")
+    keep = [(as_device(t[0], torch.int32), as_device(t[1], torch.float64)) for t in trees]
+    if any(ft.dim() != 1 or sp.shape != ft.shape for ft, sp in keep):
+        return None
+    nodes = (C.c_int32 * nt)(*[ft.shape[0] for ft, _ in keep])
+    nbytes = int(_lib.lib.lbt_update_trees_workspace_bytes(n, f, _DT[X.dtype], k, nt, nodes))
+    if nbytes == 0:
+        return None
+    try:
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=X.device)
+    except torch.OutOfMemoryError:
+        return None
+    out = [(torch.empty((m, k), dtype=torch.float64, device=X.device), torch.empty((m, k), dtype=torch.float64, device=X.device))
+           for m in nodes]
+    ptrs = C.c_void_p * nt
+    rc = _lib.lib.lbt_update_trees(
+        _stream(), X.data_ptr(), _DT[X.dtype], n, f, _OBJECTIVES[objective], y.data_ptr(),
+        w.data_ptr() if w is not None else None, float(learning_rate), k, nt, ptrs(*[ft.data_ptr() for ft, _ in keep]),
+        ptrs(*[sp.data_ptr() for _, sp in keep]), nodes, (C.c_double * nt)(*[t[2] for t in trees]),
+        (C.c_double * nt)(*[t[3] for t in trees]), pred.data_ptr(), ptrs(*[o[0].data_ptr() for o in out]),
+        ptrs(*[o[1].data_ptr() for o in out]), ws.data_ptr(), nbytes)
+    _lib.check(rc)
+    return out
+
+
 def add_leaf_values(pred, leaf_value, row_leaf):
     """pred += leaf_value[row_leaf], in place: the caller's `train_pred += tree.predict(X)`
     (legateboost/legateboost.py:268) from the rows' leaves recorded by build_tree(row_leaf=True)."""
