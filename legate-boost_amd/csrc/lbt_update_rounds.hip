@@ -5,7 +5,7 @@
 // trees (tree_leaves_kernel) and a round is one pass over the targets and predictions (round_kernel), which adds the leaf
 // values of the tree before, forms gradient and hessian and sums them per node. Inner nodes and outputs of all
 // trees follow at the end. One tree after the other (gradient, accumulation over X, finish, prediction update) took
-// 82 us a tree on 1,000,000 x 50 with depth 8, of which 59 were for X; now see round_kernel.
+// 82 us a tree on 1,000,000 x 50 with depth 8, of which 59 were for X; now 61 for ten trees and 8 a round.
 #include <algorithm>
 #include <type_traits>
 
@@ -26,6 +26,7 @@ constexpr size_t kOnePerCu   = 158 * 1024;
 constexpr int kMostSums      = 4096;        // nodes * outputs of a tree: two sums and the leaf values of one before in the LDS
 constexpr int kPackTrees     = 32;          // descriptors passed by value per launch
 constexpr size_t kLeafBytes  = 128u << 20;  // recorded leaves of one pass
+constexpr int kCopies        = 8;           // of a tree's sums: a workgroup adds to one of them
 constexpr int kStagedPerStep = 80;          // a scattered cache line costs as much as about 100 bytes in sequence
 
 struct PackRefs {
@@ -152,19 +153,28 @@ struct RoundArgs {
   double* pred;
   const uint16_t* leaf;       // node of every row in this round's tree
   const uint16_t* prev_leaf;  // and in the one before
-  const double* prev_G;       // [prev_nodes][K] its sums
-  const double* prev_H;
+  const double* prev_sums;    // its sums, as below
   double prev_l1, prev_l2;
-  double* G;
-  double* H;
+  double* sums;               // [kCopies][2][n_nodes][K]
 };
+
+// sums of gradients (which 0) or hessians (1) at entry i of n
+__device__ __forceinline__ double sum_of_copies(const double* sums, int n, int which, int i)
+{
+  double v = 0.0;
+#pragma unroll
+  for (int c = 0; c < kCopies; c++) v += sums[static_cast<int64_t>(2 * c + which) * n + i];
+  return v;
+}
 
 enum class Gradient { kSquared, kLogistic, kSoftmax };
 
 // One round (see above): the leaf values of the tree before are formed by every workgroup from its sums, so nothing runs
 // between two rounds. The gradient is lbt_weighted_gradient's, operation by operation. kCols: the outputs where
 // they are known (1, or a softmax row in registers), 0 any number.
-// What bounds it: predictions, targets and leaves in one sweep (28 bytes a row and output), and the LDS adds.
+// What bounds it: the workgroups' adds to the sums in memory (one address takes them in turn: with one copy of the sums 256
+// workgroups took 13.2 us and 1024 twice that; with 8 copies 8.2), then predictions, targets and leaves in one sweep (28 bytes
+// a row and output: 6 us).
 template <Gradient kKind, int kCols>
 __global__ void __launch_bounds__(kRoundThreads) round_kernel(RoundArgs a)
 {
@@ -172,7 +182,8 @@ __global__ void __launch_bounds__(kRoundThreads) round_kernel(RoundArgs a)
   const int K = kCols > 0 ? kCols : a.K, n_sums = a.n_nodes * K, n_prev = a.prev_nodes * K, tid = threadIdx.x;
   double* s_prev = reinterpret_cast<double*>(smem_raw);  // [prev_nodes][K]
   double* s_sum  = s_prev + n_prev;                      // [2][K][n_nodes]: nodes side by side in the banks
-  for (int i = tid; i < n_prev; i += kRoundThreads) s_prev[i] = updated_leaf(a.prev_G[i], a.prev_H[i], a.prev_l1, a.prev_l2);
+  for (int i = tid; i < n_prev; i += kRoundThreads)
+    s_prev[i] = updated_leaf(sum_of_copies(a.prev_sums, n_prev, 0, i), sum_of_copies(a.prev_sums, n_prev, 1, i), a.prev_l1, a.prev_l2);
   for (int i = tid; i < 2 * n_sums; i += kRoundThreads) s_sum[i] = 0.0;
   __syncthreads();
   auto add = [&](int node, int k, double g, double h) {
@@ -262,11 +273,12 @@ __global__ void __launch_bounds__(kRoundThreads) round_kernel(RoundArgs a)
     }
   }
   __syncthreads();
+  double* to = a.sums + static_cast<int64_t>(2) * n_sums * (blockIdx.x % kCopies);
   for (int i = tid; i < n_sums; i += kRoundThreads) {
     const int node = i / K, at = (i - node * K) * a.n_nodes + node;
     const double gv = s_sum[at], hv = s_sum[n_sums + at];
-    if (gv != 0.0) unsafeAtomicAdd(&a.G[i], gv);
-    if (hv != 0.0) unsafeAtomicAdd(&a.H[i], hv);
+    if (gv != 0.0) unsafeAtomicAdd(&to[i], gv);
+    if (hv != 0.0) unsafeAtomicAdd(&to[n_sums + i], hv);
   }
 }
 
@@ -283,7 +295,7 @@ __global__ void __launch_bounds__(256)
 
 struct FinishRefs {
   const int32_t* feature[kPackTrees];
-  const double* G[kPackTrees];  // [n_nodes][K], H behind it
+  const double* sums[kPackTrees];  // [kCopies][2][n_nodes][K]
   double* leaf[kPackTrees];
   double* hessian[kPackTrees];
   double l1[kPackTrees], l2[kPackTrees];
@@ -298,8 +310,8 @@ __global__ void __launch_bounds__(1024) finish_trees_kernel(FinishRefs refs, int
   double* g   = reinterpret_cast<double*>(smem_raw);
   double* h   = g + n;
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    g[i] = refs.G[t][i];
-    h[i] = refs.G[t][n + i];
+    g[i] = sum_of_copies(refs.sums[t], n, 0, i);
+    h[i] = sum_of_copies(refs.sums[t], n, 1, i);
   }
   __syncthreads();
   sum_inner_nodes(refs.feature[t], refs.n_nodes[t], K, g, h);
@@ -333,7 +345,7 @@ Plan make_plan(int64_t N, int F, size_t value_size, int K, int n_trees, const in
     if (static_cast<int64_t>(tree_nodes[t]) * K > kMostSums) return p;
     if (static_cast<size_t>(tree_nodes[t] + 1) * 2 * value_size > kNodeLds) return p;
     p.nodes += tree_nodes[t] + 1;  // an even number: trees begin on 16 bytes
-    p.sums += static_cast<int64_t>(2) * tree_nodes[t] * K;
+    p.sums += static_cast<int64_t>(2 * kCopies) * tree_nodes[t] * K;
   }
   p.pass_trees = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({kPassTrees, n_trees, static_cast<int64_t>(kLeafBytes / 2) / N})));
   const int64_t held = std::min<int64_t>(n_trees, 2 * p.pass_trees);  // the round before may be the last of the pass before
@@ -358,7 +370,7 @@ int update_rounds(hipStream_t stream, const T* X, int64_t N, int F, int objectiv
   std::vector<int64_t> node_off(n_trees + 1, 0), sum_off(n_trees + 1, 0);
   for (int t = 0; t < n_trees; t++) {
     node_off[t + 1] = node_off[t] + tree_nodes[t] + 1;
-    sum_off[t + 1]  = sum_off[t] + static_cast<int64_t>(2) * tree_nodes[t] * K;
+    sum_off[t + 1]  = sum_off[t] + static_cast<int64_t>(2 * kCopies) * tree_nodes[t] * K;
   }
   for (int first = 0; first < n_trees; first += kPackTrees) {
     PackRefs refs{};
@@ -451,13 +463,11 @@ int update_rounds(hipStream_t stream, const T* X, int64_t N, int F, int objectiv
       ra.weight  = weight;
       ra.pred    = pred;
       ra.leaf    = row_leaf + static_cast<int64_t>(t % slots) * N;
-      ra.G       = sums + sum_off[t];
-      ra.H       = ra.G + static_cast<int64_t>(tree_nodes[t]) * K;
+      ra.sums    = sums + sum_off[t];
       if (t > 0) {
         ra.prev_nodes = tree_nodes[t - 1];
         ra.prev_leaf  = row_leaf + static_cast<int64_t>((t - 1) % slots) * N;
-        ra.prev_G     = sums + sum_off[t - 1];
-        ra.prev_H     = ra.prev_G + static_cast<int64_t>(tree_nodes[t - 1]) * K;
+        ra.prev_sums  = sums + sum_off[t - 1];
         ra.prev_l1    = l1[t - 1];
         ra.prev_l2    = l2[t - 1];
       }
@@ -471,7 +481,7 @@ int update_rounds(hipStream_t stream, const T* X, int64_t N, int F, int objectiv
     int widest  = 1;
     for (int i = 0; i < n; i++) {
       refs.feature[i] = feature[first + i];
-      refs.G[i]       = sums + sum_off[first + i];
+      refs.sums[i]    = sums + sum_off[first + i];
       refs.leaf[i]    = leaf_out[first + i];
       refs.hessian[i] = hessian_out[first + i];
       refs.l1[i]      = l1[first + i];
