@@ -208,6 +208,14 @@ def _load():
 
 lib = _load()
 
+try:
+    import torch  # noqa: E402,F401  (loads the libraries that _host is linked against)
+
+    from . import _host  # noqa: E402,F401
+except ImportError as e:
+    raise ImportError("lbtree/_host.so is missing or does not load (%s): build it with `make -C legate-boost_amd/csrc` "
+                      "or __graft_entry__.build()" % e)
+
 EXPORTS = [
     "lbt_last_error", "lbt_version", "lbt_release_thread_resources", "lbt_build_tree_workspace_bytes", "lbt_build_tree", "lbt_build_tree_async", "lbt_predict",
     "lbt_predict_workspace_bytes", "lbt_predict_rows_workspace_bytes", "lbt_pack_ensemble", "lbt_predict_packed",

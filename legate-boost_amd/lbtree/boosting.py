@@ -122,11 +122,10 @@ class LBBase:
         return g, h
 
     def _predict(self, X):
-        n = X.shape[0]
-        pred = self.model_init_.reshape(1, -1).repeat(n, 1).contiguous()
+        init = self.model_init_.reshape(1, -1)
         if self.models_:
-            pred = pred + type(self.models_[0]).batch_predict(self.models_, X)
-        return pred
+            return init + type(self.models_[0]).batch_predict(self.models_, X)
+        return init.repeat(X.shape[0], 1).contiguous()
 
     def fit(self, X, y, sample_weight=None):
         X, y = self._prepare(X, y)

@@ -180,6 +180,11 @@ def build_tree(X, g, h, *, max_depth, split_samples, seed, l1_regularization=0.0
 
 
 def _tree_arrays(trees, n_outputs):
+    """Host arrays of an ensemble's (leaf_value, feature, split_value): addresses of the three, nodes of every tree, all nodes,
+    and what keeps the addresses valid."""
+    plain = _lib._host.tree_arrays(trees, n_outputs)
+    if plain is not None:
+        return plain + (int(np.frombuffer(plain[3], np.int32).sum(dtype=np.int64)), trees)
     nt = len(trees)
     leaf_p = (C.c_void_p * max(nt, 1))()
     feat_p = (C.c_void_p * max(nt, 1))()
@@ -194,7 +199,7 @@ def _tree_arrays(trees, n_outputs):
             raise _lib.LbtError("tree %d has inconsistent shapes" % i)
         keep.append((lv, ft, sp))
         leaf_p[i], feat_p[i], split_p[i], nodes[i] = lv.data_ptr(), ft.data_ptr(), sp.data_ptr(), ft.shape[0]
-    return leaf_p, feat_p, split_p, nodes, keep
+    return leaf_p, feat_p, split_p, nodes, sum(int(nodes[i]) for i in range(nt)), keep
 
 
 class PackedEnsemble:
@@ -204,9 +209,8 @@ class PackedEnsemble:
     def __init__(self, trees, n_outputs, n_features, dtype=torch.float32, device=None):
         if dtype not in _DT:
             raise _lib.LbtError("X must be float32 or float64, got %s" % dtype)
-        leaf_p, feat_p, split_p, nodes, keep = _tree_arrays(trees, n_outputs)
+        leaf_p, feat_p, split_p, nodes, total, keep = _tree_arrays(trees, n_outputs)
         nt = len(trees)
-        total = sum(int(nodes[i]) for i in range(nt))
         device = device if device is not None else (keep[0][0].device if keep else "cuda")
         nbytes = int(_lib.lib.lbt_predict_workspace_bytes(nt, total, n_outputs, _DT[dtype]))
         self.buffer = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
@@ -233,19 +237,7 @@ def predict(X, trees, n_outputs, tiled=True):
     n, f = X.shape
     nt = len(trees)
     out = torch.empty((n, n_outputs), dtype=torch.float64, device=X.device)
-    leaf_p = (C.c_void_p * max(nt, 1))()
-    feat_p = (C.c_void_p * max(nt, 1))()
-    split_p = (C.c_void_p * max(nt, 1))()
-    nodes = (C.c_int32 * max(nt, 1))()
-    keep = []
-    for i, (lv, ft, sp) in enumerate(trees):
-        lv = as_device(lv, torch.float64)
-        ft = as_device(ft, torch.int32)
-        sp = as_device(sp, torch.float64)
-        if lv.dim() != 2 or lv.shape[1] != n_outputs or ft.shape[0] != lv.shape[0] or sp.shape[0] != lv.shape[0]:
-            raise _lib.LbtError("tree %d has inconsistent shapes" % i)
-        keep.append((lv, ft, sp))
-        leaf_p[i], feat_p[i], split_p[i], nodes[i] = lv.data_ptr(), ft.data_ptr(), sp.data_ptr(), ft.shape[0]
+    leaf_p, feat_p, split_p, nodes, total, keep = _tree_arrays(trees, n_outputs)
     ws = None
     if tiled:
         nbytes = int(_lib.lib.lbt_predict_rows_workspace_bytes(n, f, nt, nodes, n_outputs, _DT[X.dtype]))
@@ -253,7 +245,7 @@ def predict(X, trees, n_outputs, tiled=True):
             ws = torch.empty(nbytes, dtype=torch.uint8, device=X.device)
         except torch.OutOfMemoryError:
             # the room for the rows' ranks is not needed, only faster
-            least = int(_lib.lib.lbt_predict_workspace_bytes(nt, sum(nodes[:nt]), n_outputs, _DT[X.dtype]))
+            least = int(_lib.lib.lbt_predict_workspace_bytes(nt, total, n_outputs, _DT[X.dtype]))
             if least >= nbytes:
                 raise
             ws = torch.empty(least, dtype=torch.uint8, device=X.device)

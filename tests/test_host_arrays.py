@@ -1,0 +1,44 @@
+"""lbtree._host.tree_arrays, the native look at an ensemble's arrays: what it does not take is left to the Python form."""
+import numpy as np
+import pytest
+import torch
+
+from lbtree import _lib, ops
+
+
+def test_anything_but_plain_device_arrays_is_left_to_the_caller():
+    take = _lib._host.tree_arrays
+    cpu = (torch.zeros(7, 1, dtype=torch.float64), torch.zeros(7, dtype=torch.int32), torch.zeros(7, dtype=torch.float64))
+    assert take([], 1) == (b"", b"", b"", b"")
+    for trees in ([cpu], [(1, 2, 3)], [cpu[:2]], [list(cpu)], [None], iter([cpu]), [(np.zeros((7, 1)),) + cpu[1:]]):
+        assert take(trees, 1) is None
+    assert take([], 0) is None
+    with pytest.raises(TypeError):
+        take([cpu])
+
+
+@pytest.mark.gpu
+def test_plain_arrays_and_those_that_are_not():
+    take = _lib._host.tree_arrays
+    leaf = torch.randn(7, 2, dtype=torch.float64).cuda()
+    feat = torch.tensor([0, 1, 0, -1, -1, -1, -1], dtype=torch.int32).cuda()
+    split = torch.rand(7, dtype=torch.float64).cuda()
+    trees = [(leaf, feat, split), (leaf[:3], feat[:3], split[:3])]
+    got = take(trees, 2)
+    assert [np.frombuffer(b, np.uint64).tolist() for b in got[:3]] == [[t[i].data_ptr() for t in trees] for i in range(3)]
+    assert np.frombuffer(got[3], np.int32).tolist() == [7, 3]
+    wide = torch.randn(7, 4, dtype=torch.float64).cuda()
+    for bad in ((wide[:, :2], feat, split), (leaf.float(), feat, split), (leaf, feat.long(), split), (leaf[:6], feat, split),
+                (leaf, feat, split[:6]), (leaf[:, 0], feat, split), (leaf, feat, torch.rand(14, dtype=torch.float64).cuda()[::2])):
+        assert take([bad], 2) is None
+    assert take(trees, 1) is None
+    # and the caller converts or refuses, as without it
+    X = torch.rand(50, 2).cuda()
+    want = ops.predict(X, trees, 2)
+    strided = torch.stack([split, split], dim=1)[:, 0]
+    mixed = [(leaf.cpu(), feat.long(), strided), tuple(t.cpu().numpy() for t in trees[1])]
+    assert torch.equal(ops.predict(X, mixed, 2), want)
+    assert torch.equal(ops.PackedEnsemble(mixed, 2, 2).predict(X), want)
+    for bad in ((leaf[:6], feat, split), (leaf[:, :1], feat, split)):
+        with pytest.raises(_lib.LbtError):
+            ops.predict(X, [bad], 2)
