@@ -113,8 +113,8 @@ int predict_impl(hipStream_t stream, const T* X, int64_t N, int F, int n_trees,
 // exactly as the per-tree launches of the reference form it.
 
 struct alignas(16) PackedTree {
-  const double* leaf;
-  int32_t rel_off;  // first node, counted from the first node of the tree's batch
+  int64_t node_off;  // first node in the packed array
+  int32_t rel_off;   // and counted from the first node of the tree's batch
   int32_t n_nodes;
 };
 
@@ -163,7 +163,7 @@ __global__ void __launch_bounds__(256)
   const int i      = blockIdx.x * 256 + threadIdx.x;
   if (i == 0) {
     PackedTree d;
-    d.leaf                        = tr.leaf;
+    d.node_off                    = b.node_off[blockIdx.y];
     d.rel_off                     = b.rel_off[blockIdx.y];
     d.n_nodes                     = tr.n_nodes;
     desc[first_tree + blockIdx.y] = d;
@@ -452,6 +452,110 @@ __global__ void __launch_bounds__(kTileThreads)
   }
 }
 
+// ---- few rows
+//
+// With few rows a call is a chain of latencies: the tile kernel above walks 32 trees at a time, each batch four dependent
+// trips to memory and the LDS (256 x 32 with 100 trees of depth 6: 12.3 us). Here a workgroup takes kFewRows rows through
+// as many batches at once as the LDS holds, a (row, tree) per lane; everything that is needed first (rows, the nodes from the
+// start of the array, the lanes' trees) is asked for before the first wait. The values pass through the LDS to the lanes
+// that add a row's in tree order: 7.3 us a launch where the tile kernel takes 12.4 (1000 x 10 f64: 16.7 and 9.9). A workgroup
+// copies the ensemble for 16 rows only: with 6433 x 94 and 117 trees of depth 7 it takes 22.0 us and the tile kernel 15.3,
+// with 4096 x 32 and 100 of depth 6 7.9 and 13.1. An ensemble of at most as many trees as a row has lanes there (up to
+// 16) is one batch there too: 52 x 5, 7 trees 3.8 and 3.9 us.
+constexpr int kFewRows        = 16;
+constexpr int64_t kFewMostRows = 4096;  // one workgroup per CU
+constexpr int kFewLanes       = kTileThreads / kFewRows;  // of a row
+constexpr int kFewWords       = 8;    // 16-byte words of nodes that a thread moves per turn
+constexpr int kFewTogether    = 2;    // trees a lane walks at once
+constexpr int kFewGroupTrees  = kFewTogether * kFewLanes;
+
+template <typename T>
+__global__ void __launch_bounds__(kTileThreads)
+  predict_few_kernel(const T* __restrict__ X, int64_t n_rows, int F, int pitch, int n_trees, int n_batches,
+                     const BatchInfo* __restrict__ batches, const PackedTree* __restrict__ desc,
+                     const PackedNode<T>* __restrict__ nodes, const double* __restrict__ leaves, int K, int node_at,
+                     int cap_words, int cap_trees, int64_t all_words, int value_at, double* __restrict__ out)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  constexpr int kNodesPerWord = 16 / sizeof(PackedNode<T>);
+  T* s_x                = reinterpret_cast<T*>(smem_raw);
+  PackedNode<T>* s_node = reinterpret_cast<PackedNode<T>*>(smem_raw + node_at);
+  double* s_value       = reinterpret_cast<double*>(smem_raw + value_at);  // [tree][row][output]
+  const int tid = threadIdx.x, r = tid % kFewRows, q = tid / kFewRows;
+  const int64_t row0  = blockIdx.x * static_cast<int64_t>(kFewRows);
+  const int rows_here = static_cast<int>(min<int64_t>(kFewRows, n_rows - row0));
+  Word16 ahead[kFewWords];
+  int64_t tree_at[kFewTogether];
+  auto fetch = [&](int64_t first_word, int64_t words) {
+    const Word16* src = reinterpret_cast<const Word16*>(nodes) + first_word;
+#pragma unroll
+    for (int c = 0; c < kFewWords; c++)
+      if (tid + c * kTileThreads < words) ahead[c] = src[tid + c * kTileThreads];
+  };
+  auto fetch_trees = [&](int first) {
+#pragma unroll
+    for (int j = 0; j < kFewTogether; j++) tree_at[j] = desc[min(first + q + j * kFewLanes, n_trees - 1)].node_off;
+  };
+  // the first group begins the array; where it ends is not known yet
+  fetch(0, min<int64_t>(cap_words, all_words));
+  fetch_trees(0);
+  for (int i = tid; i < rows_here * F; i += kTileThreads) {
+    const int row = i / F;
+    s_x[row * pitch + (i - row * F)] = X[row0 * F + i];
+  }
+  const T* my_x   = s_x + (r < rows_here ? r : 0) * pitch;
+  const int items = kFewRows * K;  // (row, output) sums, one a thread
+  double acc      = 0.0;
+  for (int b = 0; b < n_batches;) {
+    // as many batches as fit
+    const int64_t start = batches[b].node_off;
+    int count = 0, steps = 0;
+    int64_t end = start;
+    while (b < n_batches) {
+      const BatchInfo i = batches[b];
+      if ((i.node_off + i.total - start + kNodesPerWord - 1) / kNodesPerWord > cap_words || count + i.count > cap_trees) break;
+      end = i.node_off + i.total;
+      count += i.count;
+      steps = max(steps, i.steps);
+      b++;
+    }
+    if (count == 0) return;  // a batch that does not fit: the host does not launch for such ensembles
+    const int words = static_cast<int>((end - start + kNodesPerWord - 1) / kNodesPerWord);
+#pragma unroll
+    for (int c = 0; c < kFewWords; c++)
+      if (tid + c * kTileThreads < words) reinterpret_cast<Word16*>(s_node)[tid + c * kTileThreads] = ahead[c];
+    int base[kFewTogether], pos[kFewTogether];
+#pragma unroll
+    for (int j = 0; j < kFewTogether; j++) {
+      base[j] = q + j * kFewLanes < count ? static_cast<int>(tree_at[j] - start) : 0;  // lanes without a tree walk the first again
+      pos[j]  = 0;
+    }
+    __syncthreads();
+    if (b < n_batches) {
+      const int64_t next = batches[b].node_off / kNodesPerWord;
+      fetch(next, min<int64_t>(cap_words, all_words - next));
+      fetch_trees(batches[b].first);
+    }
+    for (int s = 0; s < steps; s++) {
+#pragma unroll
+      for (int j = 0; j < kFewTogether; j++) pos[j] = step_from<T>(s_node[base[j] + pos[j]], my_x);
+    }
+#pragma unroll
+    for (int j = 0; j < kFewTogether; j++)
+      if (q + j * kFewLanes < count) {
+        const double* leaf = leaves + (start + base[j] + pos[j]) * K;
+        double* value      = s_value + ((q + j * kFewLanes) * kFewRows + r) * K;
+        for (int k = 0; k < K; k++) value[k] = leaf[k];
+      }
+    __syncthreads();
+    if (tid < items) {
+#pragma unroll 8
+      for (int t = 0; t < count; t++) acc += s_value[t * items + tid];
+    }
+  }
+  if (tid < rows_here * K) out[row0 * K + tid] = acc;
+}
+
 size_t padded_nodes(int n_trees, int64_t total_nodes)
 {
   return static_cast<size_t>(total_nodes) + 2 * static_cast<size_t>(n_trees);  // batches start on 16 bytes
@@ -610,12 +714,51 @@ int pack_tiled(hipStream_t stream, int F, int n_trees, const double* const* leaf
   return LBT_OK;
 }
 
+// The kernel for few rows over a packed ensemble; *done stays false where the tile kernel is the faster one or the shapes
+// do not fit.
+template <typename T>
+int run_few(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble& ens, double* out, bool* done)
+{
+  const int F = ens.n_features, K = ens.n_outputs, pitch = F | 1;
+  if (ens.few_trees != 0 || N > kFewMostRows || kFewRows * K > kTileThreads) return LBT_OK;
+  constexpr int kNodesPerWord = 16 / sizeof(PackedNode<T>);
+  const size_t x_bytes     = (static_cast<size_t>(kFewRows) * pitch * sizeof(T) + 15) & ~size_t(15);
+  const size_t tree_values = static_cast<size_t>(kFewRows) * K * sizeof(double);
+  // a batch holds at most 32 trees; the rest of the values' share is for more of them
+  const int cap_trees = static_cast<int>(std::max<size_t>(32, std::min<size_t>(std::min(kFewGroupTrees, ens.n_trees), 32 * 1024 / tree_values)));
+  const size_t value_bytes = cap_trees * tree_values;
+  if (x_bytes + value_bytes >= kTileLds) return LBT_OK;
+  const int64_t all_words = (ens.total_nodes + ens.n_batches + kNodesPerWord - 1) / kNodesPerWord;  // batches start on whole words
+  const int64_t room      = static_cast<int64_t>((kTileLds - x_bytes - value_bytes) / 16);
+  const int64_t cap_words = std::min<int64_t>({room, all_words, static_cast<int64_t>(kFewWords) * kTileThreads});
+  const size_t tile_rows  = kTileThreads / ens.lanes;
+  const size_t tile_x     = (tile_rows * pitch * sizeof(T) + 15) & ~size_t(15);  // lds_bytes: that and the widest batch
+  if (static_cast<int64_t>(static_cast<size_t>(ens.lds_bytes) - tile_x) / 16 > cap_words + 1 && cap_words < all_words) return LBT_OK;
+  PackedLayout<T> lay(ens.data, ens.n_trees, ens.total_nodes);
+  const int node_at  = static_cast<int>(x_bytes);
+  const int value_at = static_cast<int>(x_bytes + cap_words * 16);
+  ProfScope ps(LBT_PROF_PREDICT, stream, static_cast<double>(N) * (static_cast<double>(F) * sizeof(T) + K * 8.0));
+  static std::atomic<bool> attr[kMaxDevices] = {};
+  LBT_TRY(allow_dynamic_lds(predict_few_kernel<T>, kTileLds, attr));
+  predict_few_kernel<T><<<static_cast<unsigned>((N + kFewRows - 1) / kFewRows), kTileThreads, value_at + value_bytes, stream>>>(
+    X, N, F, pitch, ens.n_trees, ens.n_batches, lay.batches, lay.desc, lay.nodes, lay.leaves, K, node_at,
+    static_cast<int>(cap_words), cap_trees, all_words, value_at, out);
+  LBT_HIP(hipGetLastError());
+  *done = true;
+  return LBT_OK;
+}
+
 // The tile kernel over a packed ensemble.
 template <typename T>
 int run_tiled(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble& ens, double* out,
               const int32_t* wanted = nullptr)
 {
   const int F = ens.n_features, K = ens.n_outputs, n_batches = ens.n_batches;
+  if (wanted == nullptr) {
+    bool done = false;
+    LBT_TRY(run_few<T>(stream, X, N, ens, out, &done));
+    if (done) return LBT_OK;
+  }
   // The lanes the ensemble was laid out for suit many rows. Batches of so many trees fit the kernels for more lanes
   // per row too (their last lanes then have no tree), and where the rows would leave most CUs without a
   // workgroup these split them further and walk fewer trees per lane: 256 x 32, 100 trees of depth 6: 19.0 us

@@ -560,3 +560,31 @@ def test_predict_takes_more_lanes_per_row_for_few_rows(f, k, n_trees, dtype):
         assert torch.equal(ops.predict(X[:rows], trees, k), want[:rows]), rows
         if packed is not None:
             assert torch.equal(packed.predict(X[:rows]), want[:rows]), rows
+
+
+@pytest.mark.parametrize("f,k,n_trees,depth,dtype", [(13, 1, 17, 3, np.float32), (13, 1, 129, 6, np.float32), (160, 1, 300, 8, np.float64),
+                                                     (7, 64, 40, 4, np.float32), (7, 65, 40, 4, np.float32), (300, 5, 33, 8, np.float64),
+                                                     (31, 8, 1000, 3, np.float32)])
+def test_predict_of_few_rows(f, k, n_trees, depth, dtype):
+    """Up to 4096 rows and more than 16 trees: rows around a workgroup's 16, trees around the 128 of a turn, outputs around the 64 that
+    its threads add, ensembles of one and of many turns: equal to the per-node kernel."""
+    from lbtree import ops
+
+    rs = np.random.RandomState(f + n_trees)
+    X = ops.as_device(rs.rand(4097, f).astype(dtype))
+    trees = []
+    for t in range(n_trees):
+        d = depth if t % 3 else rs.randint(1, depth + 1)
+        m, inner = 2 ** (d + 1) - 1, 2 ** d - 1
+        feat = -np.ones(m, np.int32)
+        feat[:inner] = rs.randint(0, f, inner)
+        if t % 2 and inner > 4:
+            feat[rs.randint(1, inner, 2)] = -1
+        trees.append(tuple(ops.as_device(a) for a in (rs.randn(m, k), feat, rs.rand(m))))
+    want = ops.predict(X, trees, k, tiled=False)
+    for rows in (1, 15, 16, 17, 255, 4095, 4096, 4097):
+        assert torch.equal(ops.predict(X[:rows], trees, k), want[:rows]), rows
+    if f <= 160 and dtype == np.float32:
+        packed = ops.PackedEnsemble(trees, k, f, X.dtype)
+        for rows in (1, 17, 4096):
+            assert torch.equal(packed.predict(X[:rows]), want[:rows]), rows
