@@ -316,22 +316,50 @@ __device__ __forceinline__ unsigned tie_key(int rp, int bin, int next)
   return (static_cast<unsigned>(pick & 511) << 11 | static_cast<unsigned>(2047 - (pick - rp))) + 1u;
 }
 
+// Places of the order a scan workgroup holds, by rows, and the LDS it then asks for at a level of n_nodes nodes
+// (see small_scan_kernel). 156 KB of the 160 leave room for its static arrays (0.6 KB).
+constexpr size_t kScanLds = 156 * 1024;
+__host__ __device__ constexpr int small_scan_places(int64_t N) { return N <= 1024 ? 1024 : N <= 2048 ? 2048 : N <= 4096 ? 4096 : kSmallMaxRows; }
+__host__ __device__ constexpr size_t small_scan_lds(int64_t N, int64_t n_nodes)
+{
+  return static_cast<size_t>((N + 1) / 2 * 2 * 8 + (small_scan_places(N) + 4) * 4 + n_nodes * 12 + (n_nodes / 2 + 1) * 4 +
+                             (N + 3) / 4 * 4 + 16);
+}
+
+// The LDS a launch asks for: the order takes the rows and what 16-byte accesses may touch behind them.
+__host__ __device__ constexpr int64_t small_scan_order(int64_t N) { return (N + 15) / 8 * 8; }
+__host__ __device__ constexpr size_t small_scan_use(int64_t N, int64_t n_nodes)
+{
+  return static_cast<size_t>((N + 1) / 2 * 2 * 8 + small_scan_order(N) * 4 + n_nodes * 12 + (n_nodes / 2 + 1) * 4 + (N + 3) / 4 * 4 + 31) / 16 * 16;
+}
+
 // kT threads take kE consecutive places of the order each (kT * kE >= N). What a place needs of its row
 // (its pair of the first output, its side) is staged in the LDS in row order: gathered from the L2 these
 // are three scattered accesses per place, and a workgroup's 8192 places then take a level 90 us
 // (5,000 rows x 500 features). Everything that does not depend on another load is asked for first: the
-// levels of a small tree are a chain of memory latencies.
-template <int kT, int kE, bool kSingle>
-__global__ void __launch_bounds__(kT)
+// levels of a small tree are a chain of memory latencies. So the nodes' sums, the parents' terms of the gain and the
+// segments are staged too where the LDS has the room (kStaged): looked up in memory whenever a thread's places
+// pass on to another node, they are a latency per node (1000 x 10, depth 8: 9.2 us a launch, with that and the
+// gains below 7.8).
+// kG: places of a thread whose gains are formed side by side (one output). A place's two quotients are a chain of 400
+// cycles or more, and one place after the other was half of the launch on 1000 x 10. With more features than CUs it is
+// the other way round: 64 registers let two workgroups of 1024 threads share a CU, and one place at a time is enough
+// (5000 x 500: 32 us a launch, now 25; with 66 registers it was one workgroup).
+template <int kT, int kE, bool kSingle, int kG, bool kStaged>
+__global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
   small_scan_kernel(SmallTreeState st, LevelArgs a)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   int2* s_q                  = reinterpret_cast<int2*>(smem_raw);               // [N]
-  uint32_t* s_order          = reinterpret_cast<uint32_t*>(s_q + (a.N + 1) / 2 * 2);  // [kT * kE + 4]
-  unsigned long long* s_gain = reinterpret_cast<unsigned long long*>(s_order + kT * kE + 4);  // [n_nodes] bits of the best gain
+  uint32_t* s_order          = reinterpret_cast<uint32_t*>(s_q + (a.N + 1) / 2 * 2);  // [small_scan_order(N)]
+  unsigned long long* s_gain = reinterpret_cast<unsigned long long*>(s_order + small_scan_order(a.N));  // [n_nodes] bits of the best gain
   unsigned* s_key            = reinterpret_cast<unsigned*>(s_gain + a.n_nodes);  // [n_nodes] its place in the order of ties
   int* s_left_before         = reinterpret_cast<int*>(s_key + a.n_nodes);        // [n_nodes / 2 + 1]
   uint8_t* s_code            = reinterpret_cast<uint8_t*>(s_left_before + a.n_nodes / 2 + 1);  // [N]
+  I64Pair* s_ns              = reinterpret_cast<I64Pair*>(smem_raw + small_scan_use(a.N, a.n_nodes));  // kStaged: [n_nodes]
+  I64Pair* s_base            = s_ns + a.n_nodes;
+  double* s_parent           = reinterpret_cast<double*>(s_base + a.n_nodes);
+  int2* s_seg                = reinterpret_cast<int2*>(s_parent + a.n_nodes);
   __shared__ I64Pair s_pair[2][kT / 64];
   __shared__ int s_wave[kT / 64];
   __shared__ int s_rp;
@@ -356,11 +384,37 @@ __global__ void __launch_bounds__(kT)
   }
   const int live = st.live[a.depth];
   int rp         = a.depth == 0 ? 0 : st.rp[f];  // first bin of the feature among all bins
-  if (kSingle && usable)
+  const double inv_g = st.scales[2], inv_h = st.scales[3];
+  const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
+  // all loads are under way before the first is stored: a loop that loads and stores waits once per turn
+  int2 pair[kSingle && kG > 1 ? kE : 1];
+  if constexpr (kSingle && kG > 1) {
+#pragma unroll
+    for (int u = 0; u < kE; u++)
+      if (tid + u * kT < a.N) pair[u] = st.qgh[tid + u * kT];
+  } else if (kSingle && usable) {
     for (int i = tid; i < a.N; i += kT) s_q[i] = st.qgh[i];
-  if (a.depth > 0)
-    for (int i = tid * 4; i < a.N; i += kT * 4)
-      *reinterpret_cast<uint32_t*>(s_code + i) = *reinterpret_cast<const uint32_t*>(st.code + i);
+  }
+  uint32_t code[kE / 4];
+#pragma unroll
+  for (int u = 0; u < kE / 4; u++)
+    if (a.depth > 0 && 4 * (tid + u * kT) < a.N) code[u] = *reinterpret_cast<const uint32_t*>(st.code + 4 * (tid + u * kT));
+  if (kStaged && usable)
+    for (int j = tid; j < a.n_nodes; j += kT) {
+      const I64Pair ns = st.node_sums[a.level_first + j];
+      s_base[j]        = st.base[a.level_first + j];
+      s_seg[j]         = st.seg[a.level_first + j];
+      s_ns[j]          = ns;
+      s_parent[j]      = leaf_gain(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, a.l1, reg);
+    }
+  if constexpr (kSingle && kG > 1) {
+#pragma unroll
+    for (int u = 0; u < kE; u++)
+      if (tid + u * kT < a.N) s_q[tid + u * kT] = pair[u];
+  }
+#pragma unroll
+  for (int u = 0; u < kE / 4; u++)
+    if (a.depth > 0 && 4 * (tid + u * kT) < a.N) *reinterpret_cast<uint32_t*>(s_code + 4 * (tid + u * kT)) = code[u];
   if (live == 0 && a.depth > 0) return;
   if (a.depth == 0) {
     int mine = 0;
@@ -391,9 +445,16 @@ __global__ void __launch_bounds__(kT)
     // node[] already is the node of this level at the place: both children of a parent lie where the
     // parent's rows lay, the left one first
     int2 seg[kE];  // the left child's
+    const bool from_lds = kStaged && usable;
+    if (!from_lds) {
 #pragma unroll
-    for (int e = 0; e < kE; e++) seg[e] = node[e] != kNone ? st.seg[a.level_first + (node[e] & ~1)] : make_int2(-1, 0);
+      for (int e = 0; e < kE; e++) seg[e] = node[e] != kNone ? st.seg[a.level_first + (node[e] & ~1)] : make_int2(-1, 0);
+    }
     __syncthreads();
+    if (from_lds) {
+#pragma unroll
+      for (int e = 0; e < kE; e++) seg[e] = node[e] != kNone ? s_seg[node[e] & ~1] : make_int2(-1, 0);
+    }
     unsigned left = 0;
 #pragma unroll
     for (int e = 0; e < kE; e++)
@@ -444,70 +505,114 @@ __global__ void __launch_bounds__(kT)
     const int nn = e + 1 < kE ? node[e + 1] : node_next;
     if (node[e] != kNone && nn == node[e] && bin[e + 1] != bin[e]) ends |= 1u << e;
   }
-  const double inv_g = st.scales[2], inv_h = st.scales[3];
-  const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
   if constexpr (kSingle) {
     // A thread's places are consecutive, so its nodes come one after the other: the best split of a node
     // that begins and ends inside the thread is final, those of its first and last node meet the
     // other threads' in the LDS. Sums, parent's term and best split of the node at hand stay in registers.
+    int2 q[kG > 1 ? kE : 1];
+    auto pair_at = [&](int e) { return i0 + e < a.N ? s_q[entry[e] & 0xffff] : make_int2(0, 0); };
     I64Pair sum{0, 0};
 #pragma unroll
-    for (int e = 0; e < kE; e++)
-      if (i0 + e < a.N) {
-        const int2 v = s_q[entry[e] & 0xffff];
-        sum.grad += v.x;
-        sum.hess += v.y;
-      }
+    for (int e = 0; e < kE; e++) {
+      const int2 v = pair_at(e);
+      if constexpr (kG > 1) q[e] = v;
+      sum.grad += v.x;
+      sum.hess += v.y;
+    }
     const int64_t ig = wave_inclusive_sum(sum.grad), ih = wave_inclusive_sum(sum.hess);
     if (lane == 63) s_pair[0][wave] = I64Pair{ig, ih};
     __syncthreads();
     I64Pair run{ig - sum.grad, ih - sum.hess};
+#pragma unroll 4  // (not all in registers at once)
     for (int w = 0; w < kT / 64; w++) {
       run.grad += w < wave ? s_pair[0][w].grad : 0;
       run.hess += w < wave ? s_pair[0][w].hess : 0;
     }
     int first_node = kNone, cur = kNone;
-    double first_gain = 0.0, cur_gain = 0.0, parent = 0.0;
+    double first_gain = 0.0, cur_gain = 0.0;
     unsigned first_key = 0, cur_key = 0;
-    I64Pair ns{0, 0}, base{0, 0};
+    auto node_at = [&](int j, I64Pair& ns, I64Pair& base, double& parent) {
+      if constexpr (kStaged) {
+        ns     = s_ns[j];
+        base   = s_base[j];
+        parent = s_parent[j];
+      } else {
+        ns     = st.node_sums[a.level_first + j];
+        base   = st.base[a.level_first + j];
+        parent = leaf_gain(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, a.l1, reg);
+      }
+    };
+    // calculate_gain with the parent's term formed once per node
+    auto gain_of = [&](const I64Pair& ls, const I64Pair& rs, double parent) {
+      return 0.0 + ((0.5 * (leaf_gain(static_cast<double>(ls.grad) * inv_g, static_cast<double>(ls.hess) * inv_h, a.l1, reg) +
+                            leaf_gain(static_cast<double>(rs.grad) * inv_g, static_cast<double>(rs.hess) * inv_h, a.l1, reg) -
+                            parent)) -
+                    a.min_split_gain);
+    };
+    auto next_node = [&](int j) {
+      if (first_node == kNone) {
+        first_node = cur;  // (kNone again while there was none before)
+        first_gain = cur_gain;
+        first_key  = cur_key;
+      } else if (cur_key != 0) {
+        s_gain[cur] = static_cast<unsigned long long>(__double_as_longlong(cur_gain));
+        s_key[cur]  = cur_key;
+      }
+      cur      = j;
+      cur_gain = 0.0;
+      cur_key  = 0;
+    };
+    auto offer = [&](double gain, int e) {
+      if (gain >= cur_gain) {
+        const unsigned key = tie_key(rp, bin[e], bin[e + 1]);
+        cur_key            = gain > cur_gain ? key : max(cur_key, key);
+        cur_gain           = gain;
+      }
+    };
+    if constexpr (kG == 1) {
+      I64Pair ns{0, 0}, base{0, 0};
+      double parent = 0.0;
 #pragma unroll
-    for (int e = 0; e < kE; e++) {
-      if (i0 + e < a.N) {
-        const int2 v = s_q[entry[e] & 0xffff];
+      for (int e = 0; e < kE; e++) {
+        const int2 v = pair_at(e);
         run.grad += v.x;
         run.hess += v.y;
+        if ((ends >> e) & 1u) {
+          if (node[e] != cur) {
+            next_node(node[e]);
+            node_at(cur, ns, base, parent);
+          }
+          const I64Pair ls{run.grad - base.grad, run.hess - base.hess}, rs{ns.grad - ls.grad, ns.hess - ls.hess};
+          if (ls.hess > 0 && rs.hess > 0) {
+            const double gain = gain_of(ls, rs, parent);
+            if (gain > 0) offer(gain, e);
+          }
+        }
       }
-      if ((ends >> e) & 1u) {
-        if (node[e] != cur) {
-          if (first_node == kNone) {
-            first_node = cur;  // (kNone again while there was none before)
-            first_gain = cur_gain;
-            first_key  = cur_key;
-          } else if (cur_key != 0) {
-            s_gain[cur] = static_cast<unsigned long long>(__double_as_longlong(cur_gain));
-            s_key[cur]  = cur_key;
-          }
-          cur      = node[e];
-          cur_gain = 0.0;
-          cur_key  = 0;
-          ns       = st.node_sums[a.level_first + cur];
-          base     = st.base[a.level_first + cur];
-          parent   = leaf_gain(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, a.l1, reg);
+    } else {
+#pragma unroll
+      for (int e0 = 0; e0 < kE; e0 += kG) {
+        double gain[kG];
+        bool wanted[kG];
+#pragma unroll
+        for (int u = 0; u < kG; u++) {
+          const int e = e0 + u;
+          run.grad += q[e].x;
+          run.hess += q[e].y;
+          I64Pair ns, base;
+          double parent;
+          node_at(node[e] != kNone ? node[e] : 0, ns, base, parent);
+          const I64Pair ls{run.grad - base.grad, run.hess - base.hess}, rs{ns.grad - ls.grad, ns.hess - ls.hess};
+          wanted[u] = ((ends >> e) & 1u) != 0 && ls.hess > 0 && rs.hess > 0;
+          gain[u]   = gain_of(ls, rs, parent);
         }
-        const I64Pair ls{run.grad - base.grad, run.hess - base.hess}, rs{ns.grad - ls.grad, ns.hess - ls.hess};
-        if (ls.hess > 0 && rs.hess > 0) {
-          // calculate_gain with the parent's term formed once per node
-          const double gain =
-            0.0 + ((0.5 * (leaf_gain(static_cast<double>(ls.grad) * inv_g, static_cast<double>(ls.hess) * inv_h, a.l1, reg) +
-                           leaf_gain(static_cast<double>(rs.grad) * inv_g, static_cast<double>(rs.hess) * inv_h, a.l1, reg) -
-                           parent)) -
-                   a.min_split_gain);
-          if (gain > 0 && gain >= cur_gain) {
-            const unsigned key = tie_key(rp, bin[e], bin[e + 1]);
-            cur_key            = gain > cur_gain ? key : max(cur_key, key);
-            cur_gain           = gain;
+        // (a node without a candidate here is none of those that the thread has to report)
+#pragma unroll
+        for (int u = 0; u < kG; u++)
+          if (wanted[u] && gain[u] > 0) {
+            if (node[e0 + u] != cur) next_node(node[e0 + u]);
+            offer(gain[u], e0 + u);
           }
-        }
       }
     }
     // one slot for the node the thread begins with, one for the node it ends with (the same one, or none)
@@ -657,7 +762,9 @@ __global__ void __launch_bounds__(kT)
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int live      = st.live[a.depth];
   const int2 seg      = st.seg[node];
-  const int64_t hess0 = st.node_sums[static_cast<int64_t>(node) * a.K].hess;
+  // what only the last lines need is asked for here
+  const double inv_g = st.scales[2], inv_h = st.scales[3];
+  const I64Pair ns0 = st.node_sums[static_cast<int64_t>(node) * a.K], base0 = st.base[static_cast<int64_t>(node) * a.K];
   const int s0 = seg.x, n = seg.y;
   if (live == 0 || n == 0) return;
   const uint32_t* order = st.order[a.depth & 1] + s0;  // feature 0's
@@ -697,7 +804,7 @@ __global__ void __launch_bounds__(kT)
       take(s_best[w], static_cast<unsigned>(p.x), p.y, p.z);
     }
   }
-  if (!(hess0 > 0 && best_key != 0 && best > 1e-5)) {
+  if (!(ns0.hess > 0 && best_key != 0 && best > 1e-5)) {
     for (int i = tid; i < n; i += kT) {
       st.node_of_pos[s0 + i] = kNone;
       if (row_leaf != nullptr) row_leaf[row_at(i)] = node;
@@ -706,6 +813,7 @@ __global__ void __launch_bounds__(kT)
   }
   const int lc = left_child(node), rc = right_child(node);
   const uint16_t* bins = st.bins + static_cast<int64_t>(ft) * st.pitch;
+  const double value   = st.proposals[static_cast<int64_t>(ft) * a.S + rel];
   int nl = 0;
   I64Pair sum{0, 0};
   for (int i = tid; i < n; i += kT) {
@@ -720,7 +828,6 @@ __global__ void __launch_bounds__(kT)
       sum.hess += q.y;
     }
   }
-  const double inv_g = st.scales[2], inv_h = st.scales[3];
   for (int k = 0;;) {
     const int64_t ig = wave_inclusive_sum(sum.grad), ih = wave_inclusive_sum(sum.hess);
     if (lane == 63) s_sum[k & 1][wave] = I64Pair{ig, ih};
@@ -729,26 +836,21 @@ __global__ void __launch_bounds__(kT)
       if (lane == 63) s_cnt[wave] = c;
     }
     __syncthreads();
-    if (tid == 0) {
+    if (tid < 2) {
+      // a child each, the left one first
       I64Pair ls{0, 0};
       for (int w = 0; w < kT / 64; w++) {
         ls.grad += s_sum[k & 1][w].grad;
         ls.hess += s_sum[k & 1][w].hess;
       }
-      const int64_t at = static_cast<int64_t>(node) * a.K + k, l = static_cast<int64_t>(lc) * a.K + k,
-                    r = static_cast<int64_t>(rc) * a.K + k;
-      const I64Pair ns = st.node_sums[at], base = st.base[at];
-      const I64Pair rs{ns.grad - ls.grad, ns.hess - ls.hess};
-      st.node_sums[l] = ls;
-      st.node_sums[r] = rs;
-      st.base[l]      = base;
-      st.base[r]      = I64Pair{base.grad + ls.grad, base.hess + ls.hess};
-      const double lg = static_cast<double>(ls.grad) * inv_g, lh = static_cast<double>(ls.hess) * inv_h;
-      const double rg = static_cast<double>(rs.grad) * inv_g, rh = static_cast<double>(rs.hess) * inv_h;
-      leaf[l]    = calculate_leaf_value(lg, lh, a.l1, a.l2);
-      leaf[r]    = calculate_leaf_value(rg, rh, a.l1, a.l2);
-      hessian[l] = lh;
-      hessian[r] = rh;
+      const int64_t at = static_cast<int64_t>(node) * a.K + k, to = static_cast<int64_t>(tid == 0 ? lc : rc) * a.K + k;
+      const I64Pair ns = k == 0 ? ns0 : st.node_sums[at], base = k == 0 ? base0 : st.base[at];
+      const I64Pair own{tid == 0 ? ls.grad : ns.grad - ls.grad, tid == 0 ? ls.hess : ns.hess - ls.hess};
+      st.node_sums[to] = own;
+      st.base[to]      = I64Pair{base.grad + (tid == 0 ? 0 : ls.grad), base.hess + (tid == 0 ? 0 : ls.hess)};
+      const double g = static_cast<double>(own.grad) * inv_g, h = static_cast<double>(own.hess) * inv_h;
+      leaf[to]    = calculate_leaf_value(g, h, a.l1, a.l2);
+      hessian[to] = h;
     }
     if (++k == a.K) break;
     sum = I64Pair{0, 0};
@@ -765,7 +867,7 @@ __global__ void __launch_bounds__(kT)
   for (int w = 0; w < kT / 64; w++) lefts += s_cnt[w];
   if (tid == 0) {
     feature[node] = ft;
-    split[node]   = st.proposals[static_cast<int64_t>(ft) * a.S + rel];
+    split[node]   = value;
     gain[node]    = best;
     st.seg[lc]    = make_int2(s0, lefts);
     st.seg[rc]    = make_int2(s0 + lefts, n - lefts);
@@ -790,29 +892,28 @@ __global__ void __launch_bounds__(256) small_count_kernel(SmallTreeState st, Lev
   }
 }
 
-// Places of the order a scan workgroup holds, by rows, and the LDS it then asks for at a level of n_nodes nodes
-// (see small_scan_kernel). 156 KB of the 160 leave room for its static arrays (0.6 KB).
-constexpr size_t kScanLds = 156 * 1024;
-constexpr int small_scan_places(int64_t N) { return N <= 1024 ? 1024 : N <= 2048 ? 2048 : N <= 4096 ? 4096 : kSmallMaxRows; }
-constexpr size_t small_scan_lds(int64_t N, int64_t n_nodes)
-{
-  return static_cast<size_t>((N + 1) / 2 * 2 * 8 + (small_scan_places(N) + 4) * 4 + n_nodes * 12 + (n_nodes / 2 + 1) * 4 +
-                             (N + 3) / 4 * 4 + 16);
-}
-
-template <int kT, int kE, bool kSingle>
-int launch_small_scan_as(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a)
+template <int kT, int kE, bool kSingle, int kG, bool kStaged>
+int launch_small_scan_as(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a, size_t lds)
 {
   static std::atomic<bool> attr_set[kMaxDevices] = {};
   LBT_REQUIRE(small_scan_places(a.N) == kT * kE, "%d rows do not take a workgroup of %d places", a.N, kT * kE);
-  LBT_TRY(allow_dynamic_lds(small_scan_kernel<kT, kE, kSingle>, kScanLds, attr_set));
-  small_scan_kernel<kT, kE, kSingle><<<a.F, kT, small_scan_lds(a.N, a.n_nodes), stream>>>(st, a);
+  LBT_TRY((allow_dynamic_lds(small_scan_kernel<kT, kE, kSingle, kG, kStaged>, kScanLds + 64, attr_set)));
+  small_scan_kernel<kT, kE, kSingle, kG, kStaged><<<a.F, kT, lds, stream>>>(st, a);
   return LBT_OK;
 }
 template <int kT, int kE>
 int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a)
 {
-  return a.K == 1 ? launch_small_scan_as<kT, kE, true>(stream, st, a) : launch_small_scan_as<kT, kE, false>(stream, st, a);
+  const size_t lds  = small_scan_use(a.N, a.n_nodes);
+  const size_t more = lds + static_cast<size_t>(a.n_nodes) * (2 * sizeof(I64Pair) + sizeof(double) + sizeof(int2));
+  if (a.K > 1) return launch_small_scan_as<kT, kE, false, 1, false>(stream, st, a, lds);
+  // staging must not cost a workgroup of the CU where there are more of them than CUs
+  auto per_cu        = [](size_t bytes) { return static_cast<int>(std::min<size_t>(2048 / kT, 160 * 1024 / (bytes + 1024))); };
+  const bool crowded = kT == 1024 && a.F > 256;
+  if (more > kScanLds || (per_cu(more) < per_cu(lds) && a.F > 256 * per_cu(more)))
+    return launch_small_scan_as<kT, kE, true, 1, false>(stream, st, a, lds);
+  if (crowded) return launch_small_scan_as<kT, kE, true, 1, true>(stream, st, a, more);
+  return launch_small_scan_as<kT, kE, true, kE == 8 ? 2 : 4, true>(stream, st, a, more);
 }
 
 }  // namespace

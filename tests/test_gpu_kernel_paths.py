@@ -588,3 +588,20 @@ def test_predict_of_few_rows(f, k, n_trees, depth, dtype):
         packed = ops.PackedEnsemble(trees, k, f, X.dtype)
         for rows in (1, 17, 4096):
             assert torch.equal(packed.predict(X[:rows]), want[:rows]), rows
+
+
+@pytest.mark.parametrize("n,f,s,depth", [(1024, 300, 64, 9), (4096, 257, 128, 8), (4097, 257, 64, 11), (8192, 260, 256, 9), (7999, 30, 256, 11),
+                                         (2049, 256, 32, 10)])
+def test_few_rows_with_the_nodes_staged_or_not(n, f, s, depth):
+    """Either side of the sizes at which the scan keeps the nodes in the LDS (levels whose nodes do not fit beside the rows) and at
+    which two of its workgroups share a CU (more features than CUs), rows around its numbers of places."""
+    import gpu_util as gu
+    import oracle_lib as orc
+
+    rs = np.random.RandomState(n + f)
+    X = rs.randn(n, f).astype(np.float32)
+    g, h = rs.randn(n, 1), 0.5 + rs.rand(n, 1)
+    kw = dict(max_depth=depth, split_samples=s, seed=3)
+    got = gu.gpu_build(X, g, h, taps=False, **kw)
+    cr = orc.build_tree(X, g, h, **kw)
+    _assert_tree(got, cr)
