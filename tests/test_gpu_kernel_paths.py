@@ -605,3 +605,30 @@ def test_few_rows_with_the_nodes_staged_or_not(n, f, s, depth):
     got = gu.gpu_build(X, g, h, taps=False, **kw)
     cr = orc.build_tree(X, g, h, **kw)
     _assert_tree(got, cr)
+
+
+# A level of up to 512 (node, feature) pairs is scanned by four or eight waves a pair, a wider one by one wave: tiles
+# of 64 bins that do not divide evenly among the waves, fewer tiles than waves, features of one bin, levels on both
+# sides of the line, outputs whose hessians vanish, a penalty and features that are not to be split.
+@pytest.mark.parametrize("f,k,s,depth,kind", [(64, 1, 512, 5, "plain"), (64, 3, 129, 5, "plain"), (5, 8, 300, 4, "l1"), (513, 1, 65, 2, "plain"),
+                                              (128, 2, 64, 4, "plain"), (9, 64, 257, 3, "plain"), (33, 5, 256, 6, "feature_set"),
+                                              (17, 4, 400, 5, "zero_output"), (40, 1, 449, 5, "zero_hessians")])
+def test_waves_that_share_a_scan(f, k, s, depth, kind):
+    import gpu_util as gu
+
+    rs = np.random.RandomState(f + k + s)
+    n = 6001
+    X = rs.randn(n, f).astype(np.float32)
+    X[:, 0] = 1.0  # one bin
+    X[:, 1] = rs.randint(0, 70, n)
+    g, h = rs.randn(n, k), rs.rand(n, k) + 0.5
+    if kind == "zero_output":
+        g[:, k - 1] = h[:, k - 1] = 0.0
+    if kind == "zero_hessians":
+        h[rs.rand(n) < 0.3] = 0.0
+    more = {"l1_regularization": 3.0} if kind == "l1" else {}
+    if kind == "feature_set":
+        more["feature_set"] = rs.rand(f) < 0.5
+    for levels in (True, False):
+        gr, cr = gu.both(X, g, h, levels=levels, max_depth=depth, split_samples=s, seed=f, **more)
+        gu.assert_tree_parity(gr, cr, levels=levels)
