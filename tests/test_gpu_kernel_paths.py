@@ -632,3 +632,30 @@ def test_waves_that_share_a_scan(f, k, s, depth, kind):
     for levels in (True, False):
         gr, cr = gu.both(X, g, h, levels=levels, max_depth=depth, split_samples=s, seed=f, **more)
         gu.assert_tree_parity(gr, cr, levels=levels)
+
+
+# The prefix counts of a level's partition: one slab of 2048 rows, edges of slabs, more slabs than threads that
+# scan them (1024), more than a thread asks for at once (8192), more parents than waves of a workgroup, than rows.
+@pytest.mark.parametrize("n,level", [(1, 0), (2047, 1), (2048, 0), (2049, 2), (5000, 5), (3000, 11), (70001, 8), (2_100_000, 3), (17_000_003, 4)])
+def test_partition_of_a_level_is_the_stable_sort(n, level):
+    from lbtree import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(n + level)
+    first, parents = (1 << level) - 1, 1 << level
+    X = torch.rand((n, 1), device="cuda", generator=gen)
+    node = torch.randint(-1, parents, (n,), device="cuda", generator=gen, dtype=torch.int32)
+    node[node % 7 == 3] = -1  # retired rows, and parents without rows
+    node = torch.where(node < 0, node, node + first).sort().values
+    rows = torch.randperm(n, device="cuda", generator=gen).to(torch.int32)
+    feature = torch.zeros(2 * parents + first, device="cuda", dtype=torch.int32)
+    feature[first + 5 :: 6] = -1  # leaves
+    split = torch.rand(feature.shape[0], device="cuda", generator=gen, dtype=torch.float64)
+    positions = torch.stack([node, rows], dim=1).contiguous()
+
+    at = node.clamp(min=0).long()
+    left = X[rows.long(), 0].double() <= split[at]
+    want = torch.where((node < 0) | (feature[at] < 0), -1, 2 * node + 2 - left.int())
+    order = torch.sort(want, stable=True).indices
+    want = torch.stack([want[order], rows[order]], dim=1).to(torch.int32)
+    ops.update_positions(X, positions, feature, split, level)
+    assert torch.equal(positions, want)
