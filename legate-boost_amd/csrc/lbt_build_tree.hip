@@ -264,22 +264,26 @@ __global__ void scales_kernel(const double* sum_a, const double* sum_b, double* 
 // Stochastic rounding of every (row, output) once per tree, stored as int32
 // pairs, plus the root sums (build_tree.cu:112-129, :168-204). The reference
 // redoes this rounding inside every histogram launch; the values are the same.
-__global__ void __launch_bounds__(kThreads)
+// Bound by memory for many rows. For fewer it is the workgroups' three additions to the same words, which take turns
+// of about 9 ns: 2048 workgroups of 256 threads took 53 us for 1,000,000 rows, 256 of 1024 take 14 (10,000,000
+// rows: 67, now 53). A thread asks for the rows of its next kQuantiseRows turns together.
+constexpr int kQuantiseThreads = 1024, kQuantiseGroups = 256, kQuantiseRows = 4;
+__global__ void __launch_bounds__(kQuantiseThreads)
   quantise_kernel(const double* g, const double* h, int64_t n_rows, int K, int64_t row_offset,
                   int64_t seed, const double* scales, int2* q_out, I64Pair* node_sums,
                   unsigned long long* qstats)
 {
-  __shared__ int64_t s_g[kThreads / 64];
-  __shared__ int64_t s_h[kThreads / 64];
-  __shared__ unsigned long long s_m[kThreads / 64];
+  __shared__ int64_t s_g[kQuantiseThreads / 64];
+  __shared__ int64_t s_h[kQuantiseThreads / 64];
+  __shared__ unsigned long long s_m[kQuantiseThreads / 64];
+  __shared__ unsigned s_bad[kQuantiseThreads / 64];
   const int k = blockIdx.y;
   const double sg = scales[0], sh = scales[1];
   int64_t sum_g = 0, sum_h = 0;
   unsigned long long mx = 0;
   unsigned bad = 0;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
-  for (int64_t row = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x; row < n_rows; row += stride) {
-    double grad = g[row * K + k], hess = h[row * K + k];
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kQuantiseThreads;
+  auto round_row = [&](int64_t row, double grad, double hess) {
     uint32_t x  = minstd_seed(static_cast<uint32_t>(
       static_cast<uint64_t>(gpair_seed(seed, row + row_offset, static_cast<int64_t>(k)))));
     double scaled_grad    = grad * sg;
@@ -299,30 +303,46 @@ __global__ void __launch_bounds__(kThreads)
     mx = ah > mx ? ah : mx;
     sum_g += qg;
     sum_h += qh;
+  };
+  for (int64_t row = blockIdx.x * static_cast<int64_t>(kQuantiseThreads) + threadIdx.x; row < n_rows;
+       row += kQuantiseRows * stride) {
+    double grad[kQuantiseRows], hess[kQuantiseRows];
+#pragma unroll
+    for (int u = 0; u < kQuantiseRows; u++) {
+      const int64_t at = row + u * stride < n_rows ? row + u * stride : row;
+      grad[u] = g[at * K + k];
+      hess[u] = h[at * K + k];
+    }
+#pragma unroll
+    for (int u = 0; u < kQuantiseRows; u++)
+      if (row + u * stride < n_rows) round_row(row + u * stride, grad[u], hess[u]);
   }
   for (int off = 32; off >= 1; off >>= 1) {
     sum_g += __shfl_down(sum_g, off, 64);
     sum_h += __shfl_down(sum_h, off, 64);
     unsigned long long o = __shfl_down(mx, off, 64);
     mx = o > mx ? o : mx;
+    bad |= __shfl_down(bad, off, 64);
   }
-  if (bad != 0) atomicOr(&qstats[1], static_cast<unsigned long long>(bad));
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   if (lane == 0) {
     s_g[wave] = sum_g;
     s_h[wave] = sum_h;
     s_m[wave] = mx;
+    s_bad[wave] = bad;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < kThreads / 64; w++) {
+    for (int w = 1; w < kQuantiseThreads / 64; w++) {
       sum_g += s_g[w];
       sum_h += s_h[w];
       mx = s_m[w] > mx ? s_m[w] : mx;
+      bad |= s_bad[w];
     }
     atomic_add_i64(&node_sums[k].grad, sum_g);
     atomic_add_i64(&node_sums[k].hess, sum_h);
     atomicMax(&qstats[0], mx);
+    if (bad != 0) atomicOr(&qstats[1], static_cast<unsigned long long>(bad));
   }
 }
 
@@ -337,8 +357,9 @@ __global__ void __launch_bounds__(kThreads)
 {
   extern __shared__ unsigned long long s_sums[];  // [K] grad, [K] hess
   __shared__ unsigned long long s_max;
+  __shared__ unsigned s_bad;
   for (int i = threadIdx.x; i < 2 * K; i += kThreads) s_sums[i] = 0;
-  if (threadIdx.x == 0) s_max = 0;
+  if (threadIdx.x == 0) s_max = s_bad = 0;
   __syncthreads();
   const double sg = scales[0], sh = scales[1];
   const int64_t n       = n_rows * K;
@@ -377,14 +398,17 @@ __global__ void __launch_bounds__(kThreads)
     atomicAdd(&s_sums[K + k], static_cast<unsigned long long>(sum_h));
     atomicMax(&s_max, mx);
   }
-  if (bad != 0) atomicOr(&qstats[1], static_cast<unsigned long long>(bad));
+  if (bad != 0) atomicOr(&s_bad, bad);
   __syncthreads();
   for (int i = threadIdx.x; i < K; i += kThreads) {
     const unsigned long long vg = s_sums[i], vh = s_sums[K + i];
     if (vg != 0) atomic_add_i64(&node_sums[i].grad, static_cast<int64_t>(vg));
     if (vh != 0) atomic_add_i64(&node_sums[i].hess, static_cast<int64_t>(vh));
   }
-  if (threadIdx.x == 0) atomicMax(&qstats[0], s_max);
+  if (threadIdx.x == 0) {
+    atomicMax(&qstats[0], s_max);
+    if (s_bad != 0) atomicOr(&qstats[1], static_cast<unsigned long long>(s_bad));
+  }
 }
 
 // build_tree.cu:1175-1185
@@ -1758,8 +1782,8 @@ int run_quantiser(hipStream_t stream, const double* g, const double* h, int64_t 
     quantise_flat_kernel<<<gx, kThreads, 2 * K * sizeof(unsigned long long), stream>>>(
       g, h, N, K, row_offset, static_cast<int64_t>(seed), scales, qgh, root_sums, qstats);
   } else {
-    dim3 grid(std::min<unsigned>(blocks(N, kThreads), 2048u), K);
-    quantise_kernel<<<grid, kThreads, 0, stream>>>(g, h, N, K, row_offset, static_cast<int64_t>(seed), scales, qgh,
+    dim3 grid(std::min<unsigned>(blocks(N, kQuantiseThreads), kQuantiseGroups), K);
+    quantise_kernel<<<grid, kQuantiseThreads, 0, stream>>>(g, h, N, K, row_offset, static_cast<int64_t>(seed), scales, qgh,
                                                    root_sums, qstats);
   }
   LBT_HIP(hipGetLastError());

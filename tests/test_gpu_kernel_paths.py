@@ -659,3 +659,17 @@ def test_partition_of_a_level_is_the_stable_sort(n, level):
     want = torch.stack([want[order], rows[order]], dim=1).to(torch.int32)
     ops.update_positions(X, positions, feature, split, level)
     assert torch.equal(positions, want)
+
+
+# Rounded gradients of one output: fewer rows than a workgroup, ragged ends of a thread's four rows, and hessians that
+# round to zero in the last row only, which decides how the levels after the root may be built.
+@pytest.mark.parametrize("n", [1, 1023, 262145, 3 * 262144 + 77, 1_300_000])
+def test_rounding_of_one_output(n):
+    import gpu_util as gu
+
+    rs = np.random.RandomState(n % 1000)
+    X = rs.randn(n, 3).astype(np.float32)
+    g, h = rs.randn(n, 1), rs.rand(n, 1) + 0.5
+    h[-1] = 1e-13
+    gr, cr = gu.both(X, g, h, levels=True, max_depth=3, split_samples=32, seed=7)
+    gu.assert_tree_parity(gr, cr, levels=True)
