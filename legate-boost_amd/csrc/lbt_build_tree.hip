@@ -579,11 +579,6 @@ __device__ __forceinline__ double leaf_gain_select(double grad, double hess, dou
   return (z * z) / (hess + reg);
 }
 
-__device__ __forceinline__ double wave_read_lane_f64(double v, int src)
-{
-  return __longlong_as_double(wave_read_lane(static_cast<int64_t>(__double_as_longlong(v)), src));
-}
-
 template <int kW>
 __global__ void __launch_bounds__(kW == 1 ? kThreads : kW * 64)
   scan_split_kernel(HistView hist, const I64Pair* __restrict__ node_sums, int F, const int32_t* __restrict__ row_pointers,

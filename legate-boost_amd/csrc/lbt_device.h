@@ -70,6 +70,11 @@ __device__ __forceinline__ int64_t wave_read_lane(int64_t v, int src)
   return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+__device__ __forceinline__ double wave_read_lane_f64(double v, int src)
+{
+  return __longlong_as_double(wave_read_lane(static_cast<int64_t>(__double_as_longlong(v)), src));
+}
+
 struct Cand {
   double gain;
   int bin;

@@ -2,7 +2,7 @@
 //
 // With many nodes a level's histograms are far larger than the rows they are made of (1,000,000 x 50 with 512
 // samples: 0.84 GB at 2048 nodes against 0.13 GB of records), and clearing, adding, reducing and scanning them took
-// 0.74 ms of the 2.7 ms of a depth-12 tree for the last level alone (now 0.24 ms). Here both siblings of every pair are
+// 0.74 ms of the 2.7 ms of a depth-12 tree for the last level alone (now 0.18 ms). Here both siblings of every pair are
 // accumulated from their rows, but a histogram never leaves the LDS: a workgroup = (node, 16 bytes of a record's
 // bins) adds its rows, scans its features' bins and keeps the best split of each. What bounds it is the
 // gather of the records and the evaluation of the bins; 64 bins without a row cost one comparison.
@@ -20,6 +20,8 @@
 // (build_tree.cu:645 leaves nothing unscanned) and it does not matter that nothing is derived by subtraction.
 #include "lbt_device.h"
 #include "lbt_internal.h"
+
+#include <type_traits>
 
 namespace lbt {
 namespace {
@@ -41,40 +43,224 @@ __device__ __forceinline__ I64Pair unpack_sums(unsigned long long w, int64_t up,
 constexpr int kDirectRange = 8192;              // positions of a range
 constexpr int kDirectLarge = 2 * kDirectRange;  // rows of a node that one workgroup takes: a range meets at most two larger ones
 
-// The rows at positions [begin, end) into the LDS histograms of the nf features of a piece, [kPer][width].
+// A thread's next rows: what a piece of their records holds and their pairs. Positions behind the last one read it again.
+constexpr int kRowsAtOnce = 4;
+struct RowBatch {
+  uint4 w[kRowsAtOnce];
+  int2 q[kRowsAtOnce];
+  __device__ __forceinline__ void load(const DirectLevel& a, const RecInfo& ri, int piece, int i, int end)
+  {
+    const unsigned char* const cache = static_cast<const unsigned char*>(a.binned) + ri.base;
+    int row[kRowsAtOnce];
+#pragma unroll
+    for (int u = 0; u < kRowsAtOnce; u++) row[u] = a.rows[min(i + u * kDirectThreads, end - 1)];
+#pragma unroll
+    for (int u = 0; u < kRowsAtOnce; u++) {
+      const unsigned char* r = cache + static_cast<int64_t>(row[u]) * ri.stride;
+      w[u] = *reinterpret_cast<const uint4*>(r + piece * 16);
+      q[u] = *reinterpret_cast<const int2*>(r + ri.q_off);
+    }
+  }
+};
+
+// The rows at positions [begin, end) into the LDS histograms [kPer][width] of the nf features of a
+// piece, cleared here. A row is two loads one after the other, its number and its record, and a workgroup of a
+// deep level has few rows: four a thread are under way together, the first ones while the histograms are cleared
+// (one at a time
+// the levels of 512, 1024 and 2048 nodes of 1,000,000 x 50 took 108, 127 and 193 us, now 92, 108 and 176; two at a time
+// the same).
 template <typename BinT>
 __device__ __forceinline__ void add_rows(const DirectLevel& a, const RecInfo& ri, int piece, int nf, int begin, int end,
                                          int width, unsigned long long* s_hist)
 {
-  constexpr int kPer = 16 / sizeof(BinT);
-  const int tid      = threadIdx.x;
-  const unsigned char* const cache = static_cast<const unsigned char*>(a.binned) + ri.base;
-  for (int i = begin + tid; i < end; i += kDirectThreads) {
-    const unsigned char* r = cache + static_cast<int64_t>(a.rows[i]) * ri.stride;
-    const uint4 w          = *reinterpret_cast<const uint4*>(r + piece * 16);
-    const int2 q           = *reinterpret_cast<const int2*>(r + ri.q_off);
-    const unsigned long long word =
-      (static_cast<unsigned long long>(static_cast<uint32_t>(q.x)) << 32) | static_cast<uint32_t>(q.y);
-    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+  constexpr int kPer  = 16 / sizeof(BinT);
+  constexpr int kStep = kRowsAtOnce * kDirectThreads;
+  int i = begin + static_cast<int>(threadIdx.x);
+  RowBatch batch;
+  if (begin < end) batch.load(a, ri, piece, i, end);
+  for (int k = threadIdx.x; k < nf * width; k += kDirectThreads) s_hist[k] = 0;
+  __syncthreads();
+  while (i < end) {
 #pragma unroll
-    for (int v = 0; v < kPer; v++)
-      if (v < nf) {
-        const unsigned bin = sizeof(BinT) == 1 ? (ws[v >> 2] >> (8 * (v & 3))) & 0xffu : (ws[v >> 1 & 3] >> (16 * (v & 1))) & 0xffffu;
-        atomicAdd(s_hist + v * width + bin, word);
-      }
+    for (int u = 0; u < kRowsAtOnce; u++) {
+      if (i + u * kDirectThreads >= end) continue;
+      const unsigned long long word =
+        (static_cast<unsigned long long>(static_cast<uint32_t>(batch.q[u].x)) << 32) | static_cast<uint32_t>(batch.q[u].y);
+      const uint32_t ws[4] = {batch.w[u].x, batch.w[u].y, batch.w[u].z, batch.w[u].w};
+#pragma unroll
+      for (int v = 0; v < kPer; v++)
+        if (v < nf) {
+          const unsigned bin = sizeof(BinT) == 1 ? (ws[v >> 2] >> (8 * (v & 3))) & 0xffu : (ws[v >> 1 & 3] >> (16 * (v & 1))) & 0xffffu;
+          atomicAdd(s_hist + v * width + bin, word);
+        }
+    }
+    i += kStep;
+    if (i < end) batch.load(a, ri, piece, i, end);
   }
+  __syncthreads();
+}
+
+// Inclusive sums over a wave of packed words. The lower halves' sums stay below 2^32, so nothing is carried and the halves
+// are summed on their own, six additions each (64 bits wide hipcc makes five instructions of a step).
+__device__ __forceinline__ unsigned long long wave_inclusive_halves(unsigned long long v)
+{
+  const uint32_t lo = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(static_cast<uint32_t>(v))));
+  const uint32_t hi = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(v >> 32)));
+  return static_cast<unsigned long long>(hi) << 32 | lo;
+}
+
+// A split candidate with what lies left of it, packed. Selects instead of branches: with `if (better) { best = c;
+// left = l; }` around the short-circuit comparison hipcc 7.2 kept the old `left` for lanes that had a candidate already.
+struct Found {
+  double gain;
+  int bin;
+  unsigned long long left;
+  __device__ __forceinline__ void take(double o_gain, int o_bin, unsigned long long o_left, bool valid)
+  {
+    const int o_rank = o_bin & 511, rank = bin & 511;  // the order of cand_better
+    const bool tie    = (o_rank > rank) | ((o_rank == rank) & (o_bin < bin));
+    const bool better = valid & (o_bin >= 0) & ((bin < 0) | (o_gain > gain) | ((o_gain == gain) & tie));
+    gain = better ? o_gain : gain;
+    bin  = better ? o_bin : bin;
+    left = better ? o_left : left;
+  }
+};
+
+// The best split of one feature, by one wave: every bin's gain as the split evaluation defines it.
+__device__ __forceinline__ Found scan_feature(const DirectLevel& a, const I64Pair& ns, int fb, int n_bins, double inv_g,
+                                              double inv_h, double reg, int64_t up, int64_t down,
+                                              const unsigned long long* s_bins)
+{
+  const int lane = threadIdx.x & 63;
+  unsigned long long before = 0;
+  double gain_before = 0.0;  // of the last bin so far: empty bins behind it have the same split
+  Found best{0.0, -1, 0};
+  for (int base = 0; base < n_bins; base += 64) {
+    const int bin                = base + lane;
+    const bool in                = bin < n_bins;
+    const unsigned long long add = in ? s_bins[bin] : 0;
+    double gain                  = gain_before;
+    unsigned long long left      = before;
+    if (__any(add != 0)) {
+      left += wave_inclusive_halves(add);
+      const I64Pair ls = unpack_sums(left, up, down);
+      bool dead        = false;
+      gain             = 0.0;
+      add_gain(gain, dead, ls, ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
+      before      = static_cast<unsigned long long>(wave_read_lane(static_cast<int64_t>(left), 63));
+      gain_before = wave_read_lane_f64(gain, 63);
+    }
+    best.take(gain, fb + bin, left, in & (gain > 0));
+  }
+  for (int off = 32; off >= 1; off >>= 1)
+    best.take(__shfl_xor(best.gain, off, 64), __shfl_xor(best.bin, off, 64), __shfl_xor(best.left, off, 64), true);
+  return best;
+}
+
+// Largest value of a wave, in every lane; values are not negative zero and not NaN
+__device__ __forceinline__ double wave_max(double v)
+{
+  auto take = [&](auto ctrl, auto rows) {
+    const int64_t bits = __double_as_longlong(v);
+    // lanes without a source take their own value
+    const int lo = __builtin_amdgcn_update_dpp(static_cast<int>(bits), static_cast<int>(bits), decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(static_cast<int>(bits >> 32), static_cast<int>(bits >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    const double o = __longlong_as_double((static_cast<int64_t>(hi) << 32) | static_cast<uint32_t>(lo));
+    v = o > v ? o : v;
+  };
+  using std::integral_constant;
+  take(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});
+  take(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
+  take(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
+  take(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
+  take(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});
+  take(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});
+  return wave_read_lane_f64(v, 63);
+}
+
+// Most bins cannot be the best split, and a shorter sum shows it. With integers gl, hl, gr, hr left and right of a bin,
+// gl^2 / (hl + reg / inv_h) + gr^2 / (hr + reg / inv_h) times inv_g^2 / inv_h is what the gain is made of without a
+// penalty (l1 = 0); formed with one approximate reciprocal (to 2^-23, the instruction's bound) it is right to 2^-22.
+// The gain is a monotone function of the two quotients' sum, and every rounding on the way to it (minus the node's own
+// term, minus a min_split_gain that is not negative, where it ends above 0) merges sums within a few units of 2^-52: so a
+// bin whose estimate is below 1 - 2^-20 of the feature's largest has a smaller gain. One gain per lane is then
+// formed exactly, of its largest estimate, and where a lane holds a second one that near (a plateau of 64 empty bins,
+// equal columns) the feature is scanned as above.
+// The levels of 512, 1024 and 2048 nodes of 1,000,000 x 50 with 512 samples: 120, 149 and 234 us with every gain, 108, 127
+// and 193 with estimates (about 60 instructions for 64 bins, and the launch is bound by them still).
+// Not used with magnitudes whose squares might leave the doubles' range.
+constexpr double kNearBest = 1.0 - 1.0 / (1 << 20);
+__device__ __forceinline__ bool estimates_hold(const DirectLevel& a, double inv_g, double inv_h, double reg)
+{
+  auto ordinary = [](double v) { return v >= 1e-60 && v <= 1e60; };
+  return a.l1 == 0.0 && a.min_split_gain >= 0.0 && ordinary(inv_g) && ordinary(inv_h) && ordinary(reg) &&
+         ordinary(reg / inv_h);
+}
+
+__device__ __forceinline__ Found scan_feature_estimated(const DirectLevel& a, const I64Pair& ns, int fb, int n_bins,
+                                                        double inv_g, double inv_h, double reg, int64_t up,
+                                                        int64_t down, const unsigned long long* s_bins)
+{
+  const int lane     = threadIdx.x & 63;
+  const double extra = reg / inv_h, all_g = static_cast<double>(ns.grad), all_h = static_cast<double>(ns.hess);
+  // grads lie in [-down, up] and up + down < 2^32: the lower 32 bits of grad + down are grad + down
+  const uint32_t down32  = static_cast<uint32_t>(down);
+  const double down_sums = static_cast<double>(down);
+  unsigned long long before = 0, left_1 = 0;
+  double last = -1.0, most = -1.0, second = -1.0;  // estimates: of the last bin so far, of this lane the two largest
+  int bin_1   = 0;
+  for (int base = 0; base < n_bins; base += 64) {
+    const int bin                = base + lane;
+    const bool in                = bin < n_bins;
+    const unsigned long long add = in ? s_bins[bin] : 0;
+    double estimate              = last;
+    unsigned long long left      = before;
+    if (__any(add != 0)) {
+      left += wave_inclusive_halves(add);
+      const double gl = static_cast<double>(static_cast<uint32_t>(left >> 32) + down32) - down_sums;
+      const double hl = static_cast<double>(static_cast<uint32_t>(left));
+      const double gr = all_g - gl, hr = all_h - hl;
+      const double pl = hl + extra, pr = hr + extra;
+      estimate = (gl * gl * pr + gr * gr * pl) * __builtin_amdgcn_rcp(pl * pr);
+      estimate = hl > 0 && hr > 0 ? estimate : -1.0;
+      before   = static_cast<unsigned long long>(wave_read_lane(static_cast<int64_t>(left), 63));
+      last     = wave_read_lane_f64(estimate, 63);
+    }
+    const bool more = in && estimate > most;
+    second = more ? most : (in && estimate > second ? estimate : second);
+    most   = more ? estimate : most;
+    left_1 = more ? left : left_1;
+    bin_1  = more ? bin : bin_1;
+  }
+  const double near = wave_max(most) * kNearBest;
+  if (near < 0) return Found{0.0, -1, 0};  // no valid split
+  if (__any(second >= near)) return scan_feature(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, s_bins);
+  const bool maybe = most >= near;
+  bool dead        = false;
+  double gain      = 0.0;
+  add_gain(gain, dead, unpack_sums(left_1, up, down), ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
+  Found best{0.0, -1, 0};
+  unsigned long long rest = __ballot(maybe && gain > 0);
+  while (rest != 0) {
+    const int from = __builtin_ctzll(rest);
+    rest &= rest - 1;
+    best.take(wave_read_lane_f64(gain, from), fb + __builtin_amdgcn_readlane(bin_1, from),
+              static_cast<unsigned long long>(wave_read_lane(static_cast<int64_t>(left_1), from)), true);
+  }
+  return best;
 }
 
 // The best split of each of the features [f0, f0 + nf) of node j from its histograms in the LDS.
 __device__ __forceinline__ void scan_features(const DirectLevel& a, int j, const I64Pair& ns, int f0, int nf, int width,
                                               const unsigned long long* s_hist)
 {
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int64_t root = a.node_sums[0].grad, all = (int64_t(1) << 31) + a.n_rows + 1024;
   const int64_t up = (all + root) / 2 + 1, down = (all - root) / 2 + 1;
   const double inv_g = a.scales[2], inv_h = a.scales[3];
   const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
-  for (int v = tid >> 6; v < nf; v += kDirectThreads / 64) {
+  const bool estimated = estimates_hold(a, inv_g, inv_h, reg);
+  for (int v = wave; v < nf; v += kDirectThreads / 64) {
     const int f    = f0 + v;
     const int64_t at = static_cast<int64_t>(j) * a.n_features + f;
     if (a.feature_set != nullptr && a.feature_set[f] == 0) {
@@ -82,41 +268,11 @@ __device__ __forceinline__ void scan_features(const DirectLevel& a, int j, const
       continue;
     }
     const int fb = a.row_pointers[f], n_bins = a.row_pointers[f + 1] - fb;
-    unsigned long long before = 0, best_left = 0;
-    double gain_before = 0.0;  // of the last bin so far: empty bins behind it have the same split
-    Cand best{0.0, -1};
-    for (int base = 0; base < n_bins; base += 64) {
-      const int bin                = base + lane;
-      const bool in                = bin < n_bins;
-      const unsigned long long add = in ? s_hist[v * width + bin] : 0;
-      double gain                  = gain_before;
-      unsigned long long left      = before;
-      if (__any(add != 0)) {
-        left += static_cast<unsigned long long>(wave_inclusive_sum(static_cast<int64_t>(add)));
-        const I64Pair ls = unpack_sums(left, up, down);
-        bool dead        = false;
-        gain             = 0.0;
-        add_gain(gain, dead, ls, ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
-        before      = static_cast<unsigned long long>(wave_read_lane(static_cast<int64_t>(left), 63));
-        gain_before = __longlong_as_double(wave_read_lane(__double_as_longlong(gain), 63));
-      }
-      const Cand c{gain, fb + bin};
-      if (in && gain > 0 && cand_better(c, best)) {
-        best      = c;
-        best_left = left;
-      }
-    }
-    for (int off = 32; off >= 1; off >>= 1) {
-      const Cand o{__shfl_xor(best.gain, off, 64), __shfl_xor(best.bin, off, 64)};
-      const unsigned long long o_left = __shfl_xor(best_left, off, 64);
-      if (cand_better(o, best)) {
-        best      = o;
-        best_left = o_left;
-      }
-    }
+    const Found best = estimated ? scan_feature_estimated(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, s_hist + v * width)
+                                 : scan_feature(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, s_hist + v * width);
     if (lane == 0) {
-      a.partial[at] = best;
-      a.left[at]    = unpack_sums(best_left, up, down);
+      a.partial[at] = Cand{best.gain, best.bin};
+      a.left[at]    = unpack_sums(best.left, up, down);
     }
   }
 }
@@ -157,10 +313,7 @@ __device__ __forceinline__ void add_range(const DirectLevel& a, int range, int p
     const int begin = a.seg[j], end = a.seg[j + 1];
     if (end - begin <= kDirectLarge || (side == 1 && (begin <= first || begin >= last))) continue;
     const Piece p = piece_of<BinT>(a, part);
-    for (int i = tid; i < p.nf * width; i += kDirectThreads) s_hist[i] = 0;
-    __syncthreads();
     add_rows<BinT>(a, p.rec, p.number, p.nf, max(first, begin), min(last, end), width, s_hist);
-    __syncthreads();
     // large nodes begin more than kDirectLarge positions apart: a slot each. Slots and counters are zero between nodes.
     const int64_t slot      = static_cast<int64_t>(begin / kDirectLarge) * pieces + part;
     unsigned long long* sum = a.large + slot * kPer * width;
@@ -210,10 +363,7 @@ __global__ void __launch_bounds__(kDirectThreads)
   const int begin = a.seg[j], end = a.seg[j + 1];
   if (ns.hess <= 0 || end - begin > kDirectLarge) return;
   const Piece p = piece_of<BinT>(a, (id >> 3) % pieces);
-  for (int i = threadIdx.x; i < p.nf * width; i += kDirectThreads) s_hist[i] = 0;
-  __syncthreads();
   add_rows<BinT>(a, p.rec, p.number, p.nf, begin, end, width, s_hist);
-  __syncthreads();
   scan_features(a, j, ns, p.f0, p.nf, width, s_hist);
 }
 

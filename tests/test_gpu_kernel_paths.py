@@ -673,3 +673,46 @@ def test_rounding_of_one_output(n):
     h[-1] = 1e-13
     gr, cr = gu.both(X, g, h, levels=True, max_depth=3, split_samples=32, seed=7)
     gu.assert_tree_parity(gr, cr, levels=True)
+
+
+# Levels without histograms in memory estimate the gains and form few of them exactly: against the oracle where many are
+# equal (columns of two values, copies of a column, plateaus of more than 64 empty bins), with penalties that rule the
+# estimate out, gains that a min_split_gain cuts off, and gradients whose squares nearly leave the doubles.
+@pytest.mark.parametrize("kind", ["copies", "two_values", "long_tails", "l1", "min_split_gain", "no_l2", "large_l2", "huge", "tiny", "one_sign"])
+def test_estimated_gains_choose_the_oracles_splits(kind):
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(len(kind))
+    n, f, s = 9001, 50, 512
+    X = rs.randn(n, f).astype(np.float32)
+    g, h = rs.randn(n, 1), 0.1 + rs.random_sample((n, 1))
+    kw = dict(max_depth=11, split_samples=s, seed=9)
+    if kind == "copies":
+        X[:, 1::2] = X[:, ::2]
+        X[:, 4] = -X[:, 0]
+    elif kind == "two_values":
+        X[:, ::3] = rs.randint(0, 2, X[:, ::3].shape)
+        g = np.sign(g)
+        h[:] = 1.0
+    elif kind == "long_tails":
+        X = np.exp(4 * X).astype(np.float32)
+        g[: n // 2] *= 1e-4
+    elif kind == "l1":
+        kw["l1_regularization"] = 2.0
+    elif kind == "min_split_gain":
+        kw["min_split_gain"] = 0.5
+    elif kind == "no_l2":
+        kw["l2_regularization"] = 0.0
+    elif kind == "large_l2":
+        kw["l2_regularization"] = 1e9
+        g *= 1e9
+    elif kind in ("huge", "tiny"):
+        g *= 1e150 if kind == "huge" else 1e-70
+        h *= 1e120 if kind == "huge" else 1e-65
+    elif kind == "one_sign":
+        g = np.abs(g)
+    Xd, gd, hd = (torch.from_numpy(a).cuda() for a in (X, g, h))
+    got = ops.build_tree(Xd, gd, hd, **kw)
+    names = {"l1_regularization": "l1", "l2_regularization": "l2"}
+    _assert_tree(got, orc.build_tree(X, g, h, **{names.get(k, k): v for k, v in kw.items()}))
