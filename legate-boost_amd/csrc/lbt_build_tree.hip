@@ -561,22 +561,10 @@ __global__ void __launch_bounds__(kThreads)
 // kW: waves that share a (node, feature), see scan_split_launch.
 constexpr int kFusedMaxK   = 64;  // lane k of the wave keeps the running sums of output k
 
-__device__ inline Cand wave_best(Cand c)
+__device__ __forceinline__ Cand wave_best(const Cand& c)  // the same in every lane
 {
-  for (int off = 32; off >= 1; off >>= 1) {
-    Cand o;
-    o.gain = __shfl_down(c.gain, off, 64);
-    o.bin  = __shfl_down(c.bin, off, 64);
-    if (cand_better(o, c)) c = o;
-  }
-  return c;  // valid on lane 0
-}
-
-// leaf_gain without branches (the lanes of a wave hold both signs), same results
-__device__ __forceinline__ double leaf_gain_select(double grad, double hess, double l1, double reg)
-{
-  const double z = grad > l1 ? grad - l1 : (grad < -l1 ? grad + l1 : 0.0);
-  return (z * z) / (hess + reg);
+  const int from = wave_best_lane(c.gain, c.bin);
+  return from < 0 ? Cand{0.0, -1} : Cand{wave_read_lane_f64(c.gain, from), __builtin_amdgcn_readlane(c.bin, from)};
 }
 
 template <int kW>

@@ -5,6 +5,8 @@
 
 #include "lbt_internal.h"
 
+#include <type_traits>
+
 namespace lbt {
 
 template <typename T>
@@ -126,6 +128,59 @@ __device__ __forceinline__ int wave_inclusive_sum32(int v)
   v += dpp_take32<0x142, 0xa>(v);
   v += dpp_take32<0x143, 0xc>(v);
   return v;
+}
+
+// Largest value of a wave, in every lane, in the lanes' own data paths (see wave_inclusive_sum): a maximum of gains by LDS
+// permutes is 18 of them one after the other, here 12 operations and more for the ties.
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v)
+{
+  auto take = [&](auto ctrl, auto rows) {
+    const unsigned o = static_cast<unsigned>(__builtin_amdgcn_update_dpp(
+      0, static_cast<int>(v), decltype(ctrl)::value, decltype(rows)::value, 0xf, true));
+    v = o > v ? o : v;
+  };
+  using std::integral_constant;
+  take(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});
+  take(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
+  take(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
+  take(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
+  take(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});
+  take(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});
+  return static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
+}
+
+// The lane that holds the best of a wave's candidates (gain, bin) in the order of cand_better; -1: there is none.
+// Candidates have bin >= 0 and a positive gain.
+__device__ __forceinline__ int wave_best_lane(double gain, int bin)
+{
+  const unsigned own_hi = bin >= 0 ? static_cast<unsigned>(__double_as_longlong(gain) >> 32) : 0u;
+  const unsigned own_lo = static_cast<unsigned>(__double_as_longlong(gain)), own_rank = static_cast<unsigned>(bin & 511) + 1u;
+  const unsigned hi = wave_max_u32(own_hi);
+  const unsigned lo = wave_max_u32(bin >= 0 && own_hi == hi ? own_lo : 0u);
+  const bool holds  = bin >= 0 && own_hi == hi && own_lo == lo;
+  const unsigned rank = wave_max_u32(holds ? own_rank : 0u);
+  const unsigned low  = wave_max_u32(holds && own_rank == rank ? ~static_cast<unsigned>(bin) : 0u);
+  const unsigned long long who = __ballot(holds && ~static_cast<unsigned>(bin) == low);
+  return who != 0 ? __builtin_ctzll(who) : -1;
+}
+
+// The largest gain of a wave and, of the lanes that hold it, the largest key.
+__device__ __forceinline__ void wave_best_key(double& best, unsigned& key)
+{
+  // gains are not negative: their bits compare as whole numbers, upper halves first
+  const unsigned own_hi = static_cast<unsigned>(__double_as_longlong(best) >> 32);
+  const unsigned own_lo = static_cast<unsigned>(__double_as_longlong(best));
+  const unsigned hi = wave_max_u32(own_hi);
+  const unsigned lo = wave_max_u32(own_hi == hi ? own_lo : 0u);
+  key  = wave_max_u32(own_hi == hi && own_lo == lo ? key : 0u);
+  best = __longlong_as_double(static_cast<int64_t>(static_cast<unsigned long long>(hi) << 32 | lo));
+}
+
+// leaf_gain without branches (the lanes of a wave hold both signs), same results
+__device__ __forceinline__ double leaf_gain_select(double grad, double hess, double l1, double reg)
+{
+  const double z = grad > l1 ? grad - l1 : (grad < -l1 ? grad + l1 : 0.0);
+  return (z * z) / (hess + reg);
 }
 
 // Sum of the threads before this one; all threads of the workgroup call it. s_wave: one int per wave.

@@ -124,6 +124,14 @@ struct Found {
     bin  = better ? o_bin : bin;
     left = better ? o_left : left;
   }
+  // the best of a wave's, the same in every lane
+  __device__ __forceinline__ Found of_wave() const
+  {
+    const int from = wave_best_lane(gain, bin);
+    if (from < 0) return Found{0.0, -1, 0};
+    return Found{wave_read_lane_f64(gain, from), __builtin_amdgcn_readlane(bin, from),
+                 static_cast<unsigned long long>(wave_read_lane(static_cast<int64_t>(left), from))};
+  }
 };
 
 // The best split of one feature, by one wave: every bin's gain as the split evaluation defines it.
@@ -152,9 +160,7 @@ __device__ __forceinline__ Found scan_feature(const DirectLevel& a, const I64Pai
     }
     best.take(gain, fb + bin, left, in & (gain > 0));
   }
-  for (int off = 32; off >= 1; off >>= 1)
-    best.take(__shfl_xor(best.gain, off, 64), __shfl_xor(best.bin, off, 64), __shfl_xor(best.left, off, 64), true);
-  return best;
+  return best.of_wave();
 }
 
 // Largest value of a wave, in every lane; values are not negative zero and not NaN
@@ -239,15 +245,7 @@ __device__ __forceinline__ Found scan_feature_estimated(const DirectLevel& a, co
   bool dead        = false;
   double gain      = 0.0;
   add_gain(gain, dead, unpack_sums(left_1, up, down), ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
-  Found best{0.0, -1, 0};
-  unsigned long long rest = __ballot(maybe && gain > 0);
-  while (rest != 0) {
-    const int from = __builtin_ctzll(rest);
-    rest &= rest - 1;
-    best.take(wave_read_lane_f64(gain, from), fb + __builtin_amdgcn_readlane(bin_1, from),
-              static_cast<unsigned long long>(wave_read_lane(static_cast<int64_t>(left_1), from)), true);
-  }
-  return best;
+  return Found{gain, maybe && gain > 0 ? fb + bin_1 : -1, left_1}.of_wave();
 }
 
 // The best split of each of the features [f0, f0 + nf) of node j from its histograms in the LDS.

@@ -716,3 +716,20 @@ def test_estimated_gains_choose_the_oracles_splits(kind):
     got = ops.build_tree(Xd, gd, hd, **kw)
     names = {"l1_regularization": "l1", "l2_regularization": "l2"}
     _assert_tree(got, orc.build_tree(X, g, h, **{names.get(k, k): v for k, v in kw.items()}))
+
+
+# The best of a wave's candidates where many gains are equal: the order of ties is the oracle's. Copies of columns,
+# columns of two values, long runs of empty bins; one wave per node and fewer lanes (more than 16 nodes).
+@pytest.mark.parametrize("n,f,k,s,depth", [(20001, 40, 1, 256, 7), (20001, 130, 1, 64, 5), (12001, 20, 3, 300, 6)])
+def test_ties_of_medium_sizes(n, f, k, s, depth):
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(f)
+    X = rs.randn(n, f).astype(np.float32)
+    X[:, 1::2] = X[:, ::2]
+    X[:, ::5] = rs.randint(0, 2, X[:, ::5].shape)
+    g, h = np.sign(rs.randn(n, k)), np.ones((n, k))
+    kw = dict(max_depth=depth, split_samples=s, seed=4)
+    got = ops.build_tree(*(torch.from_numpy(a).cuda() for a in (X, g, h)), **kw)
+    _assert_tree(got, orc.build_tree(X, g, h, **kw))
