@@ -176,6 +176,20 @@ __device__ __forceinline__ void wave_best_key(double& best, unsigned& key)
   best = __longlong_as_double(static_cast<int64_t>(static_cast<unsigned long long>(hi) << 32 | lo));
 }
 
+// The same with what belongs to the gain: its feature and the bin in it. Keys of different candidates differ.
+__device__ __forceinline__ void wave_best_split(double& gain, unsigned& key, int& ft, int& rel)
+{
+  const double own_gain  = gain;
+  const unsigned own_key = key;
+  wave_best_key(gain, key);
+  const unsigned long long who = __ballot(key != 0 && own_key == key && own_gain == gain);
+  if (who != 0) {
+    const int from = __builtin_ctzll(who);
+    ft  = __builtin_amdgcn_readlane(ft, from);
+    rel = __builtin_amdgcn_readlane(rel, from);
+  }
+}
+
 // leaf_gain without branches (the lanes of a wave hold both signs), same results
 __device__ __forceinline__ double leaf_gain_select(double grad, double hess, double l1, double reg)
 {

@@ -636,17 +636,7 @@ __device__ __forceinline__ int2 decide_node(const MidArgs& a, const MidTreeState
       take(o.gain, o.key, i, o.rel);
     }
   }
-  if (lanes == 64) {
-    const unsigned own = key;
-    const double mine  = best;
-    wave_best_key(best, key);
-    const unsigned long long who = __ballot(key != 0 && own == key && mine == best);
-    if (who != 0) {
-      const int from = __builtin_ctzll(who);
-      ft  = __builtin_amdgcn_readlane(ft, from);
-      rel = __builtin_amdgcn_readlane(rel, from);
-    }
-  }
+  if (lanes == 64) wave_best_split(best, key, ft, rel);
   for (int off = lanes == 64 ? 0 : lanes >> 1; off >= 1; off >>= 1) {
     const double g   = __shfl_xor(best, off, 64);
     const unsigned o = static_cast<unsigned>(__shfl_xor(static_cast<int>(key), off, 64));

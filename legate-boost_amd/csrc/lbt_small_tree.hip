@@ -628,16 +628,12 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     const unsigned long long have = __ballot(first_key != 0 || cur_key != 0);
     bool alone = true;
     if (have != 0) {
-      const int wave_node = __shfl(first_node, __ffsll(have) - 1, 64);
+      const int wave_node = __builtin_amdgcn_readlane(first_node, __builtin_ctzll(have));
       alone               = !__all(cur_key == 0 && (first_key == 0 || first_node == wave_node));
       if (!alone) {
-        double top = first_key != 0 ? first_gain : 0.0;
-        for (int off = 32; off >= 1; off >>= 1) {
-          const double o = __shfl_xor(top, off, 64);
-          top            = o > top ? o : top;
-        }
-        unsigned key = first_key != 0 && first_gain == top ? first_key : 0u;
-        for (int off = 32; off >= 1; off >>= 1) key = max(key, static_cast<unsigned>(__shfl_xor(static_cast<int>(key), off, 64)));
+        double top   = first_key != 0 ? first_gain : 0.0;
+        unsigned key = first_key;
+        wave_best_key(top, key);
         first_node = wave_node;
         first_gain = top;
         first_key  = lane == 0 ? key : 0u;
@@ -787,12 +783,7 @@ __global__ void __launch_bounds__(kT)
     const SmallCand o = c[i];
     take(o.gain, o.key, i, o.rel);
   }
-  for (int off = 32; off >= 1; off >>= 1) {
-    const double g   = __shfl_xor(best, off, 64);
-    const unsigned k = static_cast<unsigned>(__shfl_xor(static_cast<int>(best_key), off, 64));
-    const int f_o = __shfl_xor(ft, off, 64), r_o = __shfl_xor(rel, off, 64);
-    take(g, k, f_o, r_o);
-  }
+  wave_best_split(best, best_key, ft, rel);
   if (kT > 64) {
     if (lane == 0) {
       s_best[wave] = best;
