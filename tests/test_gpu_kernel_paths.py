@@ -733,3 +733,16 @@ def test_ties_of_medium_sizes(n, f, k, s, depth):
     kw = dict(max_depth=depth, split_samples=s, seed=4)
     got = ops.build_tree(*(torch.from_numpy(a).cuda() for a in (X, g, h)), **kw)
     _assert_tree(got, orc.build_tree(X, g, h, **kw))
+
+
+# Rows of a level find their sides in runs of eight positions a thread (up to 8 nodes and from 128 on) or in positions
+# apart: ragged ends, slabs that end inside a run, nodes that change inside one, bins of one and of two bytes.
+@pytest.mark.parametrize("n,s,depth", [(7, 8, 3), (2047, 64, 9), (2052, 300, 9), (6145, 256, 9), (20003, 400, 8)])
+def test_sides_of_a_levels_rows(n, s, depth):
+    import gpu_util as gu
+
+    rs = np.random.RandomState(n)
+    X = rs.randn(n, 6).astype(np.float32)
+    g, h = rs.randn(n, 1), rs.rand(n, 1) + 0.1
+    gr, cr = gu.both(X, g, h, levels=True, max_depth=depth, split_samples=s, seed=2)
+    gu.assert_tree_parity(gr, cr, levels=True)
