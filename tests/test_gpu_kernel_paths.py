@@ -746,3 +746,15 @@ def test_sides_of_a_levels_rows(n, s, depth):
     g, h = rs.randn(n, 1), rs.rand(n, 1) + 0.1
     gr, cr = gu.both(X, g, h, levels=True, max_depth=depth, split_samples=s, seed=2)
     gu.assert_tree_parity(gr, cr, levels=True)
+
+
+# The bin counts reach the host from a kernel up to 4096 features and by a copy beyond.
+@pytest.mark.parametrize("f", [4095, 4096, 4097])
+def test_bin_counts_for_the_host(f):
+    import gpu_util as gu
+
+    rs = np.random.RandomState(f)
+    X = rs.randint(0, 9, (9000, f)).astype(np.float32)
+    g, h = rs.randn(9000, 1), rs.rand(9000, 1) + 0.5
+    gr, cr = gu.both(X, g, h, levels=True, max_depth=2, split_samples=8, seed=1)
+    gu.assert_tree_parity(gr, cr, levels=True)
