@@ -428,7 +428,7 @@ def bench_predict(args, steps=None, warmup=None, light=False):
         return {"workload": "cfg5: PredictTask, 1000 trees of depth 8, X %dx64 f32, out f64" % rows,
                 "value": rows * steps / dt, "unit": "rows/s", "steps": steps, "warmup": max(1, warmup),
                 "ms_per_step": dt / steps * 1e3, "node_steps_per_s": rows * 8000 * steps / dt,
-                "roofline": {"kernel": "predict_tile_kernel", "bound": "hbm", "frac": achieved / HBM_PEAK_GBS,
+                "roofline": {"kernel": "walk_ranked_kernel", "bound": "hbm", "frac": achieved / HBM_PEAK_GBS,
                              "limited_by": "lds"}}
     out = {
         "metric": "PredictTask rows/s, 1000 trees depth 8, 20M×64",
@@ -440,18 +440,16 @@ def bench_predict(args, steps=None, warmup=None, light=False):
                    "rows": rows, "trees": 1000, "row_trees_per_s": rows * 1000 * steps / dt,
                    "node_steps_per_s": rows * 8000 * steps / dt},
         # X read once and the output written once are all the HBM bytes this path needs (achieved /
-        # peak / frac price those); what bounds the kernel is the LDS: every node step of a wave
-        # is two LDS reads (node, feature value), which the counters put at 8.2 cycles each
-        # (4.2 of issue, 3.4 of bank conflicts; profiles/predict_tile_kernel_cfg5_*.txt), 17 of
-        # the 17.5 cycles a CU spends per wave-level node step
+        # peak / frac price those); what bounds the walk is the LDS and the vector units, both busy for two
+        # thirds of it: every node step of a wave is two LDS reads (node, rank of the feature's value) and
+        # four vector instructions (profiles/predict_ranked_cfg5_*.txt)
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": None, "kernel": "predict_tile_kernel",
+                     "frac": achieved / HBM_PEAK_GBS, "traffic": None, "kernel": "walk_ranked_kernel",
                      "limited_by": "lds",
                      "lds": {"wave_level_node_steps": rows * 8000 / 64,
                              "cycles_per_wave_level_node_step_and_cu":
                                  dt / steps * 2.4e9 / (rows * 8000 / 64 / 256),
-                             "lds_reads_per_node_step": 2.1, "lds_cycles_per_read_measured": 8.2,
-                             "clock_assumed_GHz": 2.4}},
+                             "lds_reads_per_node_step": 2.0, "clock_assumed_GHz": 2.4}},
     }
     if not args.no_cpu_baseline and not args.only_timed:
         cores = max(1, min(16, os.cpu_count() or 1))

@@ -198,13 +198,13 @@ T* dense_out(legate::PhysicalStore store)
     split.push_back(dense_in<double, 1>(context.input(i + 2).data(), &ss));
     nodes.push_back(static_cast<int32_t>(fs.hi[0] - fs.lo[0] + 1));
   }
-  // scratch for the packed ensemble (the task class gains with_has_allocations(true))
-  int64_t total_nodes = 0;
-  for (int32_t n : nodes) total_nodes += n;
-  const size_t ws_bytes =
-    lbt_predict_workspace_bytes(static_cast<int>(leaf.size()), total_nodes, outputs, dtype);
+  // scratch for the packed ensemble and, where that is faster, the rows' ranks (the task class gains
+  // with_has_allocations(true))
+  const int features    = static_cast<int>(xs.hi[1] - xs.lo[1] + 1);
+  const size_t ws_bytes = lbt_predict_rows_workspace_bytes(rows, features, static_cast<int>(leaf.size()), nodes.data(),
+                                                           outputs, dtype);
   auto workspace = legate::create_buffer<int8_t>(ws_bytes, legate::Memory::GPU_FB_MEM, 256);
-  check(lbt_predict(context.get_task_stream(), X, dtype, rows, static_cast<int>(xs.hi[1] - xs.lo[1] + 1),
+  check(lbt_predict(context.get_task_stream(), X, dtype, rows, features,
                     static_cast<int>(leaf.size()), leaf.data(), feature.data(), split.data(), nodes.data(), outputs,
                     out, workspace.ptr(0), ws_bytes));
   // lbt_predict only enqueues; the kernels still read the workspace when this function returns.
