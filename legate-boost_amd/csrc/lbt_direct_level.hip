@@ -11,10 +11,10 @@
 // its few workgroups then were the whole level (1,000,000 x 50 with 512 samples, depth 12, noise: 3.55 ms a tree, where
 // histograms in memory took 2.55; 2,000,000 x 80, depth 11 3.93 and 2.14). So the rows of a node of more than 16384 are
 // dealt to workgroups by ranges of 8192 positions; each adds its sums to the node's histogram in memory, and the
-// last one to finish scans it: 2.07 and 2.24 ms, and 1.95 as before where the tree is balanced. It needs 8 bytes
-// per bin and 16384 rows, in the room of the histograms that are not kept. Shorter ranges add more often (4096: 2.56 and
-// 2.53 ms), longer ones leave nodes that fit none to one workgroup (16384: 2.01 and 2.13, but 250,000 x 43 1.36
-// where 8192 takes 1.20).
+// last one to finish scans it: 2.07 and 2.24 ms, and 1.95 as before where the tree is balanced (1.97, 2.16 and 1.62 with
+// the estimates below). It needs 8 bytes per bin and 16384 rows, in the room of the histograms that are not kept.
+// Shorter ranges add more often (4096: 2.56 and 2.53 ms), longer ones leave nodes that fit none to one workgroup
+// (16384: 2.01 and 2.13, but 250,000 x 43 1.36 where 8192 takes 1.20).
 //
 // Only where every rounded hessian is positive: a scanned histogram is then the running sums everywhere
 // (build_tree.cu:645 leaves nothing unscanned) and it does not matter that nothing is derived by subtraction.
