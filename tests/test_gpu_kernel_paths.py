@@ -758,3 +758,15 @@ def test_bin_counts_for_the_host(f):
     g, h = rs.randn(9000, 1), rs.rand(9000, 1) + 0.5
     gr, cr = gu.both(X, g, h, levels=True, max_depth=2, split_samples=8, seed=1)
     gu.assert_tree_parity(gr, cr, levels=True)
+
+
+# The tile plan of a level: one node a thread (up to 256) and several, nodes without rows, tiles that end inside one.
+@pytest.mark.parametrize("n,depth,hist_cache_bytes", [(3, 2, 0), (5000, 9, 0), (20001, 10, 0), (9001, 10, 200_000)])
+def test_tile_plans(n, depth, hist_cache_bytes):
+    import gpu_util as gu
+
+    rs = np.random.RandomState(n)
+    X = rs.randn(n, 4).astype(np.float32)
+    g, h = rs.randn(n, 1), rs.rand(n, 1) + 0.1
+    gr, cr = gu.both(X, g, h, levels=True, max_depth=depth, split_samples=33, seed=6, hist_cache_bytes=hist_cache_bytes)
+    gu.assert_tree_parity(gr, cr, levels=True)
