@@ -43,7 +43,7 @@ struct PackRefs {
 
 struct RankState {
   int depth, F, K, n_trees;  // n_trees: padded to whole chunks
-  int32_t* count;       // [F] thresholds of a feature
+  int32_t* count;       // [F] thresholds of a feature; [F] not 0 where a node on the feature has NaN as its threshold
   int32_t* offset;      // [F + 1]
   int32_t* overflow;    // one word: a feature has more thresholds than ranks
   uint32_t* slot;       // [n_trees << depth] place among the thresholds of the node's feature, or a marker
@@ -110,9 +110,12 @@ __global__ void __launch_bounds__(kThreads) rank_pack_kernel(PackRefs refs, int 
       else
         thr = d;
       node_feature[u] = ft;
-      if (thr == thr) {  // a comparison with NaN is never true: rank 0, below every value's
+      if (thr == thr) {
         slot[u] = kLocal ? atomicAdd(&s_count[ft], 1) : atomicAdd(&st.count[ft], 1);
         raw[at] = thr;
+      } else {
+        // a comparison with NaN is never true: rank 0, below every value's; the feature then needs ranks, whatever they are
+        st.count[st.F + ft] = 1;
       }
     }
     const int stop = ends_leaf != 0 ? __ffs(ends_leaf) - 1 : st.depth;
@@ -321,7 +324,11 @@ __global__ void __launch_bounds__(kWalkThreads)
   const int64_t split = blockIdx.x % 8 + 8 * static_cast<int64_t>(local / a.n_groups);
   const int f0 = g * kAll, nf = min(kAll, a.F - f0);
   const int first = st.offset[f0], words = st.offset[f0 + nf] - first;
-  if (words == 0) return;  // no tree asks for these features
+  if (words == 0) {
+    bool asked = false;
+    for (int i = 0; i < nf; i++) asked |= st.count[a.F + f0 + i] != 0;
+    if (!asked) return;  // no tree asks for these features
+  }
   T* const s_tab    = reinterpret_cast<T*>(smem_raw);
   uint16_t* s_start = reinterpret_cast<uint16_t*>(smem_raw + a.lds_bytes - 2 * kAll * a.cells);  // [kAll][cells]
   const bool held   = (words + 1) * static_cast<int>(sizeof(T)) + 2 * kAll * a.cells <= a.lds_bytes;
@@ -849,7 +856,7 @@ struct Layout {
     st.F       = F;
     st.K       = K;
     st.n_trees = p.padded_trees;
-    st.count    = ar.take<int32_t>(F);
+    st.count    = ar.take<int32_t>(2 * static_cast<int64_t>(F));
     st.offset   = ar.take<int32_t>(F + 1);
     st.overflow = ar.take<int32_t>(1);
     st.slot     = ar.take<uint32_t>(p.slots);
@@ -891,7 +898,7 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
   Layout<T> lay(workspace, p, F, K);
   RankState& st = lay.st;
   ProfScope ps(LBT_PROF_PREDICT, stream, static_cast<double>(N) * (static_cast<double>(F) * sizeof(T) + K * 8.0));
-  zero_counts_kernel<<<ceil_div(F, kThreads), kThreads, 0, stream>>>(st.count, F);
+  zero_counts_kernel<<<ceil_div(2 * F, kThreads), kThreads, 0, stream>>>(st.count, 2 * F);
   for (int first = 0; first < p.padded_trees; first += kPackTrees) {
     PackRefs refs{};
     const int all  = std::min(kPackTrees, p.padded_trees - first);

@@ -81,6 +81,31 @@ def test_thresholds_that_crowd_one_feature(n_trees, share, dtype):
     assert torch.equal(ops.predict(X, trees, 1), ops.predict(X, trees, 1, tiled=False))
 
 
+@pytest.mark.parametrize("n,f,n_trees,depth,nan_from", [
+    (700_001, 40, 200, 8, 32),  # the last features have NaN thresholds only
+    (600_011, 9, 200, 8, 8),
+    (3_000_003, 1, 120, 3, 0),  # and here there are no others at all
+])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_nan_thresholds_on_features_without_others(n, f, n_trees, depth, nan_from, dtype):
+    """No value is <= NaN, so every row steps to the right there, whatever the workspace held before."""
+    rs = np.random.RandomState(f)
+    trees = _ensemble(rs, n_trees, depth, f, 1, dtype, 0)
+    for t in trees:
+        t[2][t[1] >= nan_from] = float("nan")
+    X = _rows(rs, n, f, dtype, 0)
+    assert _takes_ranks(X, trees, 1)
+    want = ops.predict(X, trees, 1, tiled=False)
+    for byte in (0, 255):
+        leaf_p, feat_p, split_p, nodes, _, keep = ops._tree_arrays(trees, 1)
+        nbytes = _lib.lib.lbt_predict_rows_workspace_bytes(n, f, n_trees, nodes, 1, ops._DT[X.dtype])
+        ws = torch.full((nbytes,), byte, dtype=torch.uint8, device="cuda")
+        out = torch.empty((n, 1), dtype=torch.float64, device="cuda")
+        _lib.check(_lib.lib.lbt_predict(ops._stream(), X.data_ptr(), ops._DT[X.dtype], n, f, n_trees, leaf_p, feat_p, split_p,
+                                        nodes, 1, out.data_ptr(), ws.data_ptr(), nbytes))
+        assert torch.equal(out, want)
+
+
 def test_a_start_off_a_16_byte_boundary():
     rs = np.random.RandomState(5)
     trees = _ensemble(rs, 130, 6, 8, 1, np.float32, 0)
