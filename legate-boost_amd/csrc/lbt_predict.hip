@@ -714,6 +714,11 @@ int pack_tiled(hipStream_t stream, int F, int n_trees, const double* const* leaf
   return LBT_OK;
 }
 
+// Whether the tile kernel with 16 lanes per row has room for the values of a batch beside rows and nodes.
+constexpr size_t kBatchValues = static_cast<size_t>(TileShape<16>::kBatchTrees) * TileShape<16>::kRows * sizeof(double);
+size_t values_offset(const lbt_packed_ensemble& ens) { return (static_cast<size_t>(ens.lds_bytes) + 15) & ~size_t(15); }
+bool values_through_lds(const lbt_packed_ensemble& ens) { return ens.n_outputs == 1 && values_offset(ens) + kBatchValues <= kTileLds; }
+
 // The kernel for few rows over a packed ensemble; *done stays false where the tile kernel is the faster one or the shapes
 // do not fit.
 template <typename T>
@@ -733,7 +738,17 @@ int run_few(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble
   const int64_t cap_words = std::min<int64_t>({room, all_words, static_cast<int64_t>(kFewWords) * kTileThreads});
   const size_t tile_rows  = kTileThreads / ens.lanes;
   const size_t tile_x     = (tile_rows * pitch * sizeof(T) + 15) & ~size_t(15);  // lds_bytes: that and the widest batch
-  if (static_cast<int64_t>(static_cast<size_t>(ens.lds_bytes) - tile_x) / 16 > cap_words + 1 && cap_words < all_words) return LBT_OK;
+  const int64_t widest    = static_cast<int64_t>(static_cast<size_t>(ens.lds_bytes) - tile_x) / 16 - 1;
+  if (widest > cap_words && cap_words < all_words) return LBT_OK;
+  // Turns of one batch (of deep trees): most lanes have no tree, and a workgroup copies the ensemble for 16 rows where one of the
+  // tile kernel with 16 lanes per row does for 64. Where that one passes values through the LDS as well it is the faster one, and
+  // with several outputs below eight trees a batch. Tile kernel and this one, 256 rows, us: 1000 trees of depth 8 on
+  // 32 features 124.8 : 163.9, on 10 f64 284 : 322, 300 of depth 8 38.9 : 46.3, 100 of depth 10 45.3 : 56.3; 88 of depth 9
+  // on 15 f64 with 8 outputs 56.9 : 66.4. Without values through the LDS: 1000 of depth 8 on 160 features 196 : 170, 300 of
+  // depth 8 on 32 f64 130 : 104, with 3 outputs and 20 trees a batch 72.4 : 46.5. Two batches a turn: 300 of depth 7 on 100
+  // features 31.3 : 22.4.
+  const bool one_batch = 2 * widest > cap_words && cap_words < all_words;
+  if (one_batch && (values_through_lds(ens) || (K > 1 && ens.n_trees < 8 * ens.n_batches))) return LBT_OK;
   PackedLayout<T> lay(ens.data, ens.n_trees, ens.total_nodes);
   const int node_at  = static_cast<int>(x_bytes);
   const int value_at = static_cast<int>(x_bytes + cap_words * 16);
@@ -775,11 +790,9 @@ int run_tiled(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemb
   // chunk (each chunk's sums are formed in tree order, as in one walk).
   const int own   = K == 1 ? 0 : (K <= lanes ? 1 : 2);
   const int chunk = K == 1 ? 1 : lanes * own;
-  const size_t values  = static_cast<size_t>(TileShape<16>::kBatchTrees) * TileShape<16>::kRows * sizeof(double);
-  const size_t shared  = (static_cast<size_t>(ens.lds_bytes) + 15) & ~size_t(15);
-  const bool by_values = K == 1 && lanes == 16 && tiles <= kSmallRunGroups && shared + values <= kTileLds;
-  const int value_off  = by_values ? static_cast<int>(shared) : 0;
-  const size_t lds     = by_values ? shared + values : static_cast<size_t>(ens.lds_bytes);
+  const bool by_values = lanes == 16 && tiles <= kSmallRunGroups && values_through_lds(ens);
+  const int value_off  = by_values ? static_cast<int>(values_offset(ens)) : 0;
+  const size_t lds     = by_values ? values_offset(ens) + kBatchValues : static_cast<size_t>(ens.lds_bytes);
   auto launch = [&](auto kernel, std::atomic<bool> (&flags)[kMaxDevices]) -> int {
     LBT_TRY(allow_dynamic_lds(kernel, kTileLds, flags));
     for (int k0 = 0; k0 < K; k0 += chunk)

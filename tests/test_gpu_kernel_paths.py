@@ -564,7 +564,10 @@ def test_predict_takes_more_lanes_per_row_for_few_rows(f, k, n_trees, dtype):
 
 @pytest.mark.parametrize("f,k,n_trees,depth,dtype", [(13, 1, 17, 3, np.float32), (13, 1, 129, 6, np.float32), (160, 1, 300, 8, np.float64),
                                                      (7, 64, 40, 4, np.float32), (7, 65, 40, 4, np.float32), (300, 5, 33, 8, np.float64),
-                                                     (31, 8, 1000, 3, np.float32)])
+                                                     (31, 8, 1000, 3, np.float32),
+                                                     # turns of one batch and of two, several outputs with few trees a batch and with more
+                                                     (32, 1, 150, 8, np.float32), (100, 1, 117, 7, np.float32), (10, 1, 60, 8, np.float64),
+                                                     (12, 8, 34, 9, np.float64), (22, 2, 60, 8, np.float32)])
 def test_predict_of_few_rows(f, k, n_trees, depth, dtype):
     """Up to 4096 rows and more than 16 trees: rows around a workgroup's 16, trees around the 128 of a turn, outputs around the 64 that
     its threads add, ensembles of one and of many turns: equal to the per-node kernel."""
