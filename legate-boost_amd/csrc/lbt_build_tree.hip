@@ -1098,12 +1098,20 @@ __global__ void __launch_bounds__(kThreads)
   store_block_counts(nd, nl, s_d, s_l, block_counts);
 }
 
-// Runs of positions where the rows of a node are either dense, so that a thread's eight bins and its neighbours' share
-// cache lines, or so sparse that every bin is a line of its own anyway. In between a wave that takes 64 positions side by
-// side touches fewer lines at a time. Runs against positions apart, us a level: 10,000,000 x 100, 1 to 8 nodes 22 : 33,
-// 18 : 31, 20 : 32, 26 : 32, 16 to 64 nodes 37 : 36, 57 : 49, 68 : 65; 2,000,000 x 200 from 16 nodes on 14 : 13, 18 : 16,
-// 26 : 22; 1,000,000 x 50 with 512 samples, 128 to 1024 nodes 12 : 15, 12.5 : 15, 14 : 15, 14 : 17.
-constexpr bool classify_in_runs(int n_nodes) { return n_nodes <= 8 || n_nodes >= 128; }
+// Runs of positions cost fewer instructions and segment look-ups, which is what counts while the launch is a chain of
+// latencies: up to a million rows, at all levels, and near the root, where a thread's eight bins and its neighbours' share cache
+// lines. With more rows and nodes the launch is bound by the lines it asks for, and a wave that takes 64 positions side by
+// side asks for those that lie close together. Runs against positions apart, us for 1, 4, 8, 32, 128 and 512 nodes:
+//   400,000 x 60          4.8 : 7.7   4.8 : 6.5   5.5 : 6.9   6.2 : 7.7   7.0 : 8.8   8.7 : 9.9
+//   1,000,000 x 50        5.4 : 8.9   5.6 : 7.6   6.8 : 7.5   8.9 : 9.2   9.8 : 11.2  12.2 : 14.3
+//   1,400,000 x 60        6.2 : 9.1   6.0 : 7.7   7.9 : 8.0  10.6 : 9.7  12.1 : 12.4  17.8 : 19.3
+//   2,000,000 x 100       7.8 : 10.4  6.8 : 8.3   8.8 : 8.6  13.6 : 11.4 16.2 : 15.7
+//   4,000,000 x 100      11.6 : 13.4 10.8 : 10.9 14.3 : 11.8 23.2 : 19.0 32.4 : 30.7
+//   10,000,000 x 100     22.3 : 30.6 22.2 : 28.2 31.7 : 31.1 53.6 : 48.2 87.4 : 82.8
+//   100,000,000 x 4       125 : 208   159 : 222   260 : 263   570 : 478   974 : 897
+// Apart at 128 nodes or more with 100,000 x 32 (columns that one L2 holds): 8.7 : 8.4, 10.2 : 9.4 at 512.
+constexpr int64_t kRunsAlways = int64_t(1) << 20;
+constexpr bool classify_in_runs(int n_nodes, int64_t n_rows) { return n_nodes <= 4 || n_rows <= kRunsAlways; }
 
 // Leaf of every row that is still in a node after the last level: the node itself if it
 // did not split, else the child the row falls into.
@@ -2144,7 +2152,7 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
         kernel<<<nb, kThreads, 0, stream>>>(rows, N, seg, bseg, n_parents, level_first, bins, L.bins_t_stride, feature,
                                             L.split_bin, L.code, L.block_counts);
       };
-      const bool runs = classify_in_runs(n_parents);
+      const bool runs = classify_in_runs(n_parents, N);
       if (use_bins_t && hs.bin_bytes == 1)
         classify_bins(runs ? classify_bins_kernel<uint8_t, true> : classify_bins_kernel<uint8_t, false>,
                       static_cast<const uint8_t*>(L.bins_t));

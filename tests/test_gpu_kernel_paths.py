@@ -738,9 +738,10 @@ def test_ties_of_medium_sizes(n, f, k, s, depth):
     _assert_tree(got, orc.build_tree(X, g, h, **kw))
 
 
-# Rows of a level find their sides in runs of eight positions a thread (up to 8 nodes and from 128 on) or in positions
+# Rows of a level find their sides in runs of eight positions a thread (up to 2^20 rows, or 4 nodes) or in positions
 # apart: ragged ends, slabs that end inside a run, nodes that change inside one, bins of one and of two bytes.
-@pytest.mark.parametrize("n,s,depth", [(7, 8, 3), (2047, 64, 9), (2052, 300, 9), (6145, 256, 9), (20003, 400, 8)])
+@pytest.mark.parametrize("n,s,depth", [(7, 8, 3), (2047, 64, 9), (2052, 300, 9), (6145, 256, 9), (20003, 400, 8),
+                                       (1 << 20, 40, 5), ((1 << 20) + 5, 40, 5), ((1 << 20) + 2047, 300, 4)])
 def test_sides_of_a_levels_rows(n, s, depth):
     import gpu_util as gu
 
