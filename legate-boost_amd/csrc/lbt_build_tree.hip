@@ -763,10 +763,12 @@ __global__ void __launch_bounds__(kW == 1 ? kThreads : kW * 64)
 }
 
 // Up to 512 (node, feature) pairs a workgroup shares a pair's tiles, a wave each for up to eight of them: such
-// levels leave most of the chip idle, and a wave's tiles are a chain (us, eight against one wave, 1,000,000 x 50 with
-// 512 samples: 50 pairs 8 : 10, 200 9.5 : 13, 400 11.5 : 13.4, 800 17 : 14; four against one, 2,000,000 x 200 with
-// 8 outputs: 200 pairs 15 : 23, 400 22 : 34, 800 31 : 34, 1600 46 : 37). More pairs fill it with one wave each, and
-// the first reading of the shared form, for the tiles' sums, is then work on top.
+// levels leave most of the chip idle, and a wave's tiles are a chain (us, eight against one wave, 300,000 x 50 with
+// 512 samples: 50 pairs 6.6 : 8.4, 200 8.2 : 12.7, 400 10.9 : 12.0, 800 15.2 : 12.6; four against one with 256: 50 pairs
+// 5.5 : 5.9, 400 6.7 : 7.5, 800 9.3 : 7.8). More pairs fill it with one wave each, and the first reading of the shared form,
+// for the tiles' sums, is then work on top. A chain is as long as tiles times outputs: with 8 outputs and 512 samples sharing
+// pays up to 1280 pairs (64 : 81, 2560 110 : 80), with 3 and 256 up to 400 (11.0 : 14.4, 800 15.3 : 15.4), and with one output
+// and two tiles never (50 pairs 5.2 : 4.9, 400 5.8 : 5.0; 3 outputs 400 pairs 8.9 : 9.4, 8 outputs 320 pairs 15.3 : 17.0).
 constexpr int64_t kSharedScanPairs = 512;
 
 void scan_split_launch(hipStream_t stream, int max_bins, const HistView& hv, const I64Pair* node_sums, int F,
@@ -779,7 +781,7 @@ void scan_split_launch(hipStream_t stream, int max_bins, const HistView& hv, con
                                                                   feature_set, scales, l1, l2, min_split_gain, partial,
                                                                   store);
   };
-  if (pairs > kSharedScanPairs || max_bins <= 64)
+  if (pairs > kSharedScanPairs || max_bins <= (hv.K == 1 ? 128 : 64))
     launch(scan_split_kernel<1>, (pairs + kThreads / 64 - 1) / (kThreads / 64), kThreads);
   else if (max_bins <= 256)
     launch(scan_split_kernel<4>, pairs, 4 * 64);

@@ -610,12 +610,13 @@ def test_few_rows_with_the_nodes_staged_or_not(n, f, s, depth):
     _assert_tree(got, cr)
 
 
-# A level of up to 512 (node, feature) pairs is scanned by four or eight waves a pair, a wider one by one wave: tiles
-# of 64 bins that do not divide evenly among the waves, fewer tiles than waves, features of one bin, levels on both
+# A level of up to 512 (node, feature) pairs is scanned by four or eight waves a pair (up to 64 bins, or 128 and one output,
+# by one), a wider one by one wave: tiles of 64 bins that do not divide evenly among the waves, fewer tiles than waves, features of one bin, levels on both
 # sides of the line, outputs whose hessians vanish, a penalty and features that are not to be split.
 @pytest.mark.parametrize("f,k,s,depth,kind", [(64, 1, 512, 5, "plain"), (64, 3, 129, 5, "plain"), (5, 8, 300, 4, "l1"), (513, 1, 65, 2, "plain"),
                                               (128, 2, 64, 4, "plain"), (9, 64, 257, 3, "plain"), (33, 5, 256, 6, "feature_set"),
-                                              (17, 4, 400, 5, "zero_output"), (40, 1, 449, 5, "zero_hessians")])
+                                              (17, 4, 400, 5, "zero_output"), (40, 1, 449, 5, "zero_hessians"),
+                                              (40, 1, 128, 4, "plain"), (40, 1, 129, 4, "plain"), (40, 2, 128, 4, "plain")])
 def test_waves_that_share_a_scan(f, k, s, depth, kind):
     import gpu_util as gu
 
