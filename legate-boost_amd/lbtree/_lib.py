@@ -11,6 +11,9 @@ tried.
 """
 import ctypes as C
 import os
+import warnings
+
+import torch  # (loads the libraries that _host is linked against)
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 SO_PATH = os.environ.get("LBTREE_SO") or os.path.join(os.path.dirname(_HERE), "csrc", "liblbtree.so")
@@ -208,13 +211,18 @@ def _load():
 
 lib = _load()
 
+# The ensemble calls look their trees over in native code where it is built for the torch at hand, else in Python (ops.py):
+# the same results, 1.4 us a tree later.
 try:
-    import torch  # noqa: E402,F401  (loads the libraries that _host is linked against)
+    from . import _host
 
-    from . import _host  # noqa: E402,F401
+    built_for = getattr(_host, "torch_version", None)
+    if built_for != str(torch.__version__):
+        raise ImportError("built for torch %s, this is %s" % (built_for, torch.__version__))
 except ImportError as e:
-    raise ImportError("lbtree/_host.so is missing or does not load (%s): build it with `make -C legate-boost_amd/csrc` "
-                      "or __graft_entry__.build()" % e)
+    _host = None
+    warnings.warn("lbtree/_host.so is missing or does not load (%s): ensembles are looked over in Python, which is slower; build it "
+                  "with `make -C legate-boost_amd/csrc` or __graft_entry__.build()" % e, RuntimeWarning)
 
 EXPORTS = [
     "lbt_last_error", "lbt_version", "lbt_release_thread_resources", "lbt_build_tree_workspace_bytes", "lbt_build_tree", "lbt_build_tree_async", "lbt_predict",

@@ -182,7 +182,7 @@ def build_tree(X, g, h, *, max_depth, split_samples, seed, l1_regularization=0.0
 def _tree_arrays(trees, n_outputs):
     """Host arrays of an ensemble's (leaf_value, feature, split_value): addresses of the three, nodes of every tree, all nodes,
     and what keeps the addresses valid."""
-    plain = _lib._host.tree_arrays(trees, n_outputs)
+    plain = _lib._host.tree_arrays(trees, n_outputs) if _lib._host is not None else None
     if plain is not None:
         return plain + (int(np.frombuffer(plain[3], np.int32).sum(dtype=np.int64)), trees)
     nt = len(trees)

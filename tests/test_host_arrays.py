@@ -1,4 +1,8 @@
 """lbtree._host.tree_arrays, the native look at an ensemble's arrays: what it does not take is left to the Python form."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -15,6 +19,32 @@ def test_anything_but_plain_device_arrays_is_left_to_the_caller():
     assert take([], 0) is None
     with pytest.raises(TypeError):
         take([cpu])
+
+
+@pytest.mark.parametrize("module", ["None", "types.SimpleNamespace(torch_version='0.0', tree_arrays=None)"])
+def test_the_package_imports_without_the_native_look(module):
+    """Not built, or built against another torch: said so, and looked over in Python."""
+    code = ("import sys, types, warnings\n"
+            "sys.modules['lbtree._host'] = %s\n"
+            "with warnings.catch_warnings(record=True) as told:\n"
+            "    warnings.simplefilter('always')\n"
+            "    from lbtree import _lib, ops\n"
+            "assert _lib._host is None and any('_host.so' in str(w.message) for w in told)\n"
+            "assert ops._tree_arrays([], 1)[4] == 0\n" % module)
+    package = os.path.dirname(os.path.dirname(os.path.abspath(_lib.__file__)))
+    subprocess.run([sys.executable, "-c", code], check=True, env=dict(os.environ, PYTHONPATH=package))
+
+
+@pytest.mark.gpu
+def test_the_python_form_gives_the_same(monkeypatch):
+    rs = np.random.RandomState(3)
+    trees = [(torch.from_numpy(rs.randn(15, 2)).cuda(), torch.from_numpy(np.r_[rs.randint(0, 5, 7), -np.ones(8)].astype(np.int32)).cuda(),
+              torch.from_numpy(rs.rand(15)).cuda()) for _ in range(20)]
+    X = torch.rand(300, 5).cuda()
+    want = ops.predict(X, trees, 2)
+    monkeypatch.setattr(_lib, "_host", None)
+    assert torch.equal(ops.predict(X, trees, 2), want)
+    assert torch.equal(ops.PackedEnsemble(trees, 2, 5).predict(X), want)
 
 
 @pytest.mark.gpu
