@@ -440,9 +440,9 @@ def bench_predict(args, steps=None, warmup=None, light=False):
                    "rows": rows, "trees": 1000, "row_trees_per_s": rows * 1000 * steps / dt,
                    "node_steps_per_s": rows * 8000 * steps / dt},
         # X read once and the output written once are all the HBM bytes this path needs (achieved /
-        # peak / frac price those); what bounds the walk is the LDS and the vector units, both busy for two
-        # thirds of it: every node step of a wave is two LDS reads (node, rank of the feature's value) and
-        # four vector instructions (profiles/predict_ranked_cfg5_*.txt)
+        # peak / frac price those); what bounds the walk is the LDS (busy for 74 % of it) and the vector units
+        # (62 %): every node step of a wave is two LDS reads (node, rank of the feature's value) and four
+        # vector instructions (counters in profiles/predict_ranked_cfg5_20Mx64_1000trees.txt)
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": None, "kernel": "walk_ranked_kernel",
                      "limited_by": "lds",

@@ -66,9 +66,8 @@ struct RowBatch {
 // The rows at positions [begin, end) into the LDS histograms [kPer][width] of the nf features of a
 // piece, cleared here. A row is two loads one after the other, its number and its record, and a workgroup of a
 // deep level has few rows: four a thread are under way together, the first ones while the histograms are cleared
-// (one at a time
-// the levels of 512, 1024 and 2048 nodes of 1,000,000 x 50 took 108, 127 and 193 us, now 92, 108 and 176; two at a time
-// the same).
+// (one at a time the levels of 512, 1024 and 2048 nodes of 1,000,000 x 50 took 108, 127 and 193 us, now 92, 108 and 176; two
+// at a time the same).
 template <typename BinT>
 __device__ __forceinline__ void add_rows(const DirectLevel& a, const RecInfo& ri, int piece, int nf, int begin, int end,
                                          int width, unsigned long long* s_hist)

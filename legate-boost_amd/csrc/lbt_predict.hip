@@ -458,9 +458,10 @@ __global__ void __launch_bounds__(kTileThreads)
 // trips to memory and the LDS (256 x 32 with 100 trees of depth 6: 12.3 us). Here a workgroup takes kFewRows rows through
 // as many batches at once as the LDS holds, a (row, tree) per lane; everything that is needed first (rows, the nodes from the
 // start of the array, the lanes' trees) is asked for before the first wait. The values pass through the LDS to the lanes
-// that add a row's in tree order: 7.3 us a launch where the tile kernel takes 12.4 (1000 x 10 f64: 16.7 and 9.9). A workgroup
-// copies the ensemble for 16 rows only: with 6433 x 94 and 117 trees of depth 7 it takes 22.0 us and the tile kernel 15.3,
-// with 4096 x 32 and 100 of depth 6 7.9 and 13.1. An ensemble of at most as many trees as a row has lanes there (up to
+// that add a row's in tree order: 7.3 us a launch where the tile kernel takes 12.4 (1000 x 10 f64: 9.9 and 16.7). Ensembles and
+// rows that no cache holds, one after the other: 9.8 us a call (the host's time) and 14.3. A workgroup copies the ensemble
+// for 16 rows only: with 6433 x 94 and 117 trees of depth 7 it takes 22.0 us and the tile kernel 15.3, with 4096 x 32 and 100
+// of depth 6 7.9 and 13.1. An ensemble of at most as many trees as a row has lanes there (up to
 // 16) is one batch there too: 52 x 5, 7 trees 3.8 and 3.9 us.
 constexpr int kFewRows        = 16;
 constexpr int64_t kFewMostRows = 4096;  // one workgroup per CU
@@ -852,7 +853,8 @@ int predict_any(hipStream_t stream, const T* X, int64_t N, int F, int n_trees, c
   if (workspace != nullptr && workspace_bytes > packed) {
     LBT_TRY(predict_ranked<T>(stream, X, N, F, n_trees, leaf, feature, split, tree_nodes, K, out,
                               static_cast<char*>(workspace) + packed, workspace_bytes - packed, &done, &wanted));
-    // wanted: only the device knows whether the ranks sufficed; what follows then runs or ends at once
+    // wanted: only the device knows whether the ranks sufficed; what follows then runs or ends at once (0.14 ms of a call with
+    // 1000 trees of depth 8 for packing and a launch that reads one word)
     if (done && wanted == nullptr) return LBT_OK;
   }
   LBT_TRY(predict_tiled<T>(stream, X, N, F, n_trees, leaf, feature, split, tree_nodes, K, wanted, out, workspace,

@@ -10,8 +10,9 @@
 // depth 8: 67.9 ms). With ranks of 16 bits a node is one word (rank, feature), a value is two bytes, four times as
 // many rows share a copied node, a lane keeps one row (its value of any feature lies in the lane's own bank) and
 // adds its own leaf values, and the tree is a complete heap, so that no child index is stored: 7 cycles, 29.6 ms, and
-// 2.8 ms for the ranks. Vector instructions (four a step), LDS and L1 are then each busy for two thirds of the time; reads in
-// two staggered halves (30.7 ms) and rank loads into the upper half of a register (34.5) were no faster.
+// 2.8 ms for the ranks. The LDS is then busy for 74 % of the time (8 % conflicts), the vector units (4.4 instructions a step)
+// for 62 %, and the L1 looks up 0.66 lines a cycle (profiles/predict_ranked_cfg5_20Mx64_1000trees.txt); reads in two
+// staggered halves (30.7 ms) and rank loads into the upper half of a register (34.5) were no faster.
 #include "lbt_internal.h"
 
 #include <algorithm>
