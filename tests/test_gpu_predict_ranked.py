@@ -84,6 +84,7 @@ def test_thresholds_that_crowd_one_feature(n_trees, share, dtype):
 @pytest.mark.parametrize("n,f,n_trees,depth,nan_from", [
     (700_001, 40, 200, 8, 32),  # the last features have NaN thresholds only
     (600_011, 9, 200, 8, 8),
+    (100_003, 520, 60, 5, 512),  # features by the cache line
     (3_000_003, 1, 120, 3, 0),  # and here there are no others at all
 ])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
