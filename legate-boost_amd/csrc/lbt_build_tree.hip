@@ -2016,9 +2016,10 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
   //    ones, 193 -> 92; with level 8, whose histograms are 0.8 of the records, a balanced tree would take 1.56 ms instead of
   //    1.62, one of noise, whose large nodes are added range by range, 2.07 instead of 1.97).
   int direct_from = max_depth;
+  int range_of_large = 0;   // of a direct level
   bool large_ready = false;  // the histograms of large nodes lie where other levels' did, and begin at zero
   if (plain && L.left != nullptr && hs.binned != nullptr && hs.embed && hs.max_bins <= kDirectMaxBins &&
-      N < (int64_t(1) << 30) && direct_large_bytes(hs, N) <= L.hist_bytes) {
+      N < (int64_t(1) << 30) && (range_of_large = direct_range(hs, N, L.hist_bytes)) > 0) {
     direct_from = 2;  // at the root it is not known yet
     while (direct_from < max_depth && static_cast<double>(bytes_per_node) * static_cast<double>(int64_t(1) << direct_from) <
                                         static_cast<double>(N) * static_cast<double>(hs.max_rec_stride))
@@ -2054,7 +2055,7 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
     int64_t num_batches          = 1;
     if (nodes_in_level > max_batch_size && !(lazy && contained)) num_batches = (nodes_in_level + max_batch_size - 1) / max_batch_size;
     if (direct) {
-      const int64_t large16 = static_cast<int64_t>(direct_large_bytes(hs, N) / 16);
+      const int64_t large16 = static_cast<int64_t>(direct_large_bytes(hs, N, range_of_large) / 16);
       if (!large_ready && large16 > 0) {
         ProfScope ps(LBT_PROF_OTHER, stream, 16.0 * static_cast<double>(large16));
         zero_kernel<<<static_cast<unsigned>(std::min<int64_t>((large16 + kThreads - 1) / kThreads, 65536)), kThreads, 0, stream>>>(
@@ -2064,7 +2065,7 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
       DirectLevel dl;
       dl.level_first = level_first; dl.n_nodes = static_cast<int>(nodes_in_level); dl.n_features = F;
       dl.n_groups = hs.n_groups; dl.n_rows = N; dl.binned = hs.binned; dl.rec = hs.rec; dl.groups = hs.groups;
-      dl.block_seg = L.block_seg[cur_seg]; dl.slab = kPartBlock; dl.large = reinterpret_cast<unsigned long long*>(L.hist);
+      dl.block_seg = L.block_seg[cur_seg]; dl.slab = kPartBlock; dl.range = range_of_large; dl.large = reinterpret_cast<unsigned long long*>(L.hist);
       dl.arrivals = nullptr;
       dl.rows = L.rows[cur_pos]; dl.seg = L.seg[cur_seg]; dl.row_pointers = L.row_pointers; dl.feature_set = feature_set;
       dl.scales = L.scales; dl.l1 = prm.l1_regularization; dl.l2 = prm.l2_regularization;

@@ -9,12 +9,12 @@
 //
 // A tree need not be balanced: with gradients that are mostly noise one node of a level can hold nearly all rows, and
 // its few workgroups then were the whole level (1,000,000 x 50 with 512 samples, depth 12, noise: 3.55 ms a tree, where
-// histograms in memory took 2.55; 2,000,000 x 80, depth 11 3.93 and 2.14). So the rows of a node of more than 16384 are
-// dealt to workgroups by ranges of 8192 positions; each adds its sums to the node's histogram in memory, and the
-// last one to finish scans it: 2.07 and 2.24 ms, and 1.95 as before where the tree is balanced (1.97, 2.16 and 1.62 with
-// the estimates below). It needs 8 bytes per bin and 16384 rows, in the room of the histograms that are not kept.
-// Shorter ranges add more often (4096: 2.56 and 2.53 ms), longer ones leave nodes that fit none to one workgroup
-// (16384: 2.01 and 2.13, but 250,000 x 43 1.36 where 8192 takes 1.20).
+// histograms in memory took 2.55; 2,000,000 x 80, depth 11 3.93 and 2.14). So the rows of a node of more than two ranges
+// of positions are dealt to workgroups by range; each adds its sums to the node's histogram in memory, and the
+// last one to finish scans it. It needs 8 bytes per bin and two ranges, in the room of the histograms that are not kept.
+// 1,000,000 x 50 with 512 samples, 4 trees of depth 12, us of the launches of levels 9 to 11, with ranges of 8192 and 4096: a
+// third of the rows in large nodes 1583 and 1417, nodes of equal size 1193 and 1208, noise 1165 and 1321; 250,000 x 43 with
+// 256 samples, noise, 1068 and 889 (2048: half as much again, they add more often).
 //
 // Only where every rounded hessian is positive: a scanned histogram is then the running sums everywhere
 // (build_tree.cu:645 leaves nothing unscanned) and it does not matter that nothing is derived by subtraction.
@@ -40,8 +40,9 @@ __device__ __forceinline__ I64Pair unpack_sums(unsigned long long w, int64_t up,
   return I64Pair{g, static_cast<int64_t>(static_cast<uint32_t>(w))};
 }
 
-constexpr int kDirectRange = 8192;              // positions of a range
-constexpr int kDirectLarge = 2 * kDirectRange;  // rows of a node that one workgroup takes: a range meets at most two larger ones
+// Positions of a range: the shorter ones where their nodes' histograms have the room. A node of up to two ranges is one
+// workgroup's, so that a range meets at most two larger ones.
+constexpr int kDirectRanges[] = {4096, 8192};
 
 // A thread's next rows: what a piece of their records holds and their pairs. Positions behind the last one read it again.
 constexpr int kRowsAtOnce = 4;
@@ -162,89 +163,116 @@ __device__ __forceinline__ Found scan_feature(const DirectLevel& a, const I64Pai
   return best.of_wave();
 }
 
-// Largest value of a wave, in every lane; values are not negative zero and not NaN
-__device__ __forceinline__ double wave_max(double v)
-{
-  auto take = [&](auto ctrl, auto rows) {
-    const int64_t bits = __double_as_longlong(v);
-    // lanes without a source take their own value
-    const int lo = __builtin_amdgcn_update_dpp(static_cast<int>(bits), static_cast<int>(bits), decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(static_cast<int>(bits >> 32), static_cast<int>(bits >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
-    const double o = __longlong_as_double((static_cast<int64_t>(hi) << 32) | static_cast<uint32_t>(lo));
-    v = o > v ? o : v;
-  };
-  using std::integral_constant;
-  take(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});
-  take(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
-  take(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
-  take(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
-  take(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});
-  take(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});
-  return wave_read_lane_f64(v, 63);
-}
-
 // Most bins cannot be the best split, and a shorter sum shows it. With integers gl, hl, gr, hr left and right of a bin,
 // gl^2 / (hl + reg / inv_h) + gr^2 / (hr + reg / inv_h) times inv_g^2 / inv_h is what the gain is made of without a
-// penalty (l1 = 0); formed with one approximate reciprocal (to 2^-23, the instruction's bound) it is right to 2^-22.
+// penalty (l1 = 0). Formed in 32 bits, every term but the sums rounded once (2^-24) and one approximate reciprocal (2^-23), it
+// is right to 15 * 2^-24 < 2^-20: nothing is subtracted after the exact whole-number differences.
 // The gain is a monotone function of the two quotients' sum, and every rounding on the way to it (minus the node's own
 // term, minus a min_split_gain that is not negative, where it ends above 0) merges sums within a few units of 2^-52: so a
-// bin whose estimate is below 1 - 2^-20 of the feature's largest has a smaller gain. One gain per lane is then
-// formed exactly, of its largest estimate, and where a lane holds a second one that near (a plateau of 64 empty bins,
-// equal columns) the feature is scanned as above.
-// The levels of 512, 1024 and 2048 nodes of 1,000,000 x 50 with 512 samples: 120, 149 and 234 us with every gain, 108, 127
-// and 193 with estimates (about 60 instructions for 64 bins, and the launch is bound by them still).
-// Not used with magnitudes whose squares might leave the doubles' range.
-constexpr double kNearBest = 1.0 - 1.0 / (1 << 20);
+// bin whose estimate is below 1 - 2^-18 of the feature's largest has a smaller gain. One gain per lane is then
+// formed exactly, of its largest estimate, and where a lane holds a second one that near (equal columns) the feature
+// is scanned as above. A bin without rows has the sums of the last one with rows before it: only those are
+// estimated, and which of the bins up to the next one with rows the tie rule takes is worked out for the best.
+// A lane takes four bins in a row, so that a running sum over the lanes serves 256 bins.
+// The 12 launches of levels 9 to 11 of four trees of depth 12, 1,000,000 x 50 with 512 samples: 1361 us with estimates in
+// 64 bits of one bin a lane, now 1208; what bounds them then is the chain of loads of a workgroup's rows (75 of the 82 us of
+// level 9 without any scan).
+// Not used with magnitudes whose products might leave the range of 32-bit floats: whole numbers are below 2^33, extra
+// (reg / inv_h) below 2^40.
+constexpr float kNearBest = 1.0f - 1.0f / (1 << 18);
 __device__ __forceinline__ bool estimates_hold(const DirectLevel& a, double inv_g, double inv_h, double reg)
 {
   auto ordinary = [](double v) { return v >= 1e-60 && v <= 1e60; };
   return a.l1 == 0.0 && a.min_split_gain >= 0.0 && ordinary(inv_g) && ordinary(inv_h) && ordinary(reg) &&
-         ordinary(reg / inv_h);
+         reg / inv_h >= 1e-30 && reg / inv_h <= 1e12;
 }
 
+// kSmall: all sums of grads fit 32 bits with their sign
+template <bool kSmall>
 __device__ __forceinline__ Found scan_feature_estimated(const DirectLevel& a, const I64Pair& ns, int fb, int n_bins,
                                                         double inv_g, double inv_h, double reg, int64_t up,
                                                         int64_t down, const unsigned long long* s_bins)
 {
-  const int lane     = threadIdx.x & 63;
-  const double extra = reg / inv_h, all_g = static_cast<double>(ns.grad), all_h = static_cast<double>(ns.hess);
+  constexpr int kBins = 4;
+  const int lane        = threadIdx.x & 63;
+  const float extra     = static_cast<float>(reg / inv_h);
+  const int small_g     = static_cast<int>(ns.grad);
+  const double all_g    = static_cast<double>(ns.grad);
+  const uint32_t all_h  = static_cast<uint32_t>(ns.hess);
   // grads lie in [-down, up] and up + down < 2^32: the lower 32 bits of grad + down are grad + down
   const uint32_t down32  = static_cast<uint32_t>(down);
   const double down_sums = static_cast<double>(down);
-  unsigned long long before = 0, left_1 = 0;
-  double last = -1.0, most = -1.0, second = -1.0;  // estimates: of the last bin so far, of this lane the two largest
-  int bin_1   = 0;
-  for (int base = 0; base < n_bins; base += 64) {
-    const int bin                = base + lane;
-    const bool in                = bin < n_bins;
-    const unsigned long long add = in ? s_bins[bin] : 0;
-    double estimate              = last;
-    unsigned long long left      = before;
-    if (__any(add != 0)) {
-      left += wave_inclusive_halves(add);
-      const double gl = static_cast<double>(static_cast<uint32_t>(left >> 32) + down32) - down_sums;
-      const double hl = static_cast<double>(static_cast<uint32_t>(left));
-      const double gr = all_g - gl, hr = all_h - hl;
-      const double pl = hl + extra, pr = hr + extra;
-      estimate = (gl * gl * pr + gr * gr * pl) * __builtin_amdgcn_rcp(pl * pr);
-      estimate = hl > 0 && hr > 0 ? estimate : -1.0;
-      before   = static_cast<unsigned long long>(wave_read_lane(static_cast<int64_t>(left), 63));
-      last     = wave_read_lane_f64(estimate, 63);
+  uint32_t before_g = 0, before_h = 0, left_g = 0, left_h = 0;
+  float most = -1.0f, second = -1.0f;  // of this lane the two largest estimates
+  int bin_1  = 0;
+  for (int base = 0; base < n_bins; base += 64 * kBins) {
+    const int first = base + lane * kBins;
+    uint32_t g[kBins] = {}, h[kBins] = {};
+    if (first < n_bins) {
+      // (a feature's bins take a multiple of four places, zeros behind the last one)
+      const uint4 w0 = *reinterpret_cast<const uint4*>(s_bins + first), w1 = *reinterpret_cast<const uint4*>(s_bins + first + 2);
+      h[0] = w0.x, g[0] = w0.y, h[1] = w0.z, g[1] = w0.w;
+      h[2] = w1.x, g[2] = w1.y, h[3] = w1.z, g[3] = w1.w;
     }
-    const bool more = in && estimate > most;
-    second = more ? most : (in && estimate > second ? estimate : second);
-    most   = more ? estimate : most;
-    left_1 = more ? left : left_1;
-    bin_1  = more ? bin : bin_1;
+    // The lower halves' sums stay below 2^32, so nothing is carried and the halves are summed on their own.
+    uint32_t sum_g = 0, sum_h = 0;
+#pragma unroll
+    for (int u = 0; u < kBins; u++) sum_g += g[u], sum_h += h[u];
+    if (!__any(sum_h != 0)) continue;
+    const uint32_t to_g = before_g + static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum_g)));
+    const uint32_t to_h = before_h + static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum_h)));
+    before_g = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(to_g), 63));
+    before_h = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(to_h), 63));
+    uint32_t lg = to_g - sum_g, lh = to_h - sum_h;
+#pragma unroll
+    for (int u = 0; u < kBins; u++) {
+      lg += g[u];
+      lh += h[u];
+      float gl, gr;
+      if constexpr (kSmall) {
+        gl = static_cast<float>(static_cast<int>(lg));
+        gr = static_cast<float>(small_g - static_cast<int>(lg));
+      } else {
+        const double left = static_cast<double>(lg + down32) - down_sums;
+        gl = static_cast<float>(left);
+        gr = static_cast<float>(all_g - left);
+      }
+      const float pl = static_cast<float>(lh) + extra, pr = static_cast<float>(all_h - lh) + extra;
+      const float sum      = __builtin_fmaf(gl * gl, pr, gr * gr * pl) * __builtin_amdgcn_rcpf(pl * pr);
+      const float estimate = (h[u] != 0) & (lh != all_h) ? sum : -1.0f;
+      const bool more      = estimate > most;
+      second = __builtin_fmaxf(second, __builtin_fminf(most, estimate));
+      most   = __builtin_fmaxf(most, estimate);
+      left_g = more ? lg : left_g;
+      left_h = more ? lh : left_h;
+      bin_1  = more ? first + u : bin_1;
+    }
   }
-  const double near = wave_max(most) * kNearBest;
-  if (near < 0) return Found{0.0, -1, 0};  // no valid split
+  // positive floats compare as whole numbers; an estimate of 0 is a gain that is not positive
+  const uint32_t top = wave_max_u32(most > 0.0f ? __float_as_uint(most) : 0u);
+  if (top == 0) return Found{0.0, -1, 0};  // no valid split
+  const float near = __uint_as_float(top) * kNearBest;
   if (__any(second >= near)) return scan_feature(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, s_bins);
-  const bool maybe = most >= near;
-  bool dead        = false;
-  double gain      = 0.0;
-  add_gain(gain, dead, unpack_sums(left_1, up, down), ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
-  return Found{gain, maybe && gain > 0 ? fb + bin_1 : -1, left_1}.of_wave();
+  const unsigned long long left = static_cast<unsigned long long>(left_g) << 32 | left_h;
+  bool dead   = false;
+  double gain = 0.0;
+  add_gain(gain, dead, unpack_sums(left, up, down), ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
+  const bool maybe = most >= near && gain > 0;
+  int pick = -1;
+  for (unsigned long long left_to_do = __ballot(maybe); left_to_do != 0; left_to_do &= left_to_do - 1) {
+    const int from = __builtin_ctzll(left_to_do), bin = __builtin_amdgcn_readlane(bin_1, from);
+    int next = n_bins;  // the next bin with rows
+    for (int base = bin + 1; base < n_bins; base += 64) {
+      const unsigned long long rows = __ballot(base + lane < n_bins && static_cast<uint32_t>(s_bins[min(base + lane, n_bins - 1)]) != 0);
+      if (rows != 0) {
+        next = base + __builtin_ctzll(rows);
+        break;
+      }
+    }
+    // of bins that share a gain the one of 511 mod 512, else the last one
+    if (lane == from) pick = min((fb + bin) | 511, fb + next - 1);
+  }
+  return Found{gain, pick, left}.of_wave();
 }
 
 // The best split of each of the features [f0, f0 + nf) of node j from its histograms in the LDS.
@@ -257,6 +285,7 @@ __device__ __forceinline__ void scan_features(const DirectLevel& a, int j, const
   const double inv_g = a.scales[2], inv_h = a.scales[3];
   const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
   const bool estimated = estimates_hold(a, inv_g, inv_h, reg);
+  const bool small     = up <= 2147483647LL && down <= 2147483647LL;
   for (int v = wave; v < nf; v += kDirectThreads / 64) {
     const int f    = f0 + v;
     const int64_t at = static_cast<int64_t>(j) * a.n_features + f;
@@ -265,8 +294,10 @@ __device__ __forceinline__ void scan_features(const DirectLevel& a, int j, const
       continue;
     }
     const int fb = a.row_pointers[f], n_bins = a.row_pointers[f + 1] - fb;
-    const Found best = estimated ? scan_feature_estimated(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, s_hist + v * width)
-                                 : scan_feature(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, s_hist + v * width);
+    const unsigned long long* bins = s_hist + v * width;
+    const Found best = !estimated ? scan_feature(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, bins)
+                       : small    ? scan_feature_estimated<true>(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, bins)
+                                  : scan_feature_estimated<false>(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, bins);
     if (lane == 0) {
       a.partial[at] = Cand{best.gain, best.bin};
       a.left[at]    = unpack_sums(best.left, up, down);
@@ -302,32 +333,35 @@ __device__ __forceinline__ void add_range(const DirectLevel& a, int range, int p
 {
   constexpr int kPer = 16 / sizeof(BinT);
   const int tid   = threadIdx.x;
-  const int first = range * kDirectRange;
-  const int last  = static_cast<int>(min(a.n_rows, static_cast<int64_t>(first) + kDirectRange));
+  const int first = range * a.range;
+  const int last  = static_cast<int>(min(a.n_rows, static_cast<int64_t>(first) + a.range));
   for (int side = 0; side < 2; side++) {
     const int j = side == 0 ? a.block_seg[first / a.slab] : (last < a.n_rows ? a.block_seg[last / a.slab] : -1);
     if (j < 0) continue;
     const int begin = a.seg[j], end = a.seg[j + 1];
-    if (end - begin <= kDirectLarge || (side == 1 && (begin <= first || begin >= last))) continue;
+    if (end - begin <= 2 * a.range || (side == 1 && (begin <= first || begin >= last))) continue;
     const Piece p = piece_of<BinT>(a, part);
     add_rows<BinT>(a, p.rec, p.number, p.nf, max(first, begin), min(last, end), width, s_hist);
-    // large nodes begin more than kDirectLarge positions apart: a slot each. Slots and counters are zero between nodes.
-    const int64_t slot      = static_cast<int64_t>(begin / kDirectLarge) * pieces + part;
+    // large nodes begin more than two ranges apart: a slot each. Slots and counters are zero between nodes.
+    const int64_t slot      = static_cast<int64_t>(begin / (2 * a.range)) * pieces + part;
     unsigned long long* sum = a.large + slot * kPer * width;
     for (int i = tid; i < p.nf * width; i += kDirectThreads)
       if (s_hist[i] != 0) atomicAdd(sum + i, s_hist[i]);
-    __threadfence();
+    // Every word of the slot is added to and read by device-wide atomic operations, so it suffices that a wave's have
+    // arrived before the workgroup is counted. A __threadfence() also writes the whole L2 back, once per wave: the
+    // levels of 512 and 1024 nodes of 1,000,000 x 50, a third of the rows in large nodes, took 350 and 190 us with
+    // two of them here, 130 and 125 without.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     // (the answer goes through the histograms' LDS: a word more and only four workgroups of 512 bins share a CU)
     if (tid == 0) {
-      const int ranges = (end - 1) / kDirectRange - begin / kDirectRange + 1;
+      const int ranges = (end - 1) / a.range - begin / a.range + 1;
       s_hist[0]        = atomicAdd(a.arrivals + slot, 1) + 1 == ranges ? 1 : 0;
     }
     __syncthreads();
     const bool last_of_node = s_hist[0] != 0;
     __syncthreads();
     if (!last_of_node) continue;
-    __threadfence();
     for (int i = tid; i < p.nf * width; i += kDirectThreads) {
       s_hist[i] = __hip_atomic_load(sum + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       sum[i]    = 0;
@@ -358,7 +392,7 @@ __global__ void __launch_bounds__(kDirectThreads)
   if (j >= a.n_nodes) return;
   const I64Pair ns = a.node_sums[a.level_first + j];
   const int begin = a.seg[j], end = a.seg[j + 1];
-  if (ns.hess <= 0 || end - begin > kDirectLarge) return;
+  if (ns.hess <= 0 || end - begin > 2 * a.range) return;
   const Piece p = piece_of<BinT>(a, (id >> 3) % pieces);
   add_rows<BinT>(a, p.rec, p.number, p.nf, begin, end, width, s_hist);
   scan_features(a, j, ns, p.f0, p.nf, width, s_hist);
@@ -406,31 +440,42 @@ __global__ void __launch_bounds__(kDirectThreads) direct_apply_kernel(DirectLeve
 
 }  // namespace
 
-size_t direct_large_words(const HistSetup& hs, int64_t n_rows)
+// Words of a feature's histogram: the scan takes four bins a lane
+static int direct_width(const HistSetup& hs) { return (hs.max_bins + 3) / 4 * 4; }
+
+static size_t direct_large_words(const HistSetup& hs, int64_t n_rows, int range)
 {
-  return n_rows <= kDirectLarge ? 0 : static_cast<size_t>(n_rows / kDirectLarge + 1) * hs.pieces * (16 / hs.bin_bytes) * hs.max_bins;
+  return n_rows <= 2 * range ? 0 : static_cast<size_t>(n_rows / (2 * range) + 1) * hs.pieces * (16 / hs.bin_bytes) * direct_width(hs);
 }
 
-size_t direct_large_bytes(const HistSetup& hs, int64_t n_rows)
+size_t direct_large_bytes(const HistSetup& hs, int64_t n_rows, int range)
 {
-  const size_t counters = static_cast<size_t>(n_rows / kDirectLarge + 1) * hs.pieces * sizeof(int32_t);
-  return n_rows <= kDirectLarge ? 0 : direct_large_words(hs, n_rows) * sizeof(unsigned long long) + (counters + 15) / 16 * 16;
+  const size_t counters = static_cast<size_t>(n_rows / (2 * range) + 1) * hs.pieces * sizeof(int32_t);
+  return n_rows <= 2 * range ? 0 : direct_large_words(hs, n_rows, range) * sizeof(unsigned long long) + (counters + 15) / 16 * 16;
+}
+
+int direct_range(const HistSetup& hs, int64_t n_rows, size_t room)
+{
+  for (const int range : kDirectRanges)
+    if (direct_large_bytes(hs, n_rows, range) <= room) return range;
+  return 0;
 }
 
 int direct_level_launch(hipStream_t stream, DirectLevel a, const HistSetup& hs)
 {
-  LBT_REQUIRE(kDirectRange % a.slab == 0, "ranges of positions are whole slabs");
-  a.arrivals          = reinterpret_cast<int32_t*>(a.large + direct_large_words(hs, a.n_rows));
-  const int ranges    = a.n_rows <= kDirectLarge ? 0 : ceil_div(a.n_rows, kDirectRange);
+  LBT_REQUIRE(a.range > 0 && a.range % a.slab == 0, "ranges of positions are whole slabs");
+  a.arrivals          = reinterpret_cast<int32_t*>(a.large + direct_large_words(hs, a.n_rows, a.range));
+  const int ranges    = a.n_rows <= 2 * a.range ? 0 : ceil_div(a.n_rows, a.range);
   const int large     = (ranges + 7) / 8 * 8 * hs.pieces;
+  const int width     = direct_width(hs);
   const unsigned grid = static_cast<unsigned>(large) + static_cast<unsigned>((a.n_nodes + 7) / 8 * 8) * static_cast<unsigned>(hs.pieces);
-  const size_t lds    = static_cast<size_t>(16 / hs.bin_bytes) * hs.max_bins * sizeof(unsigned long long);
+  const size_t lds    = static_cast<size_t>(16 / hs.bin_bytes) * width * sizeof(unsigned long long);
   {
     ProfScope ps(LBT_PROF_HISTOGRAM, stream);
     if (hs.bin_bytes == 1)
-      direct_split_kernel<uint8_t><<<grid, kDirectThreads, lds, stream>>>(a, hs.pieces, hs.max_bins, ranges, large);
+      direct_split_kernel<uint8_t><<<grid, kDirectThreads, lds, stream>>>(a, hs.pieces, width, ranges, large);
     else
-      direct_split_kernel<uint16_t><<<grid, kDirectThreads, lds, stream>>>(a, hs.pieces, hs.max_bins, ranges, large);
+      direct_split_kernel<uint16_t><<<grid, kDirectThreads, lds, stream>>>(a, hs.pieces, width, ranges, large);
   }
   ProfScope ps(LBT_PROF_SPLIT, stream);
   direct_apply_kernel<<<static_cast<unsigned>((a.n_nodes + 3) / 4), kDirectThreads, 0, stream>>>(a);

@@ -501,6 +501,7 @@ struct DirectLevel {
   const int32_t* seg;
   const int32_t* block_seg;  // node that holds position b * slab (-1: a row that has stopped)
   int slab;
+  int range;                  // positions that a workgroup takes of a large node (direct_range)
   unsigned long long* large;  // histograms of large nodes, direct_large_bytes, all zero between nodes and levels
   int32_t* arrivals;          // ... of which counters (set by direct_level_launch)
   const int32_t* row_pointers;
@@ -517,7 +518,8 @@ struct DirectLevel {
   double* gain;
   int32_t* split_bin;
 };
-size_t direct_large_bytes(const HistSetup& hs, int64_t n_rows);  // multiple of 16
+int direct_range(const HistSetup& hs, int64_t n_rows, size_t room);  // 0: the large nodes' histograms have no room
+size_t direct_large_bytes(const HistSetup& hs, int64_t n_rows, int range);  // multiple of 16
 int direct_level_launch(hipStream_t stream, DirectLevel a, const HistSetup& hs);
 
 // ---------------------------------------------------------------- builder for few rows

@@ -508,7 +508,31 @@ def test_levels_without_histograms_in_memory_give_the_oracles_tree(n, f, s, dept
     _assert_tree(got, orc.build_tree(X, g, h, **kw))
 
 
-@pytest.mark.parametrize("n,f,s,depth,kind", [(16385, 3, 64, 11, "outliers"), (30001, 7, 256, 11, "outliers"), (60000, 5, 300, 12, "noise"),
+@pytest.mark.parametrize("n,f,s,depth,kind", [(9001, 9, 511, 12, "one_sign"), (9001, 6, 254, 11, "near_ties"), (20001, 5, 509, 12, "near_ties"),
+                                              (12001, 17, 61, 11, "equal_columns"), (9001, 8, 512, 12, "l2")])
+def test_deep_levels_whose_estimates_do_not_decide(n, f, s, depth, kind):
+    """Sums of grads that leave 32 bits with their sign, bins whose estimates lie closer together than they are right, equal
+    columns, a penalty far above the hessians; bins that are no multiple of the four a lane takes: the oracle's tree."""
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(s)
+    X = rs.randn(n, f).astype(np.float32)
+    g, h = rs.randn(n, 1), np.ones((n, 1))
+    kw, l2 = dict(max_depth=depth, split_samples=s, seed=6), 1.0
+    if kind == "one_sign":
+        g = 1.0 + 0.2 * rs.rand(n, 1)
+    elif kind == "near_ties":
+        g = np.where(X[:, :1] > 0, 1.0, -1.0) * (1.0 + 1e-6 * rs.rand(n, 1))
+    elif kind == "equal_columns":
+        X[:, 1::2] = X[:, :1]
+    else:
+        l2 = 1e5
+    Xd, gd, hd = (torch.from_numpy(a).cuda() for a in (X, g, h))
+    _assert_tree(ops.build_tree(Xd, gd, hd, l2_regularization=l2, **kw), orc.build_tree(X, g, h, l2=l2, **kw))
+
+
+@pytest.mark.parametrize("n,f,s,depth,kind", [(8193, 4, 256, 11, "outliers"), (12300, 2, 512, 12, "noise"), (16385, 3, 64, 11, "outliers"), (30001, 7, 256, 11, "outliers"), (60000, 5, 300, 12, "noise"),
                                               (70001, 20, 512, 11, "one_split"), (65536, 70, 64, 11, "stopped")])
 def test_deep_levels_with_one_large_node(n, f, s, depth, kind):
     """Trees that are not balanced: nodes of more rows than one workgroup takes, which begin and end inside a range of
