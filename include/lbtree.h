@@ -448,6 +448,36 @@ int lbt_weighted_gradient_sums(void* stream, int32_t objective, const double* pr
                                int32_t n_outputs, double* g, double* h, double* abs_sum_chunks);
 
 /*
+ * The initial predictions (boost_from_average) of the two objectives.
+ * Squared error (legateboost/objectives.py:131-147): mean[k] = sum_r y[r][k] w[r] / sum_r w[r], added in double in a fixed order.
+ *   sample_weight NULL: all ones.  Up to 256 outputs (lbt_weighted_mean_workspace_bytes is 0 beyond).
+ * Log loss (objectives.py:489-531): lbt_label_counts adds to stats (device int64 [3 + 256], zeros before)
+ *   [0] labels that are no whole numbers of 0 or more, [1] (maximum) the largest label below 256, [2] labels of 256 and more,
+ *   [3 + c] labels equal to c < 256;  lbt_label_priors then writes log(count / n) of n_outputs classes, or, with
+ *   n_outputs = 1, the log odds of class 1.
+ */
+size_t lbt_weighted_mean_workspace_bytes(int32_t n_outputs);
+int lbt_weighted_mean(void* stream, const double* y, const double* sample_weight, int64_t n_rows, int32_t n_outputs,
+                      double* mean, void* workspace, size_t workspace_bytes);
+int lbt_label_counts(void* stream, const double* y, int64_t n, int64_t* stats);
+int lbt_label_priors(void* stream, const int64_t* stats, int64_t n, int32_t n_outputs, double* init);
+
+/*
+ * Row subsampling (legateboost/legateboost.py:215-222): g and h [n_rows][n_outputs] of the rows with draw[r] >= limit (or NaN)
+ * are multiplied by 0, in place.
+ */
+int lbt_keep_rows(void* stream, const double* draw, double limit, int64_t n_rows, int32_t n_outputs, double* g, double* h);
+
+/*
+ * Class probabilities of log loss from the sums of an ensemble's leaf values (legateboost/legateboost.py:507-529, transform
+ * of objectives.py:489-531):
+ *   v = init + raw;  one output: out[r] = (1 - p, p) with p = 1 / (1 + exp(-v));  several: out[r] = softmax(v[r])
+ *   raw   device double [n_rows][n_outputs];  init  device double [n_outputs]
+ *   out   device double [n_rows][n_outputs], [n_rows][2] for one output (16-byte aligned); may not alias raw
+ */
+int lbt_class_probabilities(void* stream, const double* raw, const double* init, int64_t n_rows, int32_t n_outputs, double* out);
+
+/*
  * pred[r][k] += leaf_value[row_leaf[r]][k]: the update `train_pred += model.predict(X)` of
  * legateboost/legateboost.py:268 for the tree just built, from lbt_build_taps.row_leaf
  * instead of a fresh traversal of X. Same doubles, same single addition per element as

@@ -32,6 +32,10 @@ class SquaredErrorObjective:
 
     def initialise_prediction(self, y, w, boost_from_average):
         if boost_from_average:
+            per_row = w is None or (w.dim() == 1 and w.shape[0] == y.shape[0] and not w.requires_grad)
+            if y.is_cuda and 0 < y.shape[0] and 0 < y.shape[1] <= ops.MAX_MEAN_OUTPUTS and per_row and not y.requires_grad:
+                return ops.weighted_mean(y, w)
+            w = torch.ones(y.shape[0], dtype=torch.float64, device=y.device) if w is None else w
             return (y * w[:, None]).sum(dim=0) / w.sum()
         return torch.zeros(y.shape[1], dtype=torch.float64, device=y.device)
 
@@ -56,6 +60,16 @@ class LogLossObjective:
         return e_x / e_x.sum(dim=1)[:, None]
 
     def initialise_prediction(self, y, w, boost_from_average):
+        if y.is_cuda and y.numel() > 0 and not y.requires_grad:
+            stats = ops.label_counts(y)
+            bad, most, wide = stats[:3].tolist()
+            if bad:
+                raise ValueError("Expected labels to be non-zero whole numbers")
+            if not wide:  # (more classes are counted by the operators below)
+                n_targets = most + 1 if most > 1 else 1
+                if not boost_from_average:
+                    return torch.zeros(n_targets, dtype=torch.float64, device=y.device)
+                return ops.label_priors(stats, y.numel(), n_targets)
         if not bool(((y == torch.floor(y)) & (y >= 0)).all()):
             raise ValueError("Expected labels to be non-zero whole numbers")
         num_class = int(y.max().item() + 1)
@@ -100,12 +114,25 @@ class LBBase:
             y = y.reshape(-1, 1)
         return X, y
 
+    def _weights(self, y, sample_weight):
+        """The rows' weights; None (all ones) where nothing but this module's own code sees them."""
+        if sample_weight is not None:
+            return ops.as_device(sample_weight, torch.float64)
+        own = ("_get_weighted_gradient", "_loss")
+        plain = (type(self) in (LBRegressor, LBClassifier) and not any(a in vars(self) for a in own)
+                 and type(self)._get_weighted_gradient is LBBase._get_weighted_gradient
+                 and type(self._objective_instance) in (SquaredErrorObjective, LogLossObjective)
+                 and not vars(self._objective_instance) and not self.verbose)
+        return None if plain else torch.ones(y.shape[0], dtype=torch.float64, device=y.device)
+
     def _get_weighted_gradient(self, y, pred, sample_weight, learning_rate):
         fused = getattr(self._objective_instance, "fused", None)
         if fused is not None and pred.is_cuda:
             g, h = ops.weighted_gradient(fused, y, pred, sample_weight, learning_rate)
         else:
             g, h = self._objective_instance.gradient(y, self._objective_instance.transform(pred))
+            if sample_weight is None:
+                sample_weight = torch.ones(y.shape[0], dtype=torch.float64, device=y.device)
             g = g * sample_weight[:, None] * learning_rate
             h = torch.clamp(h * sample_weight[:, None], min=1e-8)
         if self.subsample < 1.0:
@@ -115,7 +142,11 @@ class LBBase:
             # from cupynumeric's XORWOW stream, so which rows are kept is not comparable with the reference.
             seed = int(self.random_state_.randint(0, 2**32, dtype=np.int64))
             gen = torch.Generator(device=g.device).manual_seed(seed)
-            mask = (torch.rand(y.shape[0], generator=gen, device=g.device, dtype=torch.float64) < self.subsample)
+            draw = torch.rand(y.shape[0], generator=gen, device=g.device, dtype=torch.float64)
+            if fused is not None and g.is_cuda:  # (g and h are this call's own)
+                ops.keep_rows(draw, self.subsample, g, h)
+                return g, h
+            mask = draw < self.subsample
             mask = mask.to(torch.float64)[:, None]
             g = g * mask
             h = h * mask
@@ -132,10 +163,9 @@ class LBBase:
         self.n_features_in_ = X.shape[1]
         if not isinstance(self.base_models, tuple) or len(self.base_models) == 0:
             raise ValueError("base_models should be a tuple")
-        w = torch.ones(y.shape[0], dtype=torch.float64, device=y.device) if sample_weight is None \
-            else ops.as_device(sample_weight, torch.float64)
         self.random_state_ = _check_random_state(self.random_state)
         self._objective_instance = self._make_objective()
+        w = self._weights(y, sample_weight)
         self.model_init_ = self._objective_instance.initialise_prediction(y, w, self.init == "average")
         self.models_ = []
         self.train_metric_ = []
@@ -155,8 +185,7 @@ class LBBase:
 
     def update(self, X, y, sample_weight=None):
         X, y = self._prepare(X, y)
-        w = torch.ones(y.shape[0], dtype=torch.float64, device=y.device) if sample_weight is None \
-            else ops.as_device(sample_weight, torch.float64)
+        w = self._weights(y, sample_weight)
         if self.models_ and all(type(m).clear is Tree.clear for m in self.models_):
             torch._foreach_zero_([a for m in self.models_ for a in (m.leaf_value, m.hessian)])
         else:
@@ -206,7 +235,17 @@ class LBClassifier(LBBase):
 
     def predict_proba(self, X):
         X = ops.as_device(X)
-        p = self._objective_instance.transform(self._predict(X))
+        objective, init = self._objective_instance, self.model_init_
+        if (type(objective) is LogLossObjective and not vars(objective) and self.models_
+                and type(self)._predict is LBBase._predict and "_predict" not in vars(self)):
+            raw = type(self.models_[0]).batch_predict(self.models_, X)
+            if all(isinstance(a, torch.Tensor) and a.dtype == torch.float64 and a.is_cuda and a.is_contiguous()
+                   and not a.requires_grad for a in (raw, init)) \
+                    and raw.dim() == 2 and init.shape == raw.shape[1:] and init.device == raw.device:
+                return ops.class_probabilities(raw, init)
+            p = objective.transform(init.reshape(1, -1) + raw)
+        else:
+            p = objective.transform(self._predict(X))
         if p.shape[1] == 1:
             p = torch.cat([1.0 - p, p], dim=1)
         return p

@@ -322,6 +322,62 @@ def weighted_gradient(objective, y, pred, sample_weight=None, learning_rate=1.0,
     return g, h
 
 
+def weighted_mean(y, sample_weight=None):
+    """The initial prediction of squared error (legateboost/objectives.py:131-147): y [n, K] CUDA float64, weighted by row."""
+    y = as_device(y, torch.float64)
+    n, k = y.shape
+    w = None
+    if sample_weight is not None:
+        w = as_device(sample_weight, torch.float64)
+        if w.numel() != n:
+            raise _lib.LbtError("sample_weight must have one entry per row")
+    mean = torch.empty(k, dtype=torch.float64, device=y.device)
+    ws = torch.empty(int(_lib.lib.lbt_weighted_mean_workspace_bytes(k)), dtype=torch.uint8, device=y.device)
+    _lib.check(_lib.lib.lbt_weighted_mean(_stream(), y.data_ptr(), w.data_ptr() if w is not None else None, n, k,
+                                          mean.data_ptr(), ws.data_ptr(), ws.numel()))
+    return mean
+
+
+MAX_MEAN_OUTPUTS = 256
+
+
+def label_counts(y):
+    """What log loss asks of its labels y (CUDA float64): a CUDA int64 [3 + 256] of entries that are no whole numbers of 0 or
+    more, the largest label below 256, entries of 256 and more, and the classes' counts."""
+    y = as_device(y, torch.float64)
+    stats = torch.zeros(3 + 256, dtype=torch.int64, device=y.device)
+    _lib.check(_lib.lib.lbt_label_counts(_stream(), y.data_ptr(), y.numel(), stats.data_ptr()))
+    return stats
+
+
+def label_priors(stats, n, n_outputs):
+    """The initial prediction of log loss (legateboost/objectives.py:489-531) from label_counts of n labels."""
+    init = torch.empty(n_outputs, dtype=torch.float64, device=stats.device)
+    _lib.check(_lib.lib.lbt_label_priors(_stream(), stats.data_ptr(), n, n_outputs, init.data_ptr()))
+    return init
+
+
+def keep_rows(draw, limit, g, h):
+    """g and h [n, K] (contiguous CUDA float64, in place) times 0 in the rows whose draw is not below `limit`."""
+    n, k = g.shape
+    if any(a.dtype != torch.float64 or not a.is_cuda or not a.is_contiguous() for a in (draw, g, h)) \
+            or draw.numel() != n or h.shape != g.shape:
+        raise _lib.LbtError("draw [n], g and h [n, K] must be contiguous CUDA float64 tensors")
+    _lib.check(_lib.lib.lbt_keep_rows(_stream(), draw.data_ptr(), float(limit), n, k, g.data_ptr(), h.data_ptr()))
+
+
+def class_probabilities(raw, init):
+    """Class probabilities of log loss (legateboost/legateboost.py:507-529) from raw [n, K], the sums of the leaf values, and
+    the initial prediction [K], both CUDA float64: [n, K], or [n, 2] for K = 1."""
+    n, k = raw.shape
+    if init.numel() != k or not (raw.is_contiguous() and init.is_contiguous()) or raw.dtype != torch.float64 \
+            or init.dtype != torch.float64 or init.device != raw.device:
+        raise _lib.LbtError("raw and init must be contiguous float64 of [n, %d] and [%d]" % (k, k))
+    out = torch.empty((n, 2 if k == 1 else k), dtype=torch.float64, device=raw.device)
+    _lib.check(_lib.lib.lbt_class_probabilities(_stream(), raw.data_ptr(), init.data_ptr(), n, k, out.data_ptr()))
+    return out
+
+
 def update_trees(X, y, sample_weight, objective, learning_rate, pred, trees):
     """The loop of LBBase.update (legateboost/legateboost.py:306-386) over `trees`, a list of (feature, split_value,
     l1_regularization, l2_regularization): per tree weighted_gradient at pred, update_tree and the prediction update.

@@ -1,0 +1,117 @@
+"""What a fit and a prediction do either side of the trees, against the operators they stand for (legateboost.py:189-224,
+507-529, objectives.py:131-147 and :489-531)."""
+import ctypes as C
+import math
+
+import numpy as np
+import pytest
+import torch
+
+
+def test_calls_check_their_arguments():
+    from lbtree import _lib
+
+    lib, one, two = _lib.lib, C.c_void_p(16), C.c_void_p(32)
+    assert lib.lbt_class_probabilities(None, one, one, 10, 0, two) == -1
+    assert lib.lbt_class_probabilities(None, one, one, 10, 1, one) == -1
+    assert lib.lbt_class_probabilities(None, one, one, 10, 1, C.c_void_p(40)) == -1
+    assert b"aligned" in lib.lbt_last_error()
+    assert lib.lbt_class_probabilities(None, None, None, 0, 3, None) == 0
+    assert lib.lbt_weighted_mean_workspace_bytes(256) > 0 and lib.lbt_weighted_mean_workspace_bytes(257) == 0
+    assert lib.lbt_weighted_mean(None, one, None, 0, 1, one, one, 1 << 20) == -1
+    assert lib.lbt_weighted_mean(None, one, None, 10, 1, one, one, 8) == -3
+    assert lib.lbt_label_counts(None, None, 10, one) == -1
+    assert lib.lbt_label_priors(None, one, 10, 257, one) == -1
+    assert lib.lbt_keep_rows(None, one, 0.5, 10, 1, two, two) == -1
+    assert lib.lbt_keep_rows(None, None, 0.5, 0, 1, None, None) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(1, 1), (257, 1), (1, 2), (255, 3), (513, 8), (300, 10), (1000, 16), (70, 7), (40, 19), (3, 300)])
+def test_class_probabilities(n, k):
+    """exp and the sums of up to 300 terms round differently from torch's: (k + 8) 2^-52 of each probability."""
+    from lbtree import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    raw = 4 * torch.randn((n, k), generator=gen, device="cuda", dtype=torch.float64)
+    raw[0] = 600.0
+    raw[-1, 0] = -600.0
+    init = torch.randn(k, generator=gen, device="cuda", dtype=torch.float64)
+    v = init + raw
+    if k == 1:
+        p = 1.0 / (1.0 + torch.exp(-v))
+        want = torch.cat([1.0 - p, p], dim=1)
+    else:
+        want = torch.softmax(v, dim=1)
+    got = ops.class_probabilities(raw, init)
+    assert got.shape == want.shape
+    # an exponent rounded to 2^-53 of up to 1200 is off by 2^-43
+    assert torch.allclose(got, want, rtol=(k + 8) * 2.0 ** -52, atol=2.0 ** -52)
+    bad = raw.clone()
+    bad[n // 2, k - 1] = float("nan")
+    assert torch.equal(torch.isnan(ops.class_probabilities(bad, init)).all(dim=1),
+                       torch.arange(n, device="cuda") == n // 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(1, 1), (1023, 1), (1000003, 1), (5, 3), (40000, 7), (33, 256), (700, 130)])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_weighted_mean(n, k, weighted):
+    """Against exactly rounded sums: a thread adds up to n / 2^18 + 1 terms and a tree joins the threads."""
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + k)
+    y, w = 1.0 + rs.rand(n, k), 0.5 + rs.rand(n) if weighted else None
+    got = ops.weighted_mean(torch.from_numpy(y).cuda(), None if w is None else torch.from_numpy(w).cuda()).cpu().numpy()
+    ones = np.ones(n) if w is None else w
+    for c in range(0, k, max(1, k // 5)):
+        want = math.fsum(y[:, c] * ones) / math.fsum(ones)
+        assert abs(got[c] - want) <= (n / 2.0 ** 18 + 600) * 2.0 ** -53 * want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,classes", [(1, 1), (1025, 2), (100003, 2), (5000, 8), (3000, 256)])
+def test_labels_and_priors(n, classes):
+    from lbtree import ops
+
+    y = np.random.RandomState(n).randint(0, classes, n).astype(np.float64)
+    stats = ops.label_counts(torch.from_numpy(y).cuda())
+    count = np.bincount(y.astype(int), minlength=256)
+    assert stats.tolist() == [0, int(y.max()), 0] + count.tolist()
+    k = classes if classes > 2 else 1
+    with np.errstate(divide="ignore"):
+        share = count / n
+        want = -np.log(1 / share[1:2] - 1) if k == 1 else np.log(share[:k])
+    assert np.allclose(ops.label_priors(stats, n, k).cpu().numpy(), want, rtol=4 * 2.0 ** -52, atol=0)
+    for value, at in ((0.5, 0), (-1.0, 0), (float("nan"), 0), (256.0, 2), (float("inf"), 2)):
+        bad = y.copy()
+        bad[n // 2] = value
+        got = ops.label_counts(torch.from_numpy(bad).cuda()).tolist()
+        assert [got[0], got[2]] == [int(at == 0), int(at == 2)]
+
+
+@pytest.mark.gpu
+def test_labels_beyond_the_counted_ones_still_fit():
+    import lbtree as lb
+
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    X = torch.rand((600, 3), generator=gen, device="cuda")
+    y = torch.arange(600, device="cuda", dtype=torch.float64) % 300
+    model = lb.LBClassifier(n_estimators=1, base_models=(lb.models.Tree(max_depth=2),), random_state=0).fit(X, y)
+    assert model.predict_proba(X).shape == (600, 300)
+    assert torch.allclose(model.model_init_, torch.full((300,), math.log(1 / 300), dtype=torch.float64, device="cuda"))
+    with pytest.raises(ValueError, match="whole numbers"):
+        lb.LBClassifier(n_estimators=1).fit(X, y - 0.5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(1, 1), (257, 1), (300, 5)])
+def test_keep_rows(n, k):
+    from lbtree import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    g, h, draw = (torch.randn(s, generator=gen, device="cuda", dtype=torch.float64) for s in ((n, k), (n, k), (n,)))
+    mask = (draw < 0.3).to(torch.float64)[:, None]
+    want = g * mask, h * mask
+    ops.keep_rows(draw, 0.3, g, h)
+    assert torch.equal(g, want[0]) and torch.equal(h, want[1])
