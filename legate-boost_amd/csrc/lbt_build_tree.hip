@@ -1698,7 +1698,7 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     st.rp         = ar.take<int32_t>(F + 1);
     st.chunk_sums = ar.take<double>(2 * ((N * K + 4095) / 4096));
     st.q          = ar.take<int2>(static_cast<size_t>(K) * st.pitch);
-    st.row_node   = ar.take<uint16_t>(st.pitch);
+    for (auto& nodes : st.row_node) nodes = ar.take<uint16_t>(st.pitch);
     st.q_stats    = ar.take<unsigned long long>(4);
     if (hist != nullptr) {
       st.hist[0]  = L.hist;

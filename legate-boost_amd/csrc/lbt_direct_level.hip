@@ -239,7 +239,7 @@ __device__ __forceinline__ Found scan_feature_estimated(const DirectLevel& a, co
       }
       const float pl = static_cast<float>(lh) + extra, pr = static_cast<float>(all_h - lh) + extra;
       const float sum      = __builtin_fmaf(gl * gl, pr, gr * gr * pl) * __builtin_amdgcn_rcpf(pl * pr);
-      const float estimate = (h[u] != 0) & (lh != all_h) ? sum : -1.0f;
+      const float estimate = ((h[u] != 0) & (lh != all_h)) ? sum : -1.0f;
       const bool more      = estimate > most;
       second = __builtin_fmaxf(second, __builtin_fminf(most, estimate));
       most   = __builtin_fmaxf(most, estimate);

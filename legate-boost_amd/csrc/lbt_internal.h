@@ -532,7 +532,7 @@ constexpr int kSmallMaxDepth   = 13;
 struct SmallCand {
   double gain;
   uint32_t key;  // order among equal gains, larger wins; 0: no candidate
-  int32_t rel;   // bin of the feature
+  int32_t rel;   // bin of the feature (the builder for medium sizes keeps a flag with it)
 };
 
 // Device buffers of a build, carved from the caller's workspace.
@@ -586,7 +586,7 @@ struct MidTreeState {
   int32_t* rp;            // [F + 1]
   double* chunk_sums;     // [2][chunks of 4096 entries]
   int2* q;                // [K][pitch]
-  uint16_t* row_node;     // [pitch] node of the level, 0xffff: none
+  uint16_t* row_node[2];  // [pitch] node of the level, 0xffff: none; of the root in the first one
   unsigned long long* q_stats;  // [4] sum of the positive rounded grads, of the negative ones, flags
   unsigned long long* images;   // packed histograms of the row ranges
   I64Pair* hist[2];       // scanned histograms, [node][K][F][S]; level d in hist[d & 1]

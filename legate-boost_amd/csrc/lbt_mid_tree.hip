@@ -13,7 +13,8 @@
 //   mid_scan_kernel       a workgroup = (pair of siblings, feature): adds the row ranges' images, running
 //                         sums, the sibling as parent minus node, gains (build_tree.cu:597-740)
 //   mid_apply_kernel      best features, the nodes' outputs and children (build_tree.cu:740-782), new node
-//                         of every row
+//                         of every row; where few workgroups share a range of rows, the next level's histogram
+//                         workgroups do that for themselves instead (a launch less)
 //
 // The reference leaves a bin as it was accumulated where neither half of its running sum is positive
 // (build_tree.cu:645). With hessians that are rounded to 0 or more, that is a bin in front of which no row of
@@ -39,6 +40,8 @@ constexpr int kRowsBin  = 256;   // rows of a binning tile
 constexpr int kQuantPer = 8192;  // entries a workgroup rounds
 constexpr int kRowsApply = 4 * kWide;
 constexpr size_t kHistLds = 128 * 1024;
+constexpr int64_t kNodesMost = 2500000;  // rows times workgroups that find the nodes of the same ones (nodes_with_histograms)
+constexpr int kCandsMost     = 4096;     // candidates a histogram workgroup goes through for that (64 KB)
 
 struct MidArgs {
   int N, F, K, S;
@@ -166,7 +169,7 @@ __global__ void __launch_bounds__(kWide)
     a.gain[i]    = 0.0;
   }
   // all rows start in the root; the places behind the last row belong to no node
-  for (int64_t i = first; i < st.pitch; i += stride) st.row_node[i] = i < a.N ? 0 : kNone;
+  for (int64_t i = first; i < st.pitch; i += stride) st.row_node[0][i] = i < a.N ? 0 : kNone;
   if (first <= a.max_depth) st.live[first] = first == 0 ? 1 : 0;
   if (first < 4) st.q_stats[first] = 0;
 }
@@ -377,28 +380,147 @@ __device__ __forceinline__ int built_of_pair(const I64Pair* __restrict__ node_su
   return hl < hr ? 2 * pair : 2 * pair + 1;
 }
 
+// Beside the bin of a candidate: its left child has the smaller hessian of the two, and is the one that is accumulated.
+constexpr int kLeftSmaller = 1 << 30;
+
+// The split of node j of the level by 1 << lanes_log lanes of a wave (`sub` numbers them), and, if `write`,
+// what follows from it: the node's outputs, its children's sums and leaf values. x: feature, -1 for a leaf;
+// y: its last bin that goes left (kLeftSmaller with it: see there). Lanes whose j is no node call it too (j < 0).
+__device__ __forceinline__ int2 decide_node(const MidArgs& a, const MidTreeState& st, const LevelPlan& p, int j, int sub,
+                                            int lanes, bool write)
+{
+  const int node = p.level_first + j;
+  double best    = 0.0;
+  unsigned key   = 0;
+  int ft = 0, rel = 0;
+  auto take = [&](double gain_o, unsigned key_o, int ft_o, int rel_o) {
+    const bool better = gain_o > best || (gain_o == best && key_o > key);
+    best = better ? gain_o : best;
+    key  = better ? key_o : key;
+    ft   = better ? ft_o : ft;
+    rel  = better ? rel_o : rel;
+  };
+  const bool here = j >= 0 && st.node_sums[static_cast<int64_t>(node) * a.K].hess > 0;
+  if (here) {
+    const SmallCand* c = st.cand + static_cast<int64_t>(j) * a.F;
+    for (int i = sub; i < a.F; i += lanes) {
+      const SmallCand o = c[i];
+      take(o.gain, o.key, i, o.rel);
+    }
+  }
+  if (lanes == 64) wave_best_split(best, key, ft, rel);
+  for (int off = lanes == 64 ? 0 : lanes >> 1; off >= 1; off >>= 1) {
+    const double g   = __shfl_xor(best, off, 64);
+    const unsigned o = static_cast<unsigned>(__shfl_xor(static_cast<int>(key), off, 64));
+    const int f_o = __shfl_xor(ft, off, 64), r_o = __shfl_xor(rel, off, 64);
+    take(g, o, f_o, r_o);
+  }
+  const bool splits = here && key != 0 && best > 1e-5;
+  if (write && j >= 0) {
+    const double inv_g = st.scales[2], inv_h = st.scales[3];
+    if (p.depth == 0)
+      for (int k = sub; k < a.K; k += lanes) {
+        const I64Pair ns = st.node_sums[k];
+        const double G = static_cast<double>(ns.grad) * inv_g, H = static_cast<double>(ns.hess) * inv_h;
+        a.leaf[k]      = calculate_leaf_value(G, H, a.l1, a.l2);
+        a.hessian[k]   = H;
+      }
+    if (splits) {
+      const int64_t fs = static_cast<int64_t>(a.F) * a.S;
+      const int lc = left_child(node), rc = right_child(node);
+      const I64Pair* h = st.hist[p.depth & 1] + static_cast<int64_t>(j) * a.K * fs + static_cast<int64_t>(ft) * a.S + (rel & ~kLeftSmaller);
+      for (int k = sub; k < a.K; k += lanes) {
+        const int64_t at = static_cast<int64_t>(node) * a.K + k, l = static_cast<int64_t>(lc) * a.K + k,
+                      r = static_cast<int64_t>(rc) * a.K + k;
+        const I64Pair ns = st.node_sums[at], ls = h[k * fs];
+        const I64Pair rs{ns.grad - ls.grad, ns.hess - ls.hess};
+        const double lg = static_cast<double>(ls.grad) * inv_g, lh = static_cast<double>(ls.hess) * inv_h;
+        const double rg = static_cast<double>(rs.grad) * inv_g, rh = static_cast<double>(rs.hess) * inv_h;
+        st.node_sums[l] = ls;
+        st.node_sums[r] = rs;
+        a.leaf[l]       = calculate_leaf_value(lg, lh, a.l1, a.l2);
+        a.leaf[r]       = calculate_leaf_value(rg, rh, a.l1, a.l2);
+        a.hessian[l]    = lh;
+        a.hessian[r]    = rh;
+      }
+      if (sub == 0) {
+        a.feature[node] = ft;
+        a.split[node]   = st.proposals[static_cast<int64_t>(ft) * a.S + (rel & ~kLeftSmaller)];
+        a.gain[node]    = best;
+        st.live[p.depth + 1] = 1;
+      }
+    }
+  }
+  return make_int2(splits ? ft : -1, rel);
+}
+
+// Four rows in a row, from r on, in the nodes node[] of a level (kNone: in none) with the splits s_split: their nodes of the
+// next level, kNone where a row ends.
+template <typename BinT>
+struct RowSplits {
+  unsigned next[4];
+  int2 sp[4];
+  __device__ __forceinline__ RowSplits(const MidArgs& a, const MidTreeState& st, const int2* s_split, const unsigned (&node)[4], int r)
+  {
+    const BinT* const bins = static_cast<const BinT*>(st.bins);
+    int bin[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      sp[u]  = node[u] != kNone ? s_split[node[u]] : make_int2(-1, 0);
+      bin[u] = sp[u].x >= 0 ? static_cast<int>(bins[static_cast<int64_t>(sp[u].x) * st.pitch + r + u]) : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      next[u] = sp[u].x >= 0 ? 2 * node[u] + (bin[u] <= (sp[u].y & ~kLeftSmaller) ? 0u : 1u) : kNone;
+  }
+  // the nodes in which rows end: all of them at the last level
+  __device__ __forceinline__ void store_leaves(const MidArgs& a, const LevelPlan& p, const unsigned (&node)[4], int r, bool last) const
+  {
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (a.row_leaf != nullptr && node[u] != kNone && (sp[u].x < 0 || last))
+        a.row_leaf[r + u] = sp[u].x < 0 ? p.level_first + static_cast<int>(node[u]) : 2 * p.level_first + 1 + static_cast<int>(next[u]);
+  }
+};
+
+// Where a level's histogram workgroups take the rows' nodes from. kCarried: row_node holds this level's. kDecide: it holds the
+// parents', whose splits every workgroup finds for itself. kDecided: the same with the splits of mid_decide_kernel.
+// Finding splits and bins takes a workgroup two loads one after the other (2 us), a launch of mid_apply_kernel 6 to 7.
+enum class Nodes { kCarried, kDecide, kDecided };
+
 // A packed word holds the sum of grads in its upper and the sum of hessians in its lower half. Rounded
 // hessians are not negative here and sum up to less than 2^32. The grads of all rows sum up to -down and +up
 // with up + down < 2^32, so a sum that left the 32 bits is recognised by lying outside these limits
 // (decode_grad).
-template <typename BinT>
+template <typename BinT, Nodes kNodes>
 __global__ void __launch_bounds__(kWide)
-  mid_histogram_kernel(MidArgs a, MidTreeState st, LevelPlan p)
+  mid_histogram_kernel(MidArgs a, MidTreeState st, LevelPlan p, LevelPlan above, int lanes_log, int writers,
+                       const uint16_t* __restrict__ from, uint16_t* __restrict__ to)
 {
+  constexpr bool kCarried = kNodes == Nodes::kCarried;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   unsigned long long* s_hist = reinterpret_cast<unsigned long long*>(smem_raw);  // [fw][bw][S]
   __shared__ uint16_t s_slot[kMidMaxLevelNodes];                                 // node -> its histogram here, kNone: none
+  __shared__ int2 s_split[kCarried ? 1 : kMidMaxLevelNodes / 2];                 // of the parents
   const int tid = threadIdx.x;
+  if (kNodes == Nodes::kDecide && static_cast<int>(blockIdx.x) < writers) {
+    // what follows from the parents' splits
+    if (level_is_empty(st, above.depth)) return;
+    const int j = static_cast<int>(blockIdx.x * kWide + threadIdx.x) >> lanes_log;
+    decide_node(a, st, above, j < above.n_nodes ? j : -1, tid & ((1 << lanes_log) - 1), 1 << lanes_log, true);
+    return;
+  }
+  const int block = static_cast<int>(blockIdx.x) - writers;
   // ranges of rows vary fastest over the XCDs, so that one range's workgroups share an L2
   const int lanes8 = p.chunks >= 8 ? 8 : 1;
-  const int low = blockIdx.x % lanes8;
-  int rest      = blockIdx.x / lanes8;
+  const int low = block % lanes8;
+  int rest      = block / lanes8;
   const int inner = p.n_fb * p.n_bb * a.K;
   const int chunk = rest / inner * lanes8 + low;
   rest            = rest % inner;
   if (chunk >= p.chunks) return;
   const int k = rest % a.K, fb = rest / a.K % p.n_fb, bb = rest / a.K / p.n_fb;
-  const bool empty = level_is_empty(st, p.depth);
+  const bool empty = level_is_empty(st, kCarried ? p.depth : above.depth);
   if (p.depth == 0 && blockIdx.x == 0 && tid == 0) {
     __hip_atomic_store(a.answer + 1, (static_cast<unsigned long long>(a.tag) << 32) | static_cast<unsigned>(st.rp[a.F]),
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -408,9 +530,23 @@ __global__ void __launch_bounds__(kWide)
   if (empty) return;
   const int f0 = fb * p.fw, nf = min(p.fw, a.F - f0);
   const int b0 = bb * p.bw, nb = min(p.bw, p.built - b0);
+  if constexpr (kNodes == Nodes::kDecided)
+    for (int j = tid; j < above.n_nodes; j += kWide) s_split[j] = st.splits[j];
+  if constexpr (kNodes == Nodes::kDecide) {
+    const int lanes = 1 << lanes_log, sub = tid & (lanes - 1);
+    for (int j0 = 0; j0 < above.n_nodes; j0 += kWide >> lanes_log) {
+      const int j   = j0 + (tid >> lanes_log);
+      const int2 sp = decide_node(a, st, above, j < above.n_nodes ? j : -1, sub, lanes, false);
+      if (sub == 0 && j < above.n_nodes) s_split[j] = sp;
+    }
+  }
+  if constexpr (!kCarried) __syncthreads();
   for (int j = tid; j < p.n_nodes; j += kWide) {
     int slot = kNone;
-    if (p.depth == 0)
+    if constexpr (!kCarried) {
+      const int2 sp = s_split[j / 2];
+      if (j / 2 >= b0 && j / 2 < b0 + nb && sp.x >= 0 && (j & 1) == ((sp.y & kLeftSmaller) != 0 ? 0 : 1)) slot = j / 2 - b0;
+    } else if (p.depth == 0)
       slot = 0;
     else if (j / 2 >= b0 && j / 2 < b0 + nb && built_of_pair(st.node_sums, p.level_first, j / 2, a.K) == j)
       slot = j / 2 - b0;
@@ -422,7 +558,7 @@ __global__ void __launch_bounds__(kWide)
   const BinT* const bins = static_cast<const BinT*>(st.bins) + static_cast<int64_t>(f0) * st.pitch;
   const int2* const q    = st.q + static_cast<int64_t>(k) * st.pitch;
   for (int r = r_begin + 4 * tid; r < r_end; r += 4 * kWide) {
-    const uint2 nd = *reinterpret_cast<const uint2*>(st.row_node + r);
+    const uint2 nd = *reinterpret_cast<const uint2*>(from + r);
     const uint4 qa = *reinterpret_cast<const uint4*>(q + r), qb = *reinterpret_cast<const uint4*>(q + r + 2);
     uint32_t w[kMaxFw][sizeof(BinT)];
 #pragma unroll
@@ -432,7 +568,16 @@ __global__ void __launch_bounds__(kWide)
 #pragma unroll
         for (int u = 0; u < static_cast<int>(sizeof(BinT)); u++) w[i][u] = src[u];
       }
-    const unsigned node[4] = {nd.x & 0xffffu, nd.x >> 16, nd.y & 0xffffu, nd.y >> 16};
+    unsigned node[4] = {nd.x & 0xffffu, nd.x >> 16, nd.y & 0xffffu, nd.y >> 16};
+    if constexpr (!kCarried) {
+      const RowSplits<BinT> rows(a, st, s_split, node, r);
+      if (fb == 0 && bb == 0 && k == 0) {
+        *reinterpret_cast<uint2*>(to + r) = make_uint2(rows.next[0] | rows.next[1] << 16, rows.next[2] | rows.next[3] << 16);
+        rows.store_leaves(a, above, node, r, false);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) node[u] = rows.next[u];
+    }
     const uint32_t qg[4] = {qa.x, qa.z, qb.x, qb.z}, qh[4] = {qa.y, qa.w, qb.y, qb.w};
 #pragma unroll
     for (int u = 0; u < 4; u++) {
@@ -483,6 +628,7 @@ __global__ void __launch_bounds__(kScan)
   __shared__ I64Pair s_carry[kMidMaxOutputs];
   __shared__ double s_best[2][kScan / 64];
   __shared__ unsigned s_bkey[2][kScan / 64];
+  __shared__ int s_less[2][kScan / 64];
   const int f = blockIdx.x % a.F, pair = blockIdx.x / a.F;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   if (level_is_empty(st, p.depth)) return;
@@ -510,11 +656,13 @@ __global__ void __launch_bounds__(kScan)
   const I64Pair* const parent = st.hist[(p.depth & 1) ^ 1] + static_cast<int64_t>(pair) * a.K * fs + static_cast<int64_t>(f) * a.S;
   double best_n = 0.0, best_s = 0.0;
   unsigned key_n = 0, key_s = 0;
+  bool less_n = false, less_s = false;  // the best split's left child has the smaller hessian (of the first output)
   for (int base = 0; base < n_bins; base += kScan) {
     const int bin = base + tid;
     const bool in = bin < n_bins;
     double gain_n = 0.0, gain_s = 0.0;
     bool dead_n = !in, dead_s = !in || root;
+    bool left_n = false, left_s = false;
     for (int k = 0; k < a.K; k++) {
       I64Pair v{0, 0}, pv{0, 0};
       const I64Pair ns = st.node_sums[static_cast<int64_t>(p.level_first + node) * a.K + k];
@@ -566,6 +714,10 @@ __global__ void __launch_bounds__(kScan)
       const double s_right = leaf_gain_select(static_cast<double>(sr.grad) * inv_g, static_cast<double>(sr.hess) * inv_h, a.l1, reg);
       const double n_own = leaf_gain_select(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, a.l1, reg);
       const double s_own = leaf_gain_select(static_cast<double>(ss.grad) * inv_g, static_cast<double>(ss.hess) * inv_h, a.l1, reg);
+      if (k == 0) {
+        left_n = nv.hess < nr.hess;
+        left_s = sv.hess < sr.hess;
+      }
       dead_n |= nv.hess <= 0 || nr.hess <= 0;
       dead_s |= sv.hess <= 0 || sr.hess <= 0;
       gain_n += 0.5 * (n_left + n_right - n_own) - a.min_split_gain;
@@ -586,100 +738,39 @@ __global__ void __launch_bounds__(kScan)
     const bool take_s = !dead_s && gain_s > 0 && (gain_s > best_s || (gain_s == best_s && key > key_s));
     best_n = take_n ? gain_n : best_n;
     key_n  = take_n ? key : key_n;
+    less_n = take_n ? left_n : less_n;
     best_s = take_s ? gain_s : best_s;
     key_s  = take_s ? key : key_s;
+    less_s = take_s ? left_s : less_s;
     if (base + kScan < n_bins) __syncthreads();
   }
+  const double own_n = best_n, own_s = best_s;
+  const unsigned own_key_n = key_n, own_key_s = key_s;
   wave_best_key(best_n, key_n);
   wave_best_key(best_s, key_s);
+  less_n = __any(less_n && own_key_n == key_n && own_n == best_n);  // (no two lanes have one key)
+  less_s = __any(less_s && own_key_s == key_s && own_s == best_s);
   if (lane == 0) {
     s_best[0][wave] = best_n;
     s_bkey[0][wave] = key_n;
+    s_less[0][wave] = less_n ? kLeftSmaller : 0;
     s_best[1][wave] = best_s;
     s_bkey[1][wave] = key_s;
+    s_less[1][wave] = less_s ? kLeftSmaller : 0;
   }
   __syncthreads();
   if (tid < (root ? 1 : 2)) {
     double best  = 0.0;
     unsigned key = 0;
+    int less     = 0;
     for (int w = 0; w < kScan / 64; w++) {
       const bool take = s_best[tid][w] > best || (s_best[tid][w] == best && s_bkey[tid][w] > key);
       best = take ? s_best[tid][w] : best;
       key  = take ? s_bkey[tid][w] : key;
+      less = take ? s_less[tid][w] : less;
     }
-    st.cand[static_cast<int64_t>(tid == 0 ? node : sib) * a.F + f] = SmallCand{best, key, key != 0 ? bin_of_tie_key(key) - rp : 0};
+    st.cand[static_cast<int64_t>(tid == 0 ? node : sib) * a.F + f] = SmallCand{best, key, key != 0 ? (bin_of_tie_key(key) - rp) | less : 0};
   }
-}
-
-// The split of node j of the level by 1 << lanes_log lanes of a wave (`sub` numbers them), and, if `write`,
-// what follows from it: the node's outputs, its children's sums and leaf values. x: feature, -1 for a leaf;
-// y: its last bin that goes left. Lanes whose j is no node call it too (j < 0).
-__device__ __forceinline__ int2 decide_node(const MidArgs& a, const MidTreeState& st, const LevelPlan& p, int j, int sub,
-                                            int lanes, bool write)
-{
-  const int node = p.level_first + j;
-  double best    = 0.0;
-  unsigned key   = 0;
-  int ft = 0, rel = 0;
-  auto take = [&](double gain_o, unsigned key_o, int ft_o, int rel_o) {
-    const bool better = gain_o > best || (gain_o == best && key_o > key);
-    best = better ? gain_o : best;
-    key  = better ? key_o : key;
-    ft   = better ? ft_o : ft;
-    rel  = better ? rel_o : rel;
-  };
-  const bool here = j >= 0 && st.node_sums[static_cast<int64_t>(node) * a.K].hess > 0;
-  if (here) {
-    const SmallCand* c = st.cand + static_cast<int64_t>(j) * a.F;
-    for (int i = sub; i < a.F; i += lanes) {
-      const SmallCand o = c[i];
-      take(o.gain, o.key, i, o.rel);
-    }
-  }
-  if (lanes == 64) wave_best_split(best, key, ft, rel);
-  for (int off = lanes == 64 ? 0 : lanes >> 1; off >= 1; off >>= 1) {
-    const double g   = __shfl_xor(best, off, 64);
-    const unsigned o = static_cast<unsigned>(__shfl_xor(static_cast<int>(key), off, 64));
-    const int f_o = __shfl_xor(ft, off, 64), r_o = __shfl_xor(rel, off, 64);
-    take(g, o, f_o, r_o);
-  }
-  const bool splits = here && key != 0 && best > 1e-5;
-  if (write && j >= 0) {
-    const double inv_g = st.scales[2], inv_h = st.scales[3];
-    if (p.depth == 0)
-      for (int k = sub; k < a.K; k += lanes) {
-        const I64Pair ns = st.node_sums[k];
-        const double G = static_cast<double>(ns.grad) * inv_g, H = static_cast<double>(ns.hess) * inv_h;
-        a.leaf[k]      = calculate_leaf_value(G, H, a.l1, a.l2);
-        a.hessian[k]   = H;
-      }
-    if (splits) {
-      const int64_t fs = static_cast<int64_t>(a.F) * a.S;
-      const int lc = left_child(node), rc = right_child(node);
-      const I64Pair* h = st.hist[p.depth & 1] + static_cast<int64_t>(j) * a.K * fs + static_cast<int64_t>(ft) * a.S + rel;
-      for (int k = sub; k < a.K; k += lanes) {
-        const int64_t at = static_cast<int64_t>(node) * a.K + k, l = static_cast<int64_t>(lc) * a.K + k,
-                      r = static_cast<int64_t>(rc) * a.K + k;
-        const I64Pair ns = st.node_sums[at], ls = h[k * fs];
-        const I64Pair rs{ns.grad - ls.grad, ns.hess - ls.hess};
-        const double lg = static_cast<double>(ls.grad) * inv_g, lh = static_cast<double>(ls.hess) * inv_h;
-        const double rg = static_cast<double>(rs.grad) * inv_g, rh = static_cast<double>(rs.hess) * inv_h;
-        st.node_sums[l] = ls;
-        st.node_sums[r] = rs;
-        a.leaf[l]       = calculate_leaf_value(lg, lh, a.l1, a.l2);
-        a.leaf[r]       = calculate_leaf_value(rg, rh, a.l1, a.l2);
-        a.hessian[l]    = lh;
-        a.hessian[r]    = rh;
-      }
-      if (sub == 0) {
-        a.feature[node] = ft;
-        a.split[node]   = st.proposals[static_cast<int64_t>(ft) * a.S + rel];
-        a.gain[node]    = best;
-        st.live[p.depth + 1] = 1;
-      }
-    }
-  }
-  return make_int2(splits ? ft : -1, rel);
 }
 
 // Splits of a level of many nodes, one group of lanes per node.
@@ -697,13 +788,13 @@ __global__ void __launch_bounds__(kScan)
 // saves a launch) and the nodes' outputs are dealt to the workgroups.
 template <typename BinT, bool kDecided>
 __global__ void __launch_bounds__(kWide)
-  mid_apply_kernel(MidArgs a, MidTreeState st, LevelPlan p, int lanes_log)
+  mid_apply_kernel(MidArgs a, MidTreeState st, LevelPlan p, int lanes_log, uint16_t* row_node)
 {
   __shared__ int2 s_split[kMidMaxLevelNodes];
   const int tid = threadIdx.x;
   const int r   = blockIdx.x * kRowsApply + 4 * tid;
   uint2 nd      = make_uint2(0xffffffffu, 0xffffffffu);
-  if (r < a.N) nd = *reinterpret_cast<const uint2*>(st.row_node + r);
+  if (r < a.N) nd = *reinterpret_cast<const uint2*>(row_node + r);
   if (level_is_empty(st, p.depth)) return;
   if constexpr (kDecided) {
     for (int j = tid; j < p.n_nodes; j += kWide) s_split[j] = st.splits[j];
@@ -718,35 +809,19 @@ __global__ void __launch_bounds__(kWide)
   }
   __syncthreads();
   if (r >= a.N) return;
-  const BinT* const bins = static_cast<const BinT*>(st.bins);
   const unsigned node[4] = {nd.x & 0xffffu, nd.x >> 16, nd.y & 0xffffu, nd.y >> 16};
-  int2 sp[4];
-  int bin[4];
-#pragma unroll
-  for (int u = 0; u < 4; u++) {
-    sp[u]  = node[u] != kNone ? s_split[node[u]] : make_int2(-1, 0);
-    bin[u] = sp[u].x >= 0 ? static_cast<int>(bins[static_cast<int64_t>(sp[u].x) * st.pitch + r + u]) : 0;
-  }
-  unsigned next[4];
-#pragma unroll
-  for (int u = 0; u < 4; u++) {
-    next[u] = kNone;
-    if (node[u] != kNone) {
-      const unsigned child = 2 * node[u] + (bin[u] <= sp[u].y ? 0u : 1u);
-      if (sp[u].x >= 0) next[u] = child;
-      if (a.row_leaf != nullptr && (sp[u].x < 0 || p.last))
-        a.row_leaf[r + u] = sp[u].x < 0 ? p.level_first + static_cast<int>(node[u])
-                                        : 2 * p.level_first + 1 + static_cast<int>(child);
-    }
-  }
-  if (!p.last) *reinterpret_cast<uint2*>(st.row_node + r) = make_uint2(next[0] | next[1] << 16, next[2] | next[3] << 16);
+  const RowSplits<BinT> rows(a, st, s_split, node, r);
+  rows.store_leaves(a, p, node, r, p.last);
+  if (!p.last)
+    *reinterpret_cast<uint2*>(row_node + r) = make_uint2(rows.next[0] | rows.next[1] << 16, rows.next[2] | rows.next[3] << 16);
 }
 
 // For the profiler: the rows of the level's nodes and of those that are accumulated.
-__global__ void __launch_bounds__(kScan) mid_count_kernel(MidArgs a, MidTreeState st, LevelPlan p, LevelMeta* total)
+__global__ void __launch_bounds__(kScan) mid_count_kernel(MidArgs a, MidTreeState st, LevelPlan p, const uint16_t* row_node,
+                                                         LevelMeta* total)
 {
   const int r    = blockIdx.x * kScan + threadIdx.x;
-  const int node = r < a.N ? st.row_node[r] : kNone;
+  const int node = r < a.N ? row_node[r] : kNone;
   const bool has = node != kNone && !level_is_empty(st, p.depth);
   const bool built = has && (p.depth == 0 || built_of_pair(st.node_sums, p.level_first, node >> 1, a.K) == node);
   const unsigned long long all = __ballot(has), some = __ballot(built);
@@ -849,36 +924,74 @@ bool mid_beats_small(int64_t N, int F, int K, int max_depth, int S)
   return 1.15 * mid_us < small_us;
 }
 
+// Whether the workgroups of level p's histograms find the nodes of their rows for themselves, which saves the launch that does.
+// All workgroups of a range of rows do so for the same rows, a byte gathered per row and workgroup: up to 2.5 million
+// such visits it pays. Fits with the launch and without, us: 100,000 x 32, depth 6, 10 rounds 1885 and 1749; 300,000 x 16 with 128
+// samples, depth 8, 4 rounds 1133 and 1066; 15,000 x 8 f64, depth 10, 5 rounds 1505 and 1342; 50,000 x 60 with 512 samples, depth 7,
+// 4 rounds 1209 and 1137; with levels of 8 million visits 1,000,000 x 30, depth 8, 3 rounds 1395 and 1441 (not taken).
+static bool nodes_with_histograms(const MidArgs& a, const LevelPlan& p)
+{
+  return p.depth > 0 && static_cast<int64_t>(p.n_fb) * p.n_bb * a.K * a.N <= kNodesMost;
+}
+
+template <typename BinT, Nodes kNodes>
+static int launch_histograms(hipStream_t stream, const MidTreeState& st, const MidArgs& a, const LevelPlan& p, const LevelPlan& above,
+                             int lanes_log, const uint16_t* from, uint16_t* to)
+{
+  ProfScope ps(LBT_PROF_HISTOGRAM, stream, 0.0, p.depth);
+  static std::atomic<bool> attr_set[kMaxDevices] = {};
+  LBT_TRY((allow_dynamic_lds(mid_histogram_kernel<BinT, kNodes>, kHistLds + 4096, attr_set)));
+  const int lanes8    = p.chunks >= 8 ? 8 : 1;
+  const int writers   = kNodes == Nodes::kDecide ? ((above.n_nodes << lanes_log) + kWide - 1) / kWide : 0;
+  const unsigned grid = static_cast<unsigned>((p.chunks + lanes8 - 1) / lanes8 * lanes8 * p.n_fb * p.n_bb * a.K + writers);
+  mid_histogram_kernel<BinT, kNodes><<<grid, kWide, static_cast<size_t>(p.fw) * p.bw * a.S * 8, stream>>>(
+    a, st, p, above, lanes_log, writers, from, to);
+  return LBT_OK;
+}
+
 template <typename T, typename BinT>
 static int queue_levels(hipStream_t stream, const MidTreeState& st, const MidArgs& a, const DeviceAnswer& answer,
                         LevelMeta* level_totals)
 {
   int lanes_log = 0;
   while (lanes_log < 6 && (1 << lanes_log) < a.F) lanes_log++;
+  int cur    = 0;                     // row_node[cur] holds the rows' nodes of the level, or of the one above it
+  Nodes how  = Nodes::kCarried;
+  LevelPlan above{};
   for (int d = 0; d < a.max_depth && (d == 0 || !answer.declined()); d++) {
     const LevelPlan p = plan_level(a.N, a.F, a.K, a.S, d, a.max_depth);
-    {
-      ProfScope ps(LBT_PROF_HISTOGRAM, stream, 0.0, d);
-      static std::atomic<bool> attr_set[kMaxDevices] = {};
-      LBT_TRY(allow_dynamic_lds(mid_histogram_kernel<BinT>, kHistLds + 4096, attr_set));
-      const int lanes8    = p.chunks >= 8 ? 8 : 1;
-      const unsigned grid = static_cast<unsigned>((p.chunks + lanes8 - 1) / lanes8 * lanes8 * p.n_fb * p.n_bb * a.K);
-      mid_histogram_kernel<BinT><<<grid, kWide, static_cast<size_t>(p.fw) * p.bw * a.S * 8, stream>>>(a, st, p);
+    const uint16_t* const from = st.row_node[cur];
+    uint16_t* const to         = st.row_node[cur ^ 1];
+    switch (how) {
+      case Nodes::kCarried: LBT_TRY((launch_histograms<BinT, Nodes::kCarried>(stream, st, a, p, above, lanes_log, from, nullptr))); break;
+      case Nodes::kDecide: LBT_TRY((launch_histograms<BinT, Nodes::kDecide>(stream, st, a, p, above, lanes_log, from, to))); break;
+      case Nodes::kDecided: LBT_TRY((launch_histograms<BinT, Nodes::kDecided>(stream, st, a, p, above, lanes_log, from, to))); break;
     }
+    if (how != Nodes::kCarried) cur ^= 1;
     if (level_totals != nullptr)
-      mid_count_kernel<<<static_cast<unsigned>((a.N + kScan - 1) / kScan), kScan, 0, stream>>>(a, st, p, level_totals + d);
+      mid_count_kernel<<<static_cast<unsigned>((a.N + kScan - 1) / kScan), kScan, 0, stream>>>(a, st, p, st.row_node[cur], level_totals + d);
     {
       ProfScope ps(LBT_PROF_SCAN, stream);
       mid_scan_kernel<<<static_cast<unsigned>(p.built) * a.F, kScan, 0, stream>>>(a, st, p);
     }
     ProfScope ps(LBT_PROF_POSITIONS, stream);
     const unsigned grid = static_cast<unsigned>((a.N + kRowsApply - 1) / kRowsApply);
-    if (p.n_nodes <= 2 * (kWide >> lanes_log)) {
-      mid_apply_kernel<BinT, false><<<grid, kWide, 0, stream>>>(a, st, p, lanes_log);
-    } else {
+    const bool later    = !p.last && nodes_with_histograms(a, plan_level(a.N, a.F, a.K, a.S, d + 1, a.max_depth));
+    // few nodes: every workgroup that asks for the splits finds them for itself (it saves a launch)
+    const bool few = p.n_nodes <= 2 * (kWide >> lanes_log);
+    if (!few || (later && static_cast<int64_t>(p.n_nodes) * a.F > kCandsMost)) {
       mid_decide_kernel<<<((p.n_nodes << lanes_log) + kScan - 1) / kScan, kScan, 0, stream>>>(a, st, p, lanes_log);
-      mid_apply_kernel<BinT, true><<<grid, kWide, 0, stream>>>(a, st, p, lanes_log);
+      how = Nodes::kDecided;
+    } else {
+      how = Nodes::kDecide;
     }
+    above = p;
+    if (later) continue;
+    if (how == Nodes::kDecide)
+      mid_apply_kernel<BinT, false><<<grid, kWide, 0, stream>>>(a, st, p, lanes_log, st.row_node[cur]);
+    else
+      mid_apply_kernel<BinT, true><<<grid, kWide, 0, stream>>>(a, st, p, lanes_log, st.row_node[cur]);
+    how = Nodes::kCarried;
   }
   LBT_HIP(hipGetLastError());
   return LBT_OK;

@@ -206,6 +206,32 @@ def test_medium_sizes(n, f, k, depth, s, dtype, options):
         gu.check_row_leaf(got, X)
 
 
+@pytest.mark.parametrize("n,f,k,depth,s", [(9001, 43, 1, 9, 256), (8500, 260, 1, 5, 64), (156250, 64, 1, 4, 64), (156251, 64, 1, 4, 64),
+                                           (20002, 10, 2, 8, 128), (30011, 17, 3, 6, 256)])
+def test_medium_sizes_whose_rows_stop_at_every_level(n, f, k, depth, s):
+    """Histogram workgroups that find their rows' nodes, by themselves or after the launch that decides many nodes, either side
+    of the number of rows where they do, in turn with levels that do not: rows end at every level, at most nodes of the last
+    ones no row is left."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + f)
+    X = rs.randn(n, f).astype(np.float32)
+    g, inside = 0.3 * rs.randn(n, k), np.ones(n, bool)
+    for level in range(depth):  # half of what is left is told from the rest, and goes on
+        inside &= X[:, level % f] > (0 if level < f else 0.5)
+        g[:, 0] += inside
+    h = 0.5 + rs.rand(n, k)
+    kw = dict(max_depth=depth, split_samples=s, seed=9, min_split_gain=2.0)
+    cr = orc.build_tree(X, g, h, **kw)
+    got = ops.build_tree(X, g, h, row_leaf=True, **kw)
+    _assert_tree(got, cr)
+    gu.check_row_leaf(got, X)
+    ends = [int((cr.feature[2 ** d - 1:2 ** (d + 1) - 1] < 0).sum()) for d in range(depth)]
+    assert ends[depth // 2] > 0 and int((cr.feature >= 0).sum()) >= depth
+
+
 def test_medium_sizes_under_an_explicit_budget():
     """Budgets either side of what the builder's histograms and images take, in a workspace of the size the query
     names for the budget: the same tree, by that builder or by the general one."""
