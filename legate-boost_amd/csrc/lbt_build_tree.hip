@@ -1669,7 +1669,7 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     st.proposals   = ar.take<double>(static_cast<size_t>(F) * S);
     st.counts      = ar.take<int32_t>(F);
     st.rp          = ar.take<int32_t>(F);
-    st.node_of_pos = ar.take<uint16_t>(st.pitch);
+    for (auto& nodes : st.node_of_pos) nodes = ar.take<uint16_t>(st.pitch);
     st.code        = ar.take<uint8_t>(st.pitch);
     st.seg         = ar.take<int2>(max_nodes);
     st.live        = ar.take<int32_t>(max_depth + 1);
@@ -1677,7 +1677,10 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     st.node_sums   = L.node_sums;
     st.qgh         = L.qgh;
     st.scales      = L.scales;
-    st.cand        = ar.take<SmallCand>(level_nodes * F);
+    const bool decides = K == 1 && F <= kSmallDecideFeatures;
+    st.cand[0]     = ar.take<SmallCand>(level_nodes * F);
+    st.cand[1]     = decides ? ar.take<SmallCand>(level_nodes * F) : st.cand[0];
+    for (auto& left : st.left) left = decides ? ar.take<I64Pair>(level_nodes * F) : nullptr;
   }
   L.mid = MidTreeState{};
   if (mid) {

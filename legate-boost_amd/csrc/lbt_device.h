@@ -77,6 +77,11 @@ __device__ __forceinline__ double wave_read_lane_f64(double v, int src)
   return __longlong_as_double(wave_read_lane(static_cast<int64_t>(__double_as_longlong(v)), src));
 }
 
+// Values that loads bring, when all of them are here: hipcc moves a load behind the branch that is its only use, where a wave
+// then waits for it alone.
+__device__ __forceinline__ void arrived(int2& v) { asm volatile("" : "+v"(v.x), "+v"(v.y)); }
+__device__ __forceinline__ void arrived(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+
 struct Cand {
   double gain;
   int bin;

@@ -536,6 +536,8 @@ struct SmallCand {
 };
 
 // Device buffers of a build, carved from the caller's workspace.
+constexpr int kSmallDecideFeatures = 64;  // a lane each of the wave that decides a node
+
 struct SmallTreeState {
   int64_t pitch;          // elements between the rows of a feature and those of the next (multiple of 8)
   uint32_t* order[2];     // [F][pitch] row | bin << 16 by (node, bin); the order of level d is order[d & 1]
@@ -543,7 +545,7 @@ struct SmallTreeState {
   double* proposals;      // [F][S]
   int32_t* counts;        // [F] proposals
   int32_t* rp;            // [F] first bin of the feature among all bins
-  uint16_t* node_of_pos;  // [pitch] node of the level that holds a place of the order, 0xffff: a leaf's
+  uint16_t* node_of_pos[2];  // [pitch] node of the level that holds a place of the order, 0xffff: a leaf's; the root's in the first one
   uint8_t* code;          // [N] side a row of a split node takes: 1 left, 2 right
   int2* seg;              // [max_nodes] places of a node's rows: the first one, and how many
   int32_t* live;          // [max_depth + 1] the level has nodes
@@ -551,7 +553,8 @@ struct SmallTreeState {
   I64Pair* node_sums;     // [max_nodes][K]
   int2* qgh;              // [N][K]
   double* scales;         // [4]
-  SmallCand* cand;        // [nodes of a level][F]
+  SmallCand* cand[2];     // [nodes of a level][F]
+  I64Pair* left[2];       // the same: what lies left of a candidate; null where no scan decides the level above it
 };
 bool small_tree_fits(int64_t N, int F, int K, int max_depth, int S);
 // n_bins: receives the number of bins of all features (null: not wanted). level_totals: [max_depth], added

@@ -14,7 +14,8 @@
 //                           (a stable partition inside every node), running sums, gains, and the best
 //                           split of the feature per node (build_tree.cu:682-740)
 //   small_apply_kernel      one workgroup per node and level: best feature, the node's outputs and its
-//                           children (build_tree.cu:740-782), the side of each of its rows
+//                           children (build_tree.cu:740-782), the side of each of its rows. Where a level has few
+//                           candidates every scan workgroup of the next one does that for itself (a launch less)
 //
 // The sums are integers, so they do not depend on the order of rows; gains and leaf values are formed
 // by the same functions from the same sums as in the other builder: the trees are identical. One rule of
@@ -24,6 +25,7 @@
 // takes the other builder.
 #include <algorithm>
 #include <limits>
+#include <type_traits>
 
 #include "lbt_device.h"
 #include "lbt_internal.h"
@@ -261,7 +263,7 @@ __global__ void __launch_bounds__(kPrologueThreads)
       a.gain[i]       = 0.0;
       st.seg[i] = make_int2(0, 0);
     }
-  for (int64_t i = first; i < a.N; i += stride) st.node_of_pos[i] = 0;
+  for (int64_t i = first; i < a.N; i += stride) st.node_of_pos[0][i] = 0;
   if (first >= 1 && first <= a.max_depth) st.live[first] = 0;
 }
 
@@ -271,6 +273,20 @@ struct LevelArgs {
   int level_first;  // first node of the level; its node j is level_first + j
   int n_nodes;
   bool last;        // no further level follows
+  const uint16_t* node_in;  // [pitch] node of this level (scan that decides: of the level above) that holds a place
+  uint16_t* node_out;       // scan that decides: of this level
+  const SmallCand* cand_above;   // scan that decides: what the level above found, [node][F]
+  const I64Pair* left_above;     // and what lies left of it
+  SmallCand* cand;          // what this level finds
+  I64Pair* left;            // null: small_apply_kernel follows
+  int lanes_log;            // scan that decides: lanes per node of the level above, log2
+  bool all_bins;            // scan that decides: the bins of all features lie in the LDS
+  double* leaf;
+  int32_t* feature;
+  double* split;
+  double* gain;
+  double* hessian;
+  int32_t* row_leaf;
   unsigned long long* n_bins;  // pinned host memory: the number of all bins (see DeviceAnswer)
   uint32_t tag;
   const uint8_t* feature_set;
@@ -282,9 +298,11 @@ struct LevelArgs {
 template <int kE>
 __device__ __forceinline__ void load_u16(const uint16_t* p, int (&out)[kE])
 {
-  static_assert(kE == 4 || kE == 8, "8 or 16 bytes per thread");
+  static_assert(kE == 2 || kE == 4 || kE == 8, "4, 8 or 16 bytes per thread");
   uint32_t w[kE / 2];
-  if constexpr (kE == 4) {
+  if constexpr (kE == 2) {
+    w[0] = *reinterpret_cast<const uint32_t*>(p);
+  } else if constexpr (kE == 4) {
     const uint2 v = *reinterpret_cast<const uint2*>(p);
     w[0] = v.x, w[1] = v.y;
   } else {
@@ -300,11 +318,23 @@ __device__ __forceinline__ void load_u16(const uint16_t* p, int (&out)[kE])
 template <int kE>
 __device__ __forceinline__ void load_u32(const uint32_t* p, uint32_t (&out)[kE])
 {
+  if constexpr (kE == 2) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    out[0] = v.x, out[1] = v.y;
+  }
 #pragma unroll
   for (int i = 0; i < kE / 4; i++) {
     const uint4 v = reinterpret_cast<const uint4*>(p)[i];
     out[4 * i] = v.x, out[4 * i + 1] = v.y, out[4 * i + 2] = v.z, out[4 * i + 3] = v.w;
   }
+}
+
+template <int kE>
+__device__ __forceinline__ void store_u32(uint32_t* p, const uint32_t (&v)[kE])
+{
+  if constexpr (kE == 2) *reinterpret_cast<uint2*>(p) = make_uint2(v[0], v[1]);
+#pragma unroll
+  for (int i = 0; i < kE / 4; i++) reinterpret_cast<uint4*>(p)[i] = make_uint4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
 }
 
 // Where a split falls among equal gains of a node (cand_better): the largest bin mod 512, counted over all
@@ -333,6 +363,29 @@ __host__ __device__ constexpr size_t small_scan_use(int64_t N, int64_t n_nodes)
   return static_cast<size_t>((N + 1) / 2 * 2 * 8 + small_scan_order(N) * 4 + n_nodes * 12 + (n_nodes / 2 + 1) * 4 + (N + 3) / 4 * 4 + 31) / 16 * 16;
 }
 
+// What a scan that decides needs beside that, of the level above.
+constexpr int kDecidePasses = 2;   // candidates a thread looks at
+constexpr int decide_loads(int threads) { return threads == 1024 ? 4 : 8; }   // 16-byte pieces of all features' bins it stages
+constexpr int kDecideRows  = 4096;  // rows up to which a scan decides: with eight places a thread it gained nothing
+constexpr int kDecideLanes = 4;  // log2 of the fewest lanes a node takes
+
+// The largest value of an aligned group of 16, 32 or 64 lanes, in all of them
+__device__ __forceinline__ unsigned group_max_u32(unsigned v, int lanes_log)
+{
+  auto take = [&](auto ctrl) {
+    const unsigned o = static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), decltype(ctrl)::value, 0xf, 0xf, true));
+    v = o > v ? o : v;
+  };
+  take(std::integral_constant<int, 0x128>{});  // the lanes of a row of 16, turned by 8, 4, 2 and 1
+  take(std::integral_constant<int, 0x124>{});
+  take(std::integral_constant<int, 0x122>{});
+  take(std::integral_constant<int, 0x121>{});
+  if (lanes_log > 4) v = max(v, static_cast<unsigned>(__shfl_xor(static_cast<int>(v), 16, 64)));
+  if (lanes_log > 5) v = max(v, static_cast<unsigned>(__shfl_xor(static_cast<int>(v), 32, 64)));
+  return v;
+}
+__host__ __device__ constexpr size_t small_decide_use(int64_t n_nodes) { return static_cast<size_t>((n_nodes / 2 + 2) / 2 * 2 * (16 + 8 + 8 + 8 + 4) + 16 + 16); }
+
 // kT threads take kE consecutive places of the order each (kT * kE >= N). What a place needs of its row
 // (its pair of the first output, its side) is staged in the LDS in row order: gathered from the L2 these
 // are three scattered accesses per place, and a workgroup's 8192 places then take a level 90 us
@@ -345,10 +398,16 @@ __host__ __device__ constexpr size_t small_scan_use(int64_t N, int64_t n_nodes)
 // cycles or more, and one place after the other was half of the launch on 1000 x 10. With more features than CUs it is
 // the other way round: 64 registers let two workgroups of 1024 threads share a CU, and one place at a time is enough
 // (5000 x 500: 32 us a launch, now 25; with 66 registers it was one workgroup).
-template <int kT, int kE, bool kSingle, int kG, bool kStaged>
+// kDecides: the level above has been scanned, not decided. Every workgroup finds all its splits (a candidate per lane), sums
+// of its children and sides of its rows for itself, feature 0's writes them down. A launch of small_apply_kernel was a third of
+// a level (1000 x 10, depth 8: 4.5 of 12.4 us and the gap in front of it). Fits with such launches and without, us: 1000 x 10 f64,
+// depth 8, 12 rounds 1580 and 1290; 2000 x 16, depth 8, 5 rounds 815 and 720; 4000 x 8, depth 6 860 and 740; 1000 x 40, depth 8 740
+// and 665; 3000 x 60, depth 7 900 and 850. From 4096 rows on (8000 x 30, 7000 x 12, 5000 x 64) it gained nothing.
+template <int kT, int kE, bool kSingle, int kG, bool kStaged, bool kDecides>
 __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
   small_scan_kernel(SmallTreeState st, LevelArgs a)
 {
+  static_assert(!kDecides || (kSingle && kStaged && kG > 1), "one output, nodes in the LDS");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   int2* s_q                  = reinterpret_cast<int2*>(smem_raw);               // [N]
   uint32_t* s_order          = reinterpret_cast<uint32_t*>(s_q + (a.N + 1) / 2 * 2);  // [small_scan_order(N)]
@@ -360,6 +419,13 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
   I64Pair* s_base            = s_ns + a.n_nodes;
   double* s_parent           = reinterpret_cast<double*>(s_base + a.n_nodes);
   int2* s_seg                = reinterpret_cast<int2*>(s_parent + a.n_nodes);
+  const int n_pad            = (a.n_nodes / 2 + 2) / 2 * 2;
+  I64Pair* s_left_above      = reinterpret_cast<I64Pair*>(s_seg + a.n_nodes);    // kDecides, of the level above: [n_pad]
+  int2* s_split              = reinterpret_cast<int2*>(s_left_above + n_pad);
+  int2* s_seg_above          = s_split + n_pad;
+  double* s_gain_above       = reinterpret_cast<double*>(s_seg_above + n_pad);
+  int* s_left_behind         = reinterpret_cast<int*>(s_gain_above + n_pad);
+  uint16_t* s_bins           = reinterpret_cast<uint16_t*>(s_left_behind + (n_pad + 3) / 4 * 4);  // all_bins: [F][pitch]
   __shared__ I64Pair s_pair[2][kT / 64];
   __shared__ int s_wave[kT / 64];
   __shared__ int s_rp;
@@ -367,39 +433,79 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
   const int wave = tid >> 6, lane = tid & 63;
   const int i0   = tid * kE;
   const bool usable = a.feature_set == nullptr || a.feature_set[f] != 0;
-  SmallCand* const out = st.cand + f;  // node j: out[j * F]
+  SmallCand* const out = a.cand + f;  // node j: out[j * F]
   const uint32_t* order_in = st.order[a.depth == 0 ? 0 : (a.depth - 1) & 1] + static_cast<int64_t>(f) * st.pitch;
+  // Places, rows and nodes past the last one are asked for as the last one: hipcc keeps a load that only some lanes ask for
+  // behind a branch, and waits for its answer before the next branch (1000 x 10, scans that decide: 23,000 cycles each, 17,000
+  // without such waits). With eight places a thread many threads have none, and what they ask for costs more.
+  constexpr bool kClamped = kE <= 4;
   uint32_t entry[kE];
-  int node[kE];
+  int node[kE], node_next = kNone;
+  if constexpr (kClamped) {
+    const int i_in = min(i0, static_cast<int>(st.pitch) - kE);
+    load_u32<kE>(order_in + i_in, entry);
+    load_u16<kE>(a.node_in + i_in, node);
+    node_next = a.node_in[min(i0 + kE, a.N - 1)];
+  } else {
 #pragma unroll
-  for (int e = 0; e < kE; e++) {
-    entry[e] = 0;
-    node[e]  = kNone;
+    for (int e = 0; e < kE; e++) {
+      entry[e] = 0;
+      node[e]  = kNone;
+    }
+    if (i0 < a.N) {
+      load_u32<kE>(order_in + i0, entry);
+      load_u16<kE>(a.node_in + i0, node);
+      if (i0 + kE < a.N) node_next = a.node_in[i0 + kE];
+    }
   }
-  int node_next = kNone;
-  if (i0 < a.N) {
-    load_u32<kE>(order_in + i0, entry);
-    load_u16<kE>(st.node_of_pos + i0, node);
-    if (i0 + kE < a.N) node_next = st.node_of_pos[i0 + kE];
-  }
-  const int live = st.live[a.depth];
+  const int live = st.live[kDecides ? a.depth - 1 : a.depth];
   int rp         = a.depth == 0 ? 0 : st.rp[f];  // first bin of the feature among all bins
   const double inv_g = st.scales[2], inv_h = st.scales[3];
   const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
+  // kDecides: what the level above has left, a candidate per lane and pass, a node per thread. (All that a workgroup
+  // reads is asked for before the first answer is waited for: what another XCD wrote takes 3000 cycles to arrive.)
+  constexpr int kPasses = kDecides ? kDecidePasses : 1, kLoads = kDecides ? decide_loads(kT) : 1;
+  const int above_first = (a.level_first - 1) / 2, n_above = a.n_nodes / 2, sub = tid & ((1 << a.lanes_log) - 1);
+  SmallCand cand_of[kPasses];
+  I64Pair left_cand[kPasses], ns_above{0, 0}, base_above{0, 0};
+  int2 seg_of{0, 0};
+  uint4 bins_of[kLoads];
+  const int n16 = a.all_bins ? a.F * static_cast<int>(st.pitch / 8) : 1;
+  if constexpr (kDecides) {
+#pragma unroll
+    for (int p = 0; p < kPasses; p++) {
+      const int j  = min((p * kT + tid) >> a.lanes_log, n_above - 1), at = j * a.F + min(sub, a.F - 1);
+      cand_of[p]   = a.cand_above[at];
+      left_cand[p] = a.left_above[at];
+    }
+    const int above = above_first + min(tid, n_above - 1);
+    ns_above        = st.node_sums[above];
+    base_above      = st.base[above];
+    seg_of          = st.seg[above];
+#pragma unroll
+    for (int u = 0; u < kLoads; u++) bins_of[u] = reinterpret_cast<const uint4*>(st.bins)[min(tid + u * kT, n16 - 1)];
+  }
   // all loads are under way before the first is stored: a loop that loads and stores waits once per turn
   int2 pair[kSingle && kG > 1 ? kE : 1];
   if constexpr (kSingle && kG > 1) {
 #pragma unroll
     for (int u = 0; u < kE; u++)
-      if (tid + u * kT < a.N) pair[u] = st.qgh[tid + u * kT];
+      if (kClamped || tid + u * kT < a.N) pair[u] = st.qgh[min(tid + u * kT, a.N - 1)];
   } else if (kSingle && usable) {
     for (int i = tid; i < a.N; i += kT) s_q[i] = st.qgh[i];
   }
-  uint32_t code[kE / 4];
+  static_assert(kE >= 4 || kDecides, "sides of four rows at a time");
+  uint32_t code[(kE + 3) / 4];
+  if (!kDecides && kClamped && a.depth > 0) {
 #pragma unroll
-  for (int u = 0; u < kE / 4; u++)
-    if (a.depth > 0 && 4 * (tid + u * kT) < a.N) code[u] = *reinterpret_cast<const uint32_t*>(st.code + 4 * (tid + u * kT));
-  if (kStaged && usable)
+    for (int u = 0; u < kE / 4; u++) code[u] = *reinterpret_cast<const uint32_t*>(st.code + min(4 * (tid + u * kT), static_cast<int>(st.pitch) - 4));
+  }
+  if (!kClamped) {
+#pragma unroll
+    for (int u = 0; u < kE / 4; u++)
+      if (a.depth > 0 && 4 * (tid + u * kT) < a.N) code[u] = *reinterpret_cast<const uint32_t*>(st.code + 4 * (tid + u * kT));
+  }
+  if (kStaged && !kDecides && usable)
     for (int j = tid; j < a.n_nodes; j += kT) {
       const I64Pair ns = st.node_sums[a.level_first + j];
       s_base[j]        = st.base[a.level_first + j];
@@ -409,13 +515,171 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     }
   if constexpr (kSingle && kG > 1) {
 #pragma unroll
+    for (int u = 0; u < (kClamped ? kE : 0); u++) arrived(pair[u]);
+#pragma unroll
     for (int u = 0; u < kE; u++)
       if (tid + u * kT < a.N) s_q[tid + u * kT] = pair[u];
   }
 #pragma unroll
   for (int u = 0; u < kE / 4; u++)
-    if (a.depth > 0 && 4 * (tid + u * kT) < a.N) *reinterpret_cast<uint32_t*>(s_code + 4 * (tid + u * kT)) = code[u];
+    if (!kDecides && a.depth > 0 && 4 * (tid + u * kT) < a.N) *reinterpret_cast<uint32_t*>(s_code + 4 * (tid + u * kT)) = code[u];
   if (live == 0 && a.depth > 0) return;
+  // (kDecides, feature 0's workgroup) what follows from the splits of the level above, when there is nothing else to do
+  double split_value = 0.0;  // thread j: of node j
+  auto write_outputs = [&]() {
+    const int j = tid;
+    if (f != 0 || j >= a.n_nodes / 2 || s_split[j].x < 0) return;
+    a.feature[above_first + j] = s_split[j].x;
+    a.split[above_first + j]   = split_value;
+    a.gain[above_first + j]    = s_gain_above[j];
+    for (int side = 0; side < 2; side++) {
+      const double g = static_cast<double>(s_ns[2 * j + side].grad) * inv_g, h = static_cast<double>(s_ns[2 * j + side].hess) * inv_h;
+      a.leaf[a.level_first + 2 * j + side]    = calculate_leaf_value(g, h, a.l1, a.l2);
+      a.hessian[a.level_first + 2 * j + side] = h;
+    }
+  };
+  if constexpr (kDecides) {
+#pragma unroll
+    for (int u = 0; u < kLoads; u++) arrived(bins_of[u]);
+    arrived(seg_of);
+    if (tid < n_above) s_seg_above[tid] = seg_of;
+#pragma unroll
+    for (int u = 0; u < kLoads; u++)
+      if (tid + u * kT < n16) reinterpret_cast<uint4*>(s_bins)[tid + u * kT] = bins_of[u];
+#pragma unroll
+    for (int p = 0; p < kPasses; p++) {
+      if ((p * kT) >> a.lanes_log < n_above) {
+        // gains are not negative: their bits compare as whole numbers, upper halves first
+        const int j        = (p * kT + tid) >> a.lanes_log;
+        const uint64_t own = static_cast<uint64_t>(__double_as_longlong(cand_of[p].gain));
+        const unsigned own_hi = static_cast<unsigned>(own >> 32), own_lo = static_cast<unsigned>(own);
+        const unsigned own_key = sub < a.F ? cand_of[p].key : 0u;  // (a copy of the last feature's is none)
+        const unsigned hi  = group_max_u32(own_hi, a.lanes_log);
+        const unsigned lo  = group_max_u32(own_hi == hi ? own_lo : 0u, a.lanes_log);
+        const unsigned key = group_max_u32(own_hi == hi && own_lo == lo ? own_key : 0u, a.lanes_log);
+        const double best  = __longlong_as_double(static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo));
+        const bool splits  = key != 0 && best > 1e-5;
+        if (j < n_above) {
+          if (!splits && sub == 0) s_split[j] = make_int2(-1, 0);
+          if (splits && sub < a.F && own_hi == hi && own_lo == lo && own_key == key) {  // (keys of different candidates differ: one lane)
+            s_split[j]      = make_int2(sub, cand_of[p].rel);
+            s_gain_above[j] = best;
+            s_left_above[j] = left_cand[p];
+          }
+        }
+      }
+    }
+    __syncthreads();
+    const bool keeps = usable || f == 0;  // this feature's order
+    if (f == 0 && tid < n_above && s_split[tid].x >= 0)
+      split_value = st.proposals[static_cast<int64_t>(s_split[tid].x) * a.S + s_split[tid].y];
+    unsigned left = 0, goes_on = 0;
+    int2 sp[kE];
+    int b[kE];
+#pragma unroll
+    for (int e = 0; e < kE; e++) {
+      sp[e] = i0 + e < a.N && node[e] != kNone ? s_split[node[e]] : make_int2(-1, 0);
+      b[e]  = 0;
+    }
+    auto bin_at = [&](int e) { return sp[e].x * static_cast<int>(st.pitch) + static_cast<int>(entry[e] & 0xffff); };
+    if (a.all_bins) {
+#pragma unroll
+      for (int e = 0; e < kE; e++)
+        if (sp[e].x >= 0) b[e] = s_bins[bin_at(e)];
+    } else if (keeps) {
+#pragma unroll
+      for (int e = 0; e < kE; e++)
+        if (sp[e].x >= 0) b[e] = st.bins[bin_at(e)];
+    }
+    if (f == 0 && a.row_leaf != nullptr) {
+#pragma unroll
+      for (int e = 0; e < kE; e++)
+        if (i0 + e < a.N && node[e] != kNone && sp[e].x < 0) a.row_leaf[entry[e] & 0xffff] = above_first + node[e];
+    }
+    if (tid < n_above) {
+      // (thread j: children of node j; without a split they have no rows and nobody asks for them)
+      const bool splits       = s_split[tid].x >= 0;
+      const I64Pair left_sums = splits ? s_left_above[tid] : I64Pair{0, 0};
+      const I64Pair right{ns_above.grad - left_sums.grad, ns_above.hess - left_sums.hess};
+      const I64Pair base_right{base_above.grad + left_sums.grad, base_above.hess + left_sums.hess};
+      s_ns[2 * tid]        = splits ? left_sums : I64Pair{0, 0};
+      s_ns[2 * tid + 1]    = splits ? right : I64Pair{0, 0};
+      s_base[2 * tid]      = base_above;
+      s_base[2 * tid + 1]  = base_right;
+      s_parent[2 * tid]    = leaf_gain(static_cast<double>(left_sums.grad) * inv_g, static_cast<double>(left_sums.hess) * inv_h, a.l1, reg);
+      s_parent[2 * tid + 1] = leaf_gain(static_cast<double>(right.grad) * inv_g, static_cast<double>(right.hess) * inv_h, a.l1, reg);
+    }
+    if (!usable)
+      for (int j = tid; j < a.n_nodes; j += kT) out[static_cast<int64_t>(j) * a.F] = SmallCand{0.0, 0u, 0};
+    if (!keeps) return;
+    for (int j = tid; j < a.n_nodes; j += kT) {
+      s_gain[j] = 0;
+      s_key[j]  = 0;
+    }
+#pragma unroll
+    for (int e = 0; e < kE; e++) {
+      goes_on |= sp[e].x >= 0 ? 1u << e : 0u;
+      left |= sp[e].x >= 0 && b[e] <= sp[e].y ? 1u << e : 0u;
+    }
+    const int before = block_exclusive_sum32<kT>(__popc(left), s_wave);
+#pragma unroll
+    for (int e = 0; e < kE; e++)
+      if ((goes_on >> e) & 1u) {
+        const int2 at = s_seg_above[node[e]];
+        if (at.x == i0 + e) s_left_before[node[e]] = before + __popc(left & ((1u << e) - 1u));
+        if (at.x + at.y - 1 == i0 + e) s_left_behind[node[e]] = before + __popc(left & ((2u << e) - 1u));
+      }
+    const bool next_goes_on = i0 + kE < a.N && node_next != kNone && s_split[node_next].x >= 0;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kE; e++) {
+      const int i = i0 + e;
+      if (i < a.N) {
+        int to = i, child = kNone;
+        if ((goes_on >> e) & 1u) {
+          const int first = s_left_before[node[e]], lefts = s_left_behind[node[e]] - first, x0 = s_seg_above[node[e]].x;
+          const int l     = before + __popc(left & ((1u << e) - 1u)) - first;
+          to    = (left >> e) & 1u ? x0 + l : i + lefts - l;
+          child = 2 * node[e] + (i - x0 < lefts ? 0 : 1);
+        }
+        s_order[to] = entry[e];
+        node[e]     = child;
+      } else {
+        node[e] = kNone;
+      }
+    }
+    if (next_goes_on) {
+      const int lefts = s_left_behind[node_next] - s_left_before[node_next];
+      node_next       = 2 * node_next + (i0 + kE - s_seg_above[node_next].x < lefts ? 0 : 1);
+    } else {
+      node_next = kNone;
+    }
+    if (f == 0) {
+      if (tid < n_above && s_split[tid].x >= 0) {
+        const int lefts = s_left_behind[tid] - s_left_before[tid], child = a.level_first + 2 * tid;
+        st.seg[child]           = make_int2(seg_of.x, lefts);
+        st.seg[child + 1]       = make_int2(seg_of.x + lefts, seg_of.y - lefts);
+        st.node_sums[child]     = s_ns[2 * tid];
+        st.node_sums[child + 1] = s_ns[2 * tid + 1];
+        st.base[child]          = s_base[2 * tid];
+        st.base[child + 1]      = s_base[2 * tid + 1];
+        st.live[a.depth]        = 1;
+      }
+#pragma unroll
+      for (int e = 0; e < kE; e++)
+        if (i0 + e < a.N) a.node_out[i0 + e] = static_cast<uint16_t>(node[e]);
+    }
+    __syncthreads();
+    uint32_t* order_out = st.order[a.depth & 1] + static_cast<int64_t>(f) * st.pitch;
+    if (i0 < a.N) {
+      load_u32<kE>(s_order + i0, entry);
+      store_u32<kE>(order_out + i0, entry);  // (entries past N are never looked at)
+    }
+    if (!usable) {
+      write_outputs();
+      return;
+    }
+  } else {
   if (a.depth == 0) {
     int mine = 0;
     for (int i = tid; i < f; i += kT) mine += st.counts[i];
@@ -441,6 +705,7 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
 #pragma unroll
   for (int e = 0; e < kE; e++)
     if (i0 + e >= a.N) node[e] = kNone;
+  if (kClamped && i0 + kE >= a.N) node_next = kNone;
   if (a.depth > 0) {
     // node[] already is the node of this level at the place: both children of a parent lie where the
     // parent's rows lay, the left one first
@@ -479,12 +744,8 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     __syncthreads();
     uint32_t* order_out = st.order[a.depth & 1] + static_cast<int64_t>(f) * st.pitch;
     if (i0 < a.N) {
-#pragma unroll
-      for (int u = 0; u < kE / 4; u++) {
-        const uint4 v = reinterpret_cast<const uint4*>(s_order + i0)[u];
-        reinterpret_cast<uint4*>(order_out + i0)[u] = v;  // (entries past N are never looked at)
-        entry[4 * u] = v.x, entry[4 * u + 1] = v.y, entry[4 * u + 2] = v.z, entry[4 * u + 3] = v.w;
-      }
+      load_u32<kE>(s_order + i0, entry);
+      store_u32<kE>(order_out + i0, entry);  // (entries past N are never looked at)
     }
   } else {
     // the neighbour's first bin is looked up below
@@ -492,6 +753,7 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     __syncthreads();
   }
   if (!usable) return;
+  }
 
   // occupied bins: the places that are the last of their (node, bin); the last rows of a node leave
   // nothing on the right: never a split
@@ -531,6 +793,12 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     int first_node = kNone, cur = kNone;
     double first_gain = 0.0, cur_gain = 0.0;
     unsigned first_key = 0, cur_key = 0;
+    // (where the next scan may decide: what lies left of a node's best split goes with it)
+    constexpr bool kLeft = kStaged && kG > 1 && kE <= 4;
+    I64Pair first_left{0, 0}, cur_left{0, 0};
+    auto put_left = [&](int j, const I64Pair& left) {
+      if (kLeft && a.left != nullptr) a.left[static_cast<int64_t>(j) * a.F + f] = left;
+    };
     auto node_at = [&](int j, I64Pair& ns, I64Pair& base, double& parent) {
       if constexpr (kStaged) {
         ns     = s_ns[j];
@@ -554,19 +822,26 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
         first_node = cur;  // (kNone again while there was none before)
         first_gain = cur_gain;
         first_key  = cur_key;
+        first_left = cur_left;
       } else if (cur_key != 0) {
         s_gain[cur] = static_cast<unsigned long long>(__double_as_longlong(cur_gain));
         s_key[cur]  = cur_key;
+        put_left(cur, cur_left);
       }
       cur      = j;
       cur_gain = 0.0;
       cur_key  = 0;
     };
-    auto offer = [&](double gain, int e) {
+    auto offer = [&](double gain, int e, const I64Pair& left) {
       if (gain >= cur_gain) {
         const unsigned key = tie_key(rp, bin[e], bin[e + 1]);
-        cur_key            = gain > cur_gain ? key : max(cur_key, key);
-        cur_gain           = gain;
+        if constexpr (kLeft) {
+          const bool better = gain > cur_gain || key > cur_key;
+          cur_left.grad     = better ? left.grad : cur_left.grad;
+          cur_left.hess     = better ? left.hess : cur_left.hess;
+        }
+        cur_key  = gain > cur_gain ? key : max(cur_key, key);
+        cur_gain = gain;
       }
     };
     if constexpr (kG == 1) {
@@ -585,7 +860,7 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
           const I64Pair ls{run.grad - base.grad, run.hess - base.hess}, rs{ns.grad - ls.grad, ns.hess - ls.hess};
           if (ls.hess > 0 && rs.hess > 0) {
             const double gain = gain_of(ls, rs, parent);
-            if (gain > 0) offer(gain, e);
+            if (gain > 0) offer(gain, e, ls);
           }
         }
       }
@@ -594,6 +869,7 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
       for (int e0 = 0; e0 < kE; e0 += kG) {
         double gain[kG];
         bool wanted[kG];
+        I64Pair left_of[kG];
 #pragma unroll
         for (int u = 0; u < kG; u++) {
           const int e = e0 + u;
@@ -604,14 +880,15 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
           node_at(node[e] != kNone ? node[e] : 0, ns, base, parent);
           const I64Pair ls{run.grad - base.grad, run.hess - base.hess}, rs{ns.grad - ls.grad, ns.hess - ls.hess};
           wanted[u] = ((ends >> e) & 1u) != 0 && ls.hess > 0 && rs.hess > 0;
-          gain[u]   = gain_of(ls, rs, parent);
+          gain[u]    = gain_of(ls, rs, parent);
+          left_of[u] = ls;
         }
         // (a node without a candidate here is none of those that the thread has to report)
 #pragma unroll
         for (int u = 0; u < kG; u++)
           if (wanted[u] && gain[u] > 0) {
             if (node[e0 + u] != cur) next_node(node[e0 + u]);
-            offer(gain[u], e0 + u);
+            offer(gain[u], e0 + u, left_of[u]);
           }
       }
     }
@@ -620,8 +897,11 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
       first_node = cur;
       first_gain = cur_gain;
       first_key  = cur_key;
+      first_left = cur_left;
       cur_key    = 0;
     }
+    const int own_node     = first_node;
+    const unsigned own_key = first_key;
     const unsigned long long first_bits = static_cast<unsigned long long>(__double_as_longlong(first_gain));
     const unsigned long long cur_bits   = static_cast<unsigned long long>(__double_as_longlong(cur_gain));
     // where a whole wave lies in one node its lanes meet first
@@ -646,6 +926,11 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     if (first_key != 0 && mine_bits == s_gain[first_node]) atomicMax(&s_key[first_node], first_key);
     if (cur_key != 0 && cur_bits == s_gain[cur]) atomicMax(&s_key[cur], cur_key);
     __syncthreads();
+    if constexpr (kLeft) {
+      // (keys of different bins differ, but one lane can hold an equal key of a smaller gain only for another bin: none)
+      if (own_key != 0 && own_key == s_key[own_node]) put_left(own_node, first_left);
+      if (cur_key != 0 && cur_key == s_key[cur]) put_left(cur, cur_left);
+    }
   } else {
     double gain[kE];
     unsigned dead = 0;
@@ -741,13 +1026,13 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     }
     out[static_cast<int64_t>(j) * a.F] = c;
   }
+  if constexpr (kDecides) write_outputs();
 }
 
 // Split of one node, its outputs, its children and the side of each of its rows.
 template <int kT>
 __global__ void __launch_bounds__(kT)
-  small_apply_kernel(SmallTreeState st, LevelArgs a, double* leaf, int32_t* feature, double* split, double* gain,
-                     double* hessian, int32_t* row_leaf)
+  small_apply_kernel(SmallTreeState st, LevelArgs a, uint16_t* node_of_pos)
 {
   __shared__ double s_best[kT / 64];
   __shared__ int4 s_pick[kT / 64];
@@ -778,7 +1063,7 @@ __global__ void __launch_bounds__(kT)
     ft       = better ? ft_o : ft;
     rel      = better ? rel_o : rel;
   };
-  const SmallCand* c = st.cand + static_cast<int64_t>(j) * a.F;
+  const SmallCand* c = a.cand + static_cast<int64_t>(j) * a.F;
   for (int i = tid; i < a.F; i += kT) {
     const SmallCand o = c[i];
     take(o.gain, o.key, i, o.rel);
@@ -797,8 +1082,8 @@ __global__ void __launch_bounds__(kT)
   }
   if (!(ns0.hess > 0 && best_key != 0 && best > 1e-5)) {
     for (int i = tid; i < n; i += kT) {
-      st.node_of_pos[s0 + i] = kNone;
-      if (row_leaf != nullptr) row_leaf[row_at(i)] = node;
+      node_of_pos[s0 + i] = kNone;
+      if (a.row_leaf != nullptr) a.row_leaf[row_at(i)] = node;
     }
     return;
   }
@@ -812,7 +1097,7 @@ __global__ void __launch_bounds__(kT)
     const int2 q    = st.qgh[r * a.K];  // (asked for beside the bin)
     const bool left = bins[r] <= rel;
     if (!a.last) st.code[r] = left ? 1 : 2;
-    if (a.last && row_leaf != nullptr) row_leaf[r] = left ? lc : rc;
+    if (a.last && a.row_leaf != nullptr) a.row_leaf[r] = left ? lc : rc;
     if (left) {
       nl++;
       sum.grad += q.x;
@@ -840,8 +1125,8 @@ __global__ void __launch_bounds__(kT)
       st.node_sums[to] = own;
       st.base[to]      = I64Pair{base.grad + (tid == 0 ? 0 : ls.grad), base.hess + (tid == 0 ? 0 : ls.hess)};
       const double g = static_cast<double>(own.grad) * inv_g, h = static_cast<double>(own.hess) * inv_h;
-      leaf[to]    = calculate_leaf_value(g, h, a.l1, a.l2);
-      hessian[to] = h;
+      a.leaf[to]    = calculate_leaf_value(g, h, a.l1, a.l2);
+      a.hessian[to] = h;
     }
     if (++k == a.K) break;
     sum = I64Pair{0, 0};
@@ -857,15 +1142,15 @@ __global__ void __launch_bounds__(kT)
   int lefts = 0;
   for (int w = 0; w < kT / 64; w++) lefts += s_cnt[w];
   if (tid == 0) {
-    feature[node] = ft;
-    split[node]   = value;
-    gain[node]    = best;
+    a.feature[node] = ft;
+    a.split[node]   = value;
+    a.gain[node]    = best;
     st.seg[lc]    = make_int2(s0, lefts);
     st.seg[rc]    = make_int2(s0 + lefts, n - lefts);
     st.live[a.depth + 1] = 1;
   }
   if (!a.last)
-    for (int i = tid; i < n; i += kT) st.node_of_pos[s0 + i] = static_cast<uint16_t>(2 * j + (i < lefts ? 0 : 1));
+    for (int i = tid; i < n; i += kT) node_of_pos[s0 + i] = static_cast<uint16_t>(2 * j + (i < lefts ? 0 : 1));
 }
 
 // For the profiler: what the histograms of the level would be built from.
@@ -883,28 +1168,56 @@ __global__ void __launch_bounds__(256) small_count_kernel(SmallTreeState st, Lev
   }
 }
 
-template <int kT, int kE, bool kSingle, int kG, bool kStaged>
+template <int kT, int kE, bool kSingle, int kG, bool kStaged, bool kDecides>
 int launch_small_scan_as(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a, size_t lds)
 {
   static std::atomic<bool> attr_set[kMaxDevices] = {};
   LBT_REQUIRE(small_scan_places(a.N) == kT * kE, "%d rows do not take a workgroup of %d places", a.N, kT * kE);
-  LBT_TRY((allow_dynamic_lds(small_scan_kernel<kT, kE, kSingle, kG, kStaged>, kScanLds + 64, attr_set)));
-  small_scan_kernel<kT, kE, kSingle, kG, kStaged><<<a.F, kT, lds, stream>>>(st, a);
+  LBT_TRY((allow_dynamic_lds(small_scan_kernel<kT, kE, kSingle, kG, kStaged, kDecides>, kScanLds + 64, attr_set)));
+  small_scan_kernel<kT, kE, kSingle, kG, kStaged, kDecides><<<a.F, kT, lds, stream>>>(st, a);
   return LBT_OK;
 }
-template <int kT, int kE>
-int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a)
+size_t small_staged_use(int64_t N, int64_t n_nodes)
 {
+  return small_scan_use(N, n_nodes) + static_cast<size_t>(n_nodes) * (2 * sizeof(I64Pair) + sizeof(double) + sizeof(int2));
+}
+template <int kT, int kE>
+int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a, bool decides)
+{
+  constexpr int kG = kE == 8 ? 2 : 4;
+  // a scan that decides has more to do per place: up to 1024 rows twice the threads with half the places each
+  constexpr int kDT = kT == 256 ? 512 : kT, kDE = kT * kE / kDT;
   const size_t lds  = small_scan_use(a.N, a.n_nodes);
-  const size_t more = lds + static_cast<size_t>(a.n_nodes) * (2 * sizeof(I64Pair) + sizeof(double) + sizeof(int2));
-  if (a.K > 1) return launch_small_scan_as<kT, kE, false, 1, false>(stream, st, a, lds);
+  const size_t more = small_staged_use(a.N, a.n_nodes);
+  if constexpr (kE == 4) {
+    if (decides) {
+      LevelArgs b       = a;
+      const size_t bins = static_cast<size_t>(a.F) * st.pitch * sizeof(uint16_t), all = more + small_decide_use(a.n_nodes);
+      b.all_bins        = bins <= static_cast<size_t>(kDT) * 16 * decide_loads(kDT) && all + bins <= kScanLds;
+      return launch_small_scan_as<kDT, kDE, true, kDE, true, true>(stream, st, b, all + (b.all_bins ? bins : 0));
+    }
+  }
+  if (a.K > 1) return launch_small_scan_as<kT, kE, false, 1, false, false>(stream, st, a, lds);
   // staging must not cost a workgroup of the CU where there are more of them than CUs
   auto per_cu        = [](size_t bytes) { return static_cast<int>(std::min<size_t>(2048 / kT, 160 * 1024 / (bytes + 1024))); };
   const bool crowded = kT == 1024 && a.F > 256;
   if (more > kScanLds || (per_cu(more) < per_cu(lds) && a.F > 256 * per_cu(more)))
-    return launch_small_scan_as<kT, kE, true, 1, false>(stream, st, a, lds);
-  if (crowded) return launch_small_scan_as<kT, kE, true, 1, true>(stream, st, a, more);
-  return launch_small_scan_as<kT, kE, true, kE == 8 ? 2 : 4, true>(stream, st, a, more);
+    return launch_small_scan_as<kT, kE, true, 1, false, false>(stream, st, a, lds);
+  if (crowded) return launch_small_scan_as<kT, kE, true, 1, true, false>(stream, st, a, more);
+  return launch_small_scan_as<kT, kE, true, kG, true, false>(stream, st, a, more);
+}
+
+// Whether the scan of the level below level `depth` finds this level's splits for itself: one output, a lane for every
+// feature and kDecidePasses of them for the nodes, a thread for every node, and the LDS for both levels' nodes.
+bool next_scan_decides(const SmallTreeState& st, int64_t N, int F, int K, int depth, int max_depth)
+{
+  if (st.left[0] == nullptr || K > 1 || depth + 1 >= max_depth || N > kDecideRows) return false;
+  const int threads = N <= 1024 ? 512 : small_scan_places(N) / 4;
+  int lanes = 1 << kDecideLanes;
+  while (lanes < F) lanes *= 2;
+  const int64_t nodes = int64_t(1) << depth;
+  return nodes * lanes <= kDecidePasses * threads && nodes <= threads &&
+         small_staged_use(N, 2 * nodes) + small_decide_use(2 * nodes) <= kScanLds;
 }
 
 }  // namespace
@@ -960,29 +1273,47 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
   a.n_bins = answer.words + 1;
   a.tag    = answer.tag;
   a.l1 = prm.l1_regularization; a.l2 = prm.l2_regularization; a.min_split_gain = prm.min_split_gain;
+  a.leaf = leaf; a.feature = feature; a.split = split; a.gain = gain; a.hessian = hessian; a.row_leaf = row_leaf;
+  a.lanes_log = kDecideLanes;
+  while ((1 << a.lanes_log) < F && a.lanes_log < 6) a.lanes_log++;
+  bool decides = false;  // the level's scan has to decide the level above
+  int nodes = 0, found = 0;  // the buffers in use
   for (int d = 0; d < prm.max_depth && (d == 0 || !answer.declined()); d++) {
     a.depth       = d;
     a.level_first = static_cast<int>(level_begin(d));
     a.n_nodes     = 1 << d;
     a.last        = d + 1 == prm.max_depth;
+    const bool next_decides = next_scan_decides(st, N, F, K, d, prm.max_depth);
+    a.node_in    = st.node_of_pos[nodes];
+    a.cand_above = st.cand[found];
+    a.left_above = st.left[found];
+    if (decides) {
+      nodes ^= 1;
+      found ^= 1;
+    }
+    a.node_out = st.node_of_pos[nodes];
+    a.cand     = st.cand[found];
+    a.left     = next_decides ? st.left[found] : nullptr;
     {
       ProfScope ps(LBT_PROF_HISTOGRAM, stream, 0.0, d);
       switch (small_scan_places(N)) {
-        case 1024: LBT_TRY((launch_small_scan<256, 4>(stream, st, a))); break;
-        case 2048: LBT_TRY((launch_small_scan<512, 4>(stream, st, a))); break;
-        case 4096: LBT_TRY((launch_small_scan<1024, 4>(stream, st, a))); break;
-        default: LBT_TRY((launch_small_scan<1024, 8>(stream, st, a)));
+        case 1024: LBT_TRY((launch_small_scan<256, 4>(stream, st, a, decides))); break;
+        case 2048: LBT_TRY((launch_small_scan<512, 4>(stream, st, a, decides))); break;
+        case 4096: LBT_TRY((launch_small_scan<1024, 4>(stream, st, a, decides))); break;
+        default: LBT_TRY((launch_small_scan<1024, 8>(stream, st, a, decides)));
       }
     }
+    decides = next_decides;
     if (level_totals != nullptr) small_count_kernel<<<1, 256, 0, stream>>>(st, a, level_totals + d);
+    if (decides) continue;
     ProfScope ps(LBT_PROF_SPLIT, stream);
     // few nodes of many rows near the root, many small ones below
     if ((N >> d) > 1024)
-      small_apply_kernel<1024><<<a.n_nodes, 1024, 0, stream>>>(st, a, leaf, feature, split, gain, hessian, row_leaf);
+      small_apply_kernel<1024><<<a.n_nodes, 1024, 0, stream>>>(st, a, st.node_of_pos[nodes]);
     else if (d <= 8)
-      small_apply_kernel<256><<<a.n_nodes, 256, 0, stream>>>(st, a, leaf, feature, split, gain, hessian, row_leaf);
+      small_apply_kernel<256><<<a.n_nodes, 256, 0, stream>>>(st, a, st.node_of_pos[nodes]);
     else
-      small_apply_kernel<64><<<a.n_nodes, 64, 0, stream>>>(st, a, leaf, feature, split, gain, hessian, row_leaf);
+      small_apply_kernel<64><<<a.n_nodes, 64, 0, stream>>>(st, a, st.node_of_pos[nodes]);
   }
   LBT_HIP(hipGetLastError());
   unsigned flags = 0;

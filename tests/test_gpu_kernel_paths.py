@@ -125,6 +125,36 @@ def test_few_rows(n, f, k, depth, s, dtype):
         gu.check_row_leaf(got, X)
 
 
+@pytest.mark.parametrize("n,f,depth,dtype", [(1024, 16, 8, np.float32), (1025, 17, 9, np.float64), (4096, 64, 7, np.float32), (4097, 10, 6, np.float32),
+                                             (3001, 65, 6, np.float32), (37, 1, 8, np.float64), (700, 33, 10, np.float32), (2048, 32, 8, np.float64)])
+@pytest.mark.parametrize("stops", [False, True])
+def test_few_rows_whose_scans_decide(n, f, depth, dtype, stops):
+    """Levels that are decided by the next one's scan, either side of the rows, features, lanes and nodes up to which they are,
+    in turn with levels that are not; rows that end at every level, features that are not used, ties between features."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + f)
+    X = rs.randn(n, f).astype(dtype)
+    if f > 8:
+        X[:, 5] = X[:, 0]
+        X[:, 7] = rs.randint(0, 2, n)
+    g, inside = rs.randn(n, 1), np.ones(n, bool)
+    if stops:
+        g *= 0.2
+        for level in range(depth):
+            inside &= X[:, level % f] > (0 if level < f else 0.3)
+            g[:, 0] += inside
+    kw = dict(max_depth=depth, split_samples=100, seed=3, min_split_gain=0.5 if stops else 0.0)
+    h = 0.5 + rs.rand(n, 1)
+    for fs in (None, np.arange(f) % 3 != 0) if f > 3 else (None,):
+        cr = orc.build_tree(X, g, h, feature_set=fs, **kw)
+        got = ops.build_tree(X, g, h, feature_set=fs, row_leaf=True, **kw)
+        _assert_tree(got, cr)
+        gu.check_row_leaf(got, X)
+
+
 @pytest.mark.parametrize("case", ["negative_hessian", "zero_hessian", "all_zero", "constant_target"])
 def test_few_rows_special_gradients(case):
     """Rows whose rounded hessian is not positive need the reference's unscanned bins: such data take the other
