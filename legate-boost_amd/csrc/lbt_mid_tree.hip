@@ -372,6 +372,14 @@ struct LevelPlan {
 // four), 1,000,000 x 50 with 512 samples 802 (737), 150,000 x 20 with 4 outputs 273 (243), 300,000 x 32 the same.
 constexpr int kMaxFw = 4;
 
+// Values (rows times features and outputs) up to which it is the images of the row ranges that cost, not the additions: a scan
+// workgroup reads 64 KB of them with 32 ranges, which takes it 6000 of 14,000 cycles however many loads are under way. One
+// workgroup for every CU then, not two, and two features each instead of four (with several outputs the ranges are few anyway): fewer
+// ranges. Fits with two workgroups and with one, us: 20,000 x 100, depth 6, 5 rounds 1040 and 945; 9000 x 200, depth 5 945 and 825; 250,000 x 43,
+// depth 8 1965 and 1890; 300,000 x 16 with 128 samples 1060 and 1005; 60,000 x 20 with 4 outputs 1235 and 1110; above, 800,000 x 45
+// with 64 samples, depth 5 985 and 1118, 112,000 x 245, depth 3 1013 and 1070 (not taken).
+constexpr int64_t kImageValues = 12000000;
+
 // Which of a pair of siblings is accumulated (build_tree.h:92-104).
 __device__ __forceinline__ int built_of_pair(const I64Pair* __restrict__ node_sums, int level_first, int pair, int K)
 {
@@ -846,14 +854,15 @@ LevelPlan plan_level(int64_t N, int F, int K, int S, int depth, int max_depth)
   p.built       = depth == 0 ? 1 : p.n_nodes / 2;
   p.last        = depth + 1 == max_depth;
   const int rows_of_lds = std::max<int>(1, static_cast<int>(kHistLds / (static_cast<size_t>(S) * 8)));
-  p.fw   = std::max(1, std::min({rows_of_lds / p.built, kMaxFw, F}));
+  const bool by_images = N * F * K <= kImageValues;
+  p.fw   = std::max(1, std::min({rows_of_lds / p.built, by_images && K == 1 ? 2 : kMaxFw, F}));
   p.bw   = std::max(1, std::min(p.built, rows_of_lds / p.fw));
   p.n_fb = (F + p.fw - 1) / p.fw;
   p.n_bb = (p.built + p.bw - 1) / p.bw;
   const int64_t inner = static_cast<int64_t>(p.n_fb) * p.n_bb * K;
   const int64_t image = static_cast<int64_t>(p.built) * K * F * S * 8;
   // two workgroups share a CU where their histograms do
-  const bool pairs    = static_cast<size_t>(p.fw) * p.bw * S * 8 <= 72 * 1024;
+  const bool pairs    = !by_images && static_cast<size_t>(p.fw) * p.bw * S * 8 <= 72 * 1024;
   int64_t chunks      = std::max<int64_t>(1, (pairs ? 512 : 256) / inner);
   // (three quarters of a workgroup's threads have rows: with 1024 rows a range, most of them had none and the scan
   // added up twice the images: 100,000 x 32, 10 rounds, 2.06 -> 1.87 ms; 60,000 x 20 with 4 outputs -9 %)
