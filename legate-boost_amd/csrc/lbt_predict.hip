@@ -126,8 +126,12 @@ struct alignas(8) BatchInfo {
   int32_t steps;     // steps that reach the deepest possible leaf of any tree of the batch
 };
 
-constexpr int kPackTrees    = 64;  // trees packed per launch (descriptors passed by value)
-constexpr int kPackBatches  = 128; // batch descriptors written per launch
+// Descriptors are passed by value, 4 KB of arguments a launch; a launch is 3.5 us of the host's time. A prediction of 1000 x 10 with
+// 100 trees took 43 us with two of them and a third for the batches, 36 with one (27 with the initial prediction added
+// by the kernel for few rows and the stream's handle without an object around it).
+constexpr int kPackTrees    = 104; // trees packed per launch
+constexpr int kFirstBatches = 10;  // and batch descriptors written by the first one
+constexpr int kPackBatches  = 128; // batch descriptors written per launch of their own
 constexpr int kTileThreads  = 1024;
 // L lanes share a row; a workgroup then covers 1024 / L rows, and a batch holds L * kLaneTrees
 // trees. Wide feature matrices take more lanes per row, so that the row tile still fits the LDS.
@@ -146,33 +150,39 @@ constexpr int kSmallRunGroups = 256;  // workgroups up to which more lanes share
 constexpr size_t kSmallEnsembleLds = 78 * 1024;  // row tile + nodes of a small ensemble: two workgroups per CU
 
 struct PackBatch {
-  TreeRef t[kPackTrees];
-  int64_t node_off[kPackTrees];
+  const double* leaf[kPackTrees];
+  const int32_t* feature[kPackTrees];
+  const double* split[kPackTrees];
+  int32_t n_nodes[kPackTrees];
+  int32_t node_off[kPackTrees];  // from first_node on
   int32_t rel_off[kPackTrees];
+  int64_t first_node;
+  BatchInfo b[kFirstBatches];
+  int32_t first_tree, n_batches;
 };
+static_assert(sizeof(PackBatch) <= 4096 - 64, "what a launch takes, with the other arguments");
 struct BatchTable {
   BatchInfo b[kPackBatches];
 };
 
 template <typename T>
 __global__ void __launch_bounds__(256)
-  pack_trees_kernel(PackBatch b, int first_tree, int F, int K, PackedTree* desc, PackedNode<T>* nodes,
-                    double* leaves)
+  pack_trees_kernel(PackBatch b, int F, int K, PackedTree* desc, BatchInfo* batches, PackedNode<T>* nodes, double* leaves)
 {
-  const TreeRef tr = b.t[blockIdx.y];
-  const int i      = blockIdx.x * 256 + threadIdx.x;
+  const int t = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x, n = b.n_nodes[t];
+  const int64_t first = b.first_node + b.node_off[t];
+  if (t == 0 && i < b.n_batches) batches[i] = b.b[i];
   if (i == 0) {
     PackedTree d;
-    d.node_off                    = b.node_off[blockIdx.y];
-    d.rel_off                     = b.rel_off[blockIdx.y];
-    d.n_nodes                     = tr.n_nodes;
-    desc[first_tree + blockIdx.y] = d;
+    d.node_off             = first;
+    d.rel_off              = b.rel_off[t];
+    d.n_nodes              = n;
+    desc[b.first_tree + t] = d;
   }
-  if (i >= tr.n_nodes) return;
+  if (i >= n) return;
   // leaf values move along, indexed like the nodes
-  for (int k = 0; k < K; k++)
-    leaves[(b.node_off[blockIdx.y] + i) * K + k] = tr.leaf[static_cast<int64_t>(i) * K + k];
-  nodes[b.node_off[blockIdx.y] + i] = pack_node<T>(i, tr.feature[i], tr.split[i], F, tr.n_nodes);
+  for (int k = 0; k < K; k++) leaves[(first + i) * K + k] = b.leaf[t][static_cast<int64_t>(i) * K + k];
+  nodes[first + i] = pack_node<T>(i, b.feature[t][i], b.split[t][i], F, n);
 }
 
 __global__ void write_batches_kernel(BatchTable t, int first, int n, BatchInfo* out)
@@ -475,7 +485,8 @@ __global__ void __launch_bounds__(kTileThreads)
   predict_few_kernel(const T* __restrict__ X, int64_t n_rows, int F, int pitch, int n_trees, int n_batches,
                      const BatchInfo* __restrict__ batches, const PackedTree* __restrict__ desc,
                      const PackedNode<T>* __restrict__ nodes, const double* __restrict__ leaves, int K, int node_at,
-                     int cap_words, int cap_trees, int64_t all_words, int value_at, double* __restrict__ out)
+                     int cap_words, int cap_trees, int64_t all_words, int value_at, const double* __restrict__ init,
+                     double* __restrict__ out)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   constexpr int kNodesPerWord = 16 / sizeof(PackedNode<T>);
@@ -554,7 +565,14 @@ __global__ void __launch_bounds__(kTileThreads)
       for (int t = 0; t < count; t++) acc += s_value[t * items + tid];
     }
   }
-  if (tid < rows_here * K) out[row0 * K + tid] = acc;
+  if (tid < rows_here * K) out[row0 * K + tid] = init != nullptr ? init[tid % K] + acc : acc;
+}
+
+// init + the sums, where the kernel that formed them did not add it
+__global__ void __launch_bounds__(kThreads) add_init_kernel(const double* __restrict__ init, int64_t n, int K, double* out)
+{
+  const int64_t i = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x;
+  if (i < n) out[i] = init[K == 1 ? 0 : i % K] + out[i];
 }
 
 size_t padded_nodes(int n_trees, int64_t total_nodes)
@@ -675,24 +693,28 @@ int pack_tiled(hipStream_t stream, int F, int n_trees, const double* const* leaf
     widest_batch = std::max(widest_batch, in_batch);
     binfo.push_back(bi);
   }
+  const int n_batches = static_cast<int>(binfo.size());
   for (int first = 0; first < n_trees; first += kPackTrees) {
-    PackBatch b{};
+    PackBatch b;
     const int n = std::min(kPackTrees, n_trees - first);
     int widest  = 1;
+    b.first_node = node_off[first];
+    b.first_tree = first;
+    b.n_batches  = first == 0 ? std::min(n_batches, kFirstBatches) : 0;
+    for (int i = 0; i < b.n_batches; i++) b.b[i] = binfo[i];
     for (int i = 0; i < n; i++) {
-      b.t[i].leaf    = leaf[first + i];
-      b.t[i].feature = feature[first + i];
-      b.t[i].split   = split[first + i];
-      b.t[i].n_nodes = tree_nodes[first + i];
-      b.node_off[i]  = node_off[first + i];
-      b.rel_off[i]   = rel_off[first + i];
-      widest         = std::max(widest, tree_nodes[first + i]);
+      b.leaf[i]     = leaf[first + i];
+      b.feature[i]  = feature[first + i];
+      b.split[i]    = split[first + i];
+      b.n_nodes[i]  = tree_nodes[first + i];
+      b.node_off[i] = static_cast<int32_t>(node_off[first + i] - b.first_node);
+      b.rel_off[i]  = rel_off[first + i];
+      widest        = std::max(widest, tree_nodes[first + i]);
     }
     dim3 grid(static_cast<unsigned>((widest + 255) / 256), n);
-    pack_trees_kernel<T><<<grid, 256, 0, stream>>>(b, first, F, K, lay.desc, lay.nodes, lay.leaves);
+    pack_trees_kernel<T><<<grid, 256, 0, stream>>>(b, F, K, lay.desc, lay.batches, lay.nodes, lay.leaves);
   }
-  const int n_batches = static_cast<int>(binfo.size());
-  for (int first = 0; first < n_batches; first += kPackBatches) {
+  for (int first = kFirstBatches; first < n_batches; first += kPackBatches) {
     BatchTable tb{};
     const int n = std::min(kPackBatches, n_batches - first);
     for (int i = 0; i < n; i++) tb.b[i] = binfo[first + i];
@@ -720,10 +742,11 @@ constexpr size_t kBatchValues = static_cast<size_t>(TileShape<16>::kBatchTrees) 
 size_t values_offset(const lbt_packed_ensemble& ens) { return (static_cast<size_t>(ens.lds_bytes) + 15) & ~size_t(15); }
 bool values_through_lds(const lbt_packed_ensemble& ens) { return ens.n_outputs == 1 && values_offset(ens) + kBatchValues <= kTileLds; }
 
+// *init (optional): what the sums are added to; null afterwards where that has been done.
 // The kernel for few rows over a packed ensemble; *done stays false where the tile kernel is the faster one or the shapes
 // do not fit.
 template <typename T>
-int run_few(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble& ens, double* out, bool* done)
+int run_few(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble& ens, const double** init, double* out, bool* done)
 {
   const int F = ens.n_features, K = ens.n_outputs, pitch = F | 1;
   if (ens.few_trees != 0 || N > kFewMostRows || kFewRows * K > kTileThreads) return LBT_OK;
@@ -758,8 +781,9 @@ int run_few(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble
   LBT_TRY(allow_dynamic_lds(predict_few_kernel<T>, kTileLds, attr));
   predict_few_kernel<T><<<static_cast<unsigned>((N + kFewRows - 1) / kFewRows), kTileThreads, value_at + value_bytes, stream>>>(
     X, N, F, pitch, ens.n_trees, ens.n_batches, lay.batches, lay.desc, lay.nodes, lay.leaves, K, node_at,
-    static_cast<int>(cap_words), cap_trees, all_words, value_at, out);
+    static_cast<int>(cap_words), cap_trees, all_words, value_at, init != nullptr ? *init : nullptr, out);
   LBT_HIP(hipGetLastError());
+  if (init != nullptr) *init = nullptr;
   *done = true;
   return LBT_OK;
 }
@@ -767,12 +791,12 @@ int run_few(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble
 // The tile kernel over a packed ensemble.
 template <typename T>
 int run_tiled(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemble& ens, double* out,
-              const int32_t* wanted = nullptr)
+              const int32_t* wanted = nullptr, const double** init = nullptr)
 {
   const int F = ens.n_features, K = ens.n_outputs, n_batches = ens.n_batches;
   if (wanted == nullptr) {
     bool done = false;
-    LBT_TRY(run_few<T>(stream, X, N, ens, out, &done));
+    LBT_TRY(run_few<T>(stream, X, N, ens, init, out, &done));
     if (done) return LBT_OK;
   }
   // The lanes the ensemble was laid out for suit many rows. Batches of so many trees fit the kernels for more lanes
@@ -828,13 +852,13 @@ int run_tiled(hipStream_t stream, const T* X, int64_t N, const lbt_packed_ensemb
 template <typename T>
 int predict_tiled(hipStream_t stream, const T* X, int64_t N, int F, int n_trees, const double* const* leaf,
                   const int32_t* const* feature, const double* const* split, const int32_t* tree_nodes, int K,
-                  const int32_t* wanted, double* out, void* workspace, size_t workspace_bytes, bool* done)
+                  const int32_t* wanted, const double** init, double* out, void* workspace, size_t workspace_bytes, bool* done)
 {
   *done = false;
   lbt_packed_ensemble ens;
   LBT_TRY(pack_tiled<T>(stream, F, n_trees, leaf, feature, split, tree_nodes, K, workspace, workspace_bytes, &ens));
   if (ens.data == nullptr) return LBT_OK;
-  LBT_TRY(run_tiled<T>(stream, X, N, ens, out, wanted));
+  LBT_TRY(run_tiled<T>(stream, X, N, ens, out, wanted, init));
   *done = true;
   return LBT_OK;
 }
@@ -842,8 +866,8 @@ int predict_tiled(hipStream_t stream, const T* X, int64_t N, int F, int n_trees,
 // By ranks where that is the faster way and the workspace has the room, else tiled, else per node.
 template <typename T>
 int predict_any(hipStream_t stream, const T* X, int64_t N, int F, int n_trees, const double* const* leaf,
-                const int32_t* const* feature, const double* const* split, const int32_t* tree_nodes, int K, double* out,
-                void* workspace, size_t workspace_bytes)
+                const int32_t* const* feature, const double* const* split, const int32_t* tree_nodes, int K, const double** init,
+                double* out, void* workspace, size_t workspace_bytes)
 {
   int64_t total = 0;
   for (int i = 0; i < n_trees; i++) total += tree_nodes[i];
@@ -857,7 +881,7 @@ int predict_any(hipStream_t stream, const T* X, int64_t N, int F, int n_trees, c
     // 1000 trees of depth 8 for packing and a launch that reads one word)
     if (done && wanted == nullptr) return LBT_OK;
   }
-  LBT_TRY(predict_tiled<T>(stream, X, N, F, n_trees, leaf, feature, split, tree_nodes, K, wanted, out, workspace,
+  LBT_TRY(predict_tiled<T>(stream, X, N, F, n_trees, leaf, feature, split, tree_nodes, K, wanted, init, out, workspace,
                            workspace_bytes, &done));
   if (done) return LBT_OK;
   return predict_impl<T>(stream, X, N, F, n_trees, leaf, feature, split, tree_nodes, K, wanted, out);
@@ -1084,10 +1108,10 @@ int update_impl(hipStream_t stream, const T* X, UpdateArgs a, double l1, double 
 
 extern "C" {
 
-int lbt_predict(void* stream, const void* X, int32_t x_dtype, int64_t n_rows, int32_t n_features,
-                int32_t n_trees, const double* const* leaf, const int32_t* const* feature,
-                const double* const* split, const int32_t* tree_nodes, int32_t n_outputs,
-                double* out, void* workspace, size_t workspace_bytes)
+int lbt_predict_from(void* stream, const void* X, int32_t x_dtype, int64_t n_rows, int32_t n_features,
+                     int32_t n_trees, const double* const* leaf, const int32_t* const* feature,
+                     const double* const* split, const int32_t* tree_nodes, int32_t n_outputs,
+                     const double* init, double* out, void* workspace, size_t workspace_bytes)
 {
   LBT_REQUIRE(x_dtype == LBT_F32 || x_dtype == LBT_F64, "unsupported X dtype %d", x_dtype);
   LBT_REQUIRE(n_features >= 1 && n_outputs >= 1 && n_trees >= 0, "bad shape");
@@ -1097,16 +1121,32 @@ int lbt_predict(void* stream, const void* X, int32_t x_dtype, int64_t n_rows, in
   LBT_REQUIRE(n_trees == 0 || (leaf && feature && split && tree_nodes), "null tree arrays");
   for (int i = 0; i < n_trees; i++)
     LBT_REQUIRE(leaf[i] && feature[i] && split[i] && tree_nodes[i] >= 1, "tree %d is incomplete", i);
-  hipStream_t s = static_cast<hipStream_t>(stream);
+  hipStream_t s   = static_cast<hipStream_t>(stream);
+  const int64_t n = n_rows * n_outputs;
   if (n_trees == 0) {
-    lbt::zero_doubles_kernel<<<static_cast<unsigned>((n_rows * n_outputs + 255) / 256), 256, 0, s>>>(
-      out, n_rows * n_outputs);
-    return LBT_OK;
+    lbt::zero_doubles_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(out, n);
+  } else if (x_dtype == LBT_F32) {
+    LBT_TRY(lbt::predict_any<float>(s, static_cast<const float*>(X), n_rows, n_features, n_trees, leaf, feature, split,
+                                    tree_nodes, n_outputs, &init, out, workspace, workspace_bytes));
+  } else {
+    LBT_TRY(lbt::predict_any<double>(s, static_cast<const double*>(X), n_rows, n_features, n_trees, leaf, feature, split,
+                                     tree_nodes, n_outputs, &init, out, workspace, workspace_bytes));
   }
-  return x_dtype == LBT_F32 ? lbt::predict_any<float>(s, static_cast<const float*>(X), n_rows, n_features, n_trees, leaf,
-                                                      feature, split, tree_nodes, n_outputs, out, workspace, workspace_bytes)
-                            : lbt::predict_any<double>(s, static_cast<const double*>(X), n_rows, n_features, n_trees, leaf,
-                                                       feature, split, tree_nodes, n_outputs, out, workspace, workspace_bytes);
+  if (init != nullptr) {
+    lbt::ProfScope ps(LBT_PROF_OTHER, s, static_cast<double>(n) * 16.0);
+    lbt::add_init_kernel<<<static_cast<unsigned>((n + lbt::kThreads - 1) / lbt::kThreads), lbt::kThreads, 0, s>>>(init, n, n_outputs, out);
+    LBT_HIP(hipGetLastError());
+  }
+  return LBT_OK;
+}
+
+int lbt_predict(void* stream, const void* X, int32_t x_dtype, int64_t n_rows, int32_t n_features,
+                int32_t n_trees, const double* const* leaf, const int32_t* const* feature,
+                const double* const* split, const int32_t* tree_nodes, int32_t n_outputs,
+                double* out, void* workspace, size_t workspace_bytes)
+{
+  return lbt_predict_from(stream, X, x_dtype, n_rows, n_features, n_trees, leaf, feature, split, tree_nodes, n_outputs, nullptr,
+                          out, workspace, workspace_bytes);
 }
 
 int lbt_pack_ensemble(void* stream, int32_t x_dtype, int32_t n_features, int32_t n_trees,

@@ -123,6 +123,9 @@ def _load():
                                    C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t, C.POINTER(BuildTaps)]
     lib.lbt_build_tree_async.restype = C.c_int
     lib.lbt_build_tree_async.argtypes = lib.lbt_build_tree.argtypes
+    lib.lbt_predict_from.restype = C.c_int
+    lib.lbt_predict_from.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_int64, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p,
+                                     C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
     lib.lbt_predict.restype = C.c_int
     lib.lbt_predict.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_int64, C.c_int32, C.c_int32, C.c_void_p,
                                 C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_size_t]
@@ -238,6 +241,7 @@ except ImportError as e:
 
 EXPORTS = [
     "lbt_last_error", "lbt_version", "lbt_release_thread_resources", "lbt_build_tree_workspace_bytes", "lbt_build_tree", "lbt_build_tree_async", "lbt_predict",
+    "lbt_predict_from",
     "lbt_predict_workspace_bytes", "lbt_predict_rows_workspace_bytes", "lbt_pack_ensemble", "lbt_predict_packed",
     "lbt_update_tree_workspace_bytes", "lbt_update_tree", "lbt_update_tree_rows", "lbt_update_trees_workspace_bytes",
     "lbt_update_trees",

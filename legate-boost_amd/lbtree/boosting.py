@@ -153,6 +153,11 @@ class LBBase:
         return g, h
 
     def _predict(self, X):
+        plain = self.model_init_
+        if (self.models_ and type(self.models_[0]).batch_predict is Tree.batch_predict and isinstance(plain, torch.Tensor)
+                and plain.dtype == torch.float64 and plain.is_cuda and plain.dim() == 1 and plain.is_contiguous()
+                and not plain.requires_grad and plain.shape[0] == self.models_[0].leaf_value.shape[1]):
+            return Tree.batch_predict_from(plain, self.models_, X)
         init = self.model_init_.reshape(1, -1)
         if self.models_:
             return init + type(self.models_[0]).batch_predict(self.models_, X)

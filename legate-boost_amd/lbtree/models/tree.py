@@ -153,6 +153,13 @@ class Tree(BaseModel):
         n_outputs = models[0].leaf_value.shape[1]
         return ops.predict(X, [(m.leaf_value, m.feature, m.split_value) for m in models], n_outputs)
 
+    @staticmethod
+    def batch_predict_from(init, models: Sequence[BaseModel], X):
+        """init + batch_predict(models, X) without a pass of its own; init: a contiguous CUDA float64 tensor of the outputs."""
+        assert all(isinstance(m, Tree) for m in models)
+        models = cast(List[Tree], models)
+        return ops.predict(X, [(m.leaf_value, m.feature, m.split_value) for m in models], init.numel(), init=init)
+
     def __str__(self) -> str:
         leaf_value = self.leaf_value.cpu().numpy()
         hessian = self.hessian.cpu().numpy()

@@ -11,7 +11,13 @@ from . import _lib
 _DT = {torch.float32: _lib.LBT_F32, torch.float64: _lib.LBT_F64}
 
 
+# the current stream's handle without an object for the stream around it (0.3 us; 2.9 with)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream():
+    if _raw_stream is not None and torch.cuda.is_initialized():
+        return C.c_void_p(_raw_stream(torch.cuda.current_device()))
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
@@ -54,7 +60,10 @@ _workspace = _Scratch()
 
 def _get_workspace(nbytes, device):
     """One grow-only scratch buffer per thread, device and stream, reused by successive calls."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    if _raw_stream is not None and device.index is not None and torch.cuda.is_initialized():
+        key = (device, _raw_stream(device.index))
+    else:
+        key = (device, torch.cuda.current_stream(device).cuda_stream)
     ws = _workspace.held.get(key)
     if ws is None or ws.numel() < nbytes:
         _workspace.held[key] = None
@@ -230,9 +239,10 @@ class PackedEnsemble:
         return out
 
 
-def predict(X, trees, n_outputs, tiled=True):
+def predict(X, trees, n_outputs, tiled=True, init=None):
     """PREDICT (legateboost/models/tree.py:245-280). trees: sequence of
-    (leaf_value [nodes,K] f64, feature [nodes] i32, split_value [nodes] f64) CUDA tensors."""
+    (leaf_value [nodes,K] f64, feature [nodes] i32, split_value [nodes] f64) CUDA tensors.
+    init: what the sums are added to, a contiguous CUDA float64 tensor of n_outputs values (none: zeros)."""
     X = _check_x(X)
     n, f = X.shape
     nt = len(trees)
@@ -249,9 +259,12 @@ def predict(X, trees, n_outputs, tiled=True):
             if least >= nbytes:
                 raise
             ws = torch.empty(least, dtype=torch.uint8, device=X.device)
-    rc = _lib.lib.lbt_predict(_stream(), X.data_ptr(), _DT[X.dtype], n, f, nt, leaf_p, feat_p, split_p, nodes,
-                              n_outputs, out.data_ptr(), ws.data_ptr() if ws is not None else None,
-                              ws.numel() if ws is not None else 0)
+    if init is not None and (init.numel() != n_outputs or init.dtype != torch.float64 or init.device != X.device
+                             or not init.is_contiguous()):
+        raise _lib.LbtError("init must be a contiguous float64 tensor of %d values beside X" % n_outputs)
+    rc = _lib.lib.lbt_predict_from(_stream(), X.data_ptr(), _DT[X.dtype], n, f, nt, leaf_p, feat_p, split_p, nodes,
+                                   n_outputs, init.data_ptr() if init is not None else None, out.data_ptr(),
+                                   ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0)
     _lib.check(rc)
     return out
 

@@ -115,3 +115,31 @@ def test_keep_rows(n, k):
     want = g * mask, h * mask
     ops.keep_rows(draw, 0.3, g, h)
     assert torch.equal(g, want[0]) and torch.equal(h, want[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n_trees,k", [(1, 17, 1), (300, 105, 1), (300, 104, 3), (4096, 30, 1), (4097, 209, 1), (50000, 60, 1), (20, 3, 2),
+                                            (33, 700, 1), (100, 0, 2)])
+def test_predict_from_an_initial_prediction(rows, n_trees, k):
+    """init + the sums, by the kernel for few rows and behind the others; trees either side of what one launch packs, batches of
+    more than its first ones: bit for bit the sum of the two."""
+    from lbtree import ops
+
+    rs = np.random.RandomState(rows + n_trees)
+    f = 12
+    trees = []
+    for t in range(n_trees):
+        m, inner = 2 ** (4 + t % 5) - 1, 2 ** (3 + t % 5) - 1
+        feat = -np.ones(m, np.int32)
+        feat[:inner] = rs.randint(0, f, inner)
+        trees.append(tuple(ops.as_device(a) for a in (rs.randn(m, k), feat, rs.rand(m))))
+    init = ops.as_device(rs.randn(k))
+    for dtype in (np.float32, np.float64):
+        X = ops.as_device(rs.rand(rows, f).astype(dtype))
+        want = ops.predict(X, trees, k, tiled=False)
+        assert torch.equal(ops.predict(X, trees, k), want)
+        assert torch.equal(ops.predict(X, trees, k, init=init), init + want)
+        assert torch.equal(ops.predict(X, trees, k, tiled=False, init=init), init + want)
+        if n_trees:
+            packed = ops.PackedEnsemble(trees, k, f, X.dtype)
+            assert torch.equal(packed.predict(X), want)
