@@ -69,7 +69,7 @@ class Tree(BaseModel):
         pred (CUDA float64 [n_rows, n_outputs], updated in place) receives that leaf's value."""
         return self._fit(X, g, h, pred)
 
-    def _fit(self, X, g, h, pred) -> "Tree":
+    def _fit(self, X, g, h, pred, abs_sum_chunks=None) -> "Tree":
         X = ops.as_device(X)
         n_features = X.shape[1]
         # the seed is drawn before the feature sample, as in tree.py:125 / :139-157
@@ -91,6 +91,7 @@ class Tree(BaseModel):
             X, g, h, max_depth=self.max_depth, split_samples=self.split_samples, seed=seed,
             l1_regularization=self.l1_regularization, l2_regularization=self.l2_regularization,
             min_split_gain=self.min_split_gain, feature_set=feature_set, row_leaf=pred is not None, wait=False,
+            abs_sum_chunks=abs_sum_chunks,
         )
         if pred is not None:
             ops.add_leaf_values(pred, r.leaf_value, r.row_leaf)

@@ -143,3 +143,27 @@ def test_predict_from_an_initial_prediction(rows, n_trees, k):
         if n_trees:
             packed = ops.PackedEnsemble(trees, k, f, X.dtype)
             assert torch.equal(packed.predict(X), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("task", ["regression", "classification"])
+def test_fit_with_the_gradient_passes_sums(task):
+    """From a million rows on the gradient pass leaves the quantiser's sums: the same model as tree by tree without them."""
+    import lbtree as lb
+
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    n = 1000003
+    X = torch.rand((n, 4), generator=gen, device="cuda")
+    y = X[:, 0].to(torch.float64) + 0.1 * torch.randn(n, generator=gen, device="cuda", dtype=torch.float64)
+    kind = lb.LBRegressor if task == "regression" else lb.LBClassifier
+    y = y if task == "regression" else (y > 0.6).to(torch.float64)
+
+    class Stepwise(kind):
+        def _get_weighted_gradient(self, *args):
+            return super()._get_weighted_gradient(*args)
+
+    models = [k(n_estimators=3, base_models=(lb.models.Tree(max_depth=5),), learning_rate=0.3, random_state=2).fit(X, y)
+              for k in (kind, Stepwise)]
+    assert torch.equal(models[0]._train_pred, models[1]._train_pred)
+    for a, b in zip(*models):
+        assert all(torch.equal(getattr(a, name), getattr(b, name)) for name in ("feature", "split_value", "leaf_value", "gain", "hessian"))
