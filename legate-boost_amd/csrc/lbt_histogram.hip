@@ -483,10 +483,46 @@ __device__ inline void merge_sub_histogram(unsigned long long* s_hist, int nb, I
 // the 16 lanes of a quarter wave then always work on 16 different features modulo 16 and never
 // conflict (7 cycles per wave-level atomic where data-dependent banks cost 10 to 11 and, with
 // the same-address collisions of the 16 rows of a wave, 15 to 16 in the kernel).
+//
+// per > 0 (W = 64, groups of 49 to 56 features): the four lanes of a row take `per` features each, lane l the features from
+// per * l on, instead of 16, 16, 16 and what is left (see spread_bins). The index modulo 16 then is 4 * (c modulo 4) + l for
+// a lane's feature c < 12, and the four rows of a quarter wave take c modulo 4 in four different orders. The one or two
+// features of a lane beyond have four or two copies in the last 16 of the 64 columns, the four rows of a quarter wave
+// use different ones; whoever reads the array adds them (a group's copies together never exceed a packed sum's range:
+// the sum of a copy and of all of them is bounded by the same rows).
 struct Stripes {
   int log_w;  // log2 W; negative: the layout is [feature][bin], one run of bins per feature
   int bins;   // bins of the widest feature (rows of the striped array)
+  int per;    // 0: column p is feature p; 13 or 14: features a lane takes
   __host__ __device__ int words() const { return bins << log_w; }
+  // the feature of a column of a group of gs, -1: none, or a copy other than the first
+  __device__ int feature(int col, int gs) const
+  {
+    int f = col;
+    if (per > 0) {
+      const int l = col & 3;
+      if (col < 48)
+        f = per * l + ((col >> 2) & 3) + 4 * (col >> 4);
+      else if (per == 13)
+        f = col < 52 ? 13 * l + 12 : gs;
+      else
+        f = (col & 4) == 0 ? 14 * l + 12 + ((col - 48) >> 3) : gs;
+    }
+    return f < gs ? f : -1;
+  }
+  // word i of the array with its copies, which are cleared
+  __device__ unsigned long long take(unsigned long long* s_hist, int i) const
+  {
+    unsigned long long v = s_hist[i];
+    if (per > 0 && (i & 63) >= 48) {
+      for (int c = 4; c < (per == 13 ? 16 : 8); c += 4) {
+        v += s_hist[i + c];
+        s_hist[i + c] = 0;
+      }
+    }
+    s_hist[i] = 0;
+    return v;
+  }
 };
 
 // Merge of a striped sub-histogram into the int64 histogram of a node; s_off[p] is the place of
@@ -500,19 +536,19 @@ __device__ inline void merge_striped(unsigned long long* s_hist, const Stripes& 
 {
   const int words = st.words();
   for (int i = threadIdx.x; i < words; i += kHistThreads) {
-    const unsigned long long v = s_hist[i];
-    const int col              = i & ((1 << st.log_w) - 1);
-    if (v != 0 && col < gs) {  // columns past the group's features collect the adds of record padding
+    const int f = st.feature(i & ((1 << st.log_w) - 1), gs);
+    if (f < 0) continue;  // columns past the group's features collect the adds of record padding
+    const unsigned long long v = st.take(s_hist, i);
+    if (v != 0) {
       int32_t gv, hv;
       unpack_pair(v, gv, hv);
-      I64Pair* d = dst + s_off[col] + (i >> st.log_w);
+      I64Pair* d = dst + s_off[f] + (i >> st.log_w);
       if (sole_owner) {
         *d = I64Pair{gv, hv};
       } else {
         if (gv != 0) atomic_add_i64(&d->grad, static_cast<int64_t>(gv));
         if (hv != 0) atomic_add_i64(&d->hess, static_cast<int64_t>(hv));
       }
-      s_hist[i] = 0;
     }
   }
 }
@@ -572,9 +608,14 @@ __device__ inline void park_sub_histogram(unsigned long long* s_hist, int nb, I6
     slot = *s_slot;
   }
   if (slot < sink.slots) {
-    // the words as they lie in the LDS (striped: all of the array)
+    // the words as they lie in the LDS (striped: all of the array that is read again)
     const int words         = st.log_w >= 0 ? st.words() : nb;
     unsigned long long* out = sink.partials + static_cast<int64_t>(slot) * sink.stride;
+    if (st.per > 0) {
+      for (int i = threadIdx.x; i < words; i += kHistThreads)
+        if (st.feature(i & 63, gs) >= 0) out[i] = st.take(s_hist, i);
+      return;
+    }
     for (int i = threadIdx.x; i < words; i += kHistThreads) {
       out[i]    = s_hist[i];
       s_hist[i] = 0;
@@ -609,9 +650,10 @@ __global__ void __launch_bounds__(kHistThreads)
   int out_bin     = bin;
   if (st.log_w >= 0) {
     if (bin >= st.words()) return;
-    const int f = groups[group] + (bin & ((1 << st.log_w) - 1));
+    const int p = st.feature(bin & ((1 << st.log_w) - 1), groups[group + 1] - groups[group]);
+    const int f = groups[group] + p;
     const int b = bin >> st.log_w;
-    if (f >= groups[group + 1] || b >= row_pointers[f + 1] - row_pointers[f]) return;
+    if (p < 0 || b >= row_pointers[f + 1] - row_pointers[f]) return;
     out_bin = row_pointers[f] - bin0 + b;
   } else if (bin >= nb) {
     return;
@@ -1138,6 +1180,25 @@ __global__ void __launch_bounds__(kHistThreads)
     walk(std::false_type{});
 }
 
+// A lane's kPer bins of a row whose 64 record bytes the aligned group of four lanes holds, 16 bytes each: lane l's from
+// byte kPer * l on, of which up to three words lie with the lane before (all four have to be active).
+// m: how many. perm: the byte order of the results, which are the bins 0..3, 4..7 and 8..11 of the lane, each four
+// turned by its row's place in the quarter wave, and the word that begins with bin 12.
+template <int kPer>
+__device__ __forceinline__ uint4 spread_bins(const uint4& w, int m, uint32_t perm)
+{
+  static_assert(kPer == 13 || kPer == 14, "the words of a lane then begin with it or the one before and end with it");
+  auto before = [](uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x90, 0xf, 0xf, false));  // lanes 0, 0, 1, 2
+  };
+  const uint32_t p1 = before(w.y), p2 = before(w.z), p3 = before(w.w);
+  const bool one = (m & 1) != 0, two = (m & 2) != 0;
+  const uint32_t t0 = one ? p1 : p2, t1 = one ? p2 : p3, t2 = one ? p3 : w.x, t3 = one ? w.x : w.y, t4 = one ? w.y : w.z,
+                 t5 = one ? w.z : w.w;
+  const uint32_t o0 = two ? t0 : t2, o1 = two ? t1 : t3, o2 = two ? t2 : t4, o3 = two ? t3 : t5;
+  return make_uint4(__builtin_amdgcn_perm(o1, o0, perm), __builtin_amdgcn_perm(o2, o1, perm), __builtin_amdgcn_perm(o3, o2, perm), o3);
+}
+
 // Histogram of one level from the cached bins: a lane loads BV cached bins of its
 // row with one load and only accumulates.
 template <typename BinT, int BV>
@@ -1229,9 +1290,11 @@ __device__ __forceinline__ void turn_bytes(uint32_t w0, uint32_t w1, uint32_t w2
 // touches and holds registers until it returns, the move is one vector instruction. Below the root lane
 // u of the four loads the position of the tile's row u. The record is the four lanes' 64 bytes and its
 // last 8 the gradient pair: the pair comes out of the fourth lane's bins.
+// kPer (striped, four lanes per row in every group; 0: not): a lane takes kPer bins of a row instead of 16, of which the
+// fourth lane has mostly padding: 13 or 14 atomics for 16.
 constexpr int kStripeMaxW = 256;  // widest group the striped layout serves, in features
 
-template <typename BinT, int BV, bool kEmbed, bool kRoot, bool kStriped, bool kQuad>
+template <typename BinT, int BV, bool kEmbed, bool kRoot, bool kStriped, bool kQuad, int kPer>
 __global__ void __launch_bounds__(kHistThreads)
   binned_histogram_kernel(BinnedArgs a, LBT_WALK_PARAMS, const unsigned char* __restrict__ cache,
                           const int2* __restrict__ qgh, BinT* __restrict__ bins_t, int64_t bins_t_stride,
@@ -1239,6 +1302,7 @@ __global__ void __launch_bounds__(kHistThreads)
 {
   static_assert(!kStriped || BV == 16, "the striped layout is built for lanes that hold 16 one-byte bins");
   static_assert(!kQuad || (kStriped && kEmbed), "four lanes per 64-byte record: a mode of the striped kernel");
+  static_assert(kPer == 0 || (kStriped && (kQuad || !kEmbed)), "four lanes per row: a mode of the striped kernel");
   __shared__ int s_slot;
   __shared__ int s_off[kStriped ? kStripeMaxW : 1];  // striped: first bin of every feature in the group's run of bins
   using Word = typename BinVec<BinT, BV>::type;
@@ -1273,7 +1337,7 @@ __global__ void __launch_bounds__(kHistThreads)
   // that walk the same rows run the same instructions tile after tile and stay side by side
   // without waiting for each other: the cache line that holds a row's records is then still in the
   // L2 when the second of them asks for it.
-  const int lanes_per_row = kQuad ? 4 : (a.lanes > 0 ? a.lanes : (gs + BV - 1) / BV);
+  const int lanes_per_row = kQuad || kPer > 0 ? 4 : (a.lanes > 0 ? a.lanes : (gs + BV - 1) / BV);
   const int lr            = threadIdx.x % lanes_per_row;
   const int rsub          = threadIdx.x / lanes_per_row;
   const bool active       = rsub < w.rpp;
@@ -1317,6 +1381,22 @@ __global__ void __launch_bounds__(kHistThreads)
     pad_or = make_uint4(pw[0], pw[1], pw[2], pw[3]);
   }
   const int stripe_shift = st.log_w + 3;  // a bin's row of the striped array, in bytes
+  // kPer: the feature, in the group, that the lane takes at step v, and its column (see Stripes); qr: the row's place in
+  // the quarter wave
+  const int qr = (threadIdx.x >> 2) & 3;
+  auto spread_feature = [&](int v) {
+    const int c = v < 12 ? 4 * (v >> 2) + ((v + qr) & 3) : (kPer == 13 ? 12 : 12 + ((qr & 1) ^ (v - 12)));
+    return kPer * lr + c;
+  };
+  auto spread_column = [&](int v) {
+    if (v < 12) return 16 * (v >> 2) + 4 * ((v + qr) & 3) + lr;
+    return 48 + lr + (kPer == 13 ? 4 * qr : 8 * ((qr & 1) ^ (v - 12)) + 4 * (qr >> 1));
+  };
+  const int words_before     = 4 * lr - ((kPer * lr) >> 2);
+  const uint32_t bytes_ahead = static_cast<uint32_t>(kPer * lr) & 3u;
+  uint32_t spread_perm       = 0;
+#pragma unroll
+  for (int j = 0; j < 4; j++) spread_perm |= (bytes_ahead + static_cast<uint32_t>((j + qr) & 3)) << (8 * j);
   const unsigned long long max_abs = qstats[0];
   const int n_tiles = meta->n_tiles;
   const int t_begin = static_cast<int>(static_cast<int64_t>(n_tiles) * chunk / w.n_chunks);
@@ -1520,7 +1600,10 @@ __global__ void __launch_bounds__(kHistThreads)
         b_c[u].y |= pad_or.y;
         b_c[u].z |= pad_or.z;
         b_c[u].w |= pad_or.w;
-        b_c[u] = rotate_bytes(b_c[u], rot);
+        if constexpr (kPer > 0)
+          b_c[u] = spread_bins<kPer>(b_c[u], words_before, spread_perm);
+        else
+          b_c[u] = rotate_bytes(b_c[u], rot);
       }
     }
     if (!direct) {
@@ -1528,6 +1611,19 @@ __global__ void __launch_bounds__(kHistThreads)
       for (int u = 0; u < kRows; u++) {
         if (valid_c & (1u << u)) {
           const unsigned long long packed = pack_pair(qv[u].x, qv[u].y);
+          if constexpr (kPer > 0) {
+            const uint32_t q[3] = {b_c[u].x, b_c[u].y, b_c[u].z};
+#pragma unroll
+            for (int v = 0; v < kPer; v++) {
+              uint32_t bin;
+              if (v < 12)
+                bin = (q[v >> 2] >> (8 * (v & 3))) & 0xffu;
+              else
+                bin = (b_c[u].w >> (8 * (bytes_ahead + (kPer == 13 ? 0u : static_cast<uint32_t>((qr & 1) ^ (v - 12)))))) & 0xffu;
+              atomicAdd(reinterpret_cast<unsigned long long*>(smem_raw + ((bin << 9) + 8 * spread_column(v))), packed);
+            }
+            continue;
+          }
           int rel[BV];
           unpack_bins<BinT, BV>(b_c[u], rel);
 #pragma unroll
@@ -1552,11 +1648,21 @@ __global__ void __launch_bounds__(kHistThreads)
         if (valid_c & (1u << u)) {
           int rel[BV];
           unpack_bins<BinT, BV>(b_c[u], rel);
+          if constexpr (kPer > 0) {
+            // the bins from 12 on stand as they were loaded, the turned ones as the steps take them
 #pragma unroll
-          for (int v = 0; v < BV; v++) {
+            for (int v = 12; v < kPer; v++)
+              rel[v] = static_cast<int>((b_c[u].w >> (8 * (bytes_ahead + static_cast<uint32_t>(spread_feature(v) - kPer * lr - 12)))) & 0xffu);
+          }
+#pragma unroll
+          for (int v = 0; v < (kPer > 0 ? kPer : BV); v++) {
             bool mine;
             int bin;
-            if constexpr (kStriped) {
+            if constexpr (kPer > 0) {
+              const int f = spread_feature(v);
+              mine = f < gs;
+              bin  = mine ? s_off[f] + rel[v] : 0;
+            } else if constexpr (kStriped) {
               mine = (has & (1u << v)) != 0;
               bin  = mine ? s_off[c_base[v] >> 3] + rel[v] : 0;
             } else {
@@ -1632,15 +1738,15 @@ int launch_bin_rows_t(hipStream_t stream, const HistSetup& hs, const BinRowsArgs
   return launch_bin_rows<T, VEC, uint16_t, false>(stream, hs, a, b, grid);
 }
 
-template <typename BinT, int BV, bool kEmbed, bool kRoot, bool kStriped, bool kQuad = false>
+template <typename BinT, int BV, bool kEmbed, bool kRoot, bool kStriped, bool kQuad = false, int kPer = 0>
 int launch_binned_as(hipStream_t stream, const HistSetup& hs, const BinnedArgs& a, const HistBatch& b, unsigned grid,
                      const PartialSink& sink)
 {
   static std::atomic<bool> attr_set[kMaxDevices] = {};
   // the striped kernel keeps a table of feature offsets in static LDS and never asks for more than this
-  LBT_TRY(allow_dynamic_lds(binned_histogram_kernel<BinT, BV, kEmbed, kRoot, kStriped, kQuad>,
+  LBT_TRY(allow_dynamic_lds(binned_histogram_kernel<BinT, BV, kEmbed, kRoot, kStriped, kQuad, kPer>,
                             kStriped ? kLdsBudget - 8 * 1024 : kLdsBudget, attr_set));
-  binned_histogram_kernel<BinT, BV, kEmbed, kRoot, kStriped, kQuad><<<grid, kHistThreads, hs.blds_bytes, stream>>>(
+  binned_histogram_kernel<BinT, BV, kEmbed, kRoot, kStriped, kQuad, kPer><<<grid, kHistThreads, hs.blds_bytes, stream>>>(
     a, b.rows, hs.tiles, hs.meta, b.qstats, static_cast<const unsigned char*>(hs.binned), b.qgh,
     static_cast<BinT*>(hs.bins_t), hs.bins_t_stride,
     // meeting points only between workgroups that run at the same time: one that waits for a
@@ -1658,6 +1764,14 @@ int launch_binned(hipStream_t stream, const HistSetup& hs, const BinnedArgs& a, 
 {
   if constexpr (BV == 16) {
     if (a.stripes.log_w >= 0) {
+      if (a.stripes.per == 13) {
+        if (root) return launch_binned_as<BinT, BV, kEmbed, true, true, kEmbed, 13>(stream, hs, a, b, grid, sink);
+        return launch_binned_as<BinT, BV, kEmbed, false, true, kEmbed, 13>(stream, hs, a, b, grid, sink);
+      }
+      if (a.stripes.per == 14) {
+        if (root) return launch_binned_as<BinT, BV, kEmbed, true, true, kEmbed, 14>(stream, hs, a, b, grid, sink);
+        return launch_binned_as<BinT, BV, kEmbed, false, true, kEmbed, 14>(stream, hs, a, b, grid, sink);
+      }
       if constexpr (kEmbed) {
         if (hs.quad) {
           if (root) return launch_binned_as<BinT, BV, kEmbed, true, true, true>(stream, hs, a, b, grid, sink);
@@ -1778,7 +1892,7 @@ int hist_launch_t(hipStream_t stream, const HistSetup& hs, const HistBatch& b, i
     a.row_pointers = b.row_pointers;
     a.groups       = hs.groups;
     a.hist         = b.hist;
-    a.stripes      = Stripes{hs.stripe_log, hs.stripe_bins};
+    a.stripes      = Stripes{hs.stripe_log, hs.stripe_bins, hs.spread};
     a.lanes        = hs.even_lanes;
     a.sync_every   = kPairSyncTiles;
     PartialSink sink{hs.partials, hs.partial_lists, hs.partial_list_count, hs.partial_count, 0, hs.partial_stride};
@@ -2157,6 +2271,21 @@ int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, i
     for (int g = 0; g < hs.n_groups && hs.quad; g++) {
       const int lanes = hs.even_lanes > 0 ? hs.even_lanes : (groups[g + 1] - groups[g] + hs.bvec - 1) / hs.bvec;
       hs.quad         = lanes == 4 && rec[g].size == 64 && rec[g].q_off == 56;
+    }
+    // 13 or 14 bins a lane instead of 16 (kPer of binned_histogram_kernel), where the widest group then still fits the
+    // row's four lanes. Narrower groups go along with four lanes, whose record bytes all records have.
+    hs.spread = 0;
+    if (hs.stripe_log == 6 && (hs.quad || !hs.embed)) {
+      int widest  = 0;
+      bool whole = true;
+      for (int g = 0; g < hs.n_groups; g++) {
+        widest = std::max(widest, groups[g + 1] - groups[g]);
+        whole  = whole && rec[g].size >= 64;
+      }
+      if (whole && widest >= 49 && widest <= 56) {
+        hs.spread = widest <= 52 ? 13 : 14;
+        if (!hs.embed) hs.even_lanes = 4;
+      }
     }
     for (int g = 0; g < hs.n_groups; g++) {
       RecInfo& ri = rec[g];

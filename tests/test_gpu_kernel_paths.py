@@ -855,3 +855,26 @@ def test_tile_plans(n, depth, hist_cache_bytes):
     g, h = rs.randn(n, 1), rs.rand(n, 1) + 0.1
     gr, cr = gu.both(X, g, h, levels=True, max_depth=depth, split_samples=33, seed=6, hist_cache_bytes=hist_cache_bytes)
     gu.assert_tree_parity(gr, cr, levels=True)
+
+
+# groups of 49 to 56 features: 13 or 14 bins of a row per lane, and what lies beside (48 and 57); 100 is 52 and 48
+@pytest.mark.parametrize("f,k,s,dtype", [(48, 1, 256, np.float32), (49, 1, 256, np.float32), (49, 3, 256, np.float64), (50, 1, 64, np.float64),
+                                         (50, 2, 256, np.float32), (52, 1, 100, np.float32), (52, 5, 256, np.float32), (53, 1, 256, np.float32),
+                                         (53, 2, 64, np.float32), (54, 3, 256, np.float64), (56, 1, 256, np.float32), (56, 2, 256, np.float32),
+                                         (57, 2, 256, np.float32), (100, 1, 256, np.float32), (100, 3, 256, np.float32), (111, 2, 256, np.float32)])
+# one gradient that fills the packed sums within a tile (every row is then added by itself), after one, or never
+@pytest.mark.parametrize("share", [0.0, 1.0 / 1500.0, 0.5])
+def test_bins_spread_over_the_lanes_of_a_row(f, k, s, dtype, share):
+    import gpu_util as gu
+
+    n = 7001
+    rs = np.random.RandomState(f + k + s)
+    X = rs.randn(n, f).astype(dtype)
+    X[:, ::7] = np.floor(3 * X[:, ::7])
+    g, h = rs.randn(n, k), rs.rand(n, k) + 0.5
+    if share > 0:
+        g[n // 3, k - 1] = 0.0
+        g[n // 3, k - 1] = np.abs(g).sum() * share / (1.0 - share)
+    gr, cr = gu.both(X, g, h, levels=True, max_depth=4, split_samples=s, seed=f)
+    gu.assert_tree_parity(gr, cr, levels=True)
+    assert (cr.feature != -1).sum() > 5
