@@ -484,43 +484,49 @@ __device__ inline void merge_sub_histogram(unsigned long long* s_hist, int nb, I
 // conflict (7 cycles per wave-level atomic where data-dependent banks cost 10 to 11 and, with
 // the same-address collisions of the 16 rows of a wave, 15 to 16 in the kernel).
 //
-// per > 0 (W = 64, groups of 49 to 56 features): the four lanes of a row take `per` features each, lane l the features from
+// per > 0 (W = 64, groups of 33 to 64 features): the four lanes of a row take `per` features each, lane l the features from
 // per * l on, instead of 16, 16, 16 and what is left (see spread_bins). The index modulo 16 then is 4 * (c modulo 4) + l for
-// a lane's feature c < 12, and the four rows of a quarter wave take c modulo 4 in four different orders. The one or two
-// features of a lane beyond have four or two copies in the last 16 of the 64 columns, the four rows of a quarter wave
-// use different ones; whoever reads the array adds them (a group's copies together never exceed a packed sum's range:
-// the sum of a copy and of all of them is bounded by the same rows).
+// a lane's feature c < 12 (16 of 16), and the four rows of a quarter wave take c modulo 4 in four different orders. The one
+// or two features of a lane beyond 12 have four or two copies in the last 16 of the 64 columns, the four rows of a
+// quarter wave use different ones; whoever reads the array adds them (their sum has the range of a packed sum: it is the sum of the
+// same rows). In the LDS columns 0..31 of all bins come first and columns 32..63 follow 64 KB behind: the address of a word is
+// then a byte of the row's bins between two bytes that do not depend on them, one v_perm_b32.
 struct Stripes {
   int log_w;  // log2 W; negative: the layout is [feature][bin], one run of bins per feature
   int bins;   // bins of the widest feature (rows of the striped array)
-  int per;    // 0: column p is feature p; 13 or 14: features a lane takes
+  int per;    // 0: column p is feature p; 12, 13, 14 or 16: features a lane takes
   __host__ __device__ int words() const { return bins << log_w; }
+  // where the LDS has word i
+  __device__ int place(int i) const { return per > 0 ? ((i & 32) << 8) + ((i >> 6) << 5) + (i & 31) : i; }
   // the feature of a column of a group of gs, -1: none, or a copy other than the first
   __device__ int feature(int col, int gs) const
   {
     int f = col;
     if (per > 0) {
       const int l = col & 3;
-      if (col < 48)
+      if (col < 48 || per == 16)
         f = per * l + ((col >> 2) & 3) + 4 * (col >> 4);
       else if (per == 13)
         f = col < 52 ? 13 * l + 12 : gs;
-      else
+      else if (per == 14)
         f = (col & 4) == 0 ? 14 * l + 12 + ((col - 48) >> 3) : gs;
+      else
+        f = gs;
     }
     return f < gs ? f : -1;
   }
   // word i of the array with its copies, which are cleared
   __device__ unsigned long long take(unsigned long long* s_hist, int i) const
   {
-    unsigned long long v = s_hist[i];
-    if (per > 0 && (i & 63) >= 48) {
+    const int at = place(i);
+    unsigned long long v = s_hist[at];
+    if ((per == 13 || per == 14) && (i & 63) >= 48) {
       for (int c = 4; c < (per == 13 ? 16 : 8); c += 4) {
-        v += s_hist[i + c];
-        s_hist[i + c] = 0;
+        v += s_hist[at + c];
+        s_hist[at + c] = 0;
       }
     }
-    s_hist[i] = 0;
+    s_hist[at] = 0;
     return v;
   }
 };
@@ -1182,21 +1188,22 @@ __global__ void __launch_bounds__(kHistThreads)
 
 // A lane's kPer bins of a row whose 64 record bytes the aligned group of four lanes holds, 16 bytes each: lane l's from
 // byte kPer * l on, of which up to three words lie with the lane before (all four have to be active).
-// m: how many. perm: the byte order of the results, which are the bins 0..3, 4..7 and 8..11 of the lane, each four
-// turned by its row's place in the quarter wave, and the word that begins with bin 12.
+// m: how many. perm: the byte order of the results, which are the bins 0..3, 4..7, 8..11 (and, 16 of them, 12..15) of the lane,
+// each four turned by its row's place in the quarter wave; the last word of 13 or 14 holds the others from byte
+// kPer * l modulo 4 on, unturned.
 template <int kPer>
 __device__ __forceinline__ uint4 spread_bins(const uint4& w, int m, uint32_t perm)
 {
-  static_assert(kPer == 13 || kPer == 14, "the words of a lane then begin with it or the one before and end with it");
-  auto before = [](uint32_t v) {
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x90, 0xf, 0xf, false));  // lanes 0, 0, 1, 2
-  };
+  static_assert(kPer == 12 || kPer == 13 || kPer == 14 || kPer == 16, "a lane's bins then lie in four words, the first not before the lane before");
+  auto turn = [&](uint32_t hi, uint32_t lo) { return __builtin_amdgcn_perm(hi, lo, perm); };
+  if constexpr (kPer == 16) return make_uint4(turn(w.x, w.x), turn(w.y, w.y), turn(w.z, w.z), turn(w.w, w.w));
+  auto before = [](uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x90, 0xf, 0xf, true)); };  // lanes 0, 0, 1, 2
   const uint32_t p1 = before(w.y), p2 = before(w.z), p3 = before(w.w);
   const bool one = (m & 1) != 0, two = (m & 2) != 0;
   const uint32_t t0 = one ? p1 : p2, t1 = one ? p2 : p3, t2 = one ? p3 : w.x, t3 = one ? w.x : w.y, t4 = one ? w.y : w.z,
                  t5 = one ? w.z : w.w;
   const uint32_t o0 = two ? t0 : t2, o1 = two ? t1 : t3, o2 = two ? t2 : t4, o3 = two ? t3 : t5;
-  return make_uint4(__builtin_amdgcn_perm(o1, o0, perm), __builtin_amdgcn_perm(o2, o1, perm), __builtin_amdgcn_perm(o3, o2, perm), o3);
+  return make_uint4(turn(o1, o0), turn(o2, o1), turn(o3, o2), o3);
 }
 
 // Histogram of one level from the cached bins: a lane loads BV cached bins of its
@@ -1284,30 +1291,46 @@ __device__ __forceinline__ void turn_bytes(uint32_t w0, uint32_t w1, uint32_t w2
 // costs no second pass over the cache.
 // kStriped (one-byte bins): the LDS sub-histogram is striped (see Stripes) and every lane takes the
 // 16 bins of a row in its own rotated order.
-// kQuad (striped, kEmbed): every group of the launch has four lanes per row (and a lane four rows per
-// tile), so the lanes of a row are an aligned group of four, and what all of them need one of them loads
-// and hands round with a cross-lane move: a vector memory instruction costs by the cache lines it
-// touches and holds registers until it returns, the move is one vector instruction. Below the root lane
-// u of the four loads the position of the tile's row u. The record is the four lanes' 64 bytes and its
-// last 8 the gradient pair: the pair comes out of the fourth lane's bins.
-// kPer (striped, four lanes per row in every group; 0: not): a lane takes kPer bins of a row instead of 16, of which the
-// fourth lane has mostly padding: 13 or 14 atomics for 16.
+// kPer (striped; 0: not): every group of the launch has four lanes per row (and a lane four rows per tile), so the lanes of a
+// row are an aligned group of four. They share the row's bins evenly, kPer each, instead of 16, 16, 16 and what is left, and an
+// atomic is one vector instruction beside itself (see Stripes): 2,000,000 x 200, 8 outputs: 4.6 vector instructions an atomic
+// at 13 bins a lane, 6.7 when its address took three. What all four of them need one of them loads and hands round with a
+// cross-lane move: a vector memory instruction costs by the cache lines it touches and holds registers until it
+// returns. Below the root lane u of the four loads the position of the tile's row u and, with several outputs, its
+// gradient pair. With one output (kQuad) the record is the four lanes' 64 bytes and its last 8 the pair: it comes out of
+// the fourth lane's bins.
 constexpr int kStripeMaxW = 256;  // widest group the striped layout serves, in features
+__host__ __device__ constexpr size_t spread_hist_bytes(int bins) { return 65536 + static_cast<size_t>(bins) * 256; }
+constexpr size_t kSpreadMore = (static_cast<size_t>(kTileWindow) * 16 + 64 * 4 + 4 + 15) / 16 * 16;  // tile window, offsets, slot
 
-template <typename BinT, int BV, bool kEmbed, bool kRoot, bool kStriped, bool kQuad, int kPer>
+template <typename BinT, int BV, bool kEmbed, bool kRoot, bool kStriped, int kPer>
 __global__ void __launch_bounds__(kHistThreads)
   binned_histogram_kernel(BinnedArgs a, LBT_WALK_PARAMS, const unsigned char* __restrict__ cache,
                           const int2* __restrict__ qgh, BinT* __restrict__ bins_t, int64_t bins_t_stride,
                           int32_t* pair_sync, PartialSink sink)
 {
   static_assert(!kStriped || BV == 16, "the striped layout is built for lanes that hold 16 one-byte bins");
-  static_assert(!kQuad || (kStriped && kEmbed), "four lanes per 64-byte record: a mode of the striped kernel");
-  static_assert(kPer == 0 || (kStriped && (kQuad || !kEmbed)), "four lanes per row: a mode of the striped kernel");
-  __shared__ int s_slot;
-  __shared__ int s_off[kStriped ? kStripeMaxW : 1];  // striped: first bin of every feature in the group's run of bins
+  static_assert(kPer == 0 || kStriped, "four lanes per row: a mode of the striped kernel");
+  constexpr bool kQuad = kPer > 0 && kEmbed;
   using Word = typename BinVec<BinT, BV>::type;
   constexpr int kRows = kRoot ? 4 : (BV == 16 ? kBinnedUnroll / 2 : kBinnedUnroll);  // rows per lane and tile
   extern __shared__ __align__(16) unsigned char smem_raw[];  // 16-byte aligned whatever static LDS precedes it
+  int* s_slot;
+  int* s_off;  // striped: first bin of every feature in the group's run of bins
+  int4* s_tile_window;
+  if constexpr (kPer > 0) {
+    // behind the sub-histogram, which has to begin at address 0: no static LDS (the launch looks)
+    s_tile_window = reinterpret_cast<int4*>(smem_raw + spread_hist_bytes(a.stripes.bins));
+    s_off         = reinterpret_cast<int*>(s_tile_window + kTileWindow);
+    s_slot        = s_off + 64;
+  } else {
+    __shared__ int slot_word;
+    __shared__ int offsets[kStriped ? kStripeMaxW : 1];
+    __shared__ int4 window[kTileWindow];
+    s_slot        = &slot_word;
+    s_off         = offsets;
+    s_tile_window = window;
+  }
   const TileWalk& w = a.w;
   const int xcd   = blockIdx.x & 7;
   const int slot  = blockIdx.x >> 3;
@@ -1322,7 +1345,7 @@ __global__ void __launch_bounds__(kHistThreads)
   unsigned long long* s_hist = reinterpret_cast<unsigned long long*>(smem_raw);
   const Stripes st           = a.stripes;
   if constexpr (kStriped) {
-    for (int i = threadIdx.x; i < st.words(); i += kHistThreads) s_hist[i] = 0;
+    for (int i = threadIdx.x; i < st.words(); i += kHistThreads) s_hist[st.place(i)] = 0;
     for (int i = threadIdx.x; i < (1 << st.log_w); i += kHistThreads)
       s_off[i] = i < gs ? a.row_pointers[f0 + i] - bin0 : 0;
   } else {
@@ -1337,7 +1360,7 @@ __global__ void __launch_bounds__(kHistThreads)
   // that walk the same rows run the same instructions tile after tile and stay side by side
   // without waiting for each other: the cache line that holds a row's records is then still in the
   // L2 when the second of them asks for it.
-  const int lanes_per_row = kQuad || kPer > 0 ? 4 : (a.lanes > 0 ? a.lanes : (gs + BV - 1) / BV);
+  const int lanes_per_row = kPer > 0 ? 4 : (a.lanes > 0 ? a.lanes : (gs + BV - 1) / BV);
   const int lr            = threadIdx.x % lanes_per_row;
   const int rsub          = threadIdx.x / lanes_per_row;
   const bool active       = rsub < w.rpp;
@@ -1385,18 +1408,50 @@ __global__ void __launch_bounds__(kHistThreads)
   // the quarter wave
   const int qr = (threadIdx.x >> 2) & 3;
   auto spread_feature = [&](int v) {
-    const int c = v < 12 ? 4 * (v >> 2) + ((v + qr) & 3) : (kPer == 13 ? 12 : 12 + ((qr & 1) ^ (v - 12)));
+    const int c = v < 12 || kPer == 16 ? 4 * (v >> 2) + ((v + qr) & 3) : (kPer == 13 ? 12 : 12 + ((qr & 1) ^ (v - 12)));
     return kPer * lr + c;
-  };
-  auto spread_column = [&](int v) {
-    if (v < 12) return 16 * (v >> 2) + 4 * ((v + qr) & 3) + lr;
-    return 48 + lr + (kPer == 13 ? 4 * qr : 8 * ((qr & 1) ^ (v - 12)) + 4 * (qr >> 1));
   };
   const int words_before     = 4 * lr - ((kPer * lr) >> 2);
   const uint32_t bytes_ahead = static_cast<uint32_t>(kPer * lr) & 3u;
   uint32_t spread_perm       = 0;
 #pragma unroll
   for (int j = 0; j < 4; j++) spread_perm |= (bytes_ahead + static_cast<uint32_t>((j + qr) & 3)) << (8 * j);
+  // bytes of the words' addresses: the low ones of the steps of a group of four (a 128-byte block further in the second
+  // and fourth group, which the instruction's offset adds) and, for columns from 32 on, the 1 of the 64 KB; those of the
+  // features beyond 12
+  uint32_t low_of = 0, half_of[2] = {1u << 16, 1u << 16}, beyond[2] = {0, 0};
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const uint32_t low = 8u * static_cast<uint32_t>(4 * ((j + qr) & 3) + lr);
+    low_of |= low << (8 * j);
+    if (j < 3) half_of[0] |= low << (8 * (j == 2 ? 3 : j));
+    else half_of[1] |= low;
+  }
+#pragma unroll
+  for (int e = 0; e < 2; e++) {
+    const int x       = kPer == 13 ? 0 : (qr & 1) ^ e;  // which of the lane's features beyond 12
+    const int column  = lr + (kPer == 13 ? 4 * qr : 8 * x + 4 * (qr >> 1));
+    half_of[1] |= static_cast<uint32_t>(128 + 8 * column) << (8 * (e == 0 ? 1 : 3));
+    beyond[e] = 0x0c020000u | ((4u + bytes_ahead + static_cast<uint32_t>(x)) << 8) | (e == 0 ? 1u : 3u);
+  }
+  using LdsWord = __attribute__((address_space(3))) unsigned long long;
+  auto add_spread = [&](const uint4& bins, unsigned long long packed) {
+    auto add = [&](uint32_t address, int block) {
+      __hip_atomic_fetch_add(reinterpret_cast<LdsWord*>(static_cast<uintptr_t>(address)) + 16 * block, packed, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    const uint32_t q[4] = {bins.x, bins.y, bins.z, bins.w};
+#pragma unroll
+    for (int v = 0; v < kPer; v++) {
+      const uint32_t j = static_cast<uint32_t>(v) & 3u;
+      if (v < 8)
+        add(__builtin_amdgcn_perm(q[v >> 2], low_of, 0x0c0c0000u | ((4u + j) << 8) | j), v >> 2);
+      else if (v < 12 || kPer == 16)
+        add(__builtin_amdgcn_perm(q[v >> 2], half_of[j == 3u], 0x0c020000u | ((4u + j) << 8) | (j == 3u ? 0u : (j == 2u ? 3u : j))), (v >> 2) - 2);
+      else
+        add(__builtin_amdgcn_perm(q[3], half_of[1], beyond[v - 12]), 0);
+    }
+  };
   const unsigned long long max_abs = qstats[0];
   const int n_tiles = meta->n_tiles;
   const int t_begin = static_cast<int>(static_cast<int64_t>(n_tiles) * chunk / w.n_chunks);
@@ -1415,10 +1470,10 @@ __global__ void __launch_bounds__(kHistThreads)
   __syncthreads();
 
   // positions a lane keeps per tile: with kQuad only that of the row with its own number among the four lanes
-  constexpr int kPos = kQuad && !kRoot ? 1 : kRows;
+  constexpr int kPos = kPer > 0 && !kRoot ? 1 : kRows;
   auto load_rows = [&](const Tile& t, int (&row)[kPos]) -> unsigned {
     unsigned valid = 0;
-    if constexpr (kQuad && !kRoot) {
+    if constexpr (kPer > 0 && !kRoot) {
       const int mine = t.r0 + rsub + lr * w.rpp;
       row[0]         = positions[mine < t.r1 ? mine : t.r0];
 #pragma unroll
@@ -1437,11 +1492,13 @@ __global__ void __launch_bounds__(kHistThreads)
     }
     return valid;
   };
-  // gradient pairs a lane loads per tile: none (one unused slot) when they come out of the fourth lane's bins
-  constexpr int kPairs = kQuad ? 1 : kRows;
+  // gradient pairs a lane loads per tile: none (one unused slot) when they come out of the fourth lane's bins, one for its own
+  // row where the lanes hand them round
+  constexpr int kPairs = kQuad || (kPer > 0 && !kRoot) ? 1 : kRows;
   auto load_data = [&](const int (&row)[kPos], Word (&bw)[kRows], int2 (&q)[kPairs]) {
     int rws[kRows];
-    if constexpr (kQuad && !kRoot) {
+    if constexpr (kPer > 0 && !kRoot && !kEmbed) q[0] = qgh[static_cast<int64_t>(row[0]) * a.K + k];
+    if constexpr (kPer > 0 && !kRoot) {
       rws[0] = quad_lane<0>(row[0]);
       rws[1] = quad_lane<1>(row[0]);
       rws[2] = quad_lane<2>(row[0]);
@@ -1455,7 +1512,7 @@ __global__ void __launch_bounds__(kHistThreads)
       const int64_t rw          = rws[u];
       const unsigned char* recp = my_rec + rw * stride;
       bw[u]                     = *reinterpret_cast<const Word*>(recp + my_off);
-      if constexpr (kQuad) {
+      if constexpr (kQuad || (kPer > 0 && !kRoot)) {
       } else if constexpr (kEmbed) {
         q[u] = *reinterpret_cast<const int2*>(recp + ri.q_off);
       } else {
@@ -1464,7 +1521,6 @@ __global__ void __launch_bounds__(kHistThreads)
     }
   };
 
-  __shared__ int4 s_tile_window[kTileWindow];
   TileWindow win{s_tile_window, tiles, 0, t_end};
   win.fill(t_begin);
   Tile tc{}, tn{}, tnn{};
@@ -1506,7 +1562,37 @@ __global__ void __launch_bounds__(kHistThreads)
         __syncthreads();
       }
     }
-    if (tile + 1 < t_end) load_data(row_n, b_n, q_n);
+    // kTurned: the tile's bins are taken out of the registers they were loaded into before the next tile's are asked for, so
+    // that nothing is moved at the end of the turn
+    constexpr bool kTurned = kPer > 0 && !kRoot;
+    Word bins[kTurned ? kRows : 1];
+    int2 pairs[kTurned ? kRows : 1];
+    if constexpr (kTurned) {
+      if constexpr (!kQuad) {
+        pairs[0] = make_int2(quad_lane<0>(q_c[0].x), quad_lane<0>(q_c[0].y));
+        pairs[1] = make_int2(quad_lane<1>(q_c[0].x), quad_lane<1>(q_c[0].y));
+        pairs[2] = make_int2(quad_lane<2>(q_c[0].x), quad_lane<2>(q_c[0].y));
+        pairs[3] = make_int2(quad_lane<3>(q_c[0].x), quad_lane<3>(q_c[0].y));
+      }
+#pragma unroll
+      for (int u = 0; u < kRows; u++) {
+        Word w = b_c[u];
+        if constexpr (kQuad) {
+          pairs[u] = make_int2(quad_lane<3>(static_cast<int>(w.z)), quad_lane<3>(static_cast<int>(w.w)));
+          w.z      = strip ? 0u : w.z;
+          w.w      = strip ? 0u : w.w;
+        }
+        w.x |= pad_or.x;
+        w.y |= pad_or.y;
+        w.z |= pad_or.z;
+        w.w |= pad_or.w;
+        bins[u] = spread_bins<kPer>(w, words_before, spread_perm);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (tile + 1 < t_end) load_data(row_n, b_c, q_c);
+    } else {
+      if (tile + 1 < t_end) load_data(row_n, b_n, q_n);
+    }
     if (tile + 2 < t_end) {
       tnn      = win.get(tile + 2);
       valid_nn = load_rows(tnn, row_nn);
@@ -1519,7 +1605,7 @@ __global__ void __launch_bounds__(kHistThreads)
         __syncthreads();
         if (cur_node >= 0)
           park_sub_histogram(s_hist, nb, a.hist.at(cur_node, k, bin0), sink,
-                             (cur_node - w.level_first - w.j0) * w.n_gk + gk, &s_slot,
+                             (cur_node - w.level_first - w.j0) * w.n_gk + gk, s_slot,
                              owners && tc.node != cur_node && !node_flushed && node_rows == node_total, st, s_off,
                              gs);
         __syncthreads();
@@ -1537,12 +1623,14 @@ __global__ void __launch_bounds__(kHistThreads)
     int2 qv[kRows];
 #pragma unroll
     for (int u = 0; u < kRows; u++) {
-      if constexpr (kQuad)
+      if constexpr (kTurned)
+        qv[u] = pairs[u];
+      else if constexpr (kQuad)
         qv[u] = make_int2(quad_lane<3>(static_cast<int>(b_c[u].z)), quad_lane<3>(static_cast<int>(b_c[u].w)));
       else
         qv[u] = q_c[u];
     }
-    if constexpr (kEmbed && BV == 16) {
+    if constexpr (kEmbed && BV == 16 && !kTurned) {
 #pragma unroll
       for (int u = 0; u < kRows; u++) {
         b_c[u].z = strip ? 0u : b_c[u].z;
@@ -1592,7 +1680,7 @@ __global__ void __launch_bounds__(kHistThreads)
         }
       }
     }
-    if constexpr (kStriped) {
+    if constexpr (kStriped && !kTurned) {
       // from here on a lane's bins stand in its own order (the feature-major copy above took them as loaded)
 #pragma unroll
       for (int u = 0; u < kRows; u++) {
@@ -1612,16 +1700,10 @@ __global__ void __launch_bounds__(kHistThreads)
         if (valid_c & (1u << u)) {
           const unsigned long long packed = pack_pair(qv[u].x, qv[u].y);
           if constexpr (kPer > 0) {
-            const uint32_t q[3] = {b_c[u].x, b_c[u].y, b_c[u].z};
-#pragma unroll
-            for (int v = 0; v < kPer; v++) {
-              uint32_t bin;
-              if (v < 12)
-                bin = (q[v >> 2] >> (8 * (v & 3))) & 0xffu;
-              else
-                bin = (b_c[u].w >> (8 * (bytes_ahead + (kPer == 13 ? 0u : static_cast<uint32_t>((qr & 1) ^ (v - 12)))))) & 0xffu;
-              atomicAdd(reinterpret_cast<unsigned long long*>(smem_raw + ((bin << 9) + 8 * spread_column(v))), packed);
-            }
+            if constexpr (kTurned)
+              add_spread(bins[u], packed);
+            else
+              add_spread(b_c[u], packed);
             continue;
           }
           int rel[BV];
@@ -1647,12 +1729,16 @@ __global__ void __launch_bounds__(kHistThreads)
       for (int u = 0; u < kRows; u++) {
         if (valid_c & (1u << u)) {
           int rel[BV];
-          unpack_bins<BinT, BV>(b_c[u], rel);
-          if constexpr (kPer > 0) {
+          if constexpr (kTurned)
+            unpack_bins<BinT, BV>(bins[u], rel);
+          else
+            unpack_bins<BinT, BV>(b_c[u], rel);
+          if constexpr (kPer == 13 || kPer == 14) {
             // the bins from 12 on stand as they were loaded, the turned ones as the steps take them
+            const uint32_t last = kTurned ? bins[kTurned ? u : 0].w : b_c[u].w;
 #pragma unroll
             for (int v = 12; v < kPer; v++)
-              rel[v] = static_cast<int>((b_c[u].w >> (8 * (bytes_ahead + static_cast<uint32_t>(spread_feature(v) - kPer * lr - 12)))) & 0xffu);
+              rel[v] = static_cast<int>((last >> (8 * (bytes_ahead + static_cast<uint32_t>(spread_feature(v) - kPer * lr - 12)))) & 0xffu);
           }
 #pragma unroll
           for (int v = 0; v < (kPer > 0 ? kPer : BV); v++) {
@@ -1686,15 +1772,17 @@ __global__ void __launch_bounds__(kHistThreads)
       row_c[u] = row_n[u];
       row_n[u] = row_nn[u];
     }
+    if constexpr (!kTurned) {
 #pragma unroll
-    for (int u = 0; u < kRows; u++) b_c[u] = b_n[u];
+      for (int u = 0; u < kRows; u++) b_c[u] = b_n[u];
 #pragma unroll
-    for (int u = 0; u < kPairs; u++) q_c[u] = q_n[u];
+      for (int u = 0; u < kPairs; u++) q_c[u] = q_n[u];
+    }
   }
   __syncthreads();
   if (cur_node >= 0)
     park_sub_histogram(s_hist, nb, a.hist.at(cur_node, k, bin0), sink, (cur_node - w.level_first - w.j0) * w.n_gk + gk,
-                       &s_slot, owners && !node_flushed && node_rows == node_total, st, s_off, gs);
+                       s_slot, owners && !node_flushed && node_rows == node_total, st, s_off, gs);
 }
 
 template <typename T, int VEC, bool kIdentityRows>
@@ -1738,15 +1826,24 @@ int launch_bin_rows_t(hipStream_t stream, const HistSetup& hs, const BinRowsArgs
   return launch_bin_rows<T, VEC, uint16_t, false>(stream, hs, a, b, grid);
 }
 
-template <typename BinT, int BV, bool kEmbed, bool kRoot, bool kStriped, bool kQuad = false, int kPer = 0>
+template <typename BinT, int BV, bool kEmbed, bool kRoot, bool kStriped, int kPer = 0>
 int launch_binned_as(hipStream_t stream, const HistSetup& hs, const BinnedArgs& a, const HistBatch& b, unsigned grid,
                      const PartialSink& sink)
 {
   static std::atomic<bool> attr_set[kMaxDevices] = {};
   // the striped kernel keeps a table of feature offsets in static LDS and never asks for more than this
-  LBT_TRY(allow_dynamic_lds(binned_histogram_kernel<BinT, BV, kEmbed, kRoot, kStriped, kQuad, kPer>,
+  LBT_TRY(allow_dynamic_lds(binned_histogram_kernel<BinT, BV, kEmbed, kRoot, kStriped, kPer>,
                             kStriped ? kLdsBudget - 8 * 1024 : kLdsBudget, attr_set));
-  binned_histogram_kernel<BinT, BV, kEmbed, kRoot, kStriped, kQuad, kPer><<<grid, kHistThreads, hs.blds_bytes, stream>>>(
+  if constexpr (kPer > 0) {
+    static std::atomic<int> static_lds{-1};
+    if (static_lds.load(std::memory_order_relaxed) < 0) {
+      hipFuncAttributes at{};
+      LBT_HIP(hipFuncGetAttributes(&at, reinterpret_cast<const void*>(&binned_histogram_kernel<BinT, BV, kEmbed, kRoot, kStriped, kPer>)));
+      static_lds.store(static_cast<int>(at.sharedSizeBytes), std::memory_order_relaxed);
+    }
+    LBT_REQUIRE(static_lds.load(std::memory_order_relaxed) == 0, "the sub-histogram has to begin at address 0 of the LDS");
+  }
+  binned_histogram_kernel<BinT, BV, kEmbed, kRoot, kStriped, kPer><<<grid, kHistThreads, hs.blds_bytes, stream>>>(
     a, b.rows, hs.tiles, hs.meta, b.qstats, static_cast<const unsigned char*>(hs.binned), b.qgh,
     static_cast<BinT*>(hs.bins_t), hs.bins_t_stride,
     // meeting points only between workgroups that run at the same time: one that waits for a
@@ -1764,19 +1861,19 @@ int launch_binned(hipStream_t stream, const HistSetup& hs, const BinnedArgs& a, 
 {
   if constexpr (BV == 16) {
     if (a.stripes.log_w >= 0) {
-      if (a.stripes.per == 13) {
-        if (root) return launch_binned_as<BinT, BV, kEmbed, true, true, kEmbed, 13>(stream, hs, a, b, grid, sink);
-        return launch_binned_as<BinT, BV, kEmbed, false, true, kEmbed, 13>(stream, hs, a, b, grid, sink);
-      }
-      if (a.stripes.per == 14) {
-        if (root) return launch_binned_as<BinT, BV, kEmbed, true, true, kEmbed, 14>(stream, hs, a, b, grid, sink);
-        return launch_binned_as<BinT, BV, kEmbed, false, true, kEmbed, 14>(stream, hs, a, b, grid, sink);
-      }
-      if constexpr (kEmbed) {
-        if (hs.quad) {
-          if (root) return launch_binned_as<BinT, BV, kEmbed, true, true, true>(stream, hs, a, b, grid, sink);
-          return launch_binned_as<BinT, BV, kEmbed, false, true, true>(stream, hs, a, b, grid, sink);
-        }
+      auto spread = [&](auto per_c) {
+        constexpr int kPer = decltype(per_c)::value;
+        if (root) return launch_binned_as<BinT, BV, kEmbed, true, true, kPer>(stream, hs, a, b, grid, sink);
+        return launch_binned_as<BinT, BV, kEmbed, false, true, kPer>(stream, hs, a, b, grid, sink);
+      };
+      switch (a.stripes.per) {
+        case 12: return spread(std::integral_constant<int, 12>{});
+        case 13: return spread(std::integral_constant<int, 13>{});
+        case 14: return spread(std::integral_constant<int, 14>{});
+        case 16:
+          if constexpr (!kEmbed) return spread(std::integral_constant<int, 16>{});
+          break;
+        default: break;
       }
       if (root) return launch_binned_as<BinT, BV, kEmbed, true, true>(stream, hs, a, b, grid, sink);
       return launch_binned_as<BinT, BV, kEmbed, false, true>(stream, hs, a, b, grid, sink);
@@ -2264,27 +2361,22 @@ int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, i
       fits = fits && lanes * hs.bvec <= (1 << hs.stripe_log);
       if (fits) hs.even_lanes = lanes;
     }
-    // the kernel's mode for four lanes per row (see binned_histogram_kernel): single-output trees whose
-    // groups all have four lanes per row, by their own width or by even_lanes, and records of those lanes'
-    // 64 bytes with the pair in the last 8 (with several outputs the mode saves no load and was no faster)
-    hs.quad = hs.stripe_log >= 0 && hs.embed && kBinnedUnroll / 2 == 4;
-    for (int g = 0; g < hs.n_groups && hs.quad; g++) {
-      const int lanes = hs.even_lanes > 0 ? hs.even_lanes : (groups[g + 1] - groups[g] + hs.bvec - 1) / hs.bvec;
-      hs.quad         = lanes == 4 && rec[g].size == 64 && rec[g].q_off == 56;
-    }
-    // 13 or 14 bins a lane instead of 16 (kPer of binned_histogram_kernel), where the widest group then still fits the
-    // row's four lanes. Narrower groups go along with four lanes, whose record bytes all records have.
+    // Four lanes per row that share its bins evenly (kPer of binned_histogram_kernel), where the widest group needs three or
+    // four lanes of 16 and all records have the bytes of four; with one output the pair in the last 8 of 64. Groups of up to 48
+    // features take four lanes of 12 for three of 16.
     hs.spread = 0;
-    if (hs.stripe_log == 6 && (hs.quad || !hs.embed)) {
+    if (hs.stripe_log == 6) {
       int widest  = 0;
       bool whole = true;
       for (int g = 0; g < hs.n_groups; g++) {
         widest = std::max(widest, groups[g + 1] - groups[g]);
-        whole  = whole && rec[g].size >= 64;
+        whole  = whole && (hs.embed ? rec[g].size == 64 && rec[g].q_off == 56 : rec[g].size >= 64);
       }
-      if (whole && widest >= 49 && widest <= 56) {
-        hs.spread = widest <= 52 ? 13 : 14;
-        if (!hs.embed) hs.even_lanes = 4;
+      if (whole) {
+        hs.spread     = widest <= 48 ? 12 : (widest <= 52 ? 13 : (widest <= 56 ? 14 : 16));
+        hs.even_lanes = 4;
+        hs.brpp       = kHistThreads / 4;
+        hs.blds_bytes = spread_hist_bytes(hs.stripe_bins) + kSpreadMore;
       }
     }
     for (int g = 0; g < hs.n_groups; g++) {

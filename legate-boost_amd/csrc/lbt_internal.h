@@ -412,8 +412,7 @@ struct HistSetup {
   int stripe_log       = -1;       // log2 of the striped layout's row width in features; negative: [feature][bin]
   int stripe_bins      = 0;        // bins of the widest feature (rows of the striped array)
   int even_lanes       = 0;        // lanes per row shared by all groups of a histogram launch; 0: per group
-  int spread           = 0;        // bins a lane takes of a row where 16 would leave the fourth lane padding (Stripes::per); 0: 16
-  bool quad            = false;    // single-output trees, four lanes per 64-byte record in every group: the histogram kernel's kQuad mode
+  int spread           = 0;        // bins a lane takes of a row where four lanes share them evenly (Stripes::per); 0: they do not
   RecInfo* rec         = nullptr;  // [n_groups]
   int64_t max_rec_stride = 0;      // widest record, bytes
   int pieces           = 0;        // 16-byte pieces of bins of a row's records

@@ -857,11 +857,14 @@ def test_tile_plans(n, depth, hist_cache_bytes):
     gu.assert_tree_parity(gr, cr, levels=True)
 
 
-# groups of 49 to 56 features: 13 or 14 bins of a row per lane, and what lies beside (48 and 57); 100 is 52 and 48
-@pytest.mark.parametrize("f,k,s,dtype", [(48, 1, 256, np.float32), (49, 1, 256, np.float32), (49, 3, 256, np.float64), (50, 1, 64, np.float64),
-                                         (50, 2, 256, np.float32), (52, 1, 100, np.float32), (52, 5, 256, np.float32), (53, 1, 256, np.float32),
-                                         (53, 2, 64, np.float32), (54, 3, 256, np.float64), (56, 1, 256, np.float32), (56, 2, 256, np.float32),
-                                         (57, 2, 256, np.float32), (100, 1, 256, np.float32), (100, 3, 256, np.float32), (111, 2, 256, np.float32)])
+# groups of 33 to 64 features: 12, 13, 14 or 16 bins of a row per lane (one output: up to 56), and what lies beside; 100 is 52 and 48
+@pytest.mark.parametrize("f,k,s,dtype", [(32, 1, 256, np.float32), (33, 1, 256, np.float32), (33, 2, 256, np.float64), (43, 1, 200, np.float32),
+                                         (47, 3, 256, np.float32), (48, 1, 256, np.float32), (49, 1, 256, np.float32), (49, 3, 256, np.float64),
+                                         (50, 1, 64, np.float64), (50, 2, 256, np.float32), (52, 1, 100, np.float32), (52, 5, 256, np.float32),
+                                         (53, 1, 256, np.float32), (53, 2, 64, np.float32), (54, 3, 256, np.float64), (56, 1, 256, np.float32),
+                                         (56, 2, 256, np.float32), (57, 1, 256, np.float32), (57, 2, 256, np.float32), (64, 1, 8, np.float32),
+                                         (64, 2, 256, np.float32), (65, 2, 32, np.float32), (80, 1, 256, np.float32), (90, 2, 256, np.float32),
+                                         (100, 1, 256, np.float32), (100, 3, 256, np.float32), (111, 2, 256, np.float32), (130, 1, 256, np.float32)])
 # one gradient that fills the packed sums within a tile (every row is then added by itself), after one, or never
 @pytest.mark.parametrize("share", [0.0, 1.0 / 1500.0, 0.5])
 def test_bins_spread_over_the_lanes_of_a_row(f, k, s, dtype, share):
