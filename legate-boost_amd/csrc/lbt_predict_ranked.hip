@@ -311,8 +311,11 @@ __device__ __forceinline__ int row_place(int row) { return (row & ~63) + 2 * (ro
 // ranks: [tile][feature][place of the row]
 // What bounds it are vector instructions, four per probe of a search and feature. With cells to start from a feature
 // of 4000 evenly spread thresholds takes 4 or 5 probes instead of 12 (20,000,000 x 64: 6.1 ms without cells, 2.8 with).
+// The features of a line come without their next row on its way; two workgroups to a CU wait for one another's rows instead: floats four
+// features at a time (59 registers, eight waves a SIMD; 500,003 x 200 with 50 trees and 8 outputs 468 -> 448 us a call against eight
+// at a time, 74 registers). Doubles take 63 with a spill that way and gained nothing: eight at a time, 87.
 template <typename T, int kGroup, int kSub>
-__global__ void __launch_bounds__(kWalkThreads)
+__global__ void __launch_bounds__(kWalkThreads, kSub > 1 && sizeof(T) == 4 ? 8 : 4)
   rank_rows_kernel(const T* __restrict__ X, RankRows a, RankState st, const T* __restrict__ sorted,
                    uint16_t* __restrict__ ranks)
 {
@@ -440,6 +443,7 @@ __global__ void __launch_bounds__(kWalkThreads)
     const uint32_t at0 = 2 * row_place(static_cast<int>(row) & ((1 << a.tile_shift) - 1));
 #pragma unroll
     for (int s = 0; s < kSub; s++) {
+      if (s * kGroup >= nf) break;  // the last features' workgroups
       if constexpr (kSub > 1) {
         asm volatile("" ::: "memory");  // not kept in registers for all groups
         take_features(s);
@@ -976,7 +980,11 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
       case 2: LBT_TRY(rank_chunk(integral_constant<int, 2>{}, one, rank_attr[1], x, rows)); break;
       case 4: LBT_TRY(rank_chunk(integral_constant<int, 4>{}, one, rank_attr[2], x, rows)); break;
       case 8: LBT_TRY(rank_chunk(integral_constant<int, 8>{}, one, rank_attr[3], x, rows)); break;
-      default: LBT_TRY(rank_chunk(integral_constant<int, 8>{}, integral_constant<int, 16 / sizeof(T)>{}, rank_attr[4], x, rows)); break;
+      default: {
+        constexpr int kLineGroup = sizeof(T) == 4 ? 4 : 8;
+        LBT_TRY(rank_chunk(integral_constant<int, kLineGroup>{}, integral_constant<int, 128 / (kLineGroup * sizeof(T))>{}, rank_attr[4], x, rows));
+        break;
+      }
     }
     auto with = [&](auto adds_c, auto items_c, int at) -> int {
       switch (p.shape.j) {
