@@ -107,6 +107,17 @@ def test_nan_thresholds_on_features_without_others(n, f, n_trees, depth, nan_fro
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("f", [513, 515, 516, 518, 543])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_last_features_of_a_cache_line(f, dtype):
+    """Features by the cache line, a few at a time: the last line has one, some of a step's, a step's and more, all but one."""
+    rs = np.random.RandomState(f)
+    trees = _ensemble(rs, 40, 5, f, 1, dtype, 0)
+    X = _rows(rs, 70_003, f, dtype, 0)
+    assert _takes_ranks(X, trees, 1)
+    assert torch.equal(ops.predict(X, trees, 1), ops.predict(X, trees, 1, tiled=False))
+
+
 def test_a_start_off_a_16_byte_boundary():
     rs = np.random.RandomState(5)
     trees = _ensemble(rs, 130, 6, 8, 1, np.float32, 0)
