@@ -65,3 +65,10 @@ def test_histogram_kernels_keep_their_registers(kernels, arguments, spilled):
     match = [k for name, k in kernels.items() if "binned_histogram_kernelI" + arguments + "E" in name]
     assert len(match) == 1
     assert match[0].get(".vgpr_spill_count", 0) <= spilled
+
+
+def test_scans_that_decide_use_no_scratch_memory(kernels):
+    """They ask for all that they read before the first answer is waited for; what is kept in scratch memory is waited for."""
+    match = [k for name, k in kernels.items() if "small_scan_kernelI" in name and "ELb1ELb1EE" in name]
+    assert len(match) == 3
+    assert [k[".private_segment_fixed_size"] for k in match] == [0, 0, 0]
