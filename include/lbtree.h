@@ -324,7 +324,7 @@ int lbt_predict(void* stream, const void* X, int32_t x_dtype, int64_t n_rows, in
                 double* out, void* workspace, size_t workspace_bytes);
 
 /* The same with out = init + the sums (LBBase._predict, legateboost/legateboost.py:507-529); init: device double
- * [n_outputs], or NULL: lbt_predict. May not alias out. */
+ * [n_outputs], or NULL: lbt_predict. May not overlap out. */
 int lbt_predict_from(void* stream, const void* X, int32_t x_dtype, int64_t n_rows, int32_t n_features,
                      int32_t n_trees, const double* const* leaf, const int32_t* const* feature,
                      const double* const* split, const int32_t* tree_nodes, int32_t n_outputs,

@@ -1118,11 +1118,14 @@ int lbt_predict_from(void* stream, const void* X, int32_t x_dtype, int64_t n_row
   // predict.cu:35: a shard without rows has nothing to do
   if (n_rows < 1) return LBT_OK;
   LBT_REQUIRE(X && out, "null X or output");
+  const int64_t n = n_rows * n_outputs;
+  LBT_REQUIRE(init == nullptr || reinterpret_cast<uintptr_t>(init + n_outputs) <= reinterpret_cast<uintptr_t>(out) ||
+                reinterpret_cast<uintptr_t>(out + n) <= reinterpret_cast<uintptr_t>(init),
+              "the initial prediction and the output overlap");
   LBT_REQUIRE(n_trees == 0 || (leaf && feature && split && tree_nodes), "null tree arrays");
   for (int i = 0; i < n_trees; i++)
     LBT_REQUIRE(leaf[i] && feature[i] && split[i] && tree_nodes[i] >= 1, "tree %d is incomplete", i);
-  hipStream_t s   = static_cast<hipStream_t>(stream);
-  const int64_t n = n_rows * n_outputs;
+  hipStream_t s = static_cast<hipStream_t>(stream);
   if (n_trees == 0) {
     lbt::zero_doubles_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(out, n);
   } else if (x_dtype == LBT_F32) {

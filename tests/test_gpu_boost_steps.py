@@ -26,6 +26,19 @@ def test_calls_check_their_arguments():
     assert lib.lbt_keep_rows(None, None, 0.5, 0, 1, None, None) == 0
 
 
+@pytest.mark.parametrize("init,out,refused", [(512, 512, True), (512 + 8 * 29, 512, True), (512, 512 + 8 * 2, True),
+                                              (512 - 8 * 3, 512, False), (512 + 8 * 30, 512, False)])
+def test_initial_predictions_may_not_lie_in_the_output(init, out, refused):
+    """10 rows of 3 outputs. What is not refused here goes on to the next check, a tree without nodes."""
+    from lbtree import _lib
+
+    ptr, nodes = (C.c_void_p * 1)(16), (C.c_int32 * 1)(0)
+    rc = _lib.lib.lbt_predict_from(None, C.c_void_p(16), _lib.LBT_F32, 10, 4, 1, ptr, ptr, ptr, nodes, 3, C.c_void_p(init),
+                                   C.c_void_p(out), None, 0)
+    assert rc == -1
+    assert (b"overlap" in _lib.lib.lbt_last_error()) == refused
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,k", [(1, 1), (257, 1), (1, 2), (255, 3), (513, 8), (300, 10), (1000, 16), (70, 7), (40, 19), (3, 300)])
 def test_class_probabilities(n, k):
