@@ -21,6 +21,18 @@ def _check_random_state(seed):
     raise ValueError("%r cannot be used to seed a RandomState" % seed)
 
 
+def _as_defined(obj, owner, *names):
+    """Whether these methods of obj are the ones this package defines for `owner`: overridden by no subclass and replaced neither
+    on the object nor on a class. What bypasses a method asks this first."""
+    return all(getattr(type(obj), n) is _DEFINED[owner][n] and n not in vars(obj) for n in names)
+
+
+def _float64_on_device(a):
+    """Whether the library's kernels can take `a` as it is, and no gradient is recorded through it."""
+    return (isinstance(a, torch.Tensor) and a.dtype == torch.float64 and a.is_cuda and a.is_contiguous()
+            and not a.requires_grad)
+
+
 class SquaredErrorObjective:
     fused = "squared_error"  # ops.weighted_gradient computes transform + gradient + weighting in one pass
 
@@ -118,11 +130,11 @@ class LBBase:
         """The rows' weights; None (all ones) where nothing but this module's own code sees them."""
         if sample_weight is not None:
             return ops.as_device(sample_weight, torch.float64)
-        own = ("_get_weighted_gradient", "_loss")
-        plain = (type(self) in (LBRegressor, LBClassifier) and not any(a in vars(self) for a in own)
-                 and type(self)._get_weighted_gradient is LBBase._get_weighted_gradient
-                 and type(self._objective_instance) in (SquaredErrorObjective, LogLossObjective)
-                 and not vars(self._objective_instance) and not self.verbose)
+        objective = self._objective_instance
+        plain = (type(self) in (LBRegressor, LBClassifier) and not self.verbose
+                 and _as_defined(self, LBBase, "_get_weighted_gradient")
+                 and type(objective) in (SquaredErrorObjective, LogLossObjective) and not vars(objective)
+                 and _as_defined(objective, type(objective), "gradient", "transform", "initialise_prediction"))
         return None if plain else torch.ones(y.shape[0], dtype=torch.float64, device=y.device)
 
     def _get_weighted_gradient(self, y, pred, sample_weight, learning_rate):
@@ -154,9 +166,8 @@ class LBBase:
 
     def _predict(self, X):
         plain = self.model_init_
-        if (self.models_ and type(self.models_[0]).batch_predict is Tree.batch_predict and isinstance(plain, torch.Tensor)
-                and plain.dtype == torch.float64 and plain.is_cuda and plain.dim() == 1 and plain.is_contiguous()
-                and not plain.requires_grad and plain.shape[0] == self.models_[0].leaf_value.shape[1]):
+        if (self.models_ and _as_defined(self.models_[0], Tree, "batch_predict") and _float64_on_device(plain)
+                and plain.dim() == 1 and plain.shape[0] == self.models_[0].leaf_value.shape[1]):
             return Tree.batch_predict_from(plain, self.models_, X)
         init = self.model_init_.reshape(1, -1)
         if self.models_:
@@ -181,13 +192,10 @@ class LBBase:
         fused = getattr(self._objective_instance, "fused", None)
         sums = (fused is not None and self.subsample == 1.0 and train_pred.is_cuda
                 and train_pred.shape[1] == 1 and train_pred.shape[0] >= 1000000
-                and type(self)._get_weighted_gradient is LBBase._get_weighted_gradient
-                and "_get_weighted_gradient" not in vars(self))
-        own = ("fit", "fit_update_predictions", "_fit")
+                and _as_defined(self, LBBase, "_get_weighted_gradient"))
         for i in range(self.n_estimators):
             model = deepcopy(self.base_models[i % len(self.base_models)]).set_random_state(self.random_state_)
-            if sums and isinstance(model, Tree) and all(getattr(type(model), a) is getattr(Tree, a) and a not in vars(model)
-                                                        for a in own):
+            if sums and isinstance(model, Tree) and _as_defined(model, Tree, "fit", "fit_update_predictions", "_fit"):
                 g, h, chunks = ops.weighted_gradient(fused, y, train_pred, w, self.learning_rate, sums=True)
                 model._fit(X, g, h, train_pred, chunks)
             else:
@@ -214,7 +222,7 @@ class LBBase:
         pred = self.model_init_.reshape(1, -1).repeat(X.shape[0], 1).contiguous()
         fused = getattr(self._objective_instance, "fused", None)
         if (fused is not None and self.subsample == 1.0 and X.shape[0] > 0
-                and type(self)._get_weighted_gradient is LBBase._get_weighted_gradient
+                and _as_defined(self, LBBase, "_get_weighted_gradient")
                 and Tree.update_rounds(self.models_, X, y, w, fused, self.learning_rate, pred)):
             return self
         for m in self.models_:
@@ -255,12 +263,11 @@ class LBClassifier(LBBase):
     def predict_proba(self, X):
         X = ops.as_device(X)
         objective, init = self._objective_instance, self.model_init_
-        if (type(objective) is LogLossObjective and not vars(objective) and self.models_
-                and type(self)._predict is LBBase._predict and "_predict" not in vars(self)):
+        if (type(objective) is LogLossObjective and _as_defined(objective, LogLossObjective, "transform") and self.models_
+                and _as_defined(self, LBBase, "_predict")):
             raw = type(self.models_[0]).batch_predict(self.models_, X)
-            if all(isinstance(a, torch.Tensor) and a.dtype == torch.float64 and a.is_cuda and a.is_contiguous()
-                   and not a.requires_grad for a in (raw, init)) \
-                    and raw.dim() == 2 and init.shape == raw.shape[1:] and init.device == raw.device:
+            if (_float64_on_device(raw) and _float64_on_device(init) and raw.dim() == 2
+                    and init.shape == raw.shape[1:] and init.device == raw.device):
                 return ops.class_probabilities(raw, init)
             p = objective.transform(init.reshape(1, -1) + raw)
         else:
@@ -271,3 +278,12 @@ class LBClassifier(LBBase):
 
     def predict(self, X):
         return self.predict_proba(X).argmax(dim=1)
+
+
+# the methods as they stand here, whatever is put in their place later
+_DEFINED = {cls: {n: getattr(cls, n) for n in names} for cls, names in (
+    (LBBase, ("_get_weighted_gradient", "_predict")),
+    (SquaredErrorObjective, ("gradient", "transform", "initialise_prediction")),
+    (LogLossObjective, ("gradient", "transform", "initialise_prediction")),
+    (Tree, ("fit", "fit_update_predictions", "_fit", "batch_predict")),
+)}

@@ -180,3 +180,50 @@ def test_fit_with_the_gradient_passes_sums(task):
     assert torch.equal(models[0]._train_pred, models[1]._train_pred)
     for a, b in zip(*models):
         assert all(torch.equal(getattr(a, name), getattr(b, name)) for name in ("feature", "split_value", "leaf_value", "gain", "hessian"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [5000, 1000000])
+def test_fits_and_updates_call_a_replaced_gradient_step(monkeypatch, rows):
+    """Replaced on the class that defines it, not on a subclass: the fits that form the gradients themselves must not pass it by."""
+    import lbtree as lb
+    from lbtree.boosting import LBBase
+
+    seen, own = [], LBBase._get_weighted_gradient
+
+    def step(self, y, pred, sample_weight, learning_rate):
+        seen.append(tuple(sample_weight.shape))
+        return own(self, y, pred, sample_weight, learning_rate)
+
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    X = torch.rand((rows, 4), generator=gen, device="cuda")
+    model = lb.LBRegressor(n_estimators=2, base_models=(lb.models.Tree(max_depth=2, split_samples=16),), random_state=1)
+    monkeypatch.setattr(LBBase, "_get_weighted_gradient", step)
+    model.fit(X, X[:, 0].double())
+    assert seen == 2 * [(rows,)]
+    model.update(X, X[:, 1].double())
+    assert seen == 4 * [(rows,)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("owner,name", [("LBBase", "_predict"), ("LogLossObjective", "transform"), ("Tree", "batch_predict")])
+def test_predictions_call_what_has_been_replaced(monkeypatch, owner, name):
+    import lbtree as lb
+    from lbtree import boosting
+
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    X = torch.rand((300, 4), generator=gen, device="cuda")
+    model = lb.LBClassifier(n_estimators=2, base_models=(lb.models.Tree(max_depth=2, split_samples=16),), random_state=1)
+    model.fit(X, (X[:, 0] > 0.5).double())
+    want = model.predict_proba(X)
+    cls, calls = getattr(boosting, owner), []
+    own = getattr(cls, name)
+
+    def replaced(*args):
+        calls.append(name)
+        return own(*args)
+
+    monkeypatch.setattr(cls, name, staticmethod(replaced) if name == "batch_predict" else replaced)
+    assert torch.allclose(model.predict_proba(X), want, rtol=0, atol=1e-15) and len(calls) == 1
+    model._predict(X)
+    assert len(calls) == (1 if name == "transform" else 2)
