@@ -1241,7 +1241,7 @@ int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelA
 // feature and kDecidePasses of them for the nodes, a thread for every node, and the LDS for both levels' nodes.
 bool next_scan_decides(const SmallTreeState& st, int64_t N, int F, int K, int depth, int max_depth)
 {
-  if (st.left[0] == nullptr || K > 1 || depth + 1 >= max_depth || N > kDecideRows) return false;
+  if (st.left[0] == nullptr || K > 1 || F > kSmallDecideFeatures || depth + 1 >= max_depth || N > kDecideRows) return false;
   const int threads = N <= 1024 ? 512 : small_scan_places(N) / 4;
   int lanes = 1 << kDecideLanes;
   while (lanes < F) lanes *= 2;
