@@ -1314,6 +1314,7 @@ __global__ void __launch_bounds__(kHistThreads)
   constexpr bool kQuad = kPer > 0 && kEmbed;
   using Word = typename BinVec<BinT, BV>::type;
   constexpr int kRows = kRoot ? 4 : (BV == 16 ? kBinnedUnroll / 2 : kBinnedUnroll);  // rows per lane and tile
+  static_assert(kPer == 0 || kRows == 4, "each of a row's four lanes asks for one of the tile's four rows");
   extern __shared__ __align__(16) unsigned char smem_raw[];  // 16-byte aligned whatever static LDS precedes it
   int* s_slot;
   int* s_off;  // striped: first bin of every feature in the group's run of bins
@@ -1834,7 +1835,8 @@ int launch_binned_as(hipStream_t stream, const HistSetup& hs, const BinnedArgs& 
                      const PartialSink& sink)
 {
   static std::atomic<bool> attr_set[kMaxDevices] = {};
-  // the striped kernel keeps a table of feature offsets in static LDS and never asks for more than this
+  // the striped kernel without kPer keeps a table of feature offsets and its tile window in static LDS; with kPer they lie behind the
+  // sub-histogram: neither asks for more than this
   LBT_TRY(allow_dynamic_lds(binned_histogram_kernel<BinT, BV, kEmbed, kRoot, kStriped, kPer>,
                             kStriped ? kLdsBudget - 8 * 1024 : kLdsBudget, attr_set));
   if constexpr (kPer > 0) {

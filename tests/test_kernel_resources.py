@@ -1,6 +1,7 @@
 """What the compiler gave the kernels, from the metadata of the gfx950 code objects in liblbtree.so (built here from source):
 registers that were moved to memory, and bytes of scratch memory per lane."""
 import os
+import re
 import struct
 
 import pytest
@@ -72,3 +73,10 @@ def test_scans_that_decide_use_no_scratch_memory(kernels):
     match = [k for name, k in kernels.items() if "small_scan_kernelI" in name and "ELb1ELb1EE" in name]
     assert len(match) == 3
     assert [k[".private_segment_fixed_size"] for k in match] == [0, 0, 0]
+
+
+def test_histogram_kernels_that_address_the_lds_from_0_have_no_static_lds(kernels):
+    """Their launch refuses to run otherwise: this is where a __shared__ variable too many shows."""
+    match = [k for name, k in kernels.items() if "binned_histogram_kernelIhLi16E" in name and re.search("ELb1ELi1[2346]EE", name)]
+    assert len(match) == 14
+    assert {k[".group_segment_fixed_size"] for k in match} == {0}
