@@ -347,10 +347,17 @@ __device__ __forceinline__ void add_range(const DirectLevel& a, int range, int p
     unsigned long long* sum = a.large + slot * kPer * width;
     for (int i = tid; i < p.nf * width; i += kDirectThreads)
       if (s_hist[i] != 0) atomicAdd(sum + i, s_hist[i]);
-    // Every word of the slot is added to and read by device-wide atomic operations, so it suffices that a wave's have
-    // arrived before the workgroup is counted. A __threadfence() also writes the whole L2 back, once per wave: the
-    // levels of 512 and 1024 nodes of 1,000,000 x 50, a third of the rows in large nodes, took 350 and 190 us with
-    // two of them here, 130 and 125 without.
+    // What orders these adds before the last arriver's loads is the target, not the memory model of the language, in which all of them are
+    // relaxed: (1) vmcnt counts an atomic without result until it has been performed at the scope it was asked with, so behind the wait
+    // and the barrier all waves' adds are where the whole device sees them before the workgroup is counted; (2) a load at
+    // device scope is not answered from a cache of its own XCD that could be stale. The slot is cleared by plain stores: nothing
+    // touches it again within the launch, and its end writes them back.
+    // The model's own means, us of the launches of levels 9 to 11 of 1,000,000 x 50 with 512 samples, noise, and of 2,000,000 x 80,
+    // depth 11: as here 341 and 184; one thread's release (it writes the whole L2 back) and the last arriver's acquire 516 and
+    // 313; the acquire alone, which orders nothing without the release, 356 and 187.
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "written for what gfx950 guarantees of waited atomics and of loads at device scope"
+#endif
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     // (the answer goes through the histograms' LDS: a word more and only four workgroups of 512 bins share a CU)
