@@ -364,6 +364,7 @@ struct LevelPlan {
   int bw, n_bb;     // built nodes per workgroup, blocks of them
   int chunks;       // row ranges
   int chunk_rows;   // multiple of 4
+  bool pairs;       // two workgroups share a CU
   bool last;
 };
 
@@ -376,8 +377,11 @@ constexpr int kMaxFw = 4;
 // workgroup reads 64 KB of them with 32 ranges, which takes it 6000 of 14,000 cycles however many loads are under way. One
 // workgroup for every CU then, not two, and two features each instead of four (with several outputs the ranges are few anyway): fewer
 // ranges. Fits with two workgroups and with one, us: 20,000 x 100, depth 6, 5 rounds 1040 and 945; 9000 x 200, depth 5 945 and 825; 250,000 x 43,
-// depth 8 1965 and 1890; 300,000 x 16 with 128 samples 1060 and 1005; 60,000 x 20 with 4 outputs 1235 and 1110; above, 800,000 x 45
-// with 64 samples, depth 5 985 and 1118, 112,000 x 245, depth 3 1013 and 1070 (not taken).
+// depth 8 1965 and 1890; 300,000 x 16 with 128 samples 1060 and 1005; 60,000 x 20 with 4 outputs 1235 and 1110. Trees of depth 6 with 256
+// samples just below the line: 595,000 x 20 227 and 205, 119,000 x 100 228 and 218, 29,750 x 400 283 and 275; with 64, whose images are a
+// quarter, 209 and 190, 197 and 197, 47,600 x 250 208 and 211. Above it, not taken: 240,000 x 100 270 and 273, 400,000 x 45 with 64 samples
+// 219 and 231, 60,000 x 300 285 and 304, 100,000 x 40 with 4 outputs and 128 samples 227 and 234; few columns would still gain (1,000,000 x
+// 20, depth 8 365 and 344).
 constexpr int64_t kImageValues = 12000000;
 
 // Which of a pair of siblings is accumulated (build_tree.h:92-104).
@@ -861,9 +865,12 @@ LevelPlan plan_level(int64_t N, int F, int K, int S, int depth, int max_depth)
   p.n_bb = (p.built + p.bw - 1) / p.bw;
   const int64_t inner = static_cast<int64_t>(p.n_fb) * p.n_bb * K;
   const int64_t image = static_cast<int64_t>(p.built) * K * F * S * 8;
-  // two workgroups share a CU where their histograms do
-  const bool pairs    = !by_images && static_cast<size_t>(p.fw) * p.bw * S * 8 <= 72 * 1024;
-  int64_t chunks      = std::max<int64_t>(1, (pairs ? 512 : 256) / inner);
+  // Two workgroups share a CU where their histograms do. By images too where only that leaves the eight ranges that the
+  // XCDs take one each (several outputs: 50,000 x 20 with 8, depth 6, 278 us a tree with six ranges, 258 with eight; 20,000 x 10
+  // with 16 361 and 318): with fewer, whichever it is, the images count more (30,000 x 25 with 16 outputs 335 with two, 378 with four).
+  const bool too_few  = K > 1 && 256 / inner < 8 && 512 / inner >= 8;
+  p.pairs             = (!by_images || too_few) && static_cast<size_t>(p.fw) * p.bw * S * 8 <= 72 * 1024;
+  int64_t chunks      = std::max<int64_t>(1, (p.pairs ? 512 : 256) / inner);
   // (three quarters of a workgroup's threads have rows: with 1024 rows a range, most of them had none and the scan
   // added up twice the images: 100,000 x 32, 10 rounds, 2.06 -> 1.87 ms; 60,000 x 20 with 4 outputs -9 %)
   chunks              = std::min(chunks, std::max<int64_t>({1, N / 3072, std::min<int64_t>(16, N / 1024)}));
