@@ -942,12 +942,14 @@ bool mid_beats_small(int64_t N, int F, int K, int max_depth, int S)
 
 // Whether the workgroups of level p's histograms find the nodes of their rows for themselves, which saves the launch that does.
 // All workgroups of a range of rows do so for the same rows, a byte gathered per row and workgroup: up to 2.5 million
-// such visits it pays. Fits with the launch and without, us: 100,000 x 32, depth 6, 10 rounds 1885 and 1749; 300,000 x 16 with 128
-// samples, depth 8, 4 rounds 1133 and 1066; 15,000 x 8 f64, depth 10, 5 rounds 1505 and 1342; 50,000 x 60 with 512 samples, depth 7,
-// 4 rounds 1209 and 1137; with levels of 8 million visits 1,000,000 x 30, depth 8, 3 rounds 1395 and 1441 (not taken).
+// such visits it pays. Trees with the launch and without, us: 78,125 x 64, depth 6 (2.5 million) 167 and 155; 100,000 x 32, depth 6 162
+// and 151; 60,000 x 20 with 4 outputs, depth 6 197 and 184; 400,000 x 12, depth 6 169 and 156. By one workgroup of two features to a CU
+// it still gains 3 % at 4 million and nothing at 6; with four features 800,000 x 16, depth 8 (3.2 million) takes 287 and 291, 1,000,000 x
+// 30 with 8 million 3 % more. Where two workgroups share a CU, half as many: with 8 outputs, depth 6 and 8, 20,000 x 20 (0.8 million)
+// 251 and 245, 343 and 334; 35,000 x 20 (1.4 million) 256 and 258, 350 and 354; 62,000 x 20 266 and 270, 365 and 371.
 static bool nodes_with_histograms(const MidArgs& a, const LevelPlan& p)
 {
-  return p.depth > 0 && static_cast<int64_t>(p.n_fb) * p.n_bb * a.K * a.N <= kNodesMost;
+  return p.depth > 0 && static_cast<int64_t>(p.n_fb) * p.n_bb * a.K * a.N <= (p.pairs ? kNodesMost / 2 : kNodesMost);
 }
 
 template <typename BinT, Nodes kNodes>

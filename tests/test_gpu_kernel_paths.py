@@ -237,11 +237,12 @@ def test_medium_sizes(n, f, k, depth, s, dtype, options):
 
 
 @pytest.mark.parametrize("n,f,k,depth,s", [(9001, 43, 1, 9, 256), (8500, 260, 1, 5, 64), (156250, 64, 1, 4, 64), (156251, 64, 1, 4, 64), (200003, 61, 1, 4, 64),
-                                           (20002, 10, 2, 8, 128), (30011, 17, 3, 6, 256)])
+                                           (20002, 10, 2, 8, 128), (30011, 17, 3, 6, 256), (78125, 64, 1, 4, 64), (78126, 64, 1, 4, 64),
+                                           (31250, 20, 8, 4, 64), (31251, 20, 8, 4, 64)])
 def test_medium_sizes_whose_rows_stop_at_every_level(n, f, k, depth, s):
     """Histogram workgroups that find their rows' nodes, by themselves or after the launch that decides many nodes, either side
-    of the number of rows where they do, in turn with levels that do not: rows end at every level, at most nodes of the last
-    ones no row is left."""
+    of the number of rows where they do (one workgroup to a CU, and two), in turn with levels that do not: rows end at every level,
+    at most nodes of the last ones no row is left."""
     import gpu_util as gu
     import oracle_lib as orc
     from lbtree import ops
