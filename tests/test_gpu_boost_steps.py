@@ -161,11 +161,11 @@ def test_predict_from_an_initial_prediction(rows, n_trees, k):
 @pytest.mark.gpu
 @pytest.mark.parametrize("task", ["regression", "classification"])
 def test_fit_with_the_gradient_passes_sums(task):
-    """From a million rows on the gradient pass leaves the quantiser's sums: the same model as tree by tree without them."""
+    """From four million rows on the gradient pass leaves the quantiser's sums: the same model as tree by tree without them."""
     import lbtree as lb
 
     gen = torch.Generator(device="cuda").manual_seed(4)
-    n = 1000003
+    n = 4000003
     X = torch.rand((n, 4), generator=gen, device="cuda")
     y = X[:, 0].to(torch.float64) + 0.1 * torch.randn(n, generator=gen, device="cuda", dtype=torch.float64)
     kind = lb.LBRegressor if task == "regression" else lb.LBClassifier
@@ -183,7 +183,7 @@ def test_fit_with_the_gradient_passes_sums(task):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows", [5000, 1000000])
+@pytest.mark.parametrize("rows", [5000, 4000000])
 def test_fits_and_updates_call_a_replaced_gradient_step(monkeypatch, rows):
     """Replaced on the class that defines it, not on a subclass: the fits that form the gradients themselves must not pass it by."""
     import lbtree as lb
