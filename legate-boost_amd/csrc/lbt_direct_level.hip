@@ -173,7 +173,9 @@ __device__ __forceinline__ Found scan_feature(const DirectLevel& a, const I64Pai
 // formed exactly, of its largest estimate, and where a lane holds a second one that near (equal columns) the feature
 // is scanned as above. A bin without rows has the sums of the last one with rows before it: only those are
 // estimated, and which of the bins up to the next one with rows the tie rule takes is worked out for the best.
-// A lane takes four bins in a row, so that a running sum over the lanes serves 256 bins.
+// A lane takes four bins in a row, so that a running sum over the lanes serves 256 bins; one where they are at most 64, of which
+// four a lane would leave three lanes of four idle (the four levels of 60,000 x 200 with 64 samples, depth 11: 275 us with four, and
+// a tree 949; 909 with one).
 // The 12 launches of levels 9 to 11 of four trees of depth 12, 1,000,000 x 50 with 512 samples: 1361 us with estimates in
 // 64 bits of one bin a lane, now 1208; what bounds them then is the chain of loads of a workgroup's rows (75 of the 82 us of
 // level 9 without any scan).
@@ -187,13 +189,13 @@ __device__ __forceinline__ bool estimates_hold(const DirectLevel& a, double inv_
          reg / inv_h >= 1e-30 && reg / inv_h <= 1e12;
 }
 
-// kSmall: all sums of grads fit 32 bits with their sign
-template <bool kSmall>
+// kSmall: all sums of grads fit 32 bits with their sign. kBins: bins in a row of a lane
+template <bool kSmall, int kBins>
 __device__ __forceinline__ Found scan_feature_estimated(const DirectLevel& a, const I64Pair& ns, int fb, int n_bins,
                                                         double inv_g, double inv_h, double reg, int64_t up,
                                                         int64_t down, const unsigned long long* s_bins)
 {
-  constexpr int kBins = 4;
+  static_assert(kBins == 1 || kBins == 4);
   const int lane        = threadIdx.x & 63;
   const float extra     = static_cast<float>(reg / inv_h);
   const int small_g     = static_cast<int>(ns.grad);
@@ -208,11 +210,14 @@ __device__ __forceinline__ Found scan_feature_estimated(const DirectLevel& a, co
   for (int base = 0; base < n_bins; base += 64 * kBins) {
     const int first = base + lane * kBins;
     uint32_t g[kBins] = {}, h[kBins] = {};
-    if (first < n_bins) {
+    if (kBins == 1 && first < n_bins) {
+      const unsigned long long w = s_bins[first];
+      h[0] = static_cast<uint32_t>(w), g[0] = static_cast<uint32_t>(w >> 32);
+    } else if (kBins == 4 && first < n_bins) {
       // (a feature's bins take a multiple of four places, zeros behind the last one)
       const uint4 w0 = *reinterpret_cast<const uint4*>(s_bins + first), w1 = *reinterpret_cast<const uint4*>(s_bins + first + 2);
-      h[0] = w0.x, g[0] = w0.y, h[1] = w0.z, g[1] = w0.w;
-      h[2] = w1.x, g[2] = w1.y, h[3] = w1.z, g[3] = w1.w;
+      h[0] = w0.x, g[0] = w0.y, h[1 % kBins] = w0.z, g[1 % kBins] = w0.w;
+      h[2 % kBins] = w1.x, g[2 % kBins] = w1.y, h[3 % kBins] = w1.z, g[3 % kBins] = w1.w;
     }
     // The lower halves' sums stay below 2^32, so nothing is carried and the halves are summed on their own.
     uint32_t sum_g = 0, sum_h = 0;
@@ -295,9 +300,14 @@ __device__ __forceinline__ void scan_features(const DirectLevel& a, int j, const
     }
     const int fb = a.row_pointers[f], n_bins = a.row_pointers[f + 1] - fb;
     const unsigned long long* bins = s_hist + v * width;
+    auto estimate    = [&](auto small_c) {
+      constexpr bool kSmall = decltype(small_c)::value;
+      return n_bins <= 64 ? scan_feature_estimated<kSmall, 1>(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, bins)
+                          : scan_feature_estimated<kSmall, 4>(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, bins);
+    };
     const Found best = !estimated ? scan_feature(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, bins)
-                       : small    ? scan_feature_estimated<true>(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, bins)
-                                  : scan_feature_estimated<false>(a, ns, fb, n_bins, inv_g, inv_h, reg, up, down, bins);
+                       : small    ? estimate(std::true_type{})
+                                  : estimate(std::false_type{});
     if (lane == 0) {
       a.partial[at] = Cand{best.gain, best.bin};
       a.left[at]    = unpack_sums(best.left, up, down);
