@@ -427,11 +427,13 @@ __host__ __device__ constexpr size_t small_decide_use(int64_t n_nodes) { return 
 // a level (1000 x 10, depth 8: 4.5 of 12.4 us and the gap in front of it). Fits with such launches and without, us: 1000 x 10 f64,
 // depth 8, 12 rounds 1580 and 1290; 2000 x 16, depth 8, 5 rounds 815 and 720; 4000 x 8, depth 6 860 and 740; 1000 x 40, depth 8 740
 // and 665; 3000 x 60, depth 7 900 and 850. From 4096 rows on (8000 x 30, 7000 x 12, 5000 x 64) it gained nothing.
-template <int kT, int kE, bool kSingle, int kG, bool kStaged, bool kDecides>
+// kLeft: the next scan may decide, so what lies left of a node's best split goes with it (the scans that decide always have
+// it). 2500 x 150, whose scans never decide: 12.0 us a launch with it, 11.2 without.
+template <int kT, int kE, bool kSingle, int kG, bool kStaged, bool kDecides, bool kLeft = kDecides>
 __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
   small_scan_kernel(SmallTreeState st, LevelArgs a)
 {
-  static_assert(!kDecides || (kSingle && kStaged && kG > 1), "one output, nodes in the LDS");
+  static_assert(!(kDecides || kLeft) || (kSingle && kStaged && kG > 1), "one output, nodes in the LDS");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   int2* s_q                  = reinterpret_cast<int2*>(smem_raw);               // [N]
   uint32_t* s_order          = reinterpret_cast<uint32_t*>(s_q + (a.N + 1) / 2 * 2);  // [small_scan_order(N)]
@@ -823,8 +825,6 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     int first_node = kNone, cur = kNone;
     double first_gain = 0.0, cur_gain = 0.0;
     unsigned first_key = 0, cur_key = 0;
-    // (where the next scan may decide: what lies left of a node's best split goes with it)
-    constexpr bool kLeft = kStaged && kG > 1 && kE <= 4;
     I64Pair first_left{0, 0}, cur_left{0, 0};
     auto put_left = [&](int j, const I64Pair& left) {
       if (kLeft && a.left != nullptr) a.left[static_cast<int64_t>(j) * a.F + f] = left;
@@ -1198,13 +1198,13 @@ __global__ void __launch_bounds__(256) small_count_kernel(SmallTreeState st, Lev
   }
 }
 
-template <int kT, int kE, bool kSingle, int kG, bool kStaged, bool kDecides>
+template <int kT, int kE, bool kSingle, int kG, bool kStaged, bool kDecides, bool kLeft = kDecides>
 int launch_small_scan_as(hipStream_t stream, const SmallTreeState& st, const LevelArgs& a, size_t lds)
 {
   static std::atomic<bool> attr_set[kMaxDevices] = {};
   LBT_REQUIRE(small_scan_places(a.N) == kT * kE, "%d rows do not take a workgroup of %d places", a.N, kT * kE);
-  LBT_TRY((allow_dynamic_lds(small_scan_kernel<kT, kE, kSingle, kG, kStaged, kDecides>, kScanLds + 64, attr_set)));
-  small_scan_kernel<kT, kE, kSingle, kG, kStaged, kDecides><<<a.F, kT, lds, stream>>>(st, a);
+  LBT_TRY((allow_dynamic_lds(small_scan_kernel<kT, kE, kSingle, kG, kStaged, kDecides, kLeft>, kScanLds + 64, attr_set)));
+  small_scan_kernel<kT, kE, kSingle, kG, kStaged, kDecides, kLeft><<<a.F, kT, lds, stream>>>(st, a);
   return LBT_OK;
 }
 size_t small_staged_use(int64_t N, int64_t n_nodes)
@@ -1234,6 +1234,9 @@ int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelA
   if (more > kScanLds || (per_cu(more) < per_cu(lds) && a.F > 256 * per_cu(more)))
     return launch_small_scan_as<kT, kE, true, 1, false, false>(stream, st, a, lds);
   if (crowded) return launch_small_scan_as<kT, kE, true, 1, true, false>(stream, st, a, more);
+  if constexpr (kE <= 4) {
+    if (a.left != nullptr) return launch_small_scan_as<kT, kE, true, kG, true, false, true>(stream, st, a, more);
+  }
   return launch_small_scan_as<kT, kE, true, kG, true, false>(stream, st, a, more);
 }
 
