@@ -566,10 +566,12 @@ def test_levels_without_histograms_in_memory_give_the_oracles_tree(n, f, s, dept
 
 
 @pytest.mark.parametrize("n,f,s,depth,kind", [(9001, 9, 511, 12, "one_sign"), (9001, 6, 254, 11, "near_ties"), (20001, 5, 509, 12, "near_ties"),
-                                              (12001, 17, 61, 11, "equal_columns"), (9001, 8, 512, 12, "l2")])
+                                              (12001, 17, 61, 11, "equal_columns"), (9001, 8, 512, 12, "l2"),
+                                              (9001, 9, 64, 11, "one_sign"), (20001, 6, 64, 11, "near_ties"), (9001, 6, 65, 11, "near_ties")])
 def test_deep_levels_whose_estimates_do_not_decide(n, f, s, depth, kind):
     """Sums of grads that leave 32 bits with their sign, bins whose estimates lie closer together than they are right, equal
-    columns, a penalty far above the hessians; bins that are no multiple of the four a lane takes: the oracle's tree."""
+    columns, a penalty far above the hessians; bins that are no multiple of the four a lane takes, and up to 64 bins, of which it takes
+    one: the oracle's tree."""
     import oracle_lib as orc
     from lbtree import ops
 
