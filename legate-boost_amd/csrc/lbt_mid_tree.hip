@@ -633,6 +633,9 @@ __device__ __forceinline__ int64_t decode_grad(uint32_t v, int64_t up, int64_t d
 // of 250,000 x 43 took 90 us, now 79; the six of 100,000 x 32 50 and 43. All loads in front of the first wait
 // instead, with the terms that do not depend on the bin formed once, was slower: 8.3 to 9.5 us a narrow level where it
 // had been 7.5 to 8.1.
+// kLess: kLeftSmaller beside the candidates' bins, for histogram workgroups that decide (42.2 us a launch on 5000 x 200 with 8 outputs, depth 5, to
+// 41.1 without).
+template <bool kLess>
 __global__ void __launch_bounds__(kScan)
   mid_scan_kernel(MidArgs a, MidTreeState st, LevelPlan p)
 {
@@ -726,7 +729,7 @@ __global__ void __launch_bounds__(kScan)
       const double s_right = leaf_gain_select(static_cast<double>(sr.grad) * inv_g, static_cast<double>(sr.hess) * inv_h, a.l1, reg);
       const double n_own = leaf_gain_select(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, a.l1, reg);
       const double s_own = leaf_gain_select(static_cast<double>(ss.grad) * inv_g, static_cast<double>(ss.hess) * inv_h, a.l1, reg);
-      if (k == 0) {
+      if (kLess && k == 0) {
         left_n = nv.hess < nr.hess;
         left_s = sv.hess < sr.hess;
       }
@@ -750,18 +753,20 @@ __global__ void __launch_bounds__(kScan)
     const bool take_s = !dead_s && gain_s > 0 && (gain_s > best_s || (gain_s == best_s && key > key_s));
     best_n = take_n ? gain_n : best_n;
     key_n  = take_n ? key : key_n;
-    less_n = take_n ? left_n : less_n;
+    if constexpr (kLess) less_n = take_n ? left_n : less_n;
     best_s = take_s ? gain_s : best_s;
     key_s  = take_s ? key : key_s;
-    less_s = take_s ? left_s : less_s;
+    if constexpr (kLess) less_s = take_s ? left_s : less_s;
     if (base + kScan < n_bins) __syncthreads();
   }
   const double own_n = best_n, own_s = best_s;
   const unsigned own_key_n = key_n, own_key_s = key_s;
   wave_best_key(best_n, key_n);
   wave_best_key(best_s, key_s);
-  less_n = __any(less_n && own_key_n == key_n && own_n == best_n);  // (no two lanes have one key)
-  less_s = __any(less_s && own_key_s == key_s && own_s == best_s);
+  if constexpr (kLess) {
+    less_n = __any(less_n && own_key_n == key_n && own_n == best_n);  // (no two lanes have one key)
+    less_s = __any(less_s && own_key_s == key_s && own_s == best_s);
+  }
   if (lane == 0) {
     s_best[0][wave] = best_n;
     s_bkey[0][wave] = key_n;
@@ -980,6 +985,7 @@ static int queue_levels(hipStream_t stream, const MidTreeState& st, const MidArg
     const LevelPlan p = plan_level(a.N, a.F, a.K, a.S, d, a.max_depth);
     const uint16_t* const from = st.row_node[cur];
     uint16_t* const to         = st.row_node[cur ^ 1];
+    const bool later           = !p.last && nodes_with_histograms(a, plan_level(a.N, a.F, a.K, a.S, d + 1, a.max_depth));
     switch (how) {
       case Nodes::kCarried: LBT_TRY((launch_histograms<BinT, Nodes::kCarried>(stream, st, a, p, above, lanes_log, from, nullptr))); break;
       case Nodes::kDecide: LBT_TRY((launch_histograms<BinT, Nodes::kDecide>(stream, st, a, p, above, lanes_log, from, to))); break;
@@ -990,11 +996,14 @@ static int queue_levels(hipStream_t stream, const MidTreeState& st, const MidArg
       mid_count_kernel<<<static_cast<unsigned>((a.N + kScan - 1) / kScan), kScan, 0, stream>>>(a, st, p, st.row_node[cur], level_totals + d);
     {
       ProfScope ps(LBT_PROF_SCAN, stream);
-      mid_scan_kernel<<<static_cast<unsigned>(p.built) * a.F, kScan, 0, stream>>>(a, st, p);
+      const unsigned grid = static_cast<unsigned>(p.built) * a.F;
+      if (later)
+        mid_scan_kernel<true><<<grid, kScan, 0, stream>>>(a, st, p);
+      else
+        mid_scan_kernel<false><<<grid, kScan, 0, stream>>>(a, st, p);
     }
     ProfScope ps(LBT_PROF_POSITIONS, stream);
     const unsigned grid = static_cast<unsigned>((a.N + kRowsApply - 1) / kRowsApply);
-    const bool later    = !p.last && nodes_with_histograms(a, plan_level(a.N, a.F, a.K, a.S, d + 1, a.max_depth));
     // few nodes: every workgroup that asks for the splits finds them for itself (it saves a launch)
     const bool few = p.n_nodes <= 2 * (kWide >> lanes_log);
     if (!few || (later && static_cast<int64_t>(p.n_nodes) * a.F > kCandsMost)) {
