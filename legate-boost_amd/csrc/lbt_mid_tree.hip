@@ -951,10 +951,13 @@ bool mid_beats_small(int64_t N, int F, int K, int max_depth, int S)
 // and 151; 60,000 x 20 with 4 outputs, depth 6 197 and 184; 400,000 x 12, depth 6 169 and 156. By one workgroup of two features to a CU
 // it still gains 3 % at 4 million and nothing at 6; with four features 800,000 x 16, depth 8 (3.2 million) takes 287 and 291, 1,000,000 x
 // 30 with 8 million 3 % more. Where two workgroups share a CU, half as many: with 8 outputs, depth 6 and 8, 20,000 x 20 (0.8 million)
-// 251 and 245, 343 and 334; 35,000 x 20 (1.4 million) 256 and 258, 350 and 354; 62,000 x 20 266 and 270, 365 and 371.
+// 251 and 245, 343 and 334; 35,000 x 20 (1.4 million) 256 and 258, 350 and 354; 62,000 x 20 266 and 270, 365 and 371. And where they
+// are no more than the CUs: those that wait for a CU decide all over again (depth 5: 9000 x 500, 250 workgroups, 181 and 170, 6000 x 500 with
+// 2 outputs, 250, 206 and 194; 6500 x 700, 350, 219 and 224, 6000 x 500 with 3, 375, 244 and 249).
 static bool nodes_with_histograms(const MidArgs& a, const LevelPlan& p)
 {
-  return p.depth > 0 && static_cast<int64_t>(p.n_fb) * p.n_bb * a.K * a.N <= (p.pairs ? kNodesMost / 2 : kNodesMost);
+  const int64_t inner = static_cast<int64_t>(p.n_fb) * p.n_bb * a.K;  // workgroups of a range of rows
+  return p.depth > 0 && inner <= 256 && inner * a.N <= (p.pairs ? kNodesMost / 2 : kNodesMost);
 }
 
 template <typename BinT, Nodes kNodes>

@@ -237,7 +237,7 @@ def test_medium_sizes(n, f, k, depth, s, dtype, options):
 
 
 @pytest.mark.parametrize("n,f,k,depth,s", [(9001, 43, 1, 9, 256), (8500, 260, 1, 5, 64), (156250, 64, 1, 4, 64), (156251, 64, 1, 4, 64), (200003, 61, 1, 4, 64),
-                                           (20002, 10, 2, 8, 128), (30011, 17, 3, 6, 256), (78125, 64, 1, 4, 64), (78126, 64, 1, 4, 64),
+                                           (20002, 10, 2, 8, 128), (30011, 17, 3, 6, 256), (78125, 64, 1, 4, 64), (78126, 64, 1, 4, 64), (9000, 512, 1, 4, 64), (9000, 514, 1, 4, 64),
                                            (31250, 20, 8, 4, 64), (31251, 20, 8, 4, 64)])
 def test_medium_sizes_whose_rows_stop_at_every_level(n, f, k, depth, s):
     """Histogram workgroups that find their rows' nodes, by themselves or after the launch that decides many nodes, either side
