@@ -40,9 +40,11 @@ def test_initial_predictions_may_not_lie_in_the_output(init, out, refused):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,k", [(1, 1), (257, 1), (1, 2), (255, 3), (513, 8), (300, 10), (1000, 16), (70, 7), (40, 19), (3, 300)])
+@pytest.mark.parametrize("n,k", [(1, 1), (257, 1), (1, 2), (255, 3), (513, 8), (300, 10), (1000, 16), (70, 7), (40, 19), (3, 300),
+                                 (255, 9), (131, 12), (77, 13), (130, 24), (65, 25), (9, 33), (33, 48), (17, 49), (5, 64), (7, 65),
+                                 (9, 128), (5, 129), (3, 256), (5, 257), (2, 1000)])
 def test_class_probabilities(n, k):
-    """exp and the sums of up to 300 terms round differently from torch's: (k + 8) 2^-52 of each probability."""
+    """exp and the sums of up to 1000 terms round differently from torch's: (k + 8) 2^-52 of each probability."""
     from lbtree import ops
 
     gen = torch.Generator(device="cuda").manual_seed(n + k)
