@@ -430,9 +430,9 @@ __global__ void __launch_bounds__(kBoostThreads)
   label_counts_kernel(const double* __restrict__ y, int64_t n, unsigned long long* __restrict__ stats)
 {
   __shared__ unsigned s_count[kLabelCopies][kLabelMost];
-  __shared__ unsigned s_bad, s_wide;
+  __shared__ unsigned s_bad, s_wide, s_most;
   for (int i = threadIdx.x; i < kLabelCopies * kLabelMost; i += kBoostThreads) (&s_count[0][0])[i] = 0;
-  if (threadIdx.x == 0) s_bad = s_wide = 0;
+  if (threadIdx.x == 0) s_bad = s_wide = s_most = 0;
   __syncthreads();
   unsigned* const count = s_count[threadIdx.x >> 6];
   const int64_t step    = static_cast<int64_t>(gridDim.x) * kBoostThreads;
@@ -462,10 +462,13 @@ __global__ void __launch_bounds__(kBoostThreads)
     for (int w = 0; w < kLabelCopies; w++) all += s_count[w][c];
     if (all != 0) {
       atomicAdd(stats + 3 + c, all);
-      atomicMax(stats + 1, static_cast<unsigned long long>(c));
+      atomicMax(&s_most, static_cast<unsigned>(c));
     }
   }
+  __syncthreads();
   if (threadIdx.x == 0) {
+    // (once a workgroup: all of them at one address are waited for one after the other)
+    if (s_most != 0) atomicMax(stats + 1, static_cast<unsigned long long>(s_most));
     if (s_bad != 0) atomicAdd(stats, static_cast<unsigned long long>(s_bad));
     if (s_wide != 0) atomicAdd(stats + 2, static_cast<unsigned long long>(s_wide));
   }
@@ -634,7 +637,7 @@ int lbt_label_counts(void* stream, const double* y, int64_t n, int64_t* stats)
   LBT_REQUIRE(n >= 1 && n < (int64_t(1) << 38), "bad shape");
   LBT_REQUIRE(y && stats, "null pointer");
   hipStream_t s    = static_cast<hipStream_t>(stream);
-  const int groups = static_cast<int>(std::min<int64_t>((n + 4 * lbt::kBoostThreads - 1) / (4 * lbt::kBoostThreads), 1024));
+  const int groups = static_cast<int>(std::min<int64_t>((n + 8 * lbt::kBoostThreads - 1) / (8 * lbt::kBoostThreads), 1024));
   lbt::ProfScope ps(LBT_PROF_OTHER, s, static_cast<double>(n) * 8.0);
   lbt::label_counts_kernel<<<groups, lbt::kBoostThreads, 0, s>>>(y, n, reinterpret_cast<unsigned long long*>(stats));
   LBT_HIP(hipGetLastError());

@@ -72,7 +72,8 @@ class LogLossObjective:
         return e_x / e_x.sum(dim=1)[:, None]
 
     def initialise_prediction(self, y, w, boost_from_average):
-        if y.is_cuda and y.numel() > 0 and not y.requires_grad:
+        counted = y.is_cuda and y.numel() > 0 and not y.requires_grad
+        if counted:
             stats = ops.label_counts(y)
             bad, most, wide = stats[:3].tolist()
             if bad:
@@ -82,7 +83,7 @@ class LogLossObjective:
                 if not boost_from_average:
                     return torch.zeros(n_targets, dtype=torch.float64, device=y.device)
                 return ops.label_priors(stats, y.numel(), n_targets)
-        if not bool(((y == torch.floor(y)) & (y >= 0)).all()):
+        if not counted and not bool(((y == torch.floor(y)) & (y >= 0)).all()):
             raise ValueError("Expected labels to be non-zero whole numbers")
         num_class = int(y.max().item() + 1)
         n_targets = num_class if num_class > 2 else 1
