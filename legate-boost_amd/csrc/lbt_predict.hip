@@ -179,10 +179,13 @@ __global__ void __launch_bounds__(256)
     d.n_nodes              = n;
     desc[b.first_tree + t] = d;
   }
-  if (i >= n) return;
-  // leaf values move along, indexed like the nodes
-  for (int k = 0; k < K; k++) leaves[(first + i) * K + k] = b.leaf[t][static_cast<int64_t>(i) * K + k];
-  nodes[first + i] = pack_node<T>(i, b.feature[t][i], b.split[t][i], F, n);
+  if (i < n) nodes[first + i] = pack_node<T>(i, b.feature[t][i], b.split[t][i], F, n);
+  // leaf values move along, indexed like the nodes: the workgroup's in one run
+  const int64_t from        = static_cast<int64_t>(blockIdx.x) * 256 * K;
+  const int here            = min(256, n - static_cast<int>(blockIdx.x) * 256) * K;
+  const double* const leaf  = b.leaf[t] + from;
+  double* const packed      = leaves + first * K + from;
+  for (int e = threadIdx.x; e < here; e += 256) packed[e] = leaf[e];
 }
 
 __global__ void write_batches_kernel(BatchTable t, int first, int n, BatchInfo* out)
