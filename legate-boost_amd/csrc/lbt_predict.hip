@@ -571,11 +571,22 @@ __global__ void __launch_bounds__(kTileThreads)
   if (tid < rows_here * K) out[row0 * K + tid] = init != nullptr ? init[tid % K] + acc : acc;
 }
 
-// init + the sums, where the kernel that formed them did not add it
+// init + the sums, where the kernel that formed them did not add it. kWide: out is 16-byte aligned, two entries at a time
+// (300,000 x 8: 10.5 us with one and remainders of 64 bits, which take several times those of 32).
+template <bool kWide>
 __global__ void __launch_bounds__(kThreads) add_init_kernel(const double* __restrict__ init, int64_t n, int K, double* out)
 {
-  const int64_t i = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x;
-  if (i < n) out[i] = init[K == 1 ? 0 : i % K] + out[i];
+  constexpr int kAtOnce = kWide ? 2 : 1;
+  const int64_t i       = kAtOnce * (blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x);
+  if (i >= n) return;
+  const int k = K == 1 ? 0 : (n >> 32) == 0 ? static_cast<int>(static_cast<uint32_t>(i) % static_cast<uint32_t>(K)) : static_cast<int>(i % K);
+  if (kWide && i + 1 < n) {
+    double2* const o = reinterpret_cast<double2*>(out + i);
+    const double2 v  = *o;
+    *o               = make_double2(init[k] + v.x, init[k + 1 == K ? 0 : k + 1] + v.y);
+  } else {
+    out[i] = init[k] + out[i];
+  }
 }
 
 size_t padded_nodes(int n_trees, int64_t total_nodes)
@@ -1140,7 +1151,13 @@ int lbt_predict_from(void* stream, const void* X, int32_t x_dtype, int64_t n_row
   }
   if (init != nullptr) {
     lbt::ProfScope ps(LBT_PROF_OTHER, s, static_cast<double>(n) * 16.0);
-    lbt::add_init_kernel<<<static_cast<unsigned>((n + lbt::kThreads - 1) / lbt::kThreads), lbt::kThreads, 0, s>>>(init, n, n_outputs, out);
+    const bool wide     = reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    const int64_t per   = (wide ? 2 : 1) * lbt::kThreads;
+    const unsigned grid = static_cast<unsigned>((n + per - 1) / per);
+    if (wide)
+      lbt::add_init_kernel<true><<<grid, lbt::kThreads, 0, s>>>(init, n, n_outputs, out);
+    else
+      lbt::add_init_kernel<false><<<grid, lbt::kThreads, 0, s>>>(init, n, n_outputs, out);
     LBT_HIP(hipGetLastError());
   }
   return LBT_OK;

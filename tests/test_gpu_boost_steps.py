@@ -161,6 +161,26 @@ def test_predict_from_an_initial_prediction(rows, n_trees, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(1, 1), (5000, 1), (4099, 3), (4096, 2)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_predict_from_into_an_output_that_begins_off_16_bytes(n, k, off):
+    """The initial prediction is added two entries at a time where the output lies on 16 bytes: odd counts, and outputs that do not."""
+    from lbtree import _lib, ops
+
+    rs = np.random.RandomState(n + k)
+    X = ops.as_device(rs.rand(n, 5))
+    tree = tuple(ops.as_device(a) for a in (rs.randn(7, k), np.array([0, 1, 2, -1, -1, -1, -1], np.int32), rs.rand(7)))
+    init = ops.as_device(rs.randn(k))
+    room = torch.full((n * k + 3,), 7.0, dtype=torch.float64, device="cuda")
+    ptrs = [(C.c_void_p * 1)(a.data_ptr()) for a in tree]
+    _lib.check(_lib.lib.lbt_predict_from(ops._stream(), X.data_ptr(), _lib.LBT_F64, n, 5, 1, *ptrs, (C.c_int32 * 1)(7), k,
+                                         init.data_ptr(), room.data_ptr() + 8 * off, None, 0))
+    got = room[off:off + n * k].reshape(n, k)
+    assert torch.equal(got, init + ops.predict(X, [tree], k, tiled=False))
+    assert bool((room[off + n * k:] == 7.0).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("task", ["regression", "classification"])
 def test_fit_with_the_gradient_passes_sums(task):
     """From four million rows on the gradient pass leaves the quantiser's sums: the same model as tree by tree without them."""
