@@ -313,9 +313,12 @@ __device__ __forceinline__ int row_place(int row) { return (row & ~63) + 2 * (ro
 // of 4000 evenly spread thresholds takes 4 or 5 probes instead of 12 (20,000,000 x 64: 6.1 ms without cells, 2.8 with).
 // The features of a line come without their next row on its way; two workgroups to a CU wait for one another's rows instead: floats four
 // features at a time (59 registers, eight waves a SIMD; 500,003 x 200 with 50 trees and 8 outputs 468 -> 448 us a call against eight
-// at a time, 74 registers). Doubles take 63 with a spill that way and gained nothing: eight at a time, 87.
+// at a time, 74 registers). Doubles take 63 with a spill that way and gained nothing: eight at a time, 87. So do floats whose rows are no
+// whole 16-byte words: a line's values are then 32 loads a row, and those of two workgroups leave no line in the L1 until its
+// last one is read (1,000,000 rows: 301 features with 60 trees 1680 us with two workgroups, 1209 with one; 499 with 20 2099 and 1530,
+// 33 with 40 trees of 8 outputs 435 and 385).
 template <typename T, int kGroup, int kSub>
-__global__ void __launch_bounds__(kWalkThreads, kSub > 1 && sizeof(T) == 4 ? 8 : 4)
+__global__ void __launch_bounds__(kWalkThreads, kSub > 1 && sizeof(T) == 4 && kGroup == 4 ? 8 : 4)
   rank_rows_kernel(const T* __restrict__ X, RankRows a, RankState st, const T* __restrict__ sorted,
                    uint16_t* __restrict__ ranks)
 {
@@ -930,8 +933,9 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
   rank_thresholds_kernel<T><<<dim3(F, p.thresholds > kSortMost<T> ? kRankBlocks : 1), kSortThreads,
                               sort_size * (sizeof(T) + sizeof(uint32_t)), stream>>>(st, static_cast<int>(sort_size), lay.grouped, lay.sorted);
 
-  static std::atomic<bool> rank_attr[5][kMaxDevices] = {};
+  static std::atomic<bool> rank_attr[6][kMaxDevices] = {};
   static std::atomic<bool> walk_attr[4][4][kMaxDevices] = {};
+  auto whole_words = [&](const T* x) { return (static_cast<size_t>(F) * sizeof(T)) % 16 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0; };
   auto rank_chunk = [&](auto group_c, auto sub_c, std::atomic<bool> (&flags)[kMaxDevices], const T* x, int64_t rows) -> int {
     constexpr int kG = decltype(group_c)::value, kS = decltype(sub_c)::value;
     LBT_TRY((allow_dynamic_lds(rank_rows_kernel<T, kG, kS>, kLds - 1024, flags)));
@@ -946,8 +950,7 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
     const int per_cu     = kLds / 2 >= static_cast<size_t>(p.rank_lds) + 1024 ? 2 : 1;
     const int64_t splits = 8 * std::max<int64_t>(1, std::min<int64_t>(32 * per_cu / a.n_groups, ceil_div(rows, 8 * kWalkThreads)));
     a.rows_per_split     = (rows + splits * kWalkThreads - 1) / (splits * kWalkThreads) * kWalkThreads;
-    a.wide = (static_cast<size_t>(F) * sizeof(T)) % 16 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-             kG * sizeof(T) >= 16;
+    a.wide = whole_words(x) && kG * sizeof(T) >= 16;
     rank_rows_kernel<T, kG, kS><<<static_cast<unsigned>(splits * a.n_groups), kWalkThreads, p.rank_lds, stream>>>(x, a, st, lay.sorted, lay.ranks);
     return LBT_OK;
   };
@@ -980,11 +983,12 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
       case 2: LBT_TRY(rank_chunk(integral_constant<int, 2>{}, one, rank_attr[1], x, rows)); break;
       case 4: LBT_TRY(rank_chunk(integral_constant<int, 4>{}, one, rank_attr[2], x, rows)); break;
       case 8: LBT_TRY(rank_chunk(integral_constant<int, 8>{}, one, rank_attr[3], x, rows)); break;
-      default: {
-        constexpr int kLineGroup = sizeof(T) == 4 ? 4 : 8;
-        LBT_TRY(rank_chunk(integral_constant<int, kLineGroup>{}, integral_constant<int, 128 / (kLineGroup * sizeof(T))>{}, rank_attr[4], x, rows));
+      default:
+        if (sizeof(T) == 4 && whole_words(x))
+          LBT_TRY(rank_chunk(integral_constant<int, 4>{}, integral_constant<int, 32 / sizeof(T)>{}, rank_attr[4], x, rows));
+        else
+          LBT_TRY(rank_chunk(integral_constant<int, 8>{}, integral_constant<int, 16 / sizeof(T)>{}, rank_attr[5], x, rows));
         break;
-      }
     }
     auto with = [&](auto adds_c, auto items_c, int at) -> int {
       switch (p.shape.j) {

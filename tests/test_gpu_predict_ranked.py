@@ -118,10 +118,11 @@ def test_last_features_of_a_cache_line(f, dtype):
     assert torch.equal(ops.predict(X, trees, 1), ops.predict(X, trees, 1, tiled=False))
 
 
-def test_a_start_off_a_16_byte_boundary():
+@pytest.mark.parametrize("n,f,n_trees,depth", [(1_000_000, 8, 130, 6), (70_000, 516, 40, 5)])
+def test_a_start_off_a_16_byte_boundary(n, f, n_trees, depth):
     rs = np.random.RandomState(5)
-    trees = _ensemble(rs, 130, 6, 8, 1, np.float32, 0)
-    base = _rows(rs, 1_000_001, 8, np.float32, 0).reshape(-1)
-    X = base[1:1 + 1_000_000 * 8].view(1_000_000, 8)
+    trees = _ensemble(rs, n_trees, depth, f, 1, np.float32, 0)
+    base = _rows(rs, n + 1, f, np.float32, 0).reshape(-1)
+    X = base[1:1 + n * f].view(n, f)
     assert X.data_ptr() % 16 != 0 and _takes_ranks(X, trees, 1)
     assert torch.equal(ops.predict(X, trees, 1), ops.predict(X, trees, 1, tiled=False))
