@@ -929,11 +929,13 @@ bool mid_tree_fits(int64_t N, int F, int K, int max_depth, int S)
 // Of two builders that both could, the one for few rows or this one. A level costs the first less to begin with and
 // more per entry (one workgroup per feature walks them in order, output by output); here it is the histograms that
 // count, and a scan workgroup per node and feature. The two sums are times of a tree in us, fitted to 190 shapes (300
-// to 8192 rows, 3 to 500 features, 1 to 16 outputs, depth 2 to 10, 64 to 1024 samples, float and double) to within a
-// tenth or so, hence the 15 % in favour of the first: so none of the shapes where this builder is taken is more than 3 %
-// slower for it. Both, few rows against medium: 10 features, depth 8 at 1000, 4096 and 8192 rows 128, 180, 254 and 179,
-// 198, 205; 8192 x 32, depth 6 205 and 155; 8192 x 100, depth 8 262 and 290; 20 features, 4 outputs, depth 6 at
-// 1000, 2048 and 8192 rows 160, 201, 601 and 166, 180, 197.
+// to 8192 rows, 3 to 500 features, 1 to 16 outputs, depth 2 to 10, 64 to 1024 samples, float and double) when both
+// builders took a launch more per level, with 15 % in favour of the first. Of 188 shapes timed again since (1000 to 8192 rows, 8 to 250 features, 1 and
+// 4 outputs, depth 4 to 10) none where this builder is taken is slower for it; 24 where the first one is taken would be 3 to 38 % faster
+// here, most of them one output of 4097 to 6500 rows and up to 60 features: the line lies too high there. Both now, few rows against
+// medium: 8 features, depth 8 at 1000, 4096 and 8192 rows 83, 129, 215 and 138, 152, 156; 5000 x 8, depth 6 147 and 113; 8192 x 20,
+// depth 6 172 and 120; 8192 x 100, depth 8 221 and 239; 20 features, 4 outputs, depth 6 at 1000, 2000 and 8192 rows 148, 188, 582 and
+// 142, 151, 168.
 bool mid_beats_small(int64_t N, int F, int K, int max_depth, int S)
 {
   const double d = max_depth, n = static_cast<double>(N), f = F, k = K;

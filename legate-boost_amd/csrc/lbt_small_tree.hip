@@ -1258,7 +1258,7 @@ bool next_scan_decides(const SmallTreeState& st, int64_t N, int F, int K, int de
 // What can be held: a feature's order the registers of one workgroup (8192 rows); the quantiser's workgroup takes
 // kQuantChunks chunks; the rows and a slot for each node of a level share the LDS (of 13 levels up to 7732 rows). Up
 // to there it is the faster builder of these sizes unless mid_beats_small says otherwise; against the general one:
-// 8192 x 20, depth 12 364 us and 954, 8192 x 500, depth 10 544 and 1028, 1000 x 10, depth 8 128 and 407.
+// 8192 x 20, depth 12 314 us and 806, 8192 x 500, depth 10 483 and 939, 1000 x 10, depth 8 86 and 367.
 bool small_tree_fits(int64_t N, int F, int K, int max_depth, int S)
 {
   return N <= kSmallMaxRows && K <= kSmallMaxOutputs && N * K <= kQuantChunks * 4096 && max_depth >= 1 &&
