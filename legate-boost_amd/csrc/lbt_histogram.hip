@@ -1320,7 +1320,7 @@ __device__ __forceinline__ void turn_bytes(uint32_t w0, uint32_t w1, uint32_t w2
 // 16 bins of a row in its own rotated order.
 // kPer (striped; 0: not): every group of the launch has four lanes per row (and a lane four rows per tile), so the lanes of a
 // row are an aligned group of four. They share the row's bins evenly, kPer each, instead of 16, 16, 16 and what is left, and an
-// atomic is one vector instruction beside itself (see Stripes): 2,000,000 x 200, 8 outputs: 4.6 vector instructions an atomic
+// atomic is one vector instruction beside itself (see Stripes): 2,000,000 x 200, 8 outputs: 4.4 vector instructions an atomic
 // at 13 bins a lane, 6.7 when its address took three. What all four of them need one of them loads and hands round with a
 // cross-lane move: a vector memory instruction costs by the cache lines it touches and holds registers until it
 // returns. Below the root lane u of the four loads the position of the tile's row u and, with several outputs, its
