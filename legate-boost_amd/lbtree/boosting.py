@@ -24,7 +24,11 @@ def _check_random_state(seed):
 def _as_defined(obj, owner, *names):
     """Whether these methods of obj are the ones this package defines for `owner`: overridden by no subclass and replaced neither
     on the object nor on a class. What bypasses a method asks this first."""
-    return all(getattr(type(obj), n) is _DEFINED[owner][n] and n not in vars(obj) for n in names)
+    cls, own, defined = type(obj), vars(obj), _DEFINED[owner]
+    for n in names:
+        if n in own or getattr(cls, n) is not defined[n]:
+            return False
+    return True
 
 
 def _float64_on_device(a):
