@@ -1515,13 +1515,11 @@ struct Layout {
   size_t upload_bytes;
   int32_t* groups;
   int32_t* sgroups;
-  int64_t* bin_base;
-  int32_t* bin_stride;
-  int32_t* bin_tail;
+  int2* bin_lanes;
   RecInfo* rec;
   void* binned;
   size_t binned_bytes;
-  uint32_t* tables;
+  uint2* tables;
   void* map_x;
   float* map_t;
   int32_t* straight;
@@ -1597,16 +1595,14 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
   const size_t upload_at = ar.used;
   L.groups       = ar.take<int32_t>(F + 1);
   L.sgroups      = ar.take<int32_t>(F + 1);
-  L.bin_base     = ar.take<int64_t>(F);
-  L.bin_stride   = ar.take<int32_t>(F);
-  L.bin_tail     = ar.take<int32_t>(F);
+  L.bin_lanes    = ar.take<int2>(4 * static_cast<size_t>(F) + 16);
   L.rec          = ar.take<RecInfo>(F);
   L.upload_block = L.groups;
   L.upload_bytes = ar.used - upload_at;
   // bin cache: one or two bytes per (row, feature); used when the tree has at least two levels
-  L.binned_bytes = max_depth >= 2 ? static_cast<size_t>(N) * bin_row_bytes_max(F, S) : 0;
+  L.binned_bytes = max_depth >= 2 ? bin_cache_bytes(N, F, S) : 0;
   L.binned       = max_depth >= 2 ? static_cast<void*>(ar.take<char>(L.binned_bytes + 16)) : nullptr;
-  L.tables       = ar.take<uint32_t>(2 * static_cast<size_t>(F) * kMaxCells / 16);
+  L.tables       = ar.take<uint2>(2 * static_cast<size_t>(F) * kMaxCells / 32);
   L.map_x        = ar.take<double>(4 * static_cast<size_t>(F));
   L.map_t        = ar.take<float>(2 * static_cast<size_t>(F));
   L.straight     = ar.take<int32_t>(F);
@@ -1694,7 +1690,7 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     st.proposals  = ar.take<double>(fs);
     st.cells      = 128;  // eight cells per proposal
     while (st.cells < 8 * S && st.cells < kMaxCells) st.cells *= 2;
-    st.tables     = ar.take<uint32_t>(static_cast<size_t>(F) * st.cells / 16);
+    st.tables     = ar.take<uint2>(static_cast<size_t>(F) * st.cells / 32);
     st.map_x      = ar.take<char>(2 * static_cast<size_t>(F) * elem);
     st.map_t      = ar.take<float>(2 * static_cast<size_t>(F));
     st.counts     = ar.take<int32_t>(F);
@@ -1950,9 +1946,7 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
   hs.tiles      = L.tiles;
   hs.binned     = L.binned;
   hs.binned_capacity = L.binned_bytes;
-  hs.bin_base   = L.bin_base;
-  hs.bin_stride = L.bin_stride;
-  hs.bin_tail   = L.bin_tail;
+  hs.bin_lanes  = L.bin_lanes;
   hs.rec        = L.rec;
   hs.upload_block = L.upload_block;
   hs.upload_bytes = L.upload_bytes;
@@ -2025,7 +2019,7 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
       N < (int64_t(1) << 30) && (range_of_large = direct_range(hs, N, L.hist_bytes)) > 0) {
     direct_from = 2;  // at the root it is not known yet
     while (direct_from < max_depth && static_cast<double>(bytes_per_node) * static_cast<double>(int64_t(1) << direct_from) <
-                                        static_cast<double>(N) * static_cast<double>(hs.max_rec_stride))
+                                        static_cast<double>(N) * static_cast<double>(hs.row_bytes))
       direct_from++;
   }
   int cur_pos = 0, cur_seg = 0;
@@ -2703,15 +2697,13 @@ struct HistStageLayout {
   // independent of the level, so that the bin cache of one call is where the next call looks for it
   int32_t* groups;
   int32_t* sgroups;
-  int64_t* bin_base;
-  int32_t* bin_stride;
-  int32_t* bin_tail;
+  int2* bin_lanes;
   RecInfo* rec;
   void* upload_block;
   size_t upload_bytes;
   void* binned;
   size_t binned_bytes;
-  uint32_t* tables;
+  uint2* tables;
   void* map_x;
   float* map_t;
   int32_t* straight;
@@ -2738,15 +2730,13 @@ void make_hist_stage_layout(Arena& ar, HistStageLayout& L, int64_t N, int F, int
   const size_t upload_at    = ar.used;
   L.groups       = ar.take<int32_t>(F + 1);
   L.sgroups      = ar.take<int32_t>(F + 1);
-  L.bin_base     = ar.take<int64_t>(F);
-  L.bin_stride   = ar.take<int32_t>(F);
-  L.bin_tail     = ar.take<int32_t>(F);
+  L.bin_lanes    = ar.take<int2>(4 * static_cast<size_t>(F) + 16);
   L.rec          = ar.take<RecInfo>(F);
   L.upload_block = L.groups;
   L.upload_bytes = ar.used - upload_at;
-  L.binned_bytes = static_cast<size_t>(N) * bin_row_bytes_max(F, S);
+  L.binned_bytes = bin_cache_bytes(N, F, S);
   L.binned       = ar.take<char>(L.binned_bytes + 16);
-  L.tables       = ar.take<uint32_t>(2 * static_cast<size_t>(F) * kMaxCells / 16);
+  L.tables       = ar.take<uint2>(2 * static_cast<size_t>(F) * kMaxCells / 32);
   L.map_x        = ar.take<double>(4 * static_cast<size_t>(F));
   L.map_t        = ar.take<float>(2 * static_cast<size_t>(F));
   L.straight     = ar.take<int32_t>(F);
@@ -2907,7 +2897,7 @@ int lbt_histogram_level(void* stream, const void* X, int32_t x_dtype, int64_t n_
   HistSetup hs;
   hs.groups = L.groups; hs.sgroups = L.sgroups; hs.tables = L.tables; hs.map_x = L.map_x; hs.map_t = L.map_t; hs.straight = L.straight;
   hs.tile_start = L.tile_start; hs.tiles = L.tiles; hs.binned = L.binned; hs.binned_capacity = L.binned_bytes;
-  hs.bin_base = L.bin_base; hs.bin_stride = L.bin_stride; hs.bin_tail = L.bin_tail; hs.rec = L.rec;
+  hs.bin_lanes = L.bin_lanes; hs.rec = L.rec;
   hs.upload_block = L.upload_block; hs.upload_bytes = L.upload_bytes;
   hs.bins_t = nullptr;  // the feature-major copy serves the position updates of a whole build only
   hs.bins_t_stride = 0;

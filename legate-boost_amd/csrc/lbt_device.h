@@ -387,12 +387,22 @@ __device__ __forceinline__ int straight_cell_of(T x, T a, T b, float cmax)
   return static_cast<int>(__builtin_amdgcn_fmed3f(static_cast<float>(fma(x, a, b)), 0.0f, cmax));
 }
 
-constexpr int kCellsPerWord = 16;
-constexpr int kCellShift    = 4;  // log2(kCellsPerWord); cells are never negative
+// A table holds, for every 32 cells, the number of proposals in all cells before them (y) and a bit per proposal of theirs (x), at
+// its cell or, where another one has taken that, at the next free cell of the entry (at none behind the last). A value's start, y and
+// the bits below its cell, so never exceeds the number of proposals below it, and where its cell's bit is not set it is that number.
+// A field whose width the hardware takes modulo 32 and a count that adds give the start in two
+// vector instructions (six with 16 cells and the count in one word).
+constexpr int kCellsPerEntry = 32;
+constexpr int kCellShift     = 5;  // log2(kCellsPerEntry); cells are never negative
 
-__device__ inline int table_start(uint32_t word, int cell)
+__device__ __forceinline__ int table_start(const uint2& entry, int cell)
 {
-  return static_cast<int>(word >> 16) + __popc(word & ((1u << (cell & (kCellsPerWord - 1))) - 1u));
+  return static_cast<int>(entry.y) + __popc(__builtin_amdgcn_ubfe(entry.x, 0, static_cast<unsigned>(cell)));
+}
+// all ones where the cell's bit is set, else zero: the value's bin then is the start itself
+__device__ __forceinline__ int table_occupied(const uint2& entry, int cell)
+{
+  return __builtin_amdgcn_sbfe(static_cast<int>(entry.x), static_cast<unsigned>(cell), 1);
 }
 
 // The bent map of a feature is the one of a few candidates (linear; logarithmic on both sides of a
@@ -447,32 +457,41 @@ __device__ __forceinline__ int crowded_proposals(int c, const T* p, int n, int C
   return crowded;
 }
 
-// Table words of a feature under the cell function `cell`.
+// Table of a feature under the cell function `cell`, by the whole workgroup. The first proposal of an
+// entry says how many are before it (the cells of ascending proposals ascend), then a thread per entry places its bits.
+struct CellScratch {  // LDS
+  uint16_t cell[LBT_MAX_SPLIT_SAMPLES];
+  int count[kMaxCells / kCellsPerEntry + 1];
+};
 template <typename T, typename CellFn>
-__device__ inline void write_cell_words(const T* p, int n, int words, uint32_t* table, CellFn cell)
+__device__ __forceinline__ void write_cell_entries(const T* p, int n, int entries, CellScratch& s, uint2* table, CellFn cell)
 {
-  for (int w = threadIdx.x; w < words; w += blockDim.x) {
-    // first proposal whose cell is >= the first cell of the word (the cells of the ascending
-    // proposals ascend too)
-    const int c0 = w * kCellsPerWord;
-    int a = 0, len = n;
-    while (len > 0) {
-      int half = len >> 1;
-      if (cell(p[a + half]) < c0) {
-        a += half + 1;
-        len -= half + 1;
-      } else {
-        len = half;
-      }
-    }
-    uint32_t bits = 0;
-    for (int i = a; i < n; i++) {
-      const int c = cell(p[i]);
-      if (c >= c0 + kCellsPerWord) break;
-      bits |= 1u << (c - c0);
-    }
-    table[w] = (static_cast<uint32_t>(a) << 16) | bits;
+  constexpr uint16_t kNan = 0xffff;  // sampled NaNs (in front of the last proposal) have no cell
+  static_assert(kMaxCells < kNan, "a cell fits the scratch");
+  for (int i = threadIdx.x; i < n; i += blockDim.x) s.cell[i] = p[i] == p[i] ? static_cast<uint16_t>(cell(p[i])) : kNan;
+  for (int e = threadIdx.x; e <= entries; e += blockDim.x) s.count[e] = n;
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    if (s.cell[i] == kNan) continue;
+    int before = i - 1;
+    while (before >= 0 && s.cell[before] == kNan) before--;
+    const int last = s.cell[i] >> kCellShift;
+    for (int e = before < 0 ? 0 : (s.cell[before] >> kCellShift) + 1; e <= last; e++) s.count[e] = i;
   }
+  __syncthreads();
+  for (int e = threadIdx.x; e < entries; e += blockDim.x) {
+    const int i0 = s.count[e], i1 = s.count[e + 1];
+    uint32_t bits = 0;
+    int at        = -1;
+    for (int i = i0; i < i1; i++) {
+      if (s.cell[i] == kNan) continue;
+      at = max(static_cast<int>(s.cell[i]) & (kCellsPerEntry - 1), at + 1);
+      if (at >= kCellsPerEntry) break;
+      bits |= 1u << at;
+    }
+    table[e] = make_uint2(bits, static_cast<uint32_t>(i0));
+  }
+  __syncthreads();
 }
 
 // Number of proposals in [p, p+n) that are < x (branch-free, fixed trip count).

@@ -362,6 +362,7 @@ struct LevelMeta {
 // bytes up to zero_end, and (single-output trees) the row's packed (grad, hess) pair at q_off.
 struct RecInfo {
   int64_t base;      // byte offset of row 0's record
+  int32_t in_row;    // of them, from the first byte of row 0 of its plane (see hist_prepare)
   int32_t stride;    // bytes between the records of consecutive rows (multiple of 32)
   int32_t size;      // bytes of one record (multiple of 32)
   int32_t q_off;     // byte offset of the int2 (grad, hess) inside a record, or -1
@@ -383,7 +384,7 @@ struct HistSetup {
   int32_t* groups    = nullptr;  // [n_groups + 1]
   int32_t* sgroups   = nullptr;  // [n_sgroups + 1]; the same array as groups when the cache is off
   // lookup tables and cell functions of the search (see build_cells_kernel)
-  uint32_t* tables   = nullptr;  // [2][n_features][cells / 16]: one word per 16 cells
+  uint2* tables      = nullptr;  // [2][n_features][cells / 32]: one entry per 32 cells
   void* map_x        = nullptr;  // X dtype [2][n_features][2]
   float* map_t       = nullptr;  // [n_features][2]
   int32_t* straight  = nullptr;  // [n_features]
@@ -414,17 +415,16 @@ struct HistSetup {
   int even_lanes       = 0;        // lanes per row shared by all groups of a histogram launch; 0: per group
   int spread           = 0;        // bins a lane takes of a row where four lanes share them evenly (Stripes::per); 0: they do not
   RecInfo* rec         = nullptr;  // [n_groups]
-  int64_t max_rec_stride = 0;      // widest record, bytes
+  int64_t max_rec_stride = 0;      // widest row of a plane, bytes
+  int64_t row_bytes      = 0;      // bytes of a row in all planes
   int pieces           = 0;        // 16-byte pieces of bins of a row's records
   int max_bins         = 0;        // bins of the widest feature
-  int64_t* bin_base    = nullptr;  // [n_features] element offset of the feature's bin of row 0
-  int32_t* bin_stride  = nullptr;  // [n_features] elements between consecutive rows
-  int32_t* bin_tail    = nullptr;  // [n_features] g + 1 for the last feature of histogram group g, else 0
+  int2* bin_lanes      = nullptr;  // [4 * n_features + 16] lanes of a row in the binning pass (see bin_lanes)
   // feature-major copy of the bins, [feature][row], written by the root histogram launch for the
   // position updates (null: not wanted)
   void* bins_t           = nullptr;
   int64_t bins_t_stride  = 0;      // elements between consecutive features (multiple of 128)
-  // the part of the workspace that holds groups, sgroups, bin_base, bin_stride, bin_tail and rec
+  // the part of the workspace that holds groups, sgroups, bin_lanes and rec
   // (and nothing else): hist_prepare fills it with one copy
   void* upload_block   = nullptr;
   size_t upload_bytes  = 0;
@@ -432,7 +432,7 @@ struct HistSetup {
   int brpp             = 0;        // rows per workgroup pass, histogram kernel on cached bins
 };
 
-constexpr int kMaxCells = 16384;  // table cells per feature at most (one 32-bit word per 16 cells)
+constexpr int kMaxCells = 16384;  // table cells per feature at most (one entry of 8 bytes per 32 cells)
 constexpr int kPairSyncSlots = 4096;
 // bins of the widest feature group that fits the LDS beside the lanes' spare slots
 constexpr int kPartialStrideMax = (160 * 1024 - 512 - 4096 - 8 * 1024) / 8;
@@ -456,6 +456,13 @@ inline int64_t bin_row_bytes_max(int n_features, int split_samples)
   // one more for the uneven widths of a balanced split, two more that may be taken to fill idle CUs
   const int64_t groups_max = (n_features + cap - 1) / cap + 3;
   return static_cast<int64_t>(n_features) * bin_bytes + groups_max * 48;
+}
+
+// ... and the cache as a whole: at most a plane per feature, each starting on a multiple of kPlaneAlign bytes
+constexpr int kPlaneAlign = 128;
+inline size_t bin_cache_bytes(int64_t n_rows, int n_features, int split_samples)
+{
+  return static_cast<size_t>(n_rows * bin_row_bytes_max(n_features, split_samples)) + static_cast<size_t>(kPlaneAlign) * n_features;
 }
 
 struct HistBatch {
@@ -582,7 +589,7 @@ struct MidTreeState {
   void* props;            // X dtype [F][S]
   double* proposals;      // [F][S] the same
   int cells;              // cell functions and tables of the bin search, [F] each (see build_cells_kernel)
-  uint32_t* tables;       // [F][cells / 16]
+  uint2* tables;          // [F][cells / 32]
   void* map_x;            // X dtype [F][2]
   float* map_t;           // [F][2]
   int32_t* counts;        // [F]

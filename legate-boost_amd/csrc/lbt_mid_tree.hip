@@ -133,9 +133,10 @@ __global__ void __launch_bounds__(kWide)
       if (s_crowded[c] < s_crowded[best]) best = c;
     const CellMap<T> m = cell_map_candidate(best, p, n, static_cast<float>(st.cells));
     const float cmax   = static_cast<float>(st.cells - 1);
-    const int words    = st.cells / kCellsPerWord;
-    write_cell_words(p, n, words, st.tables + static_cast<int64_t>(block) * words,
-                     [&](T x) { return cell_of(x, m.scale, m.shift, m.invw, m.nlo, cmax); });
+    const int entries  = st.cells / kCellsPerEntry;
+    __shared__ CellScratch s_cells;
+    write_cell_entries(p, n, entries, s_cells, st.tables + static_cast<int64_t>(block) * entries,
+                       [&](T x) { return cell_of(x, m.scale, m.shift, m.invw, m.nlo, cmax); });
     if (tid == 0) {
       static_cast<T*>(st.map_x)[2 * block]     = m.scale;
       static_cast<T*>(st.map_x)[2 * block + 1] = m.shift;
@@ -280,16 +281,16 @@ __global__ void __launch_bounds__(kWide)
   const int block = static_cast<int>(blockIdx.x) - p.quant_groups;
   const int fblk = block % p.n_fb, rg = block / p.n_fb;
   const int f0 = fblk * p.fb, nf = min(p.fb, a.F - f0);
-  const int pitch = prop_pitch(a.S), words = st.cells / kCellsPerWord, tpitch = words | 1;
-  T* s_prop         = reinterpret_cast<T*>(smem_raw);                              // [fb][pitch]
-  uint32_t* s_table = reinterpret_cast<uint32_t*>(s_prop + static_cast<size_t>(p.fb) * pitch);  // [fb][tpitch]
-  int* s_n          = reinterpret_cast<int*>(s_table + p.fb * tpitch);
+  const int pitch = prop_pitch(a.S), entries = st.cells / kCellsPerEntry, tpitch = entries | 1;
+  uint2* s_table = reinterpret_cast<uint2*>(smem_raw);            // [fb][tpitch]
+  T* s_prop      = reinterpret_cast<T*>(s_table + p.fb * tpitch);  // [fb][pitch]
+  int* s_n       = reinterpret_cast<int*>(s_prop + static_cast<size_t>(p.fb) * pitch);
   constexpr int kTilePitch = kRowsBin + 4 / sizeof(BinT);
   BinT* s_bin       = reinterpret_cast<BinT*>(s_n + p.fb);  // [fb][kTilePitch]
   for (int i = tid; i < nf; i += kWide) s_n[i] = st.counts[f0 + i];
-  for (int i = tid; i < nf * words; i += kWide) {
-    const int fi = i / words, j = i - fi * words;
-    s_table[fi * tpitch + j] = st.tables[static_cast<int64_t>(f0 + fi) * words + j];
+  for (int i = tid; i < nf * entries; i += kWide) {
+    const int fi = i / entries, j = i - fi * entries;
+    s_table[fi * tpitch + j] = st.tables[static_cast<int64_t>(f0 + fi) * entries + j];
   }
   __syncthreads();
   for (int i = tid; i < nf * pitch; i += kWide) {
@@ -306,8 +307,8 @@ __global__ void __launch_bounds__(kWide)
   for (int tile = rg; tile < tiles; tile += p.row_groups) {
     __syncthreads();
     if (fi < nf) {
-      const T* prop         = s_prop + fi * pitch;
-      const uint32_t* table = s_table + fi * tpitch;
+      const T* prop      = s_prop + fi * pitch;
+      const uint2* table = s_table + fi * tpitch;
       // four rows at a time, their searches side by side: the table's start, three probes at once, and for the
       // few lanes that need more four further ones and a binary search (as in bin_rows_kernel)
       for (int r = r_first; r < kRowsBin; r += 4 * r_step) {
@@ -1072,7 +1073,7 @@ int mid_tree_build(hipStream_t stream, const MidTreeState& st, const T* X, int64
     p.search_steps = 0;
     while ((1 << p.search_steps) < a.S + 1) p.search_steps++;
     // features of a workgroup: what the search needs of them fits 64 KB, two workgroups a CU
-    const size_t per_feature = prop_pitch(a.S) * sizeof(T) + (st.cells / 16 + 1) * 4 + 4 + (kRowsBin + 4) * st.bin_bytes;
+    const size_t per_feature = prop_pitch(a.S) * sizeof(T) + (st.cells / kCellsPerEntry + 1) * sizeof(uint2) + 4 + (kRowsBin + 4) * st.bin_bytes;
     p.fb     = std::max(1, std::min<int>(F, std::min<int>(32, static_cast<int>(64 * 1024 / per_feature))));
     p.fb_log = 0;
     while ((1 << p.fb_log) < p.fb) p.fb_log++;
