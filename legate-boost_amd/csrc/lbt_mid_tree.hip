@@ -37,7 +37,8 @@ constexpr int kWide     = 1024;  // threads of all kernels but the scan
 constexpr int kScan     = 256;
 constexpr int kNone     = 0xffff;
 constexpr int kRowsBin  = 256;   // rows of a binning tile
-constexpr int kQuantPer = 8192;  // entries a workgroup rounds
+template <typename T>
+constexpr int kMaxFb    = 128 / sizeof(T);  // features of a binning workgroup: a cache line of a row
 constexpr int kRowsApply = 4 * kWide;
 constexpr size_t kHistLds = 128 * 1024;
 constexpr int64_t kNodesMost = 2500000;  // rows times workgroups that find the nodes of the same ones (nodes_with_histograms)
@@ -177,6 +178,7 @@ __global__ void __launch_bounds__(kWide)
 
 struct BinPlan {
   int quant_groups;  // workgroups of the quantiser
+  int quant_per;     // entries that one of them rounds, a multiple of kWide
   int fb;            // features of a binning workgroup
   int fb_log;        // lanes per row, log2
   int n_fb;          // feature blocks
@@ -187,8 +189,12 @@ struct BinPlan {
 // LDS elements per feature: the proposals, the +inf entries a window of probes may touch, and an odd pitch
 __host__ __device__ constexpr int prop_pitch(int S) { return (S + 8) | 1; }
 
+// What bounds it is latency: a few tiles per workgroup behind a chain of launch, tables and first rows, and the quantiser's own
+// chain beside it. With the first rows asked for before the tables, all of a thread's loads of these under way together, the searches side by
+// side and 1024 entries to a workgroup of the quantiser 100,000 x 32 takes 11 us (20.5), 250,000 x 43 30 (41), 1,500,000 x 33 118 (150),
+// 1,304,790 x 26 in double with 3 outputs 116 (166). Two workgroups to a CU: 64 registers.
 template <typename T, typename BinT>
-__global__ void __launch_bounds__(kWide)
+__global__ void __launch_bounds__(kWide, 8)
   mid_bin_kernel(const T* __restrict__ X, MidArgs a, MidTreeState st, BinPlan p)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -230,15 +236,25 @@ __global__ void __launch_bounds__(kWide)
       if (tid == kWide - 1) st.rp[a.F] = run;
     }
     const int64_t n  = static_cast<int64_t>(a.N) * a.K;
-    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * kQuantPer, e1 = e0 + kQuantPer < n ? e0 + kQuantPer : n;
+    const int64_t e0 = static_cast<int64_t>(blockIdx.x) * p.quant_per, e1 = e0 + p.quant_per < n ? e0 + p.quant_per : n;
     int64_t sum_g = 0, sum_h = 0;
     unsigned long long up = 0, down = 0;
     unsigned flags = 0;
+    double grad = 0.0, hess = 0.0;
+    if (e0 + tid < e1) {
+      grad = a.g[e0 + tid];
+      hess = a.h[e0 + tid];
+    }
     for (int64_t e = e0 + tid; e < e1; e += kWide) {
+      const double g = grad, h = hess;
+      if (e + kWide < e1) {
+        grad = a.g[e + kWide];
+        hess = a.h[e + kWide];
+      }
       const int64_t row = a.K == 1 ? e : e / a.K;
       const int k       = a.K == 1 ? 0 : static_cast<int>(e - row * a.K);
       int64_t qg, qh;
-      quantise_pair(a.g[e], a.h[e], sg, sh, static_cast<int64_t>(a.seed), row + a.row_offset, k, &qg, &qh);
+      quantise_pair(g, h, sg, sh, static_cast<int64_t>(a.seed), row + a.row_offset, k, &qg, &qh);
       if (qg > 2147483647LL || qg < -2147483647LL || qh > 2147483647LL || qh < -2147483647LL) flags |= 2u;
       if (qh < 0 || (qh == 0 && qg != 0 && !a.zeros_kept)) flags |= 1u;
       st.q[static_cast<int64_t>(k) * st.pitch + row] = make_int2(static_cast<int>(qg), static_cast<int>(qh));
@@ -287,60 +303,102 @@ __global__ void __launch_bounds__(kWide)
   int* s_n       = reinterpret_cast<int*>(s_prop + static_cast<size_t>(p.fb) * pitch);
   constexpr int kTilePitch = kRowsBin + 4 / sizeof(BinT);
   BinT* s_bin       = reinterpret_cast<BinT*>(s_n + p.fb);  // [fb][kTilePitch]
-  for (int i = tid; i < nf; i += kWide) s_n[i] = st.counts[f0 + i];
-  for (int i = tid; i < nf * entries; i += kWide) {
-    const int fi = i / entries, j = i - fi * entries;
-    s_table[fi * tpitch + j] = st.tables[static_cast<int64_t>(f0 + fi) * entries + j];
-  }
-  __syncthreads();
-  for (int i = tid; i < nf * pitch; i += kWide) {
-    const int fi = i / pitch, j = i - fi * pitch;
-    // +inf behind the last proposal, for the probes that run past it
-    s_prop[i] = j < s_n[fi] ? static_cast<const T*>(st.props)[static_cast<int64_t>(f0 + fi) * a.S + j] : std::numeric_limits<T>::infinity();
-  }
   const int fi = tid & ((1 << p.fb_log) - 1), r_first = tid >> p.fb_log, r_step = kWide >> p.fb_log;
-  const int fm = min(f0 + fi, a.F - 1);
-  const T scale = static_cast<const T*>(st.map_x)[2 * fm], shift = static_cast<const T*>(st.map_x)[2 * fm + 1];
-  const float invw = st.map_t[2 * fm], nlo = st.map_t[2 * fm + 1], cmax = static_cast<float>(st.cells - 1);
+  const int fm = f0 + min(fi, nf - 1);  // lanes without a feature of their own search the last one's values
   const int tiles = (a.N + kRowsBin - 1) / kRowsBin;
-  BinT* const out = static_cast<BinT*>(st.bins);
-  for (int tile = rg; tile < tiles; tile += p.row_groups) {
-    __syncthreads();
-    if (fi < nf) {
-      const T* prop      = s_prop + fi * pitch;
-      const uint2* table = s_table + fi * tpitch;
-      // four rows at a time, their searches side by side: the table's start, three probes at once, and for the
-      // few lanes that need more four further ones and a binary search (as in bin_rows_kernel)
-      for (int r = r_first; r < kRowsBin; r += 4 * r_step) {
-        T x[4];
-        int bn[4], cnt[4];
+  // A thread's values of a tile: on their way while the tables come into the LDS, or while the tile before is written.
+  constexpr int kMost  = kRowsBin * kMaxFb<T> / kWide;
+  constexpr int kBatch = sizeof(T) == 4 ? 4 : 2;  // values searched side by side
+  T x[kMost];
+  auto fetch = [&](int tile) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-          const int64_t row = static_cast<int64_t>(tile) * kRowsBin + r + u * r_step;
-          x[u]              = r + u * r_step < kRowsBin && row < a.N ? X[row * a.F + f0 + fi] : T(0);
-        }
+    for (int u = 0; u < kMost; u++) {
+      const int r       = min(r_first + u * r_step, kRowsBin - 1);
+      const int64_t row = min(static_cast<int64_t>(tile) * kRowsBin + r, static_cast<int64_t>(a.N) - 1);
+      x[u]              = X[row * a.F + fm];
+    }
+  };
+  fetch(rg);
+  for (int i = tid; i < nf; i += kWide) s_n[i] = st.counts[f0 + i];
+  // a feature per half wave, what lies behind its last proposal is set apart below
+  {
+    const int half = tid >> 5, j0 = tid & 31;
+    for (int c = half; c < nf; c += kWide / 32) {
+      const uint2* src = st.tables + static_cast<int64_t>(f0 + c) * entries;
+      const T* from    = static_cast<const T*>(st.props) + static_cast<int64_t>(f0 + c) * a.S;
+      uint2 e[2];
+      T v[8];
+      for (int b = 0; b < max(entries, (a.S + 3) / 4); b += 64) {  // 64 entries and 256 samples under way at once
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-          const int cell = cell_of(x[u], scale, shift, invw, nlo, cmax);
-          bn[u]          = table_start(table[static_cast<unsigned>(cell) >> kCellShift], cell);
-          const T* pp    = prop + bn[u];
-          cnt[u]         = (pp[0] < x[u] ? 1 : 0) + (pp[1] < x[u] ? 1 : 0) + (pp[2] < x[u] ? 1 : 0);
-        }
+        for (int u = 0; u < 2; u++) e[u] = src[min(b + j0 + 32 * u, entries - 1)];
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-          if (__any(cnt[u] == 3)) {
-            const T* pp  = prop + bn[u] + 3;
-            const int c2 = (pp[0] < x[u] ? 1 : 0) + (pp[1] < x[u] ? 1 : 0) + (pp[2] < x[u] ? 1 : 0) + (pp[3] < x[u] ? 1 : 0);
-            cnt[u] += cnt[u] == 3 ? c2 : 0;
-            if (__any(cnt[u] == 7)) {
-              const int left = cnt[u] == 7 ? s_n[fi] - (bn[u] + 7) : 0;
-              cnt[u] += count_less(pp + 4, left, x[u], p.search_steps);
-            }
-          }
-          if (r + u * r_step < kRowsBin) s_bin[fi * kTilePitch + r + u * r_step] = static_cast<BinT>(bn[u] + cnt[u]);
-        }
+        for (int u = 0; u < 8; u++) v[u] = from[min(4 * b + j0 + 32 * u, a.S - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+          if (b + j0 + 32 * u < entries) s_table[c * tpitch + b + j0 + 32 * u] = e[u];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+          if (4 * b + j0 + 32 * u < a.S) s_prop[c * pitch + 4 * b + j0 + 32 * u] = v[u];
       }
     }
+  }
+  __syncthreads();
+  // +inf from the last proposal on, for the probes that run past it
+  for (int i = tid; i < nf * 8; i += kWide) s_prop[(i >> 3) * pitch + s_n[i >> 3] - 1 + (i & 7)] = std::numeric_limits<T>::infinity();
+  const T scale = static_cast<const T*>(st.map_x)[2 * fm], shift = static_cast<const T*>(st.map_x)[2 * fm + 1];
+  const float invw = st.map_t[2 * fm], nlo = st.map_t[2 * fm + 1], cmax = static_cast<float>(st.cells - 1);
+  BinT* const out = static_cast<BinT*>(st.bins);
+  const T* prop      = s_prop + min(fi, nf - 1) * pitch;
+  const uint2* table = s_table + min(fi, nf - 1) * tpitch;
+  for (int tile = rg; tile < tiles; tile += p.row_groups) {
+    __syncthreads();
+    // the searches of a batch go stage by stage, as in bin_rows_kernel: the table's entries, three probes at once, and for the
+    // few lanes that need more four further ones and a binary search
+#pragma unroll
+    for (int u0 = 0; u0 < kMost; u0 += kBatch) {
+      if (u0 * r_step >= kRowsBin) break;
+      int bn[kBatch], cell[kBatch];
+      uint2 entry[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; u++) {
+        cell[u]  = cell_of(x[u0 + u], scale, shift, invw, nlo, cmax);
+        entry[u] = table[static_cast<unsigned>(cell[u]) >> kCellShift];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      T probe[kBatch][3];
+#pragma unroll
+      for (int u = 0; u < kBatch; u++) {
+        bn[u] = table_start(entry[u], cell[u]);
+#pragma unroll
+        for (int i = 0; i < 3; i++) probe[u][i] = prop[bn[u] + i];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      bool more = false;
+#pragma unroll
+      for (int u = 0; u < kBatch; u++) {
+        const T v = x[u0 + u];
+        bn[u] += (probe[u][0] < v ? 1 : 0) + (probe[u][1] < v ? 1 : 0) + (probe[u][2] < v ? 1 : 0);
+        more = more || probe[u][2] < v;
+      }
+      if (__any(more)) {
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) {
+          const T v   = x[u0 + u];
+          const T* pp = prop + bn[u];
+          if (!__any(pp[0] < v)) continue;
+          const int c2 = (pp[0] < v ? 1 : 0) + (pp[1] < v ? 1 : 0) + (pp[2] < v ? 1 : 0) + (pp[3] < v ? 1 : 0);
+          bn[u] += c2;
+          if (__any(c2 == 4)) bn[u] += count_less(pp + 4, c2 == 4 ? s_n[min(fi, nf - 1)] - bn[u] : 0, v, p.search_steps);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; u++) {
+        const int r = r_first + (u0 + u) * r_step;
+        if (fi < nf && r < kRowsBin) s_bin[fi * kTilePitch + r] = static_cast<BinT>(bn[u]);
+      }
+    }
+    if (tile + p.row_groups < tiles) fetch(tile + p.row_groups);
     __syncthreads();
     constexpr int kPer = 4 / sizeof(BinT);  // bins per word
     for (int i = tid; i < nf * (kRowsBin / kPer); i += kWide) {
@@ -1069,17 +1127,27 @@ int mid_tree_build(hipStream_t stream, const MidTreeState& st, const T* X, int64
   {
     ProfScope ps(LBT_PROF_BINNING, stream);
     BinPlan p;
-    p.quant_groups = static_cast<int>((N * K + kQuantPer - 1) / kQuantPer);
+    // few entries a thread: the launch lasts as long as the quantiser's chain of loads, roundings and sums (8192 a workgroup:
+    // 18 us on 100,000 x 32, whatever the binning took)
+    p.quant_per    = static_cast<int>(std::min<int64_t>(8, std::max<int64_t>(1, (N * K + 128 * kWide - 1) / (128 * kWide)))) * kWide;
+    p.quant_groups = static_cast<int>((N * K + p.quant_per - 1) / p.quant_per);
     p.search_steps = 0;
     while ((1 << p.search_steps) < a.S + 1) p.search_steps++;
     // features of a workgroup: what the search needs of them fits 64 KB, two workgroups a CU
     const size_t per_feature = prop_pitch(a.S) * sizeof(T) + (st.cells / kCellsPerEntry + 1) * sizeof(uint2) + 4 + (kRowsBin + 4) * st.bin_bytes;
-    p.fb     = std::max(1, std::min<int>(F, std::min<int>(32, static_cast<int>(64 * 1024 / per_feature))));
+    p.fb     = std::max(1, std::min<int>(F, std::min<int>(kMaxFb<T>, static_cast<int>(64 * 1024 / per_feature))));
+    p.n_fb   = (F + p.fb - 1) / p.fb;
+    p.fb     = (F + p.n_fb - 1) / p.n_fb;  // blocks of even width
     p.fb_log = 0;
     while ((1 << p.fb_log) < p.fb) p.fb_log++;
-    p.n_fb       = (F + p.fb - 1) / p.fb;
     const int tiles = static_cast<int>((N + kRowsBin - 1) / kRowsBin);
-    p.row_groups = std::max(1, std::min(tiles, 1024 / p.n_fb));
+    // Tiles in equal shares to no more workgroups than run at once, two to a CU (with a few more than that the last ones take all of a second
+    // turn: 250,000 x 43 in 77 us for 29): beside the quantiser's, or behind them, whichever ends sooner by some 4 us a tile and 2 us
+    // for 1024 entries.
+    auto tiles_each = [&](int beside) { const int most = std::max(1, (512 - beside) / p.n_fb); return (tiles + most - 1) / most; };
+    const int beside = tiles_each(std::min(384, p.quant_groups)), behind = tiles_each(0);
+    const int each   = 4 * beside <= 4 * behind + 4 + 2 * (p.quant_per / kWide) ? beside : behind;
+    p.row_groups     = (tiles + each - 1) / each;
     const size_t lds = std::max<size_t>(static_cast<size_t>(p.fb) * per_feature + 16, 2 * kWide * sizeof(double));
     static std::atomic<bool> attr_set[2][kMaxDevices] = {};
     const unsigned grid = static_cast<unsigned>(p.quant_groups + p.n_fb * p.row_groups);

@@ -64,3 +64,19 @@ def test_root_histogram_of_binned_rows(n, f, k, dtype, samples):
         for j in range(k):
             np.add.at(want[j], rp[c] + b, q[:, j].astype(np.int64))
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n,f,k,dtype,samples", [
+    (8447, 33, 1, np.float32, 256), (9000, 17, 1, np.float64, 300), (12345, 65, 1, np.float32, 64), (8961, 1, 2, np.float32, 16),
+    (140000, 5, 1, np.float32, 512), (10241, 3, 3, np.float64, 1024),
+])
+def test_medium_builder_bins(n, f, k, dtype, samples):
+    """The builder for medium sizes: blocks of features of even width, tiles and samples that fill no whole turn."""
+    import gpu_util as gu
+
+    rs = np.random.RandomState(n)
+    X = np.abs(_columns(n, f, dtype, rs))
+    X[~np.isfinite(X)] = 1  # (which samples are taken is up to the seed)
+    g, h = rs.normal(size=(n, k)), 0.5 + rs.rand(n, k)
+    gr, cr = gu.both(X, g, h, max_depth=3, split_samples=samples, seed=5)
+    gu.assert_tree_parity(gr, cr)
