@@ -82,6 +82,22 @@ __device__ __forceinline__ double wave_read_lane_f64(double v, int src)
 __device__ __forceinline__ void arrived(int2& v) { asm volatile("" : "+v"(v.x), "+v"(v.y)); }
 __device__ __forceinline__ void arrived(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 
+// put(i, take(i)) for i = threadIdx.x, + kT, ... below n: kAhead loads are under way at once. (A loop over both, as hipcc
+// leaves it, waits for every load: 2 us each where another die wrote what it reads.)
+template <int kT, int kAhead, typename Take, typename Put>
+__device__ __forceinline__ void copy_ahead(int n, Take take, Put put)
+{
+  for (int i0 = threadIdx.x; i0 < n; i0 += kT * kAhead) {
+    decltype(take(0)) v[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) v[u] = take(min(i0 + u * kT, n - 1));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kAhead; u++)
+      if (i0 + u * kT < n) put(i0 + u * kT, v[u]);
+  }
+}
+
 struct Cand {
   double gain;
   int bin;

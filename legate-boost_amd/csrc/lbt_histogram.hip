@@ -995,8 +995,13 @@ __global__ void __launch_bounds__(kHistThreads)
   T* s_prop        = reinterpret_cast<T*>(smem_raw);
   const int cell_at = ((nb + kProbePad * (gs + 1) + kProbeSlack) * static_cast<int>(sizeof(T)) + 7) & ~7;
   uint2* s_cell    = reinterpret_cast<uint2*>(smem_raw + cell_at);
-  for (int i = threadIdx.x; i < nb; i += kHistThreads)
-    s_prop[i + kProbePad * (a.bin_feature[bin0 + i] - f0 + 1)] = a.proposals[bin0 + i];
+  struct Proposal {
+    T value;
+    int feature;
+  };
+  copy_ahead<kHistThreads, 8>(
+    nb, [&](int i) { return Proposal{a.proposals[bin0 + i], a.bin_feature[bin0 + i]}; },
+    [&](int i, const Proposal& p) { s_prop[i + kProbePad * (p.feature - f0 + 1)] = p.value; });
   for (int i = threadIdx.x; i < kProbePad * (gs + 1) + kProbeSlack; i += kHistThreads) {
     const int f = min(i / kProbePad, gs);  // the pad in front of feature f; the slack follows the last one
     s_prop[a.row_pointers[f0 + f] - bin0 + i] = std::numeric_limits<T>::infinity();
@@ -1008,7 +1013,7 @@ __global__ void __launch_bounds__(kHistThreads)
   {
     const uint2* src  = a.tables + static_cast<int64_t>(bent ? f0 : a.F + f0) * (C / kCellsPerEntry);
     const int entries = gs * (C / kCellsPerEntry);
-    for (int i = threadIdx.x; i < entries; i += kHistThreads) s_cell[i] = src[i];
+    copy_ahead<kHistThreads, 8>(entries, [&](int i) { return src[i]; }, [&](int i, const uint2& e) { s_cell[i] = e; });
   }
   // The lanes of a row (see bin_lanes). Every lane that owns bins owns VEC real features (the last one of a ragged row: `mine` of them).
   const int2 head   = a.lanes[2 * group], plane = a.lanes[2 * group + 1];
