@@ -18,7 +18,7 @@ namespace {
 constexpr int kPassTrees     = 16;          // trees whose nodes lie in the LDS at a time
 constexpr int kLeafThreads   = 512;
 constexpr int kRoundThreads  = 1024;
-constexpr int kTogether      = 4;           // trees a lane walks at once
+constexpr int kTogether      = 4;           // trees a lane walks at once, at most
 constexpr int kAheadWords    = 8;           // 16-byte words of the next tile that a lane holds
 constexpr size_t kNodeLds    = 64 * 1024;
 constexpr size_t kTwoPerCu   = 78 * 1024;
@@ -60,8 +60,9 @@ typedef unsigned int Word16 __attribute__((ext_vector_type(4)));
 
 // The node every row stops in, for up to kPassTrees trees. Their nodes stay in the LDS; kStaged: so do the rows of a tile, whose
 // successor is on its way into registers meanwhile (rows too wide for that are walked in memory). The lanes of a row take its
-// trees in turn. What bounds it is X in one sweep.
-template <typename T, bool kStaged>
+// trees in turn, kWalks each side by side. What bounds it are the walk's LDS reads, two a step and lane: walks that no tree needs are as dear as
+// others (1,000,000 x 50, 10 trees of depth 8, four lanes a row: with four walks each 61 us, with three 55).
+template <typename T, bool kStaged, int kWalks>
 __global__ void __launch_bounds__(kLeafThreads)
   tree_leaves_kernel(const T* __restrict__ X, LeavesArgs a, const PackedNode<T>* __restrict__ nodes, uint16_t* __restrict__ row_leaf)
 {
@@ -125,19 +126,19 @@ __global__ void __launch_bounds__(kLeafThreads)
     const int64_t row = tile * a.tile_rows + r;
     const bool valid  = row < a.n_rows;
     const T* x        = kStaged ? s_x + (valid ? r : 0) * a.pitch : X + (valid ? row : 0) * a.F;
-    for (int t0 = q; t0 < a.n_trees; t0 += kTogether * lanes) {
-      int base[kTogether], pos[kTogether];
+    for (int t0 = q; t0 < a.n_trees; t0 += kWalks * lanes) {
+      int base[kWalks], pos[kWalks];
 #pragma unroll
-      for (int j = 0; j < kTogether; j++) {
+      for (int j = 0; j < kWalks; j++) {
         base[j] = a.node_off[min(t0 + j * lanes, a.n_trees - 1)];
         pos[j]  = 0;
       }
       for (int s = 0; s < a.steps; s++) {
 #pragma unroll
-        for (int j = 0; j < kTogether; j++) pos[j] = step_from<T>(s_nodes[base[j] + pos[j]], x);
+        for (int j = 0; j < kWalks; j++) pos[j] = step_from<T>(s_nodes[base[j] + pos[j]], x);
       }
 #pragma unroll
-      for (int j = 0; j < kTogether; j++)
+      for (int j = 0; j < kWalks; j++)
         if (valid && t0 + j * lanes < a.n_trees)
           row_leaf[static_cast<int64_t>(t0 + j * lanes) * a.n_rows + row] = static_cast<uint16_t>(pos[j]);
     }
@@ -387,7 +388,7 @@ int update_rounds(hipStream_t stream, const T* X, int64_t N, int F, int objectiv
   }
   zero_sums_kernel<<<ceil_div(p.sums, 256), 256, 0, stream>>>(sums, p.sums);
 
-  static std::atomic<bool> leaf_attr[2][kMaxDevices] = {}, round_attr[13][kMaxDevices] = {}, finish_attr[kMaxDevices] = {};
+  static std::atomic<bool> round_attr[13][kMaxDevices] = {}, finish_attr[kMaxDevices] = {};
   const unsigned round_grid = static_cast<unsigned>(std::min<int64_t>(256, ceil_div(N, kRoundThreads)));
   auto round = [&](auto kind_c, auto cols_c, std::atomic<bool> (&flags)[kMaxDevices], const RoundArgs& a) -> int {
     constexpr Gradient kKind = decltype(kind_c)::value;
@@ -446,13 +447,26 @@ int update_rounds(hipStream_t stream, const T* X, int64_t N, int F, int objectiv
     uint16_t* to      = row_leaf + static_cast<int64_t>(t % slots) * N;
     const int per_cu  = staged && lds > kTwoPerCu ? 1 : 2;
     const unsigned grid = static_cast<unsigned>(std::min<int64_t>(a.n_tiles, 256 * per_cu));
-    if (staged) {
-      LBT_TRY((allow_dynamic_lds(tree_leaves_kernel<T, true>, kOnePerCu, leaf_attr[0])));
-      tree_leaves_kernel<T, true><<<grid, kLeafThreads, lds, stream>>>(X, a, nodes + node_off[t], to);
-    } else {
-      LBT_TRY((allow_dynamic_lds(tree_leaves_kernel<T, false>, kNodeLds, leaf_attr[1])));
-      tree_leaves_kernel<T, false><<<grid, kLeafThreads, node_lds, stream>>>(X, a, nodes + node_off[t], to);
-    }
+    // a lane's trees in as few turns as kTogether allows, and as many in each
+    const int row_lanes = kLeafThreads / a.tile_rows, trees_each = ceil_div(n, row_lanes);
+    const int walks     = ceil_div(trees_each, ceil_div(trees_each, kTogether));
+    auto launch         = [&](auto in_lds, auto together) -> int {
+      constexpr bool kStaged = decltype(in_lds)::value;
+      constexpr int kWalks   = decltype(together)::value;
+      static std::atomic<bool> attr[kMaxDevices] = {};
+      LBT_TRY((allow_dynamic_lds(tree_leaves_kernel<T, kStaged, kWalks>, kStaged ? kOnePerCu : kNodeLds, attr)));
+      tree_leaves_kernel<T, kStaged, kWalks><<<grid, kLeafThreads, kStaged ? lds : node_lds, stream>>>(X, a, nodes + node_off[t], to);
+      return LBT_OK;
+    };
+    auto launch_walks = [&](auto in_lds) -> int {
+      switch (walks) {
+        case 1: return launch(in_lds, integral_constant<int, 1>{});
+        case 2: return launch(in_lds, integral_constant<int, 2>{});
+        case 3: return launch(in_lds, integral_constant<int, 3>{});
+        default: return launch(in_lds, integral_constant<int, 4>{});
+      }
+    };
+    LBT_TRY((staged ? launch_walks(std::true_type{}) : launch_walks(std::false_type{})));
     for (int end = t + n; t < end; t++) {
       RoundArgs ra{};
       ra.n_rows  = N;
