@@ -304,26 +304,87 @@ __device__ __forceinline__ int cell_of(T x, T lo, T scale, int cells)
 // rows r and r + 32 of a wave share a word, so that those lanes read 32 banks whatever features they ask for.
 __device__ __forceinline__ int row_place(int row) { return (row & ~63) + 2 * (row & 31) + ((row >> 5) & 1); }
 
-// A workgroup has the thresholds of kSub * kGroup neighbouring features in its LDS and a lane takes its row's values of those,
-// kGroup at a time. Where the tables leave the room they are the features of one 128-byte line of a row: with fewer,
-// every line is fetched by several workgroups (500,003 x 200: 288 us with 8 features a workgroup, 228 with 32). The
-// workgroups of one row range are neighbours on one XCD, so that they find such lines in its L2.
+// Stores a wave's ranks of its 64 rows (a block of 64 of a tile) for kN neighbouring features, of which `here` exist: the lanes of two features exchange
+// halves, so that a lane holds the two rows of a word and a store is two whole cache lines. `to`: the block's word 0 of the first
+// feature. All lanes take part; what rows past the last one get is never read. (Where the search is what bounds a pass it gained
+// nothing: 20,000,000 x 64, eight features a lane, 2.56 ms with stores of two bytes, 2.63 with these.)
+template <int kN>
+__device__ __forceinline__ void store_ranks(const uint32_t (&code)[kN], int here, int tile_shift, char* to)
+{
+  const int lane = threadIdx.x & 63;
+  static_assert(kN % 2 == 0, "features in pairs");
+#pragma unroll
+  for (int j = 0; j < kN; j += 2) {
+    // of the second feature the lower lanes, of the first one the upper lanes
+    const auto swapped = __builtin_amdgcn_permlane32_swap(code[j], code[j + 1], false, false);
+    const int f        = j + (lane >> 5);
+    if (f < here)
+      *reinterpret_cast<uint32_t*>(to + ((static_cast<uint32_t>(2 * f) << tile_shift) + 4u * (static_cast<uint32_t>(lane) & 31u))) =
+        swapped[0] | swapped[1] << 16;
+  }
+}
+
+// What a workgroup's searches begin with: for each of its kAll features the cells' first places, how many probes tell the places of a
+// cell from one another, and the cell function. s_place, s_count: where its thresholds begin and how many there are. A wave per feature.
+template <typename T, int kAll>
+__device__ __forceinline__ void rank_cells(int cells, const T* s_tab, uint16_t* s_start, const int (&s_place)[kAll], const int (&s_count)[kAll],
+                                           int (&s_most)[kAll], T (&s_lo)[kAll], T (&s_scale)[kAll])
+{
+  const int tid = threadIdx.x;
+  for (int i = tid >> 6; i < kAll; i += kWalkWaves) {
+    const int m = s_count[i], lane = tid & 63;
+    if (m == 0) {
+      if (lane == 0) s_lo[i] = s_scale[i] = T(0);
+      continue;
+    }
+    const T* tab    = s_tab + s_place[i];
+    uint16_t* start = s_start + i * cells;
+    T lo            = tab[0];
+    T scale         = static_cast<T>(cells) / (tab[m - 1] - lo);
+    // the first threshold of a cell counts those before it, for that cell and the empty ones below it
+    int most = 0;
+    for (int e = lane; e < m; e += 64) {
+      const int c = cell_of(tab[e], lo, scale, cells);
+      const int p = e == 0 ? -1 : cell_of(tab[e - 1], lo, scale, cells);
+      for (int b = p + 1; b <= c; b++) start[b] = static_cast<uint16_t>(e);
+      if (e == m - 1)
+        for (int b = c + 1; b < cells; b++) start[b] = static_cast<uint16_t>(m);
+    }
+    wave_lds_fence();
+    for (int c = lane; c < cells; c += 64) most = max(most, (c + 1 < cells ? start[c + 1] : m) - start[c]);
+    for (int d = 32; d > 0; d /= 2) most = max(most, __shfl_xor(most, d, 64));
+    int probes = 32 - __clz(most);  // they tell 2^probes places from one another
+    wave_lds_fence();
+    if ((1 << probes) - 1 > m) {
+      // nearly all in one cell: two cells instead, below and above the threshold that a plain search asks first
+      probes = 31 - __clz(m);
+      lo     = tab[(1 << probes) - 1];
+      scale  = static_cast<T>(__builtin_huge_val());
+      for (int c = lane; c < cells; c += 64) start[c] = c == cells - 1 ? 0xffff : 0;
+    }
+    // a search may begin earlier (the thresholds before its cell are below x), and must where it would probe past the end
+    const int last = m + 1 - (1 << probes);
+    for (int c = lane; c < cells; c += 64) start[c] = static_cast<uint16_t>(min(static_cast<int>(start[c]), last));
+    if (lane == 0) {
+      s_most[i]  = probes;
+      s_lo[i]    = lo;
+      s_scale[i] = scale;
+    }
+  }
+}
+
+// A workgroup has the thresholds of kGroup neighbouring features in its LDS and a lane takes its row's values of those. The
+// workgroups of one row range are neighbours on one XCD, so that they find a line that several of them ask for in its L2.
 // ranks: [tile][feature][place of the row]
-// What bounds it are vector instructions, four per probe of a search and feature. With cells to start from a feature
-// of 4000 evenly spread thresholds takes 4 or 5 probes instead of 12 (20,000,000 x 64: 6.1 ms without cells, 2.8 with).
-// The features of a line come without their next row on its way; two workgroups to a CU wait for one another's rows instead: floats four
-// features at a time (59 registers, eight waves a SIMD; 500,003 x 200 with 50 trees and 8 outputs 468 -> 448 us a call against eight
-// at a time, 74 registers). Doubles take 63 with a spill that way and gained nothing: eight at a time, 87. So do floats whose rows are no
-// whole 16-byte words: a line's values are then 32 loads a row, and those of two workgroups leave no line in the L1 until its
-// last one is read (1,000,000 rows: 301 features with 60 trees 1680 us with two workgroups, 1209 with one; 499 with 20 2099 and 1530,
-// 33 with 40 trees of 8 outputs 435 and 385).
-template <typename T, int kGroup, int kSub>
-__global__ void __launch_bounds__(kWalkThreads, kSub > 1 && sizeof(T) == 4 && kGroup == 4 ? 8 : 4)
+// What bounds it are the LDS and vector instructions, a read and four instructions per probe of a search and feature. With cells to start
+// from a feature of 4000 evenly spread thresholds takes 4 or 5 probes instead of 12 (20,000,000 x 64: 6.1 ms without cells, 2.8 with, 2.56
+// since features with fewer probes take no part in the others').
+template <typename T, int kAll>
+__global__ void __launch_bounds__(kWalkThreads, 4)
   rank_rows_kernel(const T* __restrict__ X, RankRows a, RankState st, const T* __restrict__ sorted,
                    uint16_t* __restrict__ ranks)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  constexpr int kAll = kGroup * kSub;
   __shared__ int s_most[kAll], s_place[kAll], s_count[kAll];
   __shared__ T s_lo[kAll], s_scale[kAll];
   if (*st.overflow != 0) return;
@@ -351,49 +412,7 @@ __global__ void __launch_bounds__(kWalkThreads, kSub > 1 && sizeof(T) == 4 && kG
     for (int c = tid; c < kAll * a.cells; c += kWalkThreads) s_start[c] = 0;
   }
   __syncthreads();
-  if (held) {
-    // a wave per feature
-    for (int i = tid >> 6; i < kAll; i += kWalkWaves) {
-      const int m = s_count[i], lane = tid & 63;
-      if (m == 0) {
-        if (lane == 0) s_lo[i] = s_scale[i] = T(0);
-        continue;
-      }
-      const T* tab    = s_tab + s_place[i];
-      uint16_t* start = s_start + i * a.cells;
-      T lo            = tab[0];
-      T scale         = static_cast<T>(a.cells) / (tab[m - 1] - lo);
-      // the first threshold of a cell counts those before it, for that cell and the empty ones below it
-      int most = 0;
-      for (int e = lane; e < m; e += 64) {
-        const int c = cell_of(tab[e], lo, scale, a.cells);
-        const int p = e == 0 ? -1 : cell_of(tab[e - 1], lo, scale, a.cells);
-        for (int b = p + 1; b <= c; b++) start[b] = static_cast<uint16_t>(e);
-        if (e == m - 1)
-          for (int b = c + 1; b < a.cells; b++) start[b] = static_cast<uint16_t>(m);
-      }
-      wave_lds_fence();
-      for (int c = lane; c < a.cells; c += 64) most = max(most, (c + 1 < a.cells ? start[c + 1] : m) - start[c]);
-      for (int d = 32; d > 0; d /= 2) most = max(most, __shfl_xor(most, d, 64));
-      int probes = 32 - __clz(most);  // they tell 2^probes places from one another
-      wave_lds_fence();
-      if ((1 << probes) - 1 > m) {
-        // nearly all in one cell: two cells instead, below and above the threshold that a plain search asks first
-        probes = 31 - __clz(m);
-        lo     = tab[(1 << probes) - 1];
-        scale  = static_cast<T>(__builtin_huge_val());
-        for (int c = lane; c < a.cells; c += 64) start[c] = c == a.cells - 1 ? 0xffff : 0;
-      }
-      // a search may begin earlier (the thresholds before its cell are below x), and must where it would probe past the end
-      const int last = m + 1 - (1 << probes);
-      for (int c = lane; c < a.cells; c += 64) start[c] = static_cast<uint16_t>(min(static_cast<int>(start[c]), last));
-      if (lane == 0) {
-        s_most[i]  = probes;
-        s_lo[i]    = lo;
-        s_scale[i] = scale;
-      }
-    }
-  }
+  if (held) rank_cells<T, kAll>(a.cells, s_tab, s_start, s_place, s_count, s_most, s_lo, s_scale);
   __syncthreads();
   const int64_t end = min<int64_t>(a.n_rows, (split + 1) * a.rows_per_split);
   typedef T Vec __attribute__((ext_vector_type(16 / sizeof(T))));
@@ -413,72 +432,184 @@ __global__ void __launch_bounds__(kWalkThreads, kSub > 1 && sizeof(T) == 4 && kG
       for (int i = 0; i < kAll; i++) x[i] = src[i < nf ? i : 0];
     }
   };
-  int place[kGroup], probes[kGroup], most_probes = 0;
-  T lo[kGroup], scale[kGroup];
-  auto take_features = [&](int s) {
-    most_probes = 0;
+  int place[kAll], probes[kAll], most_probes = 0;
+  T lo[kAll], scale[kAll];
 #pragma unroll
-    for (int i = 0; i < kGroup; i++) {
-      place[i]    = __builtin_amdgcn_readfirstlane(s_place[s * kGroup + i]);
-      probes[i]   = __builtin_amdgcn_readfirstlane(s_most[s * kGroup + i]);
-      lo[i]       = s_lo[s * kGroup + i];
-      scale[i]    = s_scale[s * kGroup + i];
-      most_probes = max(most_probes, probes[i]);
-    }
-  };
-  take_features(0);
-  int64_t row = split * a.rows_per_split + tid;
-  T x[kAll], next[kSub == 1 ? kAll : 1];  // one group: its next row is fetched ahead
-  if constexpr (kSub == 1) {
-    if (row < end) load(row, next);
+  for (int i = 0; i < kAll; i++) {
+    place[i]    = __builtin_amdgcn_readfirstlane(s_place[i]);
+    probes[i]   = __builtin_amdgcn_readfirstlane(s_most[i]);
+    lo[i]       = s_lo[i];
+    scale[i]    = s_scale[i];
+    most_probes = max(most_probes, probes[i]);
   }
+  int64_t row = split * a.rows_per_split + tid;
+  T x[kAll], next[kAll];
+  if (row < end) load(row, next);
   for (; row < end; row += kWalkThreads) {
-    if constexpr (kSub == 1) {
 #pragma unroll
-      for (int i = 0; i < kAll; i++) x[i] = next[i];
-      if (row + kWalkThreads < end) load(row + kWalkThreads, next);
-    } else {
-      load(row, x);
-    }
+    for (int i = 0; i < kAll; i++) x[i] = next[i];
+    if (row + kWalkThreads < end) load(row + kWalkThreads, next);
     // tile rows are a power of two; a tile's ranks lie within 32 bits of bytes
     const int64_t tile = row >> a.tile_shift;
     char* base         = reinterpret_cast<char*>(ranks + (tile * a.F + f0) * (int64_t(1) << a.tile_shift));
     const uint32_t at0 = 2 * row_place(static_cast<int>(row) & ((1 << a.tile_shift) - 1));
+    int at[kAll];
+    if (held) {
 #pragma unroll
-    for (int s = 0; s < kSub; s++) {
-      if (s * kGroup >= nf) break;  // the last features' workgroups
-      if constexpr (kSub > 1) {
-        asm volatile("" ::: "memory");  // not kept in registers for all groups
-        take_features(s);
-      }
-      int at[kGroup];
-      if (held) {
+      for (int i = 0; i < kAll; i++) at[i] = s_start[i * a.cells + cell_of(x[i], lo[i], scale[i], a.cells)];
+      for (int p = most_probes - 1; p >= 0; p--) {
 #pragma unroll
-        for (int i = 0; i < kGroup; i++)
-          at[i] = s_start[(s * kGroup + i) * a.cells + cell_of(x[s * kGroup + i], lo[i], scale[i], a.cells)];
-        for (int p = most_probes - 1; p >= 0; p--) {
-#pragma unroll
-          for (int i = 0; i < kGroup; i++) {
-            const int step = p < probes[i] ? 1 << p : 0;  // a feature with fewer probes waits
-            const T v      = s_tab[place[i] + max(step - 1, 0) + at[i]];
-            at[i] += v < x[s * kGroup + i] ? step : 0;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < kGroup; i++) {
-          const int f = s * kGroup + i;
-          at[i]       = lower_bound(sorted + first + s_place[f], s_count[f], x[f]);
+        for (int i = 0; i < kAll; i++) {
+          if (p >= probes[i]) continue;  // (the same for the whole wave)
+          const T v = s_tab[place[i] + ((1 << p) - 1) + at[i]];
+          at[i] += v < x[i] ? 1 << p : 0;
         }
       }
+    } else {
 #pragma unroll
-      for (int i = 0; i < kGroup; i++) {
-        const int f         = s * kGroup + i;
-        const uint32_t code = x[f] == x[f] ? static_cast<uint32_t>(at[i]) + 1 : kNanRank;
-        if (f < nf)
-          *reinterpret_cast<uint16_t*>(base + (at0 + (static_cast<uint32_t>(2 * f) << a.tile_shift))) = static_cast<uint16_t>(code);
-      }
+      for (int i = 0; i < kAll; i++) at[i] = lower_bound(sorted + first + s_place[i], s_count[i], x[i]);
     }
+#pragma unroll
+    for (int i = 0; i < kAll; i++) {
+      const uint32_t code = x[i] == x[i] ? static_cast<uint32_t>(at[i]) + 1 : kNanRank;
+      if (i < nf)
+        *reinterpret_cast<uint16_t*>(base + (at0 + (static_cast<uint32_t>(2 * i) << a.tile_shift))) = static_cast<uint16_t>(code);
+    }
+  }
+}
+
+// The same for the features of one 128-byte line of a row, where their tables leave two such workgroups to a CU. Eight lanes take a row's
+// line, 16 bytes each: a wave's load so touches eight whole lines (a row a lane touched 64, once for each of its eight loads of 16
+// bytes: without any search 500,003 x 200 took 186 of 202 us that way). The values are turned in the LDS, and then a lane has a row and a
+// wave four or eight features, whose search it keeps in scalar registers; the rows of one feature share many of its LDS reads.
+// What bounds it is the memory: 500,003 x 200 (0.6 GB) 158 us.
+constexpr int kLineRows = 256;  // rows of a turn
+template <typename T>
+constexpr int kLineFeatures = 128 / sizeof(T);
+template <typename T>
+constexpr int kLinePitch = kLineRows + (sizeof(T) == 4 ? 2 : 4);  // the eight lanes of a row, eight rows: 64 banks
+template <typename T>
+constexpr int kLineStage = kLineFeatures<T> * kLinePitch<T> * static_cast<int>(sizeof(T));
+template <typename T>
+__global__ void __launch_bounds__(kWalkThreads, 8)
+  rank_lines_kernel(const T* __restrict__ X, RankRows a, RankState st, const T* __restrict__ sorted, uint16_t* __restrict__ ranks)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  constexpr int kAll = kLineFeatures<T>, kPer = 16 / sizeof(T), kPitch = kLinePitch<T>;
+  __shared__ int s_most[kAll], s_place[kAll], s_count[kAll];
+  __shared__ T s_lo[kAll], s_scale[kAll];
+  if (*st.overflow != 0) return;
+  const int tid = threadIdx.x, local = blockIdx.x / 8, g = local % a.n_groups;
+  const int64_t split = blockIdx.x % 8 + 8 * static_cast<int64_t>(local / a.n_groups);
+  const int f0 = g * kAll, nf = min(kAll, a.F - f0);
+  const int first = st.offset[f0], words = st.offset[f0 + nf] - first;
+  if (words == 0) {
+    bool asked = false;
+    for (int i = 0; i < nf; i++) asked |= st.count[a.F + f0 + i] != 0;
+    if (!asked) return;  // no tree asks for these features
+  }
+  // a lane's piece of its rows
+  const int q = tid & 7, r = tid >> 3, fq = f0 + kPer * q;  // rows r and r + 128
+  const int64_t begin = split * a.rows_per_split, end = min<int64_t>(a.n_rows, begin + a.rows_per_split);
+  typedef T Vec __attribute__((ext_vector_type(kPer)));
+  auto load = [&](int64_t row, T (&x)[kPer]) {
+    const T* src = X + min(row, end - 1) * a.F;
+    if (a.wide) {
+      // rows of whole 16-byte words: a word lies inside the features or past them
+      const Vec v = *reinterpret_cast<const Vec*>(src + (fq < a.F ? fq : f0));
+#pragma unroll
+      for (int j = 0; j < kPer; j++) x[j] = v[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < kPer; j++) x[j] = src[min(fq + j, a.F - 1)];
+    }
+  };
+  T x0[kPer], x1[kPer];
+  if (begin < end) {
+    load(begin + r, x0);
+    load(begin + r + kLineRows / 2, x1);
+  }
+  T* const s_x      = reinterpret_cast<T*>(smem_raw);  // [kAll][kPitch]
+  T* const s_tab    = reinterpret_cast<T*>(smem_raw + kLineStage<T>);
+  uint16_t* s_start = reinterpret_cast<uint16_t*>(smem_raw + kLineStage<T> + a.lds_bytes - 2 * kAll * a.cells);  // [kAll][cells]
+  const bool held   = (words + 1) * static_cast<int>(sizeof(T)) + 2 * kAll * a.cells <= a.lds_bytes;
+  if (tid < kAll) {
+    const int at = st.offset[f0 + min(tid, nf)];
+    s_most[tid]  = 0;
+    s_place[tid] = at - first;
+    s_count[tid] = tid < nf ? st.offset[f0 + tid + 1] - at : 0;
+  }
+  if (held) {
+    for (int e = tid; e < words; e += kWalkThreads) s_tab[e] = sorted[first + e];
+    if (tid == 0) s_tab[words] = T(0);  // read, not used, by features without thresholds
+    for (int c = tid; c < kAll * a.cells; c += kWalkThreads) s_start[c] = 0;
+  }
+  __syncthreads();
+  if (held) rank_cells<T, kAll>(a.cells, s_tab, s_start, s_place, s_count, s_most, s_lo, s_scale);
+  __syncthreads();
+  // a wave's features of 64 rows
+  constexpr int kOwn = kAll / 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), own = wave % 4 * kOwn, row_of = wave / 4 * 64 + (tid & 63);
+  int place[kOwn], probes[kOwn], most_probes = 0;
+  T lo[kOwn], scale[kOwn];
+  auto uniform = [](T v) {
+    uint32_t w[sizeof(T) / 4];
+    __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+    for (uint32_t& u : w) u = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(u)));
+    __builtin_memcpy(&v, w, sizeof(T));
+    return v;
+  };
+#pragma unroll
+  for (int j = 0; j < kOwn; j++) {
+    place[j]    = __builtin_amdgcn_readfirstlane(s_place[own + j]);
+    probes[j]   = __builtin_amdgcn_readfirstlane(s_most[own + j]);
+    lo[j]       = uniform(s_lo[own + j]);
+    scale[j]    = uniform(s_scale[own + j]);
+    most_probes = max(most_probes, probes[j]);
+  }
+  const uint16_t* const start = s_start + own * a.cells;
+  for (int64_t row0 = begin; row0 < end; row0 += kLineRows) {
+#pragma unroll
+    for (int j = 0; j < kPer; j++) {
+      s_x[(kPer * q + j) * kPitch + r]                 = x0[j];
+      s_x[(kPer * q + j) * kPitch + r + kLineRows / 2] = x1[j];
+    }
+    if (row0 + kLineRows < end) {
+      load(row0 + kLineRows + r, x0);
+      load(row0 + kLineRows + r + kLineRows / 2, x1);
+    }
+    __syncthreads();
+    T x[kOwn];
+    int at[kOwn];
+#pragma unroll
+    for (int j = 0; j < kOwn; j++) x[j] = s_x[(own + j) * kPitch + row_of];
+    if (held) {
+#pragma unroll
+      for (int j = 0; j < kOwn; j++) at[j] = start[j * a.cells + cell_of(x[j], lo[j], scale[j], a.cells)];
+      for (int p = most_probes - 1; p >= 0; p--) {
+#pragma unroll
+        for (int j = 0; j < kOwn; j++) {
+          if (p >= probes[j]) continue;  // (the same for the whole wave)
+          const T v = s_tab[place[j] + ((1 << p) - 1) + at[j]];
+          at[j] += v < x[j] ? 1 << p : 0;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < kOwn; j++) at[j] = lower_bound(sorted + first + place[j], s_count[own + j], x[j]);
+    }
+    const int64_t block = row0 + wave / 4 * 64;  // (a split ends with a block, or with the last row)
+    if (block < end) {
+      uint32_t code[kOwn];
+#pragma unroll
+      for (int j = 0; j < kOwn; j++) code[j] = x[j] == x[j] ? static_cast<uint32_t>(at[j]) + 1 : kNanRank;
+      // tile rows are a power of two, 64 or more; a tile's ranks lie within 32 bits of bytes
+      const int64_t tile = block >> a.tile_shift;
+      char* const base   = reinterpret_cast<char*>(ranks + (tile * a.F + f0 + own) * (int64_t(1) << a.tile_shift));
+      store_ranks(code, nf - own, a.tile_shift, base + 2 * (static_cast<int>(block) & ((1 << a.tile_shift) - 1)));
+    }
+    __syncthreads();
   }
 }
 
@@ -830,7 +961,7 @@ Plan make_plan(int64_t N, int F, int n_trees, const int32_t* tree_nodes, int K, 
     return (group * mean + 4.0 * std::sqrt(group * mean) + group) * static_cast<double>(value_size) + 2.0 * group * p.cells;
   };
   // the features of a 128-byte line if two such workgroups share a CU; else at most eight, in powers of two
-  const int line = static_cast<int>(128 / value_size);
+  const int line = static_cast<int>(128 / value_size), stage = value_size == 4 ? kLineStage<float> : kLineStage<double>;
   if (F > kGroupMax && 2 * bytes_for(line) <= static_cast<double>(kLds / 2 - 1024)) {
     p.group = line;
   } else {
@@ -840,7 +971,7 @@ Plan make_plan(int64_t N, int F, int n_trees, const int32_t* tree_nodes, int K, 
   // what all thresholds on these features would take, or room for twice the mean
   const double all_here = (static_cast<double>(thresholds) + 1) * static_cast<double>(value_size) + 2.0 * p.group * p.cells;
   const double room     = std::min(all_here, std::max(2.0 * bytes_for(p.group), 32.0 * 1024)) + 15;
-  p.rank_lds = static_cast<int>(std::min(room, static_cast<double>(kLds - 1024))) / 16 * 16;
+  p.rank_lds = static_cast<int>(std::min(room, static_cast<double>(p.group == line ? kLds / 2 - 1024 - stage : kLds - 1024))) / 16 * 16;
   const int64_t tiles = (N + s.tile_rows - 1) / s.tile_rows;
   const int64_t most  = std::max<int64_t>(256, static_cast<int64_t>(kRankedChunkBytes / (static_cast<size_t>(s.tile_rows) * F * 2)) / 256 * 256);
   p.chunk_rows = std::min(tiles, most) * s.tile_rows;
@@ -933,25 +1064,34 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
   rank_thresholds_kernel<T><<<dim3(F, p.thresholds > kSortMost<T> ? kRankBlocks : 1), kSortThreads,
                               sort_size * (sizeof(T) + sizeof(uint32_t)), stream>>>(st, static_cast<int>(sort_size), lay.grouped, lay.sorted);
 
-  static std::atomic<bool> rank_attr[6][kMaxDevices] = {};
+  static std::atomic<bool> rank_attr[5][kMaxDevices] = {};
   static std::atomic<bool> walk_attr[4][4][kMaxDevices] = {};
   auto whole_words = [&](const T* x) { return (static_cast<size_t>(F) * sizeof(T)) % 16 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0; };
-  auto rank_chunk = [&](auto group_c, auto sub_c, std::atomic<bool> (&flags)[kMaxDevices], const T* x, int64_t rows) -> int {
-    constexpr int kG = decltype(group_c)::value, kS = decltype(sub_c)::value;
-    LBT_TRY((allow_dynamic_lds(rank_rows_kernel<T, kG, kS>, kLds - 1024, flags)));
+  auto rank_chunk = [&](auto group_c, std::atomic<bool> (&flags)[kMaxDevices], const T* x, int64_t rows) -> int {
+    constexpr int kG     = decltype(group_c)::value;
+    constexpr bool kLine = kG > kGroupMax;
+    if constexpr (kLine)
+      LBT_TRY((allow_dynamic_lds(rank_lines_kernel<T>, kLds - 1024, flags)));
+    else
+      LBT_TRY((allow_dynamic_lds(rank_rows_kernel<T, kG>, kLds - 1024, flags)));
     RankRows a{};
     a.n_rows    = rows;
     a.F         = F;
-    a.n_groups  = ceil_div(F, kG * kS);
+    a.n_groups  = ceil_div(F, kG);
     a.tile_shift = 31 - __builtin_clz(static_cast<unsigned>(p.shape.tile_rows));
     a.cells     = p.cells;
     a.lds_bytes = p.rank_lds;
     // row ranges in multiples of the XCDs, as many as run at once
-    const int per_cu     = kLds / 2 >= static_cast<size_t>(p.rank_lds) + 1024 ? 2 : 1;
+    const size_t lds     = p.rank_lds + (kLine ? kLineStage<T> : 0);
+    const int per_cu     = kLds / 2 >= lds + 1024 ? 2 : 1;
     const int64_t splits = 8 * std::max<int64_t>(1, std::min<int64_t>(32 * per_cu / a.n_groups, ceil_div(rows, 8 * kWalkThreads)));
     a.rows_per_split     = (rows + splits * kWalkThreads - 1) / (splits * kWalkThreads) * kWalkThreads;
     a.wide = whole_words(x) && kG * sizeof(T) >= 16;
-    rank_rows_kernel<T, kG, kS><<<static_cast<unsigned>(splits * a.n_groups), kWalkThreads, p.rank_lds, stream>>>(x, a, st, lay.sorted, lay.ranks);
+    const unsigned grid = static_cast<unsigned>(splits * a.n_groups);
+    if constexpr (kLine)
+      rank_lines_kernel<T><<<grid, kWalkThreads, lds, stream>>>(x, a, st, lay.sorted, lay.ranks);
+    else
+      rank_rows_kernel<T, kG><<<grid, kWalkThreads, lds, stream>>>(x, a, st, lay.sorted, lay.ranks);
     return LBT_OK;
   };
   auto walk_chunk = [&](auto adds_c, auto items_c, auto j_c, std::atomic<bool> (&flags)[kMaxDevices], int64_t rows, double* o) -> int {
@@ -979,16 +1119,11 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
     double* o  = out + row * K;
     const integral_constant<int, 1> one{};
     switch (p.group) {
-      case 1: LBT_TRY(rank_chunk(one, one, rank_attr[0], x, rows)); break;
-      case 2: LBT_TRY(rank_chunk(integral_constant<int, 2>{}, one, rank_attr[1], x, rows)); break;
-      case 4: LBT_TRY(rank_chunk(integral_constant<int, 4>{}, one, rank_attr[2], x, rows)); break;
-      case 8: LBT_TRY(rank_chunk(integral_constant<int, 8>{}, one, rank_attr[3], x, rows)); break;
-      default:
-        if (sizeof(T) == 4 && whole_words(x))
-          LBT_TRY(rank_chunk(integral_constant<int, 4>{}, integral_constant<int, 32 / sizeof(T)>{}, rank_attr[4], x, rows));
-        else
-          LBT_TRY(rank_chunk(integral_constant<int, 8>{}, integral_constant<int, 16 / sizeof(T)>{}, rank_attr[5], x, rows));
-        break;
+      case 1: LBT_TRY(rank_chunk(one, rank_attr[0], x, rows)); break;
+      case 2: LBT_TRY(rank_chunk(integral_constant<int, 2>{}, rank_attr[1], x, rows)); break;
+      case 4: LBT_TRY(rank_chunk(integral_constant<int, 4>{}, rank_attr[2], x, rows)); break;
+      case 8: LBT_TRY(rank_chunk(integral_constant<int, 8>{}, rank_attr[3], x, rows)); break;
+      default: LBT_TRY(rank_chunk(integral_constant<int, kLineFeatures<T>>{}, rank_attr[4], x, rows)); break;
     }
     auto with = [&](auto adds_c, auto items_c, int at) -> int {
       switch (p.shape.j) {
