@@ -536,7 +536,7 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     for (int u = 0; u < kE / 4; u++)
       if (a.depth > 0 && 4 * (tid + u * kT) < a.N) code[u] = *reinterpret_cast<const uint32_t*>(st.code + 4 * (tid + u * kT));
   }
-  if (kStaged && !kDecides && usable)
+  if (kStaged && kSingle && !kDecides && usable)
     for (int j = tid; j < a.n_nodes; j += kT) {
       const I64Pair ns = st.node_sums[a.level_first + j];
       s_base[j]        = st.base[a.level_first + j];
@@ -742,7 +742,7 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     // node[] already is the node of this level at the place: both children of a parent lie where the
     // parent's rows lay, the left one first
     int2 seg[kE];  // the left child's
-    const bool from_lds = kStaged && usable;
+    const bool from_lds = kStaged && kSingle && usable;
     if (!from_lds) {
 #pragma unroll
       for (int e = 0; e < kE; e++) seg[e] = node[e] != kNone ? st.seg[a.level_first + (node[e] & ~1)] : make_int2(-1, 0);
@@ -966,16 +966,46 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     unsigned dead = 0;
 #pragma unroll
     for (int e = 0; e < kE; e++) gain[e] = 0.0;
+    // The pairs of the next output, and what the nodes have of it, are on their way while this one's sums and gains are formed, and lie in the
+    // LDS when they are asked for: gathered from the L2 place by place, with the nodes' sums behind the places' sums, they were two latencies
+    // an output: 590 x 118 with 8 outputs, depth 9, 24.7 us a launch, now 20.5; 7000 x 300 with 2, depth 8, 96 and 83. kStaged: the nodes' sums, bases and terms of the gain, a thread each, those of one
+    // output beside those of the next.
+    I64Pair* const s_of_k    = reinterpret_cast<I64Pair*>(smem_raw + small_scan_use(a.N, a.n_nodes));  // [2][2][n_nodes]
+    double* const s_parent_k = reinterpret_cast<double*>(s_of_k + 4 * a.n_nodes);                      // [2][n_nodes]
+    const int64_t own_at     = static_cast<int64_t>(a.level_first + min(tid, a.n_nodes - 1)) * a.K;
+    int2 q_next[kE];
+    I64Pair ns_next{0, 0}, base_next{0, 0};
+    auto fetch = [&](int k) {
+#pragma unroll
+      for (int u = 0; u < kE; u++) q_next[u] = st.qgh[min(tid + u * kT, a.N - 1) * a.K + k];
+      if constexpr (kStaged) {
+        ns_next   = st.node_sums[own_at + k];
+        base_next = st.base[own_at + k];
+      }
+    };
+    fetch(0);
     for (int k = 0; k < a.K; k++) {
+      I64Pair* const ns_of = s_of_k + 2 * (k & 1) * a.n_nodes;
+      I64Pair* const base_of = ns_of + a.n_nodes;
+      double* const parent_of_k = s_parent_k + (k & 1) * a.n_nodes;
+      // (nobody looks at the pairs of the output before any more: a barrier lies behind those looks)
+#pragma unroll
+      for (int u = 0; u < kE; u++)
+        if (tid + u * kT < a.N) s_q[tid + u * kT] = q_next[u];
+      if constexpr (kStaged) {
+        if (tid < a.n_nodes) {
+          ns_of[tid]       = ns_next;
+          base_of[tid]     = base_next;
+          parent_of_k[tid] = leaf_gain(static_cast<double>(ns_next.grad) * inv_g, static_cast<double>(ns_next.hess) * inv_h, a.l1, reg);
+        }
+      }
+      if (k + 1 < a.K) fetch(k + 1);
+      __syncthreads();
       int2 q[kE];
       I64Pair sum{0, 0};
 #pragma unroll
       for (int e = 0; e < kE; e++) {
-        q[e] = make_int2(0, 0);
-        if (i0 + e < a.N) {
-          const int r = static_cast<int>(entry[e] & 0xffff);
-          q[e]        = st.qgh[r * a.K + k];
-        }
+        q[e] = i0 + e < a.N ? s_q[entry[e] & 0xffff] : make_int2(0, 0);
         sum.grad += q[e].x;
         sum.hess += q[e].y;
       }
@@ -988,20 +1018,40 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
         before.grad += w < wave ? s_tot[w].grad : 0;
         before.hess += w < wave ? s_tot[w].hess : 0;
       }
+      auto offer = [&](int e, int j) {
+        I64Pair ns, base;
+        double parent;
+        if constexpr (kStaged) {
+          ns     = ns_of[j];
+          base   = base_of[j];
+          parent = parent_of_k[j];
+        } else {
+          const int64_t at = static_cast<int64_t>(a.level_first + j) * a.K + k;
+          ns     = st.node_sums[at];
+          base   = st.base[at];
+          parent = leaf_gain_select(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, a.l1, reg);
+        }
+        const I64Pair ls{before.grad - base.grad, before.hess - base.hess}, rs{ns.grad - ls.grad, ns.hess - ls.hess};
+        // build_tree.cu:727-730: one output without a valid split on this bin voids the bin
+        dead |= ls.hess <= 0 || rs.hess <= 0 ? 1u << e : 0u;
+        gain[e] += (0.5 * (leaf_gain_select(static_cast<double>(ls.grad) * inv_g, static_cast<double>(ls.hess) * inv_h, a.l1, reg) +
+                           leaf_gain_select(static_cast<double>(rs.grad) * inv_g, static_cast<double>(rs.hess) * inv_h, a.l1, reg) -
+                           parent)) -
+                   a.min_split_gain;
+      };
+      // a few waves: the places' quotients side by side, without branches (a place whose bin does not end there has no say below);
+      // sixteen of them hide each other's chains, and only the places that have a say are worth the time
 #pragma unroll
       for (int e = 0; e < kE; e++) {
         before.grad += q[e].x;
         before.hess += q[e].y;
-        if ((ends >> e) & 1u) {
-          const int64_t at = static_cast<int64_t>(a.level_first + node[e]) * a.K + k;
-          const I64Pair ns = st.node_sums[at], base = st.base[at];
-          const I64Pair ls{before.grad - base.grad, before.hess - base.hess};
-          bool d = (dead >> e) & 1u;
-          add_gain(gain[e], d, ls, ns, inv_g, inv_h, a.l1, reg, a.min_split_gain);
-          dead |= d ? 1u << e : 0u;
-        }
+        if constexpr (kT < 1024)
+          offer(e, node[e] != kNone ? node[e] : 0);
+        else if (((ends & ~dead) >> e) & 1u)
+          offer(e, node[e]);
       }
     }
+    ends &= ~dead;
     // best gain per node: a thread's runs of one node first, then, where a whole wave lies in one
     // node, the wave
     {
@@ -1227,7 +1277,15 @@ int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelA
       return launch_small_scan_as<kDT, kDE, true, kDE, true, true>(stream, st, b, all + (b.all_bins ? bins : 0));
     }
   }
-  if (a.K > 1) return launch_small_scan_as<kT, kE, false, 1, false, false>(stream, st, a, lds);
+  if (a.K > 1) {
+    const size_t both = lds + static_cast<size_t>(a.n_nodes) * 2 * (2 * sizeof(I64Pair) + sizeof(double));
+    // two outputs' nodes; no workgroup of the CU is given up for them (of 1024 threads with these registers there is one) where there are
+    // more workgroups than CUs
+    auto at_once = [](size_t bytes) { return std::min<size_t>(1024 / kT, 160 * 1024 / (bytes + 1024)); };
+    if (a.n_nodes <= kT && both <= kScanLds && (a.F <= 256 || at_once(both) >= at_once(lds)))
+      return launch_small_scan_as<kT, kE, false, 1, true, false>(stream, st, a, both);
+    return launch_small_scan_as<kT, kE, false, 1, false, false>(stream, st, a, lds);
+  }
   // staging must not cost a workgroup of the CU where there are more of them than CUs
   auto per_cu        = [](size_t bytes) { return static_cast<int>(std::min<size_t>(2048 / kT, 160 * 1024 / (bytes + 1024))); };
   const bool crowded = kT == 1024 && a.F > 256;
