@@ -5,7 +5,7 @@ UPDATE_TREE) this class calls the matching C-ABI entry point of liblbtree.so
 with the same scalars in the same order. Arrays are CUDA tensors."""
 import copy
 import warnings
-from typing import Any, Callable, List, Sequence, Union, cast
+from typing import Any, Callable, Sequence, Union, cast
 
 import numpy as np
 import torch
@@ -149,17 +149,13 @@ class Tree(BaseModel):
 
     @staticmethod
     def batch_predict(models: Sequence[BaseModel], X):
-        assert all(isinstance(m, Tree) for m in models)
-        models = cast(List[Tree], models)
-        n_outputs = models[0].leaf_value.shape[1]
-        return ops.predict(X, [(m.leaf_value, m.feature, m.split_value) for m in models], n_outputs)
+        n_outputs = cast(Tree, models[0]).leaf_value.shape[1]
+        return ops.predict_models(X, models, Tree, n_outputs)
 
     @staticmethod
     def batch_predict_from(init, models: Sequence[BaseModel], X):
         """init + batch_predict(models, X) without a pass of its own; init: a contiguous CUDA float64 tensor of the outputs."""
-        assert all(isinstance(m, Tree) for m in models)
-        models = cast(List[Tree], models)
-        return ops.predict(X, [(m.leaf_value, m.feature, m.split_value) for m in models], init.numel(), init=init)
+        return ops.predict_models(X, models, Tree, init.numel(), init=init)
 
     def __str__(self) -> str:
         leaf_value = self.leaf_value.cpu().numpy()

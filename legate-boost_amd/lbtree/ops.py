@@ -188,12 +188,16 @@ def build_tree(X, g, h, *, max_depth, split_samples, seed, l1_regularization=0.0
     return r
 
 
+def _all_nodes(nodes):
+    return int(np.frombuffer(nodes, np.int32).sum(dtype=np.int64))
+
+
 def _tree_arrays(trees, n_outputs):
     """Host arrays of an ensemble's (leaf_value, feature, split_value): addresses of the three, nodes of every tree, all nodes,
     and what keeps the addresses valid."""
     plain = _lib._host.tree_arrays(trees, n_outputs) if _lib._host is not None else None
     if plain is not None:
-        return plain + (int(np.frombuffer(plain[3], np.int32).sum(dtype=np.int64)), trees)
+        return plain + (_all_nodes(plain[3]), trees)
     nt = len(trees)
     leaf_p = (C.c_void_p * max(nt, 1))()
     feat_p = (C.c_void_p * max(nt, 1))()
@@ -209,6 +213,12 @@ def _tree_arrays(trees, n_outputs):
         keep.append((lv, ft, sp))
         leaf_p[i], feat_p[i], split_p[i], nodes[i] = lv.data_ptr(), ft.data_ptr(), sp.data_ptr(), ft.shape[0]
     return leaf_p, feat_p, split_p, nodes, sum(int(nodes[i]) for i in range(nt)), keep
+
+
+# the whole call in native code where it is built and torch hands out a stream's address (a call takes the host 5.3 us; through Python 7.1, more than the kernel of a
+# few hundred rows)
+_predict_packed = _lib._host.predict_packed if _lib._host is not None and _raw_stream is not None else None
+_PREDICT_PACKED = C.cast(_lib.lib.lbt_predict_packed, C.c_void_p).value
 
 
 class PackedEnsemble:
@@ -230,6 +240,13 @@ class PackedEnsemble:
         _lib.check(rc)
 
     def predict(self, X):
+        if _predict_packed is not None and torch.cuda.is_initialized():
+            out = _predict_packed(X, _PREDICT_PACKED, _raw_stream(torch.cuda.current_device()), C.addressof(self.desc), _DT[self.dtype],
+                                  self.n_outputs)
+            if isinstance(out, torch.Tensor):
+                return out
+            if out is not None:
+                _lib.check(out)
         X = _check_x(X)
         n, f = X.shape
         out = torch.empty((n, self.n_outputs), dtype=torch.float64, device=X.device)
@@ -243,11 +260,25 @@ def predict(X, trees, n_outputs, tiled=True, init=None):
     """PREDICT (legateboost/models/tree.py:245-280). trees: sequence of
     (leaf_value [nodes,K] f64, feature [nodes] i32, split_value [nodes] f64) CUDA tensors.
     init: what the sums are added to, a contiguous CUDA float64 tensor of n_outputs values (none: zeros)."""
-    X = _check_x(X)
+    return _predict(_check_x(X), len(trees), _tree_arrays(trees, n_outputs), n_outputs, tiled, init)
+
+
+_ARRAYS = ("leaf_value", "feature", "split_value")
+
+
+def predict_models(X, models, kind, n_outputs, init=None):
+    """predict on the arrays of `models`, objects of class `kind` that have them as attributes."""
+    arrays = _lib._host.model_arrays(models, kind, _ARRAYS, n_outputs) if _lib._host is not None else None
+    if arrays is None:
+        assert all(isinstance(m, kind) for m in models)
+        return predict(X, [(m.leaf_value, m.feature, m.split_value) for m in models], n_outputs, init=init)
+    return _predict(_check_x(X), len(models), arrays[:4] + (None, arrays[4]), n_outputs, True, init)
+
+
+def _predict(X, nt, arrays, n_outputs, tiled, init):
     n, f = X.shape
-    nt = len(trees)
     out = torch.empty((n, n_outputs), dtype=torch.float64, device=X.device)
-    leaf_p, feat_p, split_p, nodes, total, keep = _tree_arrays(trees, n_outputs)
+    leaf_p, feat_p, split_p, nodes, total, keep = arrays
     ws = None
     if tiled:
         nbytes = int(_lib.lib.lbt_predict_rows_workspace_bytes(n, f, nt, nodes, n_outputs, _DT[X.dtype]))
@@ -255,6 +286,7 @@ def predict(X, trees, n_outputs, tiled=True, init=None):
             ws = torch.empty(nbytes, dtype=torch.uint8, device=X.device)
         except torch.OutOfMemoryError:
             # the room for the rows' ranks is not needed, only faster
+            total = total if total is not None else _all_nodes(nodes)
             least = int(_lib.lib.lbt_predict_workspace_bytes(nt, total, n_outputs, _DT[X.dtype]))
             if least >= nbytes:
                 raise

@@ -72,3 +72,62 @@ def test_plain_arrays_and_those_that_are_not():
     for bad in ((leaf[:6], feat, split), (leaf[:, :1], feat, split)):
         with pytest.raises(_lib.LbtError):
             ops.predict(X, [bad], 2)
+
+
+def test_models_that_are_no_trees_are_left_to_the_caller():
+    take = _lib._host.model_arrays
+    names = ("a", "b", "c")
+
+    class Model:
+        a, b, c = torch.zeros(7, 1, dtype=torch.float64), torch.zeros(7, dtype=torch.int32), torch.zeros(7, dtype=torch.float64)
+
+    class Bare:
+        a = 1
+
+    assert take([], Model, names, 1) == (b"", b"", b"", b"", [])
+    for models in ([Model()], [Bare()], [None], iter([])):  # arrays of the CPU, others, none
+        assert take(models, Model, names, 1) is None
+    assert take([Bare()], Bare, names, 1) is None
+    assert take([], Model, names, 0) is None and take([], 1, names, 1) is None and take([], Model, names[:2], 1) is None
+    assert _lib._host.predict_packed(np.zeros((2, 2)), 0, 0, 0, 0, 1) is None
+    assert _lib._host.predict_packed(torch.zeros(2, 2), 0, 0, 0, 0, 1) is None
+    with pytest.raises(TypeError):
+        _lib._host.predict_packed(torch.zeros(2, 2), 0, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("k", [1, 3])
+def test_a_packed_prediction_in_native_code_and_through_python(monkeypatch, dtype, k):
+    rs = np.random.RandomState(k)
+    trees = [(torch.from_numpy(rs.randn(15, k)).cuda(), torch.from_numpy(np.r_[rs.randint(0, 5, 7), -np.ones(8)].astype(np.int32)).cuda(),
+              torch.from_numpy(rs.rand(15)).cuda()) for _ in range(20)]
+    packed = ops.PackedEnsemble(trees, k, 5, dtype)
+    wide = torch.rand(300, 10, dtype=dtype).cuda()
+    good = [wide[:, :5].contiguous(), wide[:, :5], wide[:, ::2], wide[:5].t(), wide[:0, :5], wide[:1, :5].clone().requires_grad_(),
+            wide[:, :5].cpu(), wide[7:9, :5].cpu().numpy()]
+    bad = [wide, wide[0, :5], wide[:, :5].to(torch.float32 if dtype == torch.float64 else torch.float64), wide[:, :5].long()]
+    got = [packed.predict(X) for X in good]
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        aside = packed.predict(good[0])
+    stream.synchronize()
+    refused = []
+    for X in bad:
+        with pytest.raises(_lib.LbtError) as e:
+            packed.predict(X)
+        refused.append(str(e.value))
+    with pytest.raises(Exception):
+        torch.func.vmap(packed.predict)(wide[:4, :5].reshape(2, 2, 5))
+    monkeypatch.setattr(ops, "_predict_packed", None)
+    for X, out in zip(good, got):
+        want = packed.predict(X)
+        assert torch.equal(out, want) and out.dtype == want.dtype and out.device == want.device and not out.requires_grad
+    assert torch.equal(aside, got[0])
+    for X, told in zip(bad, refused):
+        with pytest.raises(_lib.LbtError) as e:
+            packed.predict(X)
+        assert str(e.value) == told
+    with pytest.raises(Exception):
+        torch.func.vmap(packed.predict)(wide[:4, :5].reshape(2, 2, 5))
