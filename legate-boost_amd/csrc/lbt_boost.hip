@@ -34,12 +34,12 @@ __global__ void __launch_bounds__(kBoostThreads)
 }
 
 // One row per thread: softmax over the row's K outputs, then the class gradient.
-// kCols > 0 keeps the row in registers; 0 recomputes the exponentials instead.
+// kCols > 0 keeps the row in registers; 0 recomputes the exponentials instead. See softmax_by_entry.
 template <int kCols>
 __global__ void __launch_bounds__(kBoostThreads)
-  gradient_softmax_kernel(const double* __restrict__ pred, const double* __restrict__ y,
-                          const double* __restrict__ weight, double lr, int64_t n_rows, int K,
-                          double* __restrict__ g, double* __restrict__ h)
+  gradient_softmax_rows_kernel(const double* __restrict__ pred, const double* __restrict__ y,
+                               const double* __restrict__ weight, double lr, int64_t n_rows, int K,
+                               double* __restrict__ g, double* __restrict__ h)
 {
   const int64_t r = blockIdx.x * static_cast<int64_t>(kBoostThreads) + threadIdx.x;
   if (r >= n_rows) return;
@@ -137,18 +137,123 @@ __global__ void __launch_bounds__(kBoostThreads)
   store_chunk_sums(xa, xb, sa, sb, sum_g, sum_h);
 }
 
-// Softmax: a workgroup computes the rows that meet its chunk of entries (a row that straddles
+// Softmax of rows of up to kSoftmaxCols outputs: a thread has entries, and only the row's maximum and the sum of its exponentials are a
+// row's work, which a thread each does from the LDS, in the order of the outputs. Bound by memory: pred is read and g and h are written in whole
+// lines (a thread with a row of 8 outputs met 64 lines with each load and store), and with kSums the pass that sums |g| and |h| is
+// none of its own. A stage is kSumStage entries: with kSums lane t's entries t + 256 j of a chunk's first stage are its j = 0 .. 7, those of the
+// second its j = 8 .. 15; without it a workgroup has one stage. Rows that straddle two stages have their other outputs read, and their
+// exponentials formed, for each of them.
+constexpr int kSumStage    = 2048;
+constexpr int kSoftmaxCols = 128;
+constexpr int kStageTurns  = kSumStage / kBoostThreads;
+// a place behind every row of a multiple of four outputs: a thread with a row meets other banks than its neighbours
+constexpr int kStagePlaces = kSumStage * 5 / 4 + 3 * kSoftmaxCols;
+constexpr int kStageRows   = kSumStage / 2 + 2;
+static_assert(2 * kSoftmaxCols <= kBoostThreads, "the outputs of straddling rows are one a thread");
+template <bool kSums>
+__global__ void __launch_bounds__(kBoostThreads)
+  gradient_softmax_kernel(const double* __restrict__ pred, const double* __restrict__ y, const double* __restrict__ weight, double lr,
+                          int64_t n_rows, int K, double* __restrict__ g, double* __restrict__ h, double* __restrict__ sum_g,
+                          double* __restrict__ sum_h)
+{
+  __shared__ double s_p[kStagePlaces];
+  __shared__ double s_row[kStageRows];
+  static_assert(kStagePlaces >= 2 * kBoostThreads, "the chunk's sums are formed in the same place");
+  const int tid       = static_cast<int>(threadIdx.x);
+  const int64_t n     = n_rows * K;
+  const unsigned inverse = ((1u << 20) + static_cast<unsigned>(K) - 1) / static_cast<unsigned>(K);  // i / K for i below a stage and two rows
+  const int pad       = K % 4 == 0 ? 1 : 0;
+  double xa = 0.0, xb = 0.0;
+  for (int stage = 0; stage < (kSums ? kSumChunk / kSumStage : 1); stage++) {
+    const int64_t e0 = (blockIdx.x * static_cast<int64_t>(kSums ? kSumChunk / kSumStage : 1) + stage) * kSumStage;
+    if (e0 >= n) break;
+    const int64_t r0 = e0 / K, f0 = r0 * K;
+    const int front = static_cast<int>(e0 - f0);                                   // outputs of the first row that lie before the stage
+    const int in    = static_cast<int>(n - e0 < kSumStage ? n - e0 : kSumStage);   // entries of the stage
+    const int rows  = static_cast<int>(static_cast<unsigned>(front + in + K - 1) * inverse >> 20);
+    const int back  = rows * K - front - in;                                       // of the last row behind it
+    double p[kStageTurns], w[kStageTurns];
+    int at[kStageTurns], row[kStageTurns];  // place in the LDS, row of the stage
+    unsigned hits = 0;                      // bit j: the entry is that of its row's label
+#pragma unroll
+    for (int j = 0; j < kStageTurns; j++) {
+      const int i = front + min(tid + kBoostThreads * j, in - 1);
+      p[j]        = pred[f0 + i];
+      row[j]      = static_cast<int>(static_cast<unsigned>(i) * inverse >> 20);
+      hits |= (static_cast<int>(y[r0 + row[j]]) == i - row[j] * K ? 1u : 0u) << j;
+      w[j]        = weight != nullptr ? weight[r0 + row[j]] : 1.0;
+      at[j]       = i + row[j] * pad;
+    }
+    const bool extra = tid < front + back;
+    const int xi     = extra ? (tid < front ? tid : tid + in) : 0;
+    const int xrow   = static_cast<int>(static_cast<unsigned>(xi) * inverse >> 20);
+    double xp        = pred[f0 + xi];
+    if (stage > 0) __syncthreads();  // the rows' sums before are still read
+#pragma unroll
+    for (int j = 0; j < kStageTurns; j++)
+      if (tid + kBoostThreads * j < in) s_p[at[j]] = p[j];
+    if (extra) s_p[xi + xrow * pad] = xp;
+    __syncthreads();
+    for (int r = tid; r < rows; r += kBoostThreads) {
+      const double* const of = s_p + r * (K + pad);
+      double top = of[0];
+      for (int k = 1; k < K; k++) top = fmax(top, of[k]);
+      s_row[r] = top;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kStageTurns; j++) {
+      p[j] = exp(p[j] - s_row[row[j]]);
+      if (tid + kBoostThreads * j < in) s_p[at[j]] = p[j];
+    }
+    if (extra) s_p[xi + xrow * pad] = exp(xp - s_row[xrow]);
+    __syncthreads();
+    for (int r = tid; r < rows; r += kBoostThreads) {
+      const double* const of = s_p + r * (K + pad);
+      double div = 0.0;
+      for (int k = 0; k < K; k++) div += of[k];
+      s_row[r] = div;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kStageTurns; j++) {
+      const int i = tid + kBoostThreads * j;
+      if (i < in) {
+        const double q = p[j] / s_row[row[j]];
+        double go, ho;
+        weigh((hits >> j & 1) != 0 ? q + -1.0 : q, q * (1.0 - q), w[j], lr, &go, &ho);
+        g[e0 + i] = go;
+        h[e0 + i] = ho;
+        xa += fabs(go);
+        xb += fabs(ho);
+      }
+    }
+  }
+  if constexpr (kSums) {
+    __syncthreads();
+    store_chunk_sums(xa, xb, s_p, s_p + kBoostThreads, sum_g, sum_h);
+  }
+}
+
+// us with a thread for an entry and one for a row: 16,000,000 entries in rows of 2 83 : 78, of 4 78 : 80, of 8 75 : 103, of 16 74 : 129;
+// 5,000,000 of 5 24.8 : 26.1, of 8 23 : 31; 1,280,000 of 5 10.6 : 8.9, of 8 10.0 : 10.6; 20,000 of 8 5.3 : 3.1. Rows that are not held in registers
+// never: 20,000 of 9 5.4 : 7.4, 16,000,000 75 : 598, of 20 75 : 1108, of 64 77 : 802.
+inline bool softmax_by_entry(int64_t n, int K)
+{
+  const bool in_registers = K <= 8 || K == 10 || K == 16;
+  return K <= kSoftmaxCols && (!in_registers || (K >= 5 && n >= 4000000));
+}
+
+// The same for rows of more outputs: a workgroup computes the rows that meet its chunk of entries (a row that straddles
 // two stages or chunks is computed for each of them, which stores the same values), keeps the
 // entries in the LDS and adds them up from there in the quantiser's order. The chunk is taken
 // in stages of 2048 entries: lane t's entries t + 256 j of the first stage are its j = 0 .. 7,
 // those of the second its j = 8 .. 15, so the order of its sum is the same.
-constexpr int kSumStage = 2048;
-template <int kCols>
 __global__ void __launch_bounds__(kBoostThreads)
-  gradient_softmax_sums_kernel(const double* __restrict__ pred, const double* __restrict__ y,
-                               const double* __restrict__ weight, double lr, int64_t n_rows, int K,
-                               double* __restrict__ g, double* __restrict__ h, double* __restrict__ sum_g,
-                               double* __restrict__ sum_h)
+  gradient_softmax_rows_sums_kernel(const double* __restrict__ pred, const double* __restrict__ y,
+                                    const double* __restrict__ weight, double lr, int64_t n_rows, int K,
+                                    double* __restrict__ g, double* __restrict__ h, double* __restrict__ sum_g,
+                                    double* __restrict__ sum_h)
 {
   __shared__ double s_g[kSumStage];
   __shared__ double s_h[kSumStage];
@@ -176,30 +281,12 @@ __global__ void __launch_bounds__(kBoostThreads)
             s_h[e - e0] = ho;
           }
         };
-        // the same arithmetic, in the same order, as gradient_softmax_kernel
-        if constexpr (kCols > 0) {
-          double ex[kCols > 0 ? kCols : 1];
-          double top = p[0];
-#pragma unroll
-          for (int k = 0; k < kCols; k++) {
-            ex[k] = p[k];
-            top   = fmax(top, ex[k]);
-          }
-          double div = 0.0;
-#pragma unroll
-          for (int k = 0; k < kCols; k++) {
-            ex[k] = exp(ex[k] - top);
-            div += ex[k];
-          }
-#pragma unroll
-          for (int k = 0; k < kCols; k++) emit(k, ex[k] / div);
-        } else {
-          double top = p[0];
-          for (int k = 1; k < K; k++) top = fmax(top, p[k]);
-          double div = 0.0;
-          for (int k = 0; k < K; k++) div += exp(p[k] - top);
-          for (int k = 0; k < K; k++) emit(k, exp(p[k] - top) / div);
-        }
+        // the same arithmetic, in the same order, as gradient_softmax_rows_kernel
+        double top = p[0];
+        for (int k = 1; k < K; k++) top = fmax(top, p[k]);
+        double div = 0.0;
+        for (int k = 0; k < K; k++) div += exp(p[k] - top);
+        for (int k = 0; k < K; k++) emit(k, exp(p[k] - top) / div);
       }
     }
     __syncthreads();
@@ -539,24 +626,12 @@ int lbt_weighted_gradient_sums(void* stream, int32_t objective, const double* pr
   else if (n_outputs == 1)
     lbt::gradient_elementwise_sums_kernel<true><<<grid, lbt::kBoostThreads, 0, s>>>(
       pred, y, sample_weight, learning_rate, n, 1, g, h, sum_g, sum_h);
-  else {
-#define LBT_SOFTMAX_SUMS(C)                                                                                  \
-  lbt::gradient_softmax_sums_kernel<C><<<grid, lbt::kBoostThreads, 0, s>>>(pred, y, sample_weight, learning_rate, \
-                                                                           n_rows, n_outputs, g, h, sum_g, sum_h)
-    switch (n_outputs) {
-      case 2: LBT_SOFTMAX_SUMS(2); break;
-      case 3: LBT_SOFTMAX_SUMS(3); break;
-      case 4: LBT_SOFTMAX_SUMS(4); break;
-      case 5: LBT_SOFTMAX_SUMS(5); break;
-      case 6: LBT_SOFTMAX_SUMS(6); break;
-      case 7: LBT_SOFTMAX_SUMS(7); break;
-      case 8: LBT_SOFTMAX_SUMS(8); break;
-      case 10: LBT_SOFTMAX_SUMS(10); break;
-      case 16: LBT_SOFTMAX_SUMS(16); break;
-      default: LBT_SOFTMAX_SUMS(0); break;
-    }
-#undef LBT_SOFTMAX_SUMS
-  }
+  else if (n_outputs <= lbt::kSoftmaxCols)
+    lbt::gradient_softmax_kernel<true><<<grid, lbt::kBoostThreads, 0, s>>>(pred, y, sample_weight, learning_rate, n_rows, n_outputs, g, h,
+                                                                           sum_g, sum_h);
+  else
+    lbt::gradient_softmax_rows_sums_kernel<<<grid, lbt::kBoostThreads, 0, s>>>(pred, y, sample_weight, learning_rate, n_rows, n_outputs, g,
+                                                                               h, sum_g, sum_h);
   LBT_HIP(hipGetLastError());
   return LBT_OK;
 }
@@ -580,12 +655,15 @@ int lbt_weighted_gradient(void* stream, int32_t objective, const double* pred, c
   } else if (n_outputs == 1) {
     lbt::gradient_elementwise_kernel<true><<<lbt::grid_for(n), lbt::kBoostThreads, 0, s>>>(
       pred, y, sample_weight, learning_rate, n, 1, g, h);
+  } else if (lbt::softmax_by_entry(n, n_outputs)) {
+    const unsigned grid = static_cast<unsigned>((n + lbt::kSumStage - 1) / lbt::kSumStage);
+    lbt::gradient_softmax_kernel<false><<<grid, lbt::kBoostThreads, 0, s>>>(pred, y, sample_weight, learning_rate, n_rows, n_outputs, g, h,
+                                                                            nullptr, nullptr);
   } else {
     const unsigned grid = lbt::grid_for(n_rows);
-#define LBT_SOFTMAX(C)                                                                            \
-  lbt::gradient_softmax_kernel<C><<<grid, lbt::kBoostThreads, 0, s>>>(pred, y, sample_weight,     \
-                                                                      learning_rate, n_rows,      \
-                                                                      n_outputs, g, h)
+#define LBT_SOFTMAX(C)                                                                                                      \
+  lbt::gradient_softmax_rows_kernel<C><<<grid, lbt::kBoostThreads, 0, s>>>(pred, y, sample_weight, learning_rate, n_rows, \
+                                                                           n_outputs, g, h)
     switch (n_outputs) {
       case 2: LBT_SOFTMAX(2); break;
       case 3: LBT_SOFTMAX(3); break;

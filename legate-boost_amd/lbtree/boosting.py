@@ -192,13 +192,15 @@ class LBBase:
         self.train_metric_ = []
         train_pred = self._predict(X)
         # The gradient pass can leave the quantiser's first sums where g and h reach the tree as it wrote them. It then has a
-        # workgroup per 4096 entries: below four million of them the pass over g and h that it saves costs less, and with the
-        # softmax of several outputs as much. Fits of 5 rounds of depth 6 with the sums and without, ms: 300,000 x 20 1.21 and
+        # workgroup per 4096 entries: below four million of them (several outputs: eight) the pass over g and h that it saves costs
+        # less. Fits of 5 rounds of depth 6 with the sums and without, ms: 300,000 x 20 1.21 and
         # 1.18, 1,000,000 x 50 2.14 and 2.10, 2,000,000 x 40 2.95 and 2.92, 4,000,000 x 30 3.71 and 3.72, 6,000,000 x 30 5.28 and
-        # 5.29 (two classes 5.37 and 5.40), 10,000,000 x 100 17.98 and 18.08.
+        # 5.29 (two classes 5.37 and 5.40), 10,000,000 x 100 17.98 and 18.08; three classes, 1,500,000 x 20 2.65 and 2.62,
+        # 2,000,000 x 30 4.01 and 4.00; two outputs, 4,000,000 x 30 5.42 and 5.50; eight classes, 600,000 x 20 3.12 and 3.13,
+        # 2,000,000 x 30 6.65 and 6.85; 16, 3,000,000 x 30 12.7 and 13.3.
         fused = getattr(self._objective_instance, "fused", None)
         sums = (fused is not None and self.subsample == 1.0 and train_pred.is_cuda
-                and train_pred.shape[1] == 1 and train_pred.shape[0] >= 4000000
+                and train_pred.numel() >= (4000000 if train_pred.shape[1] == 1 else 8000000)
                 and _as_defined(self, LBBase, "_get_weighted_gradient"))
         for i in range(self.n_estimators):
             model = deepcopy(self.base_models[i % len(self.base_models)]).set_random_state(self.random_state_)

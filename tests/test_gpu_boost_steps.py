@@ -249,3 +249,53 @@ def test_predictions_call_what_has_been_replaced(monkeypatch, owner, name):
     assert torch.allclose(model.predict_proba(X), want, rtol=0, atol=1e-15) and len(calls) == 1
     model._predict(X)
     assert len(calls) == (1 if name == "transform" else 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [2, 3, 4, 5, 8, 9, 10, 16, 33, 64, 127, 128, 129])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_softmax_gradients_by_entry_and_by_row(k, weighted):
+    """Rows that straddle stages and chunks, with and without the chunk sums (which ask for a thread per entry at any size): the same
+    bits, torch's softmax to rounding, and the sums in the quantiser's order."""
+    from lbtree import ops
+
+    torch.manual_seed(k)
+    for n in (1, 2, 2048 // k + 1, 4096 // k, 12345 // k + 2, 40000 // k + 1):
+        pred = torch.randn(n, k, dtype=torch.float64).cuda() * 4
+        y = torch.randint(0, k, (n,)).double().cuda()
+        w = torch.rand(n, dtype=torch.float64).cuda() if weighted else None
+        g, h = ops.weighted_gradient("log_loss", y, pred, w, 0.5)
+        gs, hs, sums = ops.weighted_gradient("log_loss", y, pred, w, 0.5, sums=True)
+        assert torch.equal(g, gs) and torch.equal(h, hs)
+        q = torch.softmax(pred, dim=1)
+        weight = w[:, None] if weighted else 1.0
+        # a quotient: an argument within 1 ulp of up to 32, k additions, exponentials and the division to an ulp each
+        bound = (k + 80) * 2.0 ** -52
+        assert ((gs - 0.5 * weight * (q - torch.nn.functional.one_hot(y.long(), k))).abs() <= bound).all()
+        assert ((hs - (weight * q * (1 - q)).clamp(min=1e-8)).abs() <= bound).all()  # (hessians are at least 1e-8)
+        for a, got in ((gs, sums[0]), (hs, sums[1])):
+            flat = torch.zeros(got.numel() * 4096, dtype=torch.float64)
+            flat[: n * k] = a.cpu().reshape(-1).abs()
+            lanes = torch.zeros(got.numel(), 256, dtype=torch.float64)
+            for part in flat.reshape(-1, 16, 256).unbind(1):
+                lanes = lanes + part
+            while lanes.shape[1] > 1:
+                lanes = lanes[:, : lanes.shape[1] // 2] + lanes[:, lanes.shape[1] // 2:]
+            assert torch.equal(lanes[:, 0], got.cpu())
+
+
+@pytest.mark.gpu
+def test_softmax_gradients_of_many_entries():
+    """Enough entries for a thread each without the sums too, in rows that a thread holds otherwise."""
+    from lbtree import ops
+
+    torch.manual_seed(1)
+    n, k = 800_003, 5
+    pred = torch.randn(n, k, dtype=torch.float64).cuda()
+    y = torch.randint(0, k, (n,)).double().cuda()
+    g, h = ops.weighted_gradient("log_loss", y, pred, None, 1.0)
+    some = 700_001  # fewer entries: a thread per row
+    g1, h1 = ops.weighted_gradient("log_loss", y[:some].contiguous(), pred[:some].contiguous(), None, 1.0)
+    assert torch.equal(g[:some], g1) and torch.equal(h[:some], h1)
+    g2, h2 = ops.weighted_gradient("log_loss", y[some:].contiguous(), pred[some:].contiguous(), None, 1.0)
+    assert torch.equal(g[some:], g2) and torch.equal(h[some:], h2)
