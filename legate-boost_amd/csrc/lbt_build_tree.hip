@@ -570,14 +570,23 @@ __global__ void __launch_bounds__(kThreads)
 // :613) the bins of that output stay as they are in memory, for the node and for its sibling,
 // and the gains are formed from those values, as the reference's split kernel would read them.
 //
-// Bound by its instructions while the histograms lie in the caches, then by memory (the last level of 2,000,000 x 200
-// with 8 outputs: 838 MB in 226 us). What a wave shares is told to the compiler (the number of its wave), so that
+// Bound by its instructions, and by memory where it stores what it scanned (2,000,000 x 200 with 8 outputs: 64 nodes 0.84 GB read and
+// written in 120 us). What a wave shares is told to the compiler (the number of its wave), so that
 // addresses and conditions are scalar; the nodes' sums and the gain terms that do not depend on the bin are formed once,
 // in lane k for output k (in the loop they were a third of the quotients, and the sibling's sums a load to wait for per
-// tile and output); and the four quotients of a bin and its sibling's have no branch between them. All levels of
-// 2,000,000 x 200 with 8 outputs: 908 -> 625 us; the nine of 1,000,000 x 50 with 512 samples: 233 -> 172.
+// tile and output); and the four quotients of a bin and its sibling's have no branch between them. Sums are formed in 32 bits
+// (narrow_sums_hold) and turned into doubles from there, differences are differences of doubles, and quotients are formed without
+// what only the ends of the exponent need (plain_quotients): of 190 instructions a tile and output without a derived sibling 115
+// are left. The 18 launches with a wave a pair of three trees of 2,000,000 x 200 with 8 outputs: 1740 -> 1426 us (32 bits alone
+// 1591); the 20 of four trees of 1,000,000 x 50 with 512 samples: 464 -> 402.
 // kW: waves that share a (node, feature), see scan_split_launch.
 constexpr int kFusedMaxK   = 64;  // lane k of the wave keeps the running sums of output k
+
+// The running sums are formed in their lower 32 bits, one instruction a step where 64 bits take four. The absolute values of an output's
+// grads (hessians) sum up to less than 2^31 + N + 1024; with the root's sum G of them, sums over any rows lie between -down and
+// up, down = (2^31 + N + 1024 - G) / 2 + 1, up with + G, less than 2^32 apart: the lower half of a sum + down is the sum + down. Whole numbers
+// of that size are exact as doubles, and so are their differences.
+constexpr bool narrow_sums_hold(int64_t n_rows) { return n_rows < (int64_t(1) << 31) - 4096; }
 
 __device__ __forceinline__ Cand wave_best(const Cand& c)  // the same in every lane
 {
@@ -585,14 +594,32 @@ __device__ __forceinline__ Cand wave_best(const Cand& c)  // the same in every l
   return from < 0 ? Cand{0.0, -1} : Cand{wave_read_lane_f64(c.gain, from), __builtin_amdgcn_readlane(c.bin, from)};
 }
 
+// n / d correctly rounded, where neither is near the ends of the exponent's range: an approximate reciprocal, two steps of Newton's
+// iteration and the remainder's correction. It is what `/` does without the scaling and the special cases, three instructions of eleven.
+__device__ __forceinline__ double quotient_plain(double n, double d)
+{
+  double r = __builtin_amdgcn_rcp(d);
+  r        = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  r        = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+// Without l1 the sums of grads are squared as they are. Sums are whole numbers below 2^35 times inv_g (inv_h); a denominator is at
+// least reg where its quotient counts.
+__device__ __forceinline__ bool plain_quotients(double l1, double inv_g, double inv_h, double reg)
+{
+  auto ordinary = [](double v) { return v >= 1e-60 && v <= 1e60; };
+  return l1 == 0.0 && ordinary(inv_g) && ordinary(inv_h) && ordinary(reg);
+}
+
 template <int kW>
 __global__ void __launch_bounds__(kW == 1 ? kThreads : kW * 64)
   scan_split_kernel(HistView hist, const I64Pair* __restrict__ node_sums, int F, const int32_t* __restrict__ row_pointers,
                     int node_begin, int n_nodes, const uint8_t* __restrict__ feature_set,
                     const double* __restrict__ scales, double l1, double l2, double min_split_gain, Cand* partial,
-                    bool store)
+                    int64_t n_rows, bool store)
 {
-  __shared__ I64Pair s_total[kW][kFusedMaxK];
+  __shared__ uint2 s_total[kW][kFusedMaxK];
   __shared__ Cand s_best[2][kW];
   const int lane  = threadIdx.x & 63;
   const int wave  = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -631,31 +658,41 @@ __global__ void __launch_bounds__(kW == 1 ? kThreads : kW * 64)
   const double reg   = 1e-5 > l2 ? 1e-5 : l2;
   const double own_n = leaf_gain(static_cast<double>(sum_n.grad) * inv_g, static_cast<double>(sum_n.hess) * inv_h, l1, reg);
   const double own_s = leaf_gain(static_cast<double>(sum_s.grad) * inv_g, static_cast<double>(sum_s.hess) * inv_h, l1, reg);
+  // lane k: the lower halves' origin of output k, see narrow_sums_hold
+  uint32_t down_g = 0, down_h = 0;
+  if (lane < K) {
+    const I64Pair root = node_sums[lane];
+    const int64_t most = (int64_t(1) << 31) + n_rows + 1024;
+    down_g = static_cast<uint32_t>((most - root.grad) / 2 + 1);
+    down_h = static_cast<uint32_t>((most - root.hess) / 2 + 1);
+  }
+  const double all_ng = static_cast<double>(sum_n.grad), all_nh = static_cast<double>(sum_n.hess);
+  const double all_sg = static_cast<double>(sum_s.grad), all_sh = static_cast<double>(sum_s.hess);
   const int fb = row_pointers[i], fe = row_pointers[i + 1];
   const int n_tiles = (fe - fb + 63) / 64;
   const int t0 = n_tiles * slice / kW, t1 = n_tiles * (slice + 1) / kW;
   const I64Pair* const bins_n = hist.at(node, 0, 0);
   const I64Pair* const bins_p = derive ? hist.at(parent, 0, 0) : bins_n;
   const I64Pair* const bins_s = derive ? hist.at(sib, 0, 0) : bins_n;
-  int64_t agg_g = 0, agg_h = 0;  // lane k: sums of output k over the tiles done so far
+  uint32_t agg_g = 0, agg_h = 0;  // lane k: sums of output k over the tiles done so far, lower halves
   if constexpr (kW > 1) {
     // every wave adds up its tiles, then takes over the sums of the tiles in front of them
     for (int k = 0; k < K; k++) {
-      I64Pair t{0, 0};
+      uint32_t g = 0, h = 0;
       for (int tile = t0; tile < t1; tile++) {
         const int b     = fb + tile * 64 + lane;
         const I64Pair v = bins_n[static_cast<int64_t>(k) * hist.B + min(b, fe - 1)];
-        t.grad += b < fe ? v.grad : 0;
-        t.hess += b < fe ? v.hess : 0;
+        g += b < fe ? static_cast<uint32_t>(v.grad) : 0u;
+        h += b < fe ? static_cast<uint32_t>(v.hess) : 0u;
       }
-      const int64_t tg = wave_inclusive_sum(t.grad), th = wave_inclusive_sum(t.hess);
-      if (lane == 63) s_total[wave][k] = I64Pair{tg, th};
+      const int all_g = wave_inclusive_sum32(static_cast<int>(g)), all_h = wave_inclusive_sum32(static_cast<int>(h));
+      if (lane == 63) s_total[wave][k] = make_uint2(static_cast<uint32_t>(all_g), static_cast<uint32_t>(all_h));
     }
     __syncthreads();
     if (lane < K) {
       for (int w = 0; w < wave; w++) {
-        agg_g += s_total[w][lane].grad;
-        agg_h += s_total[w][lane].hess;
+        agg_g += s_total[w][lane].x;
+        agg_h += s_total[w][lane].y;
       }
     }
   }
@@ -664,8 +701,14 @@ __global__ void __launch_bounds__(kW == 1 ? kThreads : kW * 64)
   // are scanned and stored: the stores would otherwise keep every load behind them, and a wave
   // would wait for memory once per tile and output. (Two or four of them ahead: no faster.)
   const int n_items = (t1 - t0) * K;
-  auto run = [&](auto derives) {
+  auto run = [&](auto derives, auto plains) {
     constexpr bool kDerive = decltype(derives)::value;
+    auto quotient = [&](double grad, double hess) {
+      if constexpr (decltype(plains)::value)
+        return quotient_plain(grad * grad, hess + reg);
+      else
+        return leaf_gain_select(grad, hess, l1, reg);
+    };
     I64Pair val_next{0, 0}, other_next{0, 0};
     int fetch_t = t0, fetch_k = 0;
     auto fetch = [&]() {
@@ -687,37 +730,56 @@ __global__ void __launch_bounds__(kW == 1 ? kThreads : kW * 64)
       I64Pair val   = in ? val_next : I64Pair{0, 0}, sval = other_next;
       if (item + 1 < n_items) fetch();
       const int64_t at = static_cast<int64_t>(k) * hist.B + bin;
+      double lg, lh;  // what lies left of the bin
       if ((scans >> k & 1) != 0) {
-        int64_t eg = wave_inclusive_sum(val.grad), eh = wave_inclusive_sum(val.hess);
-        const int64_t tile_g = wave_read_lane(eg, 63), tile_h = wave_read_lane(eh, 63);
-        eg += wave_read_lane(agg_g, k);
-        eh += wave_read_lane(agg_h, k);
+        const uint32_t raw_g = static_cast<uint32_t>(val.grad), raw_h = static_cast<uint32_t>(val.hess);
+        const uint32_t to_g = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(raw_g)) + __builtin_amdgcn_readlane(agg_g, k));
+        const uint32_t to_h = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(raw_h)) + __builtin_amdgcn_readlane(agg_h, k));
+        const int tile_g = __builtin_amdgcn_readlane(to_g, 63), tile_h = __builtin_amdgcn_readlane(to_h, 63);
         if (lane == k) {
-          agg_g += tile_g;
-          agg_h += tile_h;
+          agg_g = static_cast<uint32_t>(tile_g);
+          agg_h = static_cast<uint32_t>(tile_h);
         }
+        const uint32_t from_g = static_cast<uint32_t>(__builtin_amdgcn_readlane(down_g, k));
+        const uint32_t from_h = static_cast<uint32_t>(__builtin_amdgcn_readlane(down_h, k));
+        lg = static_cast<double>(to_g + from_g) - static_cast<double>(from_g);
+        lh = static_cast<double>(to_h + from_h) - static_cast<double>(from_h);
         // the reference skips the store when the running sum is not positive
         // (build_tree.cu:645); the raw bin value then stays in place
-        const bool positive = eg > 0 || eh > 0;
-        if (positive) val = I64Pair{eg, eh};
-        if (store && in && positive) const_cast<I64Pair*>(bins_n)[at] = val;
-        if constexpr (kDerive) {
-          sval = I64Pair{sval.grad - val.grad, sval.hess - val.hess};
-          if (store && in) const_cast<I64Pair*>(bins_s)[at] = sval;
+        const bool positive = lg > 0 || lh > 0;
+        if (store) {
+          const int64_t eg = static_cast<int64_t>(to_g + from_g) - static_cast<int64_t>(from_g);
+          const int64_t eh = static_cast<int64_t>(to_h + from_h) - static_cast<int64_t>(from_h);
+          if (in && positive) const_cast<I64Pair*>(bins_n)[at] = I64Pair{eg, eh};
+          if constexpr (kDerive) {
+            const I64Pair left = positive ? I64Pair{eg, eh} : val;
+            if (in) const_cast<I64Pair*>(bins_s)[at] = I64Pair{sval.grad - left.grad, sval.hess - left.hess};
+          }
         }
+        if (__any(!positive && (to_g | to_h | raw_g | raw_h) != 0)) {  // (else a bin that is not positive is zero, as its sum)
+          asm volatile("");  // (a branch: without it both conversions are formed every time)
+          lg = positive ? lg : static_cast<double>(val.grad);
+          lh = positive ? lh : static_cast<double>(val.hess);
+        }
+      } else {
+        lg = static_cast<double>(val.grad);
+        lh = static_cast<double>(val.hess);
       }
       // build_tree.cu:727-730: one output without a valid split on a bin voids the bin. The quotients of
-      // the node and of the sibling are formed without branches, so that their chains run side by side.
-      const int64_t ng = wave_read_lane(sum_n.grad, k) - val.grad, nh = wave_read_lane(sum_n.hess, k) - val.hess;
-      live_n = live_n && val.hess > 0 && nh > 0;
-      const double left_n = leaf_gain_select(static_cast<double>(val.grad) * inv_g, static_cast<double>(val.hess) * inv_h, l1, reg);
-      const double right_n = leaf_gain_select(static_cast<double>(ng) * inv_g, static_cast<double>(nh) * inv_h, l1, reg);
+      // the node and of the sibling are formed without branches, so that their chains run side by side. (All sums are whole
+      // numbers below 2^35, and so are their differences as doubles.)
+      const double rg = wave_read_lane_f64(all_ng, k) - lg, rh = wave_read_lane_f64(all_nh, k) - lh;
+      live_n = live_n && lh > 0 && rh > 0;
+      const double left_n  = quotient(lg * inv_g, lh * inv_h);
+      const double right_n = quotient(rg * inv_g, rh * inv_h);
       double left_s = 0.0, right_s = 0.0;
       if constexpr (kDerive) {
-        const int64_t rg = wave_read_lane(sum_s.grad, k) - sval.grad, rh = wave_read_lane(sum_s.hess, k) - sval.hess;
-        live_s  = live_s && sval.hess > 0 && rh > 0;
-        left_s  = leaf_gain_select(static_cast<double>(sval.grad) * inv_g, static_cast<double>(sval.hess) * inv_h, l1, reg);
-        right_s = leaf_gain_select(static_cast<double>(rg) * inv_g, static_cast<double>(rh) * inv_h, l1, reg);
+        const bool derived = (scans >> k & 1) != 0;
+        const double slg = static_cast<double>(sval.grad) - (derived ? lg : 0.0), slh = static_cast<double>(sval.hess) - (derived ? lh : 0.0);
+        const double srg = wave_read_lane_f64(all_sg, k) - slg, srh = wave_read_lane_f64(all_sh, k) - slh;
+        live_s  = live_s && slh > 0 && srh > 0;
+        left_s  = quotient(slg * inv_g, slh * inv_h);
+        right_s = quotient(srg * inv_g, srh * inv_h);
       }
       gain_n += 0.5 * (left_n + right_n - wave_read_lane_f64(own_n, k)) - min_split_gain;
       if constexpr (kDerive) gain_s += 0.5 * (left_s + right_s - wave_read_lane_f64(own_s, k)) - min_split_gain;
@@ -737,10 +799,17 @@ __global__ void __launch_bounds__(kW == 1 ? kThreads : kW * 64)
       }
     }
   };
-  if (derive)
-    run(std::true_type{});
-  else
-    run(std::false_type{});
+  if (plain_quotients(l1, inv_g, inv_h, reg)) {
+    if (derive)
+      run(std::true_type{}, std::true_type{});
+    else
+      run(std::false_type{}, std::true_type{});
+  } else {
+    if (derive)
+      run(std::true_type{}, std::false_type{});
+    else
+      run(std::false_type{}, std::false_type{});
+  }
   best_n = wave_best(best_n);
   if (derive) best_s = wave_best(best_s);
   if constexpr (kW > 1) {
@@ -773,13 +842,13 @@ constexpr int64_t kSharedScanPairs = 512;
 
 void scan_split_launch(hipStream_t stream, int max_bins, const HistView& hv, const I64Pair* node_sums, int F,
                        const int32_t* row_pointers, int node_begin, int n_nodes, const uint8_t* feature_set,
-                       const double* scales, double l1, double l2, double min_split_gain, Cand* partial, bool store)
+                       const double* scales, double l1, double l2, double min_split_gain, Cand* partial, int64_t n_rows, bool store)
 {
   const int64_t pairs = static_cast<int64_t>(F) * n_nodes;
   auto launch         = [&](auto kernel, int64_t groups, int threads) {
     kernel<<<static_cast<unsigned>(groups), threads, 0, stream>>>(hv, node_sums, F, row_pointers, node_begin, n_nodes,
                                                                   feature_set, scales, l1, l2, min_split_gain, partial,
-                                                                  store);
+                                                                  n_rows, store);
   };
   if (pairs > kSharedScanPairs || max_bins <= (hv.K == 1 ? 128 : 64))
     launch(scan_split_kernel<1>, (pairs + kThreads / 64 - 1) / (kThreads / 64), kThreads);
@@ -2112,13 +2181,13 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
                                               next_begin >= hv.node_begin && next_end <= hv.node_end));
       const bool wanted = next_reads || (taps && taps->histogram);
       // ... and where nothing reads them again the fused pass, which then only reads, wins as well
-      const bool fused = K <= kFusedMaxK && (K >= 2 || n_nodes <= 256 || !wanted);
+      const bool fused = narrow_sums_hold(N) && K <= kFusedMaxK && (K >= 2 || n_nodes <= 256 || !wanted);
       const bool store = !fused || wanted;
       kept             = store;
       if (fused) {
         ProfScope ps(LBT_PROF_SCAN, stream);
         scan_split_launch(stream, hs.max_bins, hv, L.node_sums, F, L.row_pointers, batch_begin, n_nodes, feature_set,
-                          L.scales, prm.l1_regularization, prm.l2_regularization, prm.min_split_gain, L.partial, store);
+                          L.scales, prm.l1_regularization, prm.l2_regularization, prm.min_split_gain, L.partial, N, store);
       } else {
         {
           ProfScope ps(LBT_PROF_SCAN, stream);

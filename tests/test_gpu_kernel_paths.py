@@ -884,3 +884,32 @@ def test_bins_spread_over_the_lanes_of_a_row(f, k, s, dtype, share):
     gr, cr = gu.both(X, g, h, levels=True, max_depth=4, split_samples=s, seed=f)
     gu.assert_tree_parity(gr, cr, levels=True)
     assert (cr.feature != -1).sum() > 5
+
+
+@pytest.mark.parametrize("kind", ["plain", "l1", "tiny", "huge", "signs", "zero_hessians"])
+@pytest.mark.parametrize("n,f,k,s", [(3000, 7, 1, 100), (2500, 5, 3, 300), (20000, 3, 8, 64)])
+def test_scanned_levels_in_32_bits(n, f, k, s, kind):
+    """Running sums formed in their lower halves and quotients without the special cases of a division: penalties, scales at the ends of
+    the exponents (the general division), grads of one sign whose sums reach 2^31, hessians of both signs and of zero, whose
+    running sums are not positive and leave bins as they are: the oracle's histograms and gains bit for bit."""
+    import gpu_util as gu
+
+    rs = np.random.RandomState(n + k)
+    X = rs.normal(size=(n, f)).astype(np.float32)
+    X[:, 0] = rs.randint(0, 3, n)
+    g, h = rs.normal(size=(n, k)), 0.01 + rs.rand(n, k)
+    kw = {}
+    if kind == "l1":
+        kw = dict(l1_regularization=0.7)
+    elif kind == "tiny":
+        g, h = g * 1e-75, h * 1e-75
+    elif kind == "huge":
+        g, h = g * 1e75, h * 1e70
+    elif kind == "signs":
+        g, h = np.abs(g) * np.where(np.arange(k) % 2, 1, -1), rs.normal(size=(n, k))
+        h[:, 0] = np.abs(h[:, 0]) + 0.5
+    elif kind == "zero_hessians":
+        h[rs.rand(n, k) < 0.6] = 0.0
+        g = -np.abs(g)
+    gr, cr = gu.both(X, g, h, max_depth=6, split_samples=s, seed=5, **kw)
+    gu.assert_tree_parity(gr, cr)
