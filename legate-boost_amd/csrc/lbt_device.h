@@ -218,6 +218,24 @@ __device__ __forceinline__ double leaf_gain_select(double grad, double hess, dou
   return (z * z) / (hess + reg);
 }
 
+// n / d correctly rounded, where neither is near the ends of the exponent's range: an approximate reciprocal, two steps of Newton's
+// iteration and the remainder's correction. It is what `/` does without the scaling and the special cases, three instructions of eleven.
+__device__ __forceinline__ double quotient_plain(double n, double d)
+{
+  double r = __builtin_amdgcn_rcp(d);
+  r        = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  r        = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+// Without l1 the sums of grads are squared as they are. Sums are whole numbers below 2^35 times inv_g (inv_h); a denominator is at
+// least reg where its quotient counts.
+__device__ __forceinline__ bool plain_quotients(double l1, double inv_g, double inv_h, double reg)
+{
+  auto ordinary = [](double v) { return v >= 1e-60 && v <= 1e60; };
+  return l1 == 0.0 && ordinary(inv_g) && ordinary(inv_h) && ordinary(reg);
+}
+
 // Sum of the threads before this one; all threads of the workgroup call it. s_wave: one int per wave.
 template <int kT>
 __device__ __forceinline__ int block_exclusive_sum32(int v, int* s_wave)

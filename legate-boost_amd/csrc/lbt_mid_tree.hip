@@ -561,8 +561,7 @@ enum class Nodes { kCarried, kDecide, kDecided };
 
 // A packed word holds the sum of grads in its upper and the sum of hessians in its lower half. Rounded
 // hessians are not negative here and sum up to less than 2^32. The grads of all rows sum up to -down and +up
-// with up + down < 2^32, so a sum that left the 32 bits is recognised by lying outside these limits
-// (decode_grad).
+// with up + down < 2^32, so the lower half of a sum + down is the sum + down (mid_scan_kernel).
 template <typename BinT, Nodes kNodes>
 __global__ void __launch_bounds__(kWide)
   mid_histogram_kernel(MidArgs a, MidTreeState st, LevelPlan p, LevelPlan above, int lanes_log, int writers,
@@ -678,14 +677,6 @@ __global__ void __launch_bounds__(kWide)
     }
 }
 
-__device__ __forceinline__ int64_t decode_grad(uint32_t v, int64_t up, int64_t down)
-{
-  int64_t s = static_cast<int32_t>(v);
-  s += s < -down ? int64_t(1) << 32 : 0;
-  s -= s > up ? int64_t(1) << 32 : 0;
-  return s;
-}
-
 // A launch of a narrow level is a chain of latencies: the images, the sums over the workgroup, the quotients, the best
 // bin. The quotients of a node and its sibling therefore have no branch between them, the nodes' sums are asked for with
 // the images, and the best of a wave is found without the LDS (18 permutes one after the other, twice): the eight levels
@@ -698,8 +689,8 @@ template <bool kLess>
 __global__ void __launch_bounds__(kScan)
   mid_scan_kernel(MidArgs a, MidTreeState st, LevelPlan p)
 {
-  __shared__ I64Pair s_tot[2][kScan / 64];
-  __shared__ I64Pair s_carry[kMidMaxOutputs];
+  __shared__ uint2 s_tot[2][kScan / 64];
+  __shared__ uint2 s_carry[kMidMaxOutputs];
   __shared__ double s_best[2][kScan / 64];
   __shared__ unsigned s_bkey[2][kScan / 64];
   __shared__ int s_less[2][kScan / 64];
@@ -722,8 +713,9 @@ __global__ void __launch_bounds__(kScan)
   }
   const int n_bins = st.counts[f], rp = st.rp[f];
   const int64_t fs = static_cast<int64_t>(a.F) * a.S;
-  const int64_t up = static_cast<int64_t>(st.q_stats[0]), down = static_cast<int64_t>(st.q_stats[1]);
-  const bool fits    = up <= 2147483647LL && down <= 2147483647LL;  // no sum of grads leaves 32 bits
+  // sums of grads over any rows lie between -down and up, less than 2^32 apart: the lower half of a sum + down is the sum + down
+  const uint32_t down  = static_cast<uint32_t>(st.q_stats[1]);
+  const double down_of = static_cast<double>(down);
   const double inv_g = st.scales[2], inv_h = st.scales[3];
   const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
   I64Pair* const hist         = st.hist[p.depth & 1];
@@ -731,93 +723,105 @@ __global__ void __launch_bounds__(kScan)
   double best_n = 0.0, best_s = 0.0;
   unsigned key_n = 0, key_s = 0;
   bool less_n = false, less_s = false;  // the best split's left child has the smaller hessian (of the first output)
-  for (int base = 0; base < n_bins; base += kScan) {
-    const int bin = base + tid;
-    const bool in = bin < n_bins;
-    double gain_n = 0.0, gain_s = 0.0;
-    bool dead_n = !in, dead_s = !in || root;
-    bool left_n = false, left_s = false;
-    for (int k = 0; k < a.K; k++) {
-      I64Pair v{0, 0}, pv{0, 0};
-      const I64Pair ns = st.node_sums[static_cast<int64_t>(p.level_first + node) * a.K + k];
-      const I64Pair ss = root ? I64Pair{0, 0} : st.node_sums[static_cast<int64_t>(p.level_first + sib) * a.K + k];
-      if (in) {
-        const unsigned long long* img = st.images + (static_cast<int64_t>(pair) * a.K + k) * fs + static_cast<int64_t>(f) * a.S + bin;
-        const int64_t step = static_cast<int64_t>(p.built) * a.K * fs;
-        if (!root) pv = parent[k * fs + bin];
-        int c = 0;
-        auto add = [&](auto width, auto plain) {
-          constexpr int kW = decltype(width)::value;
-          for (; c + kW <= p.chunks; c += kW) {
-            unsigned long long w[kW];
+  auto run = [&](auto plains) {
+    auto quotient = [&](double grad, double hess) {
+      if constexpr (decltype(plains)::value)
+        return quotient_plain(grad * grad, hess + reg);
+      else
+        return leaf_gain_select(grad, hess, a.l1, reg);
+    };
+    for (int base = 0; base < n_bins; base += kScan) {
+      const int bin = base + tid;
+      const bool in = bin < n_bins;
+      double gain_n = 0.0, gain_s = 0.0;
+      bool dead_n = !in, dead_s = !in || root;
+      bool left_n = false, left_s = false;
+      for (int k = 0; k < a.K; k++) {
+        uint32_t raw_g = 0, raw_h = 0;  // of the bin, lower halves
+        I64Pair pv{0, 0};
+        const I64Pair ns = st.node_sums[static_cast<int64_t>(p.level_first + node) * a.K + k];
+        const I64Pair ss = root ? I64Pair{0, 0} : st.node_sums[static_cast<int64_t>(p.level_first + sib) * a.K + k];
+        if (in) {
+          const unsigned long long* img = st.images + (static_cast<int64_t>(pair) * a.K + k) * fs + static_cast<int64_t>(f) * a.S + bin;
+          const int64_t step = static_cast<int64_t>(p.built) * a.K * fs;
+          if (!root) pv = parent[k * fs + bin];
+          int c = 0;
+          auto add = [&](auto width) {
+            constexpr int kW = decltype(width)::value;
+            for (; c + kW <= p.chunks; c += kW) {
+              unsigned long long w[kW];
 #pragma unroll
-            for (int u = 0; u < kW; u++) w[u] = img[(c + u) * step];
+              for (int u = 0; u < kW; u++) w[u] = img[(c + u) * step];
 #pragma unroll
-            for (int u = 0; u < kW; u++) {
-              const uint32_t hi = static_cast<uint32_t>(w[u] >> 32);
-              v.grad += decltype(plain)::value ? static_cast<int64_t>(static_cast<int32_t>(hi)) : decode_grad(hi, up, down);
-              v.hess += static_cast<uint32_t>(w[u]);
+              for (int u = 0; u < kW; u++) {
+                raw_g += static_cast<uint32_t>(w[u] >> 32);
+                raw_h += static_cast<uint32_t>(w[u]);
+              }
             }
-          }
-        };
-        if (fits) {
-          add(std::integral_constant<int, 8>{}, std::true_type{});
-          add(std::integral_constant<int, 1>{}, std::true_type{});
-        } else {
-          add(std::integral_constant<int, 1>{}, std::false_type{});
+          };
+          add(std::integral_constant<int, 8>{});
+          add(std::integral_constant<int, 1>{});
+        }
+        uint32_t g = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(raw_g)));
+        uint32_t h = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(raw_h)));
+        if (lane == 63) s_tot[k & 1][wave] = make_uint2(g, h);
+        __syncthreads();
+        if (base > 0) {
+          g += s_carry[k].x;
+          h += s_carry[k].y;
+        }
+        for (int w = 0; w < kScan / 64; w++) {
+          g += w < wave ? s_tot[k & 1][w].x : 0;
+          h += w < wave ? s_tot[k & 1][w].y : 0;
+        }
+        // the bin as it was accumulated where neither running sum is positive (build_tree.cu:645): no hessian is negative, so
+        // it then has none
+        const uint32_t kept = h == 0 && g + down <= down ? raw_g : g;
+        // whole numbers below 2^35 and their differences are exact as doubles
+        const double nlg = static_cast<double>(kept + down) - down_of, nlh = static_cast<double>(h);
+        const double slg = static_cast<double>(pv.grad) - nlg, slh = static_cast<double>(pv.hess) - nlh;
+        const double nrg = static_cast<double>(ns.grad) - nlg, nrh = static_cast<double>(ns.hess) - nlh;
+        const double srg = static_cast<double>(ss.grad) - slg, srh = static_cast<double>(ss.hess) - slh;
+        const double n_left = quotient(nlg * inv_g, nlh * inv_h), n_right = quotient(nrg * inv_g, nrh * inv_h);
+        const double s_left = quotient(slg * inv_g, slh * inv_h), s_right = quotient(srg * inv_g, srh * inv_h);
+        const double n_own = quotient(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h);
+        const double s_own = quotient(static_cast<double>(ss.grad) * inv_g, static_cast<double>(ss.hess) * inv_h);
+        if (kLess && k == 0) {
+          left_n = nlh < nrh;
+          left_s = slh < srh;
+        }
+        dead_n |= nlh <= 0 || nrh <= 0;
+        dead_s |= slh <= 0 || srh <= 0;
+        gain_n += 0.5 * (n_left + n_right - n_own) - a.min_split_gain;
+        gain_s += 0.5 * (s_left + s_right - s_own) - a.min_split_gain;
+        if (in) {
+          const int64_t at = static_cast<int64_t>(k) * fs + static_cast<int64_t>(f) * a.S + bin;
+          const I64Pair nv{static_cast<int64_t>(kept + down) - static_cast<int64_t>(down), static_cast<int64_t>(h)};
+          hist[static_cast<int64_t>(node) * a.K * fs + at] = nv;
+          if (!root) hist[static_cast<int64_t>(sib) * a.K * fs + at] = I64Pair{pv.grad - nv.grad, pv.hess - nv.hess};
+        }
+        // the carry of a tile is read by the next one; a barrier of the next output lies between
+        if (base + kScan < n_bins) {
+          __syncthreads();
+          if (tid == kScan - 1) s_carry[k] = make_uint2(g, h);
         }
       }
-      int64_t g = wave_inclusive_sum(v.grad), h = wave_inclusive_sum(v.hess);
-      if (lane == 63) s_tot[k & 1][wave] = I64Pair{g, h};
-      __syncthreads();
-      if (base > 0) {
-        g += s_carry[k].grad;
-        h += s_carry[k].hess;
-      }
-      for (int w = 0; w < kScan / 64; w++) {
-        g += w < wave ? s_tot[k & 1][w].grad : 0;
-        h += w < wave ? s_tot[k & 1][w].hess : 0;
-      }
-      // the bin as it was accumulated where neither running sum is positive (build_tree.cu:645)
-      const I64Pair nv = g > 0 || h > 0 ? I64Pair{g, h} : v;
-      const I64Pair sv{pv.grad - nv.grad, pv.hess - nv.hess};
-      const I64Pair nr{ns.grad - nv.grad, ns.hess - nv.hess}, sr{ss.grad - sv.grad, ss.hess - sv.hess};
-      const double n_left  = leaf_gain_select(static_cast<double>(nv.grad) * inv_g, static_cast<double>(nv.hess) * inv_h, a.l1, reg);
-      const double n_right = leaf_gain_select(static_cast<double>(nr.grad) * inv_g, static_cast<double>(nr.hess) * inv_h, a.l1, reg);
-      const double s_left  = leaf_gain_select(static_cast<double>(sv.grad) * inv_g, static_cast<double>(sv.hess) * inv_h, a.l1, reg);
-      const double s_right = leaf_gain_select(static_cast<double>(sr.grad) * inv_g, static_cast<double>(sr.hess) * inv_h, a.l1, reg);
-      const double n_own = leaf_gain_select(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, a.l1, reg);
-      const double s_own = leaf_gain_select(static_cast<double>(ss.grad) * inv_g, static_cast<double>(ss.hess) * inv_h, a.l1, reg);
-      if (kLess && k == 0) {
-        left_n = nv.hess < nr.hess;
-        left_s = sv.hess < sr.hess;
-      }
-      dead_n |= nv.hess <= 0 || nr.hess <= 0;
-      dead_s |= sv.hess <= 0 || sr.hess <= 0;
-      gain_n += 0.5 * (n_left + n_right - n_own) - a.min_split_gain;
-      gain_s += 0.5 * (s_left + s_right - s_own) - a.min_split_gain;
-      if (in) {
-        const int64_t at = static_cast<int64_t>(k) * fs + static_cast<int64_t>(f) * a.S + bin;
-        hist[static_cast<int64_t>(node) * a.K * fs + at] = nv;
-        if (!root) hist[static_cast<int64_t>(sib) * a.K * fs + at] = sv;
-      }
-      // the carry of a tile is read by the next one; a barrier of the next output lies between
-      if (base + kScan < n_bins) {
-        __syncthreads();
-        if (tid == kScan - 1) s_carry[k] = I64Pair{g, h};
-      }
+      const unsigned key = tie_key_of_bin(rp + bin);
+      const bool take_n = !dead_n && gain_n > 0 && (gain_n > best_n || (gain_n == best_n && key > key_n));
+      const bool take_s = !dead_s && gain_s > 0 && (gain_s > best_s || (gain_s == best_s && key > key_s));
+      best_n = take_n ? gain_n : best_n;
+      key_n  = take_n ? key : key_n;
+      if constexpr (kLess) less_n = take_n ? left_n : less_n;
+      best_s = take_s ? gain_s : best_s;
+      key_s  = take_s ? key : key_s;
+      if constexpr (kLess) less_s = take_s ? left_s : less_s;
+      if (base + kScan < n_bins) __syncthreads();
     }
-    const unsigned key = tie_key_of_bin(rp + bin);
-    const bool take_n = !dead_n && gain_n > 0 && (gain_n > best_n || (gain_n == best_n && key > key_n));
-    const bool take_s = !dead_s && gain_s > 0 && (gain_s > best_s || (gain_s == best_s && key > key_s));
-    best_n = take_n ? gain_n : best_n;
-    key_n  = take_n ? key : key_n;
-    if constexpr (kLess) less_n = take_n ? left_n : less_n;
-    best_s = take_s ? gain_s : best_s;
-    key_s  = take_s ? key : key_s;
-    if constexpr (kLess) less_s = take_s ? left_s : less_s;
-    if (base + kScan < n_bins) __syncthreads();
-  }
+  };
+  if (plain_quotients(a.l1, inv_g, inv_h, reg))
+    run(std::true_type{});
+  else
+    run(std::false_type{});
   const double own_n = best_n, own_s = best_s;
   const unsigned own_key_n = key_n, own_key_s = key_s;
   wave_best_key(best_n, key_n);
