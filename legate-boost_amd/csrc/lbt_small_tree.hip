@@ -841,7 +841,14 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
       }
     };
     // calculate_gain with the parent's term formed once per node
+    const bool plain = plain_quotients(a.l1, inv_g, inv_h, reg);
     auto gain_of = [&](const I64Pair& ls, const I64Pair& rs, double parent) {
+      if (plain) {
+        const double lg = static_cast<double>(ls.grad) * inv_g, rg = static_cast<double>(rs.grad) * inv_g;
+        return 0.0 + ((0.5 * (quotient_plain(lg * lg, static_cast<double>(ls.hess) * inv_h + reg) +
+                              quotient_plain(rg * rg, static_cast<double>(rs.hess) * inv_h + reg) - parent)) -
+                      a.min_split_gain);
+      }
       return 0.0 + ((0.5 * (leaf_gain(static_cast<double>(ls.grad) * inv_g, static_cast<double>(ls.hess) * inv_h, a.l1, reg) +
                             leaf_gain(static_cast<double>(rs.grad) * inv_g, static_cast<double>(rs.hess) * inv_h, a.l1, reg) -
                             parent)) -
