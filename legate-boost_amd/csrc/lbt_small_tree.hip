@@ -805,31 +805,44 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     // other threads' in the LDS. Sums, parent's term and best split of the node at hand stay in registers.
     int2 q[kG > 1 ? kE : 1];
     auto pair_at = [&](int e) { return i0 + e < a.N ? s_q[entry[e] & 0xffff] : make_int2(0, 0); };
-    I64Pair sum{0, 0};
+    // Sums are formed in their lower 32 bits. Absolute grads (hessians) sum up to less than 2^31 + N + 1024; with the root's sum G of them, sums
+    // over any rows lie between -down and up, down = (2^31 + N + 1024 - G) / 2 + 1, up with + G, less than 2^32 apart: the lower half of
+    // a sum + down is the sum + down. As doubles such whole numbers are exact.
+    const I64Pair all    = st.node_sums[0];
+    const int64_t most   = (int64_t(1) << 31) + a.N + 1024;
+    const uint32_t down_g = static_cast<uint32_t>((most - all.grad) / 2 + 1), down_h = static_cast<uint32_t>((most - all.hess) / 2 + 1);
+    const double from_g = static_cast<double>(down_g), from_h = static_cast<double>(down_h);
+    uint2* const s_sums = reinterpret_cast<uint2*>(s_pair[0]);
+    uint2 sum           = make_uint2(0, 0);
 #pragma unroll
     for (int e = 0; e < kE; e++) {
       const int2 v = pair_at(e);
       if constexpr (kG > 1) q[e] = v;
-      sum.grad += v.x;
-      sum.hess += v.y;
+      sum.x += static_cast<uint32_t>(v.x);
+      sum.y += static_cast<uint32_t>(v.y);
     }
-    const int64_t ig = wave_inclusive_sum(sum.grad), ih = wave_inclusive_sum(sum.hess);
-    if (lane == 63) s_pair[0][wave] = I64Pair{ig, ih};
+    const uint32_t ig = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum.x)));
+    const uint32_t ih = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum.y)));
+    if (lane == 63) s_sums[wave] = make_uint2(ig, ih);
     __syncthreads();
-    I64Pair run{ig - sum.grad, ih - sum.hess};
+    uint2 run = make_uint2(ig - sum.x, ih - sum.y);
 #pragma unroll 4  // (not all in registers at once)
     for (int w = 0; w < kT / 64; w++) {
-      run.grad += w < wave ? s_pair[0][w].grad : 0;
-      run.hess += w < wave ? s_pair[0][w].hess : 0;
+      run.x += w < wave ? s_sums[w].x : 0;
+      run.y += w < wave ? s_sums[w].y : 0;
     }
     int first_node = kNone, cur = kNone;
     double first_gain = 0.0, cur_gain = 0.0;
     unsigned first_key = 0, cur_key = 0;
-    I64Pair first_left{0, 0}, cur_left{0, 0};
-    auto put_left = [&](int j, const I64Pair& left) {
-      if (kLeft && a.left != nullptr) a.left[static_cast<int64_t>(j) * a.F + f] = left;
+    uint2 first_left = make_uint2(0, 0), cur_left = make_uint2(0, 0);  // with `down` added
+    auto put_left = [&](int j, const uint2& left) {
+      if (kLeft && a.left != nullptr)
+        a.left[static_cast<int64_t>(j) * a.F + f] =
+          I64Pair{static_cast<int64_t>(left.x) - static_cast<int64_t>(down_g), static_cast<int64_t>(left.y) - static_cast<int64_t>(down_h)};
     };
-    auto node_at = [&](int j, I64Pair& ns, I64Pair& base, double& parent) {
+    // what a running sum is added to (taken from) for the sum left (right) of it in node j, with `down` added
+    auto node_at = [&](int j, uint2& to_left, uint2& to_right, double& parent) {
+      I64Pair ns, base;
       if constexpr (kStaged) {
         ns     = s_ns[j];
         base   = s_base[j];
@@ -839,20 +852,18 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
         base   = st.base[a.level_first + j];
         parent = leaf_gain(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, a.l1, reg);
       }
+      to_left  = make_uint2(down_g - static_cast<uint32_t>(base.grad), down_h - static_cast<uint32_t>(base.hess));
+      to_right = make_uint2(down_g + static_cast<uint32_t>(base.grad) + static_cast<uint32_t>(ns.grad),
+                            down_h + static_cast<uint32_t>(base.hess) + static_cast<uint32_t>(ns.hess));
     };
+    auto grads  = [&](uint32_t v) { return static_cast<double>(v) - from_g; };
+    auto hesses = [&](uint32_t v) { return static_cast<double>(v) - from_h; };
     // calculate_gain with the parent's term formed once per node
     const bool plain = plain_quotients(a.l1, inv_g, inv_h, reg);
-    auto gain_of = [&](const I64Pair& ls, const I64Pair& rs, double parent) {
-      if (plain) {
-        const double lg = static_cast<double>(ls.grad) * inv_g, rg = static_cast<double>(rs.grad) * inv_g;
-        return 0.0 + ((0.5 * (quotient_plain(lg * lg, static_cast<double>(ls.hess) * inv_h + reg) +
-                              quotient_plain(rg * rg, static_cast<double>(rs.hess) * inv_h + reg) - parent)) -
-                      a.min_split_gain);
-      }
-      return 0.0 + ((0.5 * (leaf_gain(static_cast<double>(ls.grad) * inv_g, static_cast<double>(ls.hess) * inv_h, a.l1, reg) +
-                            leaf_gain(static_cast<double>(rs.grad) * inv_g, static_cast<double>(rs.hess) * inv_h, a.l1, reg) -
-                            parent)) -
-                    a.min_split_gain);
+    auto gain_of = [&](double lg, double lh, double rg, double rh, double parent) {
+      lg *= inv_g, rg *= inv_g, lh *= inv_h, rh *= inv_h;
+      if (plain) return 0.0 + ((0.5 * (quotient_plain(lg * lg, lh + reg) + quotient_plain(rg * rg, rh + reg) - parent)) - a.min_split_gain);
+      return 0.0 + ((0.5 * (leaf_gain(lg, lh, a.l1, reg) + leaf_gain(rg, rh, a.l1, reg) - parent)) - a.min_split_gain);
     };
     auto next_node = [&](int j) {
       if (first_node == kNone) {
@@ -869,34 +880,35 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
       cur_gain = 0.0;
       cur_key  = 0;
     };
-    auto offer = [&](double gain, int e, const I64Pair& left) {
+    auto offer = [&](double gain, int e, const uint2& left) {
       if (gain >= cur_gain) {
         const unsigned key = tie_key(rp, bin[e], bin[e + 1]);
         if constexpr (kLeft) {
           const bool better = gain > cur_gain || key > cur_key;
-          cur_left.grad     = better ? left.grad : cur_left.grad;
-          cur_left.hess     = better ? left.hess : cur_left.hess;
+          cur_left.x        = better ? left.x : cur_left.x;
+          cur_left.y        = better ? left.y : cur_left.y;
         }
         cur_key  = gain > cur_gain ? key : max(cur_key, key);
         cur_gain = gain;
       }
     };
     if constexpr (kG == 1) {
-      I64Pair ns{0, 0}, base{0, 0};
+      uint2 to_left = make_uint2(0, 0), to_right = make_uint2(0, 0);
       double parent = 0.0;
 #pragma unroll
       for (int e = 0; e < kE; e++) {
         const int2 v = pair_at(e);
-        run.grad += v.x;
-        run.hess += v.y;
+        run.x += static_cast<uint32_t>(v.x);
+        run.y += static_cast<uint32_t>(v.y);
         if ((ends >> e) & 1u) {
           if (node[e] != cur) {
             next_node(node[e]);
-            node_at(cur, ns, base, parent);
+            node_at(cur, to_left, to_right, parent);
           }
-          const I64Pair ls{run.grad - base.grad, run.hess - base.hess}, rs{ns.grad - ls.grad, ns.hess - ls.hess};
-          if (ls.hess > 0 && rs.hess > 0) {
-            const double gain = gain_of(ls, rs, parent);
+          const uint2 ls  = make_uint2(run.x + to_left.x, run.y + to_left.y);
+          const double lh = hesses(ls.y), rh = hesses(to_right.y - run.y);
+          if (lh > 0 && rh > 0) {
+            const double gain = gain_of(grads(ls.x), lh, grads(to_right.x - run.x), rh, parent);
             if (gain > 0) offer(gain, e, ls);
           }
         }
@@ -906,18 +918,19 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
       for (int e0 = 0; e0 < kE; e0 += kG) {
         double gain[kG];
         bool wanted[kG];
-        I64Pair left_of[kG];
+        uint2 left_of[kG];
 #pragma unroll
         for (int u = 0; u < kG; u++) {
           const int e = e0 + u;
-          run.grad += q[e].x;
-          run.hess += q[e].y;
-          I64Pair ns, base;
+          run.x += static_cast<uint32_t>(q[e].x);
+          run.y += static_cast<uint32_t>(q[e].y);
+          uint2 to_left, to_right;
           double parent;
-          node_at(node[e] != kNone ? node[e] : 0, ns, base, parent);
-          const I64Pair ls{run.grad - base.grad, run.hess - base.hess}, rs{ns.grad - ls.grad, ns.hess - ls.hess};
-          wanted[u] = ((ends >> e) & 1u) != 0 && ls.hess > 0 && rs.hess > 0;
-          gain[u]    = gain_of(ls, rs, parent);
+          node_at(node[e] != kNone ? node[e] : 0, to_left, to_right, parent);
+          const uint2 ls  = make_uint2(run.x + to_left.x, run.y + to_left.y);
+          const double lh = hesses(ls.y), rh = hesses(to_right.y - run.y);
+          wanted[u]  = ((ends >> e) & 1u) != 0 && lh > 0 && rh > 0;
+          gain[u]    = gain_of(grads(ls.x), lh, grads(to_right.x - run.x), rh, parent);
           left_of[u] = ls;
         }
         // (a node without a candidate here is none of those that the thread has to report)
