@@ -988,14 +988,17 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
     for (int e = 0; e < kE; e++) gain[e] = 0.0;
     // The pairs of the next output, and what the nodes have of it, are on their way while this one's sums and gains are formed, and lie in the
     // LDS when they are asked for: gathered from the L2 place by place, with the nodes' sums behind the places' sums, they were two latencies
-    // an output: 590 x 118 with 8 outputs, depth 9, 24.7 us a launch, now 20.5; 7000 x 300 with 2, depth 8, 96 and 83. kStaged: the nodes' sums, bases and terms of the gain, a thread each, those of one
+    // an output: 590 x 118 with 8 outputs, depth 9, 24.7 us a launch, and 20.5; 7000 x 300 with 2, depth 8, 96 and 83 (with
+    // sums in 32 bits and plain quotients 17.1 and 65). kStaged: the nodes' sums, bases and terms of the gain, a thread each, those of one
     // output beside those of the next.
     I64Pair* const s_of_k    = reinterpret_cast<I64Pair*>(smem_raw + small_scan_use(a.N, a.n_nodes));  // [2][2][n_nodes]
     double* const s_parent_k = reinterpret_cast<double*>(s_of_k + 4 * a.n_nodes);                      // [2][n_nodes]
     const int64_t own_at     = static_cast<int64_t>(a.level_first + min(tid, a.n_nodes - 1)) * a.K;
     int2 q_next[kE];
-    I64Pair ns_next{0, 0}, base_next{0, 0};
+    I64Pair ns_next{0, 0}, base_next{0, 0}, all_next{0, 0};
+    const bool plain = plain_quotients(a.l1, inv_g, inv_h, reg);
     auto fetch = [&](int k) {
+      all_next = st.node_sums[k];
 #pragma unroll
       for (int u = 0; u < kE; u++) q_next[u] = st.qgh[min(tid + u * kT, a.N - 1) * a.K + k];
       if constexpr (kStaged) {
@@ -1019,26 +1022,31 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
           parent_of_k[tid] = leaf_gain(static_cast<double>(ns_next.grad) * inv_g, static_cast<double>(ns_next.hess) * inv_h, a.l1, reg);
         }
       }
+      // (sums in their lower 32 bits, as with one output)
+      const int64_t most   = (int64_t(1) << 31) + a.N + 1024;
+      const uint32_t down_g = static_cast<uint32_t>((most - all_next.grad) / 2 + 1), down_h = static_cast<uint32_t>((most - all_next.hess) / 2 + 1);
+      const double from_g = static_cast<double>(down_g), from_h = static_cast<double>(down_h);
       if (k + 1 < a.K) fetch(k + 1);
       __syncthreads();
       int2 q[kE];
-      I64Pair sum{0, 0};
+      uint2 sum = make_uint2(0, 0);
 #pragma unroll
       for (int e = 0; e < kE; e++) {
         q[e] = i0 + e < a.N ? s_q[entry[e] & 0xffff] : make_int2(0, 0);
-        sum.grad += q[e].x;
-        sum.hess += q[e].y;
+        sum.x += static_cast<uint32_t>(q[e].x);
+        sum.y += static_cast<uint32_t>(q[e].y);
       }
-      const int64_t ig = wave_inclusive_sum(sum.grad), ih = wave_inclusive_sum(sum.hess);
-      I64Pair* const s_tot = s_pair[k & 1];
-      if (lane == 63) s_tot[wave] = I64Pair{ig, ih};
+      const uint32_t ig = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum.x)));
+      const uint32_t ih = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum.y)));
+      uint2* const s_tot = reinterpret_cast<uint2*>(s_pair[k & 1]);
+      if (lane == 63) s_tot[wave] = make_uint2(ig, ih);
       __syncthreads();
-      I64Pair before{ig - sum.grad, ih - sum.hess};
+      uint2 before = make_uint2(ig - sum.x, ih - sum.y);
       for (int w = 0; w < kT / 64; w++) {
-        before.grad += w < wave ? s_tot[w].grad : 0;
-        before.hess += w < wave ? s_tot[w].hess : 0;
+        before.x += w < wave ? s_tot[w].x : 0;
+        before.y += w < wave ? s_tot[w].y : 0;
       }
-      auto offer = [&](int e, int j) {
+      auto offer = [&](int e, int j, auto plains) {
         I64Pair ns, base;
         double parent;
         if constexpr (kStaged) {
@@ -1051,25 +1059,36 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
           base   = st.base[at];
           parent = leaf_gain_select(static_cast<double>(ns.grad) * inv_g, static_cast<double>(ns.hess) * inv_h, a.l1, reg);
         }
-        const I64Pair ls{before.grad - base.grad, before.hess - base.hess}, rs{ns.grad - ls.grad, ns.hess - ls.hess};
+        auto quotient = [&](double grad, double hess) {
+          if constexpr (decltype(plains)::value)
+            return quotient_plain(grad * grad, hess + reg);
+          else
+            return leaf_gain_select(grad, hess, a.l1, reg);
+        };
+        const uint32_t g = before.x - static_cast<uint32_t>(base.grad), h = before.y - static_cast<uint32_t>(base.hess);
+        const double lg = static_cast<double>(g + down_g) - from_g, rg = static_cast<double>(static_cast<uint32_t>(ns.grad) - g + down_g) - from_g;
+        const double lh = static_cast<double>(h + down_h) - from_h, rh = static_cast<double>(static_cast<uint32_t>(ns.hess) - h + down_h) - from_h;
         // build_tree.cu:727-730: one output without a valid split on this bin voids the bin
-        dead |= ls.hess <= 0 || rs.hess <= 0 ? 1u << e : 0u;
-        gain[e] += (0.5 * (leaf_gain_select(static_cast<double>(ls.grad) * inv_g, static_cast<double>(ls.hess) * inv_h, a.l1, reg) +
-                           leaf_gain_select(static_cast<double>(rs.grad) * inv_g, static_cast<double>(rs.hess) * inv_h, a.l1, reg) -
-                           parent)) -
-                   a.min_split_gain;
+        dead |= lh <= 0 || rh <= 0 ? 1u << e : 0u;
+        gain[e] += (0.5 * (quotient(lg * inv_g, lh * inv_h) + quotient(rg * inv_g, rh * inv_h) - parent)) - a.min_split_gain;
       };
       // a few waves: the places' quotients side by side, without branches (a place whose bin does not end there has no say below);
       // sixteen of them hide each other's chains, and only the places that have a say are worth the time
+      auto offer_all = [&](auto plains) {
 #pragma unroll
-      for (int e = 0; e < kE; e++) {
-        before.grad += q[e].x;
-        before.hess += q[e].y;
-        if constexpr (kT < 1024)
-          offer(e, node[e] != kNone ? node[e] : 0);
-        else if (((ends & ~dead) >> e) & 1u)
-          offer(e, node[e]);
-      }
+        for (int e = 0; e < kE; e++) {
+          before.x += static_cast<uint32_t>(q[e].x);
+          before.y += static_cast<uint32_t>(q[e].y);
+          if constexpr (kT < 1024)
+            offer(e, node[e] != kNone ? node[e] : 0, plains);
+          else if (((ends & ~dead) >> e) & 1u)
+            offer(e, node[e], plains);
+        }
+      };
+      if (plain)
+        offer_all(std::true_type{});
+      else
+        offer_all(std::false_type{});
     }
     ends &= ~dead;
     // best gain per node: a thread's runs of one node first, then, where a whole wave lies in one

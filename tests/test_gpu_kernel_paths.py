@@ -913,3 +913,7 @@ def test_scanned_levels_in_32_bits(n, f, k, s, kind):
         g = -np.abs(g)
     gr, cr = gu.both(X, g, h, max_depth=6, split_samples=s, seed=5, **kw)
     gu.assert_tree_parity(gr, cr)
+    # and unobserved, by the builders for few and for medium rows where they take it
+    from lbtree import ops
+    got = ops.build_tree(*(torch.from_numpy(v).cuda() for v in (X, g, h)), max_depth=6, split_samples=s, seed=5, row_leaf=True, **kw)
+    _assert_tree(got, cr)
