@@ -402,7 +402,8 @@ struct HistSetup {
   int partial_slots = 0;
   int partial_stride = 0;
   // bin cache: written by the root binning pass and read by the histogram kernel of every
-  // level instead of X; stored histogram group by histogram group as [group][row][record]
+  // level instead of X; a row's records lie side by side, [row][histogram group][record], in a plane per search group of the
+  // pass where its groups are whole histogram groups (RecInfo)
   void* binned         = nullptr;  // null: cache off
   size_t binned_capacity = 0;      // bytes available at `binned`
   int bin_bytes        = 0;        // 1 or 2
