@@ -299,16 +299,8 @@ __global__ void __launch_bounds__(kQuantiseThreads)
   unsigned bad = 0;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kQuantiseThreads;
   auto round_row = [&](int64_t row, double grad, double hess) {
-    uint32_t x  = minstd_seed(static_cast<uint32_t>(
-      static_cast<uint64_t>(gpair_seed(seed, row + row_offset, static_cast<int64_t>(k)))));
-    double scaled_grad    = grad * sg;
-    double scaled_hess    = hess * sh;
-    double grad_remainder = scaled_grad - floor(scaled_grad);
-    double hess_remainder = scaled_hess - floor(scaled_hess);
-    x = minstd_next(x);
-    int64_t qg = static_cast<int64_t>(floor(scaled_grad) + static_cast<double>(uniform01(x) < grad_remainder));
-    x = minstd_next(x);
-    int64_t qh = static_cast<int64_t>(floor(scaled_hess) + static_cast<double>(uniform01(x) < hess_remainder));
+    int64_t qg, qh;
+    quantise_pair(grad, hess, sg, sh, seed, row + row_offset, static_cast<int64_t>(k), &qg, &qh);
     bad |= qg > 2147483647LL || qg < -2147483647LL || qh > 2147483647LL || qh < -2147483647LL ? kQuantTooLarge : 0;
     bad |= qh <= 0 && (qg != 0 || qh != 0) ? kQuantHessNotPositive : 0;
     q_out[row * K + k] = make_int2(static_cast<int>(qg), static_cast<int>(qh));
@@ -364,41 +356,32 @@ __global__ void __launch_bounds__(kQuantiseThreads)
 // The same for several outputs per row: the (row, output) entries are walked in memory order
 // (the kernel above, launched once per output, would read every line K times). The grid stride
 // is a multiple of K, so a thread stays with one output and sums in registers; the outputs'
-// sums of a workgroup meet in LDS.
+// sums of a workgroup meet in LDS. As above few workgroups, whose additions to the same 2 K words take turns, and loads of the next turns
+// together: 300,000 rows of 16 outputs 102 -> 37 us, 2,000,000 of 8 110 -> 98.
 constexpr int kQuantiseFlatMaxK = 2048;
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kQuantiseThreads)
   quantise_flat_kernel(const double* g, const double* h, int64_t n_rows, int K, int64_t row_offset, int64_t seed,
                        const double* scales, int2* q_out, I64Pair* node_sums, unsigned long long* qstats)
 {
   extern __shared__ unsigned long long s_sums[];  // [K] grad, [K] hess
   __shared__ unsigned long long s_max;
   __shared__ unsigned s_bad;
-  for (int i = threadIdx.x; i < 2 * K; i += kThreads) s_sums[i] = 0;
+  for (int i = threadIdx.x; i < 2 * K; i += kQuantiseThreads) s_sums[i] = 0;
   if (threadIdx.x == 0) s_max = s_bad = 0;
   __syncthreads();
   const double sg = scales[0], sh = scales[1];
   const int64_t n       = n_rows * K;
-  const int64_t threads = static_cast<int64_t>(gridDim.x) * kThreads;
+  const int64_t threads = static_cast<int64_t>(gridDim.x) * kQuantiseThreads;
   const int64_t stride  = threads / K * K;  // the launch makes sure that threads >= K
-  const int64_t first   = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x;
+  const int64_t first   = blockIdx.x * static_cast<int64_t>(kQuantiseThreads) + threadIdx.x;
   const int k           = static_cast<int>(first % K);
   int64_t sum_g = 0, sum_h = 0;
   unsigned long long mx = 0;
   unsigned bad = 0;
   if (first < stride) {
-    for (int64_t e = first; e < n; e += stride) {
-      const int64_t row = e / K;
-      double grad = g[e], hess = h[e];
-      uint32_t x  = minstd_seed(static_cast<uint32_t>(
-        static_cast<uint64_t>(gpair_seed(seed, row + row_offset, static_cast<int64_t>(k)))));
-      double scaled_grad    = grad * sg;
-      double scaled_hess    = hess * sh;
-      double grad_remainder = scaled_grad - floor(scaled_grad);
-      double hess_remainder = scaled_hess - floor(scaled_hess);
-      x = minstd_next(x);
-      int64_t qg = static_cast<int64_t>(floor(scaled_grad) + static_cast<double>(uniform01(x) < grad_remainder));
-      x = minstd_next(x);
-      int64_t qh = static_cast<int64_t>(floor(scaled_hess) + static_cast<double>(uniform01(x) < hess_remainder));
+    auto round_entry = [&](int64_t e, int64_t row, double grad, double hess) {
+      int64_t qg, qh;
+      quantise_pair(grad, hess, sg, sh, seed, row + row_offset, static_cast<int64_t>(k), &qg, &qh);
       bad |= qg > 2147483647LL || qg < -2147483647LL || qh > 2147483647LL || qh < -2147483647LL ? kQuantTooLarge : 0;
       bad |= qh <= 0 && (qg != 0 || qh != 0) ? kQuantHessNotPositive : 0;
       q_out[e] = make_int2(static_cast<int>(qg), static_cast<int>(qh));
@@ -408,6 +391,20 @@ __global__ void __launch_bounds__(kThreads)
       mx = ah > mx ? ah : mx;
       sum_g += qg;
       sum_h += qh;
+    };
+    const int64_t step = stride / K;  // rows that a turn moves on
+    int64_t row        = first / K;
+    for (int64_t e = first; e < n; e += kQuantiseRows * stride, row += kQuantiseRows * step) {
+      double grad[kQuantiseRows], hess[kQuantiseRows];
+#pragma unroll
+      for (int u = 0; u < kQuantiseRows; u++) {
+        const int64_t at = e + u * stride < n ? e + u * stride : e;
+        grad[u] = g[at];
+        hess[u] = h[at];
+      }
+#pragma unroll
+      for (int u = 0; u < kQuantiseRows; u++)
+        if (e + u * stride < n) round_entry(e + u * stride, row + u * step, grad[u], hess[u]);
     }
     atomicAdd(&s_sums[k], static_cast<unsigned long long>(sum_g));
     atomicAdd(&s_sums[K + k], static_cast<unsigned long long>(sum_h));
@@ -415,7 +412,7 @@ __global__ void __launch_bounds__(kThreads)
   }
   if (bad != 0) atomicOr(&s_bad, bad);
   __syncthreads();
-  for (int i = threadIdx.x; i < K; i += kThreads) {
+  for (int i = threadIdx.x; i < K; i += kQuantiseThreads) {
     const unsigned long long vg = s_sums[i], vh = s_sums[K + i];
     if (vg != 0) atomic_add_i64(&node_sums[i].grad, static_cast<int64_t>(vg));
     if (vh != 0) atomic_add_i64(&node_sums[i].hess, static_cast<int64_t>(vh));
@@ -1863,9 +1860,8 @@ int run_quantiser(hipStream_t stream, const double* g, const double* h, int64_t 
   }
   scales_kernel<<<1, 64, 0, stream>>>(in_a, in_b, scales, qstats);
   if (K > 1 && K <= kQuantiseFlatMaxK) {
-    const unsigned gx =
-      std::max<unsigned>(std::min<unsigned>(blocks(N * K, kThreads), 2048u), blocks(K, kThreads));
-    quantise_flat_kernel<<<gx, kThreads, 2 * K * sizeof(unsigned long long), stream>>>(
+    const unsigned gx = std::max<unsigned>(std::min<unsigned>(blocks(N * K, kQuantiseThreads), kQuantiseGroups), blocks(K, kQuantiseThreads));
+    quantise_flat_kernel<<<gx, kQuantiseThreads, 2 * K * sizeof(unsigned long long), stream>>>(
       g, h, N, K, row_offset, static_cast<int64_t>(seed), scales, qgh, root_sums, qstats);
   } else {
     dim3 grid(std::min<unsigned>(blocks(N, kQuantiseThreads), kQuantiseGroups), K);

@@ -358,6 +358,13 @@ __device__ __forceinline__ int feature_proposals(const T* __restrict__ X, const 
 }
 
 // One stochastic rounding of a (grad, hess) pair (build_tree.cu:112-129).
+// A whole number as 64 bits: one conversion where it fits 32, as all but a value that ends the call does.
+__device__ __forceinline__ int64_t whole_to_i64(double v)
+{
+  if (__builtin_expect(fabs(v) <= 2147483647.0, 1)) return static_cast<int32_t>(v);
+  asm volatile("");  // (a branch: the general conversion is eight instructions)
+  return static_cast<int64_t>(v);
+}
 __device__ __forceinline__ void quantise_pair(double grad, double hess, double sg, double sh, int64_t seed, int64_t row,
                                               int64_t k, int64_t* qg, int64_t* qh)
 {
@@ -367,9 +374,9 @@ __device__ __forceinline__ void quantise_pair(double grad, double hess, double s
   const double grad_remainder = scaled_grad - floor(scaled_grad);
   const double hess_remainder = scaled_hess - floor(scaled_hess);
   x   = minstd_next(x);
-  *qg = static_cast<int64_t>(floor(scaled_grad) + static_cast<double>(uniform01(x) < grad_remainder));
+  *qg = whole_to_i64(floor(scaled_grad) + static_cast<double>(uniform01(x) < grad_remainder));
   x   = minstd_next(x);
-  *qh = static_cast<int64_t>(floor(scaled_hess) + static_cast<double>(uniform01(x) < hess_remainder));
+  *qh = whole_to_i64(floor(scaled_hess) + static_cast<double>(uniform01(x) < hess_remainder));
 }
 
 // ---- bin search (see build_cells_kernel for the table)

@@ -214,7 +214,11 @@ __host__ __device__ inline uint32_t minstd_discard(uint32_t x, uint64_t z)
 // thrust::uniform_real_distribution<double>(0,1) on one raw draw.
 __host__ __device__ inline double uniform01(uint32_t draw)
 {
-  return static_cast<double>(draw - 1u) / 2147483646.0;
+  // the quotient by 2147483646, correctly rounded: the product with its reciprocal and the remainder's correction (compared with the
+  // division for every draw; eight instructions less)
+  constexpr double d = 2147483646.0, r = 1.0 / d;
+  const double n = static_cast<double>(draw - 1u), q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
 }
 
 // fmix64 on a signed 64-bit value: arithmetic right shifts, wrapping multiplies
