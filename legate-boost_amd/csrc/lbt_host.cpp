@@ -16,6 +16,7 @@
 #include <cstdint>
 #include <cstring>
 #include <exception>
+#include <vector>
 
 namespace {
 
@@ -87,9 +88,20 @@ PyObject* tree_arrays(PyObject*, PyObject* args)
   return PyTuple_Pack(4, a.out[0], a.out[1], a.out[2], a.out[3]);
 }
 
+// References that are given back when they are left
+struct Held {
+  std::vector<PyObject*> objects;
+  ~Held()
+  {
+    for (PyObject* o : objects) Py_DECREF(o);
+  }
+};
+
 // model_arrays(models, type, names, n_outputs): the same for a list or tuple of objects of `type` whose three attributes `names` are the
 // arrays, and a fifth value: a list of the arrays, which keeps the addresses valid. (100 trees, 1000 rows: a call takes 24 us; through the tuples
-// above, gathered in Python, 29.)
+// above, gathered in Python, 29.) An attribute may be code that changes the list or looks at what the collector knows: None where the
+// list has another length at the end, and the arrays are no list before they are complete. What such code raises the caller meets
+// again in Python, but for what is no Exception (an interrupt): that is passed on.
 PyObject* model_arrays(PyObject*, PyObject* args)
 {
   PyObject *models, *type, *names;
@@ -100,30 +112,22 @@ PyObject* model_arrays(PyObject*, PyObject* args)
     Py_RETURN_NONE;
   const Py_ssize_t n = PySequence_Fast_GET_SIZE(models);
   Arrays a;
-  PyObject* keep = PyList_New(3 * n);
-  if (keep == nullptr || !a.open(n)) {
-    Py_XDECREF(keep);
-    return nullptr;
-  }
+  if (!a.open(n)) return nullptr;
+  Held keep;
   bool plain = true;
   try {
+    keep.objects.reserve(3 * n);
     for (Py_ssize_t t = 0; t < n && plain; t++) {
-      // (an attribute may be code that changes the list)
-      if (t >= PySequence_Fast_GET_SIZE(models)) {
-        plain = false;
-        break;
-      }
+      plain = t < PySequence_Fast_GET_SIZE(models) &&
+              PyObject_TypeCheck(PySequence_Fast_GET_ITEM(models, t), reinterpret_cast<PyTypeObject*>(type));
+      if (!plain) break;
       PyObject* model = PySequence_Fast_GET_ITEM(models, t);
-      if (!PyObject_TypeCheck(model, reinterpret_cast<PyTypeObject*>(type))) {
-        plain = false;
-        break;
-      }
       Py_INCREF(model);
       PyObject* got[3] = {};
       for (int i = 0; i < 3 && plain; i++) {
         got[i] = PyObject_GetAttr(model, PyTuple_GET_ITEM(names, i));
         plain  = got[i] != nullptr;
-        if (plain) PyList_SET_ITEM(keep, 3 * t + i, got[i]);
+        if (plain) keep.objects.push_back(got[i]);
       }
       Py_DECREF(model);
       plain = plain && a.put(t, got[0], got[1], got[2], n_outputs);
@@ -131,15 +135,17 @@ PyObject* model_arrays(PyObject*, PyObject* args)
   } catch (const std::exception&) {
     plain = false;
   }
-  PyObject* result = nullptr;
-  if (plain) {
-    result = PyTuple_Pack(5, a.out[0], a.out[1], a.out[2], a.out[3], keep);
-  } else {
-    PyErr_Clear();  // whatever it is, the caller meets it again in Python
-    Py_INCREF(Py_None);
-    result = Py_None;
+  if (PyErr_Occurred()) {
+    if (!PyErr_ExceptionMatches(PyExc_Exception)) return nullptr;
+    PyErr_Clear();
   }
-  Py_DECREF(keep);  // (places that were not reached are empty: a list may be dropped like that)
+  if (!plain || PySequence_Fast_GET_SIZE(models) != n) Py_RETURN_NONE;
+  PyObject* list = PyList_New(3 * n);
+  if (list == nullptr) return nullptr;
+  for (Py_ssize_t i = 0; i < 3 * n; i++) PyList_SET_ITEM(list, i, keep.objects[static_cast<size_t>(i)]);
+  keep.objects.clear();  // (the list has the references)
+  PyObject* result = PyTuple_Pack(5, a.out[0], a.out[1], a.out[2], a.out[3], list);
+  Py_DECREF(list);
   return result;
 }
 

@@ -272,7 +272,7 @@ def predict_models(X, models, kind, n_outputs, init=None):
     if arrays is None:
         assert all(isinstance(m, kind) for m in models)
         return predict(X, [(m.leaf_value, m.feature, m.split_value) for m in models], n_outputs, init=init)
-    return _predict(_check_x(X), len(models), arrays[:4] + (None, arrays[4]), n_outputs, True, init)
+    return _predict(_check_x(X), len(arrays[3]) // 4, arrays[:4] + (None, arrays[4]), n_outputs, True, init)
 
 
 def _predict(X, nt, arrays, n_outputs, tiled, init):

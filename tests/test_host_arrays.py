@@ -131,3 +131,69 @@ def test_a_packed_prediction_in_native_code_and_through_python(monkeypatch, dtyp
         assert str(e.value) == told
     with pytest.raises(Exception):
         torch.func.vmap(packed.predict)(wide[:4, :5].reshape(2, 2, 5))
+
+
+def test_code_behind_an_attribute_of_a_model():
+    """It may change the list of models, raise, or look at every list there is: the caller then looks closer, and no list is seen
+    before it is complete."""
+    import gc
+
+    take = _lib._host.model_arrays
+    names = ("a", "b", "c")
+    seen = []
+
+    class Model:
+        def __init__(self, act):
+            self.act = act
+
+        @property
+        def a(self):
+            self.act()
+            return 1
+
+    def interrupted():
+        raise KeyboardInterrupt
+
+    def wrong():
+        raise ValueError
+
+    def look():
+        # (the size alone: an element that is not there yet could not be touched)
+        seen.extend(len(o) for o in gc.get_objects() if type(o) is list and len(o) == 3 * 1237)
+
+    with pytest.raises(KeyboardInterrupt):
+        take([Model(interrupted)], Model, names, 1)
+    assert take([Model(wrong)], Model, names, 1) is None
+    models = []
+    models.extend(Model(models.clear) for _ in range(3))
+    assert take(models, Model, names, 1) is None and models == []
+    assert take([Model(look)] * 1237, Model, names, 1) is None and seen == []
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", ["append", "pop"])
+def test_a_list_of_models_that_changes_while_it_is_read(change):
+    """The library is told as many trees as there are addresses of."""
+    rs = np.random.RandomState(3)
+    arrays = (torch.from_numpy(rs.randn(15, 2)).cuda(), torch.from_numpy(np.r_[rs.randint(0, 5, 7), -np.ones(8)].astype(np.int32)).cuda(),
+              torch.from_numpy(rs.rand(15)).cuda())
+
+    class Model:
+        leaf_value, feature = arrays[:2]
+        act = None
+
+        @property
+        def split_value(self):
+            if self.act is not None:
+                act, self.act = self.act, None
+                act()
+            return arrays[2]
+
+    models = [Model() for _ in range(20)]
+    first = models[0]
+    first.act = (lambda: models.append(Model())) if change == "append" else models.pop
+    assert _lib._host.model_arrays(models, Model, ops._ARRAYS, 2) is None
+    X = torch.rand(300, 5).cuda()
+    first.act = (lambda: models.append(Model())) if change == "append" else models.pop
+    got = ops.predict_models(X, models, Model, 2)
+    assert torch.equal(got, ops.predict(X, [arrays] * len(models), 2))
