@@ -149,6 +149,7 @@ class Tree(BaseModel):
 
     @staticmethod
     def batch_predict(models: Sequence[BaseModel], X):
+        assert not models or isinstance(models[0], Tree)  # (the others: predict_models)
         n_outputs = cast(Tree, models[0]).leaf_value.shape[1]
         return ops.predict_models(X, models, Tree, n_outputs)
 

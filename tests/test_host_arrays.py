@@ -197,3 +197,15 @@ def test_a_list_of_models_that_changes_while_it_is_read(change):
     first.act = (lambda: models.append(Model())) if change == "append" else models.pop
     got = ops.predict_models(X, models, Model, 2)
     assert torch.equal(got, ops.predict(X, [arrays] * len(models), 2))
+
+
+def test_models_of_which_the_first_is_no_tree_are_refused():
+    from lbtree.models import Tree
+
+    class Other:
+        pass
+
+    with pytest.raises(AssertionError):
+        Tree.batch_predict([Other()], torch.zeros(2, 2))
+    with pytest.raises(IndexError):
+        Tree.batch_predict([], torch.zeros(2, 2))
