@@ -664,8 +664,8 @@ __global__ void __launch_bounds__(kW == 1 ? kThreads : kW * 64)
         g += b < fe ? static_cast<uint32_t>(v.grad) : 0u;
         h += b < fe ? static_cast<uint32_t>(v.hess) : 0u;
       }
-      const int all_g = wave_inclusive_sum32(static_cast<int>(g)), all_h = wave_inclusive_sum32(static_cast<int>(h));
-      if (lane == 63) s_total[wave][k] = make_uint2(static_cast<uint32_t>(all_g), static_cast<uint32_t>(all_h));
+      const uint32_t all_g = wave_inclusive_sum32(g), all_h = wave_inclusive_sum32(h);
+      if (lane == 63) s_total[wave][k] = make_uint2(all_g, all_h);
     }
     __syncthreads();
     if (lane < K) {
@@ -712,15 +712,14 @@ __global__ void __launch_bounds__(kW == 1 ? kThreads : kW * 64)
       double lg, lh;  // what lies left of the bin
       if ((scans >> k & 1) != 0) {
         const uint32_t raw_g = static_cast<uint32_t>(val.grad), raw_h = static_cast<uint32_t>(val.hess);
-        const uint32_t to_g = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(raw_g)) + __builtin_amdgcn_readlane(agg_g, k));
-        const uint32_t to_h = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(raw_h)) + __builtin_amdgcn_readlane(agg_h, k));
-        const int tile_g = __builtin_amdgcn_readlane(to_g, 63), tile_h = __builtin_amdgcn_readlane(to_h, 63);
+        const uint32_t to_g = wave_inclusive_sum32(raw_g) + wave_read_lane32(agg_g, k);
+        const uint32_t to_h = wave_inclusive_sum32(raw_h) + wave_read_lane32(agg_h, k);
+        const uint32_t tile_g = wave_read_lane32(to_g, 63), tile_h = wave_read_lane32(to_h, 63);
         if (lane == k) {
-          agg_g = static_cast<uint32_t>(tile_g);
-          agg_h = static_cast<uint32_t>(tile_h);
+          agg_g = tile_g;
+          agg_h = tile_h;
         }
-        const uint32_t from_g = static_cast<uint32_t>(__builtin_amdgcn_readlane(down_g, k));
-        const uint32_t from_h = static_cast<uint32_t>(__builtin_amdgcn_readlane(down_h, k));
+        const uint32_t from_g = wave_read_lane32(down_g, k), from_h = wave_read_lane32(down_h, k);
         lg = static_cast<double>(to_g + from_g) - static_cast<double>(from_g);
         lh = static_cast<double>(to_h + from_h) - static_cast<double>(from_h);
         // the reference skips the store when the running sum is not positive

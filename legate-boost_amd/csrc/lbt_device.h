@@ -72,6 +72,11 @@ __device__ __forceinline__ int64_t wave_read_lane(int64_t v, int src)
   return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+__device__ __forceinline__ uint32_t wave_read_lane32(uint32_t v, int src)
+{
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), src));
+}
+
 __device__ __forceinline__ double wave_read_lane_f64(double v, int src)
 {
   return __longlong_as_double(wave_read_lane(static_cast<int64_t>(__double_as_longlong(v)), src));
@@ -134,13 +139,13 @@ __device__ inline void add_gain(double& gain, bool& dead, const I64Pair& ls, con
                          min_split_gain);
 }
 
-// Inclusive sums over a wave, 32 bits (see wave_inclusive_sum)
+// Inclusive sums over a wave modulo 2^32 (see wave_inclusive_sum): the lower halves of longer sums wrap here
 template <int kCtrl, int kRowMask>
-__device__ __forceinline__ int dpp_take32(int v)
+__device__ __forceinline__ uint32_t dpp_take32(uint32_t v)
 {
-  return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xf, true);
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, kRowMask, 0xf, true));
 }
-__device__ __forceinline__ int wave_inclusive_sum32(int v)
+__device__ __forceinline__ uint32_t wave_inclusive_sum32(uint32_t v)
 {
   v += dpp_take32<0x111, 0xf>(v);
   v += dpp_take32<0x112, 0xf>(v);
@@ -241,7 +246,7 @@ template <int kT>
 __device__ __forceinline__ int block_exclusive_sum32(int v, int* s_wave)
 {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int incl = wave_inclusive_sum32(v);
+  const int incl = static_cast<int>(wave_inclusive_sum32(static_cast<uint32_t>(v)));
   if (lane == 63) s_wave[wave] = incl;
   __syncthreads();
   int before = 0;

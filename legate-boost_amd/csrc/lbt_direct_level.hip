@@ -104,8 +104,8 @@ __device__ __forceinline__ void add_rows(const DirectLevel& a, const RecInfo& ri
 // are summed on their own, six additions each (64 bits wide hipcc makes five instructions of a step).
 __device__ __forceinline__ unsigned long long wave_inclusive_halves(unsigned long long v)
 {
-  const uint32_t lo = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(static_cast<uint32_t>(v))));
-  const uint32_t hi = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(v >> 32)));
+  const uint32_t lo = wave_inclusive_sum32(static_cast<uint32_t>(v));
+  const uint32_t hi = wave_inclusive_sum32(static_cast<uint32_t>(v >> 32));
   return static_cast<unsigned long long>(hi) << 32 | lo;
 }
 
@@ -224,8 +224,8 @@ __device__ __forceinline__ Found scan_feature_estimated(const DirectLevel& a, co
 #pragma unroll
     for (int u = 0; u < kBins; u++) sum_g += g[u], sum_h += h[u];
     if (!__any(sum_h != 0)) continue;
-    const uint32_t to_g = before_g + static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum_g)));
-    const uint32_t to_h = before_h + static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum_h)));
+    const uint32_t to_g = before_g + wave_inclusive_sum32(sum_g);
+    const uint32_t to_h = before_h + wave_inclusive_sum32(sum_h);
     before_g = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(to_g), 63));
     before_h = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(to_h), 63));
     uint32_t lg = to_g - sum_g, lh = to_h - sum_h;

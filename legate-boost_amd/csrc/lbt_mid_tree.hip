@@ -762,8 +762,8 @@ __global__ void __launch_bounds__(kScan)
           add(std::integral_constant<int, 8>{});
           add(std::integral_constant<int, 1>{});
         }
-        uint32_t g = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(raw_g)));
-        uint32_t h = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(raw_h)));
+        uint32_t g = wave_inclusive_sum32(raw_g);
+        uint32_t h = wave_inclusive_sum32(raw_h);
         if (lane == 63) s_tot[k & 1][wave] = make_uint2(g, h);
         __syncthreads();
         if (base > 0) {

@@ -821,8 +821,8 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
       sum.x += static_cast<uint32_t>(v.x);
       sum.y += static_cast<uint32_t>(v.y);
     }
-    const uint32_t ig = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum.x)));
-    const uint32_t ih = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum.y)));
+    const uint32_t ig = wave_inclusive_sum32(sum.x);
+    const uint32_t ih = wave_inclusive_sum32(sum.y);
     if (lane == 63) s_sums[wave] = make_uint2(ig, ih);
     __syncthreads();
     uint2 run = make_uint2(ig - sum.x, ih - sum.y);
@@ -1036,8 +1036,8 @@ __global__ void __launch_bounds__(kT, kT == 1024 && kG == 1 && kSingle ? 8 : 1)
         sum.x += static_cast<uint32_t>(q[e].x);
         sum.y += static_cast<uint32_t>(q[e].y);
       }
-      const uint32_t ig = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum.x)));
-      const uint32_t ih = static_cast<uint32_t>(wave_inclusive_sum32(static_cast<int>(sum.y)));
+      const uint32_t ig = wave_inclusive_sum32(sum.x);
+      const uint32_t ih = wave_inclusive_sum32(sum.y);
       uint2* const s_tot = reinterpret_cast<uint2*>(s_pair[k & 1]);
       if (lane == 63) s_tot[wave] = make_uint2(ig, ih);
       __syncthreads();
@@ -1227,7 +1227,7 @@ __global__ void __launch_bounds__(kT)
     const int64_t ig = wave_inclusive_sum(sum.grad), ih = wave_inclusive_sum(sum.hess);
     if (lane == 63) s_sum[k & 1][wave] = I64Pair{ig, ih};
     if (k == 0) {
-      const int c = wave_inclusive_sum32(nl);
+      const int c = static_cast<int>(wave_inclusive_sum32(static_cast<uint32_t>(nl)));
       if (lane == 63) s_cnt[wave] = c;
     }
     __syncthreads();
