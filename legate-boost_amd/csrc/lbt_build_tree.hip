@@ -1642,7 +1642,7 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
   const size_t upload_at = ar.used;
   L.groups       = ar.take<int32_t>(F + 1);
   L.sgroups      = ar.take<int32_t>(F + 1);
-  L.bin_lanes    = ar.take<int2>(4 * static_cast<size_t>(F) + 16);
+  L.bin_lanes    = ar.take<int2>(bin_lanes_max(F));
   L.rec          = ar.take<RecInfo>(F);
   L.upload_block = L.groups;
   L.upload_bytes = ar.used - upload_at;
@@ -2776,7 +2776,7 @@ void make_hist_stage_layout(Arena& ar, HistStageLayout& L, int64_t N, int F, int
   const size_t upload_at    = ar.used;
   L.groups       = ar.take<int32_t>(F + 1);
   L.sgroups      = ar.take<int32_t>(F + 1);
-  L.bin_lanes    = ar.take<int2>(4 * static_cast<size_t>(F) + 16);
+  L.bin_lanes    = ar.take<int2>(bin_lanes_max(F));
   L.rec          = ar.take<RecInfo>(F);
   L.upload_block = L.groups;
   L.upload_bytes = ar.used - upload_at;

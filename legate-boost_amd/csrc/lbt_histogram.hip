@@ -2143,13 +2143,13 @@ int hist_launch_t(hipStream_t stream, const HistSetup& hs, const HistBatch& b, i
 
 // Packs consecutive features, `unit` at a time, into groups whose LDS need
 // (bytes_of(feature)) stays within the budget and whose rows take at most half a
-// workgroup of lanes (lane_vec features per lane); a second pass balances widths.
+// workgroup of lanes (lane_vec features per lane; the binning pass has more, see bin_lanes); a second pass balances widths.
 // more_groups: that many groups beyond the fewest the budget allows.
 template <typename BytesOf>
 size_t pack_groups(int F, int unit, int lane_vec, size_t budget, BytesOf bytes_of, std::vector<int32_t>& groups,
                    int more_groups = 0)
 {
-  const int max_lanes = kHistThreads / 2;  // at least two rows per pass
+  const int max_lanes = kHistThreads / 2;  // of features
   size_t lds          = 0;
   auto pack = [&](int target) {
     groups.assign(1, 0);
@@ -2195,7 +2195,9 @@ int rows_per_pass(const std::vector<int32_t>& groups, int vec)
 // words of the gradient pair (2: both, where a lane holds two words). A search group has the lanes of its features and, behind a
 // record's last ones, those of the rest of the record. Where a lane has less than four bytes (up to three features) there are lanes of
 // bins only {record, ...}, kind 1: a record's last one.
-// Returns the rows that a workgroup takes side by side: as many as fit, or up to an eighth fewer that are whole cache lines.
+// Returns the rows that a workgroup takes side by side: as many as fit, or up to an eighth fewer that are whole cache lines; 0 where a
+// row does not fit. (A search group has up to 512 lanes of features and up to 13 more for each of its records. The LDS holds the proposals
+// of 40,000 bins, and a record has 19,000 of them but where more records fill the chip better: seven at the most, some 600 lanes of the 1024.)
 int bin_lanes(const std::vector<int32_t>& sgroups, const std::vector<int32_t>& groups, const std::vector<RecInfo>& rec,
               int vec, int bin_bytes, std::vector<int2>& lanes)
 {
@@ -2566,6 +2568,10 @@ int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, i
     }
     up.add(hs.rec, rec.data(), sizeof(RecInfo) * rec.size());
     hs.rpp = bin_lanes(sgroups, groups, rec, vec, hs.bin_bytes, lanes);
+    if (hs.rpp < 1 || lanes.size() > bin_lanes_max(F)) {
+      set_error("a row takes %zu lanes of the binning pass", lanes.size());
+      return LBT_ERR_INVALID;
+    }
     up.add(hs.bin_lanes, lanes.data(), sizeof(int2) * lanes.size());
   }
   LBT_TRY(up.send(stream, hs.upload_block, hs.upload_bytes));

@@ -424,7 +424,7 @@ struct HistSetup {
   int64_t row_bytes      = 0;      // bytes of a row in all planes
   int pieces           = 0;        // 16-byte pieces of bins of a row's records
   int max_bins         = 0;        // bins of the widest feature
-  int2* bin_lanes      = nullptr;  // [4 * n_features + 16] lanes of a row in the binning pass (see bin_lanes)
+  int2* bin_lanes      = nullptr;  // [bin_lanes_max] lanes of a row in the binning pass (see bin_lanes)
   // feature-major copy of the bins, [feature][row], written by the root histogram launch for the
   // position updates (null: not wanted)
   void* bins_t           = nullptr;
@@ -465,6 +465,9 @@ inline int64_t bin_row_bytes_max(int n_features, int split_samples)
 
 // ... and the cache as a whole: at most a plane per feature, each starting on a multiple of kPlaneAlign bytes
 constexpr int kPlaneAlign = 128;
+// entries of HistSetup::bin_lanes: a lane per four features, up to 13 and two for each group, which has four features or more (up to
+// three features: a lane each)
+inline size_t bin_lanes_max(int n_features) { return 4 * static_cast<size_t>(n_features) + 16; }
 inline size_t bin_cache_bytes(int64_t n_rows, int n_features, int split_samples)
 {
   return static_cast<size_t>(n_rows * bin_row_bytes_max(n_features, split_samples)) + static_cast<size_t>(kPlaneAlign) * n_features;

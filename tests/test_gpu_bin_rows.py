@@ -66,6 +66,12 @@ def test_root_histogram_of_binned_rows(n, f, k, dtype, samples):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("n,f,k,dtype", [(301, 2051, 1, np.float32), (301, 4100, 1, np.float64), (301, 2048, 3, np.float32)])
+def test_rows_of_as_many_lanes_as_a_search_group_has(n, f, k, dtype):
+    """Few proposals a feature: what bounds a search group is its lanes, beside which those of the records have their place."""
+    test_root_histogram_of_binned_rows(n, f, k, dtype, 3)
+
+
 @pytest.mark.parametrize("n,f,k,dtype,samples", [
     (8447, 33, 1, np.float32, 256), (9000, 17, 1, np.float64, 300), (12345, 65, 1, np.float32, 64), (8961, 1, 2, np.float32, 16),
     (140000, 5, 1, np.float32, 512), (10241, 3, 3, np.float64, 1024),
