@@ -494,8 +494,12 @@ __global__ void __launch_bounds__(kWalkThreads, 4)
 // line, 16 bytes each: a wave's load so touches eight whole lines (a row a lane touched 64, once for each of its eight loads of 16
 // bytes: without any search 500,003 x 200 took 186 of 202 us that way). The values are turned in the LDS, and then a lane has a row and a
 // wave four or eight features, whose search it keeps in scalar registers; the rows of one feature share many of its LDS reads.
-// What bounds it is the memory: 500,003 x 200 (0.6 GB) 158 us.
+// What bounds it is the memory: 500,003 x 200 (0.6 GB) 158 us. A line whose tables are larger than the room beside the rows must not fall to a
+// search in memory: of 40 trees of depth 8 on 2,000,000 x 100 doubles with a third of the thresholds on the 16 features of one line the calls take 886 us with
+// fewer cells for that line, 1035 with its tables in the rows' place, 1726 searched in memory; with 0.6 of them 1049 (in the rows' place) and
+// 1724; without any such line 855. Floats need no more than fewer cells (2,000,000 x 200, 50 trees, 0.6 on one line: 1226 and 2181).
 constexpr int kLineRows = 256;  // rows of a turn
+constexpr int kFewCells = 64;   // cells of a feature at least
 template <typename T>
 constexpr int kLineFeatures = 128 / sizeof(T);
 template <typename T>
@@ -541,10 +545,19 @@ __global__ void __launch_bounds__(kWalkThreads, 8)
     load(begin + r, x0);
     load(begin + r + kLineRows / 2, x1);
   }
+  // Tables beside the turned rows, with fewer cells if need be; those of doubles that are larger in the place of such rows too, whose values
+  // then come straight from memory; the largest stay in memory.
+  const int table   = (words + 1) * static_cast<int>(sizeof(T));
+  int cells         = a.cells;
+  if (table + 2 * kAll * kFewCells <= a.lds_bytes)
+    while (table + 2 * kAll * cells > a.lds_bytes) cells /= 2;
+  const int needed  = table + 2 * kAll * cells;
+  const bool held   = needed <= a.lds_bytes + (sizeof(T) == 8 ? kLineStage<T> : 0);
+  const bool turned = sizeof(T) == 4 || needed <= a.lds_bytes || !held;
   T* const s_x      = reinterpret_cast<T*>(smem_raw);  // [kAll][kPitch]
-  T* const s_tab    = reinterpret_cast<T*>(smem_raw + kLineStage<T>);
-  uint16_t* s_start = reinterpret_cast<uint16_t*>(smem_raw + kLineStage<T> + a.lds_bytes - 2 * kAll * a.cells);  // [kAll][cells]
-  const bool held   = (words + 1) * static_cast<int>(sizeof(T)) + 2 * kAll * a.cells <= a.lds_bytes;
+  const int table_at = turned ? kLineStage<T> / static_cast<int>(sizeof(T)) : 0;
+  T* const s_tab    = s_x + table_at;
+  uint16_t* s_start = reinterpret_cast<uint16_t*>(smem_raw + kLineStage<T> + a.lds_bytes - 2 * kAll * cells);  // [kAll][cells]
   if (tid < kAll) {
     const int at = st.offset[f0 + min(tid, nf)];
     s_most[tid]  = 0;
@@ -554,10 +567,10 @@ __global__ void __launch_bounds__(kWalkThreads, 8)
   if (held) {
     for (int e = tid; e < words; e += kWalkThreads) s_tab[e] = sorted[first + e];
     if (tid == 0) s_tab[words] = T(0);  // read, not used, by features without thresholds
-    for (int c = tid; c < kAll * a.cells; c += kWalkThreads) s_start[c] = 0;
+    for (int c = tid; c < kAll * cells; c += kWalkThreads) s_start[c] = 0;
   }
   __syncthreads();
-  if (held) rank_cells<T, kAll>(a.cells, s_tab, s_start, s_place, s_count, s_most, s_lo, s_scale);
+  if (held) rank_cells<T, kAll>(cells, s_tab, s_start, s_place, s_count, s_most, s_lo, s_scale);
   __syncthreads();
   // a wave's features of 64 rows
   constexpr int kOwn = kAll / 4;
@@ -574,13 +587,62 @@ __global__ void __launch_bounds__(kWalkThreads, 8)
   };
 #pragma unroll
   for (int j = 0; j < kOwn; j++) {
-    place[j]    = __builtin_amdgcn_readfirstlane(s_place[own + j]);
+    place[j]    = table_at + __builtin_amdgcn_readfirstlane(s_place[own + j]);
     probes[j]   = __builtin_amdgcn_readfirstlane(s_most[own + j]);
     lo[j]       = uniform(s_lo[own + j]);
     scale[j]    = uniform(s_scale[own + j]);
     most_probes = max(most_probes, probes[j]);
   }
-  const uint16_t* const start = s_start + own * a.cells;
+  const uint16_t* const start = s_start + own * cells;
+  // ranks of a lane's values in the turn that begins with row0
+  auto rank_turn = [&](const T (&x)[kOwn], int64_t row0) {
+    int at[kOwn];
+    if (held) {
+#pragma unroll
+      for (int j = 0; j < kOwn; j++) at[j] = start[j * cells + cell_of(x[j], lo[j], scale[j], cells)];
+      for (int p = most_probes - 1; p >= 0; p--) {
+#pragma unroll
+        for (int j = 0; j < kOwn; j++) {
+          if (p >= probes[j]) continue;  // (the same for the whole wave)
+          const T v = s_x[place[j] + ((1 << p) - 1) + at[j]];
+          at[j] += v < x[j] ? 1 << p : 0;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < kOwn; j++) at[j] = lower_bound(sorted + first + (place[j] - table_at), s_count[own + j], x[j]);
+    }
+    const int64_t block = row0 + wave / 4 * 64;  // (a split ends with a block, or with the last row)
+    if (block < end) {
+      uint32_t code[kOwn];
+#pragma unroll
+      for (int j = 0; j < kOwn; j++) code[j] = x[j] == x[j] ? static_cast<uint32_t>(at[j]) + 1 : kNanRank;
+      // tile rows are a power of two, 64 or more; a tile's ranks lie within 32 bits of bytes
+      const int64_t tile = block >> a.tile_shift;
+      char* const base   = reinterpret_cast<char*>(ranks + (tile * a.F + f0 + own) * (int64_t(1) << a.tile_shift));
+      store_ranks(code, nf - own, a.tile_shift, base + 2 * (static_cast<int>(block) & ((1 << a.tile_shift) - 1)));
+    }
+  };
+  if (!turned) {
+    for (int64_t row0 = begin; row0 < end; row0 += kLineRows) {
+      const T* const src = X + min(row0 + row_of, end - 1) * a.F;
+      T x[kOwn];
+      if (a.wide) {
+#pragma unroll
+        for (int j = 0; j < kOwn; j += kPer) {
+          const int f = f0 + own + j;
+          const Vec v = *reinterpret_cast<const Vec*>(src + (f < a.F ? f : f0));
+#pragma unroll
+          for (int u = 0; u < kPer; u++) x[j + u] = v[u];
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < kOwn; j++) x[j] = src[min(f0 + own + j, a.F - 1)];
+      }
+      rank_turn(x, row0);
+    }
+    return;
+  }
   for (int64_t row0 = begin; row0 < end; row0 += kLineRows) {
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
@@ -593,34 +655,9 @@ __global__ void __launch_bounds__(kWalkThreads, 8)
     }
     __syncthreads();
     T x[kOwn];
-    int at[kOwn];
 #pragma unroll
     for (int j = 0; j < kOwn; j++) x[j] = s_x[(own + j) * kPitch + row_of];
-    if (held) {
-#pragma unroll
-      for (int j = 0; j < kOwn; j++) at[j] = start[j * a.cells + cell_of(x[j], lo[j], scale[j], a.cells)];
-      for (int p = most_probes - 1; p >= 0; p--) {
-#pragma unroll
-        for (int j = 0; j < kOwn; j++) {
-          if (p >= probes[j]) continue;  // (the same for the whole wave)
-          const T v = s_tab[place[j] + ((1 << p) - 1) + at[j]];
-          at[j] += v < x[j] ? 1 << p : 0;
-        }
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < kOwn; j++) at[j] = lower_bound(sorted + first + place[j], s_count[own + j], x[j]);
-    }
-    const int64_t block = row0 + wave / 4 * 64;  // (a split ends with a block, or with the last row)
-    if (block < end) {
-      uint32_t code[kOwn];
-#pragma unroll
-      for (int j = 0; j < kOwn; j++) code[j] = x[j] == x[j] ? static_cast<uint32_t>(at[j]) + 1 : kNanRank;
-      // tile rows are a power of two, 64 or more; a tile's ranks lie within 32 bits of bytes
-      const int64_t tile = block >> a.tile_shift;
-      char* const base   = reinterpret_cast<char*>(ranks + (tile * a.F + f0 + own) * (int64_t(1) << a.tile_shift));
-      store_ranks(code, nf - own, a.tile_shift, base + 2 * (static_cast<int>(block) & ((1 << a.tile_shift) - 1)));
-    }
+    rank_turn(x, row0);
     __syncthreads();
   }
 }
@@ -980,7 +1017,8 @@ Plan make_plan(int64_t N, int F, int n_trees, const int32_t* tree_nodes, int K, 
     p.group = 1;
     while (p.group < kGroupMax && p.group < F && bytes_for(2 * p.group) <= static_cast<double>(kLds - 1024)) p.group *= 2;
   }
-  // what all thresholds on these features would take, or room for twice the mean
+  // what all thresholds on these features would take, or room for twice the mean; of a line's two workgroups to a CU: as much of that as is left beside
+  // the turned rows (46,592 bytes; rank_lines_kernel makes do with fewer cells, or takes the rows' place)
   const double all_here = (static_cast<double>(thresholds) + 1) * static_cast<double>(value_size) + 2.0 * p.group * p.cells;
   const double room     = std::min(all_here, std::max(2.0 * bytes_for(p.group), 32.0 * 1024)) + 15;
   p.rank_lds = static_cast<int>(std::min(room, static_cast<double>(p.group == line ? kLds / 2 - 1024 - stage : kLds - 1024))) / 16 * 16;

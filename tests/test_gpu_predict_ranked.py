@@ -118,6 +118,27 @@ def test_last_features_of_a_cache_line(f, dtype):
     assert torch.equal(ops.predict(X, trees, 1), ops.predict(X, trees, 1, tiled=False))
 
 
+@pytest.mark.parametrize("f,n_trees,dtype", [(400, 100, np.float32), (403, 100, np.float32), (100, 40, np.float64), (103, 41, np.float64)])
+@pytest.mark.parametrize("share", [0.0, 0.33, 0.6, 0.9])
+@pytest.mark.parametrize("last", [False, True])
+def test_thresholds_that_crowd_one_cache_line(f, n_trees, dtype, share, last):
+    """255 thresholds a tree, a share of them on the features of the first or of the last line of 128 bytes. At 0 all lines' tables lie
+    in the LDS beside the rows (46,592 bytes); at 0.33 those of 9810 floats or 4460 doubles have fewer cells; 6770 doubles (0.6) take the rows'
+    place as well; 15,000 floats and 9200 doubles are searched in memory."""
+    rs = np.random.RandomState(f + int(100 * share))
+    line = 128 // np.dtype(dtype).itemsize
+    crowd = np.arange((f - 1) // line * line, f) if last else np.arange(line)
+    trees = []
+    for _ in range(n_trees):
+        feature = np.full(511, -1, np.int32)
+        feature[:255] = np.where(rs.rand(255) < share, rs.choice(crowd, 255), rs.randint(0, f, 255))
+        trees.append((torch.from_numpy(rs.randn(511, 1)).cuda(), torch.from_numpy(feature).cuda(),
+                      torch.from_numpy(rs.rand(511)).cuda()))
+    X = _rows(rs, 50_001, f, dtype, 0)
+    assert _takes_ranks(X, trees, 1)
+    assert torch.equal(ops.predict(X, trees, 1), ops.predict(X, trees, 1, tiled=False))
+
+
 @pytest.mark.parametrize("n,f,n_trees,depth", [(1_000_000, 8, 130, 6), (70_000, 516, 40, 5)])
 def test_a_start_off_a_16_byte_boundary(n, f, n_trees, depth):
     rs = np.random.RandomState(5)
