@@ -197,10 +197,13 @@ class LBBase:
         # 1.18, 1,000,000 x 50 2.14 and 2.10, 2,000,000 x 40 2.95 and 2.92, 4,000,000 x 30 3.71 and 3.72, 6,000,000 x 30 5.28 and
         # 5.29 (two classes 5.37 and 5.40), 10,000,000 x 100 17.98 and 18.08; three classes, 1,500,000 x 20 2.65 and 2.62,
         # 2,000,000 x 30 4.01 and 4.00; two outputs, 4,000,000 x 30 5.42 and 5.50; eight classes, 600,000 x 20 3.12 and 3.13,
-        # 2,000,000 x 30 6.65 and 6.85; 16, 3,000,000 x 30 12.7 and 13.3.
+        # 2,000,000 x 30 6.65 and 6.85; 16, 3,000,000 x 30 12.7 and 13.3. Rows of more than 128 classes are a thread's work, and a
+        # workgroup's entries few of them: never (two rounds of depth 3, ms: 70,000 x 4 with 130 classes 2.88 and 2.66, 20,000 with 500
+        # 8.4 and 5.1, 10,000 with 1000 14.9 and 8.8).
         fused = getattr(self._objective_instance, "fused", None)
         sums = (fused is not None and self.subsample == 1.0 and train_pred.is_cuda
                 and train_pred.numel() >= (4000000 if train_pred.shape[1] == 1 else 8000000)
+                and (fused != "log_loss" or train_pred.shape[1] <= 128)
                 and _as_defined(self, LBBase, "_get_weighted_gradient"))
         for i in range(self.n_estimators):
             model = deepcopy(self.base_models[i % len(self.base_models)]).set_random_state(self.random_state_)

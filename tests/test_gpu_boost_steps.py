@@ -299,3 +299,30 @@ def test_softmax_gradients_of_many_entries():
     assert torch.equal(g[:some], g1) and torch.equal(h[:some], h1)
     g2, h2 = ops.weighted_gradient("log_loss", y[some:].contiguous(), pred[some:].contiguous(), None, 1.0)
     assert torch.equal(g[some:], g2) and torch.equal(h[some:], h2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("task,n,k,asked", [("classes", 66_000, 128, True), ("classes", 66_000, 129, False), ("values", 66_000, 129, True),
+                                            ("classes", 60_000, 128, False)])
+def test_which_fits_ask_for_the_gradient_passes_sums(monkeypatch, task, n, k, asked):
+    """Eight million entries or more, and of a softmax rows of up to 128 outputs: beyond, the pass with the sums costs a fit of 1000
+    classes more than the trees do."""
+    import lbtree as lb
+    from lbtree import ops
+
+    own, seen = ops.weighted_gradient, []
+
+    def watched(*args, sums=False, **kw):
+        seen.append(sums)
+        return own(*args, sums=sums, **kw)
+
+    monkeypatch.setattr(ops, "weighted_gradient", watched)
+    torch.manual_seed(0)
+    X = torch.rand(n, 3).cuda()
+    tree = lb.models.Tree(max_depth=2, split_samples=8)
+    if task == "classes":
+        y = (torch.arange(n) % k).double().cuda()
+        lb.LBClassifier(n_estimators=1, base_models=(tree,), random_state=1).fit(X, y)
+    else:
+        lb.LBRegressor(n_estimators=1, base_models=(tree,), random_state=1).fit(X, torch.rand(n, k, dtype=torch.float64).cuda())
+    assert seen == [asked]
