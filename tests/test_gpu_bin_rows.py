@@ -86,3 +86,10 @@ def test_medium_builder_bins(n, f, k, dtype, samples):
     g, h = rs.normal(size=(n, k)), 0.5 + rs.rand(n, k)
     gr, cr = gu.both(X, g, h, max_depth=3, split_samples=samples, seed=5)
     gu.assert_tree_parity(gr, cr)
+
+
+@pytest.mark.parametrize("f", [1, 2, 3, 4, 7, 8, 9, 16])
+@pytest.mark.parametrize("n,dtype", [(150_001, np.float32), (150_257, np.float64)])
+def test_medium_builder_bins_of_few_features(n, f, dtype):
+    """Tiles whose rows take some of a thread's turns, and some of the waves; the last one has one row."""
+    test_medium_builder_bins(n, f, 1, dtype, 256)
