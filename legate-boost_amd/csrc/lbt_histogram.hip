@@ -947,6 +947,13 @@ __global__ void __launch_bounds__(kHistThreads)
 // What bounds it: the memory, nearly. 10,000,000 x 100 f32 (4 GB read, 1.36 GB written) takes 1.21 ms, its loads and stores without any
 // search 1.12, the same pattern of accesses in a stand-alone kernel 1.02 (1.43 before records were written by words of whole lines and
 // the searches of a lane's values went side by side); 2,000,000 x 200 0.48 ms (0.74), 1,000,000 x 50 in two-byte bins 0.086 (0.114).
+// what a lane of the quad has, for each of them two bits of kPerm
+template <int kPerm>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t v)
+{
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kPerm, 0xf, 0xf, true));
+}
+
 template <typename T>
 struct BinRowsArgs {
   int F;
@@ -964,6 +971,7 @@ struct BinRowsArgs {
   int n_sgroups;
   int n_chunks;
   int rpp;                    // rows per pass of a workgroup
+  int share;                  // lanes that share a record (kShared)
   const int2* lanes;          // lanes of a row of every search group (see bin_lanes)
   const RecInfo* rec;         // [histogram groups]
 };
@@ -972,7 +980,8 @@ struct BinRowsArgs {
 // than VEC features: it loads the VEC values that end with the row's last one and takes its
 // own from their end, and its surplus bins are zeros in the record's padding. Rows then start
 // on element boundaries only, so all lanes load with element alignment.
-template <typename T, int VEC, typename BinT, bool kRagged>
+// kShared: rows of few features, whose records of 32 bytes their lanes share evenly (share_of_record).
+template <typename T, int VEC, typename BinT, bool kRagged, bool kShared>
 __global__ void __launch_bounds__(kHistThreads)
   bin_rows_kernel(BinRowsArgs<T> a, const T* __restrict__ X, const int2* __restrict__ qgh,
                   BinT* __restrict__ binned)
@@ -1022,7 +1031,7 @@ __global__ void __launch_bounds__(kHistThreads)
   const int nth     = threadIdx.x % head.y;
   const int2 lane   = a.lanes[head.x + nth];
   constexpr int kOwn = VEC * static_cast<int>(sizeof(BinT));  // bytes of a lane's bins
-  const int fb      = kOwn >= 4 ? lane.x : f0 + nth * VEC;  // first feature of this lane
+  const int fb      = kShared || kOwn >= 4 ? lane.x : f0 + nth * VEC;  // first feature of this lane
   const int kind    = lane.y & 3;
   const int mine    = kRagged ? min(VEC, f1 - fb) : VEC;
   const int shift   = VEC - mine;     // its values are the last `mine` of the VEC it loads
@@ -1044,13 +1053,16 @@ __global__ void __launch_bounds__(kHistThreads)
   // What a lane writes of a row are kWords words: its bins, zeros, or the row's gradient pair. A wave's stores so are one run of bytes
   // and nearly always whole cache lines, which is what the memory wants: with lanes for the bins alone and masked stores
   // of 16 bytes for what follows them 10,000,000 x 100 f32 took 1.32 ms, with the same pieces written by other waves 2.44 (lines
-  // that reach the memory in parts), although a fifth fewer lanes search. Bins of fewer than four bytes a lane (up to three features)
-  // are written byte by byte, their last lane filling the record.
-  constexpr int kWords = kOwn >= 4 ? kOwn / 4 : 1;
-  const int to_off     = lane.y >> 2;  // its bytes, from the row's first
-  // kOwn < 4: the record's bytes behind the own bins up to the pair, and whether that follows
+  // that reach the memory in parts), although a fifth fewer lanes search. kShared: its even share of the record's 32 bytes, of which the first 16 are
+  // the bins of all its lanes. Bins of fewer than four bytes a lane are written byte by byte otherwise, their last lane filling the record (rows that
+  // do not begin on a multiple of their values' size).
+  constexpr int kWords   = kOwn >= 4 ? kOwn / 4 : 1;
+  constexpr bool kByByte = !kShared && kOwn < 4;
+  const int to_off       = lane.y >> 2;  // its bytes, from the row's first
+  const bool pairs       = kShared && a.rec[0].q_off >= 0;
+  // kByByte: the record's bytes behind the own bins up to the pair, and whether that follows
   int t_zero = 0, t_pair = -1;
-  if (kOwn < 4 && kind == 1) {
+  if (kByByte && kind == 1) {
     const RecInfo ri = a.rec[lane.x];
     t_zero = ri.in_row + ri.zero_end - to_off;
     t_pair = ri.q_off >= 0 ? ri.in_row + ri.q_off - to_off : -1;
@@ -1130,11 +1142,15 @@ __global__ void __launch_bounds__(kHistThreads)
   };
   const uint32_t pair_mask = kind >= 2 ? ~0u : 0u;
   // what a lane reads of a row's gradient pair, like its values: one word, or both
-  using Pair = std::conditional_t<kWords == 2 || kOwn < 4, int2, int>;
-  auto load_pair = [&](uint32_t at) { return *reinterpret_cast<const Pair*>(q_chunk + min(at, q_last)); };
+  using Pair = std::conditional_t<kWords == 2 || kOwn < 4 || kShared, int2, int>;
+  auto load_pair = [&](uint32_t at) {
+    if (kShared && !pairs) return Pair{};
+    return *reinterpret_cast<const Pair*>(q_chunk + min(at, q_last));
+  };
   // Loads come before the stores of a pass, in fixed numbers: a wait for loads behind stores would wait for these too.
   auto search_pass = [&](auto bent_cells, int first, Vec (&x_c)[kAhead], Pair (&q_c)[kAhead]) {
     uint32_t own[kUnroll][kWords];
+    Pair pair_of[kShared ? kUnroll : 1];
     // The rows of a batch go through the search side by side, stage by stage: all reads of the tables, then all
     // probes. hipcc by itself takes one value after the other, two round trips through the LDS each.
 #pragma unroll
@@ -1220,7 +1236,11 @@ __global__ void __launch_bounds__(kHistThreads)
           const int b = kRagged && v >= mine ? 0 : bn[w][v];
           words[v / kInWord] |= static_cast<uint32_t>(b) << (8 * sizeof(BinT) * (v % kInWord));
         }
-        if constexpr (kOwn >= 4) {
+        if constexpr (kShared) {
+          pair_of[u] = q_c[u % kAhead];
+#pragma unroll
+          for (int k = 0; k < kWords; k++) words[k] = kind == 0 ? words[k] : 0u;
+        } else if constexpr (!kByByte) {
           uint32_t pair[2];
           if constexpr (kWords == 2) {
             pair[0] = static_cast<uint32_t>(q_c[u % kAhead].x);
@@ -1234,31 +1254,42 @@ __global__ void __launch_bounds__(kHistThreads)
 #pragma unroll
         for (int k = 0; k < kWords; k++) own[u][k] = words[k];
         x_c[u % kAhead] = load_row(x_off + (u + kAhead) * x_step);
-        if constexpr (kOwn >= 4) q_c[u % kAhead] = load_pair(q_off + (u + kAhead) * q_step);
+        if constexpr (!kByByte) q_c[u % kAhead] = load_pair(q_off + (u + kAhead) * q_step);
       }
     }
     const int left = n_local - first - rsub;  // row u of the pass exists if u * rpp < left
-    if constexpr (kOwn >= 4) {
 #pragma unroll
-      for (int u = 0; u < kUnroll; u++) {
-        if (u * a.rpp >= left) continue;
-        unsigned char* const to = b_chunk + (b_off + u * b_step);
-        if constexpr (kWords == 2)
-          *reinterpret_cast<uint2*>(to) = make_uint2(own[u][0], own[u][1]);
-        else
-          *reinterpret_cast<uint32_t*>(to) = own[u][0];
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < kUnroll; u++) {
-        if (u * a.rpp >= left) continue;
-        unsigned char* const to = b_chunk + (b_off + u * b_step);
+    for (int u = 0; u < kUnroll; u++) {
+      if (u * a.rpp >= left) continue;  // (the same for the lanes of a row)
+      unsigned char* const to = b_chunk + (b_off + u * b_step);
+      if constexpr (kShared) {
+        const uint32_t w0 = own[u][0], w1 = kWords == 2 ? own[u][kWords - 1] : 0u;
+        const uint32_t p0 = static_cast<uint32_t>(pair_of[u].x), p1 = static_cast<uint32_t>(pair_of[u].y);
+        if (a.share == 1) {
+          *reinterpret_cast<uint4*>(to)      = make_uint4(w0, w1, 0u, 0u);
+          *reinterpret_cast<uint4*>(to + 16) = make_uint4(0u, 0u, p0, p1);
+        } else if (a.share == 2) {
+          const uint32_t o0 = quad_lane<0xb1>(w0), o1 = kWords == 2 ? quad_lane<0xb1>(w1) : 0u;  // of the other lane
+          const uint4 bins  = kOwn == 8   ? make_uint4(w0, w1, o0, o1)
+                              : kOwn == 4 ? make_uint4(w0, o0, 0u, 0u)
+                                          : make_uint4(w0 | o0 << (8 * kOwn % 32), 0u, 0u, 0u);
+          *reinterpret_cast<uint4*>(to) = to_off == 0 ? bins : make_uint4(0u, 0u, p0, p1);
+        } else {
+          const uint32_t b0 = quad_lane<0 + 4 * 2>(w0), b1 = quad_lane<1 + 4 * 3>(w0);  // lane 0: of lanes 0 and 1, lane 1: of lanes 2 and 3
+          const uint2 last  = to_off == 24 ? make_uint2(p0, p1) : make_uint2(0u, 0u);
+          *reinterpret_cast<uint2*>(to) = to_off < 16 ? make_uint2(b0, b1) : last;
+        }
+      } else if constexpr (kByByte) {
         if constexpr (kOwn == 2)
           *reinterpret_cast<uint16_t*>(to) = static_cast<uint16_t>(own[u][0]);
         else
           *to = static_cast<unsigned char>(own[u][0]);
         for (int i = kOwn; i < t_zero; i++) to[i] = 0;
         if (t_pair >= 0) *reinterpret_cast<int2*>(to + t_pair) = load_pair(q_off + u * q_step);
+      } else if constexpr (kWords == 2) {
+        *reinterpret_cast<uint2*>(to) = make_uint2(own[u][0], own[u][1]);
+      } else {
+        *reinterpret_cast<uint32_t*>(to) = own[u][0];
       }
     }
     x_off += kUnroll * x_step;
@@ -1272,7 +1303,7 @@ __global__ void __launch_bounds__(kHistThreads)
 #pragma unroll
     for (int u = 0; u < kAhead; u++) {
       x_c[u] = load_row(x_off + u * x_step);
-      if constexpr (kOwn >= 4) q_c[u] = load_pair(q_off + u * q_step);
+      if constexpr (!kByByte) q_c[u] = load_pair(q_off + u * q_step);
     }
     for (int first = 0; first < n_local; first += pass_rows) search_pass(bent_cells, first, x_c, q_c);
   };
@@ -1906,11 +1937,15 @@ int launch_search_rows(hipStream_t stream, const HistSetup& hs, const HistArgs<T
 template <typename T, int VEC, typename BinT, bool kRagged>
 int launch_bin_rows(hipStream_t stream, const HistSetup& hs, const BinRowsArgs<T>& a, const HistBatch& b, unsigned grid)
 {
-  static std::atomic<bool> attr_set[kMaxDevices] = {};
-  LBT_TRY(allow_dynamic_lds(bin_rows_kernel<T, VEC, BinT, kRagged>, kLdsBudget, attr_set));
-  bin_rows_kernel<T, VEC, BinT, kRagged><<<grid, kHistThreads, hs.lds_bytes, stream>>>(
-    a, static_cast<const T*>(b.X), b.qgh, static_cast<BinT*>(hs.binned));
-  return LBT_OK;
+  auto launch = [&](auto shared) -> int {
+    constexpr bool kShared = decltype(shared)::value;
+    static std::atomic<bool> attr_set[kMaxDevices] = {};
+    LBT_TRY(allow_dynamic_lds(bin_rows_kernel<T, VEC, BinT, kRagged, kShared>, kLdsBudget, attr_set));
+    bin_rows_kernel<T, VEC, BinT, kRagged, kShared><<<grid, kHistThreads, hs.lds_bytes, stream>>>(
+      a, static_cast<const T*>(b.X), b.qgh, static_cast<BinT*>(hs.binned));
+    return LBT_OK;
+  };
+  return hs.share > 0 ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 template <typename T, int VEC>
@@ -2034,6 +2069,7 @@ int hist_launch_t(hipStream_t stream, const HistSetup& hs, const HistBatch& b, i
     a.search_steps = hs.search_steps;
     a.n_sgroups    = hs.n_sgroups;
     a.rpp          = hs.rpp;
+    a.share        = hs.share;
     a.lanes        = hs.bin_lanes;
     a.rec          = hs.rec;
     const int per_cu = hs.lds_bytes * 2 <= 160 * 1024 ? 2 : 1;
@@ -2189,17 +2225,34 @@ int rows_per_pass(const std::vector<int32_t>& groups, int vec)
   return rpp;
 }
 
+// Lanes that share a record of the binning pass, where all records have 32 bytes of which 16 hold the bins of one, two or four lanes; more than
+// one lane: a single record, whose lanes then are side by side in a wave. 0: not so.
+// With lanes of a word each, seven of the eight of a record with four bins search for nothing, and bins written byte by byte are up to 25 stores a row.
+// 17,000,000 rows, us with shares and without: floats x 1 225 and 446, x 3 198 and 470, x 4 248 and 391, x 5 226 and 423, x 8 253 and 394, x 9 300
+// and 440, x 16 363 and 411; doubles x 1 221 and 457, x 4 288 and 449, x 8 357 and 455, x 16 587 and 599; two-byte bins:
+// floats x 3 199 and 467, x 5 226 and 250, doubles x 5 289 and 307.
+int share_of_record(const std::vector<int32_t>& groups, const std::vector<RecInfo>& rec, int vec, int bin_bytes)
+{
+  int share = 1;
+  for (size_t g = 0; g < rec.size(); g++) {
+    const int lanes = (groups[g + 1] - groups[g] + vec - 1) / vec;
+    if (rec[g].size != 32 || lanes * vec * bin_bytes > 16 || lanes > 4 || (lanes > 2 && vec * bin_bytes != 4)) return 0;
+    share = std::max(share, lanes <= 2 ? lanes : 4);
+  }
+  return share > 1 && rec.size() > 1 ? 0 : share;
+}
+
 // The lanes that hold a row in the binning pass: two entries for each search group, {where its lanes begin,
 // how many} and {bytes between the rows of its plane, where that begins in units of kPlaneAlign}, then the lanes. A lane is
 // {first feature, kind + 4 * its first byte in the plane's row} and holds vec * bin_bytes bytes of a record; kind 0: bins, 1: zeros, 2 and 3: the
 // words of the gradient pair (2: both, where a lane holds two words). A search group has the lanes of its features and, behind a
-// record's last ones, those of the rest of the record. Where a lane has less than four bytes (up to three features) there are lanes of
-// bins only {record, ...}, kind 1: a record's last one.
+// record's last ones, those of the rest of the record. share > 0: a record has that many lanes, of 32 / share bytes each; kind 1: without
+// features (share_of_record). Otherwise, where a lane has less than four bytes, there are lanes of bins only {record, ...}, kind 1: a record's last one.
 // Returns the rows that a workgroup takes side by side: as many as fit, or up to an eighth fewer that are whole cache lines; 0 where a
 // row does not fit. (A search group has up to 512 lanes of features and up to 13 more for each of its records. The LDS holds the proposals
 // of 40,000 bins, and a record has 19,000 of them but where more records fill the chip better: seven at the most, some 600 lanes of the 1024.)
 int bin_lanes(const std::vector<int32_t>& sgroups, const std::vector<int32_t>& groups, const std::vector<RecInfo>& rec,
-              int vec, int bin_bytes, std::vector<int2>& lanes)
+              int vec, int bin_bytes, int share, std::vector<int2>& lanes)
 {
   const int n_s = static_cast<int>(sgroups.size()) - 1, own = vec * bin_bytes;
   lanes.assign(2 * static_cast<size_t>(n_s), make_int2(0, 0));
@@ -2212,6 +2265,14 @@ int bin_lanes(const std::vector<int32_t>& sgroups, const std::vector<int32_t>& g
       const RecInfo& ri = rec[group];
       const int at      = ri.in_row + (f - groups[group]) * bin_bytes;
       const bool last   = f + vec >= groups[group + 1];
+      if (share > 0) {
+        for (int nth = (f - groups[group]) / vec; nth < share; nth++) {
+          const bool own_bins = nth == (f - groups[group]) / vec;
+          lanes.push_back(make_int2(f, (own_bins ? 0 : 1) + 4 * (ri.in_row + nth * 32 / share)));
+          if (!last) break;
+        }
+        continue;
+      }
       lanes.push_back(make_int2(own >= 4 ? f : static_cast<int>(group), (own < 4 && last ? 1 : 0) + 4 * at));
       if (own < 4 || !last) continue;
       const int end = ri.in_row + ri.size;
@@ -2326,7 +2387,7 @@ int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, i
   // last lane of a row then owns fewer features); the kernel that searches X itself does not.
   hs.ragged = false;
   if (hs.binned != nullptr) {
-    const int full = F >= 4 ? 4 : vec;
+    const int full = F >= 4 ? 4 : std::min(F, 2);
     if (vec < full && reinterpret_cast<uintptr_t>(X) % elem == 0) {
       vec       = full;
       hs.ragged = F % full != 0;
@@ -2567,7 +2628,8 @@ int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, i
       return LBT_ERR_WORKSPACE;
     }
     up.add(hs.rec, rec.data(), sizeof(RecInfo) * rec.size());
-    hs.rpp = bin_lanes(sgroups, groups, rec, vec, hs.bin_bytes, lanes);
+    hs.share = share_of_record(groups, rec, vec, hs.bin_bytes);
+    hs.rpp   = bin_lanes(sgroups, groups, rec, vec, hs.bin_bytes, hs.share, lanes);
     if (hs.rpp < 1 || lanes.size() > bin_lanes_max(F)) {
       set_error("a row takes %zu lanes of the binning pass", lanes.size());
       return LBT_ERR_INVALID;

@@ -424,6 +424,7 @@ struct HistSetup {
   int64_t row_bytes      = 0;      // bytes of a row in all planes
   int pieces           = 0;        // 16-byte pieces of bins of a row's records
   int max_bins         = 0;        // bins of the widest feature
+  int share            = 0;        // lanes that share a record in the binning pass, 0: each has words of its own (share_of_record)
   int2* bin_lanes      = nullptr;  // [bin_lanes_max] lanes of a row in the binning pass (see bin_lanes)
   // feature-major copy of the bins, [feature][row], written by the root histogram launch for the
   // position updates (null: not wanted)

@@ -66,6 +66,31 @@ def test_root_histogram_of_binned_rows(n, f, k, dtype, samples):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("f", [1, 2, 3, 4, 5, 7, 8, 9, 11, 12, 13, 16, 17])
+@pytest.mark.parametrize("samples", [256, 300])
+@pytest.mark.parametrize("k,dtype", [(1, np.float32), (1, np.float64), (2, np.float32)])
+def test_rows_whose_lanes_share_a_record(f, samples, k, dtype):
+    """One, two and four lanes to a record of 32 bytes, some of them without features, bins of one and two bytes; 17: no longer."""
+    test_root_histogram_of_binned_rows(4099 + f, f, k, dtype, samples)
+
+
+@pytest.mark.parametrize("f", [1, 2, 3, 4, 8, 16])
+def test_rows_whose_lanes_share_a_record_off_a_16_byte_boundary(f, monkeypatch):
+    from lbtree import ops
+
+    own = ops.histogram_level
+
+    def moved(X, *args):
+        base = torch.empty(X.numel() + 1, dtype=X.dtype, device=X.device)
+        at = base[1:].view(X.shape)
+        at.copy_(X)
+        assert at.data_ptr() % 16 != 0
+        return own(at, *args)
+
+    monkeypatch.setattr(ops, "histogram_level", moved)
+    test_root_histogram_of_binned_rows(2049, f, 1, np.float32, 256)
+
+
 @pytest.mark.parametrize("n,f,k,dtype", [(301, 2051, 1, np.float32), (301, 4100, 1, np.float64), (301, 2048, 3, np.float32)])
 def test_rows_of_as_many_lanes_as_a_search_group_has(n, f, k, dtype):
     """Few proposals a feature: what bounds a search group is its lanes, beside which those of the records have their place."""
