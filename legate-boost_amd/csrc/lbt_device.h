@@ -85,6 +85,7 @@ __device__ __forceinline__ double wave_read_lane_f64(double v, int src)
 // Values that loads bring, when all of them are here: hipcc moves a load behind the branch that is its only use, where a wave
 // then waits for it alone.
 __device__ __forceinline__ void arrived(int2& v) { asm volatile("" : "+v"(v.x), "+v"(v.y)); }
+__device__ __forceinline__ void arrived(I64Pair& v) { asm volatile("" : "+v"(v.grad), "+v"(v.hess)); }
 __device__ __forceinline__ void arrived(uint4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 
 // put(i, take(i)) for i = threadIdx.x, + kT, ... below n: kAhead loads are under way at once. (A loop over both, as hipcc
