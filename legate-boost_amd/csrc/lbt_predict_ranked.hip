@@ -62,14 +62,14 @@ __global__ void zero_counts_kernel(int32_t* count, int n)
 
 // One thread per heap slot of a tree of `depth` complete levels: slot i is inner node i (1 is the root) and leaf i of the
 // bottom. What lies below a node that ends the walk is never decisive: every bottom leaf below it has its value.
-// A workgroup takes `together` trees, up to kPackTogether, and counts their thresholds in the LDS (when kLocal: the counters fit), so that
+// A workgroup takes kTogether trees and counts their thresholds in the LDS (when kLocal: the counters fit), so that
 // a feature's counter in memory is added to once per workgroup and not once per node: adds to one address take turns
 // of about 0.1 us (64 trees of depth 8 on 64 features: 29 us a launch with an add per node and a chain of loads, 14 now).
 constexpr int kPackTogether  = 4;
 constexpr int kLeafLoads     = 8;
 constexpr int kLocalCounters = 8192;
-template <typename T, bool kLocal>
-__global__ void __launch_bounds__(kThreads) rank_pack_kernel(PackRefs refs, int first, int here, int all, int together, RankState st, T* raw)
+template <typename T, bool kLocal, int kTogether>
+__global__ void __launch_bounds__(kThreads) rank_pack_kernel(PackRefs refs, int first, int here, int all, RankState st, T* raw)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   int32_t* s_count = reinterpret_cast<int32_t*>(smem_raw);
@@ -79,13 +79,13 @@ __global__ void __launch_bounds__(kThreads) rank_pack_kernel(PackRefs refs, int 
     for (int f = threadIdx.x; f < st.F; f += kThreads) s_count[f] = 0;
     __syncthreads();
   }
-  int slot[kPackTogether], node_feature[kPackTogether];
+  int slot[kTogether], node_feature[kTogether];
 #pragma unroll
-  for (int u = 0; u < kPackTogether; u++) {
-    const int t     = blockIdx.y * together + u;
+  for (int u = 0; u < kTogether; u++) {
+    const int t     = blockIdx.y * kTogether + u;
     slot[u]         = -1;
     node_feature[u] = 0;
-    if (u >= together || i >= size || t >= all) continue;
+    if (i >= size || t >= all) continue;
     const int64_t at = (static_cast<int64_t>(first + t) << st.depth) + i;
     if (t >= here) continue;  // padding to whole chunks: a tree whose values nothing adds
     const int32_t* feature = refs.feature[t];
@@ -123,9 +123,13 @@ __global__ void __launch_bounds__(kThreads) rank_pack_kernel(PackRefs refs, int 
     const int stop = ends_leaf != 0 ? __ffs(ends_leaf) - 1 : st.depth;
     const int a    = (size + i) >> (st.depth - stop);
     // (loads of several outputs under way together: hipcc has every load wait behind the store before it, and with eight outputs
-    // 50 trees took 24 us that way, 21.5 this way)
+    // 50 trees took 24 us that way, 21.5 this way; of one output there is one, not eight of the same)
     const double* from = refs.leaf[t] + static_cast<int64_t>(a - 1) * st.K;
     double* to         = st.leaves + at * st.K;
+    if (st.K == 1) {
+      *to = *from;
+      continue;
+    }
     for (int k0 = 0; k0 < st.K; k0 += kLeafLoads) {
       double v[kLeafLoads];
 #pragma unroll
@@ -144,9 +148,9 @@ __global__ void __launch_bounds__(kThreads) rank_pack_kernel(PackRefs refs, int 
     __syncthreads();
   }
 #pragma unroll
-  for (int u = 0; u < kPackTogether; u++) {
-    const int t = blockIdx.y * together + u;
-    if (u >= together || i >= size || t >= all) continue;
+  for (int u = 0; u < kTogether; u++) {
+    const int t = blockIdx.y * kTogether + u;
+    if (i >= size || t >= all) continue;
     const int64_t at = (static_cast<int64_t>(first + t) << st.depth) + i;
     const int base   = kLocal && slot[u] >= 0 ? s_count[node_feature[u]] : 0;
     st.slot[at]      = slot[u] >= 0 ? static_cast<uint32_t>(base + slot[u]) : kNoThreshold;
@@ -1099,12 +1103,18 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
       refs.n_nodes[i] = tree_nodes[first + i];
     }
     // few trees: one to a workgroup, whose chain of loads is what the launch lasts (50 trees with 8 outputs 24 us by fours, 8 alone)
-    const int together = p.padded_trees <= 64 ? 1 : kPackTogether;
-    const dim3 grid(ceil_div(1 << p.depth, kThreads), ceil_div(all, together));
-    if (F <= kLocalCounters)
-      rank_pack_kernel<T, true><<<grid, kThreads, F * sizeof(int32_t), stream>>>(refs, first, here, all, together, st, lay.raw);
+    auto pack = [&](auto together) {
+      constexpr int kTogether = decltype(together)::value;
+      const dim3 grid(ceil_div(1 << p.depth, kThreads), ceil_div(all, kTogether));
+      if (F <= kLocalCounters)
+        rank_pack_kernel<T, true, kTogether><<<grid, kThreads, F * sizeof(int32_t), stream>>>(refs, first, here, all, st, lay.raw);
+      else
+        rank_pack_kernel<T, false, kTogether><<<grid, kThreads, 0, stream>>>(refs, first, here, all, st, lay.raw);
+    };
+    if (p.padded_trees <= 64)
+      pack(std::integral_constant<int, 1>{});
     else
-      rank_pack_kernel<T, false><<<grid, kThreads, 0, stream>>>(refs, first, here, all, together, st, lay.raw);
+      pack(std::integral_constant<int, kPackTogether>{});
   }
   rank_offsets_kernel<<<1, 1024, 0, stream>>>(st);
   rank_scatter_kernel<T><<<ceil_div(p.slots, kThreads), kThreads, 0, stream>>>(st, lay.raw, lay.grouped);
