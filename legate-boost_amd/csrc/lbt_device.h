@@ -224,16 +224,9 @@ __device__ __forceinline__ double leaf_gain_select(double grad, double hess, dou
   return (z * z) / (hess + reg);
 }
 
-// n / d correctly rounded, where neither is near the ends of the exponent's range: an approximate reciprocal, two steps of Newton's
-// iteration and the remainder's correction. It is what `/` does without the scaling and the special cases, three instructions of eleven.
-__device__ __forceinline__ double quotient_plain(double n, double d)
-{
-  double r = __builtin_amdgcn_rcp(d);
-  r        = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
-  r        = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
-  const double q = n * r;
-  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
-}
+// n / d, where neither is near the ends of the exponent's range (quotient_from). It is what `/` does without the scaling and the special
+// cases, three instructions of eleven.
+__device__ __forceinline__ double quotient_plain(double n, double d) { return quotient_from(n, d, __builtin_amdgcn_rcp(d)); }
 // Without l1 the sums of grads are squared as they are. Sums are whole numbers below 2^35 times inv_g (inv_h); a denominator is at
 // least reg where its quotient counts.
 __device__ __forceinline__ bool plain_quotients(double l1, double inv_g, double inv_h, double reg)
@@ -366,7 +359,6 @@ __device__ __forceinline__ int feature_proposals(const T* __restrict__ X, const 
   return s_n;
 }
 
-// One stochastic rounding of a (grad, hess) pair (build_tree.cu:112-129).
 // A whole number as 64 bits: one conversion where it fits 32, as all but a value that ends the call does.
 __device__ __forceinline__ int64_t whole_to_i64(double v)
 {
@@ -374,6 +366,7 @@ __device__ __forceinline__ int64_t whole_to_i64(double v)
   asm volatile("");  // (a branch: the general conversion is eight instructions)
   return static_cast<int64_t>(v);
 }
+// One stochastic rounding of a (grad, hess) pair (build_tree.cu:112-129).
 __device__ __forceinline__ void quantise_pair(double grad, double hess, double sg, double sh, int64_t seed, int64_t row,
                                               int64_t k, int64_t* qg, int64_t* qh)
 {

@@ -211,11 +211,21 @@ __host__ __device__ inline uint32_t minstd_discard(uint32_t x, uint64_t z)
   }
   return mod_m(static_cast<uint64_t>(x) * acc);
 }
+// n / d from an approximate reciprocal r of d (a relative error of 2^-23 is enough): two steps of Newton's iteration, then the remainder's
+// correction. The bits of the division where no intermediate value leaves the normal range (tests/test_quotients.py).
+__host__ __device__ inline double quotient_from(double n, double d, double r)
+{
+  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+
 // thrust::uniform_real_distribution<double>(0,1) on one raw draw.
 __host__ __device__ inline double uniform01(uint32_t draw)
 {
-  // the quotient by 2147483646, correctly rounded: the product with its reciprocal and the remainder's correction (compared with the
-  // division for every draw; eight instructions less)
+  // the quotient by 2147483646, correctly rounded for every draw (tests/test_quotients.py): the product with its reciprocal and the
+  // remainder's correction, eight instructions less than a division
   constexpr double d = 2147483646.0, r = 1.0 / d;
   const double n = static_cast<double>(draw - 1u), q = n * r;
   return __builtin_fma(__builtin_fma(-d, q, n), r, q);
