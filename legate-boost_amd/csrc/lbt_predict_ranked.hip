@@ -497,25 +497,29 @@ __global__ void __launch_bounds__(kWalkThreads, 4)
 // The same for the features of one 128-byte line of a row, where their tables leave two such workgroups to a CU. Eight lanes take a row's
 // line, 16 bytes each: a wave's load so touches eight whole lines (a row a lane touched 64, once for each of its eight loads of 16
 // bytes: without any search 500,003 x 200 took 186 of 202 us that way). The values are turned in the LDS, and then a lane has a row and a
-// wave four or eight features, whose search it keeps in scalar registers; the rows of one feature share many of its LDS reads.
-// What bounds it is the memory: 500,003 x 200 (0.6 GB) 158 us. A line whose tables are larger than the room beside the rows must not fall to a
-// search in memory: of 40 trees of depth 8 on 2,000,000 x 100 doubles with a third of the thresholds on the 16 features of one line the calls take 886 us with
-// fewer cells for that line, 1035 with its tables in the rows' place, 1726 searched in memory; with 0.6 of them 1049 (in the rows' place) and
-// 1724; without any such line 855. Floats need no more than fewer cells (2,000,000 x 200, 50 trees, 0.6 on one line: 1226 and 2181).
-constexpr int kLineRows = 256;  // rows of a turn
-constexpr int kFewCells = 64;   // cells of a feature at least
+// wave two, four or eight features, whose search it keeps in scalar registers; the rows of one feature share many of its LDS reads.
+// What bounds it is the memory: 500,003 x 200 (0.6 GB) 143 us. A line with more thresholds than there is room for beside the rows has fewer cells,
+// a probe more for each half of them, before it falls to a search in memory, every probe a load: 50 trees of depth 8 on 2,000,000 x 200, a share of 0.6 of
+// the thresholds on one line of floats 1204 us a call (2180 searched in memory, 1104 evenly), of 0.33 on one line of doubles 1525 (3377, 1456).
+constexpr int kFewCells = 64;  // cells of a feature at least
 template <typename T>
 constexpr int kLineFeatures = 128 / sizeof(T);
-template <typename T>
-constexpr int kLinePitch = kLineRows + (sizeof(T) == 4 ? 2 : 4);  // the eight lanes of a row, eight rows: 64 banks
-template <typename T>
-constexpr int kLineStage = kLineFeatures<T> * kLinePitch<T> * static_cast<int>(sizeof(T));
-template <typename T>
+// kRows: rows of a turn
+template <typename T, int kRows>
+constexpr int kLinePitch = kRows + (sizeof(T) == 4 ? 2 : 4);  // the eight lanes of a row, eight rows: 64 banks
+template <typename T, int kRows>
+constexpr int kLineStage = kLineFeatures<T> * kLinePitch<T, kRows> * static_cast<int>(sizeof(T));
+inline size_t line_stage(size_t value_size, int rows)
+{
+  return value_size == 4 ? kLineStage<float, 256> : (rows == 256 ? kLineStage<double, 256> : kLineStage<double, 128>);
+}
+template <typename T, int kRows>
 __global__ void __launch_bounds__(kWalkThreads, 8)
   rank_lines_kernel(const T* __restrict__ X, RankRows a, RankState st, const T* __restrict__ sorted, uint16_t* __restrict__ ranks)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  constexpr int kAll = kLineFeatures<T>, kPer = 16 / sizeof(T), kPitch = kLinePitch<T>;
+  constexpr int kAll = kLineFeatures<T>, kPer = 16 / sizeof(T), kPitch = kLinePitch<T, kRows>;
+  constexpr int kLoads = kRows * 8 / kWalkThreads, kShares = kWalkWaves / (kRows / 64);  // of a thread; waves that share a row's features
   __shared__ int s_most[kAll], s_place[kAll], s_count[kAll];
   __shared__ T s_lo[kAll], s_scale[kAll];
   if (*st.overflow != 0) return;
@@ -529,7 +533,7 @@ __global__ void __launch_bounds__(kWalkThreads, 8)
     if (!asked) return;  // no tree asks for these features
   }
   // a lane's piece of its rows
-  const int q = tid & 7, r = tid >> 3, fq = f0 + kPer * q;  // rows r and r + 128
+  const int q = tid & 7, r = tid >> 3, fq = f0 + kPer * q;  // rows r + 128 u
   const int64_t begin = split * a.rows_per_split, end = min<int64_t>(a.n_rows, begin + a.rows_per_split);
   typedef T Vec __attribute__((ext_vector_type(kPer)));
   auto load = [&](int64_t row, T (&x)[kPer]) {
@@ -544,24 +548,20 @@ __global__ void __launch_bounds__(kWalkThreads, 8)
       for (int j = 0; j < kPer; j++) x[j] = src[min(fq + j, a.F - 1)];
     }
   };
-  T x0[kPer], x1[kPer];
-  if (begin < end) {
-    load(begin + r, x0);
-    load(begin + r + kLineRows / 2, x1);
-  }
-  // Tables beside the turned rows, with fewer cells if need be; those of doubles that are larger in the place of such rows too, whose values
-  // then come straight from memory; the largest stay in memory.
-  const int table   = (words + 1) * static_cast<int>(sizeof(T));
-  int cells         = a.cells;
-  if (table + 2 * kAll * kFewCells <= a.lds_bytes)
-    while (table + 2 * kAll * cells > a.lds_bytes) cells /= 2;
-  const int needed  = table + 2 * kAll * cells;
-  const bool held   = needed <= a.lds_bytes + (sizeof(T) == 8 ? kLineStage<T> : 0);
-  const bool turned = sizeof(T) == 4 || needed <= a.lds_bytes || !held;
+  T ahead[kLoads][kPer];
+  auto load_turn = [&](int64_t row0) {
+#pragma unroll
+    for (int u = 0; u < kLoads; u++) load(row0 + r + u * (kWalkThreads / 8), ahead[u]);
+  };
+  if (begin < end) load_turn(begin);
+  // Tables beside the turned rows, with fewer cells if need be, or else in memory.
+  const int table = (words + 1) * static_cast<int>(sizeof(T));
+  int cells       = a.cells;
+  while (cells > kFewCells && table + 2 * kAll * cells > a.lds_bytes) cells /= 2;
+  const bool held   = table + 2 * kAll * cells <= a.lds_bytes;
   T* const s_x      = reinterpret_cast<T*>(smem_raw);  // [kAll][kPitch]
-  const int table_at = turned ? kLineStage<T> / static_cast<int>(sizeof(T)) : 0;
-  T* const s_tab    = s_x + table_at;
-  uint16_t* s_start = reinterpret_cast<uint16_t*>(smem_raw + kLineStage<T> + a.lds_bytes - 2 * kAll * cells);  // [kAll][cells]
+  T* const s_tab    = reinterpret_cast<T*>(smem_raw + kLineStage<T, kRows>);
+  uint16_t* s_start = reinterpret_cast<uint16_t*>(smem_raw + kLineStage<T, kRows> + a.lds_bytes - 2 * kAll * cells);  // [kAll][cells]
   if (tid < kAll) {
     const int at = st.offset[f0 + min(tid, nf)];
     s_most[tid]  = 0;
@@ -577,8 +577,8 @@ __global__ void __launch_bounds__(kWalkThreads, 8)
   if (held) rank_cells<T, kAll>(cells, s_tab, s_start, s_place, s_count, s_most, s_lo, s_scale);
   __syncthreads();
   // a wave's features of 64 rows
-  constexpr int kOwn = kAll / 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), own = wave % 4 * kOwn, row_of = wave / 4 * 64 + (tid & 63);
+  constexpr int kOwn = kAll / kShares;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), own = wave % kShares * kOwn, row_of = wave / kShares * 64 + (tid & 63);
   int place[kOwn], probes[kOwn], most_probes = 0;
   T lo[kOwn], scale[kOwn];
   auto uniform = [](T v) {
@@ -591,16 +591,24 @@ __global__ void __launch_bounds__(kWalkThreads, 8)
   };
 #pragma unroll
   for (int j = 0; j < kOwn; j++) {
-    place[j]    = table_at + __builtin_amdgcn_readfirstlane(s_place[own + j]);
+    place[j]    = __builtin_amdgcn_readfirstlane(s_place[own + j]);
     probes[j]   = __builtin_amdgcn_readfirstlane(s_most[own + j]);
     lo[j]       = uniform(s_lo[own + j]);
     scale[j]    = uniform(s_scale[own + j]);
     most_probes = max(most_probes, probes[j]);
   }
   const uint16_t* const start = s_start + own * cells;
-  // ranks of a lane's values in the turn that begins with row0
-  auto rank_turn = [&](const T (&x)[kOwn], int64_t row0) {
+  for (int64_t row0 = begin; row0 < end; row0 += kRows) {
+#pragma unroll
+    for (int u = 0; u < kLoads; u++)
+#pragma unroll
+      for (int j = 0; j < kPer; j++) s_x[(kPer * q + j) * kPitch + r + u * (kWalkThreads / 8)] = ahead[u][j];
+    if (row0 + kRows < end) load_turn(row0 + kRows);
+    __syncthreads();
+    T x[kOwn];
     int at[kOwn];
+#pragma unroll
+    for (int j = 0; j < kOwn; j++) x[j] = s_x[(own + j) * kPitch + row_of];
     if (held) {
 #pragma unroll
       for (int j = 0; j < kOwn; j++) at[j] = start[j * cells + cell_of(x[j], lo[j], scale[j], cells)];
@@ -608,15 +616,15 @@ __global__ void __launch_bounds__(kWalkThreads, 8)
 #pragma unroll
         for (int j = 0; j < kOwn; j++) {
           if (p >= probes[j]) continue;  // (the same for the whole wave)
-          const T v = s_x[place[j] + ((1 << p) - 1) + at[j]];
+          const T v = s_tab[place[j] + ((1 << p) - 1) + at[j]];
           at[j] += v < x[j] ? 1 << p : 0;
         }
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < kOwn; j++) at[j] = lower_bound(sorted + first + (place[j] - table_at), s_count[own + j], x[j]);
+      for (int j = 0; j < kOwn; j++) at[j] = lower_bound(sorted + first + place[j], s_count[own + j], x[j]);
     }
-    const int64_t block = row0 + wave / 4 * 64;  // (a split ends with a block, or with the last row)
+    const int64_t block = row0 + wave / kShares * 64;  // (a split ends with a block, or with the last row)
     if (block < end) {
       uint32_t code[kOwn];
 #pragma unroll
@@ -626,42 +634,6 @@ __global__ void __launch_bounds__(kWalkThreads, 8)
       char* const base   = reinterpret_cast<char*>(ranks + (tile * a.F + f0 + own) * (int64_t(1) << a.tile_shift));
       store_ranks(code, nf - own, a.tile_shift, base + 2 * (static_cast<int>(block) & ((1 << a.tile_shift) - 1)));
     }
-  };
-  if (!turned) {
-    for (int64_t row0 = begin; row0 < end; row0 += kLineRows) {
-      const T* const src = X + min(row0 + row_of, end - 1) * a.F;
-      T x[kOwn];
-      if (a.wide) {
-#pragma unroll
-        for (int j = 0; j < kOwn; j += kPer) {
-          const int f = f0 + own + j;
-          const Vec v = *reinterpret_cast<const Vec*>(src + (f < a.F ? f : f0));
-#pragma unroll
-          for (int u = 0; u < kPer; u++) x[j + u] = v[u];
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < kOwn; j++) x[j] = src[min(f0 + own + j, a.F - 1)];
-      }
-      rank_turn(x, row0);
-    }
-    return;
-  }
-  for (int64_t row0 = begin; row0 < end; row0 += kLineRows) {
-#pragma unroll
-    for (int j = 0; j < kPer; j++) {
-      s_x[(kPer * q + j) * kPitch + r]                 = x0[j];
-      s_x[(kPer * q + j) * kPitch + r + kLineRows / 2] = x1[j];
-    }
-    if (row0 + kLineRows < end) {
-      load(row0 + kLineRows + r, x0);
-      load(row0 + kLineRows + r + kLineRows / 2, x1);
-    }
-    __syncthreads();
-    T x[kOwn];
-#pragma unroll
-    for (int j = 0; j < kOwn; j++) x[j] = s_x[(own + j) * kPitch + row_of];
-    rank_turn(x, row0);
     __syncthreads();
   }
 }
@@ -946,6 +918,7 @@ Shape walk_shape(int64_t N, int F, int K, int depth)
 struct Plan {
   Shape shape;
   int depth = 0, padded_trees = 0, group = 0, cells = 0, rank_lds = 0;
+  int turn_rows = 0;  // of features by the line
   int64_t slots = 0, thresholds = 0, chunk_rows = 0;
   bool may_overflow = false;
   size_t bytes = 0;
@@ -1014,18 +987,29 @@ Plan make_plan(int64_t N, int F, int n_trees, const int32_t* tree_nodes, int K, 
     return (group * mean + 4.0 * std::sqrt(group * mean) + group) * static_cast<double>(value_size) + 2.0 * group * p.cells;
   };
   // the features of a 128-byte line if two such workgroups share a CU; else at most eight, in powers of two
-  const int line = static_cast<int>(128 / value_size), stage = value_size == 4 ? kLineStage<float> : kLineStage<double>;
+  const int line = static_cast<int>(128 / value_size);
   if (F > kGroupMax && 2 * bytes_for(line) <= static_cast<double>(kLds / 2 - 1024)) {
-    p.group = line;
+    p.group     = line;
+    p.turn_rows = 256;
   } else {
     p.group = 1;
     while (p.group < kGroupMax && p.group < F && bytes_for(2 * p.group) <= static_cast<double>(kLds - 1024)) p.group *= 2;
   }
-  // what all thresholds on these features would take, or room for twice the mean; of a line's two workgroups to a CU: as much of that as is left beside
-  // the turned rows (46,592 bytes; rank_lines_kernel makes do with fewer cells, or takes the rows' place)
+  // what all thresholds on these features would take, or room for twice the mean; of a line as much as is left beside the turned rows. Turns of
+  // doubles are half as long where such a line would not have that with few cells: 63,232 bytes instead of 46,592 (2,000,000 x 100, 50 trees of depth 8, of
+  // which a share of 0.45 on one line 969 us; 1794 searched in memory, as with whole turns. 300,000 rows, evenly: 203 and 200)
+  const double twice = 2.0 * bytes_for(p.group);
+  double room        = std::max(twice, 32.0 * 1024), most_room = static_cast<double>(kLds - 1024);
+  if (p.group == line) {
+    most_room = static_cast<double>(kLds / 2 - 1024 - line_stage(value_size, p.turn_rows));
+    if (value_size == 8 && twice - 2.0 * line * (p.cells - kFewCells) > most_room) {
+      p.turn_rows = 128;
+      most_room   = static_cast<double>(kLds / 2 - 1024 - line_stage(value_size, p.turn_rows));
+    }
+    room = most_room;
+  }
   const double all_here = (static_cast<double>(thresholds) + 1) * static_cast<double>(value_size) + 2.0 * p.group * p.cells;
-  const double room     = std::min(all_here, std::max(2.0 * bytes_for(p.group), 32.0 * 1024)) + 15;
-  p.rank_lds = static_cast<int>(std::min(room, static_cast<double>(p.group == line ? kLds / 2 - 1024 - stage : kLds - 1024))) / 16 * 16;
+  p.rank_lds = static_cast<int>(std::min(std::min(all_here, room) + 15, most_room)) / 16 * 16;
   const int64_t tiles = (N + s.tile_rows - 1) / s.tile_rows;
   const int64_t most  = std::max<int64_t>(256, static_cast<int64_t>(kRankedChunkBytes / (static_cast<size_t>(s.tile_rows) * F * 2)) / 256 * 256);
   p.chunk_rows = std::min(tiles, most) * s.tile_rows;
@@ -1126,14 +1110,15 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
   rank_thresholds_kernel<T><<<dim3(F, p.thresholds > kSortMost<T> ? kRankBlocks : 1), kSortThreads,
                               sort_size * (sizeof(T) + sizeof(uint32_t)), stream>>>(st, static_cast<int>(sort_size), lay.grouped, lay.sorted);
 
-  static std::atomic<bool> rank_attr[5][kMaxDevices] = {};
+  static std::atomic<bool> rank_attr[6][kMaxDevices] = {};
   static std::atomic<bool> walk_attr[4][4][kMaxDevices] = {};
   auto whole_words = [&](const T* x) { return (static_cast<size_t>(F) * sizeof(T)) % 16 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0; };
-  auto rank_chunk = [&](auto group_c, std::atomic<bool> (&flags)[kMaxDevices], const T* x, int64_t rows) -> int {
-    constexpr int kG     = decltype(group_c)::value;
-    constexpr bool kLine = kG > kGroupMax;
+  // features of a workgroup; rows of a turn where they are those of a line, else 0
+  auto rank_chunk = [&](auto group_c, auto turn_c, std::atomic<bool> (&flags)[kMaxDevices], const T* x, int64_t rows) -> int {
+    constexpr int kG = decltype(group_c)::value, kTurn = decltype(turn_c)::value;
+    constexpr bool kLine = kTurn > 0;
     if constexpr (kLine)
-      LBT_TRY((allow_dynamic_lds(rank_lines_kernel<T>, kLds - 1024, flags)));
+      LBT_TRY((allow_dynamic_lds(rank_lines_kernel<T, kTurn>, kLds - 1024, flags)));
     else
       LBT_TRY((allow_dynamic_lds(rank_rows_kernel<T, kG>, kLds - 1024, flags)));
     RankRows a{};
@@ -1144,14 +1129,14 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
     a.cells     = p.cells;
     a.lds_bytes = p.rank_lds;
     // row ranges in multiples of the XCDs, as many as run at once
-    const size_t lds     = p.rank_lds + (kLine ? kLineStage<T> : 0);
+    const size_t lds     = p.rank_lds + (kLine ? line_stage(sizeof(T), kTurn) : 0);
     const int per_cu     = kLds / 2 >= lds + 1024 ? 2 : 1;
     const int64_t splits = 8 * std::max<int64_t>(1, std::min<int64_t>(32 * per_cu / a.n_groups, ceil_div(rows, 8 * kWalkThreads)));
     a.rows_per_split     = (rows + splits * kWalkThreads - 1) / (splits * kWalkThreads) * kWalkThreads;
     a.wide = whole_words(x) && kG * sizeof(T) >= 16;
     const unsigned grid = static_cast<unsigned>(splits * a.n_groups);
     if constexpr (kLine)
-      rank_lines_kernel<T><<<grid, kWalkThreads, lds, stream>>>(x, a, st, lay.sorted, lay.ranks);
+      rank_lines_kernel<T, kTurn><<<grid, kWalkThreads, lds, stream>>>(x, a, st, lay.sorted, lay.ranks);
     else
       rank_rows_kernel<T, kG><<<grid, kWalkThreads, lds, stream>>>(x, a, st, lay.sorted, lay.ranks);
     return LBT_OK;
@@ -1180,12 +1165,18 @@ int predict_ranked(hipStream_t stream, const T* X, int64_t N, int F, int n_trees
     const T* x = X + row * F;
     double* o  = out + row * K;
     const integral_constant<int, 1> one{};
+    const integral_constant<int, 0> none{};
     switch (p.group) {
-      case 1: LBT_TRY(rank_chunk(one, rank_attr[0], x, rows)); break;
-      case 2: LBT_TRY(rank_chunk(integral_constant<int, 2>{}, rank_attr[1], x, rows)); break;
-      case 4: LBT_TRY(rank_chunk(integral_constant<int, 4>{}, rank_attr[2], x, rows)); break;
-      case 8: LBT_TRY(rank_chunk(integral_constant<int, 8>{}, rank_attr[3], x, rows)); break;
-      default: LBT_TRY(rank_chunk(integral_constant<int, kLineFeatures<T>>{}, rank_attr[4], x, rows)); break;
+      case 1: LBT_TRY(rank_chunk(one, none, rank_attr[0], x, rows)); break;
+      case 2: LBT_TRY(rank_chunk(integral_constant<int, 2>{}, none, rank_attr[1], x, rows)); break;
+      case 4: LBT_TRY(rank_chunk(integral_constant<int, 4>{}, none, rank_attr[2], x, rows)); break;
+      case 8: LBT_TRY(rank_chunk(integral_constant<int, 8>{}, none, rank_attr[3], x, rows)); break;
+      default:
+        if (p.turn_rows == 256)
+          LBT_TRY(rank_chunk(integral_constant<int, kLineFeatures<T>>{}, integral_constant<int, 256>{}, rank_attr[4], x, rows));
+        else if constexpr (sizeof(T) == 8)
+          LBT_TRY(rank_chunk(integral_constant<int, kLineFeatures<T>>{}, integral_constant<int, 128>{}, rank_attr[5], x, rows));
+        break;
     }
     auto with = [&](auto adds_c, auto items_c, int at) -> int {
       switch (p.shape.j) {

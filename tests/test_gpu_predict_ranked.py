@@ -118,13 +118,13 @@ def test_last_features_of_a_cache_line(f, dtype):
     assert torch.equal(ops.predict(X, trees, 1), ops.predict(X, trees, 1, tiled=False))
 
 
-@pytest.mark.parametrize("f,n_trees,dtype", [(400, 100, np.float32), (403, 100, np.float32), (100, 40, np.float64), (103, 41, np.float64)])
+@pytest.mark.parametrize("f,n_trees,dtype", [(400, 100, np.float32), (403, 100, np.float32), (100, 40, np.float64), (103, 41, np.float64), (200, 50, np.float64)])
 @pytest.mark.parametrize("share", [0.0, 0.33, 0.6, 0.9])
 @pytest.mark.parametrize("last", [False, True])
 def test_thresholds_that_crowd_one_cache_line(f, n_trees, dtype, share, last):
-    """255 thresholds a tree, a share of them on the features of the first or of the last line of 128 bytes. At 0 all lines' tables lie
-    in the LDS beside the rows (46,592 bytes); at 0.33 those of 9810 floats or 4460 doubles have fewer cells; 6770 doubles (0.6) take the rows'
-    place as well; 15,000 floats and 9200 doubles are searched in memory."""
+    """255 thresholds a tree, a share of them on the features of the first or of the last line of 128 bytes. Evenly all lines' tables lie
+    in the LDS beside the rows (46,592 bytes; 63,232 beside turns of 128 rows, of 40 trees on doubles). A line of 9810 floats (0.33), 6770
+    (0.6 of 40 trees) or 4900 doubles (0.33 of 50) has fewer cells, one of 16,000 floats, 9200 or 8000 doubles is searched in memory."""
     rs = np.random.RandomState(f + int(100 * share))
     line = 128 // np.dtype(dtype).itemsize
     crowd = np.arange((f - 1) // line * line, f) if last else np.arange(line)
