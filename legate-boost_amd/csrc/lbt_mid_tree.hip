@@ -1005,12 +1005,12 @@ bool mid_tree_fits(int64_t N, int F, int K, int max_depth, int S)
 // more per entry (one workgroup per feature walks them in order, output by output); here it is the histograms that
 // count, and a scan workgroup per node and feature. The two sums are times of a tree in us, fitted to 190 shapes (300
 // to 8192 rows, 3 to 500 features, 1 to 16 outputs, depth 2 to 10, 64 to 1024 samples, float and double) when both
-// builders took a launch more per level, with 15 % in favour of the first. Of 188 shapes timed again since (1000 to 8192 rows, 8 to 250 features, 1 and
-// 4 outputs, depth 4 to 10) none where this builder is taken is slower for it; 24 where the first one is taken would be 3 to 38 % faster
-// here, most of them one output of 4097 to 6500 rows and up to 60 features: the line lies too high there. Both now, few rows against
-// medium: 8 features, depth 8 at 1000, 4096 and 8192 rows 83, 129, 215 and 138, 152, 156; 5000 x 8, depth 6 147 and 113; 8192 x 20,
-// depth 6 172 and 120; 8192 x 100, depth 8 221 and 239; 20 features, 4 outputs, depth 6 at 1000, 2000 and 8192 rows 148, 188, 582 and
-// 142, 151, 168.
+// builders took a launch more per level, with 15 % in favour of the first. Of 260 shapes timed again with the present kernels (1000 to 8192 rows,
+// 8 to 250 features, 1 and 4 outputs, depth 4 to 10) none where this builder is taken is slower for it; 34 where the first one is taken would be 4 to
+// 39 % faster here, most of them one output of 4500 to 6500 rows and up to 60 features: the line lies too high there. Both now, few rows
+// against medium: 8 features, depth 8 at 1000, 4096 and 8192 rows 83, 122, 209 and 135, 146, 145; 5000 x 8, depth 6 140 and 105; 8192 x 20,
+// depth 6 168 and 110; 20 features, 4 outputs, depth 6 at 1000, 2000 and 8192 rows 123, 154, 437 and 131, 134, 151; 8192 x 250 with 4, depth 8
+// 686 and 591.
 bool mid_beats_small(int64_t N, int F, int K, int max_depth, int S)
 {
   const double d = max_depth, n = static_cast<double>(N), f = F, k = K;

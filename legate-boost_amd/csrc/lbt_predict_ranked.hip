@@ -929,9 +929,11 @@ struct Plan {
 // over X that reads it and writes ranks (3.5 TB/s with its searches), node steps by how many trees a wave walks at once,
 // the leaf rows of several outputs (twice as dear once the ensemble's exceed an XCD's L2). Tiled: X at 3.2 TB/s, node
 // steps by the lanes a row takes and the share of a batch's trees that fits the LDS beside the rows, leaf rows. Rows that
-// do not fit the LDS are walked in memory, 60,000 steps a microsecond. Examples, tiled against ranks: 2,410,724 x 53, 333
-// trees of depth 7: 2689 and 1716 us; 2,087,561 x 104, 626 of depth 6: 5366 and 2688; 1,330,881 x 145 f64, 831 of depth 8:
-// 31.5 and 4.4 ms; 65,071 x 54, 229 of depth 7: 77 and 163; 2,070,925 x 35, 16 of depth 5: 248 and 321.
+// do not fit the LDS are walked in memory, 60,000 steps a microsecond. Since then a pass over X by the line and the packing of up to 64 trees became
+// shorter: of 93 other shapes of these ranges ten that are tiled would be 6 to 69 % faster by ranks (1,101,139 x 9 f64, 13 trees of depth 8,
+// 2 outputs 269 and 159 us), two that take ranks 3 % faster tiled. Examples, tiled against ranks: 2,410,724 x 53, 333
+// trees of depth 7: 2702 and 1766 us; 2,087,561 x 104, 626 of depth 6: 5394 and 2736; 1,330,881 x 145 f64, 831 of depth 8:
+// 31.5 and 4.35 ms; 65,071 x 54, 229 of depth 7: 91 and 201; 2,070,925 x 35, 16 of depth 5: 265 and 265.
 bool ranks_are_faster(int64_t N, int F, int n_trees, int depth, int K, size_t value_size, const Shape& shape)
 {
   const double rows = static_cast<double>(N), walks = rows * n_trees, steps = walks * depth;
