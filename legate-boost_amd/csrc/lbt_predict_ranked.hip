@@ -498,7 +498,7 @@ __global__ void __launch_bounds__(kWalkThreads, 4)
 // line, 16 bytes each: a wave's load so touches eight whole lines (a row a lane touched 64, once for each of its eight loads of 16
 // bytes: without any search 500,003 x 200 took 186 of 202 us that way). The values are turned in the LDS, and then a lane has a row and a
 // wave two, four or eight features, whose search it keeps in scalar registers; the rows of one feature share many of its LDS reads.
-// What bounds it is the memory: 500,003 x 200 (0.6 GB) 143 us. A line with more thresholds than there is room for beside the rows has fewer cells,
+// What bounds it is the memory: 500,003 x 200 (0.6 GB) 156 us. A line with more thresholds than there is room for beside the rows has fewer cells,
 // a probe more for each half of them, before it falls to a search in memory, every probe a load: 50 trees of depth 8 on 2,000,000 x 200, a share of 0.6 of
 // the thresholds on one line of floats 1204 us a call (2180 searched in memory, 1104 evenly), of 0.33 on one line of doubles 1525 (3377, 1456).
 constexpr int kFewCells = 64;  // cells of a feature at least
