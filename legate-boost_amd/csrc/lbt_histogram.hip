@@ -61,8 +61,7 @@ constexpr int kProbeSlack    = 8;   // further entries behind the last feature t
 // tile_start[j1 - j0] = total.
 __global__ void __launch_bounds__(kPlanThreads)
   plan_tiles_kernel(int j0, int j1, int level_first, const int32_t* seg, const I64Pair* node_sums,
-                    int K, int hist_node_begin, int hist_node_end, int tile_rows, int32_t* tile_start,
-                    LevelMeta* meta, LevelMeta* level_total)
+                    HistView hist, int tile_rows, int32_t* tile_start, LevelMeta* meta, LevelMeta* level_total)
 {
   // every thread owns a run of consecutive nodes: it counts their tiles, the workgroup scans the
   // 256 counts once, and the thread walks its run again to write the starts
@@ -74,11 +73,8 @@ __global__ void __launch_bounds__(kPlanThreads)
   const int begin = j0 + min(n, static_cast<int>(threadIdx.x) * per);
   const int end   = j0 + min(n, (static_cast<int>(threadIdx.x) + 1) * per);
   auto tiles_of = [&](int j, int& rows, bool& built) {
-    const int node   = level_first + j;
-    rows             = seg[j + 1] - seg[j];
-    const int parent = parent_of(node);
-    const bool pex   = parent >= hist_node_begin && parent < hist_node_end;
-    built            = compute_histogram_bin(node, node_sums, K, pex);
+    rows  = seg[j + 1] - seg[j];
+    built = hist.builds(level_first + j, node_sums);
     return built ? (rows + tile_rows - 1) / tile_rows : 0;
   };
   int mine = 0;
@@ -166,8 +162,7 @@ __global__ void __launch_bounds__(kPlanThreads)
 constexpr int kPlanFusedNodes = 4096;
 __global__ void __launch_bounds__(kPlanThreads)
   plan_expand_tiles_kernel(int j0, int j1, int level_first, const int32_t* __restrict__ seg,
-                           const I64Pair* __restrict__ node_sums, int K, int hist_node_begin, int hist_node_end,
-                           int tile_rows, int4* tiles, LevelMeta* meta, LevelMeta* level_total, int32_t* pair_sync,
+                           const I64Pair* __restrict__ node_sums, HistView hist, int tile_rows, int4* tiles, LevelMeta* meta, LevelMeta* level_total, int32_t* pair_sync,
                            int32_t* partial_count, int32_t* partial_list_count)
 {
   __shared__ int s_scan[kPlanThreads];
@@ -190,11 +185,8 @@ __global__ void __launch_bounds__(kPlanThreads)
   const int begin = j0 + min(n, static_cast<int>(threadIdx.x) * per);
   const int end   = j0 + min(n, (static_cast<int>(threadIdx.x) + 1) * per);
   auto tiles_of = [&](int j, int& rows, bool& built) {
-    const int node   = level_first + j;
-    rows             = seg[j + 1] - seg[j];
-    const int parent = parent_of(node);
-    const bool pex   = parent >= hist_node_begin && parent < hist_node_end;
-    built            = compute_histogram_bin(node, node_sums, K, pex);
+    rows  = seg[j + 1] - seg[j];
+    built = hist.builds(level_first + j, node_sums);
     return built ? (rows + tile_rows - 1) / tile_rows : 0;
   };
   int mine = 0;
@@ -2105,12 +2097,12 @@ int hist_launch_t(hipStream_t stream, const HistSetup& hs, const HistBatch& b, i
     int32_t* const pcount   = use_cache ? hs.partial_count : nullptr;
     if (b.n_nodes <= kPlanFusedNodes) {
       plan_expand_tiles_kernel<<<egrid, kPlanThreads, 0, stream>>>(
-        b.j0, b.j0 + b.n_nodes, b.level_first, b.seg, b.node_sums, b.K, b.hist.node_begin, b.hist.node_end, w.tile_rows,
+        b.j0, b.j0 + b.n_nodes, b.level_first, b.seg, b.node_sums, b.hist, w.tile_rows,
         hs.tiles, hs.meta, b.level_total, sync, pcount, hs.partial_list_count);
     } else {
       plan_tiles_kernel<<<1, kPlanThreads, 0, stream>>>(b.j0, b.j0 + b.n_nodes, b.level_first, b.seg, b.node_sums,
-                                                        b.K, b.hist.node_begin, b.hist.node_end, w.tile_rows,
-                                                        hs.tile_start, hs.meta, b.level_total);
+                                                        b.hist, w.tile_rows, hs.tile_start,
+                                                        hs.meta, b.level_total);
       expand_tiles_kernel<<<egrid, kPlanThreads, 0, stream>>>(b.j0, b.n_nodes, b.level_first, b.seg, hs.tile_start,
                                                               hs.meta, w.tile_rows, hs.tiles, sync, pcount,
                                                               hs.partial_list_count);

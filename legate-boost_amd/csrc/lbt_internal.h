@@ -352,10 +352,20 @@ struct HistView {
   int node_end;
   int K;
   int B;
+  // One byte per node, where the level's histograms are what the rows add up to, whatever the reference leaves
+  // unscanned above it (see build_tree_impl); else null. Set: the node's own histogram is not.
+  const uint8_t* tainted;
   __device__ bool contains(int node) const { return node >= node_begin && node < node_end; }
   __device__ I64Pair* at(int node, int k, int bin) const
   {
     return data + ((static_cast<int64_t>(node - node_begin) * K + k) * B + bin);
+  }
+  // Whether rows are added to the node's histogram (else it is its parent's without its sibling's)
+  __device__ bool builds(int node, const I64Pair* node_sums) const
+  {
+    const int parent = parent_of(node);
+    if (tainted != nullptr && node > 0 && contains(parent) && tainted[parent] != 0) return true;
+    return compute_histogram_bin(node, node_sums, K, contains(parent));
   }
 };
 

@@ -450,6 +450,30 @@ def test_levels_that_outgrow_the_histogram_budget_give_the_same_tree(n, f, k, s,
                 assert torch.equal(getattr(got, name), getattr(want, name)), (budget, observed, name)
 
 
+@pytest.mark.parametrize("n,f,k,s,depth", [(9001, 60, 8, 512, 9), (8200, 40, 3, 2048, 9), (9001, 50, 1, 512, 12)])
+@pytest.mark.parametrize("share,sign", [(0.02, 0), (0.5, 0), (0.5, -1), (0.97, -1)])
+def test_levels_that_outgrow_the_budget_with_hessians_of_zero(n, f, k, s, depth, share, sign):
+    """Unscanned bins in few and in most nodes of the levels above: siblings are derived below the reference's buffer only where
+    their parent's histogram is what its rows add up to. Equal to the reference's budget, whose levels are added up from all rows, and to its observed
+    build, bit for bit."""
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + k)
+    X = rs.randn(n, f).astype(np.float32)
+    X[:, 1] = np.round(X[:, 1])
+    g, h = rs.randn(n, k), 0.1 + rs.random_sample((n, k))
+    h[rs.rand(n, k) < share] = 0.0
+    if sign:
+        g = np.where(rs.rand(n, k) < 0.9, -np.abs(g), g)
+    X, g, h = (torch.from_numpy(a).cuda() for a in (X, g, h))
+    kw = dict(max_depth=depth, split_samples=s, seed=3, row_leaf=True)
+    got = ops.build_tree(X, g, h, **kw)
+    for observed in (False, True):
+        want = ops.build_tree(X, g, h, hist_cache_bytes=10 ** 9, taps=observed, **kw)
+        for name in ("leaf_value", "feature", "split_value", "gain", "hessian", "row_leaf"):
+            assert torch.equal(getattr(got, name), getattr(want, name)), (observed, name)
+
+
 def test_a_build_does_without_the_room_that_it_cannot_have(monkeypatch):
     """Where the room for the library's own budget of histograms cannot be had the build takes place in the
     reference's, and gives the same tree; an explicit budget is not cut."""
