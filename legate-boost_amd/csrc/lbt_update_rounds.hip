@@ -27,6 +27,8 @@ constexpr int kMostSums      = 4096;        // nodes * outputs of a tree: two su
 constexpr int kPackTrees     = 32;          // descriptors passed by value per launch
 constexpr size_t kLeafBytes  = 128u << 20;  // recorded leaves of one pass
 constexpr int kCopies        = 8;           // of a tree's sums: a workgroup adds to one of them
+constexpr int kLaneCopies    = 4;           // of the sums in a workgroup's LDS, where kCopiesLds holds them: rows of one node meet less often
+constexpr size_t kCopiesLds  = 64 * 1024;
 constexpr int kStagedPerStep = 80;          // a scattered cache line costs as much as about 100 bytes in sequence
 
 struct PackRefs {
@@ -36,17 +38,16 @@ struct PackRefs {
   int32_t n_nodes[kPackTrees];
 };
 
+// n trees, a row of workgroups each; the row behind them clears the sums
 template <typename T>
-__global__ void __launch_bounds__(256) pack_update_nodes_kernel(PackRefs refs, int F, PackedNode<T>* nodes)
+__global__ void __launch_bounds__(256) pack_update_nodes_kernel(PackRefs refs, int n, int F, PackedNode<T>* nodes, double* sums, int64_t n_sums)
 {
   const int t = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
+  if (t == n) {
+    for (int64_t s = i; s < n_sums; s += static_cast<int64_t>(gridDim.x) * 256) sums[s] = 0.0;
+    return;
+  }
   if (i < refs.n_nodes[t]) nodes[refs.node_off[t] + i] = pack_node<T>(i, refs.feature[t][i], refs.split[t][i], F, refs.n_nodes[t]);
-}
-
-__global__ void __launch_bounds__(256) zero_sums_kernel(double* a, int64_t n)
-{
-  const int64_t i = blockIdx.x * static_cast<int64_t>(256) + threadIdx.x;
-  if (i < n) a[i] = 0.0;
 }
 
 struct LeavesArgs {
@@ -148,6 +149,7 @@ __global__ void __launch_bounds__(kLeafThreads)
 struct RoundArgs {
   int64_t n_rows;
   int K, n_nodes, prev_nodes;  // prev_nodes: 0 in the first round
+  int lane_copies;             // of the sums in the LDS, a power of two
   double lr;
   const double* y;
   const double* weight;
@@ -173,40 +175,60 @@ enum class Gradient { kSquared, kLogistic, kSoftmax };
 // One round (see above): the leaf values of the tree before are formed by every workgroup from its sums, so nothing runs
 // between two rounds. The gradient is lbt_weighted_gradient's, operation by operation. kCols: the outputs where
 // they are known (1, or a softmax row in registers), 0 any number.
-// What bounds it: the workgroups' adds to the sums in memory (one address takes them in turn: with one copy of the sums 256
-// workgroups took 13.2 us and 1024 twice that; with 8 copies 8.2), then predictions, targets and leaves in one sweep (28 bytes
-// a row and output: 6 us).
-template <Gradient kKind, int kCols>
+// kCounts: squared errors of rows without weights, whose hessians are ones: they are counted (a 32-bit add of the LDS for one of 64 bits).
+// What bounds it, 1,000,000 rows and trees of depth 8: 4.4 us are the launch and its barriers, 1.8 the workgroups' adds to the sums in memory
+// (one address takes them in turn: with one copy of the sums 256 workgroups took 13.2 us in all; of 4, 8, 16 and 32 copies 8 are best), 1.2 each the sums of the
+// tree before and the rows, the rest the adds in the LDS (rows apart by lanes in kLaneCopies: 9.05 -> 8.5 us a launch, counts: 8.2).
+template <Gradient kKind, int kCols, bool kCounts>
 __global__ void __launch_bounds__(kRoundThreads) round_kernel(RoundArgs a)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int K = kCols > 0 ? kCols : a.K, n_sums = a.n_nodes * K, n_prev = a.prev_nodes * K, tid = threadIdx.x;
   double* s_prev = reinterpret_cast<double*>(smem_raw);  // [prev_nodes][K]
-  double* s_sum  = s_prev + n_prev;                      // [2][K][n_nodes]: nodes side by side in the banks
-  for (int i = tid; i < n_prev; i += kRoundThreads)
-    s_prev[i] = updated_leaf(sum_of_copies(a.prev_sums, n_prev, 0, i), sum_of_copies(a.prev_sums, n_prev, 1, i), a.prev_l1, a.prev_l2);
-  for (int i = tid; i < 2 * n_sums; i += kRoundThreads) s_sum[i] = 0.0;
-  __syncthreads();
-  auto add = [&](int node, int k, double g, double h) {
-    unsafeAtomicAdd(&s_sum[k * a.n_nodes + node], g);
-    unsafeAtomicAdd(&s_sum[n_sums + k * a.n_nodes + node], h);
-  };
+  double* s_sum  = s_prev + n_prev;                      // [lane_copies][2][K][n_nodes]: nodes side by side in the banks
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kRoundThreads;
   const int64_t first  = blockIdx.x * static_cast<int64_t>(kRoundThreads) + tid;
+  // one output: the values of the next kRows rows of a thread; the first ones are asked for before the sums of the tree before
+  constexpr int kRows = 4;
+  double p_next[kRows], y_next[kRows], w_next[kRows];
+  int node_next[kRows], prev_next[kRows];
+  auto fetch = [&](int64_t row0) {
+#pragma unroll
+    for (int u = 0; u < kRows; u++) {
+      const int64_t row = min(row0 + u * stride, a.n_rows - 1);
+      p_next[u]    = a.pred[row];
+      y_next[u]    = a.y[row];
+      w_next[u]    = a.weight != nullptr ? a.weight[row] : 1.0;
+      node_next[u] = a.leaf[row];
+      prev_next[u] = n_prev > 0 ? a.prev_leaf[row] : 0;
+    }
+  };
+  if constexpr (kCols == 1) fetch(first);
+  for (int i = tid; i < n_prev; i += kRoundThreads)
+    s_prev[i] = updated_leaf(sum_of_copies(a.prev_sums, n_prev, 0, i), sum_of_copies(a.prev_sums, n_prev, 1, i), a.prev_l1, a.prev_l2);
+  for (int i = tid; i < 2 * n_sums * a.lane_copies; i += kRoundThreads) s_sum[i] = 0.0;
+  __syncthreads();
+  double* const own_sum = s_sum + (tid & (a.lane_copies - 1)) * 2 * n_sums;
+  auto add = [&](int node, int k, double g, double h) {
+    unsafeAtomicAdd(&own_sum[k * a.n_nodes + node], g);
+    if constexpr (kCounts)
+      atomicAdd(reinterpret_cast<uint32_t*>(own_sum + n_sums) + (k * a.n_nodes + node), 1u);
+    else
+      unsafeAtomicAdd(&own_sum[n_sums + k * a.n_nodes + node], h);
+  };
   if constexpr (kCols == 1) {
-    constexpr int kRows = 4;  // rows whose values are on their way at once
     for (int64_t row0 = first; row0 < a.n_rows; row0 += kRows * stride) {
       double p[kRows], y[kRows], w[kRows];
       int node[kRows], prev[kRows];
 #pragma unroll
       for (int u = 0; u < kRows; u++) {
-        const int64_t row = min(row0 + u * stride, a.n_rows - 1);
-        p[u]    = a.pred[row];
-        y[u]    = a.y[row];
-        w[u]    = a.weight != nullptr ? a.weight[row] : 1.0;
-        node[u] = a.leaf[row];
-        prev[u] = n_prev > 0 ? a.prev_leaf[row] : 0;
+        p[u]    = p_next[u];
+        y[u]    = y_next[u];
+        w[u]    = w_next[u];
+        node[u] = node_next[u];
+        prev[u] = prev_next[u];
       }
+      if (row0 + kRows * stride < a.n_rows) fetch(row0 + kRows * stride);
 #pragma unroll
       for (int u = 0; u < kRows; u++) {
         const int64_t row = row0 + u * stride;
@@ -277,21 +299,19 @@ __global__ void __launch_bounds__(kRoundThreads) round_kernel(RoundArgs a)
   double* to = a.sums + static_cast<int64_t>(2) * n_sums * (blockIdx.x % kCopies);
   for (int i = tid; i < n_sums; i += kRoundThreads) {
     const int node = i / K, at = (i - node * K) * a.n_nodes + node;
-    const double gv = s_sum[at], hv = s_sum[n_sums + at];
+    auto hess_at = [&](int c) {
+      const double* h = s_sum + 2 * n_sums * c + n_sums;
+      if constexpr (kCounts) return static_cast<double>(reinterpret_cast<const uint32_t*>(h)[at]);
+      return h[at];
+    };
+    double gv = s_sum[at], hv = hess_at(0);
+    for (int c = 1; c < a.lane_copies; c++) {
+      gv += s_sum[2 * n_sums * c + at];
+      hv += hess_at(c);
+    }
     if (gv != 0.0) unsafeAtomicAdd(&to[i], gv);
     if (hv != 0.0) unsafeAtomicAdd(&to[n_sums + i], hv);
   }
-}
-
-// the last tree's leaf values
-__global__ void __launch_bounds__(256)
-  add_last_kernel(const double* __restrict__ leaf, const uint16_t* __restrict__ row_leaf, int64_t n, int K, double* pred)
-{
-  const int64_t i = blockIdx.x * static_cast<int64_t>(256) + threadIdx.x;
-  if (i >= n) return;
-  const int64_t r = K == 1 ? i : i / K;
-  const int k     = K == 1 ? 0 : static_cast<int>(i - r * K);
-  pred[i] += leaf[row_leaf[r] * K + k];
 }
 
 struct FinishRefs {
@@ -303,12 +323,41 @@ struct FinishRefs {
   int32_t n_nodes[kPackTrees];
 };
 
-// sums of inner nodes, leaf values and hessians: a workgroup per tree
-__global__ void __launch_bounds__(1024) finish_trees_kernel(FinishRefs refs, int K)
+// Sums of inner nodes, leaf values and hessians: a workgroup per tree. The workgroups behind them add the last of these trees' values to the
+// predictions: they form them from the sums, as a round does, and wait for no other launch (8.4 us and 6.2 behind it as two
+// launches on 1,000,000 rows with ten trees, one of 11.9).
+__global__ void __launch_bounds__(1024)
+  finish_trees_kernel(FinishRefs refs, int n_trees, int K, const uint16_t* __restrict__ row_leaf, int64_t n_pred, double* pred)
 {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int t = blockIdx.x, n = refs.n_nodes[t] * K;
+  const int t = min(static_cast<int>(blockIdx.x), n_trees - 1), n = refs.n_nodes[t] * K;
   double* g   = reinterpret_cast<double*>(smem_raw);
+  if (static_cast<int>(blockIdx.x) >= n_trees) {
+    constexpr int kEntries = 4;
+    const int64_t stride   = static_cast<int64_t>(gridDim.x - n_trees) * 1024;
+    const int64_t first    = static_cast<int64_t>(blockIdx.x - n_trees) * 1024 + threadIdx.x;
+    double p[kEntries];
+    int at[kEntries];
+    auto fetch = [&](int64_t i0) {
+#pragma unroll
+      for (int u = 0; u < kEntries; u++) {
+        const int64_t i = min(i0 + u * stride, n_pred - 1), r = K == 1 ? i : i / K;
+        at[u] = row_leaf[r] * K + static_cast<int>(i - r * K);
+        p[u]  = pred[i];
+      }
+    };
+    fetch(first);
+    for (int i = threadIdx.x; i < n; i += 1024)
+      g[i] = updated_leaf(sum_of_copies(refs.sums[t], n, 0, i), sum_of_copies(refs.sums[t], n, 1, i), refs.l1[t], refs.l2[t]);
+    __syncthreads();
+    for (int64_t i0 = first; i0 < n_pred; i0 += kEntries * stride) {
+#pragma unroll
+      for (int u = 0; u < kEntries; u++)
+        if (i0 + u * stride < n_pred) pred[i0 + u * stride] = p[u] + g[at[u]];
+      if (i0 + kEntries * stride < n_pred) fetch(i0 + kEntries * stride);
+    }
+    return;
+  }
   double* h   = g + n;
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
     g[i] = sum_of_copies(refs.sums[t], n, 0, i);
@@ -384,18 +433,24 @@ int update_rounds(hipStream_t stream, const T* X, int64_t N, int F, int objectiv
       refs.n_nodes[i]  = tree_nodes[first + i];
       widest           = std::max(widest, tree_nodes[first + i]);
     }
-    pack_update_nodes_kernel<T><<<dim3(ceil_div(widest, 256), n), 256, 0, stream>>>(refs, F, nodes);
+    const bool clears = first == 0;
+    const int wide    = clears ? std::max<int>(ceil_div(widest, 256), static_cast<int>(std::min<int64_t>(256, ceil_div(p.sums, 2048)))) : ceil_div(widest, 256);
+    pack_update_nodes_kernel<T><<<dim3(wide, n + (clears ? 1 : 0)), 256, 0, stream>>>(refs, n, F, nodes, sums, p.sums);
   }
-  zero_sums_kernel<<<ceil_div(p.sums, 256), 256, 0, stream>>>(sums, p.sums);
 
-  static std::atomic<bool> round_attr[13][kMaxDevices] = {}, finish_attr[kMaxDevices] = {};
+  static std::atomic<bool> round_attr[15][kMaxDevices] = {}, finish_attr[kMaxDevices] = {};
   const unsigned round_grid = static_cast<unsigned>(std::min<int64_t>(256, ceil_div(N, kRoundThreads)));
-  auto round = [&](auto kind_c, auto cols_c, std::atomic<bool> (&flags)[kMaxDevices], const RoundArgs& a) -> int {
+  auto round = [&](auto kind_c, auto cols_c, auto counts_c, std::atomic<bool> (&flags)[kMaxDevices], const RoundArgs& a) -> int {
     constexpr Gradient kKind = decltype(kind_c)::value;
     constexpr int kCols      = decltype(cols_c)::value;
-    LBT_TRY((allow_dynamic_lds(round_kernel<kKind, kCols>, 3 * kMostSums * sizeof(double), flags)));
-    const size_t lds = (static_cast<size_t>(a.prev_nodes) + 2 * static_cast<size_t>(a.n_nodes)) * K * sizeof(double);
-    round_kernel<kKind, kCols><<<round_grid, kRoundThreads, lds, stream>>>(a);
+    constexpr bool kCounts   = decltype(counts_c)::value;
+    LBT_TRY((allow_dynamic_lds(round_kernel<kKind, kCols, kCounts>, 3 * kMostSums * sizeof(double), flags)));
+    RoundArgs b      = a;
+    b.lane_copies    = 1;
+    const size_t one = 2 * static_cast<size_t>(a.n_nodes) * K * sizeof(double);
+    while (b.lane_copies < kLaneCopies && 2 * b.lane_copies * one <= kCopiesLds) b.lane_copies *= 2;
+    const size_t lds = static_cast<size_t>(a.prev_nodes) * K * sizeof(double) + b.lane_copies * one;
+    round_kernel<kKind, kCols, kCounts><<<round_grid, kRoundThreads, lds, stream>>>(b);
     return LBT_OK;
   };
   using std::integral_constant;
@@ -403,20 +458,27 @@ int update_rounds(hipStream_t stream, const T* X, int64_t N, int F, int objectiv
   using Logistic = integral_constant<Gradient, Gradient::kLogistic>;
   using Softmax  = integral_constant<Gradient, Gradient::kSoftmax>;
   auto run_round = [&](const RoundArgs& a) -> int {
+    const std::false_type sums{};
+    if (objective == LBT_OBJ_SQUARED_ERROR && weight == nullptr) {
+      const std::true_type counts{};
+      return K == 1 ? round(Squared{}, integral_constant<int, 1>{}, counts, round_attr[13], a)
+                    : round(Squared{}, integral_constant<int, 0>{}, counts, round_attr[14], a);
+    }
     if (objective == LBT_OBJ_SQUARED_ERROR)
-      return K == 1 ? round(Squared{}, integral_constant<int, 1>{}, round_attr[0], a) : round(Squared{}, integral_constant<int, 0>{}, round_attr[1], a);
+      return K == 1 ? round(Squared{}, integral_constant<int, 1>{}, sums, round_attr[0], a)
+                    : round(Squared{}, integral_constant<int, 0>{}, sums, round_attr[1], a);
     switch (K) {
-      case 1: return round(Logistic{}, integral_constant<int, 1>{}, round_attr[2], a);
-      case 2: return round(Softmax{}, integral_constant<int, 2>{}, round_attr[3], a);
-      case 3: return round(Softmax{}, integral_constant<int, 3>{}, round_attr[4], a);
-      case 4: return round(Softmax{}, integral_constant<int, 4>{}, round_attr[5], a);
-      case 5: return round(Softmax{}, integral_constant<int, 5>{}, round_attr[6], a);
-      case 6: return round(Softmax{}, integral_constant<int, 6>{}, round_attr[7], a);
-      case 7: return round(Softmax{}, integral_constant<int, 7>{}, round_attr[8], a);
-      case 8: return round(Softmax{}, integral_constant<int, 8>{}, round_attr[9], a);
-      case 10: return round(Softmax{}, integral_constant<int, 10>{}, round_attr[10], a);
-      case 16: return round(Softmax{}, integral_constant<int, 16>{}, round_attr[11], a);
-      default: return round(Softmax{}, integral_constant<int, 0>{}, round_attr[12], a);
+      case 1: return round(Logistic{}, integral_constant<int, 1>{}, sums, round_attr[2], a);
+      case 2: return round(Softmax{}, integral_constant<int, 2>{}, sums, round_attr[3], a);
+      case 3: return round(Softmax{}, integral_constant<int, 3>{}, sums, round_attr[4], a);
+      case 4: return round(Softmax{}, integral_constant<int, 4>{}, sums, round_attr[5], a);
+      case 5: return round(Softmax{}, integral_constant<int, 5>{}, sums, round_attr[6], a);
+      case 6: return round(Softmax{}, integral_constant<int, 6>{}, sums, round_attr[7], a);
+      case 7: return round(Softmax{}, integral_constant<int, 7>{}, sums, round_attr[8], a);
+      case 8: return round(Softmax{}, integral_constant<int, 8>{}, sums, round_attr[9], a);
+      case 10: return round(Softmax{}, integral_constant<int, 10>{}, sums, round_attr[10], a);
+      case 16: return round(Softmax{}, integral_constant<int, 16>{}, sums, round_attr[11], a);
+      default: return round(Softmax{}, integral_constant<int, 0>{}, sums, round_attr[12], a);
     }
   };
   const int slots = static_cast<int>(std::min<int64_t>(n_trees, 2 * p.pass_trees));  // tree t's leaves lie in slot t % slots
@@ -503,10 +565,10 @@ int update_rounds(hipStream_t stream, const T* X, int64_t N, int F, int objectiv
       refs.n_nodes[i] = tree_nodes[first + i];
       widest          = std::max(widest, tree_nodes[first + i]);
     }
-    finish_trees_kernel<<<n, 1024, 2 * static_cast<size_t>(widest) * K * sizeof(double), stream>>>(refs, K);
+    const int adders = first + n == n_trees ? static_cast<int>(std::min<int64_t>(256, ceil_div(N * K, 4096))) : 0;
+    finish_trees_kernel<<<n + adders, 1024, 2 * static_cast<size_t>(widest) * K * sizeof(double), stream>>>(
+      refs, n, K, row_leaf + static_cast<int64_t>((n_trees - 1) % slots) * N, N * K, pred);
   }
-  add_last_kernel<<<static_cast<unsigned>((N * K + 255) / 256), 256, 0, stream>>>(
-    leaf_out[n_trees - 1], row_leaf + static_cast<int64_t>((n_trees - 1) % slots) * N, N * K, K, pred);
   LBT_HIP(hipGetLastError());
   return LBT_OK;
 }
