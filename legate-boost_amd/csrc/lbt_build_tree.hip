@@ -1740,6 +1740,10 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     const bool decides = K == 1 && F <= kSmallDecideFeatures;
     st.cand[0]     = ar.take<SmallCand>(level_nodes * F);
     st.cand[1]     = decides ? ar.take<SmallCand>(level_nodes * F) : st.cand[0];
+    if (small_tree_levels_fit(N, F, K, max_depth)) {
+      st.sync  = ar.take<uint32_t>(kSmallDecideFeatures);
+      st.found = ar.take<unsigned long long>(3 * (2 * level_nodes - 1) * F);
+    }
     for (auto& left : st.left) left = decides ? ar.take<I64Pair>(level_nodes * F) : nullptr;
   }
   L.mid = MidTreeState{};

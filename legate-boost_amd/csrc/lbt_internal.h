@@ -591,7 +591,11 @@ struct SmallTreeState {
   double* scales;         // [4]
   SmallCand* cand[2];     // [nodes of a level][F]
   I64Pair* left[2];       // the same: what lies left of a candidate; null where no scan decides the level above it
+  // all levels in one launch (else null): see small_levels_kernel
+  uint32_t* sync;             // [kSmallDecideFeatures]
+  unsigned long long* found;  // [inner nodes][3][F]
 };
+bool small_tree_levels_fit(int64_t N, int F, int K, int max_depth);
 bool small_tree_fits(int64_t N, int F, int K, int max_depth, int S);
 // n_bins: receives the number of bins of all features (null: not wanted). level_totals: [max_depth], added
 // to (null: not wanted).

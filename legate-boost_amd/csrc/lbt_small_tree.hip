@@ -1,4 +1,4 @@
-// BuildTreeTask for inputs of few rows: 1 + 2 * max_depth launches instead of about ten per level.
+// BuildTreeTask for inputs of few rows: 2 launches, or 1 + 2 * max_depth, instead of about ten per level.
 //
 // The builder of lbt_build_tree.hip is made for rows by the million. With a few thousand of them its
 // launches do almost nothing (5 us each, about 90 for a tree of depth 8) and its histograms are
@@ -13,6 +13,8 @@
 //   small_scan_kernel       one workgroup per feature and level: carries its order over to the level
 //                           (a stable partition inside every node), running sums, gains, and the best
 //                           split of the feature per node (build_tree.cu:682-740)
+//   small_levels_kernel     one output, up to 64 features and 4096 rows, trees that are not too deep: all scans and decisions in one launch,
+//                           one workgroup per feature
 //   small_apply_kernel      one workgroup per node and level: best feature, the node's outputs and its
 //                           children (build_tree.cu:740-782), the side of each of its rows. Where a level has few
 //                           candidates every scan workgroup of the next one does that for itself (a launch less)
@@ -36,6 +38,7 @@ namespace {
 constexpr int kPrologueThreads = 1024;
 constexpr int kNone            = 0xffff;  // node_of_pos of a row whose node did not split
 constexpr int kQuantChunks     = 8;       // chunks of 4096 entries the quantiser's workgroup takes
+constexpr unsigned long long kNotFound = ~0ull;  // neither bits of a gain, nor a key and a bin, nor sums of hessians (see small_levels_kernel)
 
 struct PrologueArgs {
   int64_t row_offset;
@@ -289,6 +292,11 @@ __global__ void __launch_bounds__(kPrologueThreads, 8)
     }
   for (int64_t i = first; i < a.N; i += stride) st.node_of_pos[0][i] = 0;
   if (first >= 1 && first <= a.max_depth) st.live[first] = 0;
+  if (st.sync != nullptr) {
+    if (first < kSmallDecideFeatures) st.sync[first] = 0;
+    const int64_t words = 3 * ((int64_t(1) << a.max_depth) - 1) * a.F;
+    for (int64_t i = first; i < words; i += stride) st.found[i] = kNotFound;
+  }
 }
 
 struct LevelArgs {
@@ -1272,6 +1280,503 @@ __global__ void __launch_bounds__(kT)
     for (int i = tid; i < n; i += kT) node_of_pos[s0 + i] = static_cast<uint16_t>(2 * j + (i < lefts ? 0 : 1));
 }
 
+// ---------------------------------------------------------------- all levels in one launch
+
+constexpr int kLevelsMaxDepth = 10;
+constexpr int kLevelsPolls    = 400;   // looks (about 0.7 us apart) at what the others find before a workgroup takes a feature over
+
+thread_local int levels_polls = kLevelsPolls;
+
+struct LevelsArgs {
+  int N, F, S, max_depth;
+  int lanes_log;  // lanes per node where a level is decided, log2: at least F
+  bool all_bins;  // the bins of all features lie in the LDS
+  int polls;
+  double* leaf;
+  int32_t* feature;
+  double* split;
+  double* gain;
+  double* hessian;
+  int32_t* row_leaf;
+  unsigned long long* n_bins;  // pinned host memory: the number of all bins (see DeviceAnswer)
+  uint32_t tag;
+  const uint8_t* feature_set;
+  double l1, l2, min_split_gain;
+};
+
+__host__ __device__ constexpr size_t small_levels_use(int64_t N, int max_depth)
+{
+  return static_cast<size_t>((N + 1) / 2 * 2 * 8 + small_scan_order(N) * 4 + (int64_t(1) << (max_depth - 1)) * 100 + 15) / 16 * 16;
+}
+
+__device__ __forceinline__ unsigned long long agent_load(const unsigned long long* p)
+{
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void agent_store(unsigned long long* p, unsigned long long v)
+{
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// small_scan_kernel and the decisions between its levels for trees of one output, up to 64 features and 4096 rows: a workgroup keeps its
+// feature's order in registers and the nodes in the LDS from level to level, and the workgroups tell each other what they found through memory:
+// per node with rows and feature the gain, the place among equal gains and what lies left of the split, a word each that no launch
+// has written before (the prologue leaves kNotFound in all of them), so that a word is its own signal.
+// st.found: [node][gain, key and bin, left sums][F]; st.sync[f]: feature f has a workgroup.
+// No workgroup waits for one that may not run: a feature belongs to the workgroup that takes it first, which is its own unless that has not started
+// when another one has looked `polls` times for what it finds in the root; that one then takes the feature over. A workgroup with several features keeps their orders in memory.
+template <int kT, int kE>
+__global__ void __launch_bounds__(kT) small_levels_kernel(SmallTreeState st, LevelsArgs a)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int most = 1 << (a.max_depth - 1);  // nodes of a level
+  int2* const s_q                  = reinterpret_cast<int2*>(smem_raw);                              // [N]
+  uint32_t* const s_order          = reinterpret_cast<uint32_t*>(s_q + (a.N + 1) / 2 * 2);          // [small_scan_order(N)]
+  unsigned long long* const s_gain = reinterpret_cast<unsigned long long*>(s_order + small_scan_order(a.N));  // [most], as the others
+  double* const s_parent           = reinterpret_cast<double*>(s_gain + most);
+  double* const s_best             = s_parent + most;
+  uint2* const s_sums              = reinterpret_cast<uint2*>(s_best + most);   // [2][most] lower halves, as s_base and s_left
+  uint2* const s_bases             = s_sums + 2 * most;                          // [2][most]
+  int2* const s_segs               = reinterpret_cast<int2*>(s_bases + 2 * most);  // [2][most]
+  uint2* const s_left              = reinterpret_cast<uint2*>(s_segs + 2 * most);
+  int2* const s_split              = reinterpret_cast<int2*>(s_left + most);
+  unsigned* const s_key            = reinterpret_cast<unsigned*>(s_split + most);
+  int* const s_left_before         = reinterpret_cast<int*>(s_key + most);
+  int* const s_left_behind         = s_left_before + most;
+  uint16_t* const s_bins           = reinterpret_cast<uint16_t*>(smem_raw + small_levels_use(a.N, a.max_depth));  // all_bins: [F][pitch]
+  __shared__ uint2 s_wave_sums[kT / 64];
+  __shared__ int s_wave[kT / 64];
+  __shared__ unsigned s_taken;
+  __shared__ unsigned long long s_over;
+  __shared__ int s_splits;  // the last level with a split, counted from 1
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i0   = tid * kE;
+  const int pitch = static_cast<int>(st.pitch);
+  // features that are candidates, those with a workgroup (feature 0's writes the outputs), and the first bin of each
+  const unsigned long long usable = __ballot(lane < a.F && (a.feature_set == nullptr || a.feature_set[min(lane, a.F - 1)] != 0));
+  const unsigned long long parts  = usable | 1ull;
+  const int n_parts               = __popcll(parts);
+  const int bins_here             = lane < a.F ? st.counts[lane] : 0;
+  if (static_cast<int>(blockIdx.x) >= n_parts) return;
+  unsigned long long behind = parts;
+  for (int i = 0; i < static_cast<int>(blockIdx.x); i++) behind &= behind - 1;
+  const int f_first = __builtin_ctzll(behind);
+  if (tid == 0) s_taken = __hip_atomic_exchange(&st.sync[f_first], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int live     = st.live[0];
+  const double inv_g = st.scales[2], inv_h = st.scales[3];
+  const I64Pair all  = st.node_sums[0];
+  const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
+  uint32_t entry[kE];
+  load_u32<kE>(st.order[0] + static_cast<int64_t>(f_first) * pitch + min(i0, pitch - kE), entry);
+  {
+    int2 pair[kE];
+#pragma unroll
+    for (int u = 0; u < kE; u++) pair[u] = st.qgh[min(tid + u * kT, a.N - 1)];
+    if (a.all_bins)
+      copy_ahead<kT, 4>(a.F * (pitch / 8), [&](int i) { return reinterpret_cast<const uint4*>(st.bins)[i]; },
+                        [&](int i, const uint4& v) { reinterpret_cast<uint4*>(s_bins)[i] = v; });
+#pragma unroll
+    for (int u = 0; u < kE; u++)
+      if (tid + u * kT < a.N) s_q[tid + u * kT] = pair[u];
+  }
+  const int bins_before = static_cast<int>(wave_inclusive_sum32(static_cast<uint32_t>(bins_here))) - bins_here;
+  if (f_first == 0 && tid == 0)
+    __hip_atomic_store(a.n_bins,
+                       (static_cast<unsigned long long>(a.tag) << 32) |
+                         static_cast<unsigned>(__builtin_amdgcn_readlane(bins_before + bins_here, 63)),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (live == 0) return;  // data for the other builder
+  // sums are formed in their lower halves, see small_scan_kernel
+  const int64_t range  = (int64_t(1) << 31) + a.N + 1024;
+  const uint32_t down_g = static_cast<uint32_t>((range - all.grad) / 2 + 1), down_h = static_cast<uint32_t>((range - all.hess) / 2 + 1);
+  const double from_g = static_cast<double>(down_g), from_h = static_cast<double>(down_h);
+  auto grads  = [&](uint32_t v) { return static_cast<double>(v) - from_g; };  // of a sum with `down` added
+  auto hesses = [&](uint32_t v) { return static_cast<double>(v) - from_h; };
+  if (tid == 0) {
+    s_splits    = 0;
+    s_over      = 0;
+    s_sums[0]   = make_uint2(static_cast<uint32_t>(all.grad), static_cast<uint32_t>(all.hess));
+    s_bases[0]  = make_uint2(0, 0);
+    s_segs[0]   = make_int2(0, a.N);
+    s_parent[0] = leaf_gain(static_cast<double>(all.grad) * inv_g, static_cast<double>(all.hess) * inv_h, a.l1, reg);
+  }
+  const bool plain = plain_quotients(a.l1, inv_g, inv_h, reg);
+  auto term_of = [&](double grad, double hess) { return plain ? quotient_plain(grad * grad, hess + reg) : leaf_gain(grad, hess, a.l1, reg); };
+  auto gain_of = [&](double lg, double lh, double rg, double rh, double parent) {
+    lg *= inv_g, rg *= inv_g, lh *= inv_h, rh *= inv_h;
+    if (plain) return 0.0 + ((0.5 * (quotient_plain(lg * lg, lh + reg) + quotient_plain(rg * rg, rh + reg) - parent)) - a.min_split_gain);
+    return 0.0 + ((0.5 * (leaf_gain(lg, lh, a.l1, reg) + leaf_gain(rg, rh, a.l1, reg) - parent)) - a.min_split_gain);
+  };
+  // (the writer) node `at` has split: its outputs and its children's
+  auto write_split = [&](int at, const int2& s, double best, const uint2& ls, const uint2& rs) {
+    const int to       = 2 * at + 1;
+    const double value = st.proposals[static_cast<int64_t>(s.x) * a.S + s.y];
+    const double lg = grads(ls.x + down_g) * inv_g, lh = hesses(ls.y + down_h) * inv_h;
+    const double rg = grads(rs.x + down_g) * inv_g, rh = hesses(rs.y + down_h) * inv_h;
+    a.feature[at]     = s.x;
+    a.gain[at]        = best;
+    a.leaf[to]        = calculate_leaf_value(lg, lh, a.l1, a.l2);
+    a.leaf[to + 1]    = calculate_leaf_value(rg, rh, a.l1, a.l2);
+    a.hessian[to]     = lh;
+    a.hessian[to + 1] = rh;
+    a.split[at]       = value;
+  };
+  int node[kE], child[kE], node_next, child_next;
+#pragma unroll
+  for (int e = 0; e < kE; e++) node[e] = child[e] = i0 + e < a.N ? 0 : kNone;
+  node_next = child_next = i0 + kE < a.N ? 0 : kNone;
+  __syncthreads();
+  if (s_taken != 0) return;
+  unsigned long long owned = 1ull << f_first, todo = owned;
+  bool writes       = f_first == 0;
+  bool first_here   = true;  // the first feature of the level
+  for (int d = 0;;) {
+    const int n_nodes = 1 << d, n_above = n_nodes / 2, above_first = n_above - 1;
+    const int cur = (d & 1) * most, above = most - cur;  // this level's half of the nodes' sums, and the other one
+    const bool single = (owned & (owned - 1)) == 0;
+    const int f       = __builtin_ctzll(todo);
+    todo &= todo - 1;
+    const int rp = __builtin_amdgcn_readlane(bins_before, f);
+    if (!single || (d == 0 && !first_here))
+      load_u32<kE>(st.order[d == 0 ? 0 : (d - 1) & 1] + static_cast<int64_t>(f) * pitch + min(i0, pitch - kE), entry);
+    for (int j = tid; j < n_nodes; j += kT) {
+      s_gain[j] = 0;
+      s_key[j]  = 0;
+    }
+    if (d > 0) {
+      // the feature's order of this level: a stable partition inside every node that has split
+      unsigned left = 0, goes_on = 0;
+      int2 sp[kE], at[kE];
+      int b[kE];
+#pragma unroll
+      for (int e = 0; e < kE; e++) {
+        // (no branches around the looks into the LDS: behind one, each is waited for before the next is asked for)
+        const int2 s = s_split[node[e] != kNone ? node[e] : 0];
+        sp[e]        = make_int2(node[e] != kNone ? s.x : -1, s.y);
+        at[e]        = s_segs[above + (node[e] != kNone ? node[e] : 0)];
+      }
+      auto bin_at = [&](int e) { return max(sp[e].x, 0) * pitch + min(static_cast<int>(entry[e] & 0xffff), a.N - 1); };
+      if (a.all_bins) {
+#pragma unroll
+        for (int e = 0; e < kE; e++) b[e] = s_bins[bin_at(e)];
+      } else {
+#pragma unroll
+        for (int e = 0; e < kE; e++) b[e] = st.bins[bin_at(e)];
+      }
+      if (writes && first_here && a.row_leaf != nullptr) {
+#pragma unroll
+        for (int e = 0; e < kE; e++)
+          if (node[e] != kNone && sp[e].x < 0) a.row_leaf[entry[e] & 0xffff] = above_first + node[e];
+      }
+#pragma unroll
+      for (int e = 0; e < kE; e++) {
+        goes_on |= sp[e].x >= 0 ? 1u << e : 0u;
+        left |= sp[e].x >= 0 && b[e] <= sp[e].y ? 1u << e : 0u;
+      }
+      const int before = block_exclusive_sum32<kT>(__popc(left), s_wave);
+#pragma unroll
+      for (int e = 0; e < kE; e++)
+        if ((goes_on >> e) & 1u) {
+          if (at[e].x == i0 + e) s_left_before[node[e]] = before + __popc(left & ((1u << e) - 1u));
+          if (at[e].x + at[e].y - 1 == i0 + e) s_left_behind[node[e]] = before + __popc(left & ((2u << e) - 1u));
+        }
+      const int next          = node_next != kNone ? node_next : 0;
+      const bool next_goes_on = node_next != kNone && s_split[next].x >= 0;
+      const int2 next_at      = s_segs[above + next];
+      const int mine          = min(tid, n_above - 1);
+      const bool splits       = s_split[mine].x >= 0;
+      const int2 mine_at      = s_segs[above + mine];
+      __syncthreads();
+      int first[kE], lefts[kE];
+#pragma unroll
+      for (int e = 0; e < kE; e++) {
+        const int j = node[e] != kNone ? node[e] : 0;
+        first[e]    = s_left_before[j];
+        lefts[e]    = s_left_behind[j] - first[e];
+      }
+      const int next_lefts = s_left_behind[next] - s_left_before[next], mine_lefts = s_left_behind[mine] - s_left_before[mine];
+#pragma unroll
+      for (int e = 0; e < kE; e++) {
+        const int i = i0 + e;
+        const int l = before + __popc(left & ((1u << e) - 1u)) - first[e];
+        const bool goes = ((goes_on >> e) & 1u) != 0;
+        const int to    = !goes ? i : (left >> e) & 1u ? at[e].x + l : i + lefts[e] - l;
+        child[e]        = goes ? 2 * node[e] + (i - at[e].x < lefts[e] ? 0 : 1) : kNone;
+        if (i < a.N) s_order[to] = entry[e];
+      }
+      child_next = next_goes_on ? 2 * node_next + (i0 + kE - next_at.x < next_lefts ? 0 : 1) : kNone;
+      if (tid < n_above) {
+        s_segs[cur + 2 * tid]     = make_int2(mine_at.x, splits ? mine_lefts : 0);
+        s_segs[cur + 2 * tid + 1] = make_int2(mine_at.x + (splits ? mine_lefts : 0), splits ? mine_at.y - mine_lefts : 0);
+      }
+      __syncthreads();
+      if (i0 < a.N) load_u32<kE>(s_order + i0, entry);
+      if (!single && i0 < a.N) store_u32<kE>(st.order[d & 1] + static_cast<int64_t>(f) * pitch + i0, entry);
+    } else {
+      // the neighbour's first bin is looked up below
+      if (i0 < a.N) s_order[i0] = entry[0];
+      __syncthreads();
+    }
+    unsigned long long* const found = st.found + static_cast<int64_t>(n_nodes - 1) * 3 * a.F + f;  // node j: found[(3 * j + word) * F]
+    // (the writer) what the level above has to write, taken before this level's splits lie there
+    int2 was_split = make_int2(-1, 0);
+    double was_best = 0.0;
+    uint2 was_left = make_uint2(0, 0), was_right = make_uint2(0, 0);
+    if (writes && first_here && tid < n_above) {
+      was_split = s_split[tid];
+      was_best  = s_best[tid];
+      was_left  = s_sums[cur + 2 * tid];
+      was_right = s_sums[cur + 2 * tid + 1];
+    }
+    if ((usable >> f & 1) != 0) {
+      // occupied bins, running sums and gains, the best split per node: as small_scan_kernel
+      int bin[kE + 1];
+#pragma unroll
+      for (int e = 0; e < kE; e++) bin[e] = static_cast<int>(entry[e] >> 16);
+      bin[kE] = i0 + kE < a.N ? static_cast<int>(s_order[i0 + kE] >> 16) : 0;
+      unsigned ends = 0;
+#pragma unroll
+      for (int e = 0; e < kE; e++) {
+        const int nn = e + 1 < kE ? child[e + 1] : child_next;
+        if (child[e] != kNone && nn == child[e] && bin[e + 1] != bin[e]) ends |= 1u << e;
+      }
+      int2 q[kE];
+      uint2 sum = make_uint2(0, 0);
+#pragma unroll
+      for (int e = 0; e < kE; e++) {
+        q[e] = i0 + e < a.N ? s_q[entry[e] & 0xffff] : make_int2(0, 0);
+        sum.x += static_cast<uint32_t>(q[e].x);
+        sum.y += static_cast<uint32_t>(q[e].y);
+      }
+      const uint32_t ig = wave_inclusive_sum32(sum.x), ih = wave_inclusive_sum32(sum.y);
+      if (lane == 63) s_wave_sums[wave] = make_uint2(ig, ih);
+      __syncthreads();
+      uint2 run = make_uint2(ig - sum.x, ih - sum.y);
+#pragma unroll
+      for (int w = 0; w < kT / 64; w++) {
+        run.x += w < wave ? s_wave_sums[w].x : 0;
+        run.y += w < wave ? s_wave_sums[w].y : 0;
+      }
+      int first_node = kNone, own = kNone;
+      double first_gain = 0.0, own_gain = 0.0;
+      unsigned first_key = 0, own_key = 0;
+      uint2 first_left = make_uint2(0, 0), own_left = make_uint2(0, 0);  // with `down` added
+      auto put_left = [&](int j, const uint2& left) {
+        agent_store(found + static_cast<int64_t>(3 * j + 2) * a.F, static_cast<unsigned long long>(left.x) << 32 | left.y);
+      };
+      double gain[kE];
+      bool wanted[kE];
+      uint2 left_of[kE];
+#pragma unroll
+      for (int e = 0; e < kE; e++) {
+        run.x += static_cast<uint32_t>(q[e].x);
+        run.y += static_cast<uint32_t>(q[e].y);
+        const int j       = cur + (child[e] != kNone ? child[e] : 0);
+        const uint2 total = s_sums[j], base = s_bases[j];
+        const double parent = s_parent[j - cur];
+        const uint2 ls  = make_uint2(run.x + down_g - base.x, run.y + down_h - base.y);
+        const uint2 rs  = make_uint2(total.x + base.x + down_g - run.x, total.y + base.y + down_h - run.y);
+        const double lh = hesses(ls.y), rh = hesses(rs.y);
+        wanted[e]  = ((ends >> e) & 1u) != 0 && lh > 0 && rh > 0;
+        gain[e]    = gain_of(grads(ls.x), lh, grads(rs.x), rh, parent);
+        left_of[e] = ls;
+      }
+      // (a node without a candidate here is none of those that the thread has to report)
+#pragma unroll
+      for (int e = 0; e < kE; e++)
+        if (wanted[e] && gain[e] > 0) {
+          if (child[e] != own) {
+            if (first_node == kNone) {
+              first_node = own;  // (kNone again while there was none before)
+              first_gain = own_gain;
+              first_key  = own_key;
+              first_left = own_left;
+            } else if (own_key != 0) {
+              s_gain[own] = static_cast<unsigned long long>(__double_as_longlong(own_gain));
+              s_key[own]  = own_key;
+              put_left(own, own_left);
+            }
+            own      = child[e];
+            own_gain = 0.0;
+            own_key  = 0;
+          }
+          if (gain[e] >= own_gain) {
+            const unsigned key = tie_key(rp, bin[e], bin[e + 1]);
+            const bool better  = gain[e] > own_gain || key > own_key;
+            own_left.x         = better ? left_of[e].x : own_left.x;
+            own_left.y         = better ? left_of[e].y : own_left.y;
+            own_key            = gain[e] > own_gain ? key : max(own_key, key);
+            own_gain           = gain[e];
+          }
+        }
+      // one slot for the node the thread begins with, one for the node it ends with (the same one, or none)
+      if (first_node == kNone) {
+        first_node = own;
+        first_gain = own_gain;
+        first_key  = own_key;
+        first_left = own_left;
+        own_key    = 0;
+      }
+      const int begins_in      = first_node;
+      const unsigned begin_key = first_key;
+      const unsigned long long first_bits = static_cast<unsigned long long>(__double_as_longlong(first_gain));
+      const unsigned long long own_bits   = static_cast<unsigned long long>(__double_as_longlong(own_gain));
+      // where a whole wave lies in one node its lanes meet first
+      const unsigned long long have = __ballot(first_key != 0 || own_key != 0);
+      bool alone = true;
+      if (have != 0) {
+        const int wave_node = __builtin_amdgcn_readlane(first_node, __builtin_ctzll(have));
+        alone               = !__all(own_key == 0 && (first_key == 0 || first_node == wave_node));
+        if (!alone) {
+          double top   = first_key != 0 ? first_gain : 0.0;
+          unsigned key = first_key;
+          wave_best_key(top, key);
+          first_node = wave_node;
+          first_gain = top;
+          first_key  = lane == 0 ? key : 0u;
+        }
+      }
+      const unsigned long long mine_bits = alone ? first_bits : static_cast<unsigned long long>(__double_as_longlong(first_gain));
+      if (first_key != 0) atomicMax(&s_gain[first_node], mine_bits);
+      if (own_key != 0) atomicMax(&s_gain[own], own_bits);
+      __syncthreads();
+      if (first_key != 0 && mine_bits == s_gain[first_node]) atomicMax(&s_key[first_node], first_key);
+      if (own_key != 0 && own_bits == s_gain[own]) atomicMax(&s_key[own], own_key);
+      __syncthreads();
+      // (keys of different bins differ, but one lane can hold an equal key of a smaller gain only for another bin: none)
+      if (begin_key != 0 && begin_key == s_key[begins_in]) put_left(begins_in, first_left);
+      if (own_key != 0 && own_key == s_key[own]) put_left(own, own_left);
+      for (int j = tid; j < n_nodes; j += kT) {
+        if (s_segs[cur + j].y == 0) continue;  // nobody asks
+        const unsigned key = s_key[j];
+        const int rel      = 2047 - static_cast<int>((key - 1u) & 2047u);
+        unsigned long long* const to = found + static_cast<int64_t>(3 * j) * a.F;
+        agent_store(to, key != 0 ? s_gain[j] : 0ull);
+        agent_store(to + a.F, key != 0 ? static_cast<unsigned long long>(tie_key_of_bin(rp + rel)) << 32 | static_cast<unsigned>(rel) : 0ull);
+        if (key == 0) agent_store(to + 2 * a.F, 0ull);
+      }
+    } else {
+      __syncthreads();  // (as the feature's sums do: the splits of the level above are no longer asked for)
+    }
+    if (was_split.x >= 0) write_split(above_first + tid, was_split, was_best, was_left, was_right);
+    first_here = false;
+    if (todo != 0 || !single) __syncthreads();  // (the next feature's places)
+    if (todo != 0) continue;
+    if (d + 1 == a.max_depth && !writes) return;
+    // the splits of the level's nodes: 2^lanes_log lanes a node, a feature each
+    const int up = cur, down = above;
+    const int sub = tid & ((1 << a.lanes_log) - 1), turn = kT >> a.lanes_log;
+    const bool asks = sub < a.F && (usable >> min(sub, 63) & 1) != 0;
+    constexpr int kTurns = 2;
+    for (int j0 = tid >> a.lanes_log; j0 - (tid >> a.lanes_log) < n_nodes; j0 += kTurns * turn) {
+      unsigned long long g_of[kTurns], k_of[kTurns], l_of[kTurns];
+      bool here[kTurns];
+#pragma unroll
+      for (int u = 0; u < kTurns; u++) here[u] = asks && j0 + u * turn < n_nodes && s_segs[up + min(j0 + u * turn, n_nodes - 1)].y > 0;
+      bool any = false;
+#pragma unroll
+      for (int u = 0; u < kTurns; u++) {
+        any |= here[u];
+        g_of[u] = k_of[u] = l_of[u] = 0;
+      }
+      for (int polls = 0; __any(any);) {
+#pragma unroll
+        for (int u = 0; u < kTurns; u++) {
+          const unsigned long long* const at = st.found + static_cast<int64_t>(3 * (n_nodes - 1 + min(j0 + u * turn, n_nodes - 1))) * a.F + min(sub, a.F - 1);
+          g_of[u] = agent_load(at);
+          k_of[u] = agent_load(at + a.F);
+          l_of[u] = agent_load(at + 2 * a.F);
+        }
+        bool waits = false;
+#pragma unroll
+        for (int u = 0; u < kTurns; u++) waits |= here[u] && (g_of[u] == kNotFound || k_of[u] == kNotFound || l_of[u] == kNotFound);
+        if (!__any(waits)) break;
+        if (d > 0 || ++polls <= a.polls) continue;
+        // a feature of the root without a workgroup, or with one that is on its way
+        polls = 0;
+        const unsigned long long alone = __ballot(waits && __hip_atomic_load(&st.sync[sub], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0);
+        const bool takes = alone != 0 && lane == static_cast<int>(__builtin_ctzll(alone)) &&
+                           __hip_atomic_exchange(&st.sync[sub], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+        if (__any(takes)) {
+          if (takes) s_over = 1ull << sub;
+          break;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kTurns; u++) {
+        // gains are not negative: their bits compare as whole numbers, upper halves first
+        const int j           = j0 + u * turn;
+        const unsigned own_hi = here[u] ? static_cast<unsigned>(g_of[u] >> 32) : 0u, own_lo = here[u] ? static_cast<unsigned>(g_of[u]) : 0u;
+        const unsigned own_key = here[u] ? static_cast<unsigned>(k_of[u] >> 32) : 0u;
+        const unsigned hi  = group_max_u32(own_hi, a.lanes_log);
+        const unsigned lo  = group_max_u32(own_hi == hi ? own_lo : 0u, a.lanes_log);
+        const unsigned key = group_max_u32(own_hi == hi && own_lo == lo ? own_key : 0u, a.lanes_log);
+        const double best  = __longlong_as_double(static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo));
+        const bool splits  = key != 0 && best > 1e-5;
+        if (j < n_nodes) {
+          if (!splits && sub == 0) s_split[j] = make_int2(-1, 0);
+          if (splits && here[u] && own_hi == hi && own_lo == lo && own_key == key) {  // (keys of different candidates differ: one lane)
+            s_splits   = d + 1;
+            s_split[j] = make_int2(sub, static_cast<int>(k_of[u] & 0xffffffffull));
+            s_best[j]  = best;
+            s_left[j]  = make_uint2(static_cast<uint32_t>(l_of[u] >> 32) - down_g, static_cast<uint32_t>(l_of[u]) - down_h);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    if (d == 0 && s_over != 0) {
+      // features that this workgroup has taken over
+      todo = s_over;
+      owned |= todo;
+      writes |= (todo & 1) != 0;
+      __syncthreads();
+      if (tid == 0) {
+        s_over   = 0;
+        s_splits = 0;
+      }
+      continue;
+    }
+    d++;
+    todo       = owned;
+    first_here = true;
+#pragma unroll
+    for (int e = 0; e < kE; e++) node[e] = child[e];
+    node_next = child_next;
+    const int n_up = n_nodes, up_first = n_nodes - 1;
+    const bool ends = d == a.max_depth || s_splits != d;
+    if (!ends && tid < 2 * n_up) {
+      // (a thread for each child; without a split they have no rows and nobody asks for them)
+      const int j = tid >> 1, side = tid & 1;
+      const bool splits = s_split[j].x >= 0;
+      const uint2 total = s_sums[up + j], base = s_bases[up + j], ls = splits ? s_left[j] : make_uint2(0, 0);
+      const uint2 own   = side == 0 || !splits ? ls : make_uint2(total.x - ls.x, total.y - ls.y);
+      s_sums[down + tid]  = own;
+      s_bases[down + tid] = side == 0 ? base : make_uint2(base.x + ls.x, base.y + ls.y);
+      s_parent[tid]       = term_of(grads(own.x + down_g) * inv_g, hesses(own.y + down_h) * inv_h);
+    }
+    if (ends) {
+      if (writes && tid < n_up && s_split[tid].x >= 0) {
+        const uint2 total = s_sums[up + tid], ls = s_left[tid];
+        write_split(up_first + tid, s_split[tid], s_best[tid], ls, make_uint2(total.x - ls.x, total.y - ls.y));
+      }
+      if (writes && a.row_leaf != nullptr) {
+        if ((owned & (owned - 1)) != 0)
+          load_u32<kE>(st.order[(d - 1) & 1] + min(i0, pitch - kE), entry);  // (feature 0's)
+#pragma unroll
+        for (int e = 0; e < kE; e++)
+          if (node[e] != kNone) {
+            const int2 s  = s_split[node[e]];
+            const int row = static_cast<int>(entry[e] & 0xffff), at = up_first + node[e];
+            a.row_leaf[row] = s.x < 0 ? at : 2 * at + (st.bins[s.x * pitch + row] <= s.y ? 1 : 2);
+          }
+      }
+      return;
+    }
+  }
+}
+
 // For the profiler: what the histograms of the level would be built from.
 __global__ void __launch_bounds__(256) small_count_kernel(SmallTreeState st, LevelArgs a, LevelMeta* total)
 {
@@ -1337,6 +1842,17 @@ int launch_small_scan(hipStream_t stream, const SmallTreeState& st, const LevelA
   return launch_small_scan_as<kT, kE, true, kG, true, false>(stream, st, a, more);
 }
 
+template <int kT, int kE>
+int launch_small_levels(hipStream_t stream, const SmallTreeState& st, const LevelsArgs& a, size_t lds)
+{
+  static std::atomic<bool> attr_set[kMaxDevices] = {};
+  LBT_REQUIRE(a.N <= kT * kE && a.F <= kSmallDecideFeatures && a.max_depth <= kLevelsMaxDepth, "%d rows do not take a workgroup of %d places",
+              a.N, kT * kE);
+  LBT_TRY((allow_dynamic_lds(small_levels_kernel<kT, kE>, kScanLds, attr_set)));
+  small_levels_kernel<kT, kE><<<a.F, kT, lds, stream>>>(st, a);
+  return LBT_OK;
+}
+
 // Whether the scan of the level below level `depth` finds this level's splits for itself: one output, a lane for every
 // feature and kDecidePasses of them for the nodes, a thread for every node, and the LDS for both levels' nodes.
 bool next_scan_decides(const SmallTreeState& st, int64_t N, int F, int K, int depth, int max_depth)
@@ -1362,6 +1878,17 @@ bool small_tree_fits(int64_t N, int F, int K, int max_depth, int S)
          max_depth <= kSmallMaxDepth && small_scan_lds(N, int64_t(1) << (max_depth - 1)) <= kScanLds &&
          S <= LBT_MAX_SPLIT_SAMPLES && static_cast<int64_t>(F) * S < (int64_t(1) << 26) &&
          (static_cast<int64_t>(F) << (max_depth - 1)) <= (int64_t(1) << 22);
+}
+
+// All levels in one launch (small_levels_kernel) where a workgroup's look at a level's nodes, which every workgroup has to take for itself, stays
+// short: 16,384 lanes for the nodes of the last level, 8192 where a node takes a whole wave. Kernels of a tree and the gaps between them, us, before and
+// with one launch: 1000 x 10 depth 8 90 : 61, 500 x 4 depth 3 42 : 32, 4096 x 32 depth 8 135 : 116, 2000 x 32 depth 10 143 : 118,
+// 4096 x 64 depth 8 138 : 127; with more lanes 1000 x 64 depth 9 115 : 120, 4096 x 64 depth 10 173 : 199.
+bool small_tree_levels_fit(int64_t N, int F, int K, int max_depth)
+{
+  const int64_t last = int64_t(1) << (max_depth - 1);
+  return K == 1 && F <= kSmallDecideFeatures && N <= kDecideRows && max_depth <= kLevelsMaxDepth &&
+         (F > 32 ? 64 * last <= 8192 : F > 16 ? 32 * last <= 16384 : 16 * last <= 16384) && small_levels_use(N, max_depth) <= kScanLds;
 }
 
 template <typename T>
@@ -1394,8 +1921,36 @@ int small_tree_build(hipStream_t stream, const SmallTreeState& st, const T* X, i
     const size_t feature_lds = static_cast<size_t>(P) * (kProposalScratch<T> + 4) + 16 + N * 4 + 16;
     const size_t quant_lds   = (2048 + 2 * kQuantChunks + 4 + 2 * static_cast<size_t>(K)) * 8;
     const int64_t clear      = std::max<int64_t>(static_cast<int64_t>(prm.max_nodes) * K, N);
-    const int clearers       = static_cast<int>(std::min<int64_t>((clear + kPrologueThreads - 1) / kPrologueThreads, 64));
+    const int64_t words      = st.sync != nullptr ? 3 * static_cast<int64_t>(prm.max_nodes / 2) * F : 0;
+    const int clearers       = static_cast<int>(std::min<int64_t>((std::max(clear, words / 4) + kPrologueThreads - 1) / kPrologueThreads, 64));
     small_prologue_kernel<T><<<1 + F + clearers, kPrologueThreads, std::max(feature_lds, quant_lds), stream>>>(X, pa, st);
+  }
+  if (st.sync != nullptr && level_totals == nullptr) {
+    LevelsArgs a;
+    a.N = static_cast<int>(N); a.F = F; a.S = prm.split_samples; a.max_depth = prm.max_depth;
+    a.lanes_log = kDecideLanes;
+    while ((1 << a.lanes_log) < F) a.lanes_log++;
+    const size_t lds = small_levels_use(N, prm.max_depth), bins = static_cast<size_t>(F) * st.pitch * sizeof(uint16_t);
+    a.all_bins = lds + bins <= kScanLds;
+    a.polls    = levels_polls;
+    a.leaf = leaf; a.feature = feature; a.split = split; a.gain = gain; a.hessian = hessian; a.row_leaf = row_leaf;
+    a.n_bins = answer.words + 1;
+    a.tag    = answer.tag;
+    a.feature_set = feature_set;
+    a.l1 = prm.l1_regularization; a.l2 = prm.l2_regularization; a.min_split_gain = prm.min_split_gain;
+    ProfScope ps(LBT_PROF_HISTOGRAM, stream, 0.0, 0);
+    const size_t use = lds + (a.all_bins ? bins : 0);
+    if (N <= 1024)
+      LBT_TRY((launch_small_levels<512, 2>(stream, st, a, use)));
+    else if (N <= 2048)
+      LBT_TRY((launch_small_levels<1024, 2>(stream, st, a, use)));
+    else
+      LBT_TRY((launch_small_levels<1024, 4>(stream, st, a, use)));
+    LBT_HIP(hipGetLastError());
+    unsigned flags = 0;
+    LBT_TRY(answer.wait(&flags, n_bins));
+    *taken = flags == 0;
+    return LBT_OK;
   }
   LevelArgs a;
   a.N = static_cast<int>(N); a.F = F; a.K = K; a.S = prm.split_samples;
@@ -1460,3 +2015,6 @@ template int small_tree_build<double>(hipStream_t, const SmallTreeState&, const 
                                       int32_t*, double*, double*, double*, int32_t*, int32_t*, LevelMeta*, bool*);
 
 }  // namespace lbt
+
+// For tests, of the calling thread: with 0 looks features are taken over that nobody need take over; below 0: as it is without this call.
+extern "C" void lbt_small_levels_polls(int polls) { lbt::levels_polls = polls < 0 ? lbt::kLevelsPolls : polls; }
