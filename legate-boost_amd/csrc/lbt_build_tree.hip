@@ -64,17 +64,20 @@ __global__ void zero_kernel(uint4* p, int64_t n16)
   for (; i < n16; i += stride) p[i] = make_uint4(0, 0, 0, 0);
 }
 
-// Clears the histograms of the nodes of [node_begin, node_begin + gridDim.x) that rows will be added to: of two
-// siblings one, the other one is written whole by the scan. gridDim.y workgroups share a node.
-__global__ void __launch_bounds__(kThreads) zero_built_kernel(HistView hist, const I64Pair* node_sums, int node_begin)
+// Clears the node's histogram if rows will be added to it: of two siblings one, the other one is written whole by the scan. `parts`
+// workgroups share a node.
+__device__ __forceinline__ void clear_built(const HistView& hist, const I64Pair* node_sums, int node, int part, int parts)
 {
-  const int node = node_begin + blockIdx.x;
   if (node_sums[static_cast<int64_t>(node) * hist.K].hess <= 0) return;
   if (!hist.builds(node, node_sums)) return;
   uint4* const p   = reinterpret_cast<uint4*>(hist.at(node, 0, 0));
   const int64_t n  = static_cast<int64_t>(hist.K) * hist.B;
-  const int64_t st = static_cast<int64_t>(gridDim.y) * kThreads;
-  for (int64_t i = blockIdx.y * static_cast<int64_t>(kThreads) + threadIdx.x; i < n; i += st) p[i] = make_uint4(0, 0, 0, 0);
+  const int64_t st = static_cast<int64_t>(parts) * kThreads;
+  for (int64_t i = part * static_cast<int64_t>(kThreads) + threadIdx.x; i < n; i += st) p[i] = make_uint4(0, 0, 0, 0);
+}
+__global__ void __launch_bounds__(kThreads) zero_built_kernel(HistView hist, const I64Pair* node_sums, int node_begin)
+{
+  clear_built(hist, node_sums, node_begin + blockIdx.x, blockIdx.y, gridDim.y);
 }
 
 // ---------------------------------------------------------------------------
@@ -991,11 +994,11 @@ struct SlabSegments {
 
 // All threads of the workgroup call this; s_seg has kSegLds entries.
 __device__ inline SlabSegments load_slab_segments(const int32_t* __restrict__ seg, int n_parents,
-                                                  const int32_t* __restrict__ block_seg, int64_t base, int64_t n,
-                                                  int* s_seg)
+                                                  const int32_t* __restrict__ block_seg, int slab, int64_t base,
+                                                  int64_t n, int* s_seg)
 {
   SlabSegments ss;
-  ss.j0         = block_seg[blockIdx.x];
+  ss.j0         = block_seg[slab];
   const int end = static_cast<int>(base + kPartBlock < n ? base + kPartBlock : n);
   ss.m          = 0;
   // the starts ascend, so those inside the slab are a prefix of seg[j0+1 ..]
@@ -1069,7 +1072,7 @@ __global__ void __launch_bounds__(kThreads)
   __shared__ int s_d[kThreads / 64];
   __shared__ int s_l[kThreads / 64];
   const int64_t base    = blockIdx.x * static_cast<int64_t>(kPartBlock);
-  const SlabSegments ss = load_slab_segments(seg, n_parents, block_seg, base, n, s_seg);
+  const SlabSegments ss = load_slab_segments(seg, n_parents, block_seg, blockIdx.x, base, n, s_seg);
   int nd = 0, nl = 0;
 #pragma unroll
   for (int u = 0; u < kPartItems; u++) {
@@ -1100,13 +1103,75 @@ constexpr int kTransRows = 128;  // the feature-major bins are padded to whole g
 // decides the side and consecutive rows of a node read consecutive bytes.
 // kRun: a thread takes eight positions in a row: their row numbers are two loads, their codes one store, and mostly they
 // lie in one node; else positions kThreads apart, so that a wave's bins lie close together (see classify_in_runs).
-template <typename BinT, bool kRun>
+// kDecides: the level's splits have not been applied (split_apply_kernel): every workgroup finds those of the segments that meet its slab, a wave for
+// each, and the workgroup in whose slab a segment begins writes the node's outputs: a launch less a level.
+struct DecideArgs {
+  HistView hist;
+  I64Pair* node_sums;
+  const int32_t* bin_feature;
+  const double* proposals;
+  const double* scales;
+  double l1, l2;
+  int n_cands;  // per node
+  const Cand* partial;
+  double* leaf;
+  int32_t* feature;
+  double* split;
+  double* gain;
+  const int32_t* row_pointers;
+  int32_t* split_bin;
+};
+constexpr int kDecideCands = 512;  // of a node, at most: every slab reads those of its nodes
+constexpr int kDecideNodes = 512;
+// Every slab reads its nodes' candidates and waits for them, 1 us at 1,000,000 x 50 and 7 at 10,000,000 x 100, whose 4900 slabs are bound by
+// what they read; a launch of split_apply_kernel and the gap in front of it are 6 to 7.
+constexpr int64_t kDecideRows = int64_t(1) << 22;
+
+// The split of level node j by one wave: feature and bin in every lane, feature -1: none. writes: its outputs as well.
+__device__ __forceinline__ int2 decide_node(const DecideArgs& a, int level_first, int j, int lane, bool writes)
+{
+  const int node = level_first + j, K = a.hist.K;
+  const bool usable = a.node_sums[static_cast<int64_t>(node) * K].hess > 0;
+  Cand best{0.0, -1};
+  for (int c = lane; c < a.n_cands; c += 64) {
+    const Cand o = a.partial[static_cast<int64_t>(j) * a.n_cands + c];
+    if (cand_better(o, best)) best = o;
+  }
+  best = wave_best(best);
+  if (!usable || !(best.bin >= 0 && best.gain > 1e-5)) return make_int2(-1, 0);
+  const int ft = a.bin_feature[best.bin], bin = best.bin - a.row_pointers[ft];
+  if (writes) {
+    const double inv_g = a.scales[2], inv_h = a.scales[3];
+    const int lc = left_child(node), rc = right_child(node);
+    if (lane < K) {
+      const I64Pair ns = a.node_sums[static_cast<int64_t>(node) * K + lane];
+      const I64Pair ls = *a.hist.at(node, lane, best.bin);
+      const I64Pair rs{ns.grad - ls.grad, ns.hess - ls.hess};
+      a.node_sums[static_cast<int64_t>(lc) * K + lane] = ls;
+      a.node_sums[static_cast<int64_t>(rc) * K + lane] = rs;
+      a.leaf[static_cast<int64_t>(lc) * K + lane]      = calculate_leaf_value(
+        static_cast<double>(ls.grad) * inv_g, static_cast<double>(ls.hess) * inv_h, a.l1, a.l2);
+      a.leaf[static_cast<int64_t>(rc) * K + lane] = calculate_leaf_value(
+        static_cast<double>(rs.grad) * inv_g, static_cast<double>(rs.hess) * inv_h, a.l1, a.l2);
+    }
+    if (lane == 0) {
+      a.feature[node]   = ft;
+      a.split[node]     = a.proposals[best.bin];
+      a.gain[node]      = best.gain;
+      a.split_bin[node] = bin;
+    }
+  }
+  return make_int2(ft, bin);
+}
+
+template <typename BinT, bool kRun, bool kDecides>
 __global__ void __launch_bounds__(kThreads)
   classify_bins_kernel(const int32_t* __restrict__ rows, int64_t n, const int32_t* __restrict__ seg,
                        const int32_t* __restrict__ block_seg, int n_parents, int level_first,
                        const BinT* __restrict__ bins_t, int64_t bins_stride, const int32_t* feature,
-                       const int32_t* split_bin, uint8_t* code, int2* block_counts)
+                       const int32_t* split_bin, uint8_t* code, int2* block_counts, DecideArgs decide)
 {
+  __shared__ int2 s_split[kDecides ? kDecideNodes + 1 : 1];  // of the slab's segments
   __shared__ int s_seg[kSegLds];
   __shared__ int s_d[kThreads / 64];
   __shared__ int s_l[kThreads / 64];
@@ -1125,11 +1190,34 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
     for (int u = 0; u < kPartItems; u++) row[u] = i0 + u * kGap < n ? rows[i0 + u * kGap] : 0;
   }
-  const SlabSegments ss = load_slab_segments(seg, n_parents, block_seg, base, n, s_seg);
+  const SlabSegments ss = load_slab_segments(seg, n_parents, block_seg, blockIdx.x, base, n, s_seg);
+  if constexpr (kDecides) {
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    static_assert(kDecideNodes <= kSegLds, "the starts of a level's segments are in the LDS");
+    // (an empty segment has no rows that ask, and no split; the others begin in the one slab that has their first position)
+    int turn = 0;
+    for (int i0 = 0; i0 <= ss.m; i0 += 64) {
+      const int i    = i0 + lane;
+      const bool has = i <= ss.m && ss.j0 + i >= 0 && (i == ss.m || i == 0 || s_seg[i] > s_seg[i - 1]);
+      for (unsigned long long here = __ballot(has); here != 0; here &= here - 1) {
+        if ((turn++ & (kThreads / 64 - 1)) != wave) continue;
+        const int at    = i0 + __builtin_ctzll(here), j = ss.j0 + at;
+        const int begin = at > 0 ? s_seg[at - 1] : seg[j];
+        const int2 s    = decide_node(decide, level_first, j, lane, begin >= base);
+        if (lane == 0) s_split[at] = s;
+      }
+    }
+    __syncthreads();
+  }
   int ft[kPartItems], sb[kPartItems];
   auto look_up = [&](int u, int j) {
-    ft[u] = j >= 0 ? feature[level_first + j] : -1;
-    sb[u] = j >= 0 ? split_bin[level_first + j] : 0;
+    if constexpr (kDecides) {
+      const int2 s = j >= 0 ? s_split[j - ss.j0] : make_int2(-1, 0);
+      ft[u] = s.x, sb[u] = s.y;
+    } else {
+      ft[u] = j >= 0 ? feature[level_first + j] : -1;
+      sb[u] = j >= 0 ? split_bin[level_first + j] : 0;
+    }
   };
   auto segment_at = [&](int64_t i) { return i < n ? segment_of(ss, s_seg, seg, static_cast<int>(i)) : -1; };
   const int first = segment_at(i0);
@@ -1188,7 +1276,7 @@ __global__ void __launch_bounds__(kThreads)
 {
   __shared__ int s_seg[kSegLds];
   const int64_t base    = blockIdx.x * static_cast<int64_t>(kPartBlock);
-  const SlabSegments ss = load_slab_segments(seg, n_parents, block_seg, base, n, s_seg);
+  const SlabSegments ss = load_slab_segments(seg, n_parents, block_seg, blockIdx.x, base, n, s_seg);
 #pragma unroll
   for (int u = 0; u < kPartItems; u++) {
     const int64_t i = base + u * kThreads + threadIdx.x;
@@ -1452,15 +1540,36 @@ __device__ inline int prefix_popc(unsigned long long mask)
 // pass 3: scatter every row to its place in the next level's order. Rows are
 // taken in slabs of one workgroup width (coalesced); inside a slab the ranks
 // come from wave ballots, across waves and slabs from a 32-entry scan.
-__global__ void __launch_bounds__(kThreads)
-  scatter_kernel(const int32_t* __restrict__ rows, int64_t n, const uint8_t* code, const int2* block_offsets,
-                 const int32_t* __restrict__ seg, const int32_t* __restrict__ block_seg, const int2* seg_prefix,
-                 const int32_t* seg_next, int level_first, int n_parents, int32_t* rows_out, int32_t* row_leaf)
+struct ScatterArgs {
+  const int32_t* rows;
+  int64_t n;
+  const uint8_t* code;
+  const int2* block_offsets;
+  const int32_t* seg;
+  const int32_t* block_seg;
+  const int2* seg_prefix;
+  const int32_t* seg_next;
+  int level_first, n_parents;
+  int32_t* rows_out;
+  int32_t* row_leaf;
+};
+__device__ __forceinline__ void scatter_slab(const ScatterArgs& a, int slab)
 {
+  const int32_t* __restrict__ const rows      = a.rows;
+  const int32_t* __restrict__ const seg       = a.seg;
+  const int32_t* __restrict__ const block_seg = a.block_seg;
+  const int2* const block_offsets             = a.block_offsets;
+  const int2* const seg_prefix                = a.seg_prefix;
+  const int32_t* const seg_next               = a.seg_next;
+  const uint8_t* const code                   = a.code;
+  int32_t* const rows_out                     = a.rows_out;
+  int32_t* const row_leaf                     = a.row_leaf;
+  const int64_t n                             = a.n;
+  const int level_first = a.level_first, n_parents = a.n_parents;
   constexpr int kWaves = kThreads / 64;
   __shared__ int s_seg[kSegLds];
   __shared__ int s_cnt[kPartItems * kWaves];  // retired << 16 | left, in row order
-  const int64_t base = blockIdx.x * static_cast<int64_t>(kPartBlock);
+  const int64_t base = slab * static_cast<int64_t>(kPartBlock);
   const int wave     = threadIdx.x >> 6;
   int row[kPartItems];
   int c[kPartItems];
@@ -1476,8 +1585,8 @@ __global__ void __launch_bounds__(kThreads)
       c[u]   = code[i];
     }
   }
-  const SlabSegments ss = load_slab_segments(seg, n_parents, block_seg, base, n, s_seg);
-  const int2 boff       = block_offsets[blockIdx.x];
+  const SlabSegments ss = load_slab_segments(seg, n_parents, block_seg, slab, base, n, s_seg);
+  const int2 boff       = block_offsets[slab];
   // Per row: its segment and what its destination is counted from. A left row goes to
   // seg_next[2j] + (left rows of the segment before it), a right row to seg_next[2j+1] + (right
   // rows of the segment before it); both counts are differences of prefix counts, whose
@@ -1538,6 +1647,27 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
+__global__ void __launch_bounds__(kThreads) scatter_kernel(ScatterArgs a) { scatter_slab(a, blockIdx.x); }
+
+// What a level begins with, in one launch: its rows in their places, the tiles of its built nodes, and their histograms cleared. None of the
+// three waits for another; as launches of their own the tiles were 5 us and a gap behind every scatter, the clearing 6 to 65. With that and the
+// splits applied where rows are classified, kernels of a tree and their gaps, us: 1,000,000 x 50 depth 12 with 512 samples 1582 -> 1498, 1,000,000 x 60
+// with 3 outputs depth 10 1708 -> 1598, 2,000,000 x 120 depth 8 1696 -> 1617; 10,000,000 x 100, whose scatter is bound by memory, as before.
+__global__ void __launch_bounds__(kThreads) level_start_kernel(PlanArgs plan, ScatterArgs scatter, int n_slabs, int clear_from, int clear_parts)
+{
+  static_assert(kThreads == kPlanThreads, "one size of workgroup");
+  int block = blockIdx.x;
+  const int plan_blocks = (plan.blocks + 7) / 8 * 8;  // a slab stays with the XCD whose L2 has its rows and codes
+  if (block < plan_blocks) {
+    if (block < plan.blocks) plan_tiles_block(plan, block);
+    return;
+  }
+  block -= plan_blocks;
+  if (block < n_slabs) return scatter_slab(scatter, block);
+  block -= n_slabs;
+  clear_built(plan.hist, plan.node_sums, clear_from + block / clear_parts, block % clear_parts, clear_parts);
+}
+
 // The reference's (node, row) pairs, for the observation points: node of the level that the
 // order belongs to, -1 for retired rows.
 __global__ void __launch_bounds__(kThreads)
@@ -1546,7 +1676,7 @@ __global__ void __launch_bounds__(kThreads)
 {
   __shared__ int s_seg[kSegLds];
   const int64_t base    = blockIdx.x * static_cast<int64_t>(kPartBlock);
-  const SlabSegments ss = load_slab_segments(seg, n_parents, block_seg, base, n, s_seg);
+  const SlabSegments ss = load_slab_segments(seg, n_parents, block_seg, blockIdx.x, base, n, s_seg);
 #pragma unroll
   for (int u = 0; u < kPartItems; u++) {
     const int64_t i = base + u * kThreads + threadIdx.x;
@@ -2102,13 +2232,24 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
   const bool use_bins_t = hs.binned != nullptr && L.bins_t != nullptr;
   int32_t* row_leaf     = taps ? taps->row_leaf : nullptr;
   const int n_chunks = (B + kSplitChunk - 1) / kSplitChunk;
+  ScatterArgs scatter{};
+  bool scatter_due = false;
+  auto scatter_now = [&]() {
+    if (!scatter_due) return;
+    ProfScope ps(LBT_PROF_POSITIONS, stream, static_cast<double>(N) * (4 + 1 + 4));
+    scatter_kernel<<<blocks(N, kPartBlock), kThreads, 0, stream>>>(scatter);
+    scatter_due = false;
+  };
   for (int depth = 0; depth < max_depth; depth++) {
     const int64_t nodes_in_level = int64_t(1) << depth;
     const int level_first        = static_cast<int>(level_begin(depth));
-    if (taps && taps->positions_per_level)
+    if (taps && taps->positions_per_level) {
+      scatter_now();
       expand_positions_kernel<<<blocks(N, kPartBlock), kThreads, 0, stream>>>(
         L.rows[cur_pos], N, L.seg[cur_seg], L.block_seg[cur_seg], static_cast<int>(nodes_in_level), level_first,
         reinterpret_cast<int2*>(taps->positions_per_level) + static_cast<size_t>(depth) * N);
+    }
+    int clear_from = 0, clear_nodes = 0, clear_parts = 1;  // built histograms of the level to clear
     const bool direct = lazy && depth >= direct_from;
     if (lazy && !direct) {
       const int64_t end = level_end(depth);
@@ -2118,10 +2259,9 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
         if (strict) hv.tainted = L.tainted;
       }
       if (end <= hv.node_end && hv.node_begin == 0 && end > cleared_end) {
-        const int from    = std::max(cleared_end, level_first);
-        const int64_t per = std::max<int64_t>(1, std::min<int64_t>(static_cast<int64_t>(K) * B / (4 * kThreads), 64));
-        zero_built_kernel<<<dim3(static_cast<unsigned>(end - from), static_cast<unsigned>(per)), kThreads, 0, stream>>>(
-          hv, L.node_sums, from);
+        clear_from  = std::max(cleared_end, level_first);
+        clear_nodes = static_cast<int>(end) - clear_from;
+        clear_parts = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(static_cast<int64_t>(K) * B / (4 * kThreads), 64)));
         cleared_end = static_cast<int>(end);
       }
     }
@@ -2129,6 +2269,34 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
     const bool contained         = level_first >= hv.node_begin && level_end(depth) <= hv.node_end;
     int64_t num_batches          = 1;
     if (nodes_in_level > max_batch_size && !(lazy && contained)) num_batches = (nodes_in_level + max_batch_size - 1) / max_batch_size;
+    auto batch_of = [&](int j0, int j1) {
+      HistBatch hb;
+      hb.X = X; hb.F = F; hb.qgh = L.qgh; hb.K = K; hb.rows = L.rows[cur_pos]; hb.seg = L.seg[cur_seg];
+      hb.j0 = j0; hb.n_nodes = j1 - j0; hb.level_first = level_first; hb.proposals = L.proposals;
+      hb.row_pointers = L.row_pointers; hb.bin_feature = L.bin_feature; hb.hist = hv; hb.qstats = L.qstats; hb.node_sums = L.node_sums;
+      hb.level_total = L.level_totals + depth; hb.n_rows = N;
+      // the root's rows are still in their original order, and its launch fills the bin cache first
+      hb.fill_cache = depth == 0; hb.identity = depth == 0;
+      return hb;
+    };
+    bool planned = false, decides = false;  // decides: the level's splits are applied where its rows are classified
+    DecideArgs decide{};
+    if (scatter_due && !direct && num_batches == 1 && contained) {
+      PlanArgs plan;
+      LBT_TRY(hist_plan(hs, batch_of(0, static_cast<int>(nodes_in_level)), &plan));
+      if (plan.blocks > 0) {
+        ProfScope ps(LBT_PROF_POSITIONS, stream, static_cast<double>(N) * (4 + 1 + 4));
+        const unsigned nb = blocks(N, kPartBlock);
+        level_start_kernel<<<(plan.blocks + 7) / 8 * 8 + nb + clear_nodes * clear_parts, kThreads, 0, stream>>>(plan, scatter, static_cast<int>(nb), clear_from,
+                                                                                                 clear_parts);
+        scatter_due = false;
+        clear_nodes = 0;
+        planned     = true;
+      }
+    }
+    scatter_now();
+    if (clear_nodes > 0)
+      zero_built_kernel<<<dim3(clear_nodes, clear_parts), kThreads, 0, stream>>>(hv, L.node_sums, clear_from);
     if (direct) {
       const int64_t large16 = static_cast<int64_t>(direct_large_bytes(hs, N, range_of_large) / 16);
       if (!large_ready && large16 > 0) {
@@ -2167,13 +2335,8 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
       }
       const int n_nodes = j1 - j0;
       {
-        HistBatch hb;
-        hb.X = X; hb.F = F; hb.qgh = L.qgh; hb.K = K; hb.rows = L.rows[cur_pos]; hb.seg = L.seg[cur_seg];
-        hb.j0 = j0; hb.n_nodes = n_nodes; hb.level_first = level_first; hb.proposals = L.proposals;
-        hb.row_pointers = L.row_pointers; hb.bin_feature = L.bin_feature; hb.hist = hv; hb.qstats = L.qstats; hb.node_sums = L.node_sums;
-        hb.level_total = L.level_totals + depth; hb.n_rows = N;
-        // the root's rows are still in their original order, and its launch fills the bin cache first
-        hb.fill_cache = depth == 0; hb.identity = depth == 0;
+        HistBatch hb = batch_of(j0, j1);
+        hb.planned   = planned;
         LBT_TRY(hist_launch(stream, hs, hb, depth));
       }
       // One pass that scans and evaluates reads the histograms once instead of twice and saves a
@@ -2194,6 +2357,10 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
       const bool fused = narrow_sums_hold(N) && K <= kFusedMaxK && (K >= 2 || n_nodes <= 256 || !wanted);
       const bool store = !fused || wanted;
       kept             = store;
+      const int n_cands = fused ? F : n_chunks;
+      // (with negative hessians a node without rows may have a split)
+      decides = N <= kDecideRows && (depth == 0 || lazy) && depth < max_depth - 1 && use_bins_t && num_batches == 1 && store &&
+                n_cands <= kDecideCands && K <= 64 && nodes_in_level <= kDecideNodes;
       if (fused) {
         ProfScope ps(LBT_PROF_SCAN, stream);
         scan_split_launch(stream, hs.max_bins, hv, L.node_sums, F, L.row_pointers, batch_begin, n_nodes, feature_set,
@@ -2211,9 +2378,11 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
                                                          prm.l1_regularization, prm.l2_regularization,
                                                          prm.min_split_gain, batch_begin, n_chunks, L.partial);
       }
-      {
+      if (decides) {
+        decide = DecideArgs{hv, L.node_sums, L.bin_feature, L.proposals_d, L.scales, prm.l1_regularization, prm.l2_regularization, n_cands,
+                            L.partial, leaf, feature, split, gain, L.row_pointers, L.split_bin};
+      } else {
         ProfScope ps(LBT_PROF_SPLIT, stream);
-        const int n_cands = fused ? F : n_chunks;
         split_apply_kernel<<<n_nodes, 64, 0, stream>>>(hv, L.node_sums, L.bin_feature, L.proposals_d, L.scales,
                                                        prm.l1_regularization, prm.l2_regularization, batch_begin,
                                                        n_cands, L.partial, leaf, feature, split, gain, L.row_pointers,
@@ -2229,24 +2398,29 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
       const int32_t* bseg = L.block_seg[cur_seg];
       auto classify_bins = [&](auto kernel, const auto* bins) {
         kernel<<<nb, kThreads, 0, stream>>>(rows, N, seg, bseg, n_parents, level_first, bins, L.bins_t_stride, feature,
-                                            L.split_bin, L.code, L.block_counts);
+                                            L.split_bin, L.code, L.block_counts, decide);
       };
       const bool runs = classify_in_runs(n_parents, N);
+      auto classify_as = [&](auto bin, auto decides_c) {
+        using BinT          = decltype(bin);
+        constexpr bool kDec = decltype(decides_c)::value;
+        classify_bins(runs ? classify_bins_kernel<BinT, true, kDec> : classify_bins_kernel<BinT, false, kDec>,
+                      static_cast<const BinT*>(L.bins_t));
+      };
+      auto classify_of = [&](auto bin) { decides ? classify_as(bin, std::true_type{}) : classify_as(bin, std::false_type{}); };
       if (use_bins_t && hs.bin_bytes == 1)
-        classify_bins(runs ? classify_bins_kernel<uint8_t, true> : classify_bins_kernel<uint8_t, false>,
-                      static_cast<const uint8_t*>(L.bins_t));
+        classify_of(uint8_t{});
       else if (use_bins_t)
-        classify_bins(runs ? classify_bins_kernel<uint16_t, true> : classify_bins_kernel<uint16_t, false>,
-                      static_cast<const uint16_t*>(L.bins_t));
+        classify_of(uint16_t{});
       else
         classify_kernel<T><<<nb, kThreads, 0, stream>>>(rows, N, seg, bseg, n_parents, level_first, X, F, feature, split,
                                                         L.code, L.block_counts);
       child_segments_kernel<<<blocks(n_parents, kScanThreads / 64), kScanThreads, 0, stream>>>(
         seg, n_parents, N, L.code, L.block_counts, static_cast<int>(nb), L.block_offsets, L.seg_prefix,
         L.seg[cur_seg ^ 1], L.block_seg[cur_seg ^ 1]);
-      scatter_kernel<<<nb, kThreads, 0, stream>>>(rows, N, L.code, L.block_offsets, seg, bseg, L.seg_prefix,
-                                                  L.seg[cur_seg ^ 1], level_first, n_parents, L.rows[cur_pos ^ 1],
-                                                  row_leaf);
+      scatter = ScatterArgs{rows, N, L.code, L.block_offsets, seg, bseg, L.seg_prefix, L.seg[cur_seg ^ 1], level_first, n_parents,
+                            L.rows[cur_pos ^ 1], row_leaf};
+      scatter_due = true;  // with what the next level begins with
       cur_pos ^= 1;
       cur_seg ^= 1;
     }
@@ -3140,8 +3314,8 @@ int lbt_update_positions(void* stream, const void* X, int32_t x_dtype, int64_t n
   child_segments_kernel<<<blocks(n_parents, kScanThreads / 64), kScanThreads, 0, s>>>(
     L.seg[0], n_parents, N, L.code, L.block_counts, static_cast<int>(nb), L.block_offsets, L.seg_prefix, L.seg[1],
     L.block_seg[1]);
-  scatter_kernel<<<nb, kThreads, 0, s>>>(L.rows[0], N, L.code, L.block_offsets, L.seg[0], L.block_seg[0], L.seg_prefix,
-                                         L.seg[1], level_first, n_parents, L.rows[1], nullptr);
+  scatter_kernel<<<nb, kThreads, 0, s>>>(ScatterArgs{L.rows[0], N, L.code, L.block_offsets, L.seg[0], L.block_seg[0], L.seg_prefix, L.seg[1],
+                                                     level_first, n_parents, L.rows[1], nullptr});
   expand_positions_kernel<<<nb, kThreads, 0, s>>>(L.rows[1], N, L.seg[1], L.block_seg[1], 2 * n_parents,
                                                   static_cast<int>(level_begin(level + 1)), pairs);
   LBT_HIP(hipGetLastError());

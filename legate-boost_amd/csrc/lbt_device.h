@@ -552,4 +552,122 @@ __device__ inline int count_less(const T* p, int n, T x, int steps)
 }
 
 
+// The tiles of a batch, a workgroup of kPlanThreads for 256 of them: every workgroup
+// repeats the count and the scan of the nodes' tiles (a few loads per thread) instead of waiting
+// for a launch that does it once, then writes the descriptors of its own 256 tiles. Workgroup 0
+// also leaves the batch's totals and clears the counters of the launch that follows.
+// Bound by latency: the nodes' sums and segments, a scan, the descriptors. The scan is one barrier, the totals are summed by
+// waves, what they are added to is asked for at the start, and up to 256 nodes a descriptor needs nothing more from memory
+// (1,000,000 x 50, 8 to 256 nodes: 4.7, 5.7, 6.8, 10.5, 7, 9 us, now 4.8, 3.9, 3.6, 3.6, 3.3, 3.9).
+__device__ __forceinline__ void plan_tiles_block(const PlanArgs& a, int block)
+{
+  const int j0 = a.j0, j1 = a.j1, level_first = a.level_first, tile_rows = a.tile_rows;
+  const int32_t* __restrict__ const seg       = a.seg;
+  const I64Pair* __restrict__ const node_sums = a.node_sums;
+  const HistView& hist                        = a.hist;
+  int32_t* const pair_sync                    = a.pair_sync;
+  int32_t* const partial_count                = a.partial_count;
+  int32_t* const partial_list_count           = a.partial_list_count;
+  LevelMeta* const meta                       = a.meta;
+  LevelMeta* const level_total                = a.level_total;
+  int4* const tiles                           = a.tiles;
+  __shared__ int s_scan[kPlanThreads];
+  __shared__ int2 s_seg[kPlanThreads];
+  __shared__ int s_wave[kPlanThreads / 64];
+  __shared__ int64_t s_sums[3][kPlanThreads / 64];
+  const bool first_wg = block == 0;
+  LevelMeta level_before{};
+  if (first_wg) {
+    if (threadIdx.x == 0) level_before = *level_total;
+    if (pair_sync != nullptr)
+      for (int i = threadIdx.x; i < kPairSyncSlots; i += kPlanThreads) pair_sync[i] = 0;
+    if (partial_count != nullptr) {
+      if (threadIdx.x == 0) *partial_count = 0;
+      for (int i = threadIdx.x; i < kPartialMaxLists; i += kPlanThreads) partial_list_count[i] = 0;
+    }
+  }
+  const int n     = j1 - j0;
+  const int per   = (n + kPlanThreads - 1) / kPlanThreads;
+  const int begin = j0 + min(n, static_cast<int>(threadIdx.x) * per);
+  const int end   = j0 + min(n, (static_cast<int>(threadIdx.x) + 1) * per);
+  auto tiles_of = [&](int j, int& rows, bool& built) {
+    rows  = seg[j + 1] - seg[j];
+    built = hist.builds(level_first + j, node_sums);
+    return built ? (rows + tile_rows - 1) / tile_rows : 0;
+  };
+  int mine = 0;
+  int64_t rb = 0, rc = 0, nb = 0;
+  for (int j = begin; j < end; j++) {
+    int rows;
+    bool built;
+    mine += tiles_of(j, rows, built);
+    rb += rows;
+    if (built && rows > 0) {
+      rc += rows;
+      nb += 1;
+    }
+  }
+  // (a thread's only node: its tiles are written from here, by whoever owns them)
+  s_seg[threadIdx.x] = begin < end ? make_int2(seg[begin], seg[begin + 1]) : make_int2(0, 0);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int before = block_exclusive_sum32<kPlanThreads>(mine, s_wave);
+  s_scan[threadIdx.x] = before + mine;
+  if (first_wg) {
+    rb = wave_inclusive_sum(rb);
+    rc = wave_inclusive_sum(rc);
+    nb = wave_inclusive_sum(nb);
+    if (lane == 63) {
+      s_sums[0][wave] = rb;
+      s_sums[1][wave] = rc;
+      s_sums[2][wave] = nb;
+    }
+  }
+  __syncthreads();
+  const int total = s_scan[kPlanThreads - 1];
+  if (first_wg && threadIdx.x == 0) {
+    int64_t sum[3] = {0, 0, 0};
+    for (int q = 0; q < 3; q++)
+      for (int w = 0; w < kPlanThreads / 64; w++) sum[q] += s_sums[q][w];
+    meta->n_tiles         = total;
+    meta->instances       = sum[0];
+    meta->built_instances = sum[1];
+    meta->built_nodes     = sum[2];
+    level_total->instances       = level_before.instances + sum[0];
+    level_total->built_instances = level_before.built_instances + sum[1];
+    level_total->built_nodes     = level_before.built_nodes + sum[2];
+  }
+  const int tile = block * kPlanThreads + threadIdx.x;
+  if (tile >= total) return;
+  // the thread whose run of nodes holds the tile: the last one whose inclusive count exceeds it
+  int lo = 0, hi = kPlanThreads - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (s_scan[mid] > tile)
+      hi = mid;
+    else
+      lo = mid + 1;
+  }
+  if (per == 1) {
+    const int2 sg = s_seg[lo];
+    const int r0  = sg.x + (tile - (lo > 0 ? s_scan[lo - 1] : 0)) * tile_rows;
+    tiles[tile]   = make_int4(level_first + j0 + lo, r0, min(sg.y, r0 + tile_rows), sg.y - sg.x);
+    return;
+  }
+  int run       = lo > 0 ? s_scan[lo - 1] : 0;  // first tile of that thread's run
+  const int b2  = j0 + min(n, lo * per);
+  const int e2  = j0 + min(n, (lo + 1) * per);
+  for (int j = b2; j < e2; j++) {
+    int rows;
+    bool built;
+    const int t = tiles_of(j, rows, built);
+    if (tile < run + t) {
+      const int seg_lo = seg[j], seg_hi = seg[j + 1];
+      const int r0     = seg_lo + (tile - run) * tile_rows;
+      tiles[tile]      = make_int4(level_first + j, r0, min(seg_hi, r0 + tile_rows), seg_hi - seg_lo);
+      return;
+    }
+    run += t;
+  }
+}
+
 }  // namespace lbt

@@ -45,7 +45,6 @@
 namespace lbt {
 namespace {
 
-constexpr int kPlanThreads   = 256;
 constexpr int kSmallNodeRows = 64;  // below this a node goes straight to global atomics
 constexpr int kUnroll        = 4;   // rows per lane and tile, search kernels
 constexpr int kBinnedUnroll  = 8;   // rows per lane and tile, histogram kernel (halved for 16-byte loads)
@@ -152,117 +151,9 @@ __global__ void __launch_bounds__(kPlanThreads)
   tiles[tile]      = make_int4(level_first + j, r0, min(seg_hi, r0 + tile_rows), seg_hi - seg_lo);
 }
 
-// Both of the above in one launch, for batches of up to kPlanFusedNodes nodes: every workgroup
-// repeats the count and the scan of the nodes' tiles (a few loads per thread) instead of waiting
-// for a launch that does it once, then writes the descriptors of its own 256 tiles. Workgroup 0
-// also leaves the batch's totals and clears the counters of the launch that follows.
-// Bound by latency: the nodes' sums and segments, a scan, the descriptors. The scan is one barrier, the totals are summed by
-// waves, what they are added to is asked for at the start, and up to 256 nodes a descriptor needs nothing more from memory
-// (1,000,000 x 50, 8 to 256 nodes: 4.7, 5.7, 6.8, 10.5, 7, 9 us, now 4.8, 3.9, 3.6, 3.6, 3.3, 3.9).
+// Both of the above in one launch, for batches of up to kPlanFusedNodes nodes (plan_tiles_block)
 constexpr int kPlanFusedNodes = 4096;
-__global__ void __launch_bounds__(kPlanThreads)
-  plan_expand_tiles_kernel(int j0, int j1, int level_first, const int32_t* __restrict__ seg,
-                           const I64Pair* __restrict__ node_sums, HistView hist, int tile_rows, int4* tiles, LevelMeta* meta, LevelMeta* level_total, int32_t* pair_sync,
-                           int32_t* partial_count, int32_t* partial_list_count)
-{
-  __shared__ int s_scan[kPlanThreads];
-  __shared__ int2 s_seg[kPlanThreads];
-  __shared__ int s_wave[kPlanThreads / 64];
-  __shared__ int64_t s_sums[3][kPlanThreads / 64];
-  const bool first_wg = blockIdx.x == 0;
-  LevelMeta level_before{};
-  if (first_wg) {
-    if (threadIdx.x == 0) level_before = *level_total;
-    if (pair_sync != nullptr)
-      for (int i = threadIdx.x; i < kPairSyncSlots; i += kPlanThreads) pair_sync[i] = 0;
-    if (partial_count != nullptr) {
-      if (threadIdx.x == 0) *partial_count = 0;
-      for (int i = threadIdx.x; i < kPartialMaxLists; i += kPlanThreads) partial_list_count[i] = 0;
-    }
-  }
-  const int n     = j1 - j0;
-  const int per   = (n + kPlanThreads - 1) / kPlanThreads;
-  const int begin = j0 + min(n, static_cast<int>(threadIdx.x) * per);
-  const int end   = j0 + min(n, (static_cast<int>(threadIdx.x) + 1) * per);
-  auto tiles_of = [&](int j, int& rows, bool& built) {
-    rows  = seg[j + 1] - seg[j];
-    built = hist.builds(level_first + j, node_sums);
-    return built ? (rows + tile_rows - 1) / tile_rows : 0;
-  };
-  int mine = 0;
-  int64_t rb = 0, rc = 0, nb = 0;
-  for (int j = begin; j < end; j++) {
-    int rows;
-    bool built;
-    mine += tiles_of(j, rows, built);
-    rb += rows;
-    if (built && rows > 0) {
-      rc += rows;
-      nb += 1;
-    }
-  }
-  // (a thread's only node: its tiles are written from here, by whoever owns them)
-  s_seg[threadIdx.x] = begin < end ? make_int2(seg[begin], seg[begin + 1]) : make_int2(0, 0);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int before = block_exclusive_sum32<kPlanThreads>(mine, s_wave);
-  s_scan[threadIdx.x] = before + mine;
-  if (first_wg) {
-    rb = wave_inclusive_sum(rb);
-    rc = wave_inclusive_sum(rc);
-    nb = wave_inclusive_sum(nb);
-    if (lane == 63) {
-      s_sums[0][wave] = rb;
-      s_sums[1][wave] = rc;
-      s_sums[2][wave] = nb;
-    }
-  }
-  __syncthreads();
-  const int total = s_scan[kPlanThreads - 1];
-  if (first_wg && threadIdx.x == 0) {
-    int64_t sum[3] = {0, 0, 0};
-    for (int q = 0; q < 3; q++)
-      for (int w = 0; w < kPlanThreads / 64; w++) sum[q] += s_sums[q][w];
-    meta->n_tiles         = total;
-    meta->instances       = sum[0];
-    meta->built_instances = sum[1];
-    meta->built_nodes     = sum[2];
-    level_total->instances       = level_before.instances + sum[0];
-    level_total->built_instances = level_before.built_instances + sum[1];
-    level_total->built_nodes     = level_before.built_nodes + sum[2];
-  }
-  const int tile = blockIdx.x * kPlanThreads + threadIdx.x;
-  if (tile >= total) return;
-  // the thread whose run of nodes holds the tile: the last one whose inclusive count exceeds it
-  int lo = 0, hi = kPlanThreads - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (s_scan[mid] > tile)
-      hi = mid;
-    else
-      lo = mid + 1;
-  }
-  if (per == 1) {
-    const int2 sg = s_seg[lo];
-    const int r0  = sg.x + (tile - (lo > 0 ? s_scan[lo - 1] : 0)) * tile_rows;
-    tiles[tile]   = make_int4(level_first + j0 + lo, r0, min(sg.y, r0 + tile_rows), sg.y - sg.x);
-    return;
-  }
-  int run       = lo > 0 ? s_scan[lo - 1] : 0;  // first tile of that thread's run
-  const int b2  = j0 + min(n, lo * per);
-  const int e2  = j0 + min(n, (lo + 1) * per);
-  for (int j = b2; j < e2; j++) {
-    int rows;
-    bool built;
-    const int t = tiles_of(j, rows, built);
-    if (tile < run + t) {
-      const int seg_lo = seg[j], seg_hi = seg[j + 1];
-      const int r0     = seg_lo + (tile - run) * tile_rows;
-      tiles[tile]      = make_int4(level_first + j, r0, min(seg_hi, r0 + tile_rows), seg_hi - seg_lo);
-      return;
-    }
-    run += t;
-  }
-}
+__global__ void __launch_bounds__(kPlanThreads) plan_expand_tiles_kernel(PlanArgs a) { plan_tiles_block(a, blockIdx.x); }
 
 // Lookup table of a feature: the value range is cut into C fine cells (many more than there
 // are proposals) and the table holds one entry per 32 cells (see table_start). For a value in cell c,
@@ -2032,6 +1923,18 @@ int fill_walk(TileWalk& w, const HistBatch& b, int n_cu, int n_groups, int rpp, 
   return LBT_OK;
 }
 
+PlanArgs plan_of(const HistSetup& hs, const HistBatch& b, const TileWalk& w)
+{
+  PlanArgs p{b.j0, b.j0 + b.n_nodes, b.level_first, b.seg, b.node_sums, b.hist, w.tile_rows, hs.tiles, hs.meta, b.level_total, nullptr,
+             hs.binned != nullptr ? hs.partial_count : nullptr, hs.partial_list_count, 0};
+  const int64_t max_tiles = (b.n_rows + w.tile_rows - 1) / w.tile_rows + b.n_nodes;
+  p.blocks                = static_cast<int>((max_tiles + kPlanThreads - 1) / kPlanThreads);
+  return p;
+}
+
+// rows per lane and tile on cached bins below the root
+int level_unroll(const HistSetup& hs) { return hs.bvec == 16 ? kBinnedUnroll / 2 : kBinnedUnroll; }
+
 template <typename T>
 int hist_launch_t(hipStream_t stream, const HistSetup& hs, const HistBatch& b, int depth)
 {
@@ -2087,25 +1990,20 @@ int hist_launch_t(hipStream_t stream, const HistSetup& hs, const HistBatch& b, i
   TileWalk w;
   unsigned grid = 0;
   LBT_TRY(fill_walk(w, b, n_cu, hs.n_groups, use_cache ? hs.brpp : hs.rpp,
-                    use_cache ? (root ? 4 : (hs.bvec == 16 ? kBinnedUnroll / 2 : kBinnedUnroll)) : kUnroll,
+                    use_cache ? (root ? 4 : level_unroll(hs)) : kUnroll,
                     use_cache ? hs.blds_bytes : hs.lds_bytes, &grid));
-  {
+  if (!b.planned) {
     ProfScope ps(LBT_PROF_OTHER, stream);
-    const int64_t max_tiles = (b.n_rows + w.tile_rows - 1) / w.tile_rows + b.n_nodes;
-    const unsigned egrid    = static_cast<unsigned>((max_tiles + kPlanThreads - 1) / kPlanThreads);
-    int32_t* const sync     = root && w.n_chunks <= kPairSyncSlots ? hs.pair_sync : nullptr;
-    int32_t* const pcount   = use_cache ? hs.partial_count : nullptr;
+    PlanArgs p = plan_of(hs, b, w);
+    if (root && w.n_chunks <= kPairSyncSlots) p.pair_sync = hs.pair_sync;
     if (b.n_nodes <= kPlanFusedNodes) {
-      plan_expand_tiles_kernel<<<egrid, kPlanThreads, 0, stream>>>(
-        b.j0, b.j0 + b.n_nodes, b.level_first, b.seg, b.node_sums, b.hist, w.tile_rows,
-        hs.tiles, hs.meta, b.level_total, sync, pcount, hs.partial_list_count);
+      plan_expand_tiles_kernel<<<p.blocks, kPlanThreads, 0, stream>>>(p);
     } else {
-      plan_tiles_kernel<<<1, kPlanThreads, 0, stream>>>(b.j0, b.j0 + b.n_nodes, b.level_first, b.seg, b.node_sums,
-                                                        b.hist, w.tile_rows, hs.tile_start,
-                                                        hs.meta, b.level_total);
-      expand_tiles_kernel<<<egrid, kPlanThreads, 0, stream>>>(b.j0, b.n_nodes, b.level_first, b.seg, hs.tile_start,
-                                                              hs.meta, w.tile_rows, hs.tiles, sync, pcount,
-                                                              hs.partial_list_count);
+      plan_tiles_kernel<<<1, kPlanThreads, 0, stream>>>(b.j0, b.j0 + b.n_nodes, b.level_first, b.seg, b.node_sums, b.hist, w.tile_rows,
+                                                        hs.tile_start, hs.meta, b.level_total);
+      expand_tiles_kernel<<<p.blocks, kPlanThreads, 0, stream>>>(b.j0, b.n_nodes, b.level_first, b.seg, hs.tile_start, hs.meta,
+                                                                 w.tile_rows, hs.tiles, p.pair_sync, p.partial_count,
+                                                                 hs.partial_list_count);
     }
   }
   if (use_cache) {
@@ -2636,6 +2534,17 @@ int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, i
   else
     build_cells_kernel<float><<<F, 256, 0, stream>>>(static_cast<const float*>(proposals), row_pointers, F, cells,
                                                     hs.tables, static_cast<float*>(hs.map_x), hs.map_t, hs.straight);
+  return LBT_OK;
+}
+
+int hist_plan(const HistSetup& hs, const HistBatch& b, PlanArgs* plan)
+{
+  *plan = PlanArgs{};
+  if (hs.binned == nullptr || b.identity || b.fill_cache || b.n_nodes > kPlanFusedNodes) return LBT_OK;
+  TileWalk w;
+  unsigned grid = 0;
+  LBT_TRY(fill_walk(w, b, 256, hs.n_groups, hs.brpp, level_unroll(hs), hs.blds_bytes, &grid));
+  *plan = plan_of(hs, b, w);
   return LBT_OK;
 }
 

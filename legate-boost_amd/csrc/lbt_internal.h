@@ -514,7 +514,27 @@ struct HistBatch {
   int64_t n_rows;
   bool fill_cache;  // run the binning pass first (the bin cache does not hold this X and these proposals yet)
   bool identity;    // rows[i] == i for every i (the root of a tree that starts from the original order)
+  bool planned = false;  // the tiles have been planned (hist_plan)
 };
+
+// Which nodes of a batch are built, and their tiles (plan_tiles_block)
+struct PlanArgs {
+  int j0, j1, level_first;
+  const int32_t* seg;
+  const I64Pair* node_sums;
+  HistView hist;
+  int tile_rows;
+  int4* tiles;
+  LevelMeta* meta;
+  LevelMeta* level_total;
+  int32_t* pair_sync;
+  int32_t* partial_count;
+  int32_t* partial_list_count;
+  int blocks;  // workgroups of kPlanThreads
+};
+constexpr int kPlanThreads = 256;
+// What plans a batch below the root in a launch of the caller's; blocks: 0 where hist_launch has to do it.
+int hist_plan(const HistSetup& hs, const HistBatch& b, PlanArgs* plan);
 
 // Chooses groups / table size from the host copy of the row pointers and builds
 // the tables on the device.

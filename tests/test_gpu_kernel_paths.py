@@ -941,3 +941,38 @@ def test_scanned_levels_in_32_bits(n, f, k, s, kind):
     from lbtree import ops
     got = ops.build_tree(*(torch.from_numpy(v).cuda() for v in (X, g, h)), max_depth=6, split_samples=s, seed=5, row_leaf=True, **kw)
     _assert_tree(got, cr)
+
+
+@pytest.mark.parametrize("n,f,k,s,depth,kind", [
+    (9001, 60, 1, 512, 12, "plain"),        # more nodes than a slab decides, at last
+    (9001, 513, 2, 64, 9, "plain"),         # more candidates than a slab reads: a launch of its own
+    (8200, 100, 3, 256, 10, "empty"),       # most nodes without rows
+    (20479, 90, 1, 256, 10, "retired"),     # rows that stop early lie in front
+    (20480, 80, 1, 300, 10, "zero"),
+    (20481, 80, 2, 300, 10, "negative"),    # splits of nodes without rows: a launch of its own
+])
+def test_levels_of_the_general_builder_that_begin_in_one_launch(n, f, k, s, depth, kind):
+    """Splits found where rows are classified, tiles planned and histograms cleared where they are scattered: equal to the observed build,
+    whose histograms and levels the oracle's tests cover, in everything that both return."""
+    import gpu_util as gu
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + f)
+    X = rs.randn(n, f).astype(np.float32)
+    g, h = rs.randn(n, k), 0.1 + rs.random_sample((n, k))
+    if kind == "empty":
+        X = np.round(X)
+        g = np.repeat((X[:, :1] > 1) * 5.0, k, axis=1)
+    elif kind == "retired":
+        g = np.where(X[:, :1] > 0, np.sign(X[:, :1]), g)
+    elif kind == "zero":
+        h[rs.rand(n, k) < 0.3] = 0.0
+    elif kind == "negative":
+        h[rs.rand(n, k) < 0.3] *= -0.5
+    Xd, gd, hd = (torch.from_numpy(a).cuda() for a in (X, g, h))
+    kw = dict(max_depth=depth, split_samples=s, seed=2, row_leaf=True, hist_cache_bytes=10 ** 9)
+    want = ops.build_tree(Xd, gd, hd, taps=True, **kw)
+    got = ops.build_tree(Xd, gd, hd, **kw)
+    for name in ("leaf_value", "feature", "split_value", "gain", "hessian", "row_leaf"):
+        assert torch.equal(getattr(got, name), getattr(want, name)), name
+    gu.check_row_leaf(got, X)
