@@ -420,6 +420,13 @@ int lbt_weighted_gradient(void* stream, int32_t objective, const double* pred, c
                           int32_t n_outputs, double* g, double* h);
 
 /*
+ * The feature sample of a tree (legateboost/models/tree.py:139-157) on the device: feature_set[i] = host_mask[i] != 0.
+ *   host_mask    HOST bytes [n_features], read before the call returns
+ *   feature_set  device uint8 [n_features], as lbt_build_tree takes it; valid in stream order
+ */
+int lbt_feature_mask(void* stream, const uint8_t* host_mask, int32_t n_features, uint8_t* feature_set);
+
+/*
  * LBBase.update (legateboost/legateboost.py:306-386) over n_trees trees in one call: for every tree in order
  *   (g, h) = lbt_weighted_gradient(objective, pred, y, sample_weight, learning_rate)
  *   leaf_out[t], hessian_out[t] = lbt_update_tree(X, g, h, feature[t], split[t], l1[t], l2[t])

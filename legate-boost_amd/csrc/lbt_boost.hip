@@ -11,6 +11,7 @@
 
 namespace lbt {
 
+constexpr int kMaskFeatures = 8192;  // bits of a launch's arguments
 constexpr int kBoostThreads = 256;
 // One element per thread: squared error (any number of outputs) and log loss with one output.
 template <bool kLogistic>
@@ -580,6 +581,17 @@ __global__ void __launch_bounds__(kBoostThreads)
   h[i] *= 0.0;
 }
 
+// Bits by value: a copy from the host would have the host wait for all that is queued (memory that is not pinned), or the stream for another
+// engine.
+struct MaskBits {
+  uint32_t words[kMaskFeatures / 32];
+};
+__global__ void __launch_bounds__(kBoostThreads) feature_mask_kernel(MaskBits bits, int n, uint8_t* mask)
+{
+  const int i = blockIdx.x * kBoostThreads + threadIdx.x;
+  if (i < n) mask[i] = static_cast<uint8_t>(bits.words[i >> 5] >> (i & 31) & 1u);
+}
+
 inline unsigned grid_for(int64_t n) { return static_cast<unsigned>((n + kBoostThreads - 1) / kBoostThreads); }
 
 }  // namespace lbt
@@ -744,6 +756,24 @@ int lbt_keep_rows(void* stream, const double* draw, double limit, int64_t n_rows
   const int64_t n = n_rows * n_outputs;
   lbt::ProfScope ps(LBT_PROF_OTHER, s, static_cast<double>(n) * 8.0);
   lbt::keep_rows_kernel<<<lbt::grid_for(n), lbt::kBoostThreads, 0, s>>>(draw, limit, n, n_outputs, g, h);
+  LBT_HIP(hipGetLastError());
+  return LBT_OK;
+}
+
+int lbt_feature_mask(void* stream, const uint8_t* host_mask, int32_t n_features, uint8_t* feature_set)
+{
+  LBT_REQUIRE(n_features >= 0, "bad shape");
+  if (n_features == 0) return LBT_OK;
+  LBT_REQUIRE(host_mask && feature_set, "null pointer");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  lbt::ProfScope ps(LBT_PROF_OTHER, s, static_cast<double>(n_features));
+  for (int32_t first = 0; first < n_features; first += lbt::kMaskFeatures) {
+    const int n = std::min(lbt::kMaskFeatures, n_features - first);
+    lbt::MaskBits bits{};
+    for (int i = 0; i < n; i++)
+      if (host_mask[first + i] != 0) bits.words[i >> 5] |= 1u << (i & 31);
+    lbt::feature_mask_kernel<<<lbt::grid_for(n), lbt::kBoostThreads, 0, s>>>(bits, n, feature_set + first);
+  }
   LBT_HIP(hipGetLastError());
   return LBT_OK;
 }

@@ -11,12 +11,15 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/Device.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
 #include <cstring>
 #include <exception>
 #include <vector>
+
+#include "../../include/lbtree.h"
 
 namespace {
 
@@ -187,10 +190,203 @@ PyObject* predict_packed(PyObject*, PyObject* const* args, Py_ssize_t n_args)
   }
 }
 
+// Whether torch is being listened to: the calls below then go through Python
+bool listened_to() { return at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set(); }
+
+// A dense, contiguous device tensor of `type` and `dims` dimensions; null: something else
+const at::Tensor* dense(PyObject* o, at::ScalarType type, int64_t dims)
+{
+  if (!THPVariable_CheckExact(o)) return nullptr;
+  const at::Tensor& t = THPVariable_Unpack(o);
+  if (!t.defined() || t.layout() != at::kStrided || !t.is_cuda() || t.scalar_type() != type || t.dim() != dims || !t.is_contiguous()) return nullptr;
+  return &t;
+}
+
+bool integers(PyObject* const* args, int n, int64_t* out)
+{
+  for (int i = 0; i < n; i++) {
+    out[i] = PyLong_AsLongLong(args[i]);
+    if (out[i] == -1 && PyErr_Occurred()) return false;
+  }
+  return true;
+}
+bool numbers(PyObject* const* args, int n, double* out)
+{
+  for (int i = 0; i < n; i++) {
+    out[i] = PyFloat_AsDouble(args[i]);
+    if (out[i] == -1.0 && PyErr_Occurred()) return false;
+  }
+  return true;
+}
+
+// build_tree(X, g, h, mask, workspace, entry, size_entry, stream, row_offset, max_depth, split_samples, seed, cache, row_leaf, l1, l2, gain):
+// lbt_build_tree_async and lbt_build_tree_workspace_bytes, whose addresses are `entry` and `size_entry`, for a float or double matrix and gradients as they
+// have to be on the device; mask: a uint8 tensor there or None; workspace(bytes, device): the scratch tensor. Returns (leaf_value, feature,
+// split_value, gain, hessian, row_leaf or None), or the status where that is not 0, or None, with nothing done, for anything else: the
+// caller then goes through Python. A round of boosting on 1000 x 10 took its host 57 us, with this, the two calls below and no copy of a plain learner 36.
+using BuildTree      = decltype(&lbt_build_tree_async);
+using WorkspaceBytes = decltype(&lbt_build_tree_workspace_bytes);
+PyObject* build_tree(PyObject*, PyObject* const* args, Py_ssize_t n_args)
+{
+  if (n_args != 17) {
+    PyErr_SetString(PyExc_TypeError, "build_tree takes 17 arguments");
+    return nullptr;
+  }
+  int64_t v[9];
+  double r[3];
+  if (!integers(args + 5, 9, v) || !numbers(args + 14, 3, r)) {
+    if (!PyErr_ExceptionMatches(PyExc_Exception)) return nullptr;
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  const int64_t row_offset = v[3], max_depth = v[4], samples = v[5], seed = v[6], cache = v[7];
+  const bool row_leaf = v[8] != 0;
+  try {
+    if (listened_to()) Py_RETURN_NONE;
+    const at::Tensor* x = dense(args[0], at::kFloat, 2);
+    const bool wide     = x == nullptr;
+    if (wide) x = dense(args[0], at::kDouble, 2);
+    const at::Tensor *g = dense(args[1], at::kDouble, 2), *h = dense(args[2], at::kDouble, 2);
+    if (x == nullptr || g == nullptr || h == nullptr || g->sizes() != h->sizes() || g->size(0) != x->size(0) || g->device() != x->device() ||
+        h->device() != x->device() || max_depth < 0 || max_depth > 24 || samples < INT32_MIN || samples > INT32_MAX || seed < INT32_MIN ||
+        seed > INT32_MAX || x->size(1) > INT32_MAX || g->size(1) > INT32_MAX)
+      Py_RETURN_NONE;
+    const at::Tensor* mask = nullptr;
+    if (args[3] != Py_None) {
+      mask = dense(args[3], at::kByte, 1);
+      if (mask == nullptr || mask->size(0) != x->size(1) || mask->device() != x->device()) Py_RETURN_NONE;
+    }
+    const int64_t n = x->size(0);
+    const int32_t f = static_cast<int32_t>(x->size(1)), k = static_cast<int32_t>(g->size(1));
+    const int32_t type = wide ? LBT_F64 : LBT_F32, nodes = (1 << (max_depth + 1)) - 1;
+    lbt_build_params prm{};
+    prm.struct_bytes = sizeof(prm);
+    prm.max_depth = static_cast<int32_t>(max_depth), prm.max_nodes = nodes, prm.split_samples = static_cast<int32_t>(samples);
+    prm.seed = static_cast<int32_t>(seed), prm.dataset_rows = n;
+    prm.l1_regularization = r[0], prm.l2_regularization = r[1], prm.min_split_gain = r[2];
+    prm.hist_cache_bytes = cache;
+    const size_t bytes = reinterpret_cast<WorkspaceBytes>(v[1])(n, f, k, prm.max_depth, prm.split_samples, type, cache);
+    if (bytes == 0) Py_RETURN_NONE;  // an argument that is refused
+    PyObject* device  = THPDevice_New(x->device());
+    PyObject* scratch = device != nullptr ? PyObject_CallFunction(args[4], "KO", static_cast<unsigned long long>(bytes), device) : nullptr;
+    Py_XDECREF(device);
+    if (scratch == nullptr) {
+      if (!PyErr_ExceptionMatches(PyExc_Exception)) return nullptr;
+      PyErr_Clear();
+      Py_RETURN_NONE;
+    }
+    Held keep;
+    keep.objects.push_back(scratch);
+    const at::Tensor* ws = dense(scratch, at::kByte, 1);
+    if (ws == nullptr || ws->device() != x->device()) Py_RETURN_NONE;
+    const auto real = x->options().dtype(at::kDouble), whole = x->options().dtype(at::kInt);
+    at::Tensor leaf = at::empty({nodes, k}, real), feature = at::empty({nodes}, whole), split = at::empty({nodes}, real),
+               gain = at::empty({nodes}, real), hessian = at::empty({nodes, k}, real), rows;
+    lbt_build_taps taps{};
+    if (row_leaf) {
+      rows          = at::empty({n}, whole);
+      taps.row_leaf = rows.mutable_data_ptr<int32_t>();
+    }
+    const void* const from       = x->const_data_ptr();
+    const double* const grad     = g->const_data_ptr<double>();
+    const double* const hess     = h->const_data_ptr<double>();
+    const uint8_t* const allowed = mask != nullptr ? mask->const_data_ptr<uint8_t>() : nullptr;
+    double* const to_leaf = leaf.mutable_data_ptr<double>();
+    int32_t* const to_feature = feature.mutable_data_ptr<int32_t>();
+    double* const to_split = split.mutable_data_ptr<double>();
+    double* const to_gain = gain.mutable_data_ptr<double>();
+    double* const to_hessian = hessian.mutable_data_ptr<double>();
+    void* const room = ws->data_ptr();
+    const size_t has = static_cast<size_t>(ws->numel());
+    int status       = 0;
+    Py_BEGIN_ALLOW_THREADS
+    status = reinterpret_cast<BuildTree>(v[0])(reinterpret_cast<void*>(v[2]), from, type, row_offset, n, f, grad, hess, k, allowed, &prm, to_leaf,
+                                               to_feature, to_split, to_gain, to_hessian, room, has, row_leaf ? &taps : nullptr);
+    Py_END_ALLOW_THREADS
+    if (status != 0) return PyLong_FromLong(status);
+    PyObject* out = PyTuple_New(6);
+    if (out == nullptr) return nullptr;
+    at::Tensor* const all[5] = {&leaf, &feature, &split, &gain, &hessian};
+    for (int i = 0; i < 5; i++) PyTuple_SET_ITEM(out, i, THPVariable_Wrap(std::move(*all[i])));
+    if (!row_leaf) Py_INCREF(Py_None);
+    PyTuple_SET_ITEM(out, 5, row_leaf ? THPVariable_Wrap(std::move(rows)) : Py_None);
+    return out;
+  } catch (const std::exception&) {
+    if (PyErr_Occurred()) PyErr_Clear();
+    Py_RETURN_NONE;  // whatever it is, the caller meets it again in Python
+  }
+}
+
+// weighted_gradient(y, pred, weight, entry, stream, objective, learning_rate): lbt_weighted_gradient on device doubles; weight: [rows] or None.
+// Returns (g, h), a status that is not 0, or None as above.
+PyObject* weighted_gradient(PyObject*, PyObject* const* args, Py_ssize_t n_args)
+{
+  if (n_args != 7) {
+    PyErr_SetString(PyExc_TypeError, "weighted_gradient takes seven arguments");
+    return nullptr;
+  }
+  int64_t v[3];
+  double rate;
+  if (!integers(args + 3, 3, v) || !numbers(args + 6, 1, &rate)) return nullptr;
+  try {
+    if (listened_to()) Py_RETURN_NONE;
+    const at::Tensor *y = dense(args[0], at::kDouble, 2), *pred = dense(args[1], at::kDouble, 2);
+    if (y == nullptr || pred == nullptr || y->device() != pred->device() || pred->size(1) > INT32_MAX) Py_RETURN_NONE;
+    const int64_t n = pred->size(0), k = pred->size(1);
+    if (y->numel() != (v[2] == LBT_OBJ_LOG_LOSS && k > 1 ? n : n * k)) Py_RETURN_NONE;
+    const at::Tensor* w = nullptr;
+    if (args[2] != Py_None) {
+      w = dense(args[2], at::kDouble, 1);
+      if (w == nullptr || w->numel() != n || w->device() != pred->device()) Py_RETURN_NONE;
+    }
+    const auto real = pred->options().requires_grad(false);
+    at::Tensor g = at::empty({n, k}, real), h = at::empty({n, k}, real);
+    const int status = reinterpret_cast<decltype(&lbt_weighted_gradient)>(v[0])(
+      reinterpret_cast<void*>(v[1]), static_cast<int32_t>(v[2]), pred->const_data_ptr<double>(), y->const_data_ptr<double>(),
+      w != nullptr ? w->const_data_ptr<double>() : nullptr, rate, n, static_cast<int32_t>(k), g.mutable_data_ptr<double>(), h.mutable_data_ptr<double>());
+    if (status != 0) return PyLong_FromLong(status);
+    PyObject* out = PyTuple_New(2);
+    if (out == nullptr) return nullptr;
+    PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(g)));
+    PyTuple_SET_ITEM(out, 1, THPVariable_Wrap(std::move(h)));
+    return out;
+  } catch (const std::exception&) {
+    Py_RETURN_NONE;
+  }
+}
+
+// add_leaf_values(pred, leaf_value, row_leaf, entry, stream): lbt_add_leaf_values. Returns the status, or None as above.
+PyObject* add_leaf_values(PyObject*, PyObject* const* args, Py_ssize_t n_args)
+{
+  if (n_args != 5) {
+    PyErr_SetString(PyExc_TypeError, "add_leaf_values takes five arguments");
+    return nullptr;
+  }
+  int64_t v[2];
+  if (!integers(args + 3, 2, v)) return nullptr;
+  try {
+    if (listened_to()) Py_RETURN_NONE;
+    const at::Tensor *pred = dense(args[0], at::kDouble, 2), *leaf = dense(args[1], at::kDouble, 2), *rows = dense(args[2], at::kInt, 1);
+    if (pred == nullptr || leaf == nullptr || rows == nullptr || leaf->size(1) != pred->size(1) || rows->size(0) != pred->size(0) ||
+        leaf->device() != pred->device() || rows->device() != pred->device() || pred->size(1) > INT32_MAX || leaf->size(0) > INT32_MAX)
+      Py_RETURN_NONE;
+    return PyLong_FromLong(reinterpret_cast<decltype(&lbt_add_leaf_values)>(v[0])(
+      reinterpret_cast<void*>(v[1]), leaf->const_data_ptr<double>(), static_cast<int32_t>(leaf->size(0)), rows->const_data_ptr<int32_t>(),
+      pred->size(0), static_cast<int32_t>(pred->size(1)), static_cast<double*>(pred->data_ptr())));
+  } catch (const std::exception&) {
+    Py_RETURN_NONE;
+  }
+}
+
 PyMethodDef methods[] = {{"tree_arrays", tree_arrays, METH_VARARGS, "addresses and node counts of an ensemble's arrays"},
                          {"model_arrays", model_arrays, METH_VARARGS, "the same from the attributes of an ensemble's models"},
                          {"predict_packed", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(predict_packed)), METH_FASTCALL,
                           "prediction with a packed ensemble"},
+                         {"build_tree", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(build_tree)), METH_FASTCALL, "one tree"},
+                         {"weighted_gradient", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(weighted_gradient)), METH_FASTCALL,
+                          "gradients and hessians of a round"},
+                         {"add_leaf_values", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(add_leaf_values)), METH_FASTCALL,
+                          "prediction update of a round"},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -170,6 +170,8 @@ def _load():
     lib.lbt_label_priors.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int32, C.c_void_p]
     lib.lbt_keep_rows.restype = C.c_int
     lib.lbt_keep_rows.argtypes = [C.c_void_p, C.c_void_p, C.c_double, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p]
+    lib.lbt_feature_mask.restype = C.c_int
+    lib.lbt_feature_mask.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p]
     lib.lbt_class_probabilities.restype = C.c_int
     lib.lbt_class_probabilities.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_int32, C.c_void_p]
     lib.lbt_weighted_gradient_sums.restype = C.c_int
@@ -246,7 +248,7 @@ EXPORTS = [
     "lbt_update_tree_workspace_bytes", "lbt_update_tree", "lbt_update_tree_rows", "lbt_update_trees_workspace_bytes",
     "lbt_update_trees",
     "lbt_weighted_gradient", "lbt_weighted_gradient_sums", "lbt_class_probabilities",
-    "lbt_weighted_mean_workspace_bytes", "lbt_weighted_mean", "lbt_label_counts", "lbt_label_priors", "lbt_keep_rows",
+    "lbt_weighted_mean_workspace_bytes", "lbt_weighted_mean", "lbt_label_counts", "lbt_label_priors", "lbt_keep_rows", "lbt_feature_mask",
     "lbt_abs_sum_chunks", "lbt_add_leaf_values",
     "lbt_gather_rows", "lbt_select_split_samples_workspace_bytes", "lbt_select_split_samples",
     "lbt_quantise_gradients_workspace_bytes", "lbt_quantise_gradients", "lbt_quantise_gradients_static",

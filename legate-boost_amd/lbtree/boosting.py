@@ -37,6 +37,20 @@ def _float64_on_device(a):
             and not a.requires_grad)
 
 
+def _copy_of(model):
+    """deepcopy(model). A tree whose attributes are numbers and names, as one that is not fitted has, is copied by them."""
+    if type(model) is Tree and not hasattr(Tree, "__deepcopy__"):
+        attributes = vars(model)
+        if all(type(v) in _NUMBERS for v in attributes.values()):
+            new = Tree.__new__(Tree)
+            vars(new).update(attributes)
+            return new
+    return deepcopy(model)
+
+
+_NUMBERS = (int, float, str, bool, type(None))
+
+
 class SquaredErrorObjective:
     fused = "squared_error"  # ops.weighted_gradient computes transform + gradient + weighting in one pass
 
@@ -206,7 +220,7 @@ class LBBase:
                 and (fused != "log_loss" or train_pred.shape[1] <= 128)
                 and _as_defined(self, LBBase, "_get_weighted_gradient"))
         for i in range(self.n_estimators):
-            model = deepcopy(self.base_models[i % len(self.base_models)]).set_random_state(self.random_state_)
+            model = _copy_of(self.base_models[i % len(self.base_models)]).set_random_state(self.random_state_)
             if sums and isinstance(model, Tree) and _as_defined(model, Tree, "fit", "fit_update_predictions", "_fit"):
                 g, h, chunks = ops.weighted_gradient(fused, y, train_pred, w, self.learning_rate, sums=True)
                 model._fit(X, g, h, train_pred, chunks)

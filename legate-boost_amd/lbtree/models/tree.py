@@ -86,7 +86,7 @@ class Tree(BaseModel):
             n_sampled_features = max(1, int(n_features * self.feature_fraction))
             selection = self.random_state.choice(n_features, n_sampled_features, False)
             mask[selection] = True
-            feature_set = torch.from_numpy(mask)
+            feature_set = ops.feature_mask(mask, X.device)
         r = ops.build_tree(
             X, g, h, max_depth=self.max_depth, split_samples=self.split_samples, seed=seed,
             l1_regularization=self.l1_regularization, l2_regularization=self.l2_regularization,

@@ -81,6 +81,24 @@ class BuildResult:
     pass
 
 
+def _address(fn):
+    return C.cast(fn, C.c_void_p).value
+
+
+# the calls of a boosting round in native code, where it is built and torch hands out a stream's address
+_NATIVE = _lib._host if _lib._host is not None and _raw_stream is not None else None
+_BUILD, _BUILD_BYTES = _address(_lib.lib.lbt_build_tree_async), _address(_lib.lib.lbt_build_tree_workspace_bytes)
+_GRADIENT, _ADD_LEAVES = _address(_lib.lib.lbt_weighted_gradient), _address(_lib.lib.lbt_add_leaf_values)
+
+
+def feature_mask(mask, device):
+    """The bools of a numpy array as the uint8 CUDA tensor that build_tree takes, without a wait for what is queued."""
+    host = np.ascontiguousarray(mask, dtype=np.bool_)
+    out = torch.empty(host.shape[0], dtype=torch.uint8, device=device)
+    _lib.check(_lib.lib.lbt_feature_mask(_stream(), host.ctypes.data, host.shape[0], out.data_ptr()))
+    return out
+
+
 def build_tree(X, g, h, *, max_depth, split_samples, seed, l1_regularization=0.0, l2_regularization=1.0,
                min_split_gain=0.0, feature_set=None, dataset_rows=None, row_offset=0, hist_cache_bytes=0,
                taps=False, taps_levels=False, row_leaf=False, wait=True, abs_sum_chunks=None):
@@ -88,6 +106,18 @@ def build_tree(X, g, h, *, max_depth, split_samples, seed, l1_regularization=0.0
     outputs as CUDA tensors; with taps=True also the observation points. wait=False returns
     without synchronising the stream (lbt_build_tree_async; not together with taps=True).
     abs_sum_chunks: the chunk sums weighted_gradient(..., sums=True) returned for these g and h."""
+    if _NATIVE is not None and not (wait or taps or taps_levels) and dataset_rows is None and abs_sum_chunks is None and torch.cuda.is_initialized():
+        got = _NATIVE.build_tree(X, g, h, feature_set, _get_workspace, _BUILD, _BUILD_BYTES, _raw_stream(torch.cuda.current_device()), row_offset,
+                                 max_depth, split_samples, seed, hist_cache_bytes, 1 if row_leaf else 0, l1_regularization,
+                                 l2_regularization, min_split_gain)
+        if got is not None:
+            if not isinstance(got, tuple):
+                _lib.check(got)
+            r = BuildResult()
+            r.leaf_value, r.feature, r.split_value, r.gain, r.hessian, rows = got
+            if row_leaf:
+                r.row_leaf = rows
+            return r
     X = _check_x(X)
     g = as_device(g, torch.float64)
     h = as_device(h, torch.float64)
@@ -334,6 +364,13 @@ def weighted_gradient(objective, y, pred, sample_weight=None, learning_rate=1.0,
     for log loss with K > 1. Returns (g, h); `out=(g, h)` reuses two buffers of pred's shape.
     sums=True (or a [2][chunks] float64 tensor to fill): also the chunk sums of |g| and |h| that
     build_tree(abs_sum_chunks=...) takes in place of its own pass over g and h; returns (g, h, sums)."""
+    if _NATIVE is not None and out is None and sums is False and objective in _OBJECTIVES and torch.cuda.is_initialized():
+        got = _NATIVE.weighted_gradient(y, pred, sample_weight, _GRADIENT, _raw_stream(torch.cuda.current_device()), _OBJECTIVES[objective],
+                                        learning_rate)
+        if got is not None:
+            if not isinstance(got, tuple):
+                _lib.check(got)
+            return got
     pred = as_device(pred, torch.float64)
     y = as_device(y, torch.float64)
     if pred.dim() != 2:
@@ -470,6 +507,11 @@ def update_trees(X, y, sample_weight, objective, learning_rate, pred, trees):
 def add_leaf_values(pred, leaf_value, row_leaf):
     """pred += leaf_value[row_leaf], in place: the caller's `train_pred += tree.predict(X)`
     (legateboost/legateboost.py:268) from the rows' leaves recorded by build_tree(row_leaf=True)."""
+    if _NATIVE is not None and torch.cuda.is_initialized():
+        rc = _NATIVE.add_leaf_values(pred, leaf_value, row_leaf, _ADD_LEAVES, _raw_stream(torch.cuda.current_device()))
+        if rc is not None:
+            _lib.check(rc)
+            return pred
     if not (pred.is_cuda and pred.dtype == torch.float64 and pred.is_contiguous() and pred.dim() == 2):
         raise _lib.LbtError("pred must be a contiguous CUDA float64 [n_rows, n_outputs] tensor")
     leaf_value = as_device(leaf_value, torch.float64)

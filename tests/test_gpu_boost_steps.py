@@ -326,3 +326,87 @@ def test_which_fits_ask_for_the_gradient_passes_sums(monkeypatch, task, n, k, as
     else:
         lb.LBRegressor(n_estimators=1, base_models=(tree,), random_state=1).fit(X, torch.rand(n, k, dtype=torch.float64).cuda())
     assert seen == [asked]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,f,k,dtype,kind", [
+    (1000, 7, 1, torch.float32, "plain"), (1000, 7, 3, torch.float64, "plain"), (999, 5, 1, torch.float32, "strided"),
+    (999, 5, 2, torch.float64, "single_gradients"), (500, 4, 1, torch.float32, "on_the_host"), (9000, 9, 1, torch.float32, "mask"),
+    (300, 3, 1, torch.float32, "vector_targets"), (1, 1, 1, torch.float64, "plain"),
+])
+def test_a_round_in_native_code_is_the_one_in_python(n, f, k, dtype, kind, monkeypatch):
+    """Gradient, tree and prediction update through lbtree._host, and for what that does not take through Python: the same bits."""
+    from lbtree import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    X = torch.randn((n, f), generator=gen, device="cuda", dtype=dtype)
+    y = torch.randn((n, k), generator=gen, device="cuda", dtype=torch.float64)
+    pred = torch.randn((n, k), generator=gen, device="cuda", dtype=torch.float64)
+    w = torch.rand(n, generator=gen, device="cuda", dtype=torch.float64)
+    mask = None
+    if kind == "strided":
+        X, y = X.t().contiguous().t(), y.t().contiguous().t()
+    elif kind == "single_gradients":
+        y = y.to(torch.float32)
+    elif kind == "on_the_host":
+        X = X.cpu().numpy()
+    elif kind == "vector_targets":
+        y = y.reshape(-1)
+    elif kind == "mask":
+        mask = ops.feature_mask(np.arange(f) % 3 != 1, "cuda")
+        assert mask.tolist() == [int(i % 3 != 1) for i in range(f)]
+    out = []
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(ops, "_NATIVE", None)
+        p = pred.clone()
+        g, h = ops.weighted_gradient("squared_error", y, p, w, 0.1)
+        g2 = g.to(torch.float32) if kind == "single_gradients" else g
+        r = ops.build_tree(X, g2, h, max_depth=5, split_samples=64, seed=4, feature_set=mask, row_leaf=True, wait=False,
+                           l2_regularization=np.float32(1.0))
+        assert ops.add_leaf_values(p, r.leaf_value, r.row_leaf) is p
+        out.append((g, h, r.leaf_value, r.feature, r.split_value, r.gain, r.hessian, r.row_leaf, p))
+    for a, b in zip(*out):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_a_refused_round_is_refused_as_before(monkeypatch):
+    from lbtree import _lib, ops
+
+    X = torch.zeros((10, 2), device="cuda")
+    g = torch.ones((10, 1), device="cuda", dtype=torch.float64)
+    for bad in (dict(max_depth=-1), dict(split_samples=0), dict(split_samples=4096), dict(max_depth=3.5)):
+        kw = dict(max_depth=3, split_samples=16, seed=1, wait=False)
+        kw.update(bad)
+        said = []
+        for native in (True, False):
+            with monkeypatch.context() as m:
+                if not native:
+                    m.setattr(ops, "_NATIVE", None)
+                with pytest.raises(Exception) as e:
+                    ops.build_tree(X, g, g, **kw)
+                said.append((type(e.value), str(e.value)))
+        assert said[0] == said[1], bad
+    with pytest.raises(_lib.LbtError):
+        ops.build_tree(X, g[:5], g, max_depth=2, split_samples=16, seed=1, wait=False)
+    with pytest.raises(_lib.LbtError):
+        ops.add_leaf_values(g, g[:3].reshape(1, 3), torch.zeros(10, dtype=torch.int32, device="cuda"))
+
+
+def test_a_plain_tree_is_copied_by_its_numbers():
+    from lbtree import boosting
+    from lbtree.models import Tree
+
+    class Own(Tree):
+        pass
+
+    plain = Tree(max_depth=3)
+    copied = boosting._copy_of(plain)
+    assert type(copied) is Tree and vars(copied) == vars(plain) and copied is not plain
+    listed = Tree(max_depth=3)
+    listed.note = [1]
+    copied = boosting._copy_of(listed)
+    assert copied.note == [1] and copied.note is not listed.note
+    assert type(boosting._copy_of(Own(max_depth=2))) is Own
+
