@@ -1842,7 +1842,10 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
   L.left          = K == 1 && max_depth >= 2 && S <= kDirectMaxBins ? ar.take<I64Pair>(level_nodes * F) : nullptr;
   // one of the builders at a time uses the room for histograms
   const size_t mid_bytes = mid_tree_fits(N, F, K, max_depth, S) ? mid_hist_bytes(N, F, K, max_depth, S) : 0;
-  bool mid               = mid_bytes > 0 && static_cast<double>(mid_bytes) <= hist_budget(cache_bytes, roomy);
+  // (counted with 16 bytes a bin: with a budget between that and the 8 it takes, its other arrays would need more than a tree one level
+  // deeper, which is not its size, does in all)
+  const double mid_counted = static_cast<double>(mid_bytes) + 2.0 * level_nodes * K * F * S * 8;
+  bool mid = mid_bytes > 0 && mid_counted <= hist_budget(cache_bytes, roomy);
   const bool small       = small_tree_fits(N, F, K, max_depth, S) && !(mid && mid_beats_small(N, F, K, max_depth, S));
   mid                    = mid && !small;
   L.hist_bytes        = hist_bytes_bound(F, K, S, max_depth, cache_bytes, roomy);
@@ -1898,13 +1901,14 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
     for (auto& nodes : st.row_node) nodes = ar.take<uint16_t>(st.pitch);
     st.q_stats    = ar.take<unsigned long long>(4);
     if (hist != nullptr) {
-      st.hist[0]  = L.hist;
-      st.hist[1]  = L.hist + level_hist;
-      st.images   = reinterpret_cast<unsigned long long*>(L.hist + 2 * level_hist);
+      st.hist[0]  = reinterpret_cast<uint2*>(L.hist);
+      st.hist[1]  = st.hist[0] + level_hist;
+      st.images   = reinterpret_cast<unsigned long long*>(st.hist[0] + 2 * level_hist);
     }
     st.node_sums  = L.node_sums;
     st.scales     = L.scales;
     st.cand       = ar.take<SmallCand>(level_nodes * F);
+    st.left       = ar.take<uint2>(level_nodes * F);
     st.splits     = ar.take<int2>(level_nodes);
     st.live       = ar.take<int32_t>(max_depth + 1);
   }

@@ -652,7 +652,8 @@ struct MidTreeState {
   uint16_t* row_node[2];  // [pitch] node of the level, 0xffff: none; of the root in the first one
   unsigned long long* q_stats;  // [4] sum of the positive rounded grads, of the negative ones, flags
   unsigned long long* images;   // packed histograms of the row ranges
-  I64Pair* hist[2];       // scanned histograms, [node][K][F][S]; level d in hist[d & 1]
+  uint2* hist[2];         // scanned histograms, lower halves of grad and hess, [node][K][F][S]; level d in hist[d & 1]
+  uint2* left;            // [nodes of the last level][F] the same of what lies left of a feature's best split (one output)
   I64Pair* node_sums;     // [max_nodes][K]
   double* scales;         // [4]
   SmallCand* cand;        // [nodes of a level][F]

@@ -11,7 +11,8 @@
 //   mid_histogram_kernel  a workgroup = (range of rows) x (some features) x (some built nodes) x (output)
 //                         with a packed histogram of all those nodes in the LDS, written out whole
 //   mid_scan_kernel       a workgroup = (pair of siblings, feature): adds the row ranges' images, running
-//                         sums, the sibling as parent minus node, gains (build_tree.cu:597-740)
+//                         sums, the sibling as parent minus node, gains (build_tree.cu:597-740); in
+//                         wide levels a wave does (mid_scan_waves_kernel)
 //   mid_apply_kernel      best features, the nodes' outputs and children (build_tree.cu:740-782), new node
 //                         of every row; where few workgroups share a range of rows, the next level's histogram
 //                         workgroups do that for themselves instead (a launch less)
@@ -42,6 +43,7 @@ constexpr int kMaxFb    = 128 / sizeof(T);  // features of a binning workgroup: 
 constexpr int kRowsApply = 4 * kWide;
 constexpr size_t kHistLds = 128 * 1024;
 constexpr int64_t kNodesMost = 2500000;  // rows times workgroups that find the nodes of the same ones (nodes_with_histograms)
+constexpr int64_t kWavePairs = 1024;     // pairs of siblings times features scanned by a wave each (mid_scan_waves_kernel)
 constexpr int kCandsMost     = 4096;     // candidates a histogram workgroup goes through for that (64 KB)
 
 struct MidArgs {
@@ -507,11 +509,16 @@ __device__ __forceinline__ int2 decide_node(const MidArgs& a, const MidTreeState
     if (splits) {
       const int64_t fs = static_cast<int64_t>(a.F) * a.S;
       const int lc = left_child(node), rc = right_child(node);
-      const I64Pair* h = st.hist[p.depth & 1] + static_cast<int64_t>(j) * a.K * fs + static_cast<int64_t>(ft) * a.S + (rel & ~kLeftSmaller);
+      // (the last level of one output stores no histograms)
+      const uint2* h = p.last && a.K == 1 ? st.left + static_cast<int64_t>(j) * a.F + ft
+                                          : st.hist[p.depth & 1] + static_cast<int64_t>(j) * a.K * fs + static_cast<int64_t>(ft) * a.S + (rel & ~kLeftSmaller);
+      const uint32_t down = static_cast<uint32_t>(st.q_stats[1]);
       for (int k = sub; k < a.K; k += lanes) {
         const int64_t at = static_cast<int64_t>(node) * a.K + k, l = static_cast<int64_t>(lc) * a.K + k,
                       r = static_cast<int64_t>(rc) * a.K + k;
-        const I64Pair ns = st.node_sums[at], ls = h[k * fs];
+        const I64Pair ns = st.node_sums[at];
+        const uint2 low  = h[k * fs];
+        const I64Pair ls{static_cast<int64_t>(low.x + down) - static_cast<int64_t>(down), static_cast<int64_t>(low.y)};
         const I64Pair rs{ns.grad - ls.grad, ns.hess - ls.hess};
         const double lg = static_cast<double>(ls.grad) * inv_g, lh = static_cast<double>(ls.hess) * inv_h;
         const double rg = static_cast<double>(rs.grad) * inv_g, rh = static_cast<double>(rs.hess) * inv_h;
@@ -693,7 +700,15 @@ __global__ void __launch_bounds__(kWide)
 // had been 7.5 to 8.1.
 // kLess: kLeftSmaller beside the candidates' bins, for histogram workgroups that decide (42.2 us a launch on 5000 x 200 with 8 outputs, depth 5, to
 // 41.1 without).
-template <bool kLess>
+// Histograms in memory are the lower halves of their sums, 8 bytes a bin, and the last level of one output (kLast) stores none, only what lies left of a
+// feature's best split. (Where the rule on zeros left a bin as it was in the parent, which has no hessian then, what a sibling keeps there can lie
+// outside of -down and up; no node below takes a split at it, and what is subtracted from it is exact in 32 bits.) With 16 bytes, and all levels
+// stored, the two deepest levels of 50,000 x 200, depth 8, took 33 and 61 us: now 18 and 28, by waves (mid_scan_waves_kernel).
+// kAhead: with several outputs a workgroup's sums of the images are asked for one output ahead, all ranges of rows that
+// kAhead holds at once. A chain of loads, sums and barriers per output took 2.5 us an output (400,000 x 12 with 8 outputs and 32
+// ranges: 20 us a narrow level, now 16; 11,094 x 120 with 5 outputs, 512 samples, depth 8: a tree in 754 us, now 635). As many
+// loads as there are ranges, up to 16: 16 always took 5000 x 200 with 8 outputs, which has 4, from 209 to 221 us, 4 take 198.
+template <bool kLess, bool kLast, int kAhead>
 __global__ void __launch_bounds__(kScan)
   mid_scan_kernel(MidArgs a, MidTreeState st, LevelPlan p)
 {
@@ -702,6 +717,7 @@ __global__ void __launch_bounds__(kScan)
   __shared__ double s_best[2][kScan / 64];
   __shared__ unsigned s_bkey[2][kScan / 64];
   __shared__ int s_less[2][kScan / 64];
+  __shared__ uint2 s_cell[kLast ? 2 : 1][kScan / 64];
   const int f = blockIdx.x % a.F, pair = blockIdx.x / a.F;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   if (level_is_empty(st, p.depth)) return;
@@ -726,11 +742,12 @@ __global__ void __launch_bounds__(kScan)
   const double down_of = static_cast<double>(down);
   const double inv_g = st.scales[2], inv_h = st.scales[3];
   const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
-  I64Pair* const hist         = st.hist[p.depth & 1];
-  const I64Pair* const parent = st.hist[(p.depth & 1) ^ 1] + static_cast<int64_t>(pair) * a.K * fs + static_cast<int64_t>(f) * a.S;
+  uint2* const hist         = st.hist[p.depth & 1];
+  const uint2* const parent = st.hist[(p.depth & 1) ^ 1] + static_cast<int64_t>(pair) * a.K * fs + static_cast<int64_t>(f) * a.S;
   double best_n = 0.0, best_s = 0.0;
   unsigned key_n = 0, key_s = 0;
   bool less_n = false, less_s = false;  // the best split's left child has the smaller hessian (of the first output)
+  uint2 best_cell_n = make_uint2(0, 0), best_cell_s = make_uint2(0, 0);  // kLast: what lies left of it
   auto run = [&](auto plains) {
     auto quotient = [&](double grad, double hess) {
       if constexpr (decltype(plains)::value)
@@ -738,21 +755,58 @@ __global__ void __launch_bounds__(kScan)
       else
         return leaf_gain_select(grad, hess, a.l1, reg);
     };
+    // kAhead: the images and the parent's bin of the next output are on their way while an output's are summed
+    unsigned long long ahead[kAhead > 0 ? kAhead : 1];
+    uint2 parent_ahead = make_uint2(0, 0);
+    const int64_t step = static_cast<int64_t>(p.built) * a.K * fs;
+    auto fetch = [&](int k, int bin) {
+      const int64_t at = k * fs + min(bin, max(n_bins, 1) - 1);
+      const unsigned long long* const img = st.images + static_cast<int64_t>(pair) * a.K * fs + static_cast<int64_t>(f) * a.S + at;
+#pragma unroll
+      for (int c = 0; c < kAhead; c++) ahead[c] = img[min(c, p.chunks - 1) * step];
+      if (!root) parent_ahead = parent[at];
+    };
+    if constexpr (kAhead > 0) fetch(0, tid);
     for (int base = 0; base < n_bins; base += kScan) {
       const int bin = base + tid;
       const bool in = bin < n_bins;
       double gain_n = 0.0, gain_s = 0.0;
       bool dead_n = !in, dead_s = !in || root;
       bool left_n = false, left_s = false;
+      uint2 cell_n = make_uint2(0, 0), cell_s = make_uint2(0, 0);  // kLast
       for (int k = 0; k < a.K; k++) {
         uint32_t raw_g = 0, raw_h = 0;  // of the bin, lower halves
-        I64Pair pv{0, 0};
+        uint2 pv = make_uint2(0, 0);
         I64Pair ns = st.node_sums[static_cast<int64_t>(p.level_first + node) * a.K + k];
         // (the root's, which has no sibling, are its own: behind a condition hipcc waits for them before it asks for anything else)
         I64Pair ss = st.node_sums[static_cast<int64_t>(p.level_first + (root ? node : sib)) * a.K + k];
-        if (in) {
+        if constexpr (kAhead > 0) {
+#pragma unroll
+          for (int c = 0; c < kAhead; c++) {
+            raw_g += c < p.chunks ? static_cast<uint32_t>(ahead[c] >> 32) : 0u;
+            raw_h += c < p.chunks ? static_cast<uint32_t>(ahead[c]) : 0u;
+          }
+          pv = parent_ahead;
+          const unsigned long long* const img =
+            st.images + (static_cast<int64_t>(pair) * a.K + k) * fs + static_cast<int64_t>(f) * a.S + min(bin, n_bins - 1);
+          for (int c = kAhead; c < p.chunks; c += kAhead) {
+            unsigned long long w[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) w[u] = img[min(c + u, p.chunks - 1) * step];
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+              raw_g += c + u < p.chunks ? static_cast<uint32_t>(w[u] >> 32) : 0u;
+              raw_h += c + u < p.chunks ? static_cast<uint32_t>(w[u]) : 0u;
+            }
+          }
+          raw_g = in ? raw_g : 0u;
+          raw_h = in ? raw_h : 0u;
+          if (k + 1 < a.K)
+            fetch(k + 1, bin);
+          else if (base + kScan < n_bins)
+            fetch(0, bin + kScan);
+        } else if (in) {
           const unsigned long long* img = st.images + (static_cast<int64_t>(pair) * a.K + k) * fs + static_cast<int64_t>(f) * a.S + bin;
-          const int64_t step = static_cast<int64_t>(p.built) * a.K * fs;
           if (!root) pv = parent[k * fs + bin];
           int c = 0;
           auto add = [&](auto width) {
@@ -788,10 +842,11 @@ __global__ void __launch_bounds__(kScan)
         const uint32_t kept = h == 0 && g + down <= down ? raw_g : g;
         // all that was asked for, before the stores below: a wait for it behind them would wait for them too (11,094 x 120, 5 outputs, 512 samples,
         // depth 8: 117 us a launch, and 101)
-        arrived(ns), arrived(ss), arrived(pv);
+        arrived(ns), arrived(ss);
+        asm volatile("" : "+v"(pv.x), "+v"(pv.y));
         // whole numbers below 2^35 and their differences are exact as doubles
         const double nlg = static_cast<double>(kept + down) - down_of, nlh = static_cast<double>(h);
-        const double slg = static_cast<double>(pv.grad) - nlg, slh = static_cast<double>(pv.hess) - nlh;
+        const double slg = static_cast<double>(pv.x + down) - down_of - nlg, slh = static_cast<double>(pv.y) - nlh;
         const double nrg = static_cast<double>(ns.grad) - nlg, nrh = static_cast<double>(ns.hess) - nlh;
         const double srg = static_cast<double>(ss.grad) - slg, srh = static_cast<double>(ss.hess) - slh;
         const double n_left = quotient(nlg * inv_g, nlh * inv_h), n_right = quotient(nrg * inv_g, nrh * inv_h);
@@ -806,11 +861,13 @@ __global__ void __launch_bounds__(kScan)
         dead_s |= slh <= 0 || srh <= 0;
         gain_n += 0.5 * (n_left + n_right - n_own) - a.min_split_gain;
         gain_s += 0.5 * (s_left + s_right - s_own) - a.min_split_gain;
-        if (in) {
+        if constexpr (kLast) {
+          cell_n = make_uint2(kept, h);
+          cell_s = make_uint2(pv.x - kept, pv.y - h);
+        } else if (in) {
           const int64_t at = static_cast<int64_t>(k) * fs + static_cast<int64_t>(f) * a.S + bin;
-          const I64Pair nv{static_cast<int64_t>(kept + down) - static_cast<int64_t>(down), static_cast<int64_t>(h)};
-          hist[static_cast<int64_t>(node) * a.K * fs + at] = nv;
-          if (!root) hist[static_cast<int64_t>(sib) * a.K * fs + at] = I64Pair{pv.grad - nv.grad, pv.hess - nv.hess};
+          hist[static_cast<int64_t>(node) * a.K * fs + at] = make_uint2(kept, h);
+          if (!root) hist[static_cast<int64_t>(sib) * a.K * fs + at] = make_uint2(pv.x - kept, pv.y - h);
         }
         // the carry of a tile is read by the next one; a barrier of the next output lies between
         if (base + kScan < n_bins) {
@@ -824,9 +881,11 @@ __global__ void __launch_bounds__(kScan)
       best_n = take_n ? gain_n : best_n;
       key_n  = take_n ? key : key_n;
       if constexpr (kLess) less_n = take_n ? left_n : less_n;
+      if constexpr (kLast) best_cell_n = make_uint2(take_n ? cell_n.x : best_cell_n.x, take_n ? cell_n.y : best_cell_n.y);
       best_s = take_s ? gain_s : best_s;
       key_s  = take_s ? key : key_s;
       if constexpr (kLess) less_s = take_s ? left_s : less_s;
+      if constexpr (kLast) best_cell_s = make_uint2(take_s ? cell_s.x : best_cell_s.x, take_s ? cell_s.y : best_cell_s.y);
       if (base + kScan < n_bins) __syncthreads();
     }
   };
@@ -842,6 +901,10 @@ __global__ void __launch_bounds__(kScan)
     less_n = __any(less_n && own_key_n == key_n && own_n == best_n);  // (no two lanes have one key)
     less_s = __any(less_s && own_key_s == key_s && own_s == best_s);
   }
+  if constexpr (kLast) {
+    if (key_n != 0 && own_key_n == key_n && own_n == best_n) s_cell[0][wave] = best_cell_n;
+    if (key_s != 0 && own_key_s == key_s && own_s == best_s) s_cell[1][wave] = best_cell_s;
+  }
   if (lane == 0) {
     s_best[0][wave] = best_n;
     s_bkey[0][wave] = key_n;
@@ -854,14 +917,174 @@ __global__ void __launch_bounds__(kScan)
   if (tid < (root ? 1 : 2)) {
     double best  = 0.0;
     unsigned key = 0;
-    int less     = 0;
+    int less     = 0, from = 0;
     for (int w = 0; w < kScan / 64; w++) {
       const bool take = s_best[tid][w] > best || (s_best[tid][w] == best && s_bkey[tid][w] > key);
       best = take ? s_best[tid][w] : best;
       key  = take ? s_bkey[tid][w] : key;
       less = take ? s_less[tid][w] : less;
+      from = take ? w : from;
     }
+    if (kLast && key != 0) st.left[static_cast<int64_t>(tid == 0 ? node : sib) * a.F + f] = s_cell[tid][from];
     st.cand[static_cast<int64_t>(tid == 0 ? node : sib) * a.F + f] = SmallCand{best, key, key != 0 ? (bin_of_tie_key(key) - rp) | less : 0};
+  }
+}
+
+// The same with a wave for a (pair of siblings, feature), 64 bins at a time: no barrier, no exchange through the LDS, and the terms that do not
+// depend on the bin once an output instead of once a thread. Below the root, where nobody asks for the smaller child, and from kWavePairs on:
+// with fewer the waves of a workgroup, which take the bins of a feature at a time, finish sooner than one that takes them in turn (50,000 x 200,
+// 256 samples, levels of 1600, 3200, 6400 and 12,800 pairs and features: 8.8, 12.2, 18.0 and 27.7 us, by workgroups with 16 bytes a bin 13.6, 19.4,
+// 33.1 and 61.2; 512 and 2048 as the bound give the same trees' times within 1 %). A tree of 50,000 x 200, depth 8: 353 us, now 297; of 20,000 x 60, 128 samples, depth 10,
+// 351 and 306; of 50,000 x 100 with 2 outputs, 64 samples, depth 9, 405 and 319.
+template <bool kLast>
+__global__ void __launch_bounds__(kScan)
+  mid_scan_waves_kernel(MidArgs a, MidTreeState st, LevelPlan p)
+{
+  const int lane = threadIdx.x & 63;
+  const int item = static_cast<int>(blockIdx.x) * (kScan / 64) + __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int f = item % a.F, pair = item / a.F;
+  if (pair >= p.built || level_is_empty(st, p.depth)) return;
+  const I64Pair* const sums = st.node_sums + static_cast<int64_t>(p.level_first + 2 * pair) * a.K;  // the left child's, then the right one's
+  const int64_t left_h = sums[0].hess, right_h = sums[a.K].hess;
+  // the children of a node that did not split have no rows
+  if (left_h <= 0) return;
+  const int own = left_h < right_h ? 0 : 1;  // built_of_pair
+  const int64_t node = 2 * pair + own, sib = node ^ 1;
+  if (a.feature_set != nullptr && a.feature_set[f] == 0) {
+    if (lane < 2) st.cand[(2 * pair + lane) * static_cast<int64_t>(a.F) + f] = SmallCand{0.0, 0u, 0};
+    return;
+  }
+  const int n_bins = st.counts[f], rp = st.rp[f];
+  const int64_t fs = static_cast<int64_t>(a.F) * a.S;
+  const uint32_t down  = static_cast<uint32_t>(st.q_stats[1]);
+  const double down_of = static_cast<double>(down);
+  const double inv_g = st.scales[2], inv_h = st.scales[3];
+  const double reg   = 1e-5 > a.l2 ? 1e-5 : a.l2;
+  uint2* const hist         = st.hist[p.depth & 1];
+  const uint2* const parent = st.hist[(p.depth & 1) ^ 1] + static_cast<int64_t>(pair) * a.K * fs + static_cast<int64_t>(f) * a.S;
+  const unsigned long long* const images = st.images + static_cast<int64_t>(pair) * a.K * fs + static_cast<int64_t>(f) * a.S;
+  const int64_t step = static_cast<int64_t>(p.built) * a.K * fs;
+  // lane k: sums of output k, and the term of the gains that does not depend on the bin
+  I64Pair ns{0, 0}, ss{0, 0};
+  if (lane < a.K) {
+    ns = sums[own * a.K + lane];
+    ss = sums[(own ^ 1) * a.K + lane];
+  }
+  const double all_ng = static_cast<double>(ns.grad), all_nh = static_cast<double>(ns.hess);
+  const double all_sg = static_cast<double>(ss.grad), all_sh = static_cast<double>(ss.hess);
+  double best_n = 0.0, best_s = 0.0;
+  unsigned key_n = 0, key_s = 0;
+  uint2 best_cell_n = make_uint2(0, 0), best_cell_s = make_uint2(0, 0);  // kLast: what lies left of it
+  auto run = [&](auto plains) {
+    auto quotient = [&](double grad, double hess) {
+      if constexpr (decltype(plains)::value)
+        return quotient_plain(grad * grad, hess + reg);
+      else
+        return leaf_gain_select(grad, hess, a.l1, reg);
+    };
+    const double own_n = quotient(all_ng * inv_g, all_nh * inv_h), own_s = quotient(all_sg * inv_g, all_sh * inv_h);
+    // the images and the parent's bins of the next 64 bins (or of the next output's) are on their way while these are summed
+    constexpr int kAhead = 4;
+    unsigned long long ahead[kAhead];
+    uint2 parent_ahead;
+    const int tiles = (n_bins + 63) / 64, items = tiles * a.K;
+    int next_k = 0, next_bin = lane;
+    auto fetch = [&]() {
+      const int64_t at = next_k * fs + min(next_bin, max(n_bins, 1) - 1);
+#pragma unroll
+      for (int c = 0; c < kAhead; c++) ahead[c] = images[at + min(c, p.chunks - 1) * step];
+      parent_ahead = parent[at];
+      if (++next_k == a.K) {
+        next_k = 0;
+        next_bin += 64;
+      }
+    };
+    fetch();
+    uint32_t agg_g = 0, agg_h = 0;  // lane k: output k's sums of the bins so far
+    int k = 0, bin = lane;
+    double gain_n = 0.0, gain_s = 0.0;
+    bool live_n = true, live_s = true;
+    for (int i = 0; i < items; i++) {
+      const bool in = bin < n_bins;
+      uint32_t raw_g = 0, raw_h = 0;
+#pragma unroll
+      for (int c = 0; c < kAhead; c++) {
+        raw_g += c < p.chunks ? static_cast<uint32_t>(ahead[c] >> 32) : 0u;
+        raw_h += c < p.chunks ? static_cast<uint32_t>(ahead[c]) : 0u;
+      }
+      const uint2 pv     = parent_ahead;
+      const int64_t here = k * fs + min(bin, n_bins - 1);
+      for (int c = kAhead; c < p.chunks; c += 4) {
+        unsigned long long w[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) w[u] = images[here + min(c + u, p.chunks - 1) * step];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          raw_g += c + u < p.chunks ? static_cast<uint32_t>(w[u] >> 32) : 0u;
+          raw_h += c + u < p.chunks ? static_cast<uint32_t>(w[u]) : 0u;
+        }
+      }
+      if (i + 1 < items) fetch();
+      raw_g = in ? raw_g : 0u;
+      raw_h = in ? raw_h : 0u;
+      const uint32_t g = wave_inclusive_sum32(raw_g) + wave_read_lane32(agg_g, k);
+      const uint32_t h = wave_inclusive_sum32(raw_h) + wave_read_lane32(agg_h, k);
+      const uint32_t to_g = wave_read_lane32(g, 63), to_h = wave_read_lane32(h, 63);
+      if (lane == k) {
+        agg_g = to_g;
+        agg_h = to_h;
+      }
+      // (the rule on bins that the reference leaves as they are, see mid_scan_kernel)
+      const uint32_t kept = h == 0 && g + down <= down ? raw_g : g;
+      const double nlg = static_cast<double>(kept + down) - down_of, nlh = static_cast<double>(h);
+      const double slg = static_cast<double>(pv.x + down) - down_of - nlg, slh = static_cast<double>(pv.y) - nlh;
+      const double nrg = wave_read_lane_f64(all_ng, k) - nlg, nrh = wave_read_lane_f64(all_nh, k) - nlh;
+      const double srg = wave_read_lane_f64(all_sg, k) - slg, srh = wave_read_lane_f64(all_sh, k) - slh;
+      const double n_left = quotient(nlg * inv_g, nlh * inv_h), n_right = quotient(nrg * inv_g, nrh * inv_h);
+      const double s_left = quotient(slg * inv_g, slh * inv_h), s_right = quotient(srg * inv_g, srh * inv_h);
+      live_n = live_n && nlh > 0 && nrh > 0;
+      live_s = live_s && slh > 0 && srh > 0;
+      gain_n += 0.5 * (n_left + n_right - wave_read_lane_f64(own_n, k)) - a.min_split_gain;
+      gain_s += 0.5 * (s_left + s_right - wave_read_lane_f64(own_s, k)) - a.min_split_gain;
+      if (!kLast && in) {
+        hist[node * a.K * fs + static_cast<int64_t>(f) * a.S + here] = make_uint2(kept, h);
+        hist[sib * a.K * fs + static_cast<int64_t>(f) * a.S + here]  = make_uint2(pv.x - kept, pv.y - h);
+      }
+      if (++k == a.K) {
+        const unsigned key = tie_key_of_bin(rp + bin);
+        const bool take_n = in && live_n && gain_n > 0 && (gain_n > best_n || (gain_n == best_n && key > key_n));
+        const bool take_s = in && live_s && gain_s > 0 && (gain_s > best_s || (gain_s == best_s && key > key_s));
+        best_n = take_n ? gain_n : best_n;
+        key_n  = take_n ? key : key_n;
+        best_s = take_s ? gain_s : best_s;
+        key_s  = take_s ? key : key_s;
+        if constexpr (kLast) {
+          best_cell_n = make_uint2(take_n ? kept : best_cell_n.x, take_n ? h : best_cell_n.y);
+          best_cell_s = make_uint2(take_s ? pv.x - kept : best_cell_s.x, take_s ? pv.y - h : best_cell_s.y);
+        }
+        k = 0;
+        bin += 64;
+        gain_n = gain_s = 0.0;
+        live_n = live_s = true;
+      }
+    }
+  };
+  if (plain_quotients(a.l1, inv_g, inv_h, reg))
+    run(std::true_type{});
+  else
+    run(std::false_type{});
+  const double lane_n = best_n, lane_s = best_s;
+  const unsigned lane_key_n = key_n, lane_key_s = key_s;
+  wave_best_key(best_n, key_n);
+  wave_best_key(best_s, key_s);
+  if constexpr (kLast) {
+    // (no two lanes have one key)
+    if (key_n != 0 && lane_key_n == key_n && lane_n == best_n) st.left[node * a.F + f] = best_cell_n;
+    if (key_s != 0 && lane_key_s == key_s && lane_s == best_s) st.left[sib * a.F + f] = best_cell_s;
+  }
+  if (lane < 2) {
+    const unsigned key = lane == 0 ? key_n : key_s;
+    st.cand[(lane == 0 ? node : sib) * a.F + f] = SmallCand{lane == 0 ? best_n : best_s, key, key != 0 ? bin_of_tie_key(key) - rp : 0};
   }
 }
 
@@ -981,7 +1204,7 @@ size_t mid_hist_bytes(int64_t N, int F, int K, int max_depth, int S)
     const LevelPlan p = plan_level(N, F, K, S, d, max_depth);
     images            = std::max(images, static_cast<int64_t>(p.chunks) * p.built * fs);
   }
-  return static_cast<size_t>(2 * (int64_t(1) << (max_depth - 1)) * fs) * sizeof(I64Pair) + static_cast<size_t>(images) * 8;
+  return static_cast<size_t>(2 * (int64_t(1) << (max_depth - 1)) * fs) * sizeof(uint2) + static_cast<size_t>(images) * 8;
 }
 
 // By size: measured against the general builder (one output, depth 8 and 256 samples unless stated), us: 20,000 x 100
@@ -1052,6 +1275,13 @@ static int launch_histograms(hipStream_t stream, const MidTreeState& st, const M
   return LBT_OK;
 }
 
+template <bool kLess>
+static auto scan_of(int K, int chunks)
+{
+  if (K == 1) return mid_scan_kernel<kLess, false, 0>;
+  return chunks <= 4 ? mid_scan_kernel<kLess, false, 4> : chunks <= 8 ? mid_scan_kernel<kLess, false, 8> : mid_scan_kernel<kLess, false, 16>;
+}
+
 template <typename T, typename BinT>
 static int queue_levels(hipStream_t stream, const MidTreeState& st, const MidArgs& a, const DeviceAnswer& answer,
                         LevelMeta* level_totals)
@@ -1078,9 +1308,15 @@ static int queue_levels(hipStream_t stream, const MidTreeState& st, const MidArg
       ProfScope ps(LBT_PROF_SCAN, stream);
       const unsigned grid = static_cast<unsigned>(p.built) * a.F;
       if (later)
-        mid_scan_kernel<true><<<grid, kScan, 0, stream>>>(a, st, p);
+        scan_of<true>(a.K, p.chunks)<<<grid, kScan, 0, stream>>>(a, st, p);
+      else if (d > 0 && static_cast<int64_t>(grid) >= kWavePairs && p.last && a.K == 1)
+        mid_scan_waves_kernel<true><<<(grid + kScan / 64 - 1) / (kScan / 64), kScan, 0, stream>>>(a, st, p);
+      else if (d > 0 && static_cast<int64_t>(grid) >= kWavePairs)
+        mid_scan_waves_kernel<false><<<(grid + kScan / 64 - 1) / (kScan / 64), kScan, 0, stream>>>(a, st, p);
+      else if (p.last && a.K == 1)
+        mid_scan_kernel<false, true, 0><<<grid, kScan, 0, stream>>>(a, st, p);
       else
-        mid_scan_kernel<false><<<grid, kScan, 0, stream>>>(a, st, p);
+        scan_of<false>(a.K, p.chunks)<<<grid, kScan, 0, stream>>>(a, st, p);
     }
     ProfScope ps(LBT_PROF_POSITIONS, stream);
     const unsigned grid = static_cast<unsigned>((a.N + kRowsApply - 1) / kRowsApply);

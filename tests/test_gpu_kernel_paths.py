@@ -976,3 +976,36 @@ def test_levels_of_the_general_builder_that_begin_in_one_launch(n, f, k, s, dept
     for name in ("leaf_value", "feature", "split_value", "gain", "hessian", "row_leaf"):
         assert torch.equal(getattr(got, name), getattr(want, name)), name
     gu.check_row_leaf(got, X)
+
+
+@pytest.mark.parametrize("n,f,k,s,depth,kind", [
+    (9000, 64, 1, 1, 6, "plain"),            # one bin, one tile
+    (9001, 65, 1, 64, 6, "plain"),           # a full tile; workgroups of which some waves have nothing left
+    (9001, 31, 1, 65, 9, "zeros"),           # one bin in the second tile
+    (12000, 131, 1, 256, 5, "excluded"),
+    (8200, 33, 2, 300, 7, "l1"),             # two-byte bins, a tile that is not full
+    (70000, 40, 3, 129, 7, "zeros"),         # ranges of rows past those asked for ahead
+    (9001, 64, 16, 32, 5, "excluded"),
+    (8193, 130, 1, 2048, 5, "l1"),
+    (200000, 16, 5, 257, 6, "plain"),        # by workgroups: 16 ranges and more, a second tile of bins, several outputs
+])
+def test_scans_of_wide_levels(n, f, k, s, depth, kind):
+    """Scans of a wave for a pair of siblings and a feature, with their neighbours: tiles and outputs in turn, loads one item ahead."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(n + f)
+    X = rs.randn(n, f).astype(np.float32)
+    X[:, 1] = np.round(X[:, 1])
+    g = rs.randn(n, k) + np.sin(2 * X[:, :1]) + X[:, 2:3] * X[:, 3:4]
+    h = rs.rand(n, k) + 0.1
+    if kind == "zeros":
+        h[rs.rand(n, k) < 0.4] = 0.0
+    mask = rs.rand(f) < 0.6 if kind == "excluded" else None
+    kw = dict(l1=0.05, l2=0.5, min_split_gain=1e-3) if kind == "l1" else {}
+    kw2 = dict(l1_regularization=0.05, l2_regularization=0.5, min_split_gain=1e-3) if kw else {}
+    cr = orc.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=n, feature_set=mask, **kw)
+    got = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=n, feature_set=mask, row_leaf=True, **kw2)
+    _assert_tree(got, cr)
+    gu.check_row_leaf(got, X)
