@@ -25,30 +25,44 @@ constexpr int kThreads = 256;
 // ---------------------------------------------------------------------------
 
 // Also what the TreeBuilder's constructor sets up (build_tree.cu:967-974, every row starts in the
-// root) and the per-level counters, so that a tree starts with one launch instead of three.
-__global__ void init_tree_kernel(double* leaf, int32_t* feature, double* split, double* gain,
-                                 I64Pair* node_sums, int64_t max_nodes, int K, int32_t* rows, int64_t n, int32_t* seg,
-                                 int32_t* block_seg, int64_t n_slabs, uint4* level_totals, int n_totals16, uint8_t* tainted)
-{
-  int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-  if (i < max_nodes * K) {
-    leaf[i]      = 0.0;
-    node_sums[i] = I64Pair{0, 0};
+// root) and the per-level counters.
+struct InitArgs {
+  double* leaf;
+  int32_t* feature;
+  double* split;
+  double* gain;
+  I64Pair* node_sums;
+  int64_t max_nodes;
+  int K;
+  int32_t* rows;
+  int64_t n;
+  int32_t* seg;
+  int32_t* block_seg;
+  int64_t n_slabs;
+  uint4* level_totals;
+  int n_totals16;
+  uint8_t* tainted;
+  __device__ __forceinline__ void entry(int64_t i) const
+  {
+    if (i < max_nodes * K) {
+      leaf[i]      = 0.0;
+      node_sums[i] = I64Pair{0, 0};
+    }
+    if (i < max_nodes) {
+      feature[i] = -1;
+      split[i]   = 0.0;
+      gain[i]    = 0.0;
+      tainted[i] = 0;
+    }
+    if (i < n) rows[i] = static_cast<int32_t>(i);
+    if (i < n_slabs) block_seg[i] = 0;
+    if (i < n_totals16) level_totals[i] = make_uint4(0, 0, 0, 0);
+    if (i == 0) {
+      seg[0] = 0;
+      seg[1] = static_cast<int32_t>(n);
+    }
   }
-  if (i < max_nodes) {
-    feature[i] = -1;
-    split[i]   = 0.0;
-    gain[i]    = 0.0;
-    tainted[i] = 0;
-  }
-  if (i < n) rows[i] = static_cast<int32_t>(i);
-  if (i < n_slabs) block_seg[i] = 0;
-  if (i < n_totals16) level_totals[i] = make_uint4(0, 0, 0, 0);
-  if (i == 0) {
-    seg[0] = 0;
-    seg[1] = static_cast<int32_t>(n);
-  }
-}
+};
 
 __global__ void write_hessian_kernel(double* hessian, const I64Pair* node_sums, int64_t n,
                                      const double* scales)
@@ -84,78 +98,84 @@ __global__ void __launch_bounds__(kThreads) zero_built_kernel(HistView hist, con
 // split proposals (build_tree.cu:867-964)
 // ---------------------------------------------------------------------------
 
-// draft[f][i] = X[row_i][f] for the S sampled rows; row_i from a fresh
-// minstd engine advanced by i (build_tree.cu:882-898).
 template <typename T>
-__global__ void gather_samples_kernel(const T* X, int64_t row_offset, int64_t n_rows, int F,
-                                      int S, int32_t seed, int64_t dataset_rows, T* draft)
+struct SampleArgs {
+  const T* X;
+  int64_t row_offset, n_rows, dataset_rows;
+  int F, S, P;  // features, samples, the power of two that holds them
+  int32_t seed;
+  T* uniq;          // [F][S]
+  int32_t* counts;  // [F]
+  int32_t* row_pointers;
+  T* proposals;
+  int32_t* bin_feature;
+  double* as_double;           // optional: the proposals as doubles, what WriteTreeOutput stores as split values
+  int32_t* host_row_pointers;  // optional: the row pointers for the host, F + 1 words
+};
+
+// Sum over a workgroup of 256, and what lies in front of the thread.
+__device__ __forceinline__ int sum_before(int mine, int* s_waves, int* all)
 {
-  int64_t idx = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-  if (idx >= static_cast<int64_t>(F) * S) return;
-  int i        = static_cast<int>(idx / F);
-  int j        = static_cast<int>(idx % F);
-  uint32_t x   = minstd_seed(static_cast<uint32_t>(seed));
-  x            = minstd_discard(x, static_cast<uint64_t>(i));
-  x            = minstd_next(x);
-  double u     = uniform01(x);
-  double b     = static_cast<double>(dataset_rows - 1) + 1.0;
-  int64_t row  = static_cast<int64_t>((u * (b - 0.0)) + 0.0);
-  bool has     = row >= row_offset && row <= row_offset + n_rows - 1;
-  draft[static_cast<int64_t>(j) * S + i] = has ? X[(row - row_offset) * F + j] : T(0);
+  const int incl = static_cast<int>(wave_inclusive_sum32(static_cast<uint32_t>(mine)));
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 63) s_waves[wave] = incl;
+  __syncthreads();
+  int before = incl - mine, total = 0;
+  for (int w = 0; w < kThreads / 64; w++) {
+    before += w < wave ? s_waves[w] : 0;
+    total += s_waves[w];
+  }
+  *all = total;
+  return before;
 }
 
-// One workgroup per feature: bitonic sort of the S samples in LDS on
-// order-preserving integer keys, then drop values equal to their predecessor
-// (thrust::sort + unique_copy, build_tree.cu:908-931).
+// A workgroup's feature: the S sampled rows' values, row_i from a fresh minstd engine advanced by i (build_tree.cu:882-898),
+// sorted in the LDS on order-preserving integer keys, without those equal to their predecessor (thrust::sort +
+// unique_copy, build_tree.cu:908-931).
 template <typename T>
-__global__ void __launch_bounds__(kThreads)
-  sort_unique_kernel(const T* draft, int S, int P, T* uniq, int32_t* counts)
+__device__ __forceinline__ void unique_samples(const SampleArgs<T>& a, int f, typename KeyOf<T>::type* keys, int* s_waves)
 {
   using Key = typename KeyOf<T>::type;
-  extern __shared__ __align__(16) unsigned char smem_raw[];  // 16-byte aligned whatever static LDS precedes it
-  Key* keys       = reinterpret_cast<Key*>(smem_raw);
-  __shared__ int s_cnt[kThreads];
-  const int f     = blockIdx.x;
-  const T* src    = draft + static_cast<int64_t>(f) * S;
-  for (int i = threadIdx.x; i < P; i += kThreads) keys[i] = i < S ? to_key(src[i]) : ~Key(0);
+  for (int i = threadIdx.x; i < a.P; i += kThreads) {
+    Key key = ~Key(0);
+    if (i < a.S) {
+      const uint32_t x = minstd_next(minstd_discard(minstd_seed(static_cast<uint32_t>(a.seed)), static_cast<uint64_t>(i)));
+      const double u   = uniform01(x);
+      const double b   = static_cast<double>(a.dataset_rows - 1) + 1.0;
+      const int64_t row = static_cast<int64_t>((u * (b - 0.0)) + 0.0);
+      const bool has    = row >= a.row_offset && row <= a.row_offset + a.n_rows - 1;
+      key = to_key(has ? a.X[(row - a.row_offset) * a.F + f] : T(0));
+    }
+    keys[i] = key;
+  }
   __syncthreads();
-  for (int size = 2; size <= P; size <<= 1) {
+  for (int size = 2; size <= a.P; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = threadIdx.x; i < P / 2; i += kThreads) {
+      for (int i = threadIdx.x; i < a.P / 2; i += kThreads) {
         int lo      = 2 * i - (i & (stride - 1));  // index with the stride bit clear
         int hi      = lo + stride;
         bool up     = (lo & size) == 0;
-        Key a = keys[lo], b = keys[hi];
-        if ((a > b) == up) {
-          keys[lo] = b;
-          keys[hi] = a;
+        Key x = keys[lo], y = keys[hi];
+        if ((x > y) == up) {
+          keys[lo] = y;
+          keys[hi] = x;
         }
       }
       __syncthreads();
     }
   }
   // thread t owns the contiguous slice [t*per, (t+1)*per)
-  const int per = (S + kThreads - 1) / kThreads;
-  int begin = threadIdx.x * per, end = min(S, begin + per);
+  const int per = (a.S + kThreads - 1) / kThreads;
+  const int begin = min(a.S, static_cast<int>(threadIdx.x) * per), end = min(a.S, begin + per);
   int cnt = 0;
   for (int i = begin; i < end; i++) {
     bool keep = i == 0 || !(from_key(keys[i]) == from_key(keys[i - 1]));
     cnt += keep ? 1 : 0;
   }
-  s_cnt[threadIdx.x] = cnt;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int t = 0; t < kThreads; t++) {
-      int c    = s_cnt[t];
-      s_cnt[t] = run;
-      run += c;
-    }
-    counts[f] = run;
-  }
-  __syncthreads();
-  int at = s_cnt[threadIdx.x];
-  T* dst = uniq + static_cast<int64_t>(f) * S;
+  int all = 0;
+  int at  = sum_before(cnt, s_waves, &all);
+  if (threadIdx.x == 0) a.counts[f] = all;
+  T* dst = a.uniq + static_cast<int64_t>(f) * a.S;
   for (int i = begin; i < end; i++) {
     bool keep = i == 0 || !(from_key(keys[i]) == from_key(keys[i - 1]));
     if (keep) dst[at++] = from_key(keys[i]);
@@ -171,53 +191,29 @@ __device__ __forceinline__ void store_for_host(int32_t* to, int32_t v)
   __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// CSR row pointers (reduce_by_key + inclusive_scan, build_tree.cu:933-949)
-// One workgroup: every thread adds up a run of consecutive counts, the runs are joined by a scan
-// over the workgroup, and the thread walks its run again to write the pointers.
-// host_row_pointers (optional): the same for the host, F + 1 words
-__global__ void __launch_bounds__(kThreads)
-  row_pointers_kernel(const int32_t* counts, int F, int32_t* row_pointers, int32_t* host_row_pointers)
-{
-  __shared__ int s_scan[kThreads];
-  const int per   = (F + kThreads - 1) / kThreads;
-  const int begin = min(F, static_cast<int>(threadIdx.x) * per);
-  const int end   = min(F, begin + per);
-  int mine = 0;
-  for (int f = begin; f < end; f++) mine += counts[f];
-  s_scan[threadIdx.x] = mine;
-  __syncthreads();
-  for (int off = 1; off < kThreads; off <<= 1) {
-    const int v = static_cast<int>(threadIdx.x) >= off ? s_scan[threadIdx.x - off] : 0;
-    __syncthreads();
-    s_scan[threadIdx.x] += v;
-    __syncthreads();
-  }
-  int run = s_scan[threadIdx.x] - mine;
-  if (threadIdx.x == 0) {
-    row_pointers[0] = 0;
-    if (host_row_pointers != nullptr) store_for_host(host_row_pointers, 0);
-  }
-  for (int f = begin; f < end; f++) {
-    run += counts[f];
-    row_pointers[f + 1] = run;
-    if (host_row_pointers != nullptr) store_for_host(host_row_pointers + f + 1, run);
-  }
-}
-
-// compact copy; the last proposal of each feature becomes +inf (build_tree.cu:953-956)
-// as_double (optional): the same values as doubles, what WriteTreeOutput stores as split values
+// A workgroup's feature: its CSR row pointer (reduce_by_key + inclusive_scan, build_tree.cu:933-949) and its proposals in
+// their place, the last one +inf (build_tree.cu:953-956).
 template <typename T>
-__global__ void compact_proposals_kernel(const T* uniq, int S, const int32_t* row_pointers,
-                                         T* proposals, int32_t* bin_feature, double* as_double)
+__device__ __forceinline__ void place_proposals(const SampleArgs<T>& a, int f, int* s_waves)
 {
-  const int f = blockIdx.x;
-  int b0 = row_pointers[f], b1 = row_pointers[f + 1];
-  for (int i = threadIdx.x; i < b1 - b0; i += blockDim.x) {
-    T v = uniq[static_cast<int64_t>(f) * S + i];
-    if (i == b1 - b0 - 1) v = std::numeric_limits<T>::infinity();
-    proposals[b0 + i]   = v;
-    bin_feature[b0 + i] = f;
-    if (as_double != nullptr) as_double[b0 + i] = static_cast<double>(v);
+  int mine = 0, b0 = 0;
+  for (int i = threadIdx.x; i < f; i += kThreads) mine += a.counts[i];
+  sum_before(mine, s_waves, &b0);
+  const int n = a.counts[f];
+  if (threadIdx.x == 0) {
+    a.row_pointers[f + 1] = b0 + n;
+    if (f == 0) a.row_pointers[0] = 0;
+    if (a.host_row_pointers != nullptr) {
+      store_for_host(a.host_row_pointers + f + 1, b0 + n);
+      if (f == 0) store_for_host(a.host_row_pointers, 0);
+    }
+  }
+  for (int i = threadIdx.x; i < n; i += kThreads) {
+    T v = a.uniq[static_cast<int64_t>(f) * a.S + i];
+    if (i == n - 1) v = std::numeric_limits<T>::infinity();
+    a.proposals[b0 + i]   = v;
+    a.bin_feature[b0 + i] = f;
+    if (a.as_double != nullptr) a.as_double[b0 + i] = static_cast<double>(v);
   }
 }
 
@@ -229,34 +225,40 @@ __global__ void compact_proposals_kernel(const T* uniq, int S, const int32_t* ro
 // entries t, t+256, ... in order, then a binary tree (strides 128..1) joins the
 // 256 lanes. The reference leaves this order to thrust::reduce
 // (build_tree.cu:82-83); fixing it makes the two scale factors reproducible.
+constexpr int kSumChunk = 4096;
+struct TwoSums {
+  double a[kThreads], b[kThreads];
+};
 template <bool kAbs>
-__global__ void __launch_bounds__(kThreads)
-  abs_sum_level_kernel(const double* a, const double* b, int64_t n, double* out_a, double* out_b)
+__device__ __forceinline__ void sum_chunk(const double* a, const double* b, int64_t n, int64_t c, TwoSums& s)
 {
-  __shared__ double sa[kThreads];
-  __shared__ double sb[kThreads];
-  const int64_t c = blockIdx.x;
   double xa = 0.0, xb = 0.0;
-  for (int j = 0; j < 16; j++) {
-    int64_t e = c * 4096 + threadIdx.x + static_cast<int64_t>(kThreads) * j;
+  for (int j = 0; j < kSumChunk / kThreads; j++) {
+    int64_t e = c * kSumChunk + threadIdx.x + static_cast<int64_t>(kThreads) * j;
     if (e < n) {
       xa += kAbs ? fabs(a[e]) : a[e];
       xb += kAbs ? fabs(b[e]) : b[e];
     }
   }
-  sa[threadIdx.x] = xa;
-  sb[threadIdx.x] = xb;
+  s.a[threadIdx.x] = xa;
+  s.b[threadIdx.x] = xb;
   __syncthreads();
   for (int stride = kThreads / 2; stride >= 1; stride >>= 1) {
     if (static_cast<int>(threadIdx.x) < stride) {
-      sa[threadIdx.x] += sa[threadIdx.x + stride];
-      sb[threadIdx.x] += sb[threadIdx.x + stride];
+      s.a[threadIdx.x] += s.a[threadIdx.x + stride];
+      s.b[threadIdx.x] += s.b[threadIdx.x + stride];
     }
     __syncthreads();
   }
+}
+__global__ void __launch_bounds__(kThreads)
+  sum_level_kernel(const double* a, const double* b, int64_t n, double* out_a, double* out_b)
+{
+  __shared__ TwoSums s;
+  sum_chunk<false>(a, b, n, blockIdx.x, s);
   if (threadIdx.x == 0) {
-    out_a[c] = sa[0];
-    out_b[c] = sb[0];
+    out_a[blockIdx.x] = s.a[0];
+    out_b[blockIdx.x] = s.b[0];
   }
 }
 
@@ -265,20 +267,79 @@ constexpr unsigned kQuantTooLarge        = 1u;  // a value does not fit the pack
                                                 // entry that holds the whole absolute sum, rounded up)
 constexpr unsigned kQuantHessNotPositive = 2u;  // an entry that is not (0, 0) and whose hessian is not positive
 constexpr unsigned kQuantHessNegative    = 4u;  // an entry whose hessian is negative
-__global__ void scales_kernel(const double* sum_a, const double* sum_b, double* scales,
-                              unsigned long long* qstats)
+
+// The absolute sums of the gradients up to one that one workgroup adds, and the scales.
+struct SumArgs {
+  const double* g;
+  const double* h;
+  int64_t n;
+  int m;                // chunks of g and h to add; 0: the caller has their sums
+  double* first[2];     // [chunks] their sums
+  const double* of[2];  // what the last level adds,
+  int n_of;             // so many
+  double* scales;       // null: no sums are wanted
+  unsigned long long* qstats;
+};
+__device__ __forceinline__ void find_scales(const SumArgs& a, TwoSums& s)
 {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    const double max_int = 2147483647.0;
-    double sg = sum_a[0] == 0 ? 1 : max_int / sum_a[0];
-    double sh = sum_b[0] == 0 ? 1 : max_int / sum_b[0];
-    scales[0] = sg;
-    scales[1] = sh;
-    scales[2] = 1.0 / sg;
-    scales[3] = 1.0 / sh;
-    qstats[0] = 0;
-    qstats[1] = 0;
+  double sum_a, sum_b;
+  if (a.n_of > 1) {
+    sum_chunk<false>(a.of[0], a.of[1], a.n_of, 0, s);
+    sum_a = s.a[0], sum_b = s.b[0];
+  } else {
+    sum_a = a.of[0][0], sum_b = a.of[1][0];
   }
+  if (threadIdx.x == 0) {
+    const double max_int = 2147483647.0;
+    double sg = sum_a == 0 ? 1 : max_int / sum_a;
+    double sh = sum_b == 0 ? 1 : max_int / sum_b;
+    a.scales[0] = sg;
+    a.scales[1] = sh;
+    a.scales[2] = 1.0 / sg;
+    a.scales[3] = 1.0 / sh;
+    a.qstats[0] = 0;
+    a.qstats[1] = 0;
+  }
+}
+
+// A tree begins in two launches of workgroups that do one thing each. The first: the features' sorted samples, the first level of
+// the absolute sums, and n_init workgroups of the state. The second: the proposals' places, and (one more workgroup, where they are
+// wanted) the sums' last level and the scales. Apart they were eight launches, each a chain of few loads, up to the
+// rounding of the gradients 58 us of a tree of 1,000,000 x 50, now 27 (of the sort's 13 us 7 were one thread's sum of 256 counts).
+template <typename T>
+__global__ void __launch_bounds__(kThreads) tree_start_kernel(SampleArgs<T> a, SumArgs sums, InitArgs init)
+{
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ TwoSums s_sums;
+  __shared__ int s_waves[kThreads / 64];
+  int id = static_cast<int>(blockIdx.x);
+  // neighbouring features, whose samples share cache lines, on one XCD
+  const int per = (a.F + 7) / 8;
+  if (id < 8 * per) {
+    const int f = (id & 7) * per + (id >> 3);
+    if (f < a.F) unique_samples(a, f, reinterpret_cast<typename KeyOf<T>::type*>(smem_raw), s_waves);
+    return;
+  }
+  id -= 8 * per;
+  if (id < sums.m) {
+    sum_chunk<true>(sums.g, sums.h, sums.n, id, s_sums);
+    if (threadIdx.x == 0) {
+      sums.first[0][id] = s_sums.a[0];
+      sums.first[1][id] = s_sums.b[0];
+    }
+    return;
+  }
+  init.entry(static_cast<int64_t>(id - sums.m) * kThreads + threadIdx.x);
+}
+template <typename T>
+__global__ void __launch_bounds__(kThreads) tree_scales_kernel(SampleArgs<T> a, SumArgs sums)
+{
+  __shared__ TwoSums s_sums;
+  __shared__ int s_waves[kThreads / 64];
+  if (static_cast<int>(blockIdx.x) < a.F)
+    place_proposals(a, blockIdx.x, s_waves);
+  else
+    find_scales(sums, s_sums);
 }
 
 // Stochastic rounding of every (row, output) once per tree, stored as int32
@@ -429,22 +490,6 @@ __global__ void __launch_bounds__(kQuantiseThreads)
     if (s_bad != 0) atomicOr(&qstats[1], static_cast<unsigned long long>(s_bad));
   }
 }
-
-// build_tree.cu:1175-1185
-// host_stats: the two words of qstats for the host
-__global__ void root_leaf_kernel(double* leaf, const I64Pair* node_sums, int K,
-                                 const double* scales, double l1, double l2, const unsigned long long* qstats,
-                                 unsigned long long* host_stats)
-{
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < 2) __hip_atomic_store(host_stats + k, qstats[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  if (k < K) {
-    double G = static_cast<double>(node_sums[k].grad) * scales[2];
-    double H = static_cast<double>(node_sums[k].hess) * scales[3];
-    leaf[k]  = calculate_leaf_value(G, H, l1, l2);
-  }
-}
-
 
 // ---------------------------------------------------------------------------
 // scan + sibling subtraction (build_tree.cu:597-668), one wave per
@@ -1697,7 +1742,6 @@ struct Layout {
   double* scales;
   unsigned long long* qstats;
   // proposals
-  void* draft;
   void* uniq;
   int32_t* counts;
   void* proposals;
@@ -1778,7 +1822,6 @@ void make_layout(Arena& ar, Layout& L, int64_t N, int F, int K, int max_depth, i
   L.tainted      = ar.take<uint8_t>(max_nodes);
   L.scales       = ar.take<double>(4);
   L.qstats       = ar.take<unsigned long long>(2);
-  L.draft        = ar.take<char>(static_cast<size_t>(F) * S * elem);
   L.uniq         = ar.take<char>(static_cast<size_t>(F) * S * elem);
   L.counts       = ar.take<int32_t>(F);
   L.proposals    = ar.take<char>(static_cast<size_t>(F) * S * elem);
@@ -1961,58 +2004,50 @@ int host_mirror(int F, ThreadResources** out)
   return LBT_OK;
 }
 
-// SelectSplitSamples (build_tree.cu:867-964): gather, sort and unique per feature, row pointers,
-// compaction. draft and uniq hold F * S values of T each, counts F and bin_feature F * S ints.
+// SelectSplitSamples (build_tree.cu:867-964) and what the quantiser rounds with (build_tree.cu:51-140): the two absolute sums in a
+// fixed order, the scales. Without samples (F = 0) or without sums (sums.scales null) only the other one. first_level: the chunk
+// sums of |g| and |h| if the caller has them already ([2][chunks], see lbt_weighted_gradient_sums), else null.
+// part_a/part_b: two levels of partial sums.
 template <typename T>
-int run_split_samples(hipStream_t stream, const T* X, int64_t row_offset, int64_t N, int F, int S, int32_t seed,
-                      int64_t dataset_rows, T* draft, T* uniq, int32_t* counts, int32_t* row_pointers, T* proposals,
-                      int32_t* bin_feature, double* proposals_as_double = nullptr, int32_t* host_row_pointers = nullptr)
+int start_tree(hipStream_t stream, SampleArgs<T> samples, const InitArgs* init, const double* g, const double* h, int64_t n,
+               double* const (&part_a)[2], double* const (&part_b)[2], double* scales, unsigned long long* qstats,
+               const double* first_level)
 {
-  auto blocks = [](int64_t n, int t) { return static_cast<unsigned>((n + t - 1) / t); };
-  gather_samples_kernel<T><<<blocks(static_cast<int64_t>(F) * S, kThreads), kThreads, 0, stream>>>(
-    X, row_offset, N, F, S, seed, dataset_rows, draft);
-  int P = 1;
-  while (P < S) P <<= 1;
-  if (P < 2) P = 2;
-  sort_unique_kernel<T><<<F, kThreads, P * sizeof(typename KeyOf<T>::type), stream>>>(draft, S, P, uniq, counts);
-  row_pointers_kernel<<<1, kThreads, 0, stream>>>(counts, F, row_pointers, host_row_pointers);
-  compact_proposals_kernel<T><<<F, kThreads, 0, stream>>>(uniq, S, row_pointers, proposals, bin_feature,
-                                                          proposals_as_double);
+  samples.P = 2;
+  while (samples.P < samples.S) samples.P <<= 1;
+  int64_t m = (n + kSumChunk - 1) / kSumChunk;
+  SumArgs sums{};
+  if (scales != nullptr) {
+    sums = SumArgs{g, h, n, first_level != nullptr ? 0 : static_cast<int>(m), {part_a[0], part_b[0]}, {part_a[0], part_b[0]}, 0, scales, qstats};
+    if (first_level != nullptr) sums.of[0] = first_level, sums.of[1] = first_level + m;
+  }
+  const int64_t n_init = init == nullptr ? 0 : (std::max({init->max_nodes * init->K, init->n, init->n_slabs, static_cast<int64_t>(init->n_totals16)}) + kThreads - 1) / kThreads;
+  const int64_t grid   = (samples.F + 7) / 8 * 8 + sums.m + n_init;
+  if (grid > 0)
+    tree_start_kernel<T><<<static_cast<unsigned>(grid), kThreads, samples.F > 0 ? samples.P * sizeof(typename KeyOf<T>::type) : 0, stream>>>(
+      samples, sums, init != nullptr ? *init : InitArgs{});
+  int cur = 0;
+  if (scales != nullptr) {
+    for (; m > kSumChunk; m = (m + kSumChunk - 1) / kSumChunk) {
+      sum_level_kernel<<<static_cast<unsigned>((m + kSumChunk - 1) / kSumChunk), kThreads, 0, stream>>>(sums.of[0], sums.of[1], m, part_a[cur ^ 1],
+                                                                                                        part_b[cur ^ 1]);
+      cur ^= 1;
+      sums.of[0] = part_a[cur];
+      sums.of[1] = part_b[cur];
+    }
+    sums.n_of = static_cast<int>(m);
+  }
+  tree_scales_kernel<T><<<static_cast<unsigned>(samples.F + (scales != nullptr ? 1 : 0)), kThreads, 0, stream>>>(samples, sums);
   LBT_HIP(hipGetLastError());
   return LBT_OK;
 }
 
-// GradientQuantiser and reduce_base_sums (build_tree.cu:51-140, :168-204): the two absolute sums
-// in a fixed order, the scales, one rounding per (row, output), and the sums of the rounded pairs
-// added to root_sums[k] (which the caller has cleared). part_a/part_b: two levels of partial sums.
-// first_level: the chunk sums of |g| and |h| if the caller has them already ([2][chunks], see
-// lbt_weighted_gradient_sums), else null.
-int run_quantiser(hipStream_t stream, const double* g, const double* h, int64_t N, int K, int64_t row_offset,
-                  int32_t seed, double* const (&part_a)[2], double* const (&part_b)[2], double* scales,
-                  unsigned long long* qstats, int2* qgh, I64Pair* root_sums, const double* first_level = nullptr)
+// GradientQuantiser and reduce_base_sums (build_tree.cu:112-129, :168-204): one rounding per (row, output), and the sums of the
+// rounded pairs added to root_sums[k] (which the caller has cleared).
+int round_gradients(hipStream_t stream, const double* g, const double* h, int64_t N, int K, int64_t row_offset, int32_t seed,
+                    const double* scales, unsigned long long* qstats, int2* qgh, I64Pair* root_sums)
 {
   auto blocks = [](int64_t n, int t) { return static_cast<unsigned>((n + t - 1) / t); };
-  int64_t n = N * K;
-  int64_t m = (n + 4095) / 4096;
-  const double* in_a = part_a[0];
-  const double* in_b = part_b[0];
-  if (first_level != nullptr) {
-    in_a = first_level;
-    in_b = first_level + m;
-  } else {
-    abs_sum_level_kernel<true><<<static_cast<unsigned>(m), kThreads, 0, stream>>>(g, h, n, part_a[0], part_b[0]);
-  }
-  int cur = 0;
-  while (m > 1) {
-    int64_t m2 = (m + 4095) / 4096;
-    abs_sum_level_kernel<false><<<static_cast<unsigned>(m2), kThreads, 0, stream>>>(in_a, in_b, m, part_a[cur ^ 1],
-                                                                                     part_b[cur ^ 1]);
-    cur ^= 1;
-    in_a = part_a[cur];
-    in_b = part_b[cur];
-    m    = m2;
-  }
-  scales_kernel<<<1, 64, 0, stream>>>(in_a, in_b, scales, qstats);
   if (K > 1 && K <= kQuantiseFlatMaxK) {
     const unsigned gx = std::max<unsigned>(std::min<unsigned>(blocks(N * K, kQuantiseThreads), kQuantiseGroups), blocks(K, kQuantiseThreads));
     quantise_flat_kernel<<<gx, kQuantiseThreads, 2 * K * sizeof(unsigned long long), stream>>>(
@@ -2024,6 +2059,21 @@ int run_quantiser(hipStream_t stream, const double* g, const double* h, int64_t 
   }
   LBT_HIP(hipGetLastError());
   return LBT_OK;
+}
+
+// Both for the stages that want nothing else.
+int run_quantiser(hipStream_t stream, const double* g, const double* h, int64_t N, int K, int64_t row_offset,
+                  int32_t seed, double* const (&part_a)[2], double* const (&part_b)[2], double* scales,
+                  unsigned long long* qstats, int2* qgh, I64Pair* root_sums)
+{
+  LBT_TRY(start_tree<float>(stream, SampleArgs<float>{}, nullptr, g, h, N * K, part_a, part_b, scales, qstats, nullptr));
+  return round_gradients(stream, g, h, N, K, row_offset, seed, scales, qstats, qgh, root_sums);
+}
+template <typename T>
+int run_split_samples(hipStream_t stream, const SampleArgs<T>& samples)
+{
+  double* const none[2] = {nullptr, nullptr};
+  return start_tree<T>(stream, samples, nullptr, nullptr, nullptr, 0, none, none, nullptr, nullptr, nullptr);
 }
 
 // Hands the level counts of a build to the profiler: copied to the host in stream order.
@@ -2078,25 +2128,19 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
   const int S         = prm.split_samples;
   auto blocks = [](int64_t n, int t) { return static_cast<unsigned>((n + t - 1) / t); };
 
-  {
-    ProfScope ps(LBT_PROF_OTHER, stream);
-    static_assert(sizeof(LevelMeta) == 32, "LevelMeta is cleared in 16-byte units");
-    const int64_t n_slabs = (N + kPartBlock - 1) / kPartBlock;
-    const int64_t widest  = std::max<int64_t>(std::max<int64_t>(static_cast<int64_t>(max_nodes) * K, N), 2 * max_depth);
-    init_tree_kernel<<<blocks(std::max<int64_t>(widest, 1), kThreads), kThreads, 0, stream>>>(
-      leaf, feature, split, gain, L.node_sums, max_nodes, K, L.rows[0], N, L.seg[0], L.block_seg[0], n_slabs,
-      reinterpret_cast<uint4*>(L.level_totals), std::max(0, max_depth * 2), L.tainted);
-  }
-
-  // ---- split proposals
+  // ---- state, split proposals, scales
   ThreadResources* hm = nullptr;
   LBT_TRY(host_mirror(F, &hm));
   int32_t* const rp_here = hm->mirror + 4;
   {
     ProfScope ps(LBT_PROF_PROPOSALS, stream);
-    LBT_TRY(run_split_samples<T>(stream, X, row_offset, N, F, S, prm.seed, prm.dataset_rows, static_cast<T*>(L.draft),
-                                 static_cast<T*>(L.uniq), L.counts, L.row_pointers, static_cast<T*>(L.proposals),
-                                 L.bin_feature, L.proposals_d, F <= kMirrorFeatures ? rp_here : nullptr));
+    static_assert(sizeof(LevelMeta) == 32, "LevelMeta is cleared in 16-byte units");
+    const InitArgs init{leaf, feature, split, gain, L.node_sums, max_nodes, K, L.rows[0], N, L.seg[0], L.block_seg[0], (N + kPartBlock - 1) / kPartBlock,
+                        reinterpret_cast<uint4*>(L.level_totals), std::max(0, max_depth * 2), L.tainted};
+    LBT_TRY(start_tree<T>(stream,
+                          SampleArgs<T>{X, row_offset, N, prm.dataset_rows, F, S, 0, prm.seed, static_cast<T*>(L.uniq), L.counts, L.row_pointers,
+                                        static_cast<T*>(L.proposals), L.bin_feature, L.proposals_d, F <= kMirrorFeatures ? rp_here : nullptr},
+                          &init, g, h, N * K, L.part_a, L.part_b, L.scales, L.qstats, prm.abs_sum_chunks));
     if (F > kMirrorFeatures)
       LBT_HIP(hipMemcpyAsync(rp_here, L.row_pointers, sizeof(int32_t) * (F + 1), hipMemcpyDeviceToHost, stream));
     LBT_HIP(hipEventRecord(hm->counts_here, stream));
@@ -2104,14 +2148,9 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
   // ---- quantiser
   {
     ProfScope ps(LBT_PROF_QUANTISE, stream, static_cast<double>(N) * K * (16 + 16 + 8));
-    LBT_TRY(run_quantiser(stream, g, h, N, K, row_offset, prm.seed, L.part_a, L.part_b, L.scales, L.qstats, L.qgh,
-                          L.node_sums, prm.abs_sum_chunks));
-    root_leaf_kernel<<<blocks(K, 64), 64, 0, stream>>>(leaf, L.node_sums, K, L.scales,
-                                                       prm.l1_regularization, prm.l2_regularization, L.qstats,
-                                                       reinterpret_cast<unsigned long long*>(hm->mirror));
+    LBT_TRY(round_gradients(stream, g, h, N, K, row_offset, prm.seed, L.scales, L.qstats, L.qgh, L.node_sums));
   }
   const unsigned long long* const h_qstats = reinterpret_cast<const unsigned long long*>(hm->mirror);
-  LBT_HIP(hipEventRecord(hm->stats_here, stream));
   bool stats_checked = false;
   // a gradient that does not fit 32 bits ends the call; asked once a level's work is queued,
   // when the answer has long arrived
@@ -2161,8 +2200,6 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
   hs.partial_list_count = L.partial_list_count;
   hs.partial_count = L.partial_count;
   hs.partial_slots = kPartialSlots;
-  LBT_TRY(hist_prepare(stream, hs, sizeof(T) == 8, F, K, N, rp, L.proposals, L.row_pointers, X));
-
   const uint64_t max_bytes = prm.hist_cache_bytes > 0 ? static_cast<uint64_t>(prm.hist_cache_bytes) : 1000000000ULL;
   const uint64_t bytes_per_node = static_cast<uint64_t>(K) * B * 16ULL;
   uint64_t max_histogram_nodes  = std::max<uint64_t>(1, max_bytes / bytes_per_node);
@@ -2172,21 +2209,27 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
   // only nodes of levels < max_depth ever get a histogram
   const int64_t used_end = max_depth > 0 ? level_end(max_depth - 1) : 0;
   HistView hv{L.hist, 0, static_cast<int>(level_end(cdepth)), K, B, nullptr};
-  auto zero_hist = [&](int node_begin, int node_end) -> int {
-    int64_t hi    = std::min<int64_t>(node_end, used_end);
-    int64_t nodes = hi - node_begin;
-    if (nodes <= 0) return LBT_OK;
-    uint64_t bytes  = static_cast<uint64_t>(nodes) * bytes_per_node;
+  // histograms [node_begin, node_end): where they begin and their 16-byte units
+  auto hist_range = [&](int node_begin, int node_end, uint4** begin, int64_t* n16) -> int {
+    const int64_t nodes = std::max<int64_t>(std::min<int64_t>(node_end, used_end) - node_begin, 0);
+    const uint64_t bytes = static_cast<uint64_t>(nodes) * bytes_per_node;
     const uint64_t skip = static_cast<uint64_t>(node_begin - hv.node_begin) * bytes_per_node;
-    if (skip + bytes > L.hist_bytes) {
+    if (nodes > 0 && skip + bytes > L.hist_bytes) {
       set_error("histogram workspace too small (%llu > %llu)", (unsigned long long)bytes,
                 (unsigned long long)L.hist_bytes);
       return LBT_ERR_WORKSPACE;
     }
-    ProfScope ps(LBT_PROF_OTHER, stream, static_cast<double>(bytes));
-    int64_t n16 = static_cast<int64_t>(bytes / 16);
-    zero_kernel<<<static_cast<unsigned>(std::min<int64_t>((n16 + kThreads - 1) / kThreads, 65536)), kThreads, 0, stream>>>(
-      reinterpret_cast<uint4*>(reinterpret_cast<char*>(L.hist) + skip), n16);
+    *begin = reinterpret_cast<uint4*>(reinterpret_cast<char*>(L.hist) + skip);
+    *n16   = static_cast<int64_t>(bytes / 16);
+    return LBT_OK;
+  };
+  auto zero_hist = [&](int node_begin, int node_end) -> int {
+    uint4* begin = nullptr;
+    int64_t n16  = 0;
+    LBT_TRY(hist_range(node_begin, node_end, &begin, &n16));
+    if (n16 == 0) return LBT_OK;
+    ProfScope ps(LBT_PROF_OTHER, stream, 16.0 * static_cast<double>(n16));
+    zero_kernel<<<static_cast<unsigned>(std::min<int64_t>((n16 + kThreads - 1) / kThreads, 65536)), kThreads, 0, stream>>>(begin, n16);
     return LBT_OK;
   };
   // Where no entry's rounded hessian is negative (known after the root's launches are queued) the children of a split have
@@ -2216,7 +2259,10 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
       first++;
     cleared_end = std::min(hv.node_end, static_cast<int>(level_end(first)));
   }
-  LBT_TRY(zero_hist(hv.node_begin, cleared_end));
+  RootArgs root{leaf, L.node_sums, K, L.scales, prm.l1_regularization, prm.l2_regularization, L.qstats, reinterpret_cast<unsigned long long*>(hm->mirror), nullptr, 0};
+  LBT_TRY(hist_range(hv.node_begin, cleared_end, &root.clear, &root.n16));
+  LBT_TRY(hist_prepare(stream, hs, sizeof(T) == 8, F, K, N, rp, L.proposals, L.row_pointers, X, &root));
+  LBT_HIP(hipEventRecord(hm->stats_here, stream));
   //  - Single-output trees: levels whose histograms are larger than the rows' records keep them in the LDS
   //    (1,000,000 x 50 with 512 samples: level 11 743 -> 176 us, level 10 356 -> 108, level 9, the first with larger
   //    ones, 193 -> 92; with level 8, whose histograms are 0.8 of the records, a balanced tree would take 1.56 ms instead of
@@ -2535,14 +2581,12 @@ int build_tree_impl(hipStream_t stream, const T* X, int64_t row_offset, int64_t 
 namespace {
 
 struct SampleScratch {
-  char* draft;
   char* uniq;
   int32_t* counts;
   int32_t* bin_feature;
 };
 void make_sample_scratch(lbt::Arena& ar, SampleScratch& w, int F, int S, size_t elem)
 {
-  w.draft       = ar.take<char>(static_cast<size_t>(F) * S * elem);
   w.uniq        = ar.take<char>(static_cast<size_t>(F) * S * elem);
   w.counts      = ar.take<int32_t>(F);
   w.bin_feature = ar.take<int32_t>(static_cast<size_t>(F) * S);
@@ -2734,15 +2778,13 @@ int lbt_select_split_samples(void* stream, const void* X, int32_t x_dtype, int64
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   lbt::ProfScope ps(LBT_PROF_PROPOSALS, s);
-  if (x_dtype == LBT_F32)
-    return lbt::run_split_samples<float>(s, static_cast<const float*>(X), row_offset, n_rows, n_features, split_samples,
-                                         seed, dataset_rows, reinterpret_cast<float*>(w.draft),
-                                         reinterpret_cast<float*>(w.uniq), w.counts, row_pointers,
-                                         static_cast<float*>(proposals), w.bin_feature);
-  return lbt::run_split_samples<double>(s, static_cast<const double*>(X), row_offset, n_rows, n_features, split_samples,
-                                        seed, dataset_rows, reinterpret_cast<double*>(w.draft),
-                                        reinterpret_cast<double*>(w.uniq), w.counts, row_pointers,
-                                        static_cast<double*>(proposals), w.bin_feature);
+  auto run = [&](auto type) {
+    using T = decltype(type);
+    return lbt::run_split_samples<T>(s, lbt::SampleArgs<T>{static_cast<const T*>(X), row_offset, n_rows, dataset_rows, n_features, split_samples, 0, seed,
+                                                           reinterpret_cast<T*>(w.uniq), w.counts, row_pointers, static_cast<T*>(proposals), w.bin_feature,
+                                                           nullptr, nullptr});
+  };
+  return x_dtype == LBT_F32 ? run(float{}) : run(double{});
 }
 
 size_t lbt_quantise_gradients_workspace_bytes(int64_t n_rows, int32_t n_outputs)
@@ -2845,7 +2887,7 @@ int lbt_quantise_gradients_static(void* stream, const double* g, const double* h
   hipStream_t s = static_cast<hipStream_t>(stream);
   lbt::ProfScope ps(LBT_PROF_QUANTISE, s, static_cast<double>(n_rows) * n_outputs * (16 + 16 + 8));
   // Nothing of an earlier call's contents is read: every partial sum that is read was written
-  // by this call, and scales_kernel resets the statistics words. The root sums are cleared by a
+  // by this call, and find_scales resets the statistics words. The root sums are cleared by a
   // kernel (a memset node would not replay in a captured graph).
   lbt::zero_kernel<<<1, lbt::kThreads, 0, s>>>(reinterpret_cast<uint4*>(root_sums), n_outputs);
   return lbt::run_quantiser(s, g, h, n_rows, n_outputs, row_offset, seed, w.part_a, w.part_b, scales, w.qstats,

@@ -536,11 +536,24 @@ constexpr int kPlanThreads = 256;
 // What plans a batch below the root in a launch of the caller's; blocks: 0 where hist_launch has to do it.
 int hist_plan(const HistSetup& hs, const HistBatch& b, PlanArgs* plan);
 
+// What else begins with the tables: the root's outputs (build_tree.cu:1175-1185), the quantiser's two words for the host, and
+// histograms to clear.
+struct RootArgs {
+  double* leaf;
+  const I64Pair* node_sums;
+  int K;
+  const double* scales;
+  double l1, l2;
+  const unsigned long long* qstats;
+  unsigned long long* host_stats;
+  uint4* clear;
+  int64_t n16;
+};
 // Chooses groups / table size from the host copy of the row pointers and builds
-// the tables on the device.
+// the tables on the device. root: optional
 int hist_prepare(hipStream_t stream, HistSetup& hs, bool is_f64, int F, int K, int64_t n_rows,
                  const std::vector<int32_t>& rp, const void* proposals, const int32_t* row_pointers,
-                 const void* X);
+                 const void* X, const RootArgs* root = nullptr);
 // Plans tiles for the batch and launches the histogram kernel.
 int hist_launch(hipStream_t stream, const HistSetup& hs, const HistBatch& b, int depth);
 

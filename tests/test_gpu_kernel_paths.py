@@ -1009,3 +1009,19 @@ def test_scans_of_wide_levels(n, f, k, s, depth, kind):
     got = ops.build_tree(X, g, h, max_depth=depth, split_samples=s, seed=n, feature_set=mask, row_leaf=True, **kw2)
     _assert_tree(got, cr)
     gu.check_row_leaf(got, X)
+
+
+@pytest.mark.parametrize("n,f,k,s,dtype", [(1, 1, 1, 1, np.float32), (4096, 7, 1, 2, np.float64), (4097, 9, 1, 2048, np.float64), (1365, 8, 3, 257, np.float32),
+                                           (1366, 65, 3, 256, np.float32), (30000, 300, 1, 5, np.float32), (9000, 900, 2, 64, np.float32)])
+def test_a_tree_of_the_general_builder_begins_in_two_launches(n, f, k, s, dtype):
+    """Samples, chunks of the absolute sums (whole, one entry more) and the state side by side, few and many tables of the host: proposals,
+    rounded gradients and the tree are the oracle's."""
+    import gpu_util as gu
+
+    rs = np.random.RandomState(n + f)
+    X = np.round(rs.randn(n, f), 2).astype(dtype)
+    g, h = rs.randn(n, k), rs.rand(n, k) + 0.5
+    gr, cr = gu.both(X, g, h, levels=True, max_depth=3, split_samples=s, seed=n)
+    gu.assert_tree_parity(gr, cr, levels=True)
+    assert np.array_equal(gu.cpu(gr.row_pointers), cr.row_pointers) and np.array_equal(gu.cpu(gr.proposals), cr.proposals)
+    assert np.array_equal(gu.cpu(gr.quantised), cr.quantised)
