@@ -504,6 +504,15 @@ int lbt_add_leaf_values(void* stream, const double* leaf_value, int32_t n_nodes,
                         const int32_t* row_leaf, int64_t n_rows, int32_t n_outputs, double* pred);
 
 /*
+ * lbt_add_leaf_values and lbt_weighted_gradient at the predictions that it leaves, the same bits: the end of a round and the
+ * beginning of the next one (legateboost.py:260-275), one launch where the objective is formed element by element.
+ * abs_sum_chunks: as lbt_weighted_gradient_sums writes them, or null. pred and leaf_value may not alias any output.
+ */
+int lbt_next_gradient(void* stream, int32_t objective, const double* leaf_value, int32_t n_nodes, const int32_t* row_leaf,
+                      double* pred, const double* y, const double* sample_weight, double learning_rate, int64_t n_rows,
+                      int32_t n_outputs, double* g, double* h, double* abs_sum_chunks);
+
+/*
  * GatherTask::gpu_variant (src/utils/gather.cu:26-91), one GPU's share: row i of `out` is
  * global row sample_rows[i] of X if this shard holds it, else zeros (the reference then
  * sums the shards' outputs; with one shard that sum is the identity).

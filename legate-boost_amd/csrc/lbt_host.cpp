@@ -378,6 +378,47 @@ PyObject* add_leaf_values(PyObject*, PyObject* const* args, Py_ssize_t n_args)
   }
 }
 
+// next_gradient(pred, leaf_value, row_leaf, y, weight, g, h, sums, entry, stream, objective, learning_rate): lbt_next_gradient; weight: [rows] or
+// None, sums: [2][chunks] or None. Returns the status, or None as above.
+PyObject* next_gradient(PyObject*, PyObject* const* args, Py_ssize_t n_args)
+{
+  if (n_args != 12) {
+    PyErr_SetString(PyExc_TypeError, "next_gradient takes twelve arguments");
+    return nullptr;
+  }
+  int64_t v[3];
+  double rate;
+  if (!integers(args + 8, 3, v) || !numbers(args + 11, 1, &rate)) return nullptr;
+  try {
+    if (listened_to()) Py_RETURN_NONE;
+    const at::Tensor *pred = dense(args[0], at::kDouble, 2), *leaf = dense(args[1], at::kDouble, 2), *rows = dense(args[2], at::kInt, 1),
+                     *y = dense(args[3], at::kDouble, 2), *g = dense(args[5], at::kDouble, 2), *h = dense(args[6], at::kDouble, 2);
+    if (pred == nullptr || leaf == nullptr || rows == nullptr || y == nullptr || g == nullptr || h == nullptr) Py_RETURN_NONE;
+    const int64_t n = pred->size(0), k = pred->size(1);
+    for (const at::Tensor* t : {leaf, rows, y, g, h})
+      if (t->device() != pred->device()) Py_RETURN_NONE;
+    if (k > INT32_MAX || leaf->size(0) > INT32_MAX || leaf->size(1) != k || rows->size(0) != n || g->sizes() != pred->sizes() ||
+        h->sizes() != pred->sizes() || y->numel() != (v[2] == LBT_OBJ_LOG_LOSS && k > 1 ? n : n * k))
+      Py_RETURN_NONE;
+    const at::Tensor *w = nullptr, *sums = nullptr;
+    if (args[4] != Py_None) {
+      w = dense(args[4], at::kDouble, 1);
+      if (w == nullptr || w->numel() != n || w->device() != pred->device()) Py_RETURN_NONE;
+    }
+    if (args[7] != Py_None) {
+      sums = dense(args[7], at::kDouble, 2);
+      if (sums == nullptr || sums->numel() != 2 * ((n * k + 4095) / 4096) || sums->device() != pred->device()) Py_RETURN_NONE;
+    }
+    return PyLong_FromLong(reinterpret_cast<decltype(&lbt_next_gradient)>(v[0])(
+      reinterpret_cast<void*>(v[1]), static_cast<int32_t>(v[2]), leaf->const_data_ptr<double>(), static_cast<int32_t>(leaf->size(0)),
+      rows->const_data_ptr<int32_t>(), static_cast<double*>(pred->data_ptr()), y->const_data_ptr<double>(),
+      w != nullptr ? w->const_data_ptr<double>() : nullptr, rate, n, static_cast<int32_t>(k), g->mutable_data_ptr<double>(),
+      h->mutable_data_ptr<double>(), sums != nullptr ? sums->mutable_data_ptr<double>() : nullptr));
+  } catch (const std::exception&) {
+    Py_RETURN_NONE;
+  }
+}
+
 PyMethodDef methods[] = {{"tree_arrays", tree_arrays, METH_VARARGS, "addresses and node counts of an ensemble's arrays"},
                          {"model_arrays", model_arrays, METH_VARARGS, "the same from the attributes of an ensemble's models"},
                          {"predict_packed", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(predict_packed)), METH_FASTCALL,
@@ -387,6 +428,8 @@ PyMethodDef methods[] = {{"tree_arrays", tree_arrays, METH_VARARGS, "addresses a
                           "gradients and hessians of a round"},
                          {"add_leaf_values", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(add_leaf_values)), METH_FASTCALL,
                           "prediction update of a round"},
+                         {"next_gradient", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(next_gradient)), METH_FASTCALL,
+                          "prediction update of a round, gradients and hessians of the next one"},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -177,6 +177,9 @@ def _load():
     lib.lbt_weighted_gradient_sums.restype = C.c_int
     lib.lbt_weighted_gradient_sums.argtypes = [C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_double,
                                                C.c_int64, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p]
+    lib.lbt_next_gradient.restype = C.c_int
+    lib.lbt_next_gradient.argtypes = [C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
+                                      C.c_double, C.c_int64, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p]
     lib.lbt_add_leaf_values.restype = C.c_int
     lib.lbt_add_leaf_values.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_int64, C.c_int32,
                                         C.c_void_p]
@@ -249,7 +252,7 @@ EXPORTS = [
     "lbt_update_trees",
     "lbt_weighted_gradient", "lbt_weighted_gradient_sums", "lbt_class_probabilities",
     "lbt_weighted_mean_workspace_bytes", "lbt_weighted_mean", "lbt_label_counts", "lbt_label_priors", "lbt_keep_rows", "lbt_feature_mask",
-    "lbt_abs_sum_chunks", "lbt_add_leaf_values",
+    "lbt_abs_sum_chunks", "lbt_add_leaf_values", "lbt_next_gradient",
     "lbt_gather_rows", "lbt_select_split_samples_workspace_bytes", "lbt_select_split_samples",
     "lbt_quantise_gradients_workspace_bytes", "lbt_quantise_gradients", "lbt_quantise_gradients_static",
     "lbt_histogram_level_workspace_bytes", "lbt_histogram_level", "lbt_scan", "lbt_best_split_workspace_bytes",

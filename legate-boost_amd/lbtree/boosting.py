@@ -215,16 +215,33 @@ class LBBase:
         # workgroup's entries few of them: never (two rounds of depth 3, ms: 70,000 x 4 with 130 classes 2.88 and 2.66, 20,000 with 500
         # 8.4 and 5.1, 10,000 with 1000 14.9 and 8.8).
         fused = getattr(self._objective_instance, "fused", None)
-        sums = (fused is not None and self.subsample == 1.0 and train_pred.is_cuda
-                and train_pred.numel() >= (4000000 if train_pred.shape[1] == 1 else 8000000)
-                and (fused != "log_loss" or train_pred.shape[1] <= 128)
-                and _as_defined(self, LBBase, "_get_weighted_gradient"))
+        plain = (fused is not None and self.subsample == 1.0 and train_pred.is_cuda and train_pred.numel() > 0
+                 and _as_defined(self, LBBase, "_get_weighted_gradient"))
+        sums = (plain and train_pred.numel() >= (4000000 if train_pred.shape[1] == 1 else 8000000)
+                and (fused != "log_loss" or train_pred.shape[1] <= 128))
+
+        def own(model):
+            return isinstance(model, Tree) and _as_defined(model, Tree, "fit", "fit_update_predictions", "_fit")
+
+        at_hand = None  # the next round's gradients, formed where the last tree's values were added
         for i in range(self.n_estimators):
             model = _copy_of(self.base_models[i % len(self.base_models)]).set_random_state(self.random_state_)
-            if sums and isinstance(model, Tree) and _as_defined(model, Tree, "fit", "fit_update_predictions", "_fit"):
-                g, h, chunks = ops.weighted_gradient(fused, y, train_pred, w, self.learning_rate, sums=True)
-                model._fit(X, g, h, train_pred, chunks)
+            if plain and own(model):
+                if at_hand is None:
+                    at_hand = ops.weighted_gradient(fused, y, train_pred, w, self.learning_rate, sums=sums)
+                g, h = at_hand[:2]
+                chunks = at_hand[2] if sums else None
+
+                def next_round(pred, leaf_value, row_leaf):
+                    ops.next_gradient(fused, leaf_value, row_leaf, pred, y, w, self.learning_rate, g, h, chunks)
+
+                if i + 1 < self.n_estimators and own(self.base_models[(i + 1) % len(self.base_models)]):
+                    model._fit(X, g, h, train_pred, chunks, next_round)
+                else:
+                    at_hand = None
+                    model._fit(X, g, h, train_pred, chunks)
             else:
+                at_hand = None
                 g, h = self._get_weighted_gradient(y, train_pred, w, self.learning_rate)
                 if hasattr(model, "fit_update_predictions"):
                     model.fit_update_predictions(X, g, h, train_pred)

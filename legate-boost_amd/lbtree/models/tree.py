@@ -69,7 +69,7 @@ class Tree(BaseModel):
         pred (CUDA float64 [n_rows, n_outputs], updated in place) receives that leaf's value."""
         return self._fit(X, g, h, pred)
 
-    def _fit(self, X, g, h, pred, abs_sum_chunks=None) -> "Tree":
+    def _fit(self, X, g, h, pred, abs_sum_chunks=None, add_leaves=None) -> "Tree":
         X = ops.as_device(X)
         n_features = X.shape[1]
         # the seed is drawn before the feature sample, as in tree.py:125 / :139-157
@@ -94,7 +94,7 @@ class Tree(BaseModel):
             abs_sum_chunks=abs_sum_chunks,
         )
         if pred is not None:
-            ops.add_leaf_values(pred, r.leaf_value, r.row_leaf)
+            (add_leaves or ops.add_leaf_values)(pred, r.leaf_value, r.row_leaf)
         self.leaf_value = r.leaf_value
         self.feature = r.feature
         self.split_value = r.split_value

@@ -89,6 +89,7 @@ def _address(fn):
 _NATIVE = _lib._host if _lib._host is not None and _raw_stream is not None else None
 _BUILD, _BUILD_BYTES = _address(_lib.lib.lbt_build_tree_async), _address(_lib.lib.lbt_build_tree_workspace_bytes)
 _GRADIENT, _ADD_LEAVES = _address(_lib.lib.lbt_weighted_gradient), _address(_lib.lib.lbt_add_leaf_values)
+_NEXT_GRADIENT = _address(_lib.lib.lbt_next_gradient)
 
 
 def feature_mask(mask, device):
@@ -523,6 +524,19 @@ def add_leaf_values(pred, leaf_value, row_leaf):
                                       pred.data_ptr())
     _lib.check(rc)
     return pred
+
+
+def next_gradient(objective, leaf_value, row_leaf, pred, y, sample_weight, learning_rate, g, h, sums=None):
+    """add_leaf_values(pred, leaf_value, row_leaf), then weighted_gradient at the new pred into g and h, and into `sums` where
+    they are given: in one call, one launch unless the classes are several (legateboost/legateboost.py:260-275)."""
+    if _NATIVE is not None and torch.cuda.is_initialized():
+        rc = _NATIVE.next_gradient(pred, leaf_value, row_leaf, y, sample_weight, g, h, sums, _NEXT_GRADIENT,
+                                   _raw_stream(torch.cuda.current_device()), _OBJECTIVES[objective], learning_rate)
+        if rc is not None:
+            _lib.check(rc)
+            return
+    add_leaf_values(pred, leaf_value, row_leaf)
+    weighted_gradient(objective, y, pred, sample_weight, learning_rate, out=(g, h), sums=False if sums is None else sums)
 
 
 def gather_rows(X, samples, row_offset=0):

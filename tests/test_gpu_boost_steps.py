@@ -410,3 +410,83 @@ def test_a_plain_tree_is_copied_by_its_numbers():
     assert copied.note == [1] and copied.note is not listed.note
     assert type(boosting._copy_of(Own(max_depth=2))) is Own
 
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 256, 257, 4096, 4097, 70_000])
+@pytest.mark.parametrize("objective,k", [("squared_error", 1), ("squared_error", 3), ("log_loss", 1), ("log_loss", 4)])
+@pytest.mark.parametrize("weighted,sums,native", [(False, False, True), (True, True, True), (True, False, False)])
+def test_the_next_gradient_is_the_two_calls(n, objective, k, weighted, sums, native, monkeypatch):
+    """Leaf values and gradients in one call: the bits of lbt_add_leaf_values and lbt_weighted_gradient(_sums); a row of no leaf keeps its
+    prediction."""
+    from lbtree import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    double = dict(device="cuda", dtype=torch.float64, generator=gen)
+    pred, leaf = torch.randn((n, k), **double), torch.randn((31, k), **double)
+    rows = torch.randint(0, 31, (n,), device="cuda", dtype=torch.int32, generator=gen)
+    rows[n // 2] = -1 if n % 2 else 31
+    labels = objective == "log_loss" and k > 1
+    y = torch.randint(0, max(k, 2), (n, 1 if labels else k), device="cuda", generator=gen).double()
+    w = torch.rand(n, **double) if weighted else None
+    if not native:
+        monkeypatch.setattr(ops, "_NATIVE", None)
+    want = ops.add_leaf_values(pred.clone(), leaf, rows)
+    told = ops.weighted_gradient(objective, y, want, w, 0.3, sums=sums)
+    got, g, h = pred.clone(), torch.zeros_like(pred), torch.zeros_like(pred)
+    part = torch.zeros_like(told[2]) if sums else None
+    ops.next_gradient(objective, leaf, rows, got, y, w, 0.3, g, h, part)
+    assert torch.equal(got, want) and torch.equal(g, told[0]) and torch.equal(h, told[1])
+    assert not sums or torch.equal(part, told[2])
+    assert torch.equal(got[n // 2], pred[n // 2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("task", ["values", "two", "classes"])
+def test_rounds_in_one_pass_are_the_rounds_step_by_step(monkeypatch, task):
+    """Whose next gradients are formed with the prediction update, and whose are not: trees of another kind in between, a sample of the
+    rows, a method replaced."""
+    import lbtree as lb
+    from lbtree import boosting, ops
+
+    class OwnTree(lb.models.Tree):
+        def fit_update_predictions(self, X, g, h, pred):
+            return super().fit_update_predictions(X, g, h, pred)
+
+    X = torch.randn((3000, 6), generator=torch.Generator().manual_seed(3)).cuda()
+    y = {"values": X[:, 0] * 2 + X[:, 1], "two": (X[:, 0] > 0), "classes": (X[:, 0] * 2).round().clamp(0, 3)}[task].double()
+    estimator = lb.LBRegressor if task == "values" else lb.LBClassifier
+    calls = []
+    own_step = ops.next_gradient
+    monkeypatch.setattr(ops, "next_gradient", lambda *a, **kw: (calls.append(1), own_step(*a, **kw))[1])
+
+    def fit(own, **kw):
+        base = tuple((OwnTree if o else lb.models.Tree)(max_depth=4, split_samples=32) for o in own)
+        del calls[:]
+        m = estimator(n_estimators=5, base_models=base, random_state=4, **kw).fit(X, y)
+        return [t.leaf_value for t in m] + [m._train_pred], len(calls)
+
+    want, n = fit([True])
+    assert n == 0
+    for own, expected in (([False], 4), ([False, True], 0), ([False, False, True], 2)):
+        got, n = fit(own)
+        assert n == expected
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert fit([False], subsample=0.5)[1] == 0
+    monkeypatch.setattr(boosting.LBBase, "_get_weighted_gradient", lambda *a: boosting._DEFINED[boosting.LBBase]["_get_weighted_gradient"](*a))
+    got, n = fit([False])
+    assert n == 0 and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_the_next_gradient_checks_its_arguments():
+    from lbtree import _lib
+
+    call, one, two, three, four = _lib.lib.lbt_next_gradient, *(C.c_void_p(v) for v in (1 << 20, 2 << 20, 3 << 20, 4 << 20))
+    assert call(None, 7, one, 3, one, two, one, None, 0.1, 10, 1, three, four, None) == -1
+    assert call(None, 0, None, 3, one, two, one, None, 0.1, 10, 1, three, four, None) == -1
+    assert call(None, 0, one, 0, one, two, one, None, 0.1, 10, 1, three, four, None) == -1
+    assert call(None, 0, two, 3, one, two, one, None, 0.1, 10, 1, three, four, None) == -1
+    assert call(None, 0, one, 3, one, two, one, None, 0.1, 10, 1, two, four, None) == -1
+    assert call(None, 0, one, 3, one, two, one, None, 0.1, 10, 1, three, four, C.c_void_p(3 << 20)) == -1
+    assert call(None, 0, None, 3, None, None, None, None, 0.1, 0, 1, None, None, None) == 0
+    assert _lib.lib.lbt_feature_mask(None, None, 3, one) == -1 and _lib.lib.lbt_feature_mask(None, one, 3, None) == -1
