@@ -1025,3 +1025,34 @@ def test_a_tree_of_the_general_builder_begins_in_two_launches(n, f, k, s, dtype)
     gu.assert_tree_parity(gr, cr, levels=True)
     assert np.array_equal(gu.cpu(gr.row_pointers), cr.row_pointers) and np.array_equal(gu.cpu(gr.proposals), cr.proposals)
     assert np.array_equal(gu.cpu(gr.quantised), cr.quantised)
+
+
+@pytest.mark.parametrize("s", [1, 2, 7, 8, 9, 33, 63, 64, 65, 128, 255, 256, 257, 511, 512, 513, 1025])
+@pytest.mark.parametrize("n,dtype", [(700, np.float32), (900, np.float64), (9001, np.float32), (9001, np.float64)])
+def test_samples_sorted_by_counting(n, dtype, s):
+    """Split proposals of the builders for few and for medium rows, of columns with ties, zeros of either sign, NaN, infinities, one value: the tree is the
+    general builder's, whose proposals a network sorts."""
+    from lbtree import ops
+
+    rs = np.random.RandomState(s + n)
+    X = np.empty((n, 9), dtype)
+    X[:, 0] = rs.randn(n)
+    X[:, 1] = rs.randint(-2, 3, n)
+    X[:, 2] = np.where(rs.rand(n) < 0.5, 0.0, -0.0) * 1.0
+    X[:, 3] = np.where(rs.rand(n) < 0.3, -0.0, rs.randn(n))
+    X[:, 4] = np.where(rs.rand(n) < 0.3, 0.0, rs.randn(n))
+    X[:, 5] = 3.0
+    X[:, 6] = np.where(rs.rand(n) < 0.1, np.inf, np.where(rs.rand(n) < 0.1, -np.inf, rs.randn(n)))
+    X[:, 7] = rs.randint(0, 300, n)
+    X[:, 8] = np.where(rs.rand(n) < 0.2, np.nan, np.round(rs.randn(n)))
+    if s > 1:
+        X[:, 1] = np.where(rs.rand(n) < 0.5, -X[:, 1], X[:, 1])
+    g, h = rs.randn(n, 1) + np.nan_to_num(X[:, :1]) + (X[:, 7:8] > 150) * X[:, 1:2], rs.rand(n, 1) + 0.1
+    Xd, gd, hd = (torch.from_numpy(a).cuda() for a in (X, g, h))
+    mask = torch.ones(9, dtype=torch.bool)
+    mask[8] = False  # (no split on the column with NaN: a traversal sends it to the right)
+    kw = dict(max_depth=4, split_samples=s, seed=s, feature_set=mask)
+    want = ops.build_tree(Xd, gd, hd, taps=True, **kw)
+    got = ops.build_tree(Xd, gd, hd, **kw)
+    for name in ("feature", "split_value", "gain", "leaf_value", "hessian"):
+        assert torch.equal(getattr(got, name), getattr(want, name)), name
