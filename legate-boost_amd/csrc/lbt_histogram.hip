@@ -187,6 +187,7 @@ __global__ void __launch_bounds__(256)
 {
   __shared__ T s_p[LBT_MAX_SPLIT_SAMPLES];
   __shared__ int s_crowded[kCellMaps];
+  __shared__ CellMap<T> s_map[kCellMaps];
   __shared__ CellScratch s_cells;
   const int f = blockIdx.x;
   if (f == F) {
@@ -218,14 +219,14 @@ __global__ void __launch_bounds__(256)
   const float cmax = static_cast<float>(C - 1);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int c = wave; c < kCellMaps; c += 4) {
-    const int crowded = crowded_proposals(c, p, n, C, lane);
+    const int crowded = crowded_proposals(c, p, n, C, lane, &s_map[c]);
     if (lane == 0) s_crowded[c] = crowded;
   }
   __syncthreads();
   int best = 0;
   for (int c = 1; c < kCellMaps; c++)
     if (s_crowded[c] < s_crowded[best]) best = c;
-  const CellMap<T> m = cell_map_candidate(best, p, n, static_cast<float>(C));
+  const CellMap<T> m = s_map[best];
   const int entries  = C / kCellsPerEntry;
   write_cell_entries(p, n, entries, s_cells, tables + static_cast<int64_t>(f) * entries,
                      [&](T x) { return cell_of(x, m.scale, m.shift, m.invw, m.nlo, cmax); });

@@ -71,7 +71,7 @@ struct MidArgs {
   uint32_t tag;
 };
 
-// Fixed-order sum of one chunk of up to 4096 entries by 256 threads (see abs_sum_level_kernel): every thread
+// Fixed-order sum of one chunk of up to 4096 entries by 256 threads (see sum_chunk in lbt_build_tree.hip): every thread
 // of the workgroup calls it, thread t of each quarter with its own chunk. s_a, s_b: [kWide].
 template <bool kAbs>
 __device__ __forceinline__ void quarter_sums(const double* __restrict__ a, const double* __restrict__ b, int64_t first,
@@ -122,19 +122,20 @@ __global__ void __launch_bounds__(kWide)
     if (tid == 0) st.counts[block] = n;
     // the cell function and table of the bin search (see build_cells_kernel), a candidate per wave
     __shared__ int s_crowded[kCellMaps];
+    __shared__ CellMap<T> s_map[kCellMaps];
     static_assert(kCellMaps <= kWide / 64, "one wave per candidate");
     T* const p = const_cast<T*>(s_prop);
     if (tid == 0) p[n - 1] = std::numeric_limits<T>::infinity();
     __syncthreads();
     if ((tid >> 6) < kCellMaps) {
-      const int crowded = crowded_proposals(tid >> 6, p, n, st.cells, tid & 63);
+      const int crowded = crowded_proposals(tid >> 6, p, n, st.cells, tid & 63, &s_map[tid >> 6]);
       if ((tid & 63) == 0) s_crowded[tid >> 6] = crowded;
     }
     __syncthreads();
     int best = 0;
     for (int c = 1; c < kCellMaps; c++)
       if (s_crowded[c] < s_crowded[best]) best = c;
-    const CellMap<T> m = cell_map_candidate(best, p, n, static_cast<float>(st.cells));
+    const CellMap<T> m = s_map[best];
     const float cmax   = static_cast<float>(st.cells - 1);
     const int entries  = st.cells / kCellsPerEntry;
     __shared__ CellScratch s_cells;

@@ -60,8 +60,8 @@ struct PrologueArgs {
   uint32_t tag;
 };
 
-// Quantiser, root sums and root outputs: the arithmetic and the order of sums of abs_sum_level_kernel,
-// scales_kernel and quantise_kernel (lbt_build_tree.hip), for at most kQuantChunks chunks.
+// Quantiser, root sums and root outputs: the arithmetic and the order of sums of sum_chunk,
+// find_scales and quantise_kernel (lbt_build_tree.hip), for at most kQuantChunks chunks.
 __device__ inline void small_quantise(const PrologueArgs& a, const SmallTreeState& st, unsigned char* smem)
 {
   double* s_a = reinterpret_cast<double*>(smem);           // [4][256]
