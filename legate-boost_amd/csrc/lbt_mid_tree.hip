@@ -935,8 +935,9 @@ __global__ void __launch_bounds__(kScan)
 // depend on the bin once an output instead of once a thread. Below the root, where nobody asks for the smaller child, and from kWavePairs on:
 // with fewer the waves of a workgroup, which take the bins of a feature at a time, finish sooner than one that takes them in turn (50,000 x 200,
 // 256 samples, levels of 1600, 3200, 6400 and 12,800 pairs and features: 8.8, 12.2, 18.0 and 27.7 us, by workgroups with 16 bytes a bin 13.6, 19.4,
-// 33.1 and 61.2; 512 and 2048 as the bound give the same trees' times within 1 %). A tree of 50,000 x 200, depth 8: 353 us, now 297; of 20,000 x 60, 128 samples, depth 10,
-// 351 and 306; of 50,000 x 100 with 2 outputs, 64 samples, depth 9, 405 and 319.
+// 33.1 and 61.2. As the bound 512 gives scans of 90 us a tree for 85 with 30,000 x 60 and 8 outputs, 98 for 103 with 50,000 x 100 and 2, 2048 86
+// and 111.) A tree of 50,000 x 200, depth 8: 353 us, now 297; of 20,000 x 60, 128 samples, depth 10, 351 and 306; of 50,000 x 100 with 2 outputs, 64
+// samples, depth 9, 405 and 319.
 template <bool kLast>
 __global__ void __launch_bounds__(kScan)
   mid_scan_waves_kernel(MidArgs a, MidTreeState st, LevelPlan p)
