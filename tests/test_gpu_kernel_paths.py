@@ -1056,3 +1056,31 @@ def test_samples_sorted_by_counting(n, dtype, s):
     got = ops.build_tree(Xd, gd, hd, **kw)
     for name in ("feature", "split_value", "gain", "leaf_value", "hessian"):
         assert torch.equal(getattr(got, name), getattr(want, name)), name
+
+
+@pytest.mark.parametrize("n", [1, 4096, 4097, 4096 * 4096, 4096 * 4096 + 1])
+def test_scales_of_the_absolute_sums(n):
+    """One, two and three levels of the fixed-order sum of |g| and |h|: the scales have the bits of the same additions on the host."""
+    from lbtree import ops
+
+    def level(a):
+        chunks = -(-len(a) // 4096)
+        a = np.concatenate([a, np.zeros(chunks * 4096 - len(a))]).reshape(chunks, 16, 256)
+        lanes = np.zeros((chunks, 256))
+        for j in range(16):  # a lane's entries in their order (one that is missing adds zero)
+            lanes = lanes + a[:, j]
+        while lanes.shape[1] > 1:
+            half = lanes.shape[1] // 2
+            lanes = lanes[:, :half] + lanes[:, half:]
+        return lanes[:, 0]
+
+    gen = torch.Generator(device="cuda").manual_seed(n % 1000)
+    g = torch.randn((n, 1), generator=gen, device="cuda", dtype=torch.float64)
+    h = torch.rand((n, 1), generator=gen, device="cuda", dtype=torch.float64)
+    q, sums, scales = ops.quantise_gradients(g, h, 3)
+    for at, a in ((0, g), (1, h)):
+        s = level(np.abs(a.cpu().numpy().reshape(-1)))
+        while len(s) > 1:
+            s = level(s)
+        assert scales[at].item() == 2147483647.0 / s[0] and scales[2 + at].item() == 1.0 / scales[at].item()
+    assert torch.equal(sums, q.to(torch.int64).sum(dim=0))
