@@ -152,6 +152,20 @@ PyObject* model_arrays(PyObject*, PyObject* args)
   return result;
 }
 
+// The library's entries run with Python's lock given back. An exception that leaves one (it has vectors of its own) takes the lock again on
+// its way to the handler, which gives references back and looks at Python's error. (Python ends a thread that asks for the
+// lock while it shuts down by unwinding it, hence noexcept(false).)
+struct Unlocked {
+  PyThreadState* const state = PyEval_SaveThread();
+  ~Unlocked() noexcept(false) { PyEval_RestoreThread(state); }
+};
+template <typename Call>
+int unlocked(Call call)
+{
+  const Unlocked free;
+  return call();
+}
+
 // predict_packed(X, entry, stream, ensemble, dtype, n_outputs): lbt_predict_packed, whose address is `entry`, on a dense float (dtype 0) or
 // double (1) matrix on the device. Returns the predictions, or the status where that is not 0, or None where X is something else or torch is
 // being listened to: the caller then goes through Python.
@@ -178,11 +192,11 @@ PyObject* predict_packed(PyObject*, PyObject* const* args, Py_ssize_t n_args)
     const auto entry = reinterpret_cast<PredictPacked>(number[0]);
     const void* from = x.const_data_ptr();
     double* const to = out.mutable_data_ptr<double>();
-    int status       = 0;
-    Py_BEGIN_ALLOW_THREADS
-    status = entry(reinterpret_cast<void*>(number[1]), from, static_cast<int32_t>(number[3]), x.size(0), static_cast<int32_t>(x.size(1)),
+    const int64_t n = x.size(0), f = x.size(1);
+    const int status = unlocked([&] {
+      return entry(reinterpret_cast<void*>(number[1]), from, static_cast<int32_t>(number[3]), n, static_cast<int32_t>(f),
                    reinterpret_cast<const void*>(number[2]), to);
-    Py_END_ALLOW_THREADS
+    });
     if (status != 0) return PyLong_FromLong(status);
     return THPVariable_Wrap(std::move(out));
   } catch (const std::exception&) {
@@ -298,11 +312,10 @@ PyObject* build_tree(PyObject*, PyObject* const* args, Py_ssize_t n_args)
     double* const to_hessian = hessian.mutable_data_ptr<double>();
     void* const room = ws->data_ptr();
     const size_t has = static_cast<size_t>(ws->numel());
-    int status       = 0;
-    Py_BEGIN_ALLOW_THREADS
-    status = reinterpret_cast<BuildTree>(v[0])(reinterpret_cast<void*>(v[2]), from, type, row_offset, n, f, grad, hess, k, allowed, &prm, to_leaf,
+    const int status = unlocked([&] {
+      return reinterpret_cast<BuildTree>(v[0])(reinterpret_cast<void*>(v[2]), from, type, row_offset, n, f, grad, hess, k, allowed, &prm, to_leaf,
                                                to_feature, to_split, to_gain, to_hessian, room, has, row_leaf ? &taps : nullptr);
-    Py_END_ALLOW_THREADS
+    });
     if (status != 0) return PyLong_FromLong(status);
     PyObject* out = PyTuple_New(6);
     if (out == nullptr) return nullptr;

@@ -209,3 +209,37 @@ def test_models_of_which_the_first_is_no_tree_are_refused():
         Tree.batch_predict([Other()], torch.zeros(2, 2))
     with pytest.raises(IndexError):
         Tree.batch_predict([], torch.zeros(2, 2))
+
+
+# ---------------------------------------------------------------- calls of the library from native code
+
+
+def _native_calls(entry, first):
+    """The calls of lbtree._host that enter the library, with another entry and another first argument (a stream's address)."""
+    import ctypes as C
+
+    n, k = 10, 1
+    double = dict(device="cuda", dtype=torch.float64)
+    X, g, h, y, pred = torch.zeros((n, 2), device="cuda"), *(torch.ones((n, k), **double) for _ in range(4))
+    rows, leaf = torch.zeros(n, dtype=torch.int32, device="cuda"), torch.zeros((3, k), **double)
+    address, host = C.cast(entry, C.c_void_p).value, _lib._host
+    return {
+        "predict_packed": lambda: host.predict_packed(X, address, first, 0, 0, k),
+        "build_tree": lambda: host.build_tree(X, g, h, None, ops._get_workspace, address, ops._BUILD_BYTES, first, 0, 2, 4, 1, 0, 1, 0.0, 1.0, 0.0),
+        "weighted_gradient": lambda: host.weighted_gradient(y, pred, None, address, first, 0, 0.1),
+        "add_leaf_values": lambda: host.add_leaf_values(pred, leaf, rows, address, first),
+        "next_gradient": lambda: host.next_gradient(pred, leaf, rows, y, None, g, h, None, address, first, 0, 0.1),
+    }
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["predict_packed", "build_tree", "weighted_gradient", "add_leaf_values", "next_gradient"])
+def test_an_exception_of_the_library_comes_back_with_the_lock_held(name):
+    """An entry that throws (std::bad_alloc): None, the caller's way through Python, and an interpreter that goes on."""
+    import ctypes as C
+
+    thrower = C.CDLL("libstdc++.so.6")._ZSt17__throw_bad_allocv
+    call = _native_calls(thrower, 0)[name]
+    for _ in range(3):
+        assert call() is None
+    assert C.pythonapi.PyGILState_Check() == 1
