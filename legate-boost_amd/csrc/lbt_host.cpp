@@ -354,9 +354,13 @@ PyObject* weighted_gradient(PyObject*, PyObject* const* args, Py_ssize_t n_args)
     }
     const auto real = pred->options().requires_grad(false);
     at::Tensor g = at::empty({n, k}, real), h = at::empty({n, k}, real);
-    const int status = reinterpret_cast<decltype(&lbt_weighted_gradient)>(v[0])(
-      reinterpret_cast<void*>(v[1]), static_cast<int32_t>(v[2]), pred->const_data_ptr<double>(), y->const_data_ptr<double>(),
-      w != nullptr ? w->const_data_ptr<double>() : nullptr, rate, n, static_cast<int32_t>(k), g.mutable_data_ptr<double>(), h.mutable_data_ptr<double>());
+    const double *const at = pred->const_data_ptr<double>(), *const target = y->const_data_ptr<double>();
+    const double* const weight = w != nullptr ? w->const_data_ptr<double>() : nullptr;
+    double *const to_g = g.mutable_data_ptr<double>(), *const to_h = h.mutable_data_ptr<double>();
+    const int status = unlocked([&] {
+      return reinterpret_cast<decltype(&lbt_weighted_gradient)>(v[0])(reinterpret_cast<void*>(v[1]), static_cast<int32_t>(v[2]), at, target, weight,
+                                                                      rate, n, static_cast<int32_t>(k), to_g, to_h);
+    });
     if (status != 0) return PyLong_FromLong(status);
     PyObject* out = PyTuple_New(2);
     if (out == nullptr) return nullptr;
@@ -383,9 +387,15 @@ PyObject* add_leaf_values(PyObject*, PyObject* const* args, Py_ssize_t n_args)
     if (pred == nullptr || leaf == nullptr || rows == nullptr || leaf->size(1) != pred->size(1) || rows->size(0) != pred->size(0) ||
         leaf->device() != pred->device() || rows->device() != pred->device() || pred->size(1) > INT32_MAX || leaf->size(0) > INT32_MAX)
       Py_RETURN_NONE;
-    return PyLong_FromLong(reinterpret_cast<decltype(&lbt_add_leaf_values)>(v[0])(
-      reinterpret_cast<void*>(v[1]), leaf->const_data_ptr<double>(), static_cast<int32_t>(leaf->size(0)), rows->const_data_ptr<int32_t>(),
-      pred->size(0), static_cast<int32_t>(pred->size(1)), static_cast<double*>(pred->data_ptr())));
+    const double* const from   = leaf->const_data_ptr<double>();
+    const int32_t* const nodes = rows->const_data_ptr<int32_t>();
+    double* const to           = static_cast<double*>(pred->data_ptr());
+    const int64_t n = pred->size(0), k = pred->size(1), n_nodes = leaf->size(0);
+    const int status = unlocked([&] {
+      return reinterpret_cast<decltype(&lbt_add_leaf_values)>(v[0])(reinterpret_cast<void*>(v[1]), from, static_cast<int32_t>(n_nodes), nodes, n,
+                                                                    static_cast<int32_t>(k), to);
+    });
+    return PyLong_FromLong(status);
   } catch (const std::exception&) {
     Py_RETURN_NONE;
   }
@@ -422,11 +432,18 @@ PyObject* next_gradient(PyObject*, PyObject* const* args, Py_ssize_t n_args)
       sums = dense(args[7], at::kDouble, 2);
       if (sums == nullptr || sums->numel() != 2 * ((n * k + 4095) / 4096) || sums->device() != pred->device()) Py_RETURN_NONE;
     }
-    return PyLong_FromLong(reinterpret_cast<decltype(&lbt_next_gradient)>(v[0])(
-      reinterpret_cast<void*>(v[1]), static_cast<int32_t>(v[2]), leaf->const_data_ptr<double>(), static_cast<int32_t>(leaf->size(0)),
-      rows->const_data_ptr<int32_t>(), static_cast<double*>(pred->data_ptr()), y->const_data_ptr<double>(),
-      w != nullptr ? w->const_data_ptr<double>() : nullptr, rate, n, static_cast<int32_t>(k), g->mutable_data_ptr<double>(),
-      h->mutable_data_ptr<double>(), sums != nullptr ? sums->mutable_data_ptr<double>() : nullptr));
+    const double *const from = leaf->const_data_ptr<double>(), *const target = y->const_data_ptr<double>();
+    const double* const weight = w != nullptr ? w->const_data_ptr<double>() : nullptr;
+    const int32_t* const nodes = rows->const_data_ptr<int32_t>();
+    double *const at = static_cast<double*>(pred->data_ptr()), *const to_g = g->mutable_data_ptr<double>(), *const to_h = h->mutable_data_ptr<double>();
+    double* const to_sums = sums != nullptr ? sums->mutable_data_ptr<double>() : nullptr;
+    const int64_t n_nodes = leaf->size(0);
+    const int status      = unlocked([&] {
+      return reinterpret_cast<decltype(&lbt_next_gradient)>(v[0])(reinterpret_cast<void*>(v[1]), static_cast<int32_t>(v[2]), from,
+                                                                  static_cast<int32_t>(n_nodes), nodes, at, target, weight, rate, n,
+                                                                  static_cast<int32_t>(k), to_g, to_h, to_sums);
+    });
+    return PyLong_FromLong(status);
   } catch (const std::exception&) {
     Py_RETURN_NONE;
   }

@@ -243,3 +243,30 @@ def test_an_exception_of_the_library_comes_back_with_the_lock_held(name):
     for _ in range(3):
         assert call() is None
     assert C.pythonapi.PyGILState_Check() == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["predict_packed", "build_tree", "weighted_gradient", "add_leaf_values", "next_gradient"])
+def test_other_threads_run_while_the_library_is_called(name):
+    """An entry that sleeps for 0.3 s (a launch waits like that while the stream's queue is full): another thread takes its turns."""
+    import ctypes as C
+    import threading
+    import time
+
+    call = _native_calls(C.CDLL("libc.so.6").usleep, 300000)[name]
+    turns, ended = [0], threading.Event()
+
+    def count():
+        while not ended.wait(0.002):
+            turns[0] += 1
+
+    other = threading.Thread(target=count)
+    other.start()
+    try:
+        before = turns[0]
+        call()
+        while_it_slept = turns[0] - before
+    finally:
+        ended.set()
+        other.join()
+    assert while_it_slept >= 10  # with the lock held none or one
