@@ -233,6 +233,15 @@ bool numbers(PyObject* const* args, int n, double* out)
   return true;
 }
 
+// After a number that is none: the caller meets it again in Python, which says what is wrong as it always did; what is no Exception (an
+// interrupt) is passed on.
+PyObject* not_a_number()
+{
+  if (!PyErr_ExceptionMatches(PyExc_Exception)) return nullptr;
+  PyErr_Clear();
+  Py_RETURN_NONE;
+}
+
 // build_tree(X, g, h, mask, workspace, entry, size_entry, stream, row_offset, max_depth, split_samples, seed, cache, row_leaf, l1, l2, gain):
 // lbt_build_tree_async and lbt_build_tree_workspace_bytes, whose addresses are `entry` and `size_entry`, for a float or double matrix and gradients as they
 // have to be on the device; mask: a uint8 tensor there or None; workspace(bytes, device): the scratch tensor. Returns (leaf_value, feature,
@@ -248,11 +257,7 @@ PyObject* build_tree(PyObject*, PyObject* const* args, Py_ssize_t n_args)
   }
   int64_t v[9];
   double r[3];
-  if (!integers(args + 5, 9, v) || !numbers(args + 14, 3, r)) {
-    if (!PyErr_ExceptionMatches(PyExc_Exception)) return nullptr;
-    PyErr_Clear();
-    Py_RETURN_NONE;
-  }
+  if (!integers(args + 5, 9, v) || !numbers(args + 14, 3, r)) return not_a_number();
   const int64_t row_offset = v[3], max_depth = v[4], samples = v[5], seed = v[6], cache = v[7];
   const bool row_leaf = v[8] != 0;
   try {
@@ -340,7 +345,7 @@ PyObject* weighted_gradient(PyObject*, PyObject* const* args, Py_ssize_t n_args)
   }
   int64_t v[3];
   double rate;
-  if (!integers(args + 3, 3, v) || !numbers(args + 6, 1, &rate)) return nullptr;
+  if (!integers(args + 3, 3, v) || !numbers(args + 6, 1, &rate)) return not_a_number();
   try {
     if (listened_to()) Py_RETURN_NONE;
     const at::Tensor *y = dense(args[0], at::kDouble, 2), *pred = dense(args[1], at::kDouble, 2);
@@ -380,7 +385,7 @@ PyObject* add_leaf_values(PyObject*, PyObject* const* args, Py_ssize_t n_args)
     return nullptr;
   }
   int64_t v[2];
-  if (!integers(args + 3, 2, v)) return nullptr;
+  if (!integers(args + 3, 2, v)) return not_a_number();
   try {
     if (listened_to()) Py_RETURN_NONE;
     const at::Tensor *pred = dense(args[0], at::kDouble, 2), *leaf = dense(args[1], at::kDouble, 2), *rows = dense(args[2], at::kInt, 1);
@@ -411,7 +416,7 @@ PyObject* next_gradient(PyObject*, PyObject* const* args, Py_ssize_t n_args)
   }
   int64_t v[3];
   double rate;
-  if (!integers(args + 8, 3, v) || !numbers(args + 11, 1, &rate)) return nullptr;
+  if (!integers(args + 8, 3, v) || !numbers(args + 11, 1, &rate)) return not_a_number();
   try {
     if (listened_to()) Py_RETURN_NONE;
     const at::Tensor *pred = dense(args[0], at::kDouble, 2), *leaf = dense(args[1], at::kDouble, 2), *rows = dense(args[2], at::kInt, 1),

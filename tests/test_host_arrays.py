@@ -270,3 +270,27 @@ def test_other_threads_run_while_the_library_is_called(name):
         ended.set()
         other.join()
     assert while_it_slept >= 10  # with the lock held none or one
+
+
+def test_numbers_that_are_none_are_left_to_the_caller():
+    """A learning rate of another type: no error of the native call's own (the Python form says what is wrong with it)."""
+    t = torch.zeros(2, 1, dtype=torch.float64)
+    for rate in ("0.1", None, 10 ** 400, [1]):
+        assert _lib._host.weighted_gradient(t, t, None, 0, 0, 0, rate) is None
+        assert _lib._host.next_gradient(t, t, t, t, None, t, t, None, 0, 0, 0, rate) is None
+    assert _lib._host.add_leaf_values(t, t, t, 0, "0") is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rate,taken", [("0.1", True), (np.float32(0.1), True), (None, False), (10 ** 400, False)])
+def test_a_learning_rate_is_taken_or_refused_as_in_python(monkeypatch, rate, taken):
+    y, pred = (torch.rand((4, 1), dtype=torch.float64, device="cuda") for _ in range(2))
+    said = []
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(ops, "_NATIVE", None)
+        try:
+            said.append(ops.weighted_gradient("squared_error", y, pred, None, rate)[0].tolist())
+        except Exception as e:
+            said.append((type(e), str(e)))
+    assert said[0] == said[1] and isinstance(said[0], list) == taken
