@@ -231,17 +231,21 @@ def _load():
 
 lib = _load()
 
-# The ensemble calls look their trees over in native code where it is built for the torch at hand, else in Python (ops.py):
-# the same results, 1.4 us a tree later.
+# The ensemble calls look their trees over in native code, and a round of boosting makes its calls there, where that is built from this
+# source for the torch at hand, else in Python (ops.py): the same results, 1.4 us a tree and some 20 us a round later.
+_HOST_CALLS = ("tree_arrays", "model_arrays", "predict_packed", "build_tree", "weighted_gradient", "add_leaf_values", "next_gradient")
 try:
     from . import _host
 
     built_for = getattr(_host, "torch_version", None)
     if built_for != str(torch.__version__):
         raise ImportError("built for torch %s, this is %s" % (built_for, torch.__version__))
+    missing = [name for name in _HOST_CALLS if not callable(getattr(_host, name, None))]
+    if missing:
+        raise ImportError("built from an older source, without %s" % ", ".join(missing))
 except ImportError as e:
     _host = None
-    warnings.warn("lbtree/_host.so is missing or does not load (%s): ensembles are looked over in Python, which is slower; build it "
+    warnings.warn("lbtree/_host.so is missing or does not load (%s): its calls are made in Python, which is slower; build it "
                   "with `make -C legate-boost_amd/csrc` or __graft_entry__.build()" % e, RuntimeWarning)
 
 EXPORTS = [

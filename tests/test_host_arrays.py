@@ -294,3 +294,25 @@ def test_a_learning_rate_is_taken_or_refused_as_in_python(monkeypatch, rate, tak
         except Exception as e:
             said.append((type(e), str(e)))
     assert said[0] == said[1] and isinstance(said[0], list) == taken
+
+
+def test_the_package_imports_without_a_native_module_of_an_older_source():
+    """Built for this torch, but without the calls of a round: said so, and Python takes them all."""
+    code = ("import sys, types, warnings, torch\n"
+            "old = types.SimpleNamespace(torch_version=str(torch.__version__), **{n: print for n in ('tree_arrays', 'model_arrays', 'predict_packed')})\n"
+            "sys.modules['lbtree._host'] = old\n"
+            "with warnings.catch_warnings(record=True) as told:\n"
+            "    warnings.simplefilter('always')\n"
+            "    from lbtree import _lib, ops\n"
+            "assert _lib._host is None and ops._NATIVE is None and ops._predict_packed is None\n"
+            "assert any('without build_tree' in str(w.message) for w in told)\n")
+    package = os.path.dirname(os.path.dirname(os.path.abspath(_lib.__file__)))
+    subprocess.run([sys.executable, "-c", code], check=True, env=dict(os.environ, PYTHONPATH=package))
+
+
+def test_every_native_call_of_the_package_is_asked_for():
+    import re
+
+    source = open(os.path.join(os.path.dirname(os.path.abspath(_lib.__file__)), "ops.py")).read()
+    called = set(re.findall(r"(?:_NATIVE|_lib\._host)\.([a-z_]+)", source))
+    assert called == set(_lib._HOST_CALLS) and all(callable(getattr(_lib._host, name)) for name in called)
