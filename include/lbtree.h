@@ -506,7 +506,8 @@ int lbt_add_leaf_values(void* stream, const double* leaf_value, int32_t n_nodes,
 /*
  * lbt_add_leaf_values and lbt_weighted_gradient at the predictions that it leaves, the same bits: the end of a round and the
  * beginning of the next one (legateboost.py:260-275), one launch where the objective is formed element by element.
- * abs_sum_chunks: as lbt_weighted_gradient_sums writes them, or null. pred and leaf_value may not alias any output.
+ * abs_sum_chunks: as lbt_weighted_gradient_sums writes them, or null. pred, g, h and the chunk sums are written and may overlap neither one
+ * another nor anything that is read (leaf_value, row_leaf, y, sample_weight).
  */
 int lbt_next_gradient(void* stream, int32_t objective, const double* leaf_value, int32_t n_nodes, const int32_t* row_leaf,
                       double* pred, const double* y, const double* sample_weight, double learning_rate, int64_t n_rows,

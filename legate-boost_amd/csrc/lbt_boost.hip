@@ -4,6 +4,7 @@
 // src/utils/gather.cu:26-91. All of it is streaming work over [n_rows][n_outputs] doubles:
 // one read of every input, one write of every output.
 #include <algorithm>
+#include <iterator>
 #include <limits>
 #include <type_traits>
 
@@ -755,7 +756,21 @@ int lbt_next_gradient(void* stream, int32_t objective, const double* leaf_value,
   if (n_rows == 0) return LBT_OK;
   LBT_REQUIRE(leaf_value && row_leaf, "null pointer");
   LBT_TRY(check_gradients(pred, y, n_rows, n_outputs, g, h, abs_sum_chunks));
-  LBT_REQUIRE(leaf_value != pred && leaf_value != g && leaf_value != h, "outputs may not alias the inputs or each other");
+  // the predictions are written while everything else is read: none of what is written may overlap what is read, or one another
+  struct Range {
+    const void* begin;
+    int64_t bytes;
+  };
+  const int64_t real = sizeof(double), all = real * n_rows * n_outputs, labels = objective == LBT_OBJ_LOG_LOSS && n_outputs > 1 ? real * n_rows : all;
+  const Range ranges[] = {{pred, all}, {g, all}, {h, all}, {abs_sum_chunks, 2 * real * lbt_abs_sum_chunks(n_rows, n_outputs)},
+                          {leaf_value, real * n_nodes * n_outputs}, {row_leaf, static_cast<int64_t>(sizeof(int32_t)) * n_rows}, {y, labels},
+                          {sample_weight, real * n_rows}};
+  constexpr int kWritten = 4;
+  for (int i = 0; i < kWritten; i++)
+    for (const Range* other = ranges + i + 1; other != std::end(ranges); other++) {
+      const char *a = static_cast<const char*>(ranges[i].begin), *b = static_cast<const char*>(other->begin);
+      LBT_REQUIRE(a == nullptr || b == nullptr || a + ranges[i].bytes <= b || b + other->bytes <= a, "outputs may not alias the inputs or each other");
+    }
   return form_gradients(static_cast<hipStream_t>(stream), objective, lbt::LeafAdd{leaf_value, n_nodes, row_leaf}, pred, y, sample_weight, learning_rate,
                         n_rows, n_outputs, g, h, abs_sum_chunks);
 }

@@ -490,3 +490,26 @@ def test_the_next_gradient_checks_its_arguments():
     assert call(None, 0, one, 3, one, two, one, None, 0.1, 10, 1, three, four, C.c_void_p(3 << 20)) == -1
     assert call(None, 0, None, 3, None, None, None, None, 0.1, 0, 1, None, None, None) == 0
     assert _lib.lib.lbt_feature_mask(None, None, 3, one) == -1 and _lib.lib.lbt_feature_mask(None, one, 3, None) == -1
+
+
+@pytest.mark.parametrize("objective,k", [(0, 1), (0, 3), (1, 1), (1, 4)])
+def test_the_next_gradient_refuses_outputs_that_overlap_what_it_reads(objective, k):
+    """The predictions are written while targets, weights, leaves and leaf values are read: whole arrays, first and last entries."""
+    from lbtree import _lib
+
+    n, nodes = 10, 3
+    size = {"leaf": 8 * nodes * k, "rows": 4 * n, "pred": 8 * n * k, "y": 8 * n * (1 if objective == 1 and k > 1 else k), "w": 8 * n,
+            "g": 8 * n * k, "h": 8 * n * k, "sums": 16}
+    at = {name: (i + 1) << 20 for i, name in enumerate(size)}
+
+    def refused(**moved):
+        a = dict(at, **moved)
+        p = {name: C.c_void_p(v) for name, v in a.items()}
+        rc = _lib.lib.lbt_next_gradient(None, objective, p["leaf"], nodes, p["rows"], p["pred"], p["y"], p["w"], 0.1, n, k, p["g"], p["h"], p["sums"])
+        return rc == -1 and b"alias" in _lib.lib.lbt_last_error()
+
+    for out in ("pred", "g", "h", "sums"):
+        for name in size:
+            if name != out:
+                for shift in (0, size[out] - 4, 4 - size[name]):
+                    assert refused(**{name: at[out] + shift}), (out, name, shift)
