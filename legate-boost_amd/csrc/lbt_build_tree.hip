@@ -191,29 +191,38 @@ __device__ __forceinline__ void store_for_host(int32_t* to, int32_t v)
   __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// A workgroup's feature: its CSR row pointer (reduce_by_key + inclusive_scan, build_tree.cu:933-949) and its proposals in
-// their place, the last one +inf (build_tree.cu:953-956).
+// A workgroup's run of features: their CSR row pointers (reduce_by_key + inclusive_scan, build_tree.cu:933-949) and their proposals in
+// their place, the last one of each +inf (build_tree.cu:953-956). What lies in front of the run every workgroup adds up for itself, from the
+// counts of the launch before. There are no more than kPlaceGroups workgroups, else these loads grow with the square of the features: both
+// launches of the proposals with 2 samples of 100,000 and 262,144 features 1118 and 6971 us by a workgroup a feature; by 512 runs 147 and 364, 1024
+// 124 and 306, 2048 113 and 280, 4096 122 and 302. (As four launches with one workgroup's scan of the counts 450 and 1053.) Up to 2048
+// features a run is one: 500 with 256 samples 13.8 us.
+constexpr int kPlaceGroups = 2048;
 template <typename T>
-__device__ __forceinline__ void place_proposals(const SampleArgs<T>& a, int f, int* s_waves)
+__device__ __forceinline__ void place_proposals(const SampleArgs<T>& a, int f0, int f1, int* s_waves)
 {
   int mine = 0, b0 = 0;
-  for (int i = threadIdx.x; i < f; i += kThreads) mine += a.counts[i];
+#pragma unroll 8
+  for (int i = threadIdx.x; i < f0; i += kThreads) mine += a.counts[i];
   sum_before(mine, s_waves, &b0);
-  const int n = a.counts[f];
-  if (threadIdx.x == 0) {
-    a.row_pointers[f + 1] = b0 + n;
-    if (f == 0) a.row_pointers[0] = 0;
-    if (a.host_row_pointers != nullptr) {
-      store_for_host(a.host_row_pointers + f + 1, b0 + n);
-      if (f == 0) store_for_host(a.host_row_pointers, 0);
+  for (int f = f0; f < f1; f++) {
+    const int n = a.counts[f];
+    if (threadIdx.x == 0) {
+      a.row_pointers[f + 1] = b0 + n;
+      if (f == 0) a.row_pointers[0] = 0;
+      if (a.host_row_pointers != nullptr) {
+        store_for_host(a.host_row_pointers + f + 1, b0 + n);
+        if (f == 0) store_for_host(a.host_row_pointers, 0);
+      }
     }
-  }
-  for (int i = threadIdx.x; i < n; i += kThreads) {
-    T v = a.uniq[static_cast<int64_t>(f) * a.S + i];
-    if (i == n - 1) v = std::numeric_limits<T>::infinity();
-    a.proposals[b0 + i]   = v;
-    a.bin_feature[b0 + i] = f;
-    if (a.as_double != nullptr) a.as_double[b0 + i] = static_cast<double>(v);
+    for (int i = threadIdx.x; i < n; i += kThreads) {
+      T v = a.uniq[static_cast<int64_t>(f) * a.S + i];
+      if (i == n - 1) v = std::numeric_limits<T>::infinity();
+      a.proposals[b0 + i]   = v;
+      a.bin_feature[b0 + i] = f;
+      if (a.as_double != nullptr) a.as_double[b0 + i] = static_cast<double>(v);
+    }
+    b0 += n;
   }
 }
 
@@ -332,12 +341,13 @@ __global__ void __launch_bounds__(kThreads) tree_start_kernel(SampleArgs<T> a, S
   init.entry(static_cast<int64_t>(id - sums.m) * kThreads + threadIdx.x);
 }
 template <typename T>
-__global__ void __launch_bounds__(kThreads) tree_scales_kernel(SampleArgs<T> a, SumArgs sums)
+__global__ void __launch_bounds__(kThreads) tree_scales_kernel(SampleArgs<T> a, int run, SumArgs sums)
 {
   __shared__ TwoSums s_sums;
   __shared__ int s_waves[kThreads / 64];
-  if (static_cast<int>(blockIdx.x) < a.F)
-    place_proposals(a, blockIdx.x, s_waves);
+  const int f = static_cast<int>(blockIdx.x) * run;  // (in range: no more than kPlaceGroups + 1 workgroups of ceil(F / kPlaceGroups))
+  if (f < a.F)
+    place_proposals(a, f, min(a.F, f + run), s_waves);
   else
     find_scales(sums, s_sums);
 }
@@ -2037,7 +2047,9 @@ int start_tree(hipStream_t stream, SampleArgs<T> samples, const InitArgs* init, 
     }
     sums.n_of = static_cast<int>(m);
   }
-  tree_scales_kernel<T><<<static_cast<unsigned>(samples.F + (scales != nullptr ? 1 : 0)), kThreads, 0, stream>>>(samples, sums);
+  const int run    = std::max(0, samples.F - 1) / kPlaceGroups + 1;  // features of a workgroup
+  const int placed = samples.F > 0 ? (samples.F - 1) / run + 1 : 0;
+  tree_scales_kernel<T><<<static_cast<unsigned>(placed + (scales != nullptr ? 1 : 0)), kThreads, 0, stream>>>(samples, run, sums);
   LBT_HIP(hipGetLastError());
   return LBT_OK;
 }

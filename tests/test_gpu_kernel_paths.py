@@ -1084,3 +1084,42 @@ def test_scales_of_the_absolute_sums(n):
             s = level(s)
         assert scales[at].item() == 2147483647.0 / s[0] and scales[2 + at].item() == 1.0 / scales[at].item()
     assert torch.equal(sums, q.to(torch.int64).sum(dim=0))
+
+
+@pytest.mark.parametrize("f,s", [(2047, 3), (2048, 2), (2049, 5), (4097, 33), (10_001, 2)])
+def test_proposals_of_many_features_are_placed(f, s):
+    """One feature a workgroup, and runs of several: row pointers and proposals are the oracle's."""
+    import gpu_util as gu
+    import oracle_lib as orc
+    from lbtree import ops
+
+    rs = np.random.RandomState(f)
+    X = np.round(rs.randn(40, f) * 2).astype(np.float32)
+    props, rp = ops.select_split_samples(torch.from_numpy(X).cuda(), s, 7)
+    want_props, want_rp = orc.split_proposals(X, 7, s)
+    assert np.array_equal(gu.cpu(rp), want_rp) and np.array_equal(gu.cpu(props), want_props)
+
+
+def test_placing_proposals_does_not_grow_with_the_square_of_the_features():
+    """8 times the features take 8 times as long at most, give or take: 262,144 of them 280 us, 6971 with a sum over all features in front for
+    each (32,768: 44 and 180)."""
+    from lbtree import _lib, ops
+
+    def best_us(f):
+        X = torch.zeros((4, f), device="cuda")
+        ws = torch.empty(_lib.lib.lbt_select_split_samples_workspace_bytes(f, 2, 0), dtype=torch.uint8, device="cuda")
+        props, rp = torch.empty(2 * f, device="cuda"), torch.empty(f + 1, dtype=torch.int32, device="cuda")
+        best = float("inf")
+        for _ in range(6):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            for _ in range(4):
+                _lib.check(_lib.lib.lbt_select_split_samples(ops._stream(), X.data_ptr(), 0, 0, 4, f, 2, 3, 4, props.data_ptr(), rp.data_ptr(),
+                                                             ws.data_ptr(), ws.numel()))
+            end.record()
+            end.synchronize()
+            best = min(best, begin.elapsed_time(end) / 4 * 1e3)
+        return best
+
+    few, many = best_us(32_768), best_us(262_144)
+    assert many < 16 * few, (few, many)
