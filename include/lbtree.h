@@ -568,6 +568,12 @@ void lbt_profile_enable(int on);
 void lbt_profile_reset(void);
 void lbt_profile_get(lbt_profile* out);
 
+/* For tests of the scheduling inside lbt_build_tree. Where few rows take all levels in one launch, a workgroup looks `looks` times for what
+ * the others find in the root before it takes over a feature whose workgroup has not begun; with 0 features are taken over
+ * that nobody need take over. The trees are the same. Holds for builds of the calling thread until it calls this again: below 0, the
+ * library's own number, which is also the most. */
+void lbt_small_levels_polls(int32_t looks);
+
 #ifdef __cplusplus
 }
 #endif

@@ -2016,5 +2016,7 @@ template int small_tree_build<double>(hipStream_t, const SmallTreeState&, const 
 
 }  // namespace lbt
 
-// For tests, of the calling thread: with 0 looks features are taken over that nobody need take over; below 0: as it is without this call.
-extern "C" void lbt_small_levels_polls(int polls) { lbt::levels_polls = polls < 0 ? lbt::kLevelsPolls : polls; }
+void lbt_small_levels_polls(int32_t looks)
+{
+  lbt::levels_polls = looks < 0 ? lbt::kLevelsPolls : std::min<int>(looks, lbt::kLevelsPolls);  // (a wait is never longer than the library's own)
+}

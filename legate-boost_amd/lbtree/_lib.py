@@ -226,6 +226,8 @@ def _load():
     lib.lbt_profile_reset.restype = None
     lib.lbt_profile_get.restype = None
     lib.lbt_profile_get.argtypes = [C.POINTER(Profile)]
+    lib.lbt_small_levels_polls.restype = None
+    lib.lbt_small_levels_polls.argtypes = [C.c_int32]
     return lib
 
 
@@ -262,7 +264,7 @@ EXPORTS = [
     "lbt_histogram_level_workspace_bytes", "lbt_histogram_level", "lbt_scan", "lbt_best_split_workspace_bytes",
     "lbt_best_split", "lbt_update_positions_workspace_bytes", "lbt_update_positions",
     "lbt_profile_enable", "lbt_profile_reset",
-    "lbt_profile_get",
+    "lbt_profile_get", "lbt_small_levels_polls",
 ]
 
 

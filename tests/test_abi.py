@@ -28,6 +28,19 @@ def test_library_exports_every_declared_symbol():
     assert _lib.lib.lbt_release_thread_resources() == 0  # nothing held yet: nothing to do, no GPU call
 
 
+def test_library_exports_nothing_that_is_not_declared():
+    """The C names of the library are those of the header, and the binding gives every one its argument types."""
+    import subprocess
+
+    from lbtree import _lib
+
+    lines = subprocess.run(["nm", "-D", "--defined-only", _lib.SO_PATH], check=True, capture_output=True, text=True).stdout.splitlines()
+    assert sorted(n for n in (line.split()[-1] for line in lines) if re.fullmatch(r"lbt_[a-z0-9_]+", n)) == declared_symbols()
+    header = open(os.path.join(ROOT, "include", "lbtree.h")).read()
+    untyped = [n for n in _lib.EXPORTS if getattr(_lib.lib, n).argtypes is None and not re.search(n + r"\s*\(void\)", header)]
+    assert untyped == []
+
+
 def test_workspace_query():
     from lbtree import _lib
 
