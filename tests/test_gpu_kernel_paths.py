@@ -945,10 +945,10 @@ def test_scanned_levels_in_32_bits(n, f, k, s, kind):
 
 @pytest.mark.parametrize("n,f,k,s,depth,kind", [
     (9001, 60, 1, 512, 12, "plain"),        # more nodes than a slab decides, at last
-    (9001, 513, 2, 64, 9, "plain"),         # more candidates than a slab reads: a launch of its own
+    (9001, 513, 2, 64, 11, "plain"),        # more candidates than a slab reads: a launch of its own
     (8200, 100, 3, 256, 10, "empty"),       # most nodes without rows
-    (20479, 90, 1, 256, 10, "retired"),     # rows that stop early lie in front
-    (20480, 80, 1, 300, 10, "zero"),
+    (20479, 90, 1, 256, 11, "retired"),     # rows that stop early lie in front
+    (20480, 80, 1, 300, 11, "zero"),
     (20481, 80, 2, 300, 10, "negative"),    # splits of nodes without rows: a launch of its own
 ])
 def test_levels_of_the_general_builder_that_begin_in_one_launch(n, f, k, s, depth, kind):
@@ -976,6 +976,29 @@ def test_levels_of_the_general_builder_that_begin_in_one_launch(n, f, k, s, dept
     for name in ("leaf_value", "feature", "split_value", "gain", "hessian", "row_leaf"):
         assert torch.equal(getattr(got, name), getattr(want, name)), name
     gu.check_row_leaf(got, X)
+    assert _takes_the_general_builder(lambda: ops.build_tree(Xd, gd, hd, **kw))
+
+
+def _takes_the_general_builder(build):
+    """The other builders round the gradients in a launch that does more, and report none of this class."""
+    from lbtree import _lib
+
+    _lib.profile_reset()
+    _lib.profile_enable(1)
+    try:
+        build()
+        return _lib.profile_get()["quantise"]["launches"] == 1
+    finally:
+        _lib.profile_enable(0)
+        _lib.profile_reset()
+
+
+def test_which_builder_a_profile_tells():
+    from lbtree import ops
+
+    for n, f, depth, general in ((1000, 5, 4, False), (9001, 9, 6, False), (9001, 50, 11, True)):
+        X, g = torch.rand((n, f), device="cuda"), torch.rand((n, 1), device="cuda", dtype=torch.float64)
+        assert _takes_the_general_builder(lambda: ops.build_tree(X, g - 0.5, g + 0.1, max_depth=depth, split_samples=64, seed=1)) == general
 
 
 @pytest.mark.parametrize("n,f,k,s,depth,kind", [
@@ -985,7 +1008,8 @@ def test_levels_of_the_general_builder_that_begin_in_one_launch(n, f, k, s, dept
     (12000, 131, 1, 256, 5, "excluded"),
     (8200, 33, 2, 300, 7, "l1"),             # two-byte bins, a tile that is not full
     (70000, 40, 3, 129, 7, "zeros"),         # ranges of rows past those asked for ahead
-    (9001, 64, 16, 32, 5, "excluded"),
+    (9001, 128, 16, 32, 5, "excluded"),      # the most outputs
+    (9001, 130, 8, 100, 5, "zeros"),         # tiles and many outputs in turn
     (8193, 130, 1, 2048, 5, "l1"),
     (200000, 16, 5, 257, 6, "plain"),        # by workgroups: 16 ranges and more, a second tile of bins, several outputs
 ])
