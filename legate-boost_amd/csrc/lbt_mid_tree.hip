@@ -1241,7 +1241,7 @@ bool mid_beats_small(int64_t N, int F, int K, int max_depth, int S)
   const double d = max_depth, n = static_cast<double>(N), f = F, k = K;
   const double small_us = 25.0 + d * (8.7 + 2.0 * k + 1.8e-3 * n * k * (N > 4096 && K > 1 ? 1.5 : 1.0) + 7.1e-6 * n * f);
   const double nodes = static_cast<double>(int64_t(1) << max_depth), tiles = (S + kScan - 1) / kScan;
-  // histograms of all nodes in MB, or of those that rows reach: four bins per value and level
+  // histograms of all nodes in MB, or of those that rows reach: four bins per value and level (16 bytes a bin, as the sum was fitted; they take 8 now)
   const double hist_mb = std::min(nodes * f * S * k * 16.0, n * f * k * d * 64.0) / 1048576.0;
   const double mid_us  = 16.0 + d * (19.5 + 1.14 * k * tiles) + 0.29 * hist_mb + 1.0e-3 * nodes * f * k * tiles + 1.74e-6 * n * f * k * d;
   return 1.15 * mid_us < small_us;
