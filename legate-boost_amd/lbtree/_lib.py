@@ -234,7 +234,7 @@ def _load():
 lib = _load()
 
 # The ensemble calls look their trees over in native code, and a round of boosting makes its calls there, where that is built from this
-# source for the torch at hand, else in Python (ops.py): the same results, 1.4 us a tree and some 20 us a round later.
+# source for the torch at hand, else in Python (ops.py): the same results, 1.4 us a tree and up to 20 us a round later.
 _HOST_CALLS = ("tree_arrays", "model_arrays", "predict_packed", "build_tree", "weighted_gradient", "add_leaf_values", "next_gradient")
 try:
     from . import _host

@@ -1125,8 +1125,8 @@ def test_proposals_of_many_features_are_placed(f, s):
 
 
 def test_placing_proposals_does_not_grow_with_the_square_of_the_features():
-    """8 times the features take 8 times as long at most, give or take: 262,144 of them 280 us, 6971 with a sum over all features in front for
-    each (32,768: 44 and 180)."""
+    """8 times the features may take 16 times as long: 32,768 and 262,144 of them 41 and 278 us (6.8 times), 165 and 6974 (42 times) with a sum
+    over all features in front for each."""
     from lbtree import _lib, ops
 
     def best_us(f):
